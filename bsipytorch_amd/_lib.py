@@ -44,6 +44,7 @@ PROTOTYPES = {
     "bsi_hip_pack_bits_batch": [_vp, _i64, _i64, _i, _i, _vp, _vp],
     "bsi_hip_decimal_stats": [_vp, _i64, _i64, _vp, _vp, _vp],
     "bsi_hip_build_fixed": [_vp, _i, _i64, _i64, _i, _i, _i, _f, _vp, _vp, _vp, _vp, _vp],
+    "bsi_hip_build_fixed_keys": [_vp, _i, _i64, _i64, _i, _i, _vp, _vp, _vp, _vp, _vp],
     "bsi_hip_slice_popcount_sum": [_vp, _i, _i, _vp, _vp],
     "bsi_hip_compress_flags_from_density": [_vp, _i, _i, _d, _vp, _vp],
     "bsi_hip_ewah_size": [_vp, _i, _i, _vp, _vp, _vp],

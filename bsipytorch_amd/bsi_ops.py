@@ -727,6 +727,13 @@ def canonical_key_planes(keys: "PrebuiltBSIKeysCUDA") -> torch.Tensor:
     return t.reshape(tiles * 16, Sb, chunks * 4)[:R, :, :W].contiguous()
 
 
+def _one_launch_key_build(f: dict, x: torch.Tensor, decimals: int) -> bool:
+    """Whether bsi_hip_build_fixed_keys makes every representation this configuration keeps of a keyset: tiled planes and
+    the row-major int8 image, from 2 to 8 bits, at most two decimal places and no clipping."""
+    return (x.numel() > 0 and 2 <= f["bits_k"] <= 8 and f["clip_k"] == 0.0 and 0 <= decimals <= 2 and f["tiled"] and f["key_image"]
+            and not f["image_tiled"])
+
+
 def build_bsi_keys_cuda(K: torch.Tensor, decimal_places: int, compress_threshold: float = 0.2):
     """bsi_cuda.cpp:863-910 (fixed-bit branch): per-row scale, Sb slices, ``Bw[r, j] = w_j * 2^shift_r``.
     Returns (handle, total_bytes_of_words, num_keys, d, W)."""
@@ -749,17 +756,27 @@ def build_bsi_keys_cuda(K: torch.Tensor, decimal_places: int, compress_threshold
         if f["debug"]:
             print(f"[BSI_HIP] build_bsi_keys_cuda (decimal): R={R} slices={S} words_per_slice={h.W}")
         return h, int(words.numel() * 8), int(R), int(d), int(h.W)
-    words, shifts, scales, _ = _build_fixed(x, int(decimal_places), f["bits_k"], False, want_ints8=False)
     h = PrebuiltBSIKeysCUDA()
     h.num_keys, h.d = int(R), int(d)
-    h.W = words.shape[2]
+    h.W = (d + 63) // 64 if d > 0 else 1
     h.Sb = f["bits_k"]
     h.decimals = int(decimal_places)
     h.threshold = float(compress_threshold)
-    h.shifts = shifts
-    h.slice_weights = (_slice_weights(h.Sb, 0, True, dev).unsqueeze(0) * scales.unsqueeze(1)).contiguous()
-    total_bytes = words.numel() * 8
-    _install_fixed_key_planes(h, words)
+    if _one_launch_key_build(f, x, h.decimals):
+        chunks = (h.W + 3) // 4
+        h.words = torch.empty(((R + 15) // 16, chunks, h.Sb, 64), dtype=torch.int64, device=dev)
+        h.layout = _lib.LAYOUT_TILED16
+        h.ints8 = torch.empty((R, chunks * 256), dtype=torch.int8, device=dev)
+        h.shifts = torch.empty((R,), dtype=torch.int32, device=dev)
+        h.slice_weights = torch.empty((R, h.Sb), dtype=torch.float32, device=dev)
+        check(lib.bsi_hip_build_fixed_keys(x.data_ptr(), _dtype_code(x), R, d, h.decimals, h.Sb, h.words.data_ptr(),
+                                           h.ints8.data_ptr(), h.shifts.data_ptr(), h.slice_weights.data_ptr(), _stream()),
+              "bsi_hip_build_fixed_keys")
+    else:
+        words, h.shifts, scales, _ = _build_fixed(x, h.decimals, h.Sb, False, want_ints8=False)
+        h.slice_weights = (_slice_weights(h.Sb, 0, True, dev).unsqueeze(0) * scales.unsqueeze(1)).contiguous()
+        _install_fixed_key_planes(h, words)
+    total_bytes = R * h.Sb * h.W * 8
     if f["debug"]:
         print(f"[BSI_HIP] build_bsi_keys_cuda: R={R} slices={h.Sb} words_per_slice={h.W} layout={h.layout}")
     return h, int(total_bytes), int(R), int(d), int(h.W)

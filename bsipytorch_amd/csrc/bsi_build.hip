@@ -10,7 +10,7 @@
 // Arithmetic follows the reference's quantiser kernels (bsi_ops/csrc/cuda/bsi_cuda_kernels_quant.cuh:
 // rounding :24-29, shift :82-108, rounded shift + clamp :205-226) and packer
 // (bsi_cuda_kernels_pack.cuh:129-174).
-#include "bsi_common.h"
+#include "bsi_quant_device.h"
 
 namespace bsi {
 
@@ -259,162 +259,62 @@ __global__ void build_fixed_chunk_kernel(const T* __restrict__ x, int64_t Q, int
     build_chunk_item<T>(x, wave, d, chunks, slices, words_per_slice, dec_scale, clip_k, words, shifts, scales, ints8, lane);
 }
 
-// The same build for the common case (at most 8 slices, no clipping, whole chunks of words), about
-// seven times fewer instructions per element.  One wave takes 8 consecutive (row, chunk) items:
-//   * round-half-away(v * 10^dec) comes from the float's mantissa in 32-bit integer arithmetic when 10^dec is
-//     an integer of at most 127 (the same integer as the exact float64 product + 0.5 and floor, checked on every
-//     float), else from that float64 sequence; everything after it is 32-bit integer work; an item holding a
-//     magnitude the 32-bit route does not cover (2^31 or more after scaling, a NaN) is handed to the 64-bit
-//     routine above, so results never differ;
-//   * the quantised values go to LDS as the int8 image (value << (8 - slices), the MFMA core's
-//     in-chunk order); the image is the bit-transpose of the planes, 32 elements at a time, so
-//     lane (item j, unit w) reads its 8 dwords, transposes the 8x8 bit blocks in registers and
-//     has one 32-bit half-word of every slice: no ballots, and all 64 lanes busy.
-// kFastItems = items per wave (1, 2, 4 or 8): fewer for small inputs, where the length of one wave's
-// instruction stream, not the throughput, sets the kernel's duration.
-template <typename T, int kFastItems>
+// The same build for the common case (at most 8 slices, no clipping, whole chunks of words, 10^dec an integer of at
+// most 127): a wave takes kItems consecutive (row, chunk) items, all loads first, and quantises each in registers
+// (bsi_quant_device.h).  The lane that loads four consecutive elements is chosen so that two DPP exchanges leave every
+// lane with one dword of the int8 image, and three more with one 32-element half-word of one plane: no LDS, and the
+// image is written 256 contiguous bytes an item.  kPlanes = false leaves the planes out (a linear layer's dot on the
+// matrix cores reads the image only).  Bound by VALU issue at about 90 instructions an item (float32; 70 for half
+// types), near the memory time of the larger inputs.
+// 4096 x 4096 bfloat16: 47 us through LDS bytes and 32-bit integers, 15.5 us this way, 12.6 us without the planes (50 MB
+// at 4 TB/s).
+template <typename T, int kItems, bool kVec, bool kPlanes>
 __global__ __launch_bounds__(kBlock) void build_fixed_chunk_fast_kernel(
-    const T* __restrict__ x, int64_t Q, int64_t d, int chunks, int slices, int words_per_slice, double dec_scale,
-    unsigned scale_int, unsigned long long* __restrict__ words, int* __restrict__ shifts, float* __restrict__ scales,
+    const T* __restrict__ x, unsigned total, int64_t d, unsigned chunks, int slices, int words_per_slice, double dec_scale,
+    float scale, unsigned long long* __restrict__ words, int* __restrict__ shifts, float* __restrict__ scales,
     int8_t* __restrict__ ints8) {
-    __shared__ uint32_t image[kWavesPerBlock][kFastItems][BSI_CHUNK_ELEMS / 4];
     const int lane = threadIdx.x & (BSI_WAVE - 1);
-    const int wib = threadIdx.x >> 6;
-    const int64_t total = Q * chunks;
-    const int64_t item0 = (static_cast<int64_t>(blockIdx.x) * kWavesPerBlock + wib) * kFastItems;
-    // (row, chunk) of item0 + j without a 64-bit division per item
-    const int64_t row0 = item0 / chunks;
-    const unsigned c0 = static_cast<unsigned>(item0 - row0 * chunks);
-#define BSI_ITEM_ROW_CHUNK(j, row, c)                                  \
-    const unsigned cj_##row = c0 + static_cast<unsigned>(j);          \
-    const unsigned dr_##row = cj_##row / static_cast<unsigned>(chunks); \
-    const int64_t row = row0 + dr_##row;                               \
-    const int c = static_cast<int>(cj_##row - dr_##row * static_cast<unsigned>(chunks));
-    const int qmax = (1 << (slices - 1)) - 1, qmin = -(1 << (slices - 1));
-    unsigned slow = 0u;  // items that took the 64-bit routine (their outputs are already written)
-    // all loads of the wave's 8 items first: one memory latency, not eight
-    float raw[kFastItems][4];
+    const unsigned item0 = (blockIdx.x * kWavesPerBlock + static_cast<unsigned>(__builtin_amdgcn_readfirstlane(threadIdx.x >> 6))) * kItems;
+    if (item0 >= total) return;
+    const ChunkLane cl = chunk_lane(lane);
+    const QuantRange range = quant_range(slices);
+    float v[kItems][4];
+    unsigned row[kItems], col[kItems];
 #pragma unroll
-    for (int j = 0; j < kFastItems; ++j) {
-        const int64_t item = item0 + j;
-        BSI_ITEM_ROW_CHUNK(j, row, c)
-        const int64_t start = static_cast<int64_t>(c) * BSI_CHUNK_ELEMS;
+    for (int j = 0; j < kItems; ++j) {
+        const unsigned item = item0 + j < total ? item0 + j : total - 1;  // a wave past the end repeats the last item
+        row[j] = item / chunks;
+        col[j] = item - row[j] * chunks;
+        load_chunk_quad<T, kVec>(x + static_cast<int64_t>(row[j]) * d, d, static_cast<int>(col[j]), cl, v[j]);
+    }
 #pragma unroll
-        for (int k = 0; k < 4; ++k) {
-            const int64_t e = start + k * BSI_WAVE + lane;
-            raw[j][k] = (item < total && e < d) ? load_as_float<T>(x, row * d + e) : 0.0f;
+    for (int j = 0; j < kItems; ++j) {
+        const unsigned item = item0 + j < total ? item0 + j : total - 1;
+        const unsigned mx = wave_max_u32(quad_max_bits(v[j]));
+        int shift;
+        uint32_t image;
+        if (mx < kQuantWideBits) {
+            shift = quant_shift(mx, scale, slices);
+            image = quantise_quad<T>(v[j], scale, shift, range);
+        } else {
+            shift = compute_shift(wave_max_u64(quad_max_wide(v[j], dec_scale)), 0.0, BSI_CHUNK_ELEMS, slices, 0.0f);
+            image = quantise_quad_wide(v[j], dec_scale, shift, slices);
         }
-    }
-#pragma unroll
-    for (int j = 0; j < kFastItems; ++j) {
-        const int64_t item = item0 + j;
-        if (item < total) {
-            BSI_ITEM_ROW_CHUNK(j, row, c)
-            (void)row;
-            const int64_t start = static_cast<int64_t>(c) * BSI_CHUNK_ELEMS;
-            const int valid = static_cast<int>((d - start) < BSI_CHUNK_ELEMS ? (d - start) : BSI_CHUNK_ELEMS);
-            // magnitudes of round-half-away(x * 10^dec): from the float's mantissa when 10^dec is a small integer
-            // (scaled_magnitude_u32), else in float64; elements past the end were loaded as 0
-            unsigned mag[4];
-            bool big = false;
-            if (scale_int != 0u) {
-#pragma unroll
-                for (int k = 0; k < 4; ++k) mag[k] = scaled_magnitude_u32(raw[j][k], scale_int, big);
-            } else {
-#pragma unroll
-                for (int k = 0; k < 4; ++k) {
-                    const double xs = __dmul_rn(static_cast<double>(raw[j][k]), dec_scale);
-                    const bool b = !(fabs(xs) < 2147483000.0);
-                    big = big || b;
-                    mag[k] = b ? 0u : static_cast<unsigned>(static_cast<int>(floor(__dadd_rn(fabs(xs), 0.5))));
-                }
-            }
-            if (__any(big)) {
-                slow |= 1u << j;  // done below by the 64-bit routine
-            } else {
-                unsigned mx = 0u;
-#pragma unroll
-                for (int k = 0; k < 4; ++k) mx = mag[k] > mx ? mag[k] : mx;
-                mx = wave_max_u32(mx);
-                const int shift = compute_shift(static_cast<unsigned long long>(mx), 0.0, valid, slices, 0.0f);
-                if (lane == 0) {
-                    shifts[item] = shift;
-                    scales[item] = static_cast<float>(1ULL << shift);
-                }
-                const unsigned round_add = (shift > 0) ? (1u << (shift - 1)) : 0u;
-                unsigned char* img = reinterpret_cast<unsigned char*>(image[wib][j]);
-#pragma unroll
-                for (int k = 0; k < 4; ++k) {
-                    const int qa = static_cast<int>((mag[k] + round_add) >> shift);
-                    int q = (raw[j][k] < 0.0f) ? -qa : qa;
-                    q = q < qmin ? qmin : (q > qmax ? qmax : q);
-                    img[mfma_byte_pos(k * BSI_WAVE + lane)] = static_cast<unsigned char>(q << (8 - slices));
-                }
-            }
+        image = chunk_image_dword(image, cl);
+        if (lane == 0) {
+            shifts[item] = shift;
+            scales[item] = static_cast<float>(1ULL << shift);
         }
-    }
-    if (slow != 0u) {
-#pragma unroll 1
-        for (int j = 0; j < kFastItems; ++j)
-            if (slow & (1u << j))
-                build_chunk_item<T>(x, item0 + j, d, chunks, slices, words_per_slice, dec_scale, 0.0f, words, shifts,
-                                    scales, ints8, lane);
-    }
-    __syncthreads();
-    // the int8 image: 256 bytes per item, one dword per lane
-    if (ints8 != nullptr) {
-#pragma unroll 1
-        for (int j = 0; j < kFastItems; ++j) {
-            const int64_t item = item0 + j;
-            if (item >= total) break;
-            if (slow & (1u << j)) continue;
-            reinterpret_cast<uint32_t*>(ints8)[static_cast<size_t>(item) * (BSI_CHUNK_ELEMS / 4) + lane] = image[wib][j][lane];
-        }
-    }
-    // the planes: lane = (item j, 32-element unit w)
-    {
-        const int j = lane >> 3, w = lane & 7;
-        const int64_t item = item0 + j;
-        if (j < kFastItems && item < total && !(slow & (1u << j))) {
-            uint32_t y[8];
-            const uint4 lo = *reinterpret_cast<const uint4*>(&image[wib][j][w * 8]);
-            const uint4 hi = *reinterpret_cast<const uint4*>(&image[wib][j][w * 8 + 4]);
-            y[0] = lo.x; y[1] = lo.y; y[2] = lo.z; y[3] = lo.w;
-            y[4] = hi.x; y[5] = hi.y; y[6] = hi.z; y[7] = hi.w;
-            // bit b of image byte (element 8m + t) <-> bit (8m + t) of plane b's half-word: an 8x8 bit transpose
-            uint32_t a[8];
-#pragma unroll
-            for (int s2 = 0; s2 < 4; ++s2) {
-                const uint32_t l = y[s2], h = y[s2 + 4];
-                a[s2] = (l & 0x0F0F0F0Fu) | ((h << 4) & 0xF0F0F0F0u);
-                a[s2 + 4] = ((l >> 4) & 0x0F0F0F0Fu) | (h & 0xF0F0F0F0u);
-            }
-#pragma unroll
-            for (int b = 0; b < 8; b += 4)
-#pragma unroll
-                for (int s2 = b; s2 < b + 2; ++s2) {
-                    const uint32_t l = a[s2], h = a[s2 + 2];
-                    y[s2] = (l & 0x33333333u) | ((h << 2) & 0xCCCCCCCCu);
-                    y[s2 + 2] = ((l >> 2) & 0x33333333u) | (h & 0xCCCCCCCCu);
-                }
-#pragma unroll
-            for (int s2 = 0; s2 < 8; s2 += 2) {
-                const uint32_t l = y[s2], h = y[s2 + 1];
-                a[s2] = (l & 0x55555555u) | ((h << 1) & 0xAAAAAAAAu);
-                a[s2 + 1] = ((l >> 1) & 0x55555555u) | (h & 0xAAAAAAAAu);
-            }
-            BSI_ITEM_ROW_CHUNK(j, row, c)
-            uint32_t* out32 = reinterpret_cast<uint32_t*>(words) +
-                              (static_cast<size_t>(row) * slices * words_per_slice + static_cast<size_t>(c) * 4) * 2 + w;
-#pragma unroll
-            for (int t = 0; t < 8; ++t) {
-                const int sl = t - (8 - slices);  // image bit t is slice t - (8 - slices)
-                if (sl >= 0) out32[static_cast<size_t>(sl) * words_per_slice * 2] = a[t];
-            }
+        if (ints8 != nullptr) reinterpret_cast<uint32_t*>(ints8)[static_cast<size_t>(item) * (BSI_CHUNK_ELEMS / 4) + lane] = image;
+        if (kPlanes) {
+            const uint32_t plane = chunk_plane_dword(image, cl);  // by all lanes: it exchanges registers between them
+            const int sl = (lane & 7) - (8 - slices);
+            if (sl >= 0)
+                reinterpret_cast<uint32_t*>(words)[(static_cast<size_t>(row[j]) * slices + sl) * (2 * words_per_slice) +
+                                                   col[j] * 8 + (lane >> 3)] = plane;
         }
     }
 }
-#undef BSI_ITEM_ROW_CHUNK
 
 // Row-scale build: one block per row; pass 1 reduces the row maximum, pass 2 (row now in cache)
 // quantises and packs, one wave per group of 4 words.
@@ -475,6 +375,196 @@ __global__ void build_fixed_row_kernel(const T* __restrict__ x, int64_t Q, int64
         }
         ballot_pack_store(v, slices, lane, c, words_per_slice,
                           words + static_cast<size_t>(row) * slices * words_per_slice);
+    }
+}
+
+// The row-scale build for the same common case, one workgroup per row: the row's quads stay in registers between the
+// maximum and the quantiser (kHeld chunks a wave; the rest of a longer row is loaded again).  Query batches whose width
+// is not a whole number of chunks come here.  77 rows of 1600: 11.0 us in two passes of 64-bit arithmetic, 4.8 us.
+template <typename T, bool kVec, bool kPlanes>
+__global__ __launch_bounds__(kBlock) void build_fixed_row_fast_kernel(const T* __restrict__ x, int64_t d, int chunks, int slices,
+                                                                      int words_per_slice, double dec_scale, float scale,
+                                                                      unsigned long long* __restrict__ words,
+                                                                      int* __restrict__ shifts, float* __restrict__ scales,
+                                                                      int8_t* __restrict__ ints8) {
+    constexpr int kHeld = 4;
+    __shared__ unsigned smax[kWavesPerBlock];
+    __shared__ unsigned long long smax64[kWavesPerBlock];
+    const int lane = threadIdx.x & (BSI_WAVE - 1);
+    const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int64_t row = blockIdx.x;
+    const T* xrow = x + row * d;
+    const ChunkLane cl = chunk_lane(lane);
+    float v[kHeld][4];
+    unsigned mx = 0u;
+#pragma unroll
+    for (int j = 0; j < kHeld; ++j) load_chunk_quad<T, kVec>(xrow, d, wid + j * kWavesPerBlock, cl, v[j]);  // past the row: zeros
+#pragma unroll
+    for (int j = 0; j < kHeld; ++j) {
+        const unsigned m = quad_max_bits(v[j]);
+        mx = m > mx ? m : mx;
+    }
+    for (int c = wid + kHeld * kWavesPerBlock; c < chunks; c += kWavesPerBlock) {
+        float t[4];
+        load_chunk_quad<T, kVec>(xrow, d, c, cl, t);
+        const unsigned m = quad_max_bits(t);
+        mx = m > mx ? m : mx;
+    }
+    mx = wave_max_u32(mx);
+    if (lane == 0) smax[wid] = mx;
+    __syncthreads();
+    mx = 0u;
+#pragma unroll
+    for (int w = 0; w < kWavesPerBlock; ++w) mx = smax[w] > mx ? smax[w] : mx;
+    const bool wide = mx >= kQuantWideBits;
+    int shift = quant_shift(mx, scale, slices);
+    if (wide) {
+        unsigned long long m64 = 0ULL;
+        for (int c = wid; c < chunks; c += kWavesPerBlock) {
+            float t[4];
+            load_chunk_quad<T, kVec>(xrow, d, c, cl, t);
+            const unsigned long long m = quad_max_wide(t, dec_scale);
+            m64 = m > m64 ? m : m64;
+        }
+        m64 = wave_max_u64(m64);
+        if (lane == 0) smax64[wid] = m64;
+        __syncthreads();
+        for (int w = 0; w < kWavesPerBlock; ++w) m64 = smax64[w] > m64 ? smax64[w] : m64;
+        shift = compute_shift(m64, 0.0, 1, slices, 0.0f);
+    }
+    if (threadIdx.x == 0) {
+        shifts[row] = shift;
+        scales[row] = static_cast<float>(1ULL << shift);
+    }
+    const QuantRange range = quant_range(slices);
+    auto emit = [&](int c, const float (&t)[4]) {
+        const uint32_t image = chunk_image_dword(wide ? quantise_quad_wide(t, dec_scale, shift, slices)
+                                                      : quantise_quad<T>(t, scale, shift, range), cl);
+        if (ints8 != nullptr)
+            reinterpret_cast<uint32_t*>(ints8)[(static_cast<size_t>(row) * chunks + c) * (BSI_CHUNK_ELEMS / 4) + lane] = image;
+        if (kPlanes) {
+            const int sl = (lane & 7) - (8 - slices), unit = c * 8 + (lane >> 3);
+            const uint32_t plane = chunk_plane_dword(image, cl);
+            if (sl >= 0 && unit < 2 * words_per_slice)
+                reinterpret_cast<uint32_t*>(words)[(static_cast<size_t>(row) * slices + sl) * (2 * words_per_slice) + unit] = plane;
+        }
+    };
+#pragma unroll
+    for (int j = 0; j < kHeld; ++j)
+        if (wid + j * kWavesPerBlock < chunks) emit(wid + j * kWavesPerBlock, v[j]);
+    for (int c = wid + kHeld * kWavesPerBlock; c < chunks; c += kWavesPerBlock) {
+        float t[4];
+        load_chunk_quad<T, kVec>(xrow, d, c, cl, t);
+        emit(c, t);
+    }
+}
+
+// The whole of a fixed-bit key build for the common case: one workgroup = 16 rows (a tile of the tiled planes), a wave
+// each.  A wave reads its row once: the signed magnitudes of the first kHeld chunks stay in registers as 16-bit pairs
+// until the row's maximum is known (a row with |x| of 256 or more, and the rest of a longer row, is read again).  It
+// writes the int8 image, 256 contiguous bytes a chunk, and puts its planes' half-words into LDS, from where the
+// workgroup writes the tile's words of eight chunks at a time as one contiguous run (a row's own words lie 128 bytes
+// apart there).  Slice weights and shifts come out of the same launch.
+// 16384 x 4096 float32: 345 us in five launches (two passes over the rows in 64-bit integers, planes, tiled planes,
+// image, weights), 95 us: 370 MB at 3.9 TB/s.
+constexpr int kKeyRows = 16, kKeyGroup = 8;
+template <typename T, bool kVec, int kHeld>
+__global__ __launch_bounds__(kKeyRows * BSI_WAVE) void build_keys_fast_kernel(
+    const T* __restrict__ x, int64_t R, int64_t d, int chunks, int slices, double dec_scale, float scale,
+    unsigned long long* __restrict__ tiled, int8_t* __restrict__ image8, int* __restrict__ shifts, float* __restrict__ weights) {
+    // [chunk][slice][word of the chunk][row], rows padded to 17 so that the half-words of a wave spread over the banks
+    constexpr int kWordStride = 17, kSliceStride = 4 * kWordStride, kChunkStride = 8 * kSliceStride;
+    __shared__ unsigned long long stage[kKeyGroup * kChunkStride];
+    const int lane = threadIdx.x & (BSI_WAVE - 1);
+    const int rr = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int64_t row = static_cast<int64_t>(blockIdx.x) * kKeyRows + rr;
+    const bool have = row < R;
+    const T* xrow = x + (have ? row : R - 1) * d;
+    const ChunkLane cl = chunk_lane(lane);
+    uint32_t held[kHeld][2];
+    unsigned mx = 0u;
+#pragma unroll
+    for (int c = 0; c < kHeld; ++c) {
+        float v[4];
+        load_chunk_quad<T, kVec>(xrow, d, c, cl, v);  // past the row: zeros
+        const unsigned m = quad_max_bits(v);
+        mx = m > mx ? m : mx;
+        uint32_t b[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+            b[k] = __float_as_uint(copysignf(scaled_magnitude_f32<T>(fabsf(v[k]), scale), v[k]) + 12582912.0f);
+        held[c][0] = __builtin_amdgcn_perm(b[1], b[0], 0x05040100u);
+        held[c][1] = __builtin_amdgcn_perm(b[3], b[2], 0x05040100u);
+    }
+    for (int c = kHeld; c < chunks; ++c) {
+        float v[4];
+        load_chunk_quad<T, kVec>(xrow, d, c, cl, v);
+        const unsigned m = quad_max_bits(v);
+        mx = m > mx ? m : mx;
+    }
+    mx = wave_max_u32(mx);
+    constexpr unsigned kHeldLimit = 0x43800000u;  // 256.0f: 127 times that fits a signed 16-bit magnitude
+    const bool wide = mx >= kQuantWideBits;
+    int shift = quant_shift(mx, scale, slices);
+    if (wide) {
+        unsigned long long m64 = 0ULL;
+        for (int c = 0; c < chunks; ++c) {
+            float v[4];
+            load_chunk_quad<T, kVec>(xrow, d, c, cl, v);
+            const unsigned long long m = quad_max_wide(v, dec_scale);
+            m64 = m > m64 ? m : m64;
+        }
+        shift = compute_shift(wave_max_u64(m64), 0.0, 1, slices, 0.0f);
+    }
+    if (have && lane < slices) {
+        const float w = static_cast<float>(1ULL << shift) * static_cast<float>(1 << lane);
+        weights[row * slices + lane] = lane == slices - 1 ? -w : w;
+        if (lane == 0) shifts[row] = shift;
+    }
+    const QuantRange range = quant_range(slices);
+    const float inv = __uint_as_float(static_cast<uint32_t>(127 - shift) << 23);
+    const int words_per_group = slices * 64;  // words of a chunk of the tile
+    for (int c0 = 0; c0 < chunks; c0 += kKeyGroup) {
+        const int n = chunks - c0 < kKeyGroup ? chunks - c0 : kKeyGroup;
+#pragma unroll
+        for (int u = 0; u < kKeyGroup; ++u) {
+            const int c = c0 + u;
+            if (u < n) {
+                uint32_t bytes;
+                if (c0 < kHeld && mx < kHeldLimit) {
+                    const uint32_t lo = c0 == 0 ? held[u][0] : held[(kKeyGroup + u) % kHeld][0];
+                    const uint32_t hi = c0 == 0 ? held[u][1] : held[(kKeyGroup + u) % kHeld][1];
+                    uint32_t b[4];
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) {
+                        const uint32_t pair = k < 2 ? lo : hi;
+                        const float t = static_cast<float>(static_cast<int>(static_cast<int16_t>(pair >> (16 * (k & 1)))));
+                        const float q = truncf(fmaf(fabsf(t), inv, 0.5f));
+                        const float s = __builtin_amdgcn_fmed3f(copysignf(q, t), range.lo, range.hi);
+                        b[k] = __float_as_uint(fmaf(s, range.up, 12582912.0f));
+                    }
+                    bytes = pack_low_bytes(b[0], b[1], b[2], b[3]);
+                } else {
+                    float v[4];
+                    load_chunk_quad<T, kVec>(xrow, d, c, cl, v);
+                    bytes = wide ? quantise_quad_wide(v, dec_scale, shift, slices) : quantise_quad<T>(v, scale, shift, range);
+                }
+                const uint32_t image = chunk_image_dword(bytes, cl);
+                if (have) reinterpret_cast<uint32_t*>(image8)[(static_cast<size_t>(row) * chunks + c) * (BSI_CHUNK_ELEMS / 4) + lane] = image;
+                const int sl = (lane & 7) - (8 - slices), unit = lane >> 3;
+                const uint32_t plane = chunk_plane_dword(image, cl);
+                if (sl >= 0)
+                    reinterpret_cast<uint32_t*>(stage)[(u * kChunkStride + sl * kSliceStride + (unit >> 1) * kWordStride + rr) * 2 + (unit & 1)] =
+                        have ? plane : 0u;
+            }
+        }
+        __syncthreads();
+        unsigned long long* dst = tiled + (static_cast<size_t>(blockIdx.x) * chunks + c0) * words_per_group;
+        for (int o = threadIdx.x; o < n * words_per_group; o += kKeyRows * BSI_WAVE) {
+            const int u = o / words_per_group, w = o - u * words_per_group;  // w = slice * 64 + word * 16 + row
+            dst[o] = stage[u * kChunkStride + (w >> 6) * kSliceStride + ((w >> 4) & 3) * kWordStride + (w & 15)];
+        }
+        __syncthreads();
     }
 }
 
@@ -726,6 +816,14 @@ extern "C" int bsi_hip_decimal_stats(const int64_t* ints, int64_t Q, int64_t d, 
 
 std::atomic<int> bsi::g_build_items{0};
 
+// Whether rows of d elements at x can be loaded a quad at a time.
+static bool quads_aligned(const void* x, int dtype, int64_t d) {
+    return d % 4 == 0 && (reinterpret_cast<uintptr_t>(x) & (dtype == BSI_DTYPE_F32 ? 15 : 7)) == 0;
+}
+#define BSI_DISPATCH_BOOL(cond, name, ...)                        \
+    if (cond) { constexpr bool name = true; __VA_ARGS__; }        \
+    else { constexpr bool name = false; __VA_ARGS__; }
+
 extern "C" int bsi_hip_build_fixed(const void* x, int dtype, int64_t Q, int64_t d, int decimal_places, int fixed_bits,
                                    int chunk_scale, float clip_k, uint64_t* words, int32_t* shifts, float* scales,
                                    int8_t* ints8, void* stream) {
@@ -733,46 +831,73 @@ extern "C" int bsi_hip_build_fixed(const void* x, int dtype, int64_t Q, int64_t 
     BSI_REQUIRE(fixed_bits >= 2 && fixed_bits <= 63, "fixed_bits must be in [2, 63]");
     BSI_REQUIRE(ints8 == nullptr || fixed_bits <= 8, "int8 output needs fixed_bits <= 8");
     if (Q == 0 || d == 0) return BSI_OK;
-    BSI_REQUIRE(x && words && shifts && scales, "null pointer");
     const int W = static_cast<int>((d + 63) / 64);
     const int chunks = static_cast<int>((d + 255) / 256);
     const double dec_scale = pow(10.0, static_cast<double>(decimal_places));
-    if (chunk_scale && fixed_bits <= 8 && !(clip_k > 0.0f) && W % 4 == 0) {
-        const int64_t items = Q * chunks;
-#define BSI_LAUNCH_FAST(N)                                                                                          \
-    {                                                                                                               \
-        const int64_t waves = (items + (N) - 1) / (N);                                                              \
-        BSI_DISPATCH_DTYPE(dtype, hipLaunchKernelGGL((build_fixed_chunk_fast_kernel<T, N>), dim3(grid_for(waves)),   \
-                                                     dim3(kBlock), 0, as_stream(stream), static_cast<const T*>(x), Q, \
-                                                     d, chunks, fixed_bits, W, dec_scale,                            \
-                                                     integer_decimal_scale(dec_scale),                               \
-                                                     reinterpret_cast<unsigned long long*>(words), shifts, scales,   \
-                                                     ints8));                                                        \
-    }
-        // a wave gets more items only once there are about 8 waves per SIMD (8192 in all); measured on
-        // 4096 ... 131072 items, every other choice is within a few percent or slower
+    const unsigned scale_int = integer_decimal_scale(dec_scale);
+    const int64_t items = Q * chunks;
+    // The register-resident kernels quantise in float32: 10^dec an integer of at most 127 (0 to 2 decimal places), at most
+    // 8 slices, no clipping; their item numbers are 32-bit.
+    const bool fast = scale_int != 0 && fixed_bits <= 8 && !(clip_k > 0.0f) && items <= 0x7fffff00LL && Q <= 0x7fffffffLL;
+    BSI_REQUIRE(x && shifts && scales && (words || (fast && ints8)), "null pointer");
+    const float scale = static_cast<float>(scale_int);
+    unsigned long long* const words64 = reinterpret_cast<unsigned long long*>(words);
+    hipStream_t st = as_stream(stream);
+    if (fast && chunk_scale && W % 4 == 0) {
+#define BSI_LAUNCH_FAST(N)                                                                                                 \
+    BSI_DISPATCH_DTYPE(dtype, BSI_DISPATCH_BOOL(quads_aligned(x, dtype, d), kVec, BSI_DISPATCH_BOOL(words != nullptr, kPlanes, \
+        hipLaunchKernelGGL((build_fixed_chunk_fast_kernel<T, N, kVec, kPlanes>), dim3(grid_for((items + (N) - 1) / (N))),  \
+                           dim3(kBlock), 0, st, static_cast<const T*>(x), static_cast<unsigned>(items), d,                 \
+                           static_cast<unsigned>(chunks), fixed_bits, W, dec_scale, scale, words64, shifts, scales, ints8))))
+        // Several items a wave share its prologue and put their loads in flight together: worth it once every SIMD has its
+        // eight waves without (16384 items: 6.5 us with one each, 6.0 with two, 6.3 with four; 65536: 18.1, 15.6, 15.4).
         int per_wave = g_build_items.load(std::memory_order_relaxed);
-        if (per_wave == 0) per_wave = items > 8 * 16384 ? 8 : (items >= 16384 ? 4 : (items >= 8192 ? 2 : 1));
-        if (per_wave == 8) BSI_LAUNCH_FAST(8)
-        else if (per_wave == 4) BSI_LAUNCH_FAST(4)
-        else if (per_wave == 2) BSI_LAUNCH_FAST(2)
-        else BSI_LAUNCH_FAST(1)
+        if (per_wave == 0) per_wave = items >= 32768 ? 4 : (items >= 16384 ? 2 : 1);
+        if (per_wave == 8) { BSI_LAUNCH_FAST(8); }
+        else if (per_wave == 4) { BSI_LAUNCH_FAST(4); }
+        else if (per_wave == 2) { BSI_LAUNCH_FAST(2); }
+        else { BSI_LAUNCH_FAST(1); }
 #undef BSI_LAUNCH_FAST
         BSI_LAUNCH_CHECK("build_fixed_chunk_fast_kernel");
+    } else if (fast && !chunk_scale) {
+        BSI_DISPATCH_DTYPE(dtype, BSI_DISPATCH_BOOL(quads_aligned(x, dtype, d), kVec, BSI_DISPATCH_BOOL(words != nullptr, kPlanes,
+            hipLaunchKernelGGL((build_fixed_row_fast_kernel<T, kVec, kPlanes>), dim3(static_cast<unsigned>(Q)), dim3(kBlock), 0, st,
+                               static_cast<const T*>(x), d, chunks, fixed_bits, W, dec_scale, scale, words64, shifts, scales,
+                               ints8))))
+        BSI_LAUNCH_CHECK("build_fixed_row_fast_kernel");
     } else if (chunk_scale) {
-        BSI_DISPATCH_DTYPE(dtype, hipLaunchKernelGGL(build_fixed_chunk_kernel<T>, dim3(grid_for(Q * chunks)),
-                                                     dim3(kBlock), 0, as_stream(stream), static_cast<const T*>(x), Q,
-                                                     d, chunks, fixed_bits, W, dec_scale, clip_k,
-                                                     reinterpret_cast<unsigned long long*>(words), shifts, scales,
-                                                     ints8));
+        BSI_REQUIRE(words != nullptr, "null pointer");
+        BSI_DISPATCH_DTYPE(dtype, hipLaunchKernelGGL(build_fixed_chunk_kernel<T>, dim3(grid_for(items)), dim3(kBlock), 0, st,
+                                                     static_cast<const T*>(x), Q, d, chunks, fixed_bits, W, dec_scale, clip_k,
+                                                     words64, shifts, scales, ints8));
         BSI_LAUNCH_CHECK("build_fixed_chunk_kernel");
     } else {
-        BSI_DISPATCH_DTYPE(dtype, hipLaunchKernelGGL(build_fixed_row_kernel<T>, dim3(static_cast<unsigned>(Q)),
-                                                     dim3(kBlock), 0, as_stream(stream), static_cast<const T*>(x), Q,
-                                                     d, fixed_bits, W, dec_scale, clip_k,
-                                                     reinterpret_cast<unsigned long long*>(words), shifts, scales,
-                                                     ints8));
+        BSI_DISPATCH_DTYPE(dtype, hipLaunchKernelGGL(build_fixed_row_kernel<T>, dim3(static_cast<unsigned>(Q)), dim3(kBlock), 0,
+                                                     st, static_cast<const T*>(x), Q, d, fixed_bits, W, dec_scale, clip_k,
+                                                     words64, shifts, scales, ints8));
         BSI_LAUNCH_CHECK("build_fixed_row_kernel");
     }
+    return BSI_OK;
+}
+
+extern "C" int bsi_hip_build_fixed_keys(const void* x, int dtype, int64_t R, int64_t d, int decimal_places, int fixed_bits,
+                                        uint64_t* tiled, int8_t* image, int32_t* shifts, float* slice_weights, void* stream) {
+    BSI_REQUIRE(R >= 0 && d >= 1, "bad shape");
+    const unsigned scale_int = integer_decimal_scale(pow(10.0, static_cast<double>(decimal_places)));
+    if (scale_int == 0 || fixed_bits < 2 || fixed_bits > 8)
+        return fail(BSI_ERR_UNSUPPORTED, "the one-launch key build takes 2 to 8 bits and 0 to 2 decimal places (got %d and %d)",
+                    fixed_bits, decimal_places);
+    if (R == 0) return BSI_OK;
+    BSI_REQUIRE(x && tiled && image && shifts && slice_weights, "null pointer");
+    BSI_REQUIRE((R + kKeyRows - 1) / kKeyRows <= 0x7fffffffLL, "too many rows for one launch");
+    const int chunks = static_cast<int>((d + 255) / 256);
+    // Chunks kept in registers: 16 for rows of 9 to 16 chunks, which then need no second read of any of them (4096 x 4096:
+    // 22.8 us against 29.5), 8 otherwise: two workgroups a CU instead of one (8192 x 2048: 19.5 us against 27.1).
+    BSI_DISPATCH_DTYPE(dtype, BSI_DISPATCH_BOOL(quads_aligned(x, dtype, d), kVec, BSI_DISPATCH_BOOL(chunks > 8 && chunks <= 16, kLong,
+        hipLaunchKernelGGL((build_keys_fast_kernel<T, kVec, kLong ? 16 : 8>), dim3(static_cast<unsigned>((R + kKeyRows - 1) / kKeyRows)),
+                           dim3(kKeyRows * BSI_WAVE), 0, as_stream(stream), static_cast<const T*>(x), R, d, chunks, fixed_bits,
+                           static_cast<double>(scale_int), static_cast<float>(scale_int),
+                           reinterpret_cast<unsigned long long*>(tiled), image, shifts, slice_weights))))
+    BSI_LAUNCH_CHECK("build_keys_fast_kernel");
     return BSI_OK;
 }

@@ -1,8 +1,8 @@
 // The dot for a few query rows (decode steps): kernels that stream the packed key planes once -- on a built int8
 // query image, with the query build inside, or with queries handed over as EWAH streams -- and the stream -> int8
 // image pass for larger batches of EWAH queries.
-#include "bsi_dot_device.h"
 #include "bsi_dot_internal.h"
+#include "bsi_quant_device.h"
 
 namespace bsi {
 
@@ -151,95 +151,9 @@ __global__ __launch_bounds__(1024) void dot_mfma_stream_kernel(
 constexpr int kFusedMaxQ = 4;
 constexpr size_t kFusedQueryLdsBytes = 96 * 1024;  // int8 image + chunk scales of all rows: chunks * Q * 260 bytes
 
-// Element i of a buffer of T as float; 0 past the descriptor's range.
-template <typename T>
-__device__ __forceinline__ float buffer_load_as_float(bsi_rsrc r, int i);
-template <>
-__device__ __forceinline__ float buffer_load_as_float<float>(bsi_rsrc r, int i) {
-    return __int_as_float(__builtin_amdgcn_raw_buffer_load_b32(r, i * 4, 0, 0));
-}
-template <>
-__device__ __forceinline__ float buffer_load_as_float<__half>(bsi_rsrc r, int i) {
-    const unsigned short h = static_cast<unsigned short>(__builtin_amdgcn_raw_buffer_load_b16(r, i * 2, 0, 0));
-    return __half2float(__ushort_as_half(h));
-}
-template <>
-__device__ __forceinline__ float buffer_load_as_float<__hip_bfloat16>(bsi_rsrc r, int i) {
-    const unsigned short h = static_cast<unsigned short>(__builtin_amdgcn_raw_buffer_load_b16(r, i * 2, 0, 0));
-    return __uint_as_float(static_cast<uint32_t>(h) << 16);
-}
-
-// One (chunk, row) item: the wave's 256 activations xv[k] = element k * 64 + lane (0 past the row's end) become 256
-// image bytes at img and one scale.  scale_int is 10^dec when that is at most 127 (else 0: float64 arithmetic).
-// Magnitudes below 2^31 (all but pathological inputs) go through 32-bit integer arithmetic; an item with a larger
-// one is left untouched and reported (true, for the whole wave) for fused_quantize_item_wide -- the same two routes,
-// with the same results, as the builder's fast kernel.
-__device__ __forceinline__ bool fused_quantize_item(const float (&xv)[4], double dec_scale, unsigned scale_int, int slices,
-                                                    int valid, int lane, unsigned char* img, float* scale_out) {
-    unsigned mag[4];
-    bool big = false;
-    if (scale_int != 0u) {
-#pragma unroll
-        for (int k = 0; k < 4; ++k) mag[k] = scaled_magnitude_u32(xv[k], scale_int, big);
-    } else {
-#pragma unroll
-        for (int k = 0; k < 4; ++k) {
-            const double xs = __dmul_rn(static_cast<double>(xv[k]), dec_scale);
-            const bool b = !(fabs(xs) < 2147483000.0);
-            big = big || b;
-            mag[k] = b ? 0u : static_cast<unsigned>(static_cast<int>(floor(__dadd_rn(fabs(xs), 0.5))));
-        }
-    }
-    if (__any(big)) return true;
-    unsigned mx = 0u;
-#pragma unroll
-    for (int k = 0; k < 4; ++k) mx = mag[k] > mx ? mag[k] : mx;
-    mx = wave_max_u32(mx);
-    // compute_shift without clipping: the bits of the largest magnitude beyond the slices' magnitude bits
-    int shift = (32 - __clz(static_cast<int>(mx))) - (slices - 1);  // mx < 2^31; __clz(0) = 32
-    shift = (shift < 0 || valid <= 0) ? 0 : shift;
-    if (lane == 0) *scale_out = static_cast<float>(1ULL << shift);
-    const unsigned round_add = (shift > 0) ? (1u << (shift - 1)) : 0u;
-    const int qmax32 = (1 << (slices - 1)) - 1, qmin32 = -(1 << (slices - 1));
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-        const int qa = static_cast<int>((mag[k] + round_add) >> shift);
-        int v = (xv[k] < 0.0f) ? -qa : qa;
-        v = v < qmin32 ? qmin32 : (v > qmax32 ? qmax32 : v);
-        img[mfma_byte_pos(k * BSI_WAVE + lane)] = static_cast<unsigned char>(v << (8 - slices));
-    }
-    return false;
-}
-
-// The rare item (a magnitude of 2^31 or more, an infinity, a NaN): the builder's 64-bit routine, reading the chunk
-// from memory (xsrc = its first element) in rolled loops, so that it costs the kernel no registers.
-template <typename T>
-__device__ __forceinline__ void fused_quantize_item_wide(const T* xsrc, double dec_scale, int slices, int valid, int lane,
-                                                         unsigned char* img, float* scale_out) {
-    const long long qmax = (1LL << (slices - 1)) - 1LL, qmin = -(1LL << (slices - 1));
-    unsigned long long mx = 0ULL;
-#pragma unroll 1
-    for (int k = 0; k < 4; ++k) {
-        const int e = k * BSI_WAVE + lane;
-        if (e < valid) {
-            const unsigned long long av = uabs_ll(round_scaled(load_as_float<T>(xsrc, e), dec_scale));
-            if (av > mx) mx = av;
-        }
-    }
-    mx = wave_max_u64(mx);
-    const int shift = (valid > 0) ? compute_shift(mx, 0.0, valid, slices, 0.0f) : 0;
-    if (lane == 0) *scale_out = static_cast<float>(1ULL << shift);
-#pragma unroll 1
-    for (int k = 0; k < 4; ++k) {
-        const int e = k * BSI_WAVE + lane;
-        const long long v = (e < valid) ? shift_clamp(round_scaled(load_as_float<T>(xsrc, e), dec_scale), shift, qmin, qmax) : 0;
-        img[mfma_byte_pos(e)] = static_cast<unsigned char>(static_cast<int>(v) << (8 - slices));
-    }
-}
-
-template <typename T, int KT, int NI>
+template <typename T, int KT, int NI, bool kVec>
 __global__ __launch_bounds__(1024) void dot_mfma_stream_fused_kernel(
-    const T* __restrict__ x, int64_t d, double dec_scale, unsigned scale_int, int slices,
+    const T* __restrict__ x, int64_t d, double dec_scale, int narrow, int slices,
     const unsigned long long* __restrict__ B64,  // tiled key planes, Sb = 6
     const float* __restrict__ Bw, int chunks, int pass_chunks, int64_t R, int Q, float scale_inv, int64_t R_total,
     float* __restrict__ out, const float* __restrict__ bias) {
@@ -279,26 +193,27 @@ __global__ __launch_bounds__(1024) void dot_mfma_stream_fused_kernel(
     const int items = chunks * Q;
     // Buffer loads, one descriptor per row: past the row's end they return 0 without a branch (with loads in
     // conditional blocks the compiler waits for every outstanding load, the key planes included, before a use).
+    const ChunkLane cl = chunk_lane(lane);
+    const QuantRange range = quant_range(slices);
+    const float scale = static_cast<float>(dec_scale);
     auto load_item = [&](int item, float (&dst)[4]) {
         const int ic = item / Q, iq = item - ic * Q;
-        const bsi_rsrc row = make_rsrc(x + static_cast<int64_t>(iq) * d, static_cast<size_t>(d) * sizeof(T));
-        const int e0 = ic * BSI_CHUNK_ELEMS + lane;
-#pragma unroll
-        for (int k = 0; k < 4; ++k) dst[k] = buffer_load_as_float<T>(row, e0 + k * BSI_WAVE);
+        load_chunk_quad<T, kVec>(x + static_cast<int64_t>(iq) * d, d, ic, cl, dst);
     };
-    auto quantize = [&](int item, const float (&xv)[4]) -> bool {
-        const int ic = item / Q;
-        const int64_t left = d - static_cast<int64_t>(ic) * BSI_CHUNK_ELEMS;
-        const int valid = static_cast<int>(left < BSI_CHUNK_ELEMS ? left : BSI_CHUNK_ELEMS);
-        return fused_quantize_item(xv, dec_scale, scale_int, slices, valid, lane, qimg + static_cast<size_t>(item) * 256,
-                                   qsc + item);
-    };
-    auto quantize_wide = [&](int item) {
-        const int ic = item / Q, iq = item - ic * Q;
-        const int64_t s0 = static_cast<int64_t>(ic) * BSI_CHUNK_ELEMS, left = d - s0;
-        const int valid = static_cast<int>(left < BSI_CHUNK_ELEMS ? left : BSI_CHUNK_ELEMS);
-        fused_quantize_item_wide<T>(x + static_cast<int64_t>(iq) * d + s0, dec_scale, slices, valid, lane,
-                                    qimg + static_cast<size_t>(item) * 256, qsc + item);
+    // One item: 256 image bytes and one scale into LDS.  narrow: 10^dec is an integer of at most 127 (quantise_quad's range).
+    auto quantize = [&](int item, const float (&xv)[4]) {
+        const unsigned mx = wave_max_u32(quad_max_bits(xv));
+        int shift;
+        uint32_t bytes;
+        if (narrow && mx < kQuantWideBits) {
+            shift = quant_shift(mx, scale, slices);
+            bytes = quantise_quad<T>(xv, scale, shift, range);
+        } else {
+            shift = compute_shift(wave_max_u64(quad_max_wide(xv, dec_scale)), 0.0, 1, slices, 0.0f);
+            bytes = quantise_quad_wide(xv, dec_scale, shift, slices);
+        }
+        reinterpret_cast<uint32_t*>(qimg)[item * 64 + lane] = chunk_image_dword(bytes, cl);
+        if (lane == 0) qsc[item] = static_cast<float>(1ULL << shift);
     };
     float xr[kFusedItems][4];
 #pragma unroll
@@ -323,14 +238,12 @@ __global__ __launch_bounds__(1024) void dot_mfma_stream_fused_kernel(
     const EpilogueOperands eo = load_epilogue_operands(Bw, bias, R, cvalid, cr);
     __builtin_amdgcn_sched_barrier(0);
     {
-        unsigned wide = 0u;  // items left to the 64-bit routine
 #pragma unroll
         for (int i = 0; i < kFusedItems; ++i) {
             // no branch here either (the compiler would sink the item's loads into it, behind the key loads): a wave
             // with fewer items repeats the last one, and writes the bytes its owner writes
             const int item = wave + i * nwaves;
-            const bool w = quantize(item < items ? item : items - 1, xr[i]);
-            wide |= (w && item < items) ? 1u << i : 0u;
+            quantize(item < items ? item : items - 1, xr[i]);
             __builtin_amdgcn_sched_barrier(0);  // one item at a time: interleaving them costs registers, gains nothing
         }
         // longer rows: the rest one item at a time (each waits for its own loads)
@@ -338,21 +251,7 @@ __global__ __launch_bounds__(1024) void dot_mfma_stream_fused_kernel(
         for (int item = wave + kFusedItems * nwaves; item < items; item += nwaves) {
             float xa[4];
             load_item(item, xa);
-            if (quantize(item, xa)) wide |= 1u << 31;
-        }
-#pragma unroll 1
-        for (int i = 0; wide != 0u && i < kFusedItems; ++i)
-            if (wide & (1u << i)) quantize_wide(wave + i * nwaves);
-        if (wide >> 31) {  // some item past the first ones: find it again (rare twice over)
-#pragma unroll 1
-            for (int item = wave + kFusedItems * nwaves; item < items; item += nwaves) {
-                float xa[4];
-                load_item(item, xa);
-                bool big = false;
-#pragma unroll
-                for (int k = 0; k < 4; ++k) big = big || !(fabs(__dmul_rn(static_cast<double>(xa[k]), dec_scale)) < 2147483000.0);
-                if (__any(big)) quantize_wide(item);
-            }
+            quantize(item, xa);
         }
         __syncthreads();
     }
@@ -667,7 +566,7 @@ static FusedPlan fused_plan(int64_t Q, int chunks, int64_t R) {
     return p;
 }
 
-template <typename T, int KT, int NI>
+template <typename T, int KT, int NI, bool kVec>
 static void launch_stream_fused(const FusedPlan& plan, const T* x, int64_t d, double dec_scale, int slices, const uint64_t* B,
                                 const float* Bw, int chunks, int64_t R, int Q, float scale_inv, int64_t R_total, float* out,
                                 const float* bias, hipStream_t st) {
@@ -680,10 +579,10 @@ static void launch_stream_fused(const FusedPlan& plan, const T* x, int64_t d, do
     if (pass_chunks > chunks) pass_chunks = chunks;
     const size_t lds = static_cast<size_t>(pass_chunks) * kSlot * sizeof(int) + query_bytes;
     static LdsOptIn once0;
-    lds_opt_in(once0, reinterpret_cast<const void*>(&dot_mfma_stream_fused_kernel<T, KT, NI>), 160 * 1024);
-    const unsigned scale_int = integer_decimal_scale(dec_scale);
-    hipLaunchKernelGGL((dot_mfma_stream_fused_kernel<T, KT, NI>), dim3(plan.grid), dim3(plan.waves * 64), lds, st, x, d,
-                       dec_scale, scale_int, slices, reinterpret_cast<const unsigned long long*>(B), Bw, chunks, pass_chunks,
+    lds_opt_in(once0, reinterpret_cast<const void*>(&dot_mfma_stream_fused_kernel<T, KT, NI, kVec>), 160 * 1024);
+    const int narrow = integer_decimal_scale(dec_scale) != 0 ? 1 : 0;
+    hipLaunchKernelGGL((dot_mfma_stream_fused_kernel<T, KT, NI, kVec>), dim3(plan.grid), dim3(plan.waves * 64), lds, st, x, d,
+                       dec_scale, narrow, slices, reinterpret_cast<const unsigned long long*>(B), Bw, chunks, pass_chunks,
                        R, Q, scale_inv, R_total, out, bias);
 }
 
@@ -692,15 +591,20 @@ static void launch_stream_fused_t(const T* x, int64_t d, double dec_scale, int s
                                   int chunks, int64_t R, int Q, float scale_inv, int64_t R_total, float* out,
                                   const float* bias, hipStream_t st) {
     const FusedPlan p = fused_plan(Q, chunks, R);
-#define BSI_FUSED_GO(KT, NI) \
-    launch_stream_fused<T, KT, NI>(p, x, d, dec_scale, slices, B, Bw, chunks, R, Q, scale_inv, R_total, out, bias, st)
+    // a lane's four consecutive activations in one load where every row allows it
+    const bool vec = d % 4 == 0 && reinterpret_cast<uintptr_t>(x) % (4 * sizeof(T)) == 0;
+#define BSI_FUSED_GO(KT, NI)                                                                                              \
+    {                                                                                                                     \
+        if (vec) launch_stream_fused<T, KT, NI, true>(p, x, d, dec_scale, slices, B, Bw, chunks, R, Q, scale_inv, R_total, out, bias, st); \
+        else launch_stream_fused<T, KT, NI, false>(p, x, d, dec_scale, slices, B, Bw, chunks, R, Q, scale_inv, R_total, out, bias, st);    \
+    }
     if (p.key_tiles == 2) {
-        if (p.upfront == 1) BSI_FUSED_GO(2, 1);
-        else BSI_FUSED_GO(2, 2);
+        if (p.upfront == 1) BSI_FUSED_GO(2, 1)
+        else BSI_FUSED_GO(2, 2)
     } else {
-        if (p.upfront == 1) BSI_FUSED_GO(1, 1);
-        else if (p.upfront == 2) BSI_FUSED_GO(1, 2);
-        else BSI_FUSED_GO(1, 4);
+        if (p.upfront == 1) BSI_FUSED_GO(1, 1)
+        else if (p.upfront == 2) BSI_FUSED_GO(1, 2)
+        else BSI_FUSED_GO(1, 4)
     }
 #undef BSI_FUSED_GO
 }

@@ -127,12 +127,23 @@ int bsi_hip_pack_bits_batch(const int64_t* ints_device, int64_t Q, int64_t d, in
  * (one fused kernel when chunk_scale != 0).  chunk_scale != 0 gives shifts/scales [Q, ceil(d/256)],
  * else [Q].  Optional extra output `ints8_device` (may be NULL): the quantised values as int8
  * [Q, chunks*256] in the MFMA core's in-chunk element order (bsi_hip_planes_to_int8 gives the same).
+ * words_device may be NULL when ints8_device is given, fixed_bits <= 8, clip_k <= 0 and decimal_places is 0, 1 or 2: the
+ * planes are then not written.
  * Replaces the host orchestration bsi_cuda_build_fixed_query_words_fused
  * (bsi_vector_cuda.cpp:401-557) and, with chunk_scale = 0 and fixed_bits = 6, the key quantiser
  * + packer (bsi_vector_cuda.cpp:559-744, 1125-1141). */
 int bsi_hip_build_fixed(const void* x_device, int dtype, int64_t Q, int64_t d, int decimal_places, int fixed_bits,
                         int chunk_scale, float clip_k, uint64_t* words_device, int32_t* shifts_device,
                         float* scales_device, int8_t* ints8_device, void* stream);
+
+/* The fixed-bit build of a key matrix [R, d] in one launch, straight into what the dot reads: tiled16 planes
+ * (bsi_hip_tile_key_planes' layout, [ceil(R/16), chunks, fixed_bits, 64] words), the row-major int8 image [R, chunks*256]
+ * (bsi_hip_planes_to_int8's), one shift per row and the slice weights [R, fixed_bits] = +-2^(slice + shift).  2 to 8 bits,
+ * decimal_places 0, 1 or 2, no clipping; anything else is refused (BSI_ERR_UNSUPPORTED).  Replaces the same reference code
+ * as bsi_hip_build_fixed with chunk_scale = 0. */
+int bsi_hip_build_fixed_keys(const void* x_device, int dtype, int64_t R, int64_t d, int decimal_places, int fixed_bits,
+                             uint64_t* tiled_device, int8_t* image_device, int32_t* shifts_device,
+                             float* slice_weights_device, void* stream);
 
 /* ---------------------------------------------------------------- EWAH */
 
