@@ -1168,10 +1168,12 @@ def linear_few_rows_is_free(x2d: torch.Tensor, keys: "PrebuiltBSIKeysCUDA") -> b
     return bool(lib.bsi_hip_linear_few_rows_upfront(int(x2d.shape[0]), int(x2d.shape[1]), int(keys.num_keys)))
 
 
-def linear_few_rows_cuda(x2d: torch.Tensor, keyset_cuda_cap, decimal_places: int, bias=None, _checked: bool = False) -> torch.Tensor:
-    """out[Q, R] float32 = BSI dot of the rows of ``x2d`` (Q <= 4) with the keyset, query build included, in one
-    launch (bsi_hip_linear_few_rows): what build_bsi_queries_cuda_batch_packed followed by
-    batch_dot_product_multiquery_cuda_batch_caps returns, bit for bit.  Not in the reference."""
+def linear_few_rows_cuda(x2d: torch.Tensor, keyset_cuda_cap, decimal_places: int, bias=None, _checked: bool = False,
+                         out_dtype: torch.dtype = torch.float32) -> torch.Tensor:
+    """out[Q, R] = BSI dot of the rows of ``x2d`` (Q <= 4) with the keyset, query build included, in one
+    launch (bsi_hip_linear_few_rows_out): what build_bsi_queries_cuda_batch_packed followed by
+    batch_dot_product_multiquery_cuda_batch_caps returns, bit for bit; in half precision, that cast to ``out_dtype`` plus
+    the bias cast to it.  Not in the reference."""
     keys = _capsule(keyset_cuda_cap, PrebuiltBSIKeysCUDA, "Invalid CUDA keys capsule")
     if not _checked:  # the layer has asked can_fuse_linear_few_rows already
         _check(x2d.dim() == 2 and can_fuse_linear_few_rows(x2d, keys), "linear_few_rows_cuda: call not served by the fused kernel")
@@ -1179,11 +1181,11 @@ def linear_few_rows_cuda(x2d: torch.Tensor, keyset_cuda_cap, decimal_places: int
            f"Decimal mismatch between queries and keys: q={int(decimal_places)} k={keys.decimals}")
     Q, R = int(x2d.shape[0]), keys.num_keys
     _check_bias(bias, R, x2d.device)
-    out = torch.empty((Q, R), dtype=torch.float32, device=x2d.device)
-    check(lib.bsi_hip_linear_few_rows(x2d.data_ptr(), _dtype_code(x2d), Q, int(x2d.shape[1]), int(decimal_places),
-                                      _flags()["bits_q"], keys.words.data_ptr(), keys.slice_weights.data_ptr(), keys.Sb,
-                                      R, _scale_inv(int(decimal_places), keys.decimals), R, _ptr(bias), out.data_ptr(),
-                                      _stream()), "bsi_hip_linear_few_rows")
+    out = torch.empty((Q, R), dtype=out_dtype, device=x2d.device)
+    check(lib.bsi_hip_linear_few_rows_out(x2d.data_ptr(), _dtype_code(x2d), Q, int(x2d.shape[1]), int(decimal_places),
+                                          _flags()["bits_q"], keys.words.data_ptr(), keys.slice_weights.data_ptr(), keys.Sb,
+                                          R, _scale_inv(int(decimal_places), keys.decimals), R, _ptr(bias), out.data_ptr(),
+                                          _dtype_code(out), _stream()), "bsi_hip_linear_few_rows_out")
     return out
 
 
@@ -1193,14 +1195,14 @@ _linear_ws: dict = {}
 
 
 def can_linear_one_call(x2d: torch.Tensor, keys: "PrebuiltBSIKeysCUDA") -> bool:
-    """Whether linear_cuda serves this call: chunk-scaled fixed-bit queries without clipping against fixed-bit keys,
-    the matrix-core route, no per-call profiling."""
+    """Whether linear_cuda serves this call: fixed-bit queries without clipping (chunk scales wherever the width has
+    them) against fixed-bit keys, the matrix-core route, no per-call profiling."""
     f = _flags()
     d = int(x2d.shape[1])
     return (x2d.shape[0] > 0 and x2d.is_cuda and x2d.is_contiguous()
             and x2d.dtype in (torch.float32, torch.float16, torch.bfloat16)
-            and keys.fixed and keys.d == d and 2 <= f["bits_q"] <= 8 and f["chunk_scale"] and f["clip_k"] == 0.0
-            and ((d + 63) // 64) % 4 == 0 and f["core"] != _lib.CORE_VALU and not f["profile"]
+            and d > 0 and keys.fixed and keys.d == d and 2 <= f["bits_q"] <= 8 and f["clip_k"] == 0.0
+            and (f["chunk_scale"] or ((d + 63) // 64) % 4 != 0) and f["core"] != _lib.CORE_VALU and not f["profile"]
             and fast_getenv("BSI_TC_DOT", "1").strip() != "0" and fast_getenv("BSI_LINEAR_ONE_CALL", "1").strip() != "0")
 
 
@@ -1241,9 +1243,18 @@ def reserve_linear_workspace(x2d: torch.Tensor) -> None:
     _reserved_linear_shapes.add(key)
 
 
+def can_output_half(keys: "PrebuiltBSIKeysCUDA", Q: int) -> bool:
+    """Whether the kernel a linear layer of Q rows runs on can write half precision: the int8-image kernel, or the few-rows
+    kernels on 6-plane tiled keys."""
+    if Q > _FEW_ROWS_MAX_Q:
+        return keys.ints8 is not None
+    return keys.Sb == 6 and keys.layout == _lib.LAYOUT_TILED16 and (keys.W + 3) // 4 <= 32768
+
+
 def linear_cuda(x2d: torch.Tensor, keyset_cuda_cap, decimal_places: int, bias=None, warm_keys=None,
-                _checked: bool = False) -> torch.Tensor:
-    """out[Q, R] float32 of a BSI-linear layer in one library call (bsi_hip_linear): the query build into a workspace
+                _checked: bool = False, out_dtype: torch.dtype = torch.float32) -> torch.Tensor:
+    """out[Q, R] of a BSI-linear layer in one library call (bsi_hip_linear_out; float32, or half precision where
+    can_output_half): the query build into a workspace
     kept per device, then the dot, bit for bit what build_bsi_queries_cuda_batch_packed followed by
     batch_dot_product_multiquery_cuda_batch_caps returns.  A call on the very tensor the workspace was last built
     from (same storage, shape, dtype and version: the next layer fed the same activations) skips the build.
@@ -1272,7 +1283,7 @@ def linear_cuda(x2d: torch.Tensor, keyset_cuda_cap, decimal_places: int, bias=No
         if mine is None:  # first eager call on this stream (allocated under it, so freed in its order too)
             mine = ws["eager"][st] = (torch.empty((ws["bytes"],), dtype=torch.uint8, device=x2d.device), [None, None])
         buf, slot = mine
-    key = tensor_build_key(x2d, int(decimal_places))
+    key = tensor_build_key(x2d, int(decimal_places), keys.Sb)
     if capturing and key is not None:
         # a build recorded by one capture is not part of another capture's graph: the capture's identifier is part
         # of what a recorded launch may reuse (a second capture starting on the same static input builds anew)
@@ -1280,17 +1291,17 @@ def linear_cuda(x2d: torch.Tensor, keyset_cuda_cap, decimal_places: int, bias=No
     rebuild = 0 if (key is not None and slot[0] == key) else 1
     slot[0], slot[1] = key, x2d  # holds the input, so that its address is not reused while the build stands for it
     wsptr = buf.data_ptr()
-    out = torch.empty((Q, R), dtype=torch.float32, device=x2d.device)
+    out = torch.empty((Q, R), dtype=out_dtype, device=x2d.device)
     core = f["core"]
     kptr, klayout = key_operand(keys, Q, bits, core)
     if Q >= _SPLIT_MIN_Q:
         _attach_split_scratch_for(x2d.device, Q, R, (d + 63) // 64)
     wptr, wbytes = _warm_region(_capsule(warm_keys, PrebuiltBSIKeysCUDA, "Invalid CUDA keys capsule") if warm_keys is not None
                                 else None, Q, bits, core)
-    check(lib.bsi_hip_linear(x2d.data_ptr(), _dtype_code(x2d), Q, d, int(decimal_places), bits, rebuild, wsptr, ws["bytes"],
+    check(lib.bsi_hip_linear_out(x2d.data_ptr(), _dtype_code(x2d), Q, d, int(decimal_places), bits, rebuild, wsptr, ws["bytes"],
                              kptr, klayout, keys.slice_weights.data_ptr(), keys.Sb, R,
-                             _scale_inv(int(decimal_places), keys.decimals), R, _ptr(bias), out.data_ptr(), core, wptr,
-                             wbytes, st), "bsi_hip_linear")
+                             _scale_inv(int(decimal_places), keys.decimals), R, _ptr(bias), out.data_ptr(), _dtype_code(out), core,
+                                 wptr, wbytes, st), "bsi_hip_linear_out")
     _last_linear_rebuilt[0] = bool(rebuild)
     return out
 

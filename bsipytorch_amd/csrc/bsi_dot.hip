@@ -98,6 +98,10 @@ extern "C" int bsi_hip_dot_split_plan(int64_t R, int64_t Q, int W64, int* tile, 
     return BSI_OK;
 }
 
+// The matrix-core kernels address a tile's operand rows with 32-bit buffer offsets inside a descriptor of at most
+// 2 GiB: 128 rows of chunks * 256 bytes must stay below that.
+constexpr int kMfmaMaxChunks = 32768;
+
 // Validation, kernel selection and launch.  `bias` (optional) is added to every output; *bias_fused tells
 // the caller whether the selected kernel did that in its own epilogue.
 static int dot_launch(const uint64_t* A, const int8_t* A_ints8, const float* A_chunk_scales, int A_scale_stride,
@@ -127,9 +131,6 @@ static int dot_launch(const uint64_t* A, const int8_t* A_ints8, const float* A_c
     BSI_REQUIRE(A || A_ints8, "neither query planes nor int8 queries given");
     hipStream_t st = as_stream(stream);
 
-    // The matrix-core kernels address a tile's operand rows with 32-bit buffer offsets inside a descriptor of at most
-    // 2 GiB: 128 rows of chunks * 256 bytes must stay below that.
-    constexpr int kMfmaMaxChunks = 32768;
     const bool mfma_ok = (Sa >= 2 && Sa <= 8 && Sb >= 2 && Sb <= 8);
     if (core == BSI_CORE_AUTO) core = (mfma_ok && chunks <= kMfmaMaxChunks) ? BSI_CORE_MFMA : BSI_CORE_VALU;
 
@@ -165,6 +166,8 @@ static int dot_launch(const uint64_t* A, const int8_t* A_ints8, const float* A_c
             *bias_fused = true;
             return BSI_OK;
         }
+        if (t_out_dtype != BSI_DTYPE_F32)
+            return fail(BSI_ERR_UNSUPPORTED, "half-precision output: the kernels on key planes for many rows write float32 only");
         const char* kernel = launch_mfma_planes(tiled, A8, A_chunk_scales, A_scale_stride, B, Bw, Sb, W64, chunks, R, Q,
                                                 down_shift, scale_inv, R_total, out, chunk_ints, st);
         BSI_LAUNCH_CHECK(kernel);
@@ -175,6 +178,7 @@ static int dot_launch(const uint64_t* A, const int8_t* A_ints8, const float* A_c
     if (b_layout == BSI_LAYOUT_INT8 || b_layout == BSI_LAYOUT_INT8_TILED)
         return fail(BSI_ERR_UNSUPPORTED, "the popcount core reads key planes, not the int8 image");
     BSI_REQUIRE(A != nullptr, "VALU core needs the query planes");
+    if (t_out_dtype != BSI_DTYPE_F32) return fail(BSI_ERR_UNSUPPORTED, "half-precision output: the popcount core writes float32 only");
     if (Sa == 7 && Sb == 6) {
         launch_valu76(b_layout == BSI_LAYOUT_TILED16, A, A_chunk_scales, A_scale_stride, B, Bw, W64, chunks, R, Q, scale_inv,
                       R_total, out, chunk_ints, st);
@@ -307,12 +311,19 @@ extern "C" int bsi_hip_linear(const void* x, int dtype, int64_t Q, int64_t d, in
                               void* workspace, size_t workspace_bytes, const uint64_t* B, int b_layout, const float* Bw,
                               int Sb, int64_t R, float scale_inv, int64_t R_total, const float* bias, float* out, int core,
                               const void* warm, size_t warm_bytes, void* stream) {
+    return bsi_hip_linear_out(x, dtype, Q, d, decimal_places, fixed_bits, rebuild, workspace, workspace_bytes, B, b_layout, Bw, Sb,
+                              R, scale_inv, R_total, bias, out, BSI_DTYPE_F32, core, warm, warm_bytes, stream);
+}
+
+extern "C" int bsi_hip_linear_out(const void* x, int dtype, int64_t Q, int64_t d, int decimal_places, int fixed_bits, int rebuild,
+                                  void* workspace, size_t workspace_bytes, const uint64_t* B, int b_layout, const float* Bw,
+                                  int Sb, int64_t R, float scale_inv, int64_t R_total, const float* bias, void* out,
+                                  int out_dtype, int core, const void* warm, size_t warm_bytes, void* stream) {
     BSI_REQUIRE(Q >= 0 && R >= 0 && d >= 1, "bad shape");
     BSI_REQUIRE(fixed_bits >= 2 && fixed_bits <= 8, "fixed_bits must be in [2, 8] (got %d)", fixed_bits);
-    const int W64 = static_cast<int>((d + 63) / 64);
-    if (W64 % 4 != 0)
-        return fail(BSI_ERR_UNSUPPORTED, "chunk scales need a multiple of 4 words per slice (d = %lld)", static_cast<long long>(d));
+    BSI_REQUIRE(out_dtype == BSI_DTYPE_F32 || out_dtype == BSI_DTYPE_F16 || out_dtype == BSI_DTYPE_BF16, "unknown dtype code %d", out_dtype);
     if (Q == 0 || R == 0) return BSI_OK;
+    const int W64 = static_cast<int>((d + 63) / 64), chunks = (W64 + 3) / 4;
     const LinearWorkspace w = linear_workspace(Q, d, fixed_bits);
     BSI_REQUIRE(workspace != nullptr && workspace_bytes >= w.total, "workspace of %zu bytes needed, %zu given", w.total,
                 workspace_bytes);
@@ -322,12 +333,22 @@ extern "C" int bsi_hip_linear(const void* x, int dtype, int64_t Q, int64_t d, in
     int32_t* shifts = reinterpret_cast<int32_t*>(ws + w.shifts);
     float* scales = reinterpret_cast<float*>(ws + w.scales);
     int8_t* ints8 = reinterpret_cast<int8_t*>(ws + w.ints8);
+    const int chunk_scale = W64 % 4 == 0 ? 1 : 0;  // the builder's rule: else one scale per row
+    // The matrix-core kernels read the int8 image only: the planes are built for the popcount core (asked for, or what
+    // BSI_CORE_AUTO falls back to for wide keys), and where the builder cannot leave them out.
+    const bool planes = core == BSI_CORE_VALU || Sb < 2 || Sb > 8 || chunks > kMfmaMaxChunks ||
+                        integer_decimal_scale(pow(10.0, static_cast<double>(decimal_places))) == 0;
     if (rebuild) {
-        const int rc = bsi_hip_build_fixed(x, dtype, Q, d, decimal_places, fixed_bits, 1, 0.0f, words, shifts, scales, ints8, stream);
+        const int rc = bsi_hip_build_fixed(x, dtype, Q, d, decimal_places, fixed_bits, chunk_scale, 0.0f, planes ? words : nullptr,
+                                           shifts, scales, ints8, stream);
         if (rc != BSI_OK) return rc;
     }
-    return bsi_hip_dot_bias_warm(words, ints8, scales, W64 / 4, fixed_bits, W64, B, b_layout, Bw, Sb, R, Q, scale_inv, R_total,
-                                 bias, out, core, nullptr, 0, warm, warm_bytes, stream);
+    t_out_dtype = out_dtype;
+    const int rc = bsi_hip_dot_bias_warm(planes ? words : nullptr, ints8, scales, chunk_scale ? chunks : 1, fixed_bits, W64, B, b_layout,
+                                         Bw, Sb, R, Q, scale_inv, R_total, bias, static_cast<float*>(out), core, nullptr, 0, warm,
+                                         warm_bytes, stream);
+    t_out_dtype = BSI_DTYPE_F32;
+    return rc;
 }
 
 extern "C" int bsi_hip_dot_timed(const uint64_t* A, const int8_t* A_ints8, const float* A_chunk_scales,

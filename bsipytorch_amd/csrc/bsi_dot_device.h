@@ -123,6 +123,27 @@ __device__ __forceinline__ EpilogueOperands load_epilogue_operands(const float* 
     return e;
 }
 
+// A linear layer's output in half precision: the fp32 result rounded to the type, then the bias rounded to the type added
+// in float32 and rounded again -- what casting the fp32 scores and adding the cast bias in separate passes gives.
+// dtype: BSI_DTYPE_F16 or BSI_DTYPE_BF16.
+__device__ __forceinline__ uint32_t half_bits(float v, int dtype) {
+    if (dtype == BSI_DTYPE_F16) return __builtin_bit_cast(unsigned short, static_cast<_Float16>(v));
+    return __builtin_bit_cast(unsigned short, static_cast<__bf16>(v));
+}
+__device__ __forceinline__ float half_value(uint32_t bits, int dtype) {
+    if (dtype == BSI_DTYPE_F16) return static_cast<float>(__builtin_bit_cast(_Float16, static_cast<unsigned short>(bits)));
+    return __uint_as_float(bits << 16);
+}
+__device__ __forceinline__ uint32_t half_output(float v, bool has_bias, float bias, int dtype) {
+    const uint32_t h = half_bits(v, dtype);
+    return has_bias ? half_bits(half_value(h, dtype) + half_value(half_bits(bias, dtype), dtype), dtype) : h;
+}
+// Element i of an output of any of the three types.
+__device__ __forceinline__ void store_output(float* out, size_t i, float v, bool has_bias, float bias, int dtype) {
+    if (dtype == BSI_DTYPE_F32) out[i] = has_bias ? v + bias : v;
+    else reinterpret_cast<unsigned short*>(out)[i] = static_cast<unsigned short>(half_output(v, has_bias, bias, dtype));
+}
+
 // The fp32 chain of one output over chunks [c0, c1): accf = fmaf(float(I_c), scale_c * down, accf) in chunk order,
 // eight chunks' integers and scales fetched ahead of their eight dependent steps (fetched one step at a time the
 // chain costs an LDS or cache round trip per chunk: 4 us of a 17 us kernel at 64 chunks).  int_at(c) / scale_at(c)

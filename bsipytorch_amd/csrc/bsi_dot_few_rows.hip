@@ -26,7 +26,7 @@ __global__ __launch_bounds__(1024) void dot_mfma_stream_kernel(
     const int8_t* __restrict__ A8, const float* __restrict__ qscale, int qscale_stride,
     const unsigned long long* __restrict__ B64,  // tiled key planes, Sb = 6
     const float* __restrict__ Bw, int chunks, int pass_chunks, int64_t R, int64_t Q, int down_shift, float scale_inv,
-    int64_t R_total, float* __restrict__ out, int* __restrict__ chunk_ints, const float* __restrict__ bias) {
+    int64_t R_total, float* __restrict__ out, int* __restrict__ chunk_ints, const float* __restrict__ bias, int out_dtype) {
     extern __shared__ __attribute__((aligned(16))) int ints[];  // [pass_chunks][KT][NT][16 queries][16 keys]
     constexpr int kSlot = KT * NT * 256;
 
@@ -133,11 +133,8 @@ __global__ __launch_bounds__(1024) void dot_mfma_stream_kernel(
         }
         if (pend < chunks) __syncthreads();
     }
-    if (cvalid) {
-        float v = (accf * eo.bw) * scale_inv;
-        if (bias != nullptr) v = v + eo.bias;
-        out[static_cast<size_t>(cq) * R_total + cr] = v;
-    }
+    if (cvalid)
+        store_output(out, static_cast<size_t>(cq) * R_total + cr, (accf * eo.bw) * scale_inv, bias != nullptr, eo.bias, out_dtype);
 }
 
 // The few-rows kernel with the query build inside (at most kFusedMaxQ rows: a decode step).  Every workgroup first
@@ -156,7 +153,7 @@ __global__ __launch_bounds__(1024) void dot_mfma_stream_fused_kernel(
     const T* __restrict__ x, int64_t d, double dec_scale, int narrow, int slices,
     const unsigned long long* __restrict__ B64,  // tiled key planes, Sb = 6
     const float* __restrict__ Bw, int chunks, int pass_chunks, int64_t R, int Q, float scale_inv, int64_t R_total,
-    float* __restrict__ out, const float* __restrict__ bias) {
+    float* __restrict__ out, const float* __restrict__ bias, int out_dtype) {
     // [pass_chunks][KT][16 queries][16 keys] ints | [chunks][Q][256] image bytes | [chunks][Q] scales
     extern __shared__ __attribute__((aligned(16))) int ints[];
     constexpr int kSlot = KT * 256;
@@ -312,11 +309,8 @@ __global__ __launch_bounds__(1024) void dot_mfma_stream_fused_kernel(
         }
         if (pend < chunks) __syncthreads();
     }
-    if (cvalid) {
-        float v = (accf * eo.bw) * scale_inv;
-        if (bias != nullptr) v = v + eo.bias;
-        out[static_cast<size_t>(cn) * R_total + cr] = v;
-    }
+    if (cvalid)
+        store_output(out, static_cast<size_t>(cn) * R_total + cr, (accf * eo.bw) * scale_inv, bias != nullptr, eo.bias, out_dtype);
 }
 
 // ------------------------------------------------------------------ EWAH-compressed queries, decode inline
@@ -527,11 +521,11 @@ static void launch_mfma_stream(const int8_t* A8, const float* qscale, int stride
     if (chunk_ints)
         hipLaunchKernelGGL((dot_mfma_stream_kernel<NT, KT, true>), grid, dim3(waves * 64), lds, st, A8, qscale, stride,
                            reinterpret_cast<const unsigned long long*>(B), Bw, chunks, pass_chunks, R, Q, down_shift,
-                           scale_inv, R_total, out, chunk_ints, bias);
+                           scale_inv, R_total, out, chunk_ints, bias, t_out_dtype);
     else
         hipLaunchKernelGGL((dot_mfma_stream_kernel<NT, KT, false>), grid, dim3(waves * 64), lds, st, A8, qscale, stride,
                            reinterpret_cast<const unsigned long long*>(B), Bw, chunks, pass_chunks, R, Q, down_shift,
-                           scale_inv, R_total, out, chunk_ints, bias);
+                           scale_inv, R_total, out, chunk_ints, bias, t_out_dtype);
 }
 
 void launch_mfma_stream_by_shape(const int8_t* A8, const float* qscale, int stride, const uint64_t* B, const float* Bw,
@@ -583,7 +577,7 @@ static void launch_stream_fused(const FusedPlan& plan, const T* x, int64_t d, do
     const int narrow = integer_decimal_scale(dec_scale) != 0 ? 1 : 0;
     hipLaunchKernelGGL((dot_mfma_stream_fused_kernel<T, KT, NI, kVec>), dim3(plan.grid), dim3(plan.waves * 64), lds, st, x, d,
                        dec_scale, narrow, slices, reinterpret_cast<const unsigned long long*>(B), Bw, chunks, pass_chunks,
-                       R, Q, scale_inv, R_total, out, bias);
+                       R, Q, scale_inv, R_total, out, bias, t_out_dtype);
 }
 
 template <typename T>
@@ -619,9 +613,9 @@ extern "C" int bsi_hip_linear_few_rows_upfront(int64_t Q, int64_t d, int64_t R) 
     return p.per_wave <= p.upfront ? 1 : 0;
 }
 
-extern "C" int bsi_hip_linear_few_rows(const void* x, int dtype, int64_t Q, int64_t d, int decimal_places, int fixed_bits,
-                                       const uint64_t* B_tiled, const float* Bw, int Sb, int64_t R, float scale_inv,
-                                       int64_t R_total, const float* bias, float* out, void* stream) {
+static int linear_few_rows(const void* x, int dtype, int64_t Q, int64_t d, int decimal_places, int fixed_bits,
+                           const uint64_t* B_tiled, const float* Bw, int Sb, int64_t R, float scale_inv, int64_t R_total,
+                           const float* bias, float* out, void* stream) {
     BSI_REQUIRE(Q >= 0 && R >= 0 && d >= 1, "bad shape");
     BSI_REQUIRE(Q <= kFusedMaxQ, "the fused few-rows kernel takes at most %d query rows (got %lld)", kFusedMaxQ,
                 static_cast<long long>(Q));
@@ -649,6 +643,23 @@ extern "C" int bsi_hip_linear_few_rows(const void* x, int dtype, int64_t Q, int6
 #undef BSI_FUSED
     BSI_LAUNCH_CHECK("dot_mfma_stream_fused_kernel");
     return BSI_OK;
+}
+
+extern "C" int bsi_hip_linear_few_rows(const void* x, int dtype, int64_t Q, int64_t d, int decimal_places, int fixed_bits,
+                                       const uint64_t* B_tiled, const float* Bw, int Sb, int64_t R, float scale_inv,
+                                       int64_t R_total, const float* bias, float* out, void* stream) {
+    return linear_few_rows(x, dtype, Q, d, decimal_places, fixed_bits, B_tiled, Bw, Sb, R, scale_inv, R_total, bias, out, stream);
+}
+
+extern "C" int bsi_hip_linear_few_rows_out(const void* x, int dtype, int64_t Q, int64_t d, int decimal_places, int fixed_bits,
+                                           const uint64_t* B_tiled, const float* Bw, int Sb, int64_t R, float scale_inv,
+                                           int64_t R_total, const float* bias, void* out, int out_dtype, void* stream) {
+    BSI_REQUIRE(out_dtype == BSI_DTYPE_F32 || out_dtype == BSI_DTYPE_F16 || out_dtype == BSI_DTYPE_BF16, "unknown dtype code %d", out_dtype);
+    t_out_dtype = out_dtype;
+    const int rc = linear_few_rows(x, dtype, Q, d, decimal_places, fixed_bits, B_tiled, Bw, Sb, R, scale_inv, R_total, bias,
+                                   static_cast<float*>(out), stream);
+    t_out_dtype = BSI_DTYPE_F32;
+    return rc;
 }
 
 // Launch of the inline-decode kernel for Q queries (groups of 16 along grid.y), or BSI_ERR_UNSUPPORTED when the

@@ -365,6 +365,50 @@ __device__ __forceinline__ bool i8_store_lines(const float (&v)[WM][WN][4], floa
     return true;
 }
 
+// The same output tile in a half-precision type (v before the bias; `bi` the biases of the lane's rows).  The lane's four
+// keys of a tile are 8 bytes; exchanging one of two vertically adjacent tiles between neighbouring lane rows
+// (v_permlane16_swap: odd rows of the first operand with even rows of the second) gives every lane eight consecutive
+// keys, so a store instruction writes 64 contiguous bytes per query.
+template <int WM, int WN>
+__device__ __forceinline__ void i8_store_half(const float (&v)[WM][WN][4], const float (&bi)[WM][4], bool has_bias, int dtype,
+                                              float* __restrict__ out, int64_t R_total, int64_t rw, int64_t qw, int64_t R,
+                                              int64_t Q, int ln, int lg) {
+    unsigned short* const out16 = reinterpret_cast<unsigned short*>(out);
+    const bool whole = rw + WM * 16 <= R && qw + WN * 16 <= Q && (R_total & 7) == 0 && (reinterpret_cast<uintptr_t>(out) & 15) == 0;
+    if (whole) {
+#pragma unroll
+        for (int a = 0; a < WM; a += 2)
+#pragma unroll
+            for (int b = 0; b < WN; ++b) {
+                uint32_t p[2][2];
+#pragma unroll
+                for (int t = 0; t < 2; ++t)
+#pragma unroll
+                    for (int h = 0; h < 2; ++h)
+                        p[t][h] = half_output(v[a + t][b][2 * h], has_bias, bi[a + t][2 * h], dtype) |
+                                  half_output(v[a + t][b][2 * h + 1], has_bias, bi[a + t][2 * h + 1], dtype) << 16;
+                const auto lo = __builtin_amdgcn_permlane16_swap(p[0][0], p[1][0], false, false);
+                const auto hi = __builtin_amdgcn_permlane16_swap(p[0][1], p[1][1], false, false);
+                const int64_t q = qw + b * 16 + ln;
+                *reinterpret_cast<uint4*>(out16 + static_cast<size_t>(q) * R_total + rw + (a + (lg & 1)) * 16 + (lg >> 1) * 8) =
+                    make_uint4(lo[0], hi[0], lo[1], hi[1]);
+            }
+        return;
+    }
+#pragma unroll
+    for (int a = 0; a < WM; ++a)
+#pragma unroll
+        for (int b = 0; b < WN; ++b) {
+            const int64_t rb = rw + a * 16 + lg * 4, q = qw + b * 16 + ln;
+            if (q >= Q) continue;
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                if (rb + e < R)
+                    out16[static_cast<size_t>(q) * R_total + rb + e] =
+                        static_cast<unsigned short>(half_output(v[a][b][e], has_bias, bi[a][e], dtype));
+        }
+}
+
 template <int TM, int TN, int kMode, bool kSplit>
 __global__ __launch_bounds__((I8Cfg<TM, TN>::kBlock)) void dot_mfma_i8_kernel(
     const int8_t* __restrict__ A8, const float* __restrict__ qscale, int qscale_stride,
@@ -373,7 +417,7 @@ __global__ __launch_bounds__((I8Cfg<TM, TN>::kBlock)) void dot_mfma_i8_kernel(
     int64_t R_total, float* __restrict__ out, int* __restrict__ chunk_ints, const float* __restrict__ bias,
     int ndig, long long dig_stride, const long long* __restrict__ key_indices, int key_tiled,
     const unsigned char* __restrict__ warm, long long warm_lines, int out_stream, float* __restrict__ split_partials,
-    unsigned* __restrict__ split_counters, float split_limit, int split_shape) {
+    unsigned* __restrict__ split_counters, float split_limit, int split_shape, int out_dtype) {
     // kSplit (chain mode only): a D-split launch.  gridDim.z workgroups share an output tile, each running the chain
     // over its own run of chunks from zero.  All operands of the chain are integers (times one power of two), so
     // as long as no value the chain takes exceeds 2^24 of its unit nothing is ever rounded, the value after every
@@ -791,9 +835,13 @@ __global__ __launch_bounds__((I8Cfg<TM, TN>::kBlock)) void dot_mfma_i8_kernel(
             for (int e = 0; e < 4; ++e) {
                 // (acc * key scale) * scale_inv, then + bias: each step rounded on its own, as separate kernels would
                 float v = ((accf[a][b][e] * down) * bs[a][e]) * scale_inv;
-                if (bias != nullptr) v = v + bi[a][e];
+                if (bias != nullptr && out_dtype == BSI_DTYPE_F32) v = v + bi[a][e];
                 accf[a][b][e] = v;
             }
+    if (kMode == kI8Chain && out_dtype != BSI_DTYPE_F32) {
+        i8_store_half<WM, WN>(accf, bi, bias != nullptr, out_dtype, out, R_total, r0 + wr * (WM * 16), q0 + wq * (WN * 16), R, Q, ln, lg);
+        return;
+    }
     if (!i8_store_lines<WM, WN>(accf, out, R_total, r0 + wr * (WM * 16), q0 + wq * (WN * 16), R, Q, ln, lg, out_stream != 0)) {
 #pragma unroll
         for (int a = 0; a < WM; ++a) {
@@ -895,7 +943,7 @@ __global__ __launch_bounds__((I8WCfg<WN>::kBlock)) void dot_mfma_i8w_kernel(
     const int8_t* __restrict__ A8, const float* __restrict__ qscale, int qscale_stride, const int8_t* __restrict__ K8,
     const float* __restrict__ Bw, int Sb, int chunks, int64_t R, int64_t Q, int down_shift, float scale_inv,
     int64_t R_total, float* __restrict__ out, int* __restrict__ chunk_ints, const float* __restrict__ bias,
-    int key_tiled, const unsigned char* __restrict__ warm, long long warm_lines, int out_stream) {
+    int key_tiled, const unsigned char* __restrict__ warm, long long warm_lines, int out_stream, int out_dtype) {
     constexpr int TM = 128, TN = 128;
     using W = I8WCfg<WN>;
     using C = typename W::Tile;
@@ -1026,9 +1074,13 @@ __global__ __launch_bounds__((I8WCfg<WN>::kBlock)) void dot_mfma_i8w_kernel(
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
                 float v = ((accf[a][b][e] * down) * bs[a][e]) * scale_inv;
-                if (bias != nullptr) v = v + bi[a][e];
+                if (bias != nullptr && out_dtype == BSI_DTYPE_F32) v = v + bi[a][e];
                 accf[a][b][e] = v;
             }
+    if (out_dtype != BSI_DTYPE_F32) {
+        i8_store_half<4, WN>(accf, bi, bias != nullptr, out_dtype, out, R_total, r0 + wr * 64, q0 + wq * (16 * WN), R, Q, ln, lg);
+        return;
+    }
     if (i8_store_lines<4, WN>(accf, out, R_total, r0 + wr * 64, q0 + wq * (16 * WN), R, Q, ln, lg, out_stream != 0)) return;
 #pragma unroll
     for (int a = 0; a < 4; ++a) {
@@ -1081,6 +1133,7 @@ thread_local size_t g_warm_bytes = 0;
 // for the 16 MiB of Q512 R8192).  Measured both ways: streamed layer outputs cost an OPT-1.3B-shaped prefill 2 %
 // (4.89 -> 5.00 ms replayed), plain dot outputs cost the standalone dot 8 %.  BSI_OPT_OUTPUT_STORES overrides.
 thread_local int t_layer_output = 0;
+thread_local int t_out_dtype = BSI_DTYPE_F32;
 std::atomic<int> g_output_stores{0};  // 0 = by entry point, 1 = always plain, 2 = always nontemporal
 static int stream_output() {
     const int forced = g_output_stores.load(std::memory_order_relaxed);
@@ -1101,7 +1154,7 @@ static void launch_mfma_i8_tm(const int8_t* A8, const float* qscale, int stride,
                        Bw, Sb, chunks, R, Q, down_shift, scale_inv, R_total, out, chunk_ints, bias, ndig, dig_stride,
                        key_indices, key_tiled, static_cast<const unsigned char*>(g_warm_ptr),
                        static_cast<long long>(g_warm_bytes / 128), stream_output(), static_cast<float*>(nullptr),
-                       static_cast<unsigned*>(nullptr), 0.0f, 0);
+                       static_cast<unsigned*>(nullptr), 0.0f, 0, t_out_dtype);
 }
 
 // The D-split launch of the chain mode: `segments` workgroups per output tile, each over its own run of chunks (see
@@ -1126,7 +1179,7 @@ static void launch_mfma_i8_split(int segments, unsigned char* scratch, const int
                        1, 0LL, static_cast<const long long*>(nullptr), key_tiled,
                        static_cast<const unsigned char*>(g_warm_ptr), static_cast<long long>(g_warm_bytes / 128),
                        stream_output(), reinterpret_cast<float*>(scratch + kSplitCounterBytes),
-                       reinterpret_cast<unsigned*>(scratch), limit, split_shape);
+                       reinterpret_cast<unsigned*>(scratch), limit, split_shape, t_out_dtype);
 }
 
 // Sum mode (ndig >= 1 digit images of the queries; int32 sums into chunk_ints when given, else the float epilogue)
@@ -1164,11 +1217,11 @@ static void launch_mfma_i8w(const int8_t* A8, const float* qscale, int stride, c
     if (chunk_ints)
         hipLaunchKernelGGL((dot_mfma_i8w_kernel<WN, true>), grid, dim3(W::kBlock), C::kLds, st, A8, qscale, stride, K8, Bw, Sb,
                            chunks, R, Q, down_shift, scale_inv, R_total, out, chunk_ints, bias, key_tiled, warm, warm_lines,
-                           stream_output());
+                           stream_output(), t_out_dtype);
     else
         hipLaunchKernelGGL((dot_mfma_i8w_kernel<WN, false>), grid, dim3(W::kBlock), C::kLds, st, A8, qscale, stride, K8, Bw, Sb,
                            chunks, R, Q, down_shift, scale_inv, R_total, out, chunk_ints, bias, key_tiled, warm, warm_lines,
-                           stream_output());
+                           stream_output(), t_out_dtype);
 }
 
 // Tile choice.  The 128 x 128 tile moves the fewest operand bytes per MAC and is the fastest whenever its grid

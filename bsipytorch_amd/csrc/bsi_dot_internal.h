@@ -27,6 +27,9 @@ extern thread_local const void* g_warm_ptr;
 extern thread_local size_t g_warm_bytes;
 // Set by the entry points of a linear layer around their launch: the next kernel of the model reads that output.
 extern thread_local int t_layer_output;
+// Set by the entry points that write a half-precision layer output around their launch (BSI_DTYPE_*; F32 otherwise).  `out`
+// is then an array of that type; kernels that write float32 only are refused by dot_launch.
+extern thread_local int t_out_dtype;
 int choose_i8_tile(int64_t R, int64_t Q, int64_t* cost_out = nullptr);
 // D-split of the chain-mode int8-image dot (bsi_hip_dot_attach_split_scratch): the calling thread's scratch region
 // (counters of kSplitCounterBytes, then the segments' partial sums) and the device it lies on; the option

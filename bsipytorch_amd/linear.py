@@ -21,6 +21,7 @@ from . import bsi_ops
 # Layers fed by the same activation tensor (q_proj / k_proj / v_proj) share one query build: the last built
 # batch is kept with a reference to its input (so its address cannot be reused) and its version counter.
 _last_query_build: Dict[str, Any] = {}
+_HALF_DTYPES = (torch.float16, torch.bfloat16)  # output types the dot's epilogue writes besides float32
 
 
 def forget_shared_builds() -> None:
@@ -205,7 +206,10 @@ class BSIQuantizedLinear(nn.Module):
         if (c.get("collect_stats") or bsi_ops.fast_getenv("BSI_QUERY_PACKED", "1") == "0" or bsi_ops.fast_getenv("BSI_QUERY_CACHE", "1") == "0"
                 or not bsi_ops.can_linear_one_call(batch_inputs, keys)):
             return None
-        fp32 = original_dtype == torch.float32
+        # the output's type and the bias go into the dot's epilogue where its kernel has them
+        half = original_dtype in _HALF_DTYPES and bsi_ops.can_output_half(keys, int(batch_inputs.shape[0]))
+        out_dtype = original_dtype if half else torch.float32
+        fuse_bias = original_dtype == out_dtype
         if fused is not None:
             group, start, stop = fused
             key = bsi_ops.tensor_build_key(batch_inputs, bsi_ops.capture_id())
@@ -216,15 +220,17 @@ class BSIQuantizedLinear(nn.Module):
                 if last[4] <= 0:
                     group.__dict__["_last_call"] = None
             else:
-                gb = bsi_ops.device_bias(group.bias, batch_inputs.device) if fp32 else None
-                all_scores = bsi_ops.linear_cuda(batch_inputs, keys, self.decimalPlaces, gb, _keys_to_warm(group.next_layer), True)
+                gb = bsi_ops.device_bias(group.bias, batch_inputs.device) if fuse_bias else None
+                all_scores = bsi_ops.linear_cuda(batch_inputs, keys, self.decimalPlaces, gb, _keys_to_warm(group.next_layer), True,
+                                                 out_dtype)
                 group.__dict__["_last_call"] = [key, batch_inputs, all_scores, gb is not None, len(group.members) - 1]
                 scores, bias_done = all_scores[:, start:stop], gb is not None
                 c["dot_calls"] += 1
                 c["build_calls"] += int(bsi_ops._last_linear_rebuilt[0])
         else:
-            b = bsi_ops.device_bias(self.bias, batch_inputs.device) if fp32 else None
-            scores = bsi_ops.linear_cuda(batch_inputs, keys, self.decimalPlaces, b, _keys_to_warm(c.get("_next_bsi_layer")), True)
+            b = bsi_ops.device_bias(self.bias, batch_inputs.device) if fuse_bias else None
+            scores = bsi_ops.linear_cuda(batch_inputs, keys, self.decimalPlaces, b, _keys_to_warm(c.get("_next_bsi_layer")), True,
+                                         out_dtype)
             bias_done = b is not None
             c["dot_calls"] += 1
             c["build_calls"] += int(bsi_ops._last_linear_rebuilt[0])
@@ -253,7 +259,8 @@ class BSIQuantizedLinear(nn.Module):
         if (torch.cuda.is_current_stream_capturing() and bsi_ops.fast_getenv("BSI_FUSED_LINEAR", "1") != "2"
                 and not bsi_ops.linear_few_rows_is_free(batch_inputs, keys)):
             return None
-        fp32 = original_dtype == torch.float32
+        out_dtype = original_dtype if original_dtype in _HALF_DTYPES else torch.float32
+        fuse_bias = original_dtype == out_dtype
         bsi_ops.warm_query_build_caches(int(batch_inputs.shape[0]))
         bsi_ops.reserve_linear_workspace(batch_inputs)  # a later capture of this forward may take the one-call path
         if fused is not None:
@@ -266,15 +273,16 @@ class BSIQuantizedLinear(nn.Module):
                 if last[4] <= 0:
                     group.__dict__["_last_few"] = None
             else:
-                gb = bsi_ops.device_bias(group.bias, batch_inputs.device) if fp32 else None
-                all_scores = bsi_ops.linear_few_rows_cuda(batch_inputs, keys, self.decimalPlaces, gb, True)
+                gb = bsi_ops.device_bias(group.bias, batch_inputs.device) if fuse_bias else None
+                all_scores = bsi_ops.linear_few_rows_cuda(batch_inputs, keys, self.decimalPlaces, gb, True, out_dtype)
                 # holds the input's storage (so that its address is not reused) until every member has been served
                 group.__dict__["_last_few"] = [key, batch_inputs, all_scores, gb is not None, len(group.members) - 1]
                 scores, bias_done = all_scores[:, start:stop], gb is not None
                 c["dot_calls"] += 1
         else:
-            b = bsi_ops.device_bias(self.bias, batch_inputs.device) if fp32 else None
-            scores, bias_done = bsi_ops.linear_few_rows_cuda(batch_inputs, keys, self.decimalPlaces, b, True), b is not None
+            b = bsi_ops.device_bias(self.bias, batch_inputs.device) if fuse_bias else None
+            scores = bsi_ops.linear_few_rows_cuda(batch_inputs, keys, self.decimalPlaces, b, True, out_dtype)
+            bias_done = b is not None
             c["dot_calls"] += 1
         q_rows = int(batch_inputs.shape[0])
         c["dot_query_vectors_total"] += q_rows
