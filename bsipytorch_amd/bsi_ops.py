@@ -28,7 +28,7 @@ from typing import List, Optional
 
 import torch
 
-from . import _lib
+from . import _lib, _native
 from ._lib import check, lib
 
 # --------------------------------------------------------------------------- flags
@@ -103,12 +103,17 @@ def _flags() -> dict:
         image_tiled=(_env_int("BSI_KEY_IMAGE_TILED", 0) or 0) != 0,
         dot_split=(_env_int("BSI_DOT_SPLIT", 1) or 0) != 0,
     )
+    f = _flag_cache
+    if (2 <= bits_q <= 8 and f["chunk_scale"] and f["clip_k"] == 0.0 and f["core"] != _lib.CORE_VALU
+            and not (f["profile"] or f["debug"] or f["dot_debug"])):
+        _native.configure(bits_q, f["core"])  # the configurations its calls serve
     return _flag_cache
 
 
 def _reset_flag_cache() -> None:
     """Test hook: re-read the environment on the next call."""
     _flag_cache.clear()
+    _native.configure()
     _DOT_DEBUG_PRINTED[0] = False
 
 
@@ -1283,11 +1288,11 @@ def linear_cuda(x2d: torch.Tensor, keyset_cuda_cap, decimal_places: int, bias=No
         if mine is None:  # first eager call on this stream (allocated under it, so freed in its order too)
             mine = ws["eager"][st] = (torch.empty((ws["bytes"],), dtype=torch.uint8, device=x2d.device), [None, None])
         buf, slot = mine
-    key = tensor_build_key(x2d, int(decimal_places), keys.Sb)
+    key = _native.build_key(x2d, int(decimal_places), keys.Sb)  # the native path's form: eager calls share their builds
     if capturing and key is not None:
         # a build recorded by one capture is not part of another capture's graph: the capture's identifier is part
         # of what a recorded launch may reuse (a second capture starting on the same static input builds anew)
-        key = key + (capture_id(),)
+        key = (key, capture_id())
     rebuild = 0 if (key is not None and slot[0] == key) else 1
     slot[0], slot[1] = key, x2d  # holds the input, so that its address is not reused while the build stands for it
     wsptr = buf.data_ptr()
@@ -1326,6 +1331,10 @@ def batch_dot_product_multiquery_cuda_batch_caps(query_batch_cap, keyset_cuda_ca
     ``bias`` (not in the reference's signature): an optional float32 [R] device tensor added to every output
     row in the same launch, rounded as ``out + bias`` would be.  ``warm_keys`` (not in the reference either): the
     keyset the next dot will use; this launch also reads it once so that it is cache-resident by then."""
+    if bias is None and warm_keys is None:
+        out = _native.dot(query_batch_cap, keyset_cuda_cap)
+        if out is not None:
+            return out, 0, 0.0, 0.0
     keys = _capsule(keyset_cuda_cap, PrebuiltBSIKeysCUDA, "Invalid CUDA keys capsule")
     if isinstance(query_batch_cap, PrebuiltBSIQueryBatchHybridCUDA):
         # the batched hybrid form: EWAH streams, decoded in the dot's load stage
@@ -1502,6 +1511,14 @@ def debug_quantize_int64_cpu(values: torch.Tensor, decimal_places: int) -> torch
     x = values.detach().to("cpu", torch.float32).to(torch.float64) * (10.0 ** int(decimal_places))
     return torch.where(x >= 0, torch.floor(x + 0.5), -torch.floor(-x + 0.5)).to(torch.int64)
 
+
+# The native host path reads these on every call, so what the functions above keep stays the one copy.
+_native.bind({name: ctypes.cast(getattr(lib, name), ctypes.c_void_p).value
+              for name in ("bsi_hip_linear_few_rows_out", "bsi_hip_linear_out", "bsi_hip_linear_workspace_bytes", "bsi_hip_dot")},
+             {"keys_type": PrebuiltBSIKeysCUDA, "batch_type": PrebuiltBSIQueryBatchCUDA, "linear_ws": _linear_ws,
+              "reserved": _reserved_linear_shapes, "warmed": _warmed_query_caches, "split_shapes": _split_shapes,
+              "attach": attach_split_scratch, "check": check},
+             FUSED_LINEAR_MAX_ROWS, _FEW_ROWS_MAX_Q, _SPLIT_MIN_Q, FUSED_LINEAR_QUERY_LDS_BYTES)
 
 # The reference's scalar ("non-CUDA") entry points (bsiFunctions.cpp:811-846): served by the device kernels here.
 from .bsi_scalar import (  # noqa: E402,F401

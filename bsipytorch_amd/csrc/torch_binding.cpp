@@ -1,0 +1,463 @@
+// bsipytorch_amd._native: the host path of an eager call, in C++.
+//
+// A small layer's forward is bound by the host: reading the layer's and the keyset's attributes, checking the operands,
+// allocating the output and entering the C ABI through ctypes took 13 us of Python for 4 us of GPU work.  The functions
+// here do the same for the default configuration on the objects the Python code keeps -- they read the layer's and the
+// handles' attributes on every call, so nothing can go stale -- and return None for any call they do not serve; the Python
+// path behind them then serves it or raises its errors.  Launches recorded into a graph always take that path.
+#include <torch/csrc/autograd/python_variable.h>
+#include <ATen/hip/EmptyTensor.h>
+#include <c10/hip/HIPFunctions.h>
+#include <c10/hip/HIPGraphsC10Utils.h>
+#include <c10/hip/HIPStream.h>
+
+#include <cstring>
+#include <unordered_map>
+
+#include "../../include/bsi_hip.h"
+
+extern char** environ;
+
+namespace {
+
+// Entry points of the library the Python side has loaded (bind()).
+struct Library {
+    decltype(&bsi_hip_linear_few_rows_out) linear_few_rows_out;
+    decltype(&bsi_hip_linear_out) linear_out;
+    decltype(&bsi_hip_linear_workspace_bytes) linear_workspace_bytes;
+    decltype(&bsi_hip_dot) dot;
+} lib;
+
+// The Python side's state (bind()): types of the handles, the workspaces and what is known about shapes.
+struct Shared {
+    PyObject *keys_type, *batch_type;      // PrebuiltBSIKeysCUDA, PrebuiltBSIQueryBatchCUDA
+    PyObject *linear_ws;                   // device index -> {"bytes", "eager": {stream: (buffer, [key, input])}, ...}
+    PyObject *reserved, *warmed;           // shapes whose workspace and constants a later capture will find
+    PyObject *split_shapes, *attach;       // (device, Q, R, W) -> whether the dot splits; attach_split_scratch
+    PyObject *check;                       // raises for a library status
+    int few_rows_max, stream_max, split_min;
+    int64_t few_rows_lds;
+} shared;
+
+// The flags of the process (configure()); off until they have been read, and for configurations the Python path serves.
+struct Config {
+    bool on = false;
+    int bits = 0, core = 0;
+    int64_t generation = 0;
+} config;
+
+#define NAMES(X)                                                                                                          \
+    X(_bsi_keys_cuda) X(_fused) X(_next_bsi_layer) X(_buffers) X(bias) X(collect_stats) X(decimalPlaces) X(fixed) X(Sb) X(W) X(d) \
+    X(num_keys) X(decimals) X(layout) X(words) X(ints8) X(ints8_tiled) X(slice_weights) X(bytes) X(eager) X(dot_calls)      \
+    X(build_calls) X(dot_query_vectors_total) X(dot_output_elements_total) X(chunk_scales) X(row_scales) X(keys)
+struct Names {
+#define X(n) PyObject* n;
+    NAMES(X)
+#undef X
+} names;
+
+// The switches that are read on every call, with the value at which they change nothing.
+bool switches_at_default() {
+    static const struct { const char* name; size_t len; const char* value; } kSwitches[] = {
+        {"BSI_TC_DOT=", 11, "1"}, {"BSI_QUERY_FP32=", 15, "0"}, {"BSI_FUSED_LINEAR=", 17, "1"},
+        {"BSI_LINEAR_ONE_CALL=", 20, "1"}, {"BSI_QUERY_PACKED=", 17, "1"}, {"BSI_QUERY_CACHE=", 16, "1"}};
+    for (char** e = environ; e && *e; ++e) {
+        if ((*e)[0] != 'B' || (*e)[1] != 'S' || (*e)[2] != 'I' || (*e)[3] != '_') continue;
+        for (const auto& s : kSwitches)
+            if (std::strncmp(*e, s.name, s.len) == 0 && std::strcmp(*e + s.len, s.value) != 0) return false;
+    }
+    return true;
+}
+
+// Borrowed reference to dict[name], or nullptr (no error left behind).
+PyObject* get(PyObject* dict, PyObject* name) { return PyDict_GetItem(dict, name); }
+bool get_int(PyObject* dict, PyObject* name, int64_t* v) {
+    PyObject* o = get(dict, name);
+    if (o == nullptr || !PyLong_Check(o)) return false;
+    *v = PyLong_AsLongLong(o);
+    return true;
+}
+const at::Tensor* get_tensor(PyObject* dict, PyObject* name) {
+    PyObject* o = get(dict, name);
+    return o != nullptr && THPVariable_Check(o) ? &THPVariable_Unpack(o) : nullptr;
+}
+void count(PyObject* dict, PyObject* name, int64_t by) {
+    int64_t v = 0;
+    if (!get_int(dict, name, &v)) return;
+    if (PyObject* n = PyLong_FromLongLong(v + by)) {
+        PyDict_SetItem(dict, name, n);
+        Py_DECREF(n);
+    }
+}
+
+struct Holder {  // an owned reference
+    PyObject* p;
+    explicit Holder(PyObject* o = nullptr) : p(o) {}
+    ~Holder() { Py_XDECREF(p); }
+    Holder(const Holder&) = delete;
+    Holder& operator=(const Holder&) = delete;
+};
+
+int dtype_code(at::ScalarType t) {
+    switch (t) {
+        case at::kFloat: return BSI_DTYPE_F32;
+        case at::kHalf: return BSI_DTYPE_F16;
+        case at::kBFloat16: return BSI_DTYPE_BF16;
+        default: return -1;
+    }
+}
+
+// A fixed-bit keyset's attributes as the dot needs them.
+struct Keys {
+    int64_t Sb, W, d, R, decimals, layout;
+    const at::Tensor *words, *ints8, *weights;
+    bool tiled_image;
+};
+bool read_keys(PyObject* handle, const at::Device& device, Keys* k) {
+    if (handle == nullptr || reinterpret_cast<PyObject*>(Py_TYPE(handle)) != shared.keys_type) return false;
+    Holder attrs(PyObject_GenericGetDict(handle, nullptr));
+    if (attrs.p == nullptr) {
+        PyErr_Clear();
+        return false;
+    }
+    if (get(attrs.p, names.fixed) != Py_True || !get_int(attrs.p, names.Sb, &k->Sb) || !get_int(attrs.p, names.W, &k->W) ||
+        !get_int(attrs.p, names.d, &k->d) || !get_int(attrs.p, names.num_keys, &k->R) ||
+        !get_int(attrs.p, names.decimals, &k->decimals) || !get_int(attrs.p, names.layout, &k->layout))
+        return false;
+    k->words = get_tensor(attrs.p, names.words);
+    k->ints8 = get_tensor(attrs.p, names.ints8);
+    k->weights = get_tensor(attrs.p, names.slice_weights);
+    k->tiled_image = get(attrs.p, names.ints8_tiled) == Py_True;
+    return k->words != nullptr && k->weights != nullptr && k->words->device() == device && k->weights->device() == device &&
+           k->weights->is_contiguous() && k->R > 0 && k->Sb >= 2 && k->Sb <= 8;
+}
+// What a dot of Q rows reads of the keyset (bsi_ops.key_operand).
+const void* key_operand(const Keys& k, int64_t Q, int* layout, size_t* bytes) {
+    const bool image = k.ints8 != nullptr && Q > shared.stream_max;
+    const at::Tensor& t = image ? *k.ints8 : *k.words;
+    *layout = image ? (k.tiled_image ? BSI_LAYOUT_INT8_TILED : BSI_LAYOUT_INT8) : static_cast<int>(k.layout);
+    *bytes = t.nbytes();
+    return t.const_data_ptr();
+}
+
+PyObject* int_tuple(std::initializer_list<int64_t> values) {
+    PyObject* t = PyTuple_New(static_cast<Py_ssize_t>(values.size()));
+    Py_ssize_t i = 0;
+    if (t != nullptr)
+        for (int64_t v : values) PyTuple_SET_ITEM(t, i++, PyLong_FromLongLong(v));
+    return t;
+}
+bool in_set(PyObject* set, std::initializer_list<int64_t> values) {
+    Holder t(int_tuple(values));
+    return t.p != nullptr && PySet_Contains(set, t.p) == 1;
+}
+
+// Attaches the split scratch if the launcher splits a dot of this shape; false: the Python side has to find out first.
+bool split_scratch(int device, int64_t Q, int64_t R, int64_t W) {
+    if (Q < shared.split_min) return true;
+    Holder t(int_tuple({device, Q, R, W}));
+    PyObject* use = t.p != nullptr ? PyDict_GetItem(shared.split_shapes, t.p) : nullptr;
+    if (use == nullptr) return false;
+    if (use == Py_True) {
+        Holder r(PyObject_CallNoArgs(shared.attach));
+        if (r.p == nullptr) {
+            PyErr_Clear();
+            return false;
+        }
+    }
+    return true;
+}
+
+PyObject* fail_status(int rc, const char* what) {
+    Holder r(PyObject_CallFunction(shared.check, "is", rc, what));  // raises
+    if (r.p != nullptr) PyErr_Format(PyExc_RuntimeError, "%s failed (code %d)", what, rc);
+    return nullptr;
+}
+
+float scale_inv(int64_t dec_q, int64_t dec_k) {
+    double p = 1.0;
+    for (int64_t i = 0; i < dec_q + dec_k; ++i) p *= 10.0;
+    return static_cast<float>(1.0 / p);
+}
+
+// What identifies the query build of a contiguous tensor for keys of Sb slices: its contents (address, shape, type,
+// version) and what the build depends on (the generation stands for the process's flags); compared byte by byte.
+struct BuildKey {
+    const void* data;
+    int64_t rows, d, version, generation;
+    int32_t dtype, decimals, Sb, unused;
+};
+BuildKey build_key_of(const at::Tensor& x, int64_t d, int64_t decimals, int64_t Sb) {
+    return BuildKey{x.const_data_ptr(), x.numel() / d, d, static_cast<int64_t>(x.unsafeGetTensorImpl()->version_counter().current_version()),
+                    config.generation, dtype_code(x.scalar_type()), static_cast<int32_t>(decimals), static_cast<int32_t>(Sb), 0};
+}
+
+// build_key(x2d, decimals, Sb) -> bytes, or None for a tensor without a version counter (inference mode), whose contents
+// cannot be tracked.
+PyObject* build_key(PyObject*, PyObject* args) {
+    PyObject* o = nullptr;
+    long long decimals = 0, Sb = 0;
+    if (!PyArg_ParseTuple(args, "OLL", &o, &decimals, &Sb)) return nullptr;
+    HANDLE_TH_ERRORS
+    if (!THPVariable_Check(o)) return PyErr_Format(PyExc_TypeError, "build_key: not a tensor");
+    const at::Tensor& x = THPVariable_Unpack(o);
+    if (x.is_inference() || x.dim() < 1 || x.numel() == 0) Py_RETURN_NONE;
+    const BuildKey key = build_key_of(x, x.size(-1), decimals, Sb);
+    return PyBytes_FromStringAndSize(reinterpret_cast<const char*>(&key), sizeof(key));
+    END_HANDLE_TH_ERRORS
+}
+
+// linear(layer.__dict__, x) -> the layer's output, or None.
+PyObject* linear(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+    if (nargs != 2 || !PyDict_Check(args[0])) {
+        PyErr_SetString(PyExc_TypeError, "linear(layer.__dict__, x)");
+        return nullptr;
+    }
+    PyObject* const layer = args[0];
+    PyObject* x_object = args[1];
+    if (!config.on || !THPVariable_CheckExact(x_object) || !switches_at_default()) Py_RETURN_NONE;
+    if (PyObject* o = get(layer, names._fused); o != nullptr && o != Py_None) Py_RETURN_NONE;
+    if (get(layer, names.collect_stats) != Py_False) Py_RETURN_NONE;
+    HANDLE_TH_ERRORS
+    at::Tensor x = THPVariable_Unpack(x_object);
+    const int in_code = dtype_code(x.scalar_type());
+    if (!x.is_cuda() || x.layout() != at::kStrided || in_code < 0 || x.dim() < 1 || x.numel() == 0) Py_RETURN_NONE;
+    const at::Device device = x.device();
+    if (device.index() != c10::hip::current_device()) Py_RETURN_NONE;
+    Keys k;
+    int64_t decimals = 0;
+    if (!read_keys(get(layer, names._bsi_keys_cuda), device, &k) || !get_int(layer, names.decimalPlaces, &decimals) ||
+        decimals != k.decimals || decimals < 0 || x.size(-1) != k.d)
+        Py_RETURN_NONE;
+    const int64_t d = k.d, rows = x.numel() / d, chunks = (k.W + 3) / 4;
+    PyObject* const buffers = get(layer, names._buffers);
+    if (buffers == nullptr || !PyDict_Check(buffers)) Py_RETURN_NONE;
+    const float* bias = nullptr;
+    if (PyObject* o = get(buffers, names.bias); o != nullptr && o != Py_None) {
+        if (!THPVariable_Check(o)) Py_RETURN_NONE;
+        const at::Tensor& b = THPVariable_Unpack(o);
+        if (b.device() != device || b.scalar_type() != at::kFloat || b.dim() != 1 || b.numel() != k.R || !b.is_contiguous())
+            Py_RETURN_NONE;
+        bias = b.const_data_ptr<float>();
+    }
+    // half-precision output: the kernels that have it (bsi_ops.can_output_half)
+    const bool six_tiled = k.Sb == 6 && k.layout == BSI_LAYOUT_TILED16;
+    if (in_code != BSI_DTYPE_F32 && !(rows > shared.stream_max ? k.ints8 != nullptr : six_tiled && chunks <= 32768)) Py_RETURN_NONE;
+    if (c10::hip::currentStreamCaptureStatusMayInitCtx() != c10::hip::CaptureStatus::None) Py_RETURN_NONE;
+    const c10::hip::HIPStream stream = c10::hip::getCurrentHIPStream(device.index());
+    hipStream_t const st = stream.stream();
+
+    const bool few = rows <= shared.few_rows_max && six_tiled && k.W % 4 == 0 && chunks * rows * 260 <= shared.few_rows_lds;
+    PyObject* slot = nullptr;
+    void* ws = nullptr;
+    int64_t ws_bytes = 0;
+    if (few) {
+        if (!in_set(shared.reserved, {device.index(), rows, d, config.bits}) || !in_set(shared.warmed, {rows, config.bits, device.index()}))
+            Py_RETURN_NONE;
+    } else {
+        Holder index(PyLong_FromLong(device.index()));
+        PyObject* record = PyDict_GetItem(shared.linear_ws, index.p);
+        if (record == nullptr || !get_int(record, names.bytes, &ws_bytes) ||
+            static_cast<size_t>(ws_bytes) < lib.linear_workspace_bytes(rows, d, config.bits))
+            Py_RETURN_NONE;
+        Holder handle(PyLong_FromVoidPtr(st));
+        PyObject* const eager = get(record, names.eager);
+        PyObject* const mine = eager != nullptr ? PyDict_GetItem(eager, handle.p) : nullptr;
+        if (mine == nullptr || !PyTuple_Check(mine) || PyTuple_GET_SIZE(mine) != 2 || !THPVariable_Check(PyTuple_GET_ITEM(mine, 0)))
+            Py_RETURN_NONE;
+        ws = THPVariable_Unpack(PyTuple_GET_ITEM(mine, 0)).data_ptr();
+        slot = PyTuple_GET_ITEM(mine, 1);
+        if (!PyList_Check(slot) || PyList_GET_SIZE(slot) != 2 || !split_scratch(device.index(), rows, k.R, k.W)) Py_RETURN_NONE;
+    }
+
+    Holder owned;  // the object that stands for x when it is not the caller's
+    if (x.requires_grad()) x = x.detach();
+    if (!x.is_contiguous()) x = x.contiguous();
+    if (&*x.unsafeGetTensorImpl() != THPVariable_Unpack(x_object).unsafeGetTensorImpl() && slot != nullptr) {
+        owned.p = THPVariable_Wrap(x);
+        x_object = owned.p;
+    }
+    c10::SmallVector<int64_t, 5> sizes(x.sizes().begin(), x.sizes().end());
+    sizes.back() = k.R;
+    at::Tensor out = at::detail::empty_cuda(sizes, x.scalar_type(), device, std::nullopt);
+    const float inv = scale_inv(decimals, k.decimals);
+    const void* const xp = x.const_data_ptr();
+    int rc = BSI_OK;
+    if (few) {
+        Py_BEGIN_ALLOW_THREADS
+        rc = lib.linear_few_rows_out(xp, in_code, rows, d, static_cast<int>(decimals), config.bits,
+                                     static_cast<const uint64_t*>(k.words->const_data_ptr()), k.weights->const_data_ptr<float>(),
+                                     static_cast<int>(k.Sb), k.R, inv, k.R, bias, out.data_ptr(), in_code, st);
+        Py_END_ALLOW_THREADS
+        if (rc != BSI_OK) return fail_status(rc, "bsi_hip_linear_few_rows_out");
+    } else {
+        // a call on the tensor the workspace was last built from skips the build, as in bsi_ops.linear_cuda
+        int rebuild = 1;
+        if (x.is_inference()) {
+            Py_INCREF(Py_None);
+            PyList_SetItem(slot, 0, Py_None);
+        } else {
+            const BuildKey key = build_key_of(x, d, decimals, k.Sb);
+            PyObject* const last = PyList_GET_ITEM(slot, 0);
+            if (PyBytes_CheckExact(last) && PyBytes_GET_SIZE(last) == sizeof(key) &&
+                std::memcmp(PyBytes_AS_STRING(last), &key, sizeof(key)) == 0)
+                rebuild = 0;
+            else
+                PyList_SetItem(slot, 0, PyBytes_FromStringAndSize(reinterpret_cast<const char*>(&key), sizeof(key)));
+        }
+        Py_INCREF(x_object);
+        PyList_SetItem(slot, 1, x_object);  // its address is not reused while the build stands for it
+        int layout = 0, warm_layout = 0;
+        size_t bytes = 0, warm_bytes = 0;
+        const void* const operand = key_operand(k, rows, &layout, &bytes);
+        const void* warm = nullptr;
+        PyObject* next = rows > shared.stream_max ? get(layer, names._next_bsi_layer) : nullptr;
+        if (next != nullptr && next != Py_None) {  // the keys of the layer that runs next, touched by this dot's kernel
+            Holder attrs(PyObject_GenericGetDict(next, nullptr));
+            PyObject* handle = attrs.p != nullptr ? get(attrs.p, names._bsi_keys_cuda) : nullptr;
+            Holder group_keys;
+            if (PyObject* g = attrs.p != nullptr ? get(attrs.p, names._fused) : nullptr; g != nullptr && PyTuple_Check(g)) {
+                group_keys.p = PyObject_GetAttr(PyTuple_GET_ITEM(g, 0), names.keys);
+                handle = group_keys.p;
+            }
+            PyErr_Clear();
+            Keys nk;
+            if (read_keys(handle, device, &nk)) warm = key_operand(nk, rows, &warm_layout, &warm_bytes);
+        }
+        // under the interpreter lock: another thread on this stream must not find the slot before the build is enqueued,
+        // nor enqueue a build of its own between the two launches
+        rc = lib.linear_out(xp, in_code, rows, d, static_cast<int>(decimals), config.bits, rebuild, ws, static_cast<size_t>(ws_bytes),
+                            static_cast<const uint64_t*>(operand), layout, k.weights->const_data_ptr<float>(), static_cast<int>(k.Sb),
+                            k.R, inv, k.R, bias, out.data_ptr(), in_code, config.core, warm, warm_bytes, st);
+        if (rc != BSI_OK) return fail_status(rc, "bsi_hip_linear_out");
+        count(layer, names.build_calls, rebuild);
+    }
+    count(layer, names.dot_calls, 1);
+    count(layer, names.dot_query_vectors_total, rows);
+    count(layer, names.dot_output_elements_total, rows * k.R);
+    return THPVariable_Wrap(std::move(out));
+    END_HANDLE_TH_ERRORS
+}
+
+// dot(query_batch, keyset) -> the float32 scores, or None: the plain dot of a fixed-bit batch that carries its int8 image.
+PyObject* dot(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+    if (nargs != 2) {
+        PyErr_SetString(PyExc_TypeError, "dot(query_batch, keyset)");
+        return nullptr;
+    }
+    if (!config.on || reinterpret_cast<PyObject*>(Py_TYPE(args[0])) != shared.batch_type || !switches_at_default()) Py_RETURN_NONE;
+    HANDLE_TH_ERRORS
+    Holder attrs(PyObject_GenericGetDict(args[0], nullptr));
+    if (attrs.p == nullptr) return nullptr;
+    const at::Tensor* const words = get_tensor(attrs.p, names.words);
+    const at::Tensor* const weights = get_tensor(attrs.p, names.slice_weights);
+    const at::Tensor* const ints8 = get_tensor(attrs.p, names.ints8);
+    const at::Tensor* const chunk_scales = get_tensor(attrs.p, names.chunk_scales);
+    const at::Tensor* const row_scales = get_tensor(attrs.p, names.row_scales);
+    int64_t decimals = 0;
+    if (get(attrs.p, names.fixed) != Py_True || words == nullptr || weights == nullptr || ints8 == nullptr || words->dim() != 3 ||
+        weights->dim() != 2 || !weights->is_cuda() || !words->is_cuda() || !get_int(attrs.p, names.decimals, &decimals))
+        Py_RETURN_NONE;
+    const at::Device device = words->device();
+    const int64_t Q = words->size(0), Sa = words->size(1), W = words->size(2), chunks = (W + 3) / 4;
+    const bool chunked = chunk_scales != nullptr && chunk_scales->numel() > 0;
+    const at::Tensor* const scales = chunked ? chunk_scales : row_scales;
+    Keys k;
+    if (device.index() != c10::hip::current_device() || !read_keys(args[1], device, &k) || k.W != W || k.decimals != decimals ||
+        decimals < 0 || Q <= 0 || Sa < 2 || Sa > 8 || weights->size(0) != Q || weights->size(1) != Sa || scales == nullptr ||
+        scales->device() != device || scales->scalar_type() != at::kFloat || !scales->is_contiguous() || ints8->device() != device ||
+        !ints8->is_contiguous() || ints8->numel() != Q * chunks * 256 || !words->is_contiguous())
+        Py_RETURN_NONE;
+    if (chunked ? (scales->dim() != 2 || scales->size(0) != Q || W % 4 != 0 || scales->size(1) != chunks) : scales->numel() != Q)
+        Py_RETURN_NONE;
+    if (c10::hip::currentStreamCaptureStatusMayInitCtx() != c10::hip::CaptureStatus::None ||
+        !split_scratch(device.index(), Q, k.R, W))
+        Py_RETURN_NONE;
+    hipStream_t const st = c10::hip::getCurrentHIPStream(device.index()).stream();
+    at::Tensor out = at::detail::empty_cuda({Q, k.R}, at::kFloat, device, std::nullopt);
+    int layout = 0, rc = BSI_OK;
+    size_t bytes = 0;
+    const void* const operand = key_operand(k, Q, &layout, &bytes);
+    Py_BEGIN_ALLOW_THREADS
+    rc = lib.dot(static_cast<const uint64_t*>(words->const_data_ptr()), static_cast<const int8_t*>(ints8->const_data_ptr()),
+                 scales->const_data_ptr<float>(), chunked ? static_cast<int>(chunks) : 1, static_cast<int>(Sa), static_cast<int>(W),
+                 static_cast<const uint64_t*>(operand), layout, k.weights->const_data_ptr<float>(), static_cast<int>(k.Sb), k.R, Q,
+                 scale_inv(decimals, k.decimals), k.R, out.data_ptr<float>(), nullptr, config.core, nullptr, 0, st);
+    Py_END_ALLOW_THREADS
+    if (rc != BSI_OK) return fail_status(rc, "bsi_hip_dot");
+    return THPVariable_Wrap(std::move(out));
+    END_HANDLE_TH_ERRORS
+}
+
+// configure(bits, core): the process's flags, or configure() to switch the native path off until they are read again.
+PyObject* configure(PyObject*, PyObject* args) {
+    int bits = 0, core = 0;
+    if (!PyArg_ParseTuple(args, "|ii", &bits, &core)) return nullptr;
+    config.on = bits != 0;
+    config.bits = bits;
+    config.core = core;
+    ++config.generation;
+    Py_RETURN_NONE;
+}
+
+bool take(PyObject* from, const char* name, PyObject** to) {
+    PyObject* o = PyDict_GetItemString(from, name);
+    if (o == nullptr) {
+        PyErr_Format(PyExc_KeyError, "bind: %s", name);
+        return false;
+    }
+    Py_INCREF(o);
+    Py_XDECREF(*to);
+    *to = o;
+    return true;
+}
+template <typename F>
+bool entry(PyObject* from, const char* name, F* to) {
+    PyObject* o = PyDict_GetItemString(from, name);
+    void* p = o != nullptr ? PyLong_AsVoidPtr(o) : nullptr;
+    if (p == nullptr) {
+        if (!PyErr_Occurred()) PyErr_Format(PyExc_KeyError, "bind: %s", name);
+        return false;
+    }
+    *to = reinterpret_cast<F>(p);
+    return true;
+}
+
+// bind(entry_points, state, limits): addresses of the library's functions, the Python side's objects, its constants.
+PyObject* bind(PyObject*, PyObject* args) {
+    PyObject *entries, *state;
+    int few, stream, split;
+    long long lds;
+    if (!PyArg_ParseTuple(args, "O!O!iiiL", &PyDict_Type, &entries, &PyDict_Type, &state, &few, &stream, &split, &lds)) return nullptr;
+    if (!entry(entries, "bsi_hip_linear_few_rows_out", &lib.linear_few_rows_out) || !entry(entries, "bsi_hip_linear_out", &lib.linear_out) ||
+        !entry(entries, "bsi_hip_linear_workspace_bytes", &lib.linear_workspace_bytes) || !entry(entries, "bsi_hip_dot", &lib.dot) ||
+        !take(state, "keys_type", &shared.keys_type) || !take(state, "batch_type", &shared.batch_type) ||
+        !take(state, "linear_ws", &shared.linear_ws) || !take(state, "reserved", &shared.reserved) ||
+        !take(state, "warmed", &shared.warmed) || !take(state, "split_shapes", &shared.split_shapes) ||
+        !take(state, "attach", &shared.attach) || !take(state, "check", &shared.check))
+        return nullptr;
+    shared.few_rows_max = few;
+    shared.stream_max = stream;
+    shared.split_min = split;
+    shared.few_rows_lds = lds;
+    Py_RETURN_NONE;
+}
+
+PyMethodDef methods[] = {
+    {"bind", bind, METH_VARARGS, nullptr},
+    {"configure", configure, METH_VARARGS, nullptr},
+    {"build_key", build_key, METH_VARARGS, nullptr},
+    {"linear", reinterpret_cast<PyCFunction>(reinterpret_cast<void*>(linear)), METH_FASTCALL, nullptr},
+    {"dot", reinterpret_cast<PyCFunction>(reinterpret_cast<void*>(dot)), METH_FASTCALL, nullptr},
+    {nullptr, nullptr, 0, nullptr},
+};
+PyModuleDef module = {PyModuleDef_HEAD_INIT, "_native", "Host path of eager calls.", -1, methods, nullptr, nullptr, nullptr, nullptr};
+
+}  // namespace
+
+PyMODINIT_FUNC PyInit__native() {
+#define X(n) names.n = PyUnicode_InternFromString(#n);
+    NAMES(X)
+#undef X
+    return PyModule_Create(&module);
+}

@@ -34,7 +34,7 @@ setup(
     description="MI355X-native bsi_ops: BSI builder, EWAH codec and the fixed-bit chunk-scale dot behind the reference's API",
     packages=["bsipytorch_amd", "bsipytorch_amd.benchmarks"],
     py_modules=["bsi_ops"],
-    package_data={"bsipytorch_amd": ["libbsi_hip.so", "libbsi_reference_launchers.so"]},
+    package_data={"bsipytorch_amd": ["libbsi_hip.so", "libbsi_reference_launchers.so", "_native.so"]},
     include_package_data=False,
     python_requires=">=3.9",
     install_requires=[],  # torch (ROCm build) supplies device memory and streams; it is not pulled in from here

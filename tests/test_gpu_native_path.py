@@ -1,0 +1,79 @@
+"""The native host path serves the default calls with the Python path's bits, follows what happens to the layer, and leaves
+everything else to the Python path."""
+import threading
+
+import pytest
+import torch
+
+from test_gpu_parity import ops  # noqa: F401  (fixture)
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
+@pytest.mark.parametrize("shape", [(512,), (1, 512), (4, 512), (2, 9, 512), (33, 512), (3, 100, 512)])
+def test_served_calls_match_the_python_path(ops, monkeypatch, shape, dtype):
+    from bsipytorch_amd import _native
+    from bsipytorch_amd.linear import BSIQuantizedLinear
+
+    torch.manual_seed(3)
+    layer = BSIQuantizedLinear(torch.nn.Linear(512, 200).cuda(), 2, 0.5)
+    x = torch.randn(*shape, device="cuda").to(dtype)
+    strided = torch.randn(*shape, 2, device="cuda").to(dtype)[..., 0]
+    with torch.no_grad():
+        layer(x)  # the first call of a shape makes the workspace
+        assert layer.dot_calls == 1
+        got = _native.linear(layer.__dict__, x)
+        assert got is not None and got.shape == shape[:-1] + (200,) and got.dtype == dtype and layer.dot_calls == 2
+        got_strided = _native.linear(layer.__dict__, strided)
+        x2 = x.clone()
+        got2 = layer(x2)
+        x2.mul_(2)
+        got3 = layer(x2)  # an in-place change is seen
+        monkeypatch.setenv("BSI_LINEAR_ONE_CALL", "0")
+        monkeypatch.setenv("BSI_FUSED_LINEAR", "0")
+        assert _native.linear(layer.__dict__, x) is None  # a switch is set
+        assert torch.equal(got, layer(x)) and torch.equal(got2, got) and torch.equal(got_strided, layer(strided))
+        assert torch.equal(got3, layer(x2))
+    assert not layer(x.requires_grad_()).requires_grad
+
+
+def test_calls_it_leaves_alone(ops):
+    from bsipytorch_amd import _native
+    from bsipytorch_amd.linear import BSIQuantizedLinear
+
+    layer = BSIQuantizedLinear(torch.nn.Linear(256, 64).cuda(), 2, 0.5)
+    x = torch.randn(8, 256, device="cuda")
+    layer(x)
+    assert _native.linear(layer.__dict__, x) is not None
+    for other in (x.cpu(), x[:0], x.double(), x[:, :128].contiguous()):
+        assert _native.linear(layer.__dict__, other) is None
+    layer.bias = layer.bias.cpu()
+    assert _native.linear(layer.__dict__, x) is None
+    ops._reset_flag_cache()
+    assert _native.linear(layer.__dict__, x) is None  # the flags have not been read yet
+    with pytest.raises(RuntimeError, match="Word count mismatch"):
+        ops.batch_dot_product_multiquery_cuda_batch_caps(ops.build_bsi_queries_cuda_batch_packed(x[:, :128].contiguous(), 2),
+                                                         layer._bsi_keys_cuda)
+
+
+def test_threads_on_one_stream(ops):
+    from bsipytorch_amd.linear import BSIQuantizedLinear
+
+    torch.manual_seed(4)
+    layers = [BSIQuantizedLinear(torch.nn.Linear(512, 256).cuda(), 2, 0.5) for _ in range(4)]
+    xs = [torch.randn(64, 512, device="cuda") for _ in range(4)]
+    with torch.no_grad():
+        want = [layer(x).clone() for layer, x in zip(layers, xs)]
+    wrong = []
+
+    def work(i):
+        with torch.no_grad():
+            for _ in range(200):
+                if not torch.equal(layers[i](xs[i]), want[i]):
+                    wrong.append(i)
+
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(4)]
+    [t.start() for t in threads]
+    [t.join() for t in threads]
+    assert not wrong
