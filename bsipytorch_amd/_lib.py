@@ -85,6 +85,8 @@ PROTOTYPES = {
     "bsi_hip_dot_weighted": [_vp, _vp, _i, _i, _vp, _i, _vp, _i, _i64, _i64, _vp, _f, _i64, _vp, _vp],
     "bsi_hip_dot_weighted_f64": [_vp, _vp, _i, _i, _vp, _i, _vp, _i, _i64, _i64, _vp, _i64, _vp, _vp],
     "bsi_hip_quantize_trunc_to_int64": [_vp, _i, _i64, _f, _vp, _vp],
+    "bsi_hip_scalar_query_max_elems": [],
+    "bsi_hip_scalar_query_dot": [_vp, _i64, _i, _d, _vp, _vp, _vp, _i, _i64, _vp, _vp, ctypes.POINTER(_f), ctypes.POINTER(_f), _vp],
     "bsi_hip_dot_timed": [_vp, _vp, _vp, _i, _i, _i, _vp, _i, _vp, _i, _i64, _i64, _f, _i64, _vp, _i, _vp, _sz, _i,
                           ctypes.POINTER(_f), _vp],
     "bsi_hip_probe_valu_popcount": [ctypes.POINTER(_d), _vp],
@@ -106,6 +108,7 @@ _RESTYPES = {
     "bsi_hip_linear_workspace_bytes": _sz,
     "bsi_hip_dot_digits_workspace_bytes": _sz,
     "bsi_hip_int8_tiled_bytes": _sz,
+    "bsi_hip_scalar_query_max_elems": _i64,
 }
 
 

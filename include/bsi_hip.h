@@ -72,6 +72,18 @@ int bsi_hip_quantize_round_to_int64(const void* x_device, int dtype, int64_t tot
 int bsi_hip_quantize_trunc_to_int64(const void* x_device, int dtype, int64_t total, float factor, int64_t* out,
                                     void* stream);
 
+/* One vector against prebuilt decimal keys (batch_dot_product_prebuilt, bsiFunctions.cpp:651-701) in two launches and one
+ * wait: x [d] float32 is built in decimal mode on the device (slice count from its largest magnitude), then
+ * out[r] = the exact integer dot with key row r (canonical planes B [R, Sb, W64], slice weights Bw [R, Sb]) as float64.
+ * info: {slices, whether a value is negative, words the slices take in stored form at `threshold`, run-length coded
+ * slices}.  out [R] and info [4] may be pinned host memory (they are complete when the call returns); workspace:
+ * 64 * ceil(d / 64) + 4 words of device memory.  build_ms / dot_ms: device-event times of the two launches.
+ * d at most bsi_hip_scalar_query_max_elems(). */
+int64_t bsi_hip_scalar_query_max_elems(void);
+int bsi_hip_scalar_query_dot(const float* x_device, int64_t d, int decimal_places, double threshold, uint64_t* workspace_device,
+                             const uint64_t* B, const float* Bw, int Sb, int64_t R, double* out, int64_t* info, float* build_ms,
+                             float* dot_ms, void* stream);
+
 /* Per-row / per-(row, 256-element chunk) shift and power-of-two scale from already rounded ints.
  * Replace launch_compute_row_shift_scale / launch_compute_chunk_shift_scale
  * (bsi_cuda_kernels_quant.cuh:670-700). shifts/scales are [Q] or [Q, chunks]. */
