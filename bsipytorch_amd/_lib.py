@@ -48,6 +48,7 @@ PROTOTYPES = {
     "bsi_hip_slice_popcount_sum": [_vp, _i, _i, _vp, _vp],
     "bsi_hip_compress_flags_from_density": [_vp, _i, _i, _d, _vp, _vp],
     "bsi_hip_ewah_size": [_vp, _i, _i, _vp, _vp, _vp],
+    "bsi_hip_ewah_measure": [_vp, _i, _i, _d, _vp, _vp, _vp, _vp, _vp],
     "bsi_hip_ewah_emit": [_vp, _i, _i, _vp, _vp, _vp, _vp, _vp],
     "bsi_hip_ewah_decompress": [_vp, _i, _i, _vp, _vp],
     "bsi_hip_ewah_decompress_batch": [_vp, _vp, _vp, _i, _i, _vp, _vp],

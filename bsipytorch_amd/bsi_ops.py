@@ -463,8 +463,9 @@ def warm_query_build_caches(Q: int) -> None:
     _warmed_query_caches.add(done)
 
 
-def _build_query_batch(q2d: torch.Tensor, decimal_places: int) -> PrebuiltBSIQueryBatchCUDA:
-    """bsi_vector_cuda.cpp:971-1064 (queries): chunk scales iff the flag is on and W64 % 4 == 0."""
+def _build_query_batch(q2d: torch.Tensor, decimal_places: int, want_ints8: bool = True) -> PrebuiltBSIQueryBatchCUDA:
+    """bsi_vector_cuda.cpp:971-1064 (queries): chunk scales iff the flag is on and W64 % 4 == 0.  ``want_ints8=False``
+    leaves the int8 image out (a batch whose planes are encoded right away)."""
     f = _flags()
     dev = _device()
     x = _as_build_input(q2d, dev)
@@ -492,7 +493,11 @@ def _build_query_batch(q2d: torch.Tensor, decimal_places: int) -> PrebuiltBSIQue
         if f["debug"]:
             print(f"[BSI_HIP] build_bsi_queries_cuda_batch_data: Q={Q} slices={S} words_per_slice={W}")
         return h
-    words, _shifts, scales, ints8 = _build_fixed(x, decimal_places, f["bits_q"], chunk_scale, want_ints8=True)
+    built = _native.build(x, int(decimal_places), True, want_ints8)  # None: a call or configuration it does not serve
+    if built is not None:
+        words, scales, ints8 = built
+    else:
+        words, _shifts, scales, ints8 = _build_fixed(x, decimal_places, f["bits_q"], chunk_scale, want_ints8)
     if prof:
         e1.record()
         e1.synchronize()
@@ -593,26 +598,15 @@ def build_bsi_query_cuda(q: torch.Tensor, decimal_places: int, compress_threshol
 
 
 def ewah_compress_slices(words2d: torch.Tensor, compress_threshold: float):
-    """Density flags + size pass + exclusive scan + emit pass for ``[S, W]`` words
-    (bsi_vector_cuda.cpp:896-951).  Returns (comp_words, comp_off int64 [S], comp_len int32 [S], flags)."""
-    S, W = words2d.shape
-    dev = words2d.device
-    st = _stream()
-    counts = torch.empty((S,), dtype=torch.int64, device=dev)
-    flags = torch.empty((S,), dtype=torch.int32, device=dev)
-    sizes = torch.empty((S,), dtype=torch.int64, device=dev)
-    check(lib.bsi_hip_slice_popcount_sum(words2d.data_ptr(), S, W, counts.data_ptr(), st), "bsi_hip_slice_popcount_sum")
-    check(lib.bsi_hip_compress_flags_from_density(counts.data_ptr(), S, W, float(compress_threshold),
-                                                  flags.data_ptr(), st), "bsi_hip_compress_flags_from_density")
-    check(lib.bsi_hip_ewah_size(words2d.data_ptr(), S, W, flags.data_ptr(), sizes.data_ptr(), st), "bsi_hip_ewah_size")
-    inclusive = sizes.cumsum(0)
-    total = int(inclusive[-1].item()) if S > 0 else 0
-    comp_off = (inclusive - sizes).contiguous()
-    comp_words = torch.empty((max(total, 1),), dtype=torch.int64, device=dev)
-    comp_len = torch.empty((S,), dtype=torch.int32, device=dev)
-    check(lib.bsi_hip_ewah_emit(words2d.data_ptr(), S, W, flags.data_ptr(), comp_off.data_ptr(),
-                                comp_words.data_ptr(), comp_len.data_ptr(), st), "bsi_hip_ewah_emit")
-    return comp_words[:total], comp_off, comp_len, flags
+    """Density flags and stream lengths, their exclusive scan, and the emit pass for ``[S, W]`` words
+    (bsi_vector_cuda.cpp:896-951); the host waits for the total length only.  Returns (comp_words, comp_off int64 [S], comp_len int32 [S], flags)."""
+    if words2d.shape[0] == 0:
+        none = torch.empty((0,), dtype=torch.int64, device=words2d.device)
+        return none, none.clone(), none.to(torch.int32), none.to(torch.int32)
+    streams = _native.ewah_streams(words2d.contiguous(), float(compress_threshold))
+    _check(streams is not None, "ewah_compress_slices: the words must be int64 on the current device, outside a graph capture "
+                                "(the total length is read back)")
+    return streams
 
 
 def build_bsi_query_cuda_hybrid(q: torch.Tensor, decimal_places: int, compress_threshold: float = 0.2):
@@ -644,7 +638,7 @@ def build_bsi_queries_cuda_batch_hybrid(q2d: torch.Tensor, decimal_places: int, 
     _check(q2d.dim() == 2, "q must be 2D [Q, d]")
     f = _flags()
     _check(2 <= f["bits_q"] <= 8, "the hybrid query batch needs fixed-bit queries of 2 to 8 bits")
-    b = _build_query_batch(q2d, int(decimal_places))
+    b = _build_query_batch(q2d, int(decimal_places), want_ints8=False)
     Q, Sa, W = b.words.shape
     _check(Q > 0, "Empty query batch")
     comp_words, comp_off, comp_len, flags = ewah_compress_slices(b.words.view(Q * Sa, W), float(compress_threshold))
@@ -1339,6 +1333,10 @@ def batch_dot_product_multiquery_cuda_batch_caps(query_batch_cap, keyset_cuda_ca
     if isinstance(query_batch_cap, PrebuiltBSIQueryBatchHybridCUDA):
         # the batched hybrid form: EWAH streams, decoded in the dot's load stage
         hb = query_batch_cap
+        if bias is None:
+            out = _native.dot_streams(hb, keys)
+            if out is not None:
+                return out, 0, 0.0, 0.0
         _check(hb.W == keys.W, "Word count mismatch between query batch and keys")
         _check(keys.num_keys > 0, "Empty keys")
         _check(hb.decimals == keys.decimals, f"Decimal mismatch between queries and keys: q={hb.decimals} k={keys.decimals}")
@@ -1514,8 +1512,11 @@ def debug_quantize_int64_cpu(values: torch.Tensor, decimal_places: int) -> torch
 
 # The native host path reads these on every call, so what the functions above keep stays the one copy.
 _native.bind({name: ctypes.cast(getattr(lib, name), ctypes.c_void_p).value
-              for name in ("bsi_hip_linear_few_rows_out", "bsi_hip_linear_out", "bsi_hip_linear_workspace_bytes", "bsi_hip_dot")},
-             {"keys_type": PrebuiltBSIKeysCUDA, "batch_type": PrebuiltBSIQueryBatchCUDA, "linear_ws": _linear_ws,
+              for name in ("bsi_hip_linear_few_rows_out", "bsi_hip_linear_out", "bsi_hip_linear_workspace_bytes", "bsi_hip_dot",
+                           "bsi_hip_build_fixed", "bsi_hip_ewah_measure", "bsi_hip_ewah_emit", "bsi_hip_dot_ewah_batch",
+                           "bsi_hip_dot_ewah_batch_workspace_bytes")},
+             {"keys_type": PrebuiltBSIKeysCUDA, "batch_type": PrebuiltBSIQueryBatchCUDA,
+              "hybrid_type": PrebuiltBSIQueryBatchHybridCUDA, "linear_ws": _linear_ws,
               "reserved": _reserved_linear_shapes, "warmed": _warmed_query_caches, "split_shapes": _split_shapes,
               "attach": attach_split_scratch, "check": check},
              FUSED_LINEAR_MAX_ROWS, _FEW_ROWS_MAX_Q, _SPLIT_MIN_Q, FUSED_LINEAR_QUERY_LDS_BYTES)

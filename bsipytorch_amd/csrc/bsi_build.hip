@@ -302,7 +302,7 @@ __global__ __launch_bounds__(kBlock) void build_fixed_chunk_fast_kernel(
         }
         image = chunk_image_dword(image, cl);
         if (lane == 0) {
-            shifts[item] = shift;
+            if (shifts != nullptr) shifts[item] = shift;
             scales[item] = static_cast<float>(1ULL << shift);
         }
         if (ints8 != nullptr) reinterpret_cast<uint32_t*>(ints8)[static_cast<size_t>(item) * (BSI_CHUNK_ELEMS / 4) + lane] = image;
@@ -433,7 +433,7 @@ __global__ __launch_bounds__(kBlock) void build_fixed_row_fast_kernel(const T* _
         shift = compute_shift(m64, 0.0, 1, slices, 0.0f);
     }
     if (threadIdx.x == 0) {
-        shifts[row] = shift;
+        if (shifts != nullptr) shifts[row] = shift;
         scales[row] = static_cast<float>(1ULL << shift);
     }
     const QuantRange range = quant_range(slices);
@@ -839,7 +839,7 @@ extern "C" int bsi_hip_build_fixed(const void* x, int dtype, int64_t Q, int64_t 
     // The register-resident kernels quantise in float32: 10^dec an integer of at most 127 (0 to 2 decimal places), at most
     // 8 slices, no clipping; their item numbers are 32-bit.
     const bool fast = scale_int != 0 && fixed_bits <= 8 && !(clip_k > 0.0f) && items <= 0x7fffff00LL && Q <= 0x7fffffffLL;
-    BSI_REQUIRE(x && shifts && scales && (words || (fast && ints8)), "null pointer");
+    BSI_REQUIRE(x && scales && (shifts || fast) && (words || (fast && ints8)), "null pointer");
     const float scale = static_cast<float>(scale_int);
     unsigned long long* const words64 = reinterpret_cast<unsigned long long*>(words);
     hipStream_t st = as_stream(stream);

@@ -57,6 +57,52 @@ __global__ void ewah_emit_kernel(const unsigned long long* __restrict__ words, i
     if (lane == 0) out_len[s] = static_cast<int>(n);
 }
 
+// Density flag and stream length of every slice in one pass (the words of a slice are counted, then measured from the
+// cache): what slice_popcount, compress_flags and ewah_size give in three launches.  One wave per slice.
+__global__ void ewah_measure_kernel(const unsigned long long* __restrict__ words, int S, int W, double threshold,
+                                    int* __restrict__ flags, int* __restrict__ lens) {
+    const int lane = threadIdx.x & (BSI_WAVE - 1);
+    const int64_t s = static_cast<int64_t>(blockIdx.x) * (kEwahBlock / BSI_WAVE) + (threadIdx.x >> 6);
+    if (s >= S) return;
+    const unsigned long long* base = words + static_cast<size_t>(s) * W;
+    unsigned long long count = 0ULL;
+    for (int w = lane; w < W; w += BSI_WAVE) count += static_cast<unsigned long long>(__popcll(base[w]));
+    const int flag = compress_flag(wave_sum_u64(count), W, threshold);
+    const unsigned long long n = flag ? ewah_encode_wave(base, W, 1, nullptr, lane) : static_cast<unsigned long long>(W > 0 ? W + 1 : 0);
+    if (lane == 0) {
+        flags[s] = flag;
+        lens[s] = static_cast<int>(n);
+    }
+}
+
+// Exclusive sums of the stream lengths, and their total to the host: one workgroup, a run of slices per thread.  The
+// total is stored with system scope, so that a host that waits for it need not wait for the kernel to end.
+constexpr int kScanBlock = 1024;
+__global__ __launch_bounds__(kScanBlock) void ewah_offsets_kernel(const int* __restrict__ lens, int S, long long* __restrict__ off,
+                                                                  long long* __restrict__ total_host) {
+    __shared__ long long wave_sums[kScanBlock / BSI_WAVE];
+    const int tid = threadIdx.x, lane = tid & (BSI_WAVE - 1), wave = tid >> 6;
+    const int run = (S + kScanBlock - 1) / kScanBlock;
+    const int first = tid * run < S ? tid * run : S, last = first + run < S ? first + run : S;
+    long long sum = 0;
+    for (int s = first; s < last; ++s) sum += lens[s];
+    long long at = sum;  // inclusive over the wave
+#pragma unroll
+    for (int o = 1; o < BSI_WAVE; o <<= 1) {
+        const long long v = __shfl_up(at, o, BSI_WAVE);
+        if (lane >= o) at += v;
+    }
+    if (lane == BSI_WAVE - 1) wave_sums[wave] = at;
+    __syncthreads();
+    for (int w = 0; w < wave; ++w) at += wave_sums[w];
+    if (tid == kScanBlock - 1) __hip_atomic_store(total_host, at, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+    at -= sum;
+    for (int s = first; s < last; ++s) {
+        off[s] = at;
+        at += lens[s];
+    }
+}
+
 // one wave per stream
 __global__ void ewah_decompress_batch_kernel(const unsigned long long* __restrict__ comp,
                                              const long long* __restrict__ off, const int* __restrict__ len, int S,
@@ -109,6 +155,19 @@ extern "C" int bsi_hip_ewah_size(const uint64_t* words, int S, int W, const int3
                        reinterpret_cast<const unsigned long long*>(words), S, W, flags,
                        reinterpret_cast<unsigned long long*>(sizes));
     BSI_LAUNCH_CHECK("ewah_size_kernel");
+    return BSI_OK;
+}
+
+extern "C" int bsi_hip_ewah_measure(const uint64_t* words, int S, int W, double threshold, int32_t* flags, int32_t* lens,
+                                    int64_t* off, int64_t* total_host, void* stream) {
+    BSI_REQUIRE(S >= 1 && W >= 0, "bad shape");
+    BSI_REQUIRE(words && flags && lens && off && total_host, "null pointer");
+    hipLaunchKernelGGL(ewah_measure_kernel, dim3((S + 3) / 4), dim3(kEwahBlock), 0, as_stream(stream),
+                       reinterpret_cast<const unsigned long long*>(words), S, W, threshold, flags, lens);
+    BSI_LAUNCH_CHECK("ewah_measure_kernel");
+    hipLaunchKernelGGL(ewah_offsets_kernel, dim3(1), dim3(kScanBlock), 0, as_stream(stream), lens, S,
+                       reinterpret_cast<long long*>(off), reinterpret_cast<long long*>(total_host));
+    BSI_LAUNCH_CHECK("ewah_offsets_kernel");
     return BSI_OK;
 }
 

@@ -6,13 +6,14 @@
 // handles' attributes on every call, so nothing can go stale -- and return None for any call they do not serve; the Python
 // path behind them then serves it or raises its errors.  Launches recorded into a graph always take that path.
 #include <torch/csrc/autograd/python_variable.h>
+#include <ATen/EmptyTensor.h>
 #include <ATen/hip/EmptyTensor.h>
 #include <c10/hip/HIPFunctions.h>
 #include <c10/hip/HIPGraphsC10Utils.h>
 #include <c10/hip/HIPStream.h>
 
+#include <chrono>
 #include <cstring>
-#include <unordered_map>
 
 #include "../../include/bsi_hip.h"
 
@@ -26,11 +27,16 @@ struct Library {
     decltype(&bsi_hip_linear_out) linear_out;
     decltype(&bsi_hip_linear_workspace_bytes) linear_workspace_bytes;
     decltype(&bsi_hip_dot) dot;
+    decltype(&bsi_hip_build_fixed) build_fixed;
+    decltype(&bsi_hip_ewah_measure) ewah_measure;
+    decltype(&bsi_hip_ewah_emit) ewah_emit;
+    decltype(&bsi_hip_dot_ewah_batch) dot_ewah_batch;
+    decltype(&bsi_hip_dot_ewah_batch_workspace_bytes) dot_ewah_batch_workspace_bytes;
 } lib;
 
 // The Python side's state (bind()): types of the handles, the workspaces and what is known about shapes.
 struct Shared {
-    PyObject *keys_type, *batch_type;      // PrebuiltBSIKeysCUDA, PrebuiltBSIQueryBatchCUDA
+    PyObject *keys_type, *batch_type, *hybrid_type;  // PrebuiltBSIKeysCUDA, PrebuiltBSIQueryBatchCUDA, ...HybridCUDA
     PyObject *linear_ws;                   // device index -> {"bytes", "eager": {stream: (buffer, [key, input])}, ...}
     PyObject *reserved, *warmed;           // shapes whose workspace and constants a later capture will find
     PyObject *split_shapes, *attach;       // (device, Q, R, W) -> whether the dot splits; attach_split_scratch
@@ -49,7 +55,8 @@ struct Config {
 #define NAMES(X)                                                                                                          \
     X(_bsi_keys_cuda) X(_fused) X(_next_bsi_layer) X(_buffers) X(bias) X(collect_stats) X(decimalPlaces) X(fixed) X(Sb) X(W) X(d) \
     X(num_keys) X(decimals) X(layout) X(words) X(ints8) X(ints8_tiled) X(slice_weights) X(bytes) X(eager) X(dot_calls)      \
-    X(build_calls) X(dot_query_vectors_total) X(dot_output_elements_total) X(chunk_scales) X(row_scales) X(keys)
+    X(build_calls) X(dot_query_vectors_total) X(dot_output_elements_total) X(chunk_scales) X(row_scales) X(keys) \
+    X(comp_words) X(comp_off) X(comp_len) X(Sa) X(Q)
 struct Names {
 #define X(n) PyObject* n;
     NAMES(X)
@@ -97,6 +104,8 @@ struct Holder {  // an owned reference
     Holder(const Holder&) = delete;
     Holder& operator=(const Holder&) = delete;
 };
+
+bool capturing() { return c10::hip::currentStreamCaptureStatusMayInitCtx() != c10::hip::CaptureStatus::None; }
 
 int dtype_code(at::ScalarType t) {
     switch (t) {
@@ -243,7 +252,7 @@ PyObject* linear(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     // half-precision output: the kernels that have it (bsi_ops.can_output_half)
     const bool six_tiled = k.Sb == 6 && k.layout == BSI_LAYOUT_TILED16;
     if (in_code != BSI_DTYPE_F32 && !(rows > shared.stream_max ? k.ints8 != nullptr : six_tiled && chunks <= 32768)) Py_RETURN_NONE;
-    if (c10::hip::currentStreamCaptureStatusMayInitCtx() != c10::hip::CaptureStatus::None) Py_RETURN_NONE;
+    if (capturing()) Py_RETURN_NONE;
     const c10::hip::HIPStream stream = c10::hip::getCurrentHIPStream(device.index());
     hipStream_t const st = stream.stream();
 
@@ -370,9 +379,7 @@ PyObject* dot(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
         Py_RETURN_NONE;
     if (chunked ? (scales->dim() != 2 || scales->size(0) != Q || W % 4 != 0 || scales->size(1) != chunks) : scales->numel() != Q)
         Py_RETURN_NONE;
-    if (c10::hip::currentStreamCaptureStatusMayInitCtx() != c10::hip::CaptureStatus::None ||
-        !split_scratch(device.index(), Q, k.R, W))
-        Py_RETURN_NONE;
+    if (capturing() || !split_scratch(device.index(), Q, k.R, W)) Py_RETURN_NONE;
     hipStream_t const st = c10::hip::getCurrentHIPStream(device.index()).stream();
     at::Tensor out = at::detail::empty_cuda({Q, k.R}, at::kFloat, device, std::nullopt);
     int layout = 0, rc = BSI_OK;
@@ -385,6 +392,134 @@ PyObject* dot(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
                  scale_inv(decimals, k.decimals), k.R, out.data_ptr<float>(), nullptr, config.core, nullptr, 0, st);
     Py_END_ALLOW_THREADS
     if (rc != BSI_OK) return fail_status(rc, "bsi_hip_dot");
+    return THPVariable_Wrap(std::move(out));
+    END_HANDLE_TH_ERRORS
+}
+
+// build(x, decimals, planes, image) -> (words [Q, bits, W] or None, chunk or row scales, int8 image or None), or None: the
+// fixed-bit query build of a contiguous [Q, d] batch on the current device.
+PyObject* build(PyObject*, PyObject* args) {
+    PyObject* o = nullptr;
+    int decimals = 0, planes = 0, image = 0;
+    if (!PyArg_ParseTuple(args, "Oipp", &o, &decimals, &planes, &image)) return nullptr;
+    if (!config.on || !THPVariable_CheckExact(o) || decimals < 0 || decimals > 2) Py_RETURN_NONE;
+    HANDLE_TH_ERRORS
+    const at::Tensor& x = THPVariable_Unpack(o);
+    const int code = dtype_code(x.scalar_type());
+    if (!x.is_cuda() || code < 0 || x.dim() != 2 || x.numel() == 0 || !x.is_contiguous() ||
+        x.device().index() != c10::hip::current_device() || capturing())
+        Py_RETURN_NONE;
+    const at::Device device = x.device();
+    const int64_t Q = x.size(0), d = x.size(1), W = (d + 63) / 64, chunks = (d + 255) / 256;
+    const bool chunked = W % 4 == 0;
+    hipStream_t const st = c10::hip::getCurrentHIPStream(device.index()).stream();
+    at::Tensor words, ints8, scales;
+    if (planes) words = at::detail::empty_cuda({Q, config.bits, W}, at::kLong, device, std::nullopt);
+    if (image) ints8 = at::detail::empty_cuda({Q, chunks * 256}, at::kChar, device, std::nullopt);
+    scales = chunked ? at::detail::empty_cuda({Q, chunks}, at::kFloat, device, std::nullopt)
+                     : at::detail::empty_cuda({Q}, at::kFloat, device, std::nullopt);
+    int rc = BSI_OK;
+    Py_BEGIN_ALLOW_THREADS
+    rc = lib.build_fixed(x.const_data_ptr(), code, Q, d, decimals, config.bits, chunked ? 1 : 0, 0.0f,
+                         planes ? static_cast<uint64_t*>(words.data_ptr()) : nullptr, nullptr, static_cast<float*>(scales.data_ptr()),
+                         image ? static_cast<int8_t*>(ints8.data_ptr()) : nullptr, st);
+    Py_END_ALLOW_THREADS
+    if (rc != BSI_OK) return fail_status(rc, "bsi_hip_build_fixed");
+    Holder w(THPVariable_Wrap(std::move(words))), s(THPVariable_Wrap(std::move(scales))), i(THPVariable_Wrap(std::move(ints8)));
+    return PyTuple_Pack(3, w.p, s.p, i.p);
+    END_HANDLE_TH_ERRORS
+}
+
+// ewah_streams(words [S, W], threshold) -> (stream words, offsets, lengths, flags) of the slices' EWAH encoding, or None.
+PyObject* ewah_streams(PyObject*, PyObject* args) {
+    PyObject* o = nullptr;
+    double threshold = 0.0;
+    if (!PyArg_ParseTuple(args, "Od", &o, &threshold)) return nullptr;
+    if (!THPVariable_CheckExact(o)) Py_RETURN_NONE;
+    HANDLE_TH_ERRORS
+    const at::Tensor& words = THPVariable_Unpack(o);
+    if (!words.is_cuda() || words.scalar_type() != at::kLong || words.dim() != 2 || words.size(0) < 1 || words.size(0) > INT32_MAX ||
+        words.size(1) > INT32_MAX || !words.is_contiguous() || words.device().index() != c10::hip::current_device() || capturing())
+        Py_RETURN_NONE;
+    const at::Device device = words.device();
+    const int S = static_cast<int>(words.size(0)), W = static_cast<int>(words.size(1));
+    hipStream_t const st = c10::hip::getCurrentHIPStream(device.index()).stream();
+    at::Tensor flags = at::detail::empty_cuda({S}, at::kInt, device, std::nullopt);
+    at::Tensor lens = at::detail::empty_cuda({S}, at::kInt, device, std::nullopt);
+    at::Tensor off = at::detail::empty_cuda({S}, at::kLong, device, std::nullopt);
+    at::Tensor total_host = at::detail::empty_cpu({1}, at::kLong, /*pin_memory=*/true);
+    volatile int64_t* const total = static_cast<volatile int64_t*>(total_host.data_ptr());
+    *total = -1;
+    const uint64_t* const w = static_cast<const uint64_t*>(words.const_data_ptr());
+    int rc = BSI_OK;
+    Py_BEGIN_ALLOW_THREADS
+    rc = lib.ewah_measure(w, S, W, threshold, static_cast<int32_t*>(flags.data_ptr()), static_cast<int32_t*>(lens.data_ptr()),
+                          static_cast<int64_t*>(off.data_ptr()), const_cast<int64_t*>(total), st);
+    // the total arrives while its kernel still runs; the stream is waited for only if it is long in coming
+    const auto until = std::chrono::steady_clock::now() + std::chrono::microseconds(200);
+    while (rc == BSI_OK && *total < 0 && std::chrono::steady_clock::now() < until) {}
+    if (rc == BSI_OK && *total < 0 && hipStreamSynchronize(st) != hipSuccess) rc = BSI_ERR_HIP;
+    Py_END_ALLOW_THREADS
+    if (rc != BSI_OK) return fail_status(rc, "bsi_hip_ewah_measure");
+    at::Tensor streams = at::detail::empty_cuda({static_cast<int64_t>(*total)}, at::kLong, device, std::nullopt);
+    if (streams.numel() > 0) {
+        Py_BEGIN_ALLOW_THREADS
+        rc = lib.ewah_emit(w, S, W, static_cast<const int32_t*>(flags.data_ptr()), static_cast<const uint64_t*>(off.data_ptr()),
+                           static_cast<uint64_t*>(streams.data_ptr()), static_cast<int32_t*>(lens.data_ptr()), st);
+        Py_END_ALLOW_THREADS
+        if (rc != BSI_OK) return fail_status(rc, "bsi_hip_ewah_emit");
+    }
+    Holder a(THPVariable_Wrap(std::move(streams))), b(THPVariable_Wrap(std::move(off))), c(THPVariable_Wrap(std::move(lens))),
+        f(THPVariable_Wrap(std::move(flags)));
+    return PyTuple_Pack(4, a.p, b.p, c.p, f.p);
+    END_HANDLE_TH_ERRORS
+}
+
+// dot_streams(hybrid_batch, keyset) -> the float32 scores, or None: the dot of a batch kept as EWAH streams.
+PyObject* dot_streams(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+    if (nargs != 2) {
+        PyErr_SetString(PyExc_TypeError, "dot_streams(hybrid_batch, keyset)");
+        return nullptr;
+    }
+    if (!config.on || reinterpret_cast<PyObject*>(Py_TYPE(args[0])) != shared.hybrid_type) Py_RETURN_NONE;
+    HANDLE_TH_ERRORS
+    Holder attrs(PyObject_GenericGetDict(args[0], nullptr));
+    if (attrs.p == nullptr) return nullptr;
+    const at::Tensor* const streams = get_tensor(attrs.p, names.comp_words);
+    const at::Tensor* const off = get_tensor(attrs.p, names.comp_off);
+    const at::Tensor* const len = get_tensor(attrs.p, names.comp_len);
+    const at::Tensor* const chunk_scales = get_tensor(attrs.p, names.chunk_scales);
+    const at::Tensor* const row_scales = get_tensor(attrs.p, names.row_scales);
+    const bool chunked = chunk_scales != nullptr && chunk_scales->numel() > 0;
+    const at::Tensor* const scales = chunked ? chunk_scales : row_scales;
+    int64_t Q = 0, Sa = 0, W = 0, decimals = 0;
+    if (streams == nullptr || off == nullptr || len == nullptr || scales == nullptr || !get_int(attrs.p, names.Q, &Q) ||
+        !get_int(attrs.p, names.Sa, &Sa) || !get_int(attrs.p, names.W, &W) || !get_int(attrs.p, names.decimals, &decimals))
+        Py_RETURN_NONE;
+    const at::Device device = streams->device();
+    const int64_t chunks = (W + 3) / 4;
+    Keys k;
+    if (!streams->is_cuda() || device.index() != c10::hip::current_device() || !read_keys(args[1], device, &k) || k.W != W ||
+        k.decimals != decimals || decimals < 0 || Q <= 0 || Sa < 2 || Sa > 8 || off->numel() != Q * Sa || len->numel() != Q * Sa ||
+        scales->device() != device || !scales->is_contiguous() || (chunked && W % 4 != 0) ||
+        scales->numel() != (chunked ? Q * chunks : Q) || capturing() || !split_scratch(device.index(), Q, k.R, W))
+        Py_RETURN_NONE;
+    hipStream_t const st = c10::hip::getCurrentHIPStream(device.index()).stream();
+    at::Tensor out = at::detail::empty_cuda({Q, k.R}, at::kFloat, device, std::nullopt);
+    const size_t need = lib.dot_ewah_batch_workspace_bytes(Q, static_cast<int>(W));
+    at::Tensor ws = at::detail::empty_cuda({static_cast<int64_t>(need)}, at::kByte, device, std::nullopt);
+    int layout = 0, rc = BSI_OK;
+    size_t bytes = 0;
+    const void* const operand = key_operand(k, Q, &layout, &bytes);
+    Py_BEGIN_ALLOW_THREADS
+    rc = lib.dot_ewah_batch(static_cast<const uint64_t*>(streams->const_data_ptr()), static_cast<const int64_t*>(off->const_data_ptr()),
+                            static_cast<const int32_t*>(len->const_data_ptr()), static_cast<int>(Sa), static_cast<int>(W),
+                            static_cast<const float*>(scales->const_data_ptr()), chunked ? static_cast<int>(chunks) : 1,
+                            static_cast<const uint64_t*>(operand), layout, static_cast<const float*>(k.weights->const_data_ptr()),
+                            static_cast<int>(k.Sb), k.R, Q, scale_inv(decimals, k.decimals), k.R, nullptr,
+                            static_cast<float*>(out.data_ptr()), nullptr, ws.data_ptr(), need, st);
+    Py_END_ALLOW_THREADS
+    if (rc != BSI_OK) return fail_status(rc, "bsi_hip_dot_ewah_batch");
     return THPVariable_Wrap(std::move(out));
     END_HANDLE_TH_ERRORS
 }
@@ -431,7 +566,11 @@ PyObject* bind(PyObject*, PyObject* args) {
     if (!PyArg_ParseTuple(args, "O!O!iiiL", &PyDict_Type, &entries, &PyDict_Type, &state, &few, &stream, &split, &lds)) return nullptr;
     if (!entry(entries, "bsi_hip_linear_few_rows_out", &lib.linear_few_rows_out) || !entry(entries, "bsi_hip_linear_out", &lib.linear_out) ||
         !entry(entries, "bsi_hip_linear_workspace_bytes", &lib.linear_workspace_bytes) || !entry(entries, "bsi_hip_dot", &lib.dot) ||
+        !entry(entries, "bsi_hip_build_fixed", &lib.build_fixed) || !entry(entries, "bsi_hip_ewah_measure", &lib.ewah_measure) ||
+        !entry(entries, "bsi_hip_ewah_emit", &lib.ewah_emit) || !entry(entries, "bsi_hip_dot_ewah_batch", &lib.dot_ewah_batch) ||
+        !entry(entries, "bsi_hip_dot_ewah_batch_workspace_bytes", &lib.dot_ewah_batch_workspace_bytes) ||
         !take(state, "keys_type", &shared.keys_type) || !take(state, "batch_type", &shared.batch_type) ||
+        !take(state, "hybrid_type", &shared.hybrid_type) ||
         !take(state, "linear_ws", &shared.linear_ws) || !take(state, "reserved", &shared.reserved) ||
         !take(state, "warmed", &shared.warmed) || !take(state, "split_shapes", &shared.split_shapes) ||
         !take(state, "attach", &shared.attach) || !take(state, "check", &shared.check))
@@ -447,6 +586,9 @@ PyMethodDef methods[] = {
     {"bind", bind, METH_VARARGS, nullptr},
     {"configure", configure, METH_VARARGS, nullptr},
     {"build_key", build_key, METH_VARARGS, nullptr},
+    {"build", build, METH_VARARGS, nullptr},
+    {"ewah_streams", ewah_streams, METH_VARARGS, nullptr},
+    {"dot_streams", reinterpret_cast<PyCFunction>(reinterpret_cast<void*>(dot_streams)), METH_FASTCALL, nullptr},
     {"linear", reinterpret_cast<PyCFunction>(reinterpret_cast<void*>(linear)), METH_FASTCALL, nullptr},
     {"dot", reinterpret_cast<PyCFunction>(reinterpret_cast<void*>(dot)), METH_FASTCALL, nullptr},
     {nullptr, nullptr, 0, nullptr},

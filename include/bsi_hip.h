@@ -140,7 +140,7 @@ int bsi_hip_pack_bits_batch(const int64_t* ints_device, int64_t Q, int64_t d, in
  * else [Q].  Optional extra output `ints8_device` (may be NULL): the quantised values as int8
  * [Q, chunks*256] in the MFMA core's in-chunk element order (bsi_hip_planes_to_int8 gives the same).
  * words_device may be NULL when ints8_device is given, fixed_bits <= 8, clip_k <= 0 and decimal_places is 0, 1 or 2: the
- * planes are then not written.
+ * planes are then not written.  (shifts_device may be NULL under the same conditions.)
  * Replaces the host orchestration bsi_cuda_build_fixed_query_words_fused
  * (bsi_vector_cuda.cpp:401-557) and, with chunk_scale = 0 and fixed_bits = 6, the key quantiser
  * + packer (bsi_vector_cuda.cpp:559-744, 1125-1141). */
@@ -168,6 +168,12 @@ int bsi_hip_compress_flags_from_density(const uint64_t* counts_device, int S, in
 /* sizes[s] = number of u64 the encoder emits for slice s.  Replaces launch_ewah_size (ewah.cuh:164-175). */
 int bsi_hip_ewah_size(const uint64_t* words_device, int S, int W, const int32_t* flags_device,
                       uint64_t* sizes_device, void* stream);
+/* The passes ahead of the emit pass in one call: density flags, stream lengths, their exclusive sums, and the total length
+ * into total_host (pinned host memory; valid once the stream has been waited for, or once it changes: it is written
+ * with system scope).  Replaces launch_slice_popcount_sum, launch_compress_flags_from_density, launch_ewah_size and the
+ * scan between them and the emit pass (bsi_vector_cuda.cpp:896-951). */
+int bsi_hip_ewah_measure(const uint64_t* words_device, int S, int W, double threshold, int32_t* flags_device,
+                         int32_t* lens_device, int64_t* off_device, int64_t* total_host, void* stream);
 /* Emit marker + literal words of every slice at off[s]; out_len[s] = words written.
  * Marker = run_bit | run_len << 1 | literal_count << 33.  Replaces launch_ewah_emit (ewah.cuh:234-247). */
 int bsi_hip_ewah_emit(const uint64_t* words_device, int S, int W, const int32_t* flags_device,
