@@ -595,7 +595,7 @@ extern "C" int bsi_hip_quantize_round_to_int64(const void* x, int dtype, int64_t
     BSI_REQUIRE(total >= 0, "total must be >= 0");
     if (total == 0) return BSI_OK;
     BSI_REQUIRE(x && out, "null pointer");
-    BSI_DISPATCH_DTYPE(dtype, hipLaunchKernelGGL(round_to_int64_kernel<T>, dim3(grid_elementwise(total)), dim3(kBlock),
+    BSI_DISPATCH_DTYPE(dtype, launch(round_to_int64_kernel<T>, dim3(grid_elementwise(total)), dim3(kBlock),
                                                  0, as_stream(stream), static_cast<const T*>(x), total, dec_scale,
                                                  reinterpret_cast<long long*>(out)));
     BSI_LAUNCH_CHECK("round_to_int64_kernel");
@@ -607,7 +607,7 @@ extern "C" int bsi_hip_quantize_trunc_to_int64(const void* x, int dtype, int64_t
     BSI_REQUIRE(total >= 0, "total must be >= 0");
     if (total == 0) return BSI_OK;
     BSI_REQUIRE(x && out, "null pointer");
-    BSI_DISPATCH_DTYPE(dtype, hipLaunchKernelGGL(trunc_to_int64_kernel<T>, dim3(grid_elementwise(total)), dim3(kBlock),
+    BSI_DISPATCH_DTYPE(dtype, launch(trunc_to_int64_kernel<T>, dim3(grid_elementwise(total)), dim3(kBlock),
                                                  0, as_stream(stream), static_cast<const T*>(x), total, factor,
                                                  reinterpret_cast<long long*>(out)));
     BSI_LAUNCH_CHECK("trunc_to_int64_kernel");
@@ -620,7 +620,7 @@ extern "C" int bsi_hip_compute_row_shift_scale(const int64_t* ints, int64_t Q, i
     if (Q == 0) return BSI_OK;
     BSI_REQUIRE(ints && shifts && scales, "null pointer");
     RoundedFromInts src{reinterpret_cast<const long long*>(ints)};
-    hipLaunchKernelGGL(row_shift_scale_kernel<RoundedFromInts>, dim3(static_cast<unsigned>(Q)), dim3(kBlock), 0,
+    launch(row_shift_scale_kernel<RoundedFromInts>, dim3(static_cast<unsigned>(Q)), dim3(kBlock), 0,
                        as_stream(stream), src, Q, d, fixed_bits, clip_k, shifts, scales);
     BSI_LAUNCH_CHECK("row_shift_scale_kernel");
     return BSI_OK;
@@ -632,7 +632,7 @@ extern "C" int bsi_hip_compute_chunk_shift_scale(const int64_t* ints, int64_t Q,
     if (Q == 0 || chunks == 0) return BSI_OK;
     BSI_REQUIRE(ints && shifts && scales, "null pointer");
     RoundedFromInts src{reinterpret_cast<const long long*>(ints)};
-    hipLaunchKernelGGL(chunk_shift_scale_kernel<RoundedFromInts>, dim3(grid_for(Q * chunks)), dim3(kBlock), 0,
+    launch(chunk_shift_scale_kernel<RoundedFromInts>, dim3(grid_for(Q * chunks)), dim3(kBlock), 0,
                        as_stream(stream), src, Q, d, chunks, fixed_bits, clip_k, shifts, scales);
     BSI_LAUNCH_CHECK("chunk_shift_scale_kernel");
     return BSI_OK;
@@ -644,7 +644,7 @@ extern "C" int bsi_hip_apply_row_shift_clamp(int64_t* ints, int64_t Q, int64_t d
     BSI_REQUIRE(fixed_bits >= 2 && fixed_bits <= 63, "fixed_bits must be in [2, 63]");
     if (Q == 0 || d == 0) return BSI_OK;
     BSI_REQUIRE(ints && shifts, "null pointer");
-    hipLaunchKernelGGL(apply_shift_clamp_kernel, dim3(grid_elementwise(Q * d)), dim3(kBlock), 0, as_stream(stream),
+    launch(apply_shift_clamp_kernel, dim3(grid_elementwise(Q * d)), dim3(kBlock), 0, as_stream(stream),
                        reinterpret_cast<long long*>(ints), Q * d, d, 0, shifts, -(1LL << (fixed_bits - 1)),
                        (1LL << (fixed_bits - 1)) - 1LL);
     BSI_LAUNCH_CHECK("apply_shift_clamp_kernel");
@@ -657,7 +657,7 @@ extern "C" int bsi_hip_apply_chunk_shift_clamp(int64_t* ints, int64_t Q, int64_t
     BSI_REQUIRE(fixed_bits >= 2 && fixed_bits <= 63, "fixed_bits must be in [2, 63]");
     if (Q == 0 || d == 0) return BSI_OK;
     BSI_REQUIRE(ints && shifts, "null pointer");
-    hipLaunchKernelGGL(apply_shift_clamp_kernel, dim3(grid_elementwise(Q * d)), dim3(kBlock), 0, as_stream(stream),
+    launch(apply_shift_clamp_kernel, dim3(grid_elementwise(Q * d)), dim3(kBlock), 0, as_stream(stream),
                        reinterpret_cast<long long*>(ints), Q * d, d, chunks, shifts, -(1LL << (fixed_bits - 1)),
                        (1LL << (fixed_bits - 1)) - 1LL);
     BSI_LAUNCH_CHECK("apply_shift_clamp_kernel");
@@ -672,7 +672,7 @@ extern "C" int bsi_hip_compute_row_shift_scale_from_input(const void* x, int dty
     BSI_REQUIRE(x && shifts && scales, "null pointer");
     BSI_DISPATCH_DTYPE(dtype, {
         RoundedFromInput<T> src{static_cast<const T*>(x), dec_scale};
-        hipLaunchKernelGGL(row_shift_scale_kernel<RoundedFromInput<T>>, dim3(static_cast<unsigned>(Q)), dim3(kBlock),
+        launch(row_shift_scale_kernel<RoundedFromInput<T>>, dim3(static_cast<unsigned>(Q)), dim3(kBlock),
                            0, as_stream(stream), src, Q, d, fixed_bits, clip_k, shifts, scales);
     });
     BSI_LAUNCH_CHECK("row_shift_scale_kernel");
@@ -687,7 +687,7 @@ extern "C" int bsi_hip_compute_chunk_shift_scale_from_input(const void* x, int d
     BSI_REQUIRE(x && shifts && scales, "null pointer");
     BSI_DISPATCH_DTYPE(dtype, {
         RoundedFromInput<T> src{static_cast<const T*>(x), dec_scale};
-        hipLaunchKernelGGL(chunk_shift_scale_kernel<RoundedFromInput<T>>, dim3(grid_for(Q * chunks)), dim3(kBlock), 0,
+        launch(chunk_shift_scale_kernel<RoundedFromInput<T>>, dim3(grid_for(Q * chunks)), dim3(kBlock), 0,
                            as_stream(stream), src, Q, d, chunks, fixed_bits, clip_k, shifts, scales);
     });
     BSI_LAUNCH_CHECK("chunk_shift_scale_kernel");
@@ -712,7 +712,7 @@ extern "C" int bsi_hip_quantize_shift_pack_row_batch(const void* x, int dtype, i
     const int groups = (words_per_slice + 3) / 4;
     BSI_DISPATCH_DTYPE(dtype, {
         RoundedFromInput<T> src{static_cast<const T*>(x), dec_scale};
-        hipLaunchKernelGGL((shift_pack_kernel<RoundedFromInput<T>, true>), dim3(grid_for(Q * groups)), dim3(kBlock), 0,
+        launch((shift_pack_kernel<RoundedFromInput<T>, true>), dim3(grid_for(Q * groups)), dim3(kBlock), 0,
                            as_stream(stream), src, Q, d, 0, slices, words_per_slice, fixed_bits, shifts,
                            reinterpret_cast<unsigned long long*>(words));
     });
@@ -732,7 +732,7 @@ extern "C" int bsi_hip_quantize_shift_pack_chunk_batch(const void* x, int dtype,
     const int groups = (words_per_slice + 3) / 4;
     BSI_DISPATCH_DTYPE(dtype, {
         RoundedFromInput<T> src{static_cast<const T*>(x), dec_scale};
-        hipLaunchKernelGGL((shift_pack_kernel<RoundedFromInput<T>, true>), dim3(grid_for(Q * groups)), dim3(kBlock), 0,
+        launch((shift_pack_kernel<RoundedFromInput<T>, true>), dim3(grid_for(Q * groups)), dim3(kBlock), 0,
                            as_stream(stream), src, Q, d, chunks, slices, words_per_slice, fixed_bits, shifts,
                            reinterpret_cast<unsigned long long*>(words));
     });
@@ -747,7 +747,7 @@ extern "C" int bsi_hip_pack_bits_batch(const int64_t* ints, int64_t Q, int64_t d
     BSI_REQUIRE(ints && words, "null pointer");
     const int groups = (words_per_slice + 3) / 4;
     RoundedFromInts src{reinterpret_cast<const long long*>(ints)};
-    hipLaunchKernelGGL((shift_pack_kernel<RoundedFromInts, false>), dim3(grid_for(Q * groups)), dim3(kBlock), 0,
+    launch((shift_pack_kernel<RoundedFromInts, false>), dim3(grid_for(Q * groups)), dim3(kBlock), 0,
                        as_stream(stream), src, Q, d, 0, slices, words_per_slice, 0, nullptr,
                        reinterpret_cast<unsigned long long*>(words));
     BSI_LAUNCH_CHECK("shift_pack_kernel");
@@ -802,12 +802,12 @@ extern "C" int bsi_hip_decimal_stats(const int64_t* ints, int64_t Q, int64_t d, 
     BSI_REQUIRE(Q >= 0 && d >= 0, "negative size");
     BSI_REQUIRE(max_abs != nullptr, "null pointer");
     BSI_REQUIRE(Q <= 0x7fffffffLL, "too many rows for one launch");
-    hipLaunchKernelGGL(clear_u64_kernel, dim3(1), dim3(1), 0, as_stream(stream),
+    launch(clear_u64_kernel, dim3(1), dim3(1), 0, as_stream(stream),
                        reinterpret_cast<unsigned long long*>(max_abs));
     BSI_LAUNCH_CHECK("clear_u64_kernel");
     if (Q == 0) return BSI_OK;
     BSI_REQUIRE(row_negative != nullptr && (ints != nullptr || d == 0), "null pointer");
-    hipLaunchKernelGGL(decimal_stats_kernel, dim3(static_cast<unsigned>(Q)), dim3(kBlock), 0, as_stream(stream),
+    launch(decimal_stats_kernel, dim3(static_cast<unsigned>(Q)), dim3(kBlock), 0, as_stream(stream),
                        reinterpret_cast<const long long*>(ints), d, reinterpret_cast<unsigned long long*>(max_abs),
                        row_negative);
     BSI_LAUNCH_CHECK("decimal_stats_kernel");
@@ -846,7 +846,7 @@ extern "C" int bsi_hip_build_fixed(const void* x, int dtype, int64_t Q, int64_t 
     if (fast && chunk_scale && W % 4 == 0) {
 #define BSI_LAUNCH_FAST(N)                                                                                                 \
     BSI_DISPATCH_DTYPE(dtype, BSI_DISPATCH_BOOL(quads_aligned(x, dtype, d), kVec, BSI_DISPATCH_BOOL(words != nullptr, kPlanes, \
-        hipLaunchKernelGGL((build_fixed_chunk_fast_kernel<T, N, kVec, kPlanes>), dim3(grid_for((items + (N) - 1) / (N))),  \
+        launch((build_fixed_chunk_fast_kernel<T, N, kVec, kPlanes>), dim3(grid_for((items + (N) - 1) / (N))),  \
                            dim3(kBlock), 0, st, static_cast<const T*>(x), static_cast<unsigned>(items), d,                 \
                            static_cast<unsigned>(chunks), fixed_bits, W, dec_scale, scale, words64, shifts, scales, ints8))))
         // Several items a wave share its prologue and put their loads in flight together: worth it once every SIMD has its
@@ -861,18 +861,18 @@ extern "C" int bsi_hip_build_fixed(const void* x, int dtype, int64_t Q, int64_t 
         BSI_LAUNCH_CHECK("build_fixed_chunk_fast_kernel");
     } else if (fast && !chunk_scale) {
         BSI_DISPATCH_DTYPE(dtype, BSI_DISPATCH_BOOL(quads_aligned(x, dtype, d), kVec, BSI_DISPATCH_BOOL(words != nullptr, kPlanes,
-            hipLaunchKernelGGL((build_fixed_row_fast_kernel<T, kVec, kPlanes>), dim3(static_cast<unsigned>(Q)), dim3(kBlock), 0, st,
+            launch((build_fixed_row_fast_kernel<T, kVec, kPlanes>), dim3(static_cast<unsigned>(Q)), dim3(kBlock), 0, st,
                                static_cast<const T*>(x), d, chunks, fixed_bits, W, dec_scale, scale, words64, shifts, scales,
                                ints8))))
         BSI_LAUNCH_CHECK("build_fixed_row_fast_kernel");
     } else if (chunk_scale) {
         BSI_REQUIRE(words != nullptr, "null pointer");
-        BSI_DISPATCH_DTYPE(dtype, hipLaunchKernelGGL(build_fixed_chunk_kernel<T>, dim3(grid_for(items)), dim3(kBlock), 0, st,
+        BSI_DISPATCH_DTYPE(dtype, launch(build_fixed_chunk_kernel<T>, dim3(grid_for(items)), dim3(kBlock), 0, st,
                                                      static_cast<const T*>(x), Q, d, chunks, fixed_bits, W, dec_scale, clip_k,
                                                      words64, shifts, scales, ints8));
         BSI_LAUNCH_CHECK("build_fixed_chunk_kernel");
     } else {
-        BSI_DISPATCH_DTYPE(dtype, hipLaunchKernelGGL(build_fixed_row_kernel<T>, dim3(static_cast<unsigned>(Q)), dim3(kBlock), 0,
+        BSI_DISPATCH_DTYPE(dtype, launch(build_fixed_row_kernel<T>, dim3(static_cast<unsigned>(Q)), dim3(kBlock), 0,
                                                      st, static_cast<const T*>(x), Q, d, fixed_bits, W, dec_scale, clip_k,
                                                      words64, shifts, scales, ints8));
         BSI_LAUNCH_CHECK("build_fixed_row_kernel");
@@ -894,7 +894,7 @@ extern "C" int bsi_hip_build_fixed_keys(const void* x, int dtype, int64_t R, int
     // Chunks kept in registers: 16 for rows of 9 to 16 chunks, which then need no second read of any of them (4096 x 4096:
     // 22.8 us against 29.5), 8 otherwise: two workgroups a CU instead of one (8192 x 2048: 19.5 us against 27.1).
     BSI_DISPATCH_DTYPE(dtype, BSI_DISPATCH_BOOL(quads_aligned(x, dtype, d), kVec, BSI_DISPATCH_BOOL(chunks > 8 && chunks <= 16, kLong,
-        hipLaunchKernelGGL((build_keys_fast_kernel<T, kVec, kLong ? 16 : 8>), dim3(static_cast<unsigned>((R + kKeyRows - 1) / kKeyRows)),
+        launch((build_keys_fast_kernel<T, kVec, kLong ? 16 : 8>), dim3(static_cast<unsigned>((R + kKeyRows - 1) / kKeyRows)),
                            dim3(kKeyRows * BSI_WAVE), 0, as_stream(stream), static_cast<const T*>(x), R, d, chunks, fixed_bits,
                            static_cast<double>(scale_int), static_cast<float>(scale_int),
                            reinterpret_cast<unsigned long long*>(tiled), image, shifts, slice_weights))))

@@ -91,7 +91,8 @@ static int time_launch(hipStream_t st, int reps, float* ms_best, F&& launch) {
         err = hipEventRecord(e0, st);
         if (err != hipSuccess) break;
         launch();
-        err = hipEventRecord(e1, st);
+        err = std::exchange(pending_config_error(), hipSuccess);
+        if (err == hipSuccess) err = hipEventRecord(e1, st);
         if (err == hipSuccess) err = hipEventSynchronize(e1);
         float ms = 0.0f;
         if (err == hipSuccess) err = hipEventElapsedTime(&ms, e0, e1);
@@ -140,7 +141,7 @@ extern "C" int bsi_hip_probe_valu_popcount(double* lane_ops_per_s, void* stream)
     const int iters = 4096, blocks = 256 * 16, threads = 256;
     float ms = 0.0f;
     int rc = time_launch(st, 5, &ms, [&] {
-        hipLaunchKernelGGL(probe_valu_kernel, dim3(blocks), dim3(threads), 0, st, sink, 12345u, iters);
+        launch(probe_valu_kernel, dim3(blocks), dim3(threads), 0, st, sink, 12345u, iters);
     });
     (void)hipFree(sink);
     if (rc) return rc;
@@ -162,7 +163,7 @@ extern "C" int bsi_hip_probe_mfma_i8_operands(int random_operands, double* ops_p
     const int iters = 4096, blocks = 256 * 8, threads = 256;
     float ms = 0.0f;
     int rc = time_launch(st, 5, &ms, [&] {
-        hipLaunchKernelGGL(probe_mfma_kernel, dim3(blocks), dim3(threads), 0, st, sink, 3, iters, random_operands);
+        launch(probe_mfma_kernel, dim3(blocks), dim3(threads), 0, st, sink, 3, iters, random_operands);
     });
     (void)hipFree(sink);
     if (rc) return rc;
@@ -179,7 +180,7 @@ extern "C" int bsi_hip_probe_stream_read(const void* buf, size_t bytes, double* 
     const size_t n16 = bytes / 16;
     float ms = 0.0f;
     int rc = time_launch(st, 5, &ms, [&] {
-        hipLaunchKernelGGL(probe_read_kernel, dim3(256 * 16), dim3(256), 0, st, static_cast<const uint4*>(buf), n16, sink);
+        launch(probe_read_kernel, dim3(256 * 16), dim3(256), 0, st, static_cast<const uint4*>(buf), n16, sink);
     });
     (void)hipFree(sink);
     if (rc) return rc;

@@ -519,11 +519,11 @@ static void launch_mfma_stream(const int8_t* A8, const float* qscale, int stride
     if (pass_chunks > chunks) pass_chunks = chunks;
     const size_t lds = static_cast<size_t>(pass_chunks) * kSlot * sizeof(int);
     if (chunk_ints)
-        hipLaunchKernelGGL((dot_mfma_stream_kernel<NT, KT, true>), grid, dim3(waves * 64), lds, st, A8, qscale, stride,
+        launch((dot_mfma_stream_kernel<NT, KT, true>), grid, dim3(waves * 64), lds, st, A8, qscale, stride,
                            reinterpret_cast<const unsigned long long*>(B), Bw, chunks, pass_chunks, R, Q, down_shift,
                            scale_inv, R_total, out, chunk_ints, bias, t_out_dtype);
     else
-        hipLaunchKernelGGL((dot_mfma_stream_kernel<NT, KT, false>), grid, dim3(waves * 64), lds, st, A8, qscale, stride,
+        launch((dot_mfma_stream_kernel<NT, KT, false>), grid, dim3(waves * 64), lds, st, A8, qscale, stride,
                            reinterpret_cast<const unsigned long long*>(B), Bw, chunks, pass_chunks, R, Q, down_shift,
                            scale_inv, R_total, out, chunk_ints, bias, t_out_dtype);
 }
@@ -575,7 +575,7 @@ static void launch_stream_fused(const FusedPlan& plan, const T* x, int64_t d, do
     static LdsOptIn once0;
     lds_opt_in(once0, reinterpret_cast<const void*>(&dot_mfma_stream_fused_kernel<T, KT, NI, kVec>), 160 * 1024);
     const int narrow = integer_decimal_scale(dec_scale) != 0 ? 1 : 0;
-    hipLaunchKernelGGL((dot_mfma_stream_fused_kernel<T, KT, NI, kVec>), dim3(plan.grid), dim3(plan.waves * 64), lds, st, x, d,
+    launch((dot_mfma_stream_fused_kernel<T, KT, NI, kVec>), dim3(plan.grid), dim3(plan.waves * 64), lds, st, x, d,
                        dec_scale, narrow, slices, reinterpret_cast<const unsigned long long*>(B), Bw, chunks, pass_chunks,
                        R, Q, scale_inv, R_total, out, bias, t_out_dtype);
 }
@@ -689,8 +689,8 @@ static int launch_stream_ewah(const uint64_t* comp_words, const int64_t* comp_of
 #define BSI_EWAH_ARGS reinterpret_cast<const unsigned long long*>(comp_words), reinterpret_cast<const long long*>(comp_off), \
                       comp_len, Sa, W64, A_chunk_scales, A_scale_stride, reinterpret_cast<const unsigned long long*>(B_tiled), \
                       Bw, chunks, pass_chunks, R, Q, group, down_shift, scale_inv, R_total, bias, out, chunk_ints
-    if (chunk_ints) hipLaunchKernelGGL((dot_mfma_stream_ewah_kernel<true>), grid, dim3(waves * 64), lds, st, BSI_EWAH_ARGS);
-    else hipLaunchKernelGGL((dot_mfma_stream_ewah_kernel<false>), grid, dim3(waves * 64), lds, st, BSI_EWAH_ARGS);
+    if (chunk_ints) launch((dot_mfma_stream_ewah_kernel<true>), grid, dim3(waves * 64), lds, st, BSI_EWAH_ARGS);
+    else launch((dot_mfma_stream_ewah_kernel<false>), grid, dim3(waves * 64), lds, st, BSI_EWAH_ARGS);
 #undef BSI_EWAH_ARGS
     BSI_LAUNCH_CHECK("dot_mfma_stream_ewah_kernel");
     return BSI_OK;
@@ -749,7 +749,7 @@ extern "C" int bsi_hip_dot_ewah_batch(const uint64_t* comp_words, const int64_t*
         return fail(BSI_ERR_UNSUPPORTED, "%d words per slice do not fit the LDS plane buffer of the stream decoder", W64);
     static LdsOptIn once;
     lds_opt_in(once, reinterpret_cast<const void*>(&ewah_streams_to_int8_kernel), 160 * 1024);
-    hipLaunchKernelGGL(ewah_streams_to_int8_kernel, dim3(static_cast<unsigned>(Q)), dim3(kEwahToInt8Block), lds, st,
+    launch(ewah_streams_to_int8_kernel, dim3(static_cast<unsigned>(Q)), dim3(kEwahToInt8Block), lds, st,
                        reinterpret_cast<const unsigned long long*>(comp_words), reinterpret_cast<const long long*>(comp_off),
                        comp_len, Sa, W64, chunks, static_cast<uint32_t*>(workspace));
     BSI_LAUNCH_CHECK("ewah_streams_to_int8_kernel");

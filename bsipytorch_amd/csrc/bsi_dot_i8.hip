@@ -1150,7 +1150,7 @@ static void launch_mfma_i8_tm(const int8_t* A8, const float* qscale, int stride,
     const dim3 grid(static_cast<unsigned>((R + TM - 1) / TM), static_cast<unsigned>((Q + TN - 1) / TN));
     static LdsOptIn once0;
     lds_opt_in(once0, reinterpret_cast<const void*>(&dot_mfma_i8_kernel<TM, TN, kMode, false>), C::kLds);
-    hipLaunchKernelGGL((dot_mfma_i8_kernel<TM, TN, kMode, false>), grid, dim3(C::kBlock), C::kLds, st, A8, qscale, stride, K8,
+    launch((dot_mfma_i8_kernel<TM, TN, kMode, false>), grid, dim3(C::kBlock), C::kLds, st, A8, qscale, stride, K8,
                        Bw, Sb, chunks, R, Q, down_shift, scale_inv, R_total, out, chunk_ints, bias, ndig, dig_stride,
                        key_indices, key_tiled, static_cast<const unsigned char*>(g_warm_ptr),
                        static_cast<long long>(g_warm_bytes / 128), stream_output(), static_cast<float*>(nullptr),
@@ -1174,7 +1174,7 @@ static void launch_mfma_i8_split(int segments, unsigned char* scratch, const int
     const float limit = __builtin_ldexpf(1.0f, 24 + down_shift - log2_segments);
     static LdsOptIn once0;
     lds_opt_in(once0, reinterpret_cast<const void*>(&dot_mfma_i8_kernel<TM, TN, kI8Chain, true>), C::kLdsSplit);
-    hipLaunchKernelGGL((dot_mfma_i8_kernel<TM, TN, kI8Chain, true>), grid, dim3(C::kBlock), C::kLdsSplit, st, A8, qscale,
+    launch((dot_mfma_i8_kernel<TM, TN, kI8Chain, true>), grid, dim3(C::kBlock), C::kLdsSplit, st, A8, qscale,
                        stride, K8, Bw, Sb, chunks, R, Q, down_shift, scale_inv, R_total, out, static_cast<int*>(nullptr), bias,
                        1, 0LL, static_cast<const long long*>(nullptr), key_tiled,
                        static_cast<const unsigned char*>(g_warm_ptr), static_cast<long long>(g_warm_bytes / 128),
@@ -1215,11 +1215,11 @@ static void launch_mfma_i8w(const int8_t* A8, const float* qscale, int stride, c
     const unsigned char* warm = static_cast<const unsigned char*>(g_warm_ptr);
     const long long warm_lines = static_cast<long long>(g_warm_bytes / 128);
     if (chunk_ints)
-        hipLaunchKernelGGL((dot_mfma_i8w_kernel<WN, true>), grid, dim3(W::kBlock), C::kLds, st, A8, qscale, stride, K8, Bw, Sb,
+        launch((dot_mfma_i8w_kernel<WN, true>), grid, dim3(W::kBlock), C::kLds, st, A8, qscale, stride, K8, Bw, Sb,
                            chunks, R, Q, down_shift, scale_inv, R_total, out, chunk_ints, bias, key_tiled, warm, warm_lines,
                            stream_output(), t_out_dtype);
     else
-        hipLaunchKernelGGL((dot_mfma_i8w_kernel<WN, false>), grid, dim3(W::kBlock), C::kLds, st, A8, qscale, stride, K8, Bw, Sb,
+        launch((dot_mfma_i8w_kernel<WN, false>), grid, dim3(W::kBlock), C::kLds, st, A8, qscale, stride, K8, Bw, Sb,
                            chunks, R, Q, down_shift, scale_inv, R_total, out, chunk_ints, bias, key_tiled, warm, warm_lines,
                            stream_output(), t_out_dtype);
 }
@@ -1405,7 +1405,7 @@ extern "C" int bsi_hip_dot_digits(const int8_t* A_digits, int nq, const float* A
                    reinterpret_cast<int32_t*>(workspace), nullptr, st, k_tiled, 1, 0, nullptr);
     BSI_LAUNCH_CHECK("dot_mfma_i8_kernel (int32 sum)");
     const int64_t total = Q * R;
-    hipLaunchKernelGGL(digits_combine_kernel, dim3(static_cast<unsigned>((total + 255) / 256)), dim3(256), 0, st,
+    launch(digits_combine_kernel, dim3(static_cast<unsigned>((total + 255) / 256)), dim3(256), 0, st,
                        reinterpret_cast<const int*>(workspace), nq, nk, Q, R, preshift, Aw, Sa, Bw, Sb,
                        reinterpret_cast<const long long*>(key_indices), scale_inv, R_total, bias, out);
     BSI_LAUNCH_CHECK("digits_combine_kernel");
@@ -1439,16 +1439,16 @@ extern "C" int bsi_hip_probe_l2_to_lds(const void* buf, size_t bytes, int loader
     for (int rep = 0; rep < 4 && err == hipSuccess; ++rep) {  // the first repetition also brings the regions into L2
         (void)hipEventRecord(e0, st);
         if (loader_pattern == 1)
-            hipLaunchKernelGGL((probe_l2_lds_kernel<4, 24, true>), dim3(static_cast<unsigned>(cus)), dim3(4 * 64), lds, st,
+            launch((probe_l2_lds_kernel<4, 24, true>), dim3(static_cast<unsigned>(cus)), dim3(4 * 64), lds, st,
                                static_cast<const unsigned char*>(buf), kRegion, kRegions, kPasses);
         else if (loader_pattern == 2)
-            hipLaunchKernelGGL((probe_l2_lds_kernel<4, 24, false>), dim3(static_cast<unsigned>(cus)), dim3(4 * 64), lds, st,
+            launch((probe_l2_lds_kernel<4, 24, false>), dim3(static_cast<unsigned>(cus)), dim3(4 * 64), lds, st,
                                static_cast<const unsigned char*>(buf), kRegion, kRegions, kPasses);
         else if (loader_pattern == 3)
-            hipLaunchKernelGGL((probe_l2_lds_kernel<8, 12, true>), dim3(static_cast<unsigned>(cus)), dim3(8 * 64), lds, st,
+            launch((probe_l2_lds_kernel<8, 12, true>), dim3(static_cast<unsigned>(cus)), dim3(8 * 64), lds, st,
                                static_cast<const unsigned char*>(buf), kRegion, kRegions, kPasses);
         else
-            hipLaunchKernelGGL((probe_l2_lds_kernel<8, 12, false>), dim3(static_cast<unsigned>(cus)), dim3(8 * 64), lds, st,
+            launch((probe_l2_lds_kernel<8, 12, false>), dim3(static_cast<unsigned>(cus)), dim3(8 * 64), lds, st,
                                static_cast<const unsigned char*>(buf), kRegion, kRegions, kPasses);
         (void)hipEventRecord(e1, st);
         err = hipEventSynchronize(e1);

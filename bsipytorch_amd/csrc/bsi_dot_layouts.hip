@@ -88,11 +88,11 @@ int launch_planes_to_int8(const uint64_t* words, int64_t rows, int S, int W64, i
     if (total == 0) return BSI_OK;
     if (tiled && (rows & 63) != 0) {  // the rows that pad the last 64-row tile read as zeros
         const size_t tile_bytes = static_cast<size_t>(chunks) * 2 * 8192;
-        hipLaunchKernelGGL(zero_uint4_kernel, dim3(static_cast<unsigned>((tile_bytes / 16 + 255) / 256)), dim3(256), 0, st,
+        launch(zero_uint4_kernel, dim3(static_cast<unsigned>((tile_bytes / 16 + 255) / 256)), dim3(256), 0, st,
                            reinterpret_cast<uint4*>(out + static_cast<size_t>(rows >> 6) * tile_bytes), tile_bytes / 16);
         BSI_LAUNCH_CHECK("zero_uint4_kernel");
     }
-    hipLaunchKernelGGL(planes_to_int8_kernel, dim3(static_cast<unsigned>((total + 255) / 256)), dim3(256), 0, st,
+    launch(planes_to_int8_kernel, dim3(static_cast<unsigned>((total + 255) / 256)), dim3(256), 0, st,
                        reinterpret_cast<const uint32_t*>(words), rows, S, W64, chunks,
                        reinterpret_cast<uint32_t*>(out), tiled);
     BSI_LAUNCH_CHECK("planes_to_int8_kernel");
@@ -109,7 +109,7 @@ extern "C" int bsi_hip_tile_key_planes(const uint64_t* words, int64_t R, int Sb,
     BSI_REQUIRE(words && out, "null pointer");
     const int chunks = (W64 + 3) / 4;
     const int64_t total = ((R + 15) / 16) * chunks * Sb * 64;
-    hipLaunchKernelGGL(tile_key_planes_kernel, dim3(static_cast<unsigned>((total + 255) / 256)), dim3(256), 0,
+    launch(tile_key_planes_kernel, dim3(static_cast<unsigned>((total + 255) / 256)), dim3(256), 0,
                        as_stream(stream), reinterpret_cast<const unsigned long long*>(words), R, Sb, W64, chunks,
                        total, reinterpret_cast<unsigned long long*>(out));
     BSI_LAUNCH_CHECK("tile_key_planes_kernel");
@@ -147,7 +147,7 @@ extern "C" int bsi_hip_planes_to_int8_digits(const uint64_t* words, int64_t rows
     const int chunks = (W64 + 3) / 4, ndig = (S + 6) / 7;
     const int64_t total = static_cast<int64_t>(ndig) * rows * chunks * 8;
     BSI_REQUIRE((total + 255) / 256 <= 0x7fffffffLL, "too large for one launch");
-    hipLaunchKernelGGL(planes_to_digits_kernel, dim3(static_cast<unsigned>((total + 255) / 256)), dim3(256), 0,
+    launch(planes_to_digits_kernel, dim3(static_cast<unsigned>((total + 255) / 256)), dim3(256), 0,
                        as_stream(stream), reinterpret_cast<const uint32_t*>(words), rows, S, W64, chunks, ndig,
                        reinterpret_cast<uint32_t*>(out));
     BSI_LAUNCH_CHECK("planes_to_digits_kernel");

@@ -287,11 +287,11 @@ static void launch_valu76(const uint64_t* A, const float* qscale, int stride, co
     const dim3 grid(static_cast<unsigned>((R + kValuTile - 1) / kValuTile),
                     static_cast<unsigned>((Q + kValuTile - 1) / kValuTile));
     if (chunk_ints)
-        hipLaunchKernelGGL((dot_valu_kernel<7, 6, kTiled, true>), grid, dim3(kValuBlock), 0, st,
+        launch((dot_valu_kernel<7, 6, kTiled, true>), grid, dim3(kValuBlock), 0, st,
                            reinterpret_cast<const uint32_t*>(A), qscale, stride, reinterpret_cast<const uint32_t*>(B),
                            Bw, W64, chunks, R, Q, scale_inv, R_total, out, chunk_ints);
     else
-        hipLaunchKernelGGL((dot_valu_kernel<7, 6, kTiled, false>), grid, dim3(kValuBlock), 0, st,
+        launch((dot_valu_kernel<7, 6, kTiled, false>), grid, dim3(kValuBlock), 0, st,
                            reinterpret_cast<const uint32_t*>(A), qscale, stride, reinterpret_cast<const uint32_t*>(B),
                            Bw, W64, chunks, R, Q, scale_inv, R_total, out, chunk_ints);
 }
@@ -307,7 +307,7 @@ void launch_valu_generic(const uint64_t* A, const float* qscale, int stride, int
                          int Sb, int W64, int chunks, int64_t R, int64_t Q, float scale_inv, int64_t R_total, float* out,
                          int32_t* chunk_ints, int tiled, hipStream_t st) {
     const int64_t total = Q * R;
-    hipLaunchKernelGGL(dot_valu_generic_kernel, dim3(static_cast<unsigned>((total + 255) / 256)), dim3(256), 0, st,
+    launch(dot_valu_generic_kernel, dim3(static_cast<unsigned>((total + 255) / 256)), dim3(256), 0, st,
                        reinterpret_cast<const unsigned long long*>(A), qscale, stride, Sa,
                        reinterpret_cast<const unsigned long long*>(B), Bw, Sb, W64, chunks, R, Q, scale_inv, R_total,
                        out, chunk_ints, tiled);
@@ -315,7 +315,7 @@ void launch_valu_generic(const uint64_t* A, const float* qscale, int stride, int
 
 void launch_add_bias(float* out, const float* bias, int64_t Q, int64_t R, int64_t R_total, hipStream_t st) {
     const int64_t total = Q * R;
-    hipLaunchKernelGGL(add_bias_kernel, dim3(static_cast<unsigned>((total + 255) / 256)), dim3(256), 0, st, out, bias, Q, R,
+    launch(add_bias_kernel, dim3(static_cast<unsigned>((total + 255) / 256)), dim3(256), 0, st, out, bias, Q, R,
                        R_total);
 }
 
@@ -332,7 +332,7 @@ static int launch_dot_weighted(const uint64_t* A, const float* Aw, int Sa, int W
     static LdsOptIn once0;
     lds_opt_in(once0, reinterpret_cast<const void*>(&dot_weighted_kernel<WB, kTiled>), 150 * 1024);
     const dim3 grid(static_cast<unsigned>((R + 31) / 32), static_cast<unsigned>((Q + 31) / 32));
-    hipLaunchKernelGGL((dot_weighted_kernel<WB, kTiled>), grid, dim3(256), lds, st,
+    launch((dot_weighted_kernel<WB, kTiled>), grid, dim3(256), lds, st,
                        reinterpret_cast<const unsigned long long*>(A), Aw, Sa, W64,
                        reinterpret_cast<const unsigned long long*>(B), Bw, Sb, (W64 + 3) / 4, R, Q,
                        reinterpret_cast<const long long*>(key_indices), scale_inv, R_total, out, out64);

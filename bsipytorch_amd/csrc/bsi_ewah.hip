@@ -128,7 +128,7 @@ extern "C" int bsi_hip_slice_popcount_sum(const uint64_t* words, int S, int W, u
     if (S == 0) return BSI_OK;
     BSI_REQUIRE(words && counts, "null pointer");
     const unsigned grid = static_cast<unsigned>((S + 3) / 4);
-    hipLaunchKernelGGL(slice_popcount_kernel, dim3(grid), dim3(kEwahBlock), 0, as_stream(stream),
+    launch(slice_popcount_kernel, dim3(grid), dim3(kEwahBlock), 0, as_stream(stream),
                        reinterpret_cast<const unsigned long long*>(words), S, W,
                        reinterpret_cast<unsigned long long*>(counts));
     BSI_LAUNCH_CHECK("slice_popcount_kernel");
@@ -140,7 +140,7 @@ extern "C" int bsi_hip_compress_flags_from_density(const uint64_t* counts, int S
     BSI_REQUIRE(S >= 0 && W >= 0, "negative size");
     if (S == 0) return BSI_OK;
     BSI_REQUIRE(counts && flags, "null pointer");
-    hipLaunchKernelGGL(compress_flags_kernel, dim3((S + 127) / 128), dim3(128), 0, as_stream(stream),
+    launch(compress_flags_kernel, dim3((S + 127) / 128), dim3(128), 0, as_stream(stream),
                        reinterpret_cast<const unsigned long long*>(counts), S, W, threshold, flags);
     BSI_LAUNCH_CHECK("compress_flags_kernel");
     return BSI_OK;
@@ -151,7 +151,7 @@ extern "C" int bsi_hip_ewah_size(const uint64_t* words, int S, int W, const int3
     BSI_REQUIRE(S >= 0 && W >= 0, "negative size");
     if (S == 0) return BSI_OK;
     BSI_REQUIRE(words && flags && sizes, "null pointer");
-    hipLaunchKernelGGL(ewah_size_kernel, dim3((S + 3) / 4), dim3(kEwahBlock), 0, as_stream(stream),
+    launch(ewah_size_kernel, dim3((S + 3) / 4), dim3(kEwahBlock), 0, as_stream(stream),
                        reinterpret_cast<const unsigned long long*>(words), S, W, flags,
                        reinterpret_cast<unsigned long long*>(sizes));
     BSI_LAUNCH_CHECK("ewah_size_kernel");
@@ -162,10 +162,10 @@ extern "C" int bsi_hip_ewah_measure(const uint64_t* words, int S, int W, double 
                                     int64_t* off, int64_t* total_host, void* stream) {
     BSI_REQUIRE(S >= 1 && W >= 0, "bad shape");
     BSI_REQUIRE(words && flags && lens && off && total_host, "null pointer");
-    hipLaunchKernelGGL(ewah_measure_kernel, dim3((S + 3) / 4), dim3(kEwahBlock), 0, as_stream(stream),
+    launch(ewah_measure_kernel, dim3((S + 3) / 4), dim3(kEwahBlock), 0, as_stream(stream),
                        reinterpret_cast<const unsigned long long*>(words), S, W, threshold, flags, lens);
     BSI_LAUNCH_CHECK("ewah_measure_kernel");
-    hipLaunchKernelGGL(ewah_offsets_kernel, dim3(1), dim3(kScanBlock), 0, as_stream(stream), lens, S,
+    launch(ewah_offsets_kernel, dim3(1), dim3(kScanBlock), 0, as_stream(stream), lens, S,
                        reinterpret_cast<long long*>(off), reinterpret_cast<long long*>(total_host));
     BSI_LAUNCH_CHECK("ewah_offsets_kernel");
     return BSI_OK;
@@ -176,7 +176,7 @@ extern "C" int bsi_hip_ewah_emit(const uint64_t* words, int S, int W, const int3
     BSI_REQUIRE(S >= 0 && W >= 0, "negative size");
     if (S == 0) return BSI_OK;
     BSI_REQUIRE(words && flags && off && out && out_len, "null pointer");
-    hipLaunchKernelGGL(ewah_emit_kernel, dim3((S + 3) / 4), dim3(kEwahBlock), 0, as_stream(stream),
+    launch(ewah_emit_kernel, dim3((S + 3) / 4), dim3(kEwahBlock), 0, as_stream(stream),
                        reinterpret_cast<const unsigned long long*>(words), S, W, flags,
                        reinterpret_cast<const unsigned long long*>(off), reinterpret_cast<unsigned long long*>(out),
                        out_len);
@@ -189,7 +189,7 @@ extern "C" int bsi_hip_ewah_decompress(const uint64_t* in, int in_len, int W, ui
     if (W == 0) return BSI_OK;
     BSI_REQUIRE(out && (in || in_len == 0), "null pointer");
     // one stream = a batch of one: `len` is read from a kernel argument instead of an array
-    hipLaunchKernelGGL(ewah_decompress_one_kernel, dim3(1), dim3(BSI_WAVE), 0, as_stream(stream),
+    launch(ewah_decompress_one_kernel, dim3(1), dim3(BSI_WAVE), 0, as_stream(stream),
                        reinterpret_cast<const unsigned long long*>(in), in_len, W,
                        reinterpret_cast<unsigned long long*>(out));
     BSI_LAUNCH_CHECK("ewah_decompress_one_kernel");
@@ -201,7 +201,7 @@ extern "C" int bsi_hip_ewah_decompress_batch(const uint64_t* comp, const int64_t
     BSI_REQUIRE(S >= 0 && W >= 0, "negative size");
     if (S == 0 || W == 0) return BSI_OK;
     BSI_REQUIRE(comp && off && len && out, "null pointer");
-    hipLaunchKernelGGL(ewah_decompress_batch_kernel, dim3((S + 3) / 4), dim3(kEwahBlock), 0, as_stream(stream),
+    launch(ewah_decompress_batch_kernel, dim3((S + 3) / 4), dim3(kEwahBlock), 0, as_stream(stream),
                        reinterpret_cast<const unsigned long long*>(comp), reinterpret_cast<const long long*>(off), len,
                        S, W, reinterpret_cast<unsigned long long*>(out));
     BSI_LAUNCH_CHECK("ewah_decompress_batch_kernel");

@@ -6,6 +6,7 @@
 // handles' attributes on every call, so nothing can go stale -- and return None for any call they do not serve; the Python
 // path behind them then serves it or raises its errors.  Launches recorded into a graph always take that path.
 #include <torch/csrc/autograd/python_variable.h>
+#include <torch/csrc/jit/frontend/tracer.h>
 #include <ATen/EmptyTensor.h>
 #include <ATen/hip/EmptyTensor.h>
 #include <c10/hip/HIPFunctions.h>
@@ -52,11 +53,17 @@ struct Config {
     int64_t generation = 0;
 } config;
 
+// nn.Module and the layer class as layer_call compares them (bind_layer()).
+struct Module {
+    PyObject *type, *base, *forward, *call, *global_hooks[4];
+} module;
+
 #define NAMES(X)                                                                                                          \
     X(_bsi_keys_cuda) X(_fused) X(_next_bsi_layer) X(_buffers) X(bias) X(collect_stats) X(decimalPlaces) X(fixed) X(Sb) X(W) X(d) \
     X(num_keys) X(decimals) X(layout) X(words) X(ints8) X(ints8_tiled) X(slice_weights) X(bytes) X(eager) X(dot_calls)      \
     X(build_calls) X(dot_query_vectors_total) X(dot_output_elements_total) X(chunk_scales) X(row_scales) X(keys) \
-    X(comp_words) X(comp_off) X(comp_len) X(Sa) X(Q)
+    X(comp_words) X(comp_off) X(comp_len) X(Sa) X(Q) X(forward) X(__call__) X(_compiled_call_impl) X(_forward_hooks)          \
+    X(_forward_pre_hooks) X(_backward_hooks) X(_backward_pre_hooks)
 struct Names {
 #define X(n) PyObject* n;
     NAMES(X)
@@ -105,7 +112,13 @@ struct Holder {  // an owned reference
     Holder& operator=(const Holder&) = delete;
 };
 
-bool capturing() { return c10::hip::currentStreamCaptureStatusMayInitCtx() != c10::hip::CaptureStatus::None; }
+// The null stream cannot be captured; asking about another one takes 0.4 us.
+bool capturing(hipStream_t st) {
+    if (st == nullptr) return false;
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    return hipStreamIsCapturing(st, &status) != hipSuccess || status != hipStreamCaptureStatusNone;
+}
+hipStream_t stream_of(const at::Device& device) { return c10::hip::getCurrentHIPStream(device.index()).stream(); }
 
 int dtype_code(at::ScalarType t) {
     switch (t) {
@@ -159,6 +172,20 @@ PyObject* int_tuple(std::initializer_list<int64_t> values) {
 bool in_set(PyObject* set, std::initializer_list<int64_t> values) {
     Holder t(int_tuple(values));
     return t.p != nullptr && PySet_Contains(set, t.p) == 1;
+}
+
+// Whether a later capture of a few-rows layer will find its workspace and constants (made by the Python side's first call of
+// the shape).  The answers of the last shapes are kept: they stay true until the flags are read again.
+bool known_few_rows(int device, int64_t rows, int64_t d) {
+    struct Known {
+        int64_t device, rows, d, generation;
+    };
+    static Known known[8] = {};
+    Known& k = known[(d / 64 + rows + device) & 7];
+    if (k.device == device && k.rows == rows && k.d == d && k.generation == config.generation) return true;
+    if (!in_set(shared.reserved, {device, rows, d, config.bits}) || !in_set(shared.warmed, {rows, config.bits, device})) return false;
+    k = Known{device, rows, d, config.generation};
+    return true;
 }
 
 // Attaches the split scratch if the launcher splits a dot of this shape; false: the Python side has to find out first.
@@ -252,17 +279,15 @@ PyObject* linear(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     // half-precision output: the kernels that have it (bsi_ops.can_output_half)
     const bool six_tiled = k.Sb == 6 && k.layout == BSI_LAYOUT_TILED16;
     if (in_code != BSI_DTYPE_F32 && !(rows > shared.stream_max ? k.ints8 != nullptr : six_tiled && chunks <= 32768)) Py_RETURN_NONE;
-    if (capturing()) Py_RETURN_NONE;
-    const c10::hip::HIPStream stream = c10::hip::getCurrentHIPStream(device.index());
-    hipStream_t const st = stream.stream();
+    hipStream_t const st = stream_of(device);
+    if (capturing(st)) Py_RETURN_NONE;
 
     const bool few = rows <= shared.few_rows_max && six_tiled && k.W % 4 == 0 && chunks * rows * 260 <= shared.few_rows_lds;
     PyObject* slot = nullptr;
     void* ws = nullptr;
     int64_t ws_bytes = 0;
     if (few) {
-        if (!in_set(shared.reserved, {device.index(), rows, d, config.bits}) || !in_set(shared.warmed, {rows, config.bits, device.index()}))
-            Py_RETURN_NONE;
+        if (!known_few_rows(device.index(), rows, d)) Py_RETURN_NONE;
     } else {
         Holder index(PyLong_FromLong(device.index()));
         PyObject* record = PyDict_GetItem(shared.linear_ws, index.p);
@@ -348,6 +373,56 @@ PyObject* linear(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     END_HANDLE_TH_ERRORS
 }
 
+// Whether nn.Module.__call__ would do nothing but call the class's own forward.
+bool plain_call(PyObject* self) {
+    static PyObject* const kHooks[] = {names._forward_hooks, names._forward_pre_hooks, names._backward_hooks, names._backward_pre_hooks};
+    PyTypeObject* const type = Py_TYPE(self);
+    if (module.base == nullptr || reinterpret_cast<PyObject*>(type) != module.type || _PyType_Lookup(type, names.forward) != module.forward ||
+        _PyType_Lookup(reinterpret_cast<PyTypeObject*>(module.base), names.__call__) != module.call || torch::jit::tracer::isTracing())
+        return false;
+    for (PyObject* hooks : module.global_hooks)
+        if (PyDict_GET_SIZE(hooks) != 0) return false;
+    PyObject** const slot = _PyObject_GetDictPtr(self);
+    PyObject* const attrs = slot != nullptr ? *slot : nullptr;
+    if (attrs == nullptr || get(attrs, names.forward) != nullptr) return false;
+    if (PyObject* o = get(attrs, names._compiled_call_impl); o != nullptr && o != Py_None) return false;
+    for (PyObject* name : kHooks) {
+        PyObject* const hooks = get(attrs, name);
+        if (hooks == nullptr || !PyDict_Check(hooks) || PyDict_GET_SIZE(hooks) != 0) return false;
+    }
+    return true;
+}
+
+// A layer's __call__: a plain call that linear() serves goes straight there (nn.Module.__call__ and the Python forward take
+// 0.8 us, a sixth of a small layer's host time); any other is nn.Module's.
+PyObject* layer_call(PyObject*, PyObject* const* args, Py_ssize_t nargs, PyObject* kwnames) {
+    if (nargs == 2 && kwnames == nullptr && plain_call(args[0])) {
+        PyObject* const call[] = {*_PyObject_GetDictPtr(args[0]), args[1]};
+        PyObject* const out = linear(nullptr, call, 2);
+        if (out != Py_None) return out;
+        Py_DECREF(out);
+    }
+    Holder base_call(PyObject_GetAttr(module.base, names.__call__));
+    return base_call.p != nullptr ? PyObject_Vectorcall(base_call.p, args, nargs, kwnames) : nullptr;
+}
+
+// bind_layer(type, nn.Module, global hook dicts): the class whose calls layer_call shortens.
+PyObject* bind_layer(PyObject*, PyObject* args) {
+    PyObject *type, *base, *hooks[4];
+    if (!PyArg_ParseTuple(args, "O!O!(O!O!O!O!)", &PyType_Type, &type, &PyType_Type, &base, &PyDict_Type, &hooks[0], &PyDict_Type,
+                          &hooks[1], &PyDict_Type, &hooks[2], &PyDict_Type, &hooks[3]))
+        return nullptr;
+    PyObject* const forward = _PyType_Lookup(reinterpret_cast<PyTypeObject*>(type), names.forward);
+    PyObject* const call = _PyType_Lookup(reinterpret_cast<PyTypeObject*>(base), names.__call__);
+    if (forward == nullptr || call == nullptr) return PyErr_Format(PyExc_TypeError, "bind_layer: no forward or no __call__");
+    module.type = Py_NewRef(type);
+    module.forward = Py_NewRef(forward);
+    module.call = Py_NewRef(call);
+    for (int i = 0; i < 4; ++i) module.global_hooks[i] = Py_NewRef(hooks[i]);
+    module.base = Py_NewRef(base);
+    Py_RETURN_NONE;
+}
+
 // dot(query_batch, keyset) -> the float32 scores, or None: the plain dot of a fixed-bit batch that carries its int8 image.
 PyObject* dot(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     if (nargs != 2) {
@@ -379,8 +454,8 @@ PyObject* dot(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
         Py_RETURN_NONE;
     if (chunked ? (scales->dim() != 2 || scales->size(0) != Q || W % 4 != 0 || scales->size(1) != chunks) : scales->numel() != Q)
         Py_RETURN_NONE;
-    if (capturing() || !split_scratch(device.index(), Q, k.R, W)) Py_RETURN_NONE;
-    hipStream_t const st = c10::hip::getCurrentHIPStream(device.index()).stream();
+    hipStream_t const st = stream_of(device);
+    if (capturing(st) || !split_scratch(device.index(), Q, k.R, W)) Py_RETURN_NONE;
     at::Tensor out = at::detail::empty_cuda({Q, k.R}, at::kFloat, device, std::nullopt);
     int layout = 0, rc = BSI_OK;
     size_t bytes = 0;
@@ -407,12 +482,13 @@ PyObject* build(PyObject*, PyObject* args) {
     const at::Tensor& x = THPVariable_Unpack(o);
     const int code = dtype_code(x.scalar_type());
     if (!x.is_cuda() || code < 0 || x.dim() != 2 || x.numel() == 0 || !x.is_contiguous() ||
-        x.device().index() != c10::hip::current_device() || capturing())
+        x.device().index() != c10::hip::current_device())
         Py_RETURN_NONE;
     const at::Device device = x.device();
+    hipStream_t const st = stream_of(device);
+    if (capturing(st)) Py_RETURN_NONE;
     const int64_t Q = x.size(0), d = x.size(1), W = (d + 63) / 64, chunks = (d + 255) / 256;
     const bool chunked = W % 4 == 0;
-    hipStream_t const st = c10::hip::getCurrentHIPStream(device.index()).stream();
     at::Tensor words, ints8, scales;
     if (planes) words = at::detail::empty_cuda({Q, config.bits, W}, at::kLong, device, std::nullopt);
     if (image) ints8 = at::detail::empty_cuda({Q, chunks * 256}, at::kChar, device, std::nullopt);
@@ -439,11 +515,12 @@ PyObject* ewah_streams(PyObject*, PyObject* args) {
     HANDLE_TH_ERRORS
     const at::Tensor& words = THPVariable_Unpack(o);
     if (!words.is_cuda() || words.scalar_type() != at::kLong || words.dim() != 2 || words.size(0) < 1 || words.size(0) > INT32_MAX ||
-        words.size(1) > INT32_MAX || !words.is_contiguous() || words.device().index() != c10::hip::current_device() || capturing())
+        words.size(1) > INT32_MAX || !words.is_contiguous() || words.device().index() != c10::hip::current_device())
         Py_RETURN_NONE;
     const at::Device device = words.device();
     const int S = static_cast<int>(words.size(0)), W = static_cast<int>(words.size(1));
-    hipStream_t const st = c10::hip::getCurrentHIPStream(device.index()).stream();
+    hipStream_t const st = stream_of(device);
+    if (capturing(st)) Py_RETURN_NONE;
     at::Tensor flags = at::detail::empty_cuda({S}, at::kInt, device, std::nullopt);
     at::Tensor lens = at::detail::empty_cuda({S}, at::kInt, device, std::nullopt);
     at::Tensor off = at::detail::empty_cuda({S}, at::kLong, device, std::nullopt);
@@ -502,9 +579,10 @@ PyObject* dot_streams(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     if (!streams->is_cuda() || device.index() != c10::hip::current_device() || !read_keys(args[1], device, &k) || k.W != W ||
         k.decimals != decimals || decimals < 0 || Q <= 0 || Sa < 2 || Sa > 8 || off->numel() != Q * Sa || len->numel() != Q * Sa ||
         scales->device() != device || !scales->is_contiguous() || (chunked && W % 4 != 0) ||
-        scales->numel() != (chunked ? Q * chunks : Q) || capturing() || !split_scratch(device.index(), Q, k.R, W))
+        scales->numel() != (chunked ? Q * chunks : Q))
         Py_RETURN_NONE;
-    hipStream_t const st = c10::hip::getCurrentHIPStream(device.index()).stream();
+    hipStream_t const st = stream_of(device);
+    if (capturing(st) || !split_scratch(device.index(), Q, k.R, W)) Py_RETURN_NONE;
     at::Tensor out = at::detail::empty_cuda({Q, k.R}, at::kFloat, device, std::nullopt);
     const size_t need = lib.dot_ewah_batch_workspace_bytes(Q, static_cast<int>(W));
     at::Tensor ws = at::detail::empty_cuda({static_cast<int64_t>(need)}, at::kByte, device, std::nullopt);
@@ -590,10 +668,12 @@ PyMethodDef methods[] = {
     {"ewah_streams", ewah_streams, METH_VARARGS, nullptr},
     {"dot_streams", reinterpret_cast<PyCFunction>(reinterpret_cast<void*>(dot_streams)), METH_FASTCALL, nullptr},
     {"linear", reinterpret_cast<PyCFunction>(reinterpret_cast<void*>(linear)), METH_FASTCALL, nullptr},
+    {"bind_layer", bind_layer, METH_VARARGS, nullptr},
+    {"layer_call", reinterpret_cast<PyCFunction>(reinterpret_cast<void*>(layer_call)), METH_FASTCALL | METH_KEYWORDS, nullptr},
     {"dot", reinterpret_cast<PyCFunction>(reinterpret_cast<void*>(dot)), METH_FASTCALL, nullptr},
     {nullptr, nullptr, 0, nullptr},
 };
-PyModuleDef module = {PyModuleDef_HEAD_INIT, "_native", "Host path of eager calls.", -1, methods, nullptr, nullptr, nullptr, nullptr};
+PyModuleDef definition = {PyModuleDef_HEAD_INIT, "_native", "Host path of eager calls.", -1, methods, nullptr, nullptr, nullptr, nullptr};
 
 }  // namespace
 
@@ -601,5 +681,13 @@ PyMODINIT_FUNC PyInit__native() {
 #define X(n) names.n = PyUnicode_InternFromString(#n);
     NAMES(X)
 #undef X
-    return PyModule_Create(&module);
+    PyObject* const m = PyModule_Create(&definition);
+    // a builtin function does not bind to an instance: the class gets this form of it
+    Holder call(m != nullptr ? PyObject_GetAttrString(m, "layer_call") : nullptr);
+    Holder method(call.p != nullptr ? PyInstanceMethod_New(call.p) : nullptr);
+    if (method.p == nullptr || PyModule_AddObjectRef(m, "layer_call", method.p) != 0) {
+        Py_XDECREF(m);
+        return nullptr;
+    }
+    return m;
 }

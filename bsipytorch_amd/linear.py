@@ -125,6 +125,8 @@ class BSIQuantizedLinear(nn.Module):
         self.max_abs_error = 0.0
         self.samples_tracked = 0
 
+    __call__ = _native.layer_call  # nn.Module.__call__, unless nothing hangs on the call
+
     def forward(self, x):
         scores = _native.linear(self.__dict__, x)  # None: a call (or a configuration) it does not serve
         if scores is not None:
@@ -314,6 +316,10 @@ class BSIQuantizedLinear(nn.Module):
         c["cosine_sum"] += float(torch.nn.functional.cosine_similarity(got, ref, dim=1).sum())
         c["max_abs_error"] = max(c["max_abs_error"], float(err.abs().max()))
         c["samples_tracked"] += n
+
+
+_native.bind_layer(BSIQuantizedLinear, nn.Module, tuple(getattr(nn.modules.module, f"_global_{which}_hooks") for which in
+                                                        ("forward", "forward_pre", "backward", "backward_pre")))
 
 
 def _keys_to_warm(layer):

@@ -1,0 +1,47 @@
+"""A BSI layer's __call__ goes straight to its native forward only where nn.Module.__call__ would do nothing else."""
+import pytest
+import torch
+
+from test_gpu_parity import ops  # noqa: F401  (fixture)
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("rows", [1, 5, 40])
+def test_whatever_hangs_on_a_call_is_honoured(ops, rows):
+    from bsipytorch_amd.linear import BSIQuantizedLinear
+    from torch.nn.modules import module as nn_module
+
+    layer = BSIQuantizedLinear(torch.nn.Linear(512, 96).cuda(), 2, 0.5)
+    x = torch.randn(rows, 512, device="cuda")
+    with torch.no_grad():
+        want = layer.forward(x)
+        assert torch.equal(layer(x), want) and torch.equal(layer(x=x), want)
+        seen = []
+        for register in (layer.register_forward_hook, nn_module.register_module_forward_hook):
+            handle = register(lambda m, i, o: seen.append(m) or o + 1)
+            assert torch.equal(layer(x), want + 1)
+            handle.remove()
+        for register in (layer.register_forward_pre_hook, nn_module.register_module_forward_pre_hook):
+            handle = register(lambda m, i: seen.append(m) or (i[0] * 0,))
+            assert torch.equal(layer(x), layer.forward(x * 0))
+            handle.remove()
+        assert len(seen) == 4 and all(m is layer for m in seen)
+        layer.forward = lambda t: t  # an instance's own forward
+        assert layer(x) is x
+        del layer.forward
+
+        class Doubled(BSIQuantizedLinear):
+            def forward(self, t):
+                return super().forward(t) * 2
+
+        assert torch.equal(Doubled(torch.nn.Linear(512, 96).cuda(), 2, 0.5)(x) * 0, want * 0)
+        original, calls = torch.nn.Module.__call__, []
+        torch.nn.Module.__call__ = lambda m, *a, **k: calls.append(m) or original(m, *a, **k)
+        try:
+            assert torch.equal(layer(x), want) and calls == [layer]
+        finally:
+            torch.nn.Module.__call__ = original
+        assert torch.equal(layer(x), want) and len(calls) == 1
+    with pytest.raises(TypeError):
+        layer(x, x)
