@@ -49,6 +49,8 @@ PROTOTYPES = {
     "bsi_hip_compress_flags_from_density": [_vp, _i, _i, _d, _vp, _vp],
     "bsi_hip_ewah_size": [_vp, _i, _i, _vp, _vp, _vp],
     "bsi_hip_ewah_measure": [_vp, _i, _i, _d, _vp, _vp, _vp, _vp, _vp],
+    "bsi_hip_build_measure": [_vp, _i, _i64, _i64, _i, _i, _i, _d, _vp, _vp, _vp, _vp, _vp, _vp, _vp],
+    "bsi_hip_ewah_emit_at": [_vp, _i, _i, _vp, _vp, _vp, _vp, _vp],
     "bsi_hip_ewah_emit": [_vp, _i, _i, _vp, _vp, _vp, _vp, _vp],
     "bsi_hip_ewah_decompress": [_vp, _i, _i, _vp, _vp],
     "bsi_hip_ewah_decompress_batch": [_vp, _vp, _vp, _i, _i, _vp, _vp],
@@ -87,7 +89,8 @@ PROTOTYPES = {
     "bsi_hip_dot_weighted_f64": [_vp, _vp, _i, _i, _vp, _i, _vp, _i, _i64, _i64, _vp, _i64, _vp, _vp],
     "bsi_hip_quantize_trunc_to_int64": [_vp, _i, _i64, _f, _vp, _vp],
     "bsi_hip_scalar_query_max_elems": [],
-    "bsi_hip_scalar_query_dot": [_vp, _i64, _i, _d, _vp, _vp, _vp, _i, _i64, _vp, _vp, ctypes.POINTER(_f), ctypes.POINTER(_f), _vp],
+    "bsi_hip_scalar_query_host_words": [_i64, _i64],
+    "bsi_hip_scalar_query_dot": [_vp, _i64, _i, _d, _vp, _vp, _i, _i64, _d, _vp, _vp, _vp, _vp, _vp, _vp],
     "bsi_hip_dot_timed": [_vp, _vp, _vp, _i, _i, _i, _vp, _i, _vp, _i, _i64, _i64, _f, _i64, _vp, _i, _vp, _sz, _i,
                           ctypes.POINTER(_f), _vp],
     "bsi_hip_probe_valu_popcount": [ctypes.POINTER(_d), _vp],
@@ -110,6 +113,7 @@ _RESTYPES = {
     "bsi_hip_dot_digits_workspace_bytes": _sz,
     "bsi_hip_int8_tiled_bytes": _sz,
     "bsi_hip_scalar_query_max_elems": _i64,
+    "bsi_hip_scalar_query_host_words": _i64,
 }
 
 

@@ -638,7 +638,23 @@ def build_bsi_queries_cuda_batch_hybrid(q2d: torch.Tensor, decimal_places: int, 
     _check(q2d.dim() == 2, "q must be 2D [Q, d]")
     f = _flags()
     _check(2 <= f["bits_q"] <= 8, "the hybrid query batch needs fixed-bit queries of 2 to 8 bits")
-    b = _build_query_batch(q2d, int(decimal_places), want_ints8=False)
+    x = _as_build_input(q2d, _device())
+    built = _native.hybrid(x, int(decimal_places), float(compress_threshold))  # None: a call or configuration it does not serve
+    if built is not None:
+        _last_build_profile[:] = [0, 0, 0]
+        h = PrebuiltBSIQueryBatchHybridCUDA()
+        h.comp_words, h.comp_off, h.comp_len, h.flags, scales, h.slice_weights = built
+        h.Sa, h.W, h.decimals, h.Q = f["bits_q"], (x.shape[1] + 63) // 64, int(decimal_places), x.shape[0]
+        if h.slice_weights is None:
+            h.chunk_scales = scales
+            h.slice_weights = _expanded_slice_weights(_slice_weights(h.Sa, 0, True, x.device), h.Q, h.Sa, x.device)
+        else:
+            h.row_scales = scales
+        scale_bytes = scales.numel() * 4
+        h.mem_bytes = h.comp_words.numel() * 8 + h.Q * h.Sa * 12 + scale_bytes
+        h.verbatim_bytes = h.Q * h.Sa * h.W * 8 + scale_bytes
+        return h
+    b = _build_query_batch(x, int(decimal_places), want_ints8=False)
     Q, Sa, W = b.words.shape
     _check(Q > 0, "Empty query batch")
     comp_words, comp_off, comp_len, flags = ewah_compress_slices(b.words.view(Q * Sa, W), float(compress_threshold))
@@ -1514,7 +1530,9 @@ def debug_quantize_int64_cpu(values: torch.Tensor, decimal_places: int) -> torch
 _native.bind({name: ctypes.cast(getattr(lib, name), ctypes.c_void_p).value
               for name in ("bsi_hip_linear_few_rows_out", "bsi_hip_linear_out", "bsi_hip_linear_workspace_bytes", "bsi_hip_dot",
                            "bsi_hip_build_fixed", "bsi_hip_ewah_measure", "bsi_hip_ewah_emit", "bsi_hip_dot_ewah_batch",
-                           "bsi_hip_dot_ewah_batch_workspace_bytes")},
+                           "bsi_hip_dot_ewah_batch_workspace_bytes", "bsi_hip_scalar_query_dot",
+                           "bsi_hip_build_measure", "bsi_hip_ewah_emit_at",
+                           "bsi_hip_scalar_query_host_words")},
              {"keys_type": PrebuiltBSIKeysCUDA, "batch_type": PrebuiltBSIQueryBatchCUDA,
               "hybrid_type": PrebuiltBSIQueryBatchHybridCUDA, "linear_ws": _linear_ws,
               "reserved": _reserved_linear_shapes, "warmed": _warmed_query_caches, "split_shapes": _split_shapes,

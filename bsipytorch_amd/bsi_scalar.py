@@ -13,15 +13,16 @@ rule and container sizes are not recoverable from the reference's tree, and noth
 Every function needs the HIP library and a GPU, like the rest of the module; inputs may live on either device and
 results come back where the reference returns them (Python numbers, CPU tensors).
 """
-import ctypes
 import os
 from typing import Tuple
 
 import numpy as np
 import torch
 
-from . import _lib
+from . import _lib, _native
 from ._lib import check, lib
+
+_SCALAR_MAX_ELEMS = lib.bsi_hip_scalar_query_max_elems()
 
 
 def _ops():
@@ -267,18 +268,14 @@ def batch_dot_product_prebuilt(q: torch.Tensor, keyset_cap, query_threshold: flo
     ops._check(q.shape[0] == keys.d, "q.size(0) must equal keys' dimension")
     thr = float(query_threshold) if query_threshold >= 0.0 else keys.threshold
     d, k = keys.d, keys.sliced
-    if 0 < d <= lib.bsi_hip_scalar_query_max_elems() and 0 < k.rows <= (1 << 24):
-        # the whole call on the device, one wait: the scores and what the query's slices take arrive in pinned memory
-        x = _vec(q, "q")
-        workspace = torch.empty((64 * k.W + 4,), dtype=torch.int64, device=x.device)
-        host = torch.empty((k.rows + 4,), dtype=torch.float64, pin_memory=True)
-        build_ms, dot_ms = ctypes.c_float(0.0), ctypes.c_float(0.0)
-        check(lib.bsi_hip_scalar_query_dot(x.data_ptr(), d, keys.decimalPlaces, thr, workspace.data_ptr(), k.words.data_ptr(),
-                                           k.weights.data_ptr(), k.S, k.rows, host.data_ptr(), host.data_ptr() + 8 * k.rows,
-                                           ctypes.byref(build_ms), ctypes.byref(dot_ms), ops._stream()), "bsi_hip_scalar_query_dot")
-        words = int(host[k.rows + 2:k.rows + 3].view(torch.int64))
-        build_ns, dot_ns = int(build_ms.value * 1.0e6), int(dot_ms.value * 1.0e6)
-        return host[:k.rows] / _scale(2 * keys.decimalPlaces), build_ns + dot_ns, build_ns, dot_ns, words * 8
+    if 0 < d <= _SCALAR_MAX_ELEMS and 0 < k.rows <= (1 << 24):
+        # the whole call in one launch: the scores and what the query's slices take arrive in pinned memory
+        scale = _scale(2 * keys.decimalPlaces)
+        got = (_native.scalar_query(q, k.words, k.weights, keys.decimalPlaces, thr, scale)
+               or _native.scalar_query(_vec(q, "q"), k.words, k.weights, keys.decimalPlaces, thr, scale))
+        if got is not None:
+            out, build_ns, dot_ns, words = got
+            return out, build_ns + dot_ns, build_ns, dot_ns, words * 8
     e0, e1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
     e0.record()
     sq = _Sliced(_ints_round(_vec(q, "q").unsqueeze(0), keys.decimalPlaces), thr)

@@ -33,6 +33,10 @@ struct Library {
     decltype(&bsi_hip_ewah_emit) ewah_emit;
     decltype(&bsi_hip_dot_ewah_batch) dot_ewah_batch;
     decltype(&bsi_hip_dot_ewah_batch_workspace_bytes) dot_ewah_batch_workspace_bytes;
+    decltype(&bsi_hip_scalar_query_dot) scalar_query_dot;
+    decltype(&bsi_hip_build_measure) build_measure;
+    decltype(&bsi_hip_ewah_emit_at) ewah_emit_at;
+    decltype(&bsi_hip_scalar_query_host_words) scalar_query_host_words;
 } lib;
 
 // The Python side's state (bind()): types of the handles, the workspaces and what is known about shapes.
@@ -552,6 +556,69 @@ PyObject* ewah_streams(PyObject*, PyObject* args) {
     END_HANDLE_TH_ERRORS
 }
 
+// hybrid(x, decimals, threshold) -> (stream words, offsets, lengths, flags, scales, slice weights or None), or None: the
+// fixed-bit build of a contiguous [Q, d] batch on the current device, every slice EWAH-encoded.  The host waits for the
+// lengths, which arrive while the build's kernel still runs: their sum is the size of the streams.
+PyObject* hybrid(PyObject*, PyObject* args) {
+    PyObject* o = nullptr;
+    int decimals = 0;
+    double threshold = 0.0;
+    if (!PyArg_ParseTuple(args, "Oid", &o, &decimals, &threshold)) return nullptr;
+    if (!config.on || !THPVariable_CheckExact(o) || decimals < 0 || decimals > 2) Py_RETURN_NONE;
+    HANDLE_TH_ERRORS
+    const at::Tensor& x = THPVariable_Unpack(o);
+    const int code = dtype_code(x.scalar_type());
+    if (!x.is_cuda() || code < 0 || x.dim() != 2 || x.numel() == 0 || !x.is_contiguous() || x.device().index() != c10::hip::current_device())
+        Py_RETURN_NONE;
+    const at::Device device = x.device();
+    hipStream_t const st = stream_of(device);
+    const int64_t Q = x.size(0), d = x.size(1), W = (d + 63) / 64, chunks = (d + 255) / 256, S = Q * config.bits;
+    if (W > 1024 || S > 8192 || capturing(st)) Py_RETURN_NONE;  // bsi_hip_build_measure's limits
+    const bool chunked = W % 4 == 0;
+    at::Tensor words = at::detail::empty_cuda({S, W}, at::kLong, device, std::nullopt);
+    at::Tensor scales = chunked ? at::detail::empty_cuda({Q, chunks}, at::kFloat, device, std::nullopt)
+                                : at::detail::empty_cuda({Q}, at::kFloat, device, std::nullopt);
+    at::Tensor weights;
+    if (!chunked) weights = at::detail::empty_cuda({Q, config.bits}, at::kFloat, device, std::nullopt);
+    at::Tensor flags = at::detail::empty_cuda({S}, at::kInt, device, std::nullopt);
+    at::Tensor lens = at::detail::empty_cuda({S}, at::kInt, device, std::nullopt);
+    at::Tensor off = at::detail::empty_cuda({S}, at::kLong, device, std::nullopt);
+    at::Tensor pinned = at::detail::empty_cpu({S}, at::kInt, /*pin_memory=*/true);
+    volatile int32_t* const host = static_cast<volatile int32_t*>(pinned.data_ptr());
+    uint64_t* const w = static_cast<uint64_t*>(words.data_ptr());
+    int64_t total = 0;
+    int rc = BSI_OK;
+    Py_BEGIN_ALLOW_THREADS
+    for (int64_t s = 0; s < S; ++s) host[s] = -1;
+    rc = lib.build_measure(x.const_data_ptr(), code, Q, d, decimals, config.bits, chunked ? 1 : 0, threshold, w,
+                           static_cast<float*>(scales.data_ptr()), chunked ? nullptr : static_cast<float*>(weights.data_ptr()),
+                           static_cast<int32_t*>(flags.data_ptr()), static_cast<int32_t*>(lens.data_ptr()), const_cast<int32_t*>(host), st);
+    // the stream is waited for only if the lengths are long in coming
+    const auto until = std::chrono::steady_clock::now() + std::chrono::microseconds(500);
+    bool waited = false;
+    for (int64_t s = 0; s < S && rc == BSI_OK; ++s) {
+        while (host[s] < 0 && !waited)
+            if (std::chrono::steady_clock::now() > until) {
+                waited = true;
+                if (hipStreamSynchronize(st) != hipSuccess) rc = BSI_ERR_HIP;
+            }
+        total += host[s];
+    }
+    Py_END_ALLOW_THREADS
+    if (rc != BSI_OK) return fail_status(rc, "bsi_hip_build_measure");
+    at::Tensor streams = at::detail::empty_cuda({total}, at::kLong, device, std::nullopt);
+    Py_BEGIN_ALLOW_THREADS
+    rc = lib.ewah_emit_at(w, static_cast<int>(S), static_cast<int>(W), static_cast<const int32_t*>(flags.data_ptr()),
+                          static_cast<const int32_t*>(lens.data_ptr()), static_cast<int64_t*>(off.data_ptr()),
+                          static_cast<uint64_t*>(streams.data_ptr()), st);
+    Py_END_ALLOW_THREADS
+    if (rc != BSI_OK) return fail_status(rc, "bsi_hip_ewah_emit_at");
+    Holder a(THPVariable_Wrap(std::move(streams))), b(THPVariable_Wrap(std::move(off))), c(THPVariable_Wrap(std::move(lens))),
+        f(THPVariable_Wrap(std::move(flags))), s(THPVariable_Wrap(std::move(scales))), v(THPVariable_Wrap(std::move(weights)));
+    return PyTuple_Pack(6, a.p, b.p, c.p, f.p, s.p, v.p);
+    END_HANDLE_TH_ERRORS
+}
+
 // dot_streams(hybrid_batch, keyset) -> the float32 scores, or None: the dot of a batch kept as EWAH streams.
 PyObject* dot_streams(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     if (nargs != 2) {
@@ -602,6 +669,47 @@ PyObject* dot_streams(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     END_HANDLE_TH_ERRORS
 }
 
+// scalar_query(x, words [R, Sb, W], weights [R, Sb], decimals, threshold, divisor) -> (scores float64 [R] on the host, build
+// ns, dot ns, words of the query's stored form), or None: one float32 vector on the current device against decimal keys.
+PyObject* scalar_query(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+    if (nargs != 6) {
+        PyErr_SetString(PyExc_TypeError, "scalar_query(x, words, weights, decimals, threshold, divisor)");
+        return nullptr;
+    }
+    if (!THPVariable_CheckExact(args[0]) || !THPVariable_Check(args[1]) || !THPVariable_Check(args[2])) Py_RETURN_NONE;
+    const long decimals = PyLong_AsLong(args[3]);
+    const double threshold = PyFloat_AsDouble(args[4]), divisor = PyFloat_AsDouble(args[5]);
+    if (PyErr_Occurred()) return nullptr;
+    HANDLE_TH_ERRORS
+    const at::Tensor &x = THPVariable_Unpack(args[0]), &words = THPVariable_Unpack(args[1]), &weights = THPVariable_Unpack(args[2]);
+    if (!x.is_cuda() || x.scalar_type() != at::kFloat || x.dim() != 1 || x.numel() == 0 || !x.is_contiguous() ||
+        x.device().index() != c10::hip::current_device())
+        Py_RETURN_NONE;
+    const at::Device device = x.device();
+    const int64_t d = x.size(0), W = (d + 63) / 64;
+    if (words.device() != device || words.scalar_type() != at::kLong || words.dim() != 3 || words.size(2) != W || !words.is_contiguous() ||
+        words.size(0) == 0 || weights.device() != device || weights.scalar_type() != at::kFloat || !weights.is_contiguous() ||
+        weights.numel() != words.size(0) * words.size(1))
+        Py_RETURN_NONE;
+    hipStream_t const st = stream_of(device);
+    if (capturing(st)) Py_RETURN_NONE;
+    const int64_t R = words.size(0);
+    at::Tensor out = at::detail::empty_cpu({R}, at::kDouble);
+    at::Tensor pinned = at::detail::empty_cpu({lib.scalar_query_host_words(d, R)}, at::kLong, /*pin_memory=*/true);
+    int64_t info[4] = {0, 0, 0, 0}, build_ns = 0, dot_ns = 0;
+    int rc = BSI_OK;
+    Py_BEGIN_ALLOW_THREADS
+    rc = lib.scalar_query_dot(x.const_data_ptr<float>(), d, static_cast<int>(decimals), threshold,
+                              static_cast<const uint64_t*>(words.const_data_ptr()), weights.const_data_ptr<float>(),
+                              static_cast<int>(words.size(1)), R, divisor, static_cast<uint64_t*>(pinned.data_ptr()),
+                              out.data_ptr<double>(), info, &build_ns, &dot_ns, st);
+    Py_END_ALLOW_THREADS
+    if (rc != BSI_OK) return fail_status(rc, "bsi_hip_scalar_query_dot");
+    Holder scores(THPVariable_Wrap(std::move(out)));
+    return Py_BuildValue("OLLL", scores.p, static_cast<long long>(build_ns), static_cast<long long>(dot_ns), static_cast<long long>(info[2]));
+    END_HANDLE_TH_ERRORS
+}
+
 // configure(bits, core): the process's flags, or configure() to switch the native path off until they are read again.
 PyObject* configure(PyObject*, PyObject* args) {
     int bits = 0, core = 0;
@@ -647,6 +755,9 @@ PyObject* bind(PyObject*, PyObject* args) {
         !entry(entries, "bsi_hip_build_fixed", &lib.build_fixed) || !entry(entries, "bsi_hip_ewah_measure", &lib.ewah_measure) ||
         !entry(entries, "bsi_hip_ewah_emit", &lib.ewah_emit) || !entry(entries, "bsi_hip_dot_ewah_batch", &lib.dot_ewah_batch) ||
         !entry(entries, "bsi_hip_dot_ewah_batch_workspace_bytes", &lib.dot_ewah_batch_workspace_bytes) ||
+        !entry(entries, "bsi_hip_build_measure", &lib.build_measure) || !entry(entries, "bsi_hip_ewah_emit_at", &lib.ewah_emit_at) ||
+        !entry(entries, "bsi_hip_scalar_query_dot", &lib.scalar_query_dot) ||
+        !entry(entries, "bsi_hip_scalar_query_host_words", &lib.scalar_query_host_words) ||
         !take(state, "keys_type", &shared.keys_type) || !take(state, "batch_type", &shared.batch_type) ||
         !take(state, "hybrid_type", &shared.hybrid_type) ||
         !take(state, "linear_ws", &shared.linear_ws) || !take(state, "reserved", &shared.reserved) ||
@@ -665,9 +776,11 @@ PyMethodDef methods[] = {
     {"configure", configure, METH_VARARGS, nullptr},
     {"build_key", build_key, METH_VARARGS, nullptr},
     {"build", build, METH_VARARGS, nullptr},
+    {"hybrid", hybrid, METH_VARARGS, nullptr},
     {"ewah_streams", ewah_streams, METH_VARARGS, nullptr},
     {"dot_streams", reinterpret_cast<PyCFunction>(reinterpret_cast<void*>(dot_streams)), METH_FASTCALL, nullptr},
     {"linear", reinterpret_cast<PyCFunction>(reinterpret_cast<void*>(linear)), METH_FASTCALL, nullptr},
+    {"scalar_query", reinterpret_cast<PyCFunction>(reinterpret_cast<void*>(scalar_query)), METH_FASTCALL, nullptr},
     {"bind_layer", bind_layer, METH_VARARGS, nullptr},
     {"layer_call", reinterpret_cast<PyCFunction>(reinterpret_cast<void*>(layer_call)), METH_FASTCALL | METH_KEYWORDS, nullptr},
     {"dot", reinterpret_cast<PyCFunction>(reinterpret_cast<void*>(dot)), METH_FASTCALL, nullptr},

@@ -72,17 +72,18 @@ int bsi_hip_quantize_round_to_int64(const void* x_device, int dtype, int64_t tot
 int bsi_hip_quantize_trunc_to_int64(const void* x_device, int dtype, int64_t total, float factor, int64_t* out,
                                     void* stream);
 
-/* One vector against prebuilt decimal keys (batch_dot_product_prebuilt, bsiFunctions.cpp:651-701) in two launches and one
- * wait: x [d] float32 is built in decimal mode on the device (slice count from its largest magnitude), then
- * out[r] = the exact integer dot with key row r (canonical planes B [R, Sb, W64], slice weights Bw [R, Sb]) as float64.
- * info: {slices, whether a value is negative, words the slices take in stored form at `threshold`, run-length coded
- * slices}.  out [R] and info [4] may be pinned host memory (they are complete when the call returns); workspace:
- * 64 * ceil(d / 64) + 4 words of device memory.  build_ms / dot_ms: device-event times of the two launches.
- * d at most bsi_hip_scalar_query_max_elems(). */
+/* One vector against prebuilt decimal keys (batch_dot_product_prebuilt, bsiFunctions.cpp:651-701) in one launch, complete
+ * when the call returns: x [d] float32 is built in decimal mode on the device (slice count from its largest magnitude), then
+ * out[r] = the exact integer dot with key row r (canonical planes B [R, Sb, W64], slice weights Bw [R, Sb]) as float64,
+ * divided by `divisor`.  info [4]: {slices, whether a value is negative, words the slices take in stored form at
+ * `threshold`, run-length coded slices}.  pinned: bsi_hip_scalar_query_host_words(d, R) words of pinned host memory;
+ * out, info: host memory.  build_ns / dot_ns: device-clock times of the two parts.  d at most
+ * bsi_hip_scalar_query_max_elems(). */
 int64_t bsi_hip_scalar_query_max_elems(void);
-int bsi_hip_scalar_query_dot(const float* x_device, int64_t d, int decimal_places, double threshold, uint64_t* workspace_device,
-                             const uint64_t* B, const float* Bw, int Sb, int64_t R, double* out, int64_t* info, float* build_ms,
-                             float* dot_ms, void* stream);
+int64_t bsi_hip_scalar_query_host_words(int64_t d, int64_t R);
+int bsi_hip_scalar_query_dot(const float* x_device, int64_t d, int decimal_places, double threshold, const uint64_t* B,
+                             const float* Bw, int Sb, int64_t R, double divisor, uint64_t* pinned, double* out, int64_t* info,
+                             int64_t* build_ns, int64_t* dot_ns, void* stream);
 
 /* Per-row / per-(row, 256-element chunk) shift and power-of-two scale from already rounded ints.
  * Replace launch_compute_row_shift_scale / launch_compute_chunk_shift_scale
@@ -178,6 +179,16 @@ int bsi_hip_ewah_measure(const uint64_t* words_device, int S, int W, double thre
  * Marker = run_bit | run_len << 1 | literal_count << 33.  Replaces launch_ewah_emit (ewah.cuh:234-247). */
 int bsi_hip_ewah_emit(const uint64_t* words_device, int S, int W, const int32_t* flags_device,
                       const uint64_t* off_device, uint64_t* out_device, int32_t* out_len_device, void* stream);
+/* The fixed-bit build of a query batch (as bsi_hip_build_fixed without clipping) with the density flag and stream length of
+ * every slice in the same launch: words [Q, fixed_bits, W64], scales [Q, ceil(d / 256)] or [Q], weights [Q, fixed_bits]
+ * (slice weights, row scales only), flags / lens [Q * fixed_bits]; lens_host: the lengths again, in pinned host memory, each
+ * stored once.  BSI_ERR_UNSUPPORTED beyond 1024 words a slice or 8192 slices.  bsi_hip_ewah_emit_at: offsets and streams
+ * from the flags and lengths (lens 16-byte aligned). */
+int bsi_hip_build_measure(const void* x_device, int dtype, int64_t Q, int64_t d, int decimal_places, int fixed_bits, int chunk_scale,
+                          double threshold, uint64_t* words, float* scales, float* weights, int32_t* flags, int32_t* lens,
+                          int32_t* lens_host, void* stream);
+int bsi_hip_ewah_emit_at(const uint64_t* words_device, int S, int W, const int32_t* flags_device, const int32_t* lens_device,
+                         int64_t* off_device, uint64_t* out_device, void* stream);
 /* One stream -> W literal words.  Replaces launch_ewah_decompress (ewah.cuh:35-42). */
 int bsi_hip_ewah_decompress(const uint64_t* in_device, int in_len, int W, uint64_t* out_device, void* stream);
 /* S streams (stream s at comp + off[s], len[s] words) -> canonical [S, W]; the batched form the
