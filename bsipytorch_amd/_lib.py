@@ -89,7 +89,7 @@ PROTOTYPES = {
     "bsi_hip_dot_weighted_f64": [_vp, _vp, _i, _i, _vp, _i, _vp, _i, _i64, _i64, _vp, _i64, _vp, _vp],
     "bsi_hip_quantize_trunc_to_int64": [_vp, _i, _i64, _f, _vp, _vp],
     "bsi_hip_scalar_query_max_elems": [],
-    "bsi_hip_scalar_query_host_words": [_i64, _i64],
+    "bsi_hip_scalar_query_host_words": [_i64],
     "bsi_hip_scalar_query_dot": [_vp, _i64, _i, _d, _vp, _vp, _i, _i64, _d, _vp, _vp, _vp, _vp, _vp, _vp],
     "bsi_hip_dot_timed": [_vp, _vp, _vp, _i, _i, _i, _vp, _i, _vp, _i, _i64, _i64, _f, _i64, _vp, _i, _vp, _sz, _i,
                           ctypes.POINTER(_f), _vp],

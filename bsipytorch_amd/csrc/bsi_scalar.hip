@@ -1,14 +1,16 @@
 // The scalar entry points' one query against prebuilt decimal keys, in one launch: every workgroup builds the query for
 // itself, in LDS.
 #include "bsi_ewah_device.h"
+#include "bsi_quant_device.h"
 
 #include <chrono>
 
 namespace bsi {
 
 constexpr int kScalarBlock = 512, kScalarWaves = kScalarBlock / BSI_WAVE;
-constexpr int64_t kScalarMaxElems = 16384;  // 64 planes of it fill 128 KiB of LDS; a longer vector takes the batched builder
+constexpr int64_t kScalarMaxElems = 12288;  // 64 planes of it and the vector take 144 KiB of LDS; a longer one the batched builder
 constexpr int kScalarMaxGroups = 512;       // two workgroups for each CU; more rows are looped over
+constexpr int kScalarStamps = 16;           // workgroups that report their clock
 constexpr unsigned long long kScalarPending = 0xFFF8DEADFFFFBEEFULL;  // a NaN no score has, and no count or clock value
 
 __device__ __forceinline__ void store_host(unsigned long long* p, unsigned long long v) {
@@ -18,88 +20,103 @@ __device__ __forceinline__ void store_host(unsigned long long* p, unsigned long 
 // out[r] = sum_{i,j,w} popcount(A[i, w] & B[r, j, w]) * Aw[i] * Bw[r, j], exact in float64 while below 2^53, where A are the
 // planes of the decimal build of x (round half away from zero of x * 10^dec, the slice count from the largest magnitude).
 // host: {slices, whether a value is negative, words of the stored form, run-length coded slices}, three clock values of
-// every workgroup (begin, query built, end), then the R scores: pinned memory, each word stored once, so that the host sees
-// from the words themselves that all have come and waits for no event.
-// kLanes lanes share a key row, a word each.  A lane puts its popcounts together over the query's slices in integers (two
-// v_bcnt and one shift a pair of slices), four key slices at a time, and multiplies by the key's weights once.  The last
-// workgroup measures the stored form (density flag and EWAH length of every slice) instead of rows.
-// Bound by latency: the first key words are requested before the query is built.  The build costs every workgroup 2 us and
-// saves the launch of its own, with one busy CU, that it was before (9.0 + 6.8 us for 2048 elements against 1024 keys).
-template <int kLanes>
+// kScalarStamps workgroups (begin, query built, end), then the R scores: pinned memory, each word stored once, so that the
+// host sees from the words themselves that all have come and waits for no event.
+// A wave takes a key row: kWords words by 64 / kWords parts of its slices.  A lane puts its popcounts together over the
+// query's slices in integers (two v_and, two v_bcnt and a shift a pair of slices), three key slices at a time, and
+// multiplies by the key's weights once.  The last workgroup measures the stored form (density flag and EWAH length of every
+// slice) instead of rows.
+// Bound by latency and by VALU issue in the slicing and the popcounts; the first key words are requested before the query is
+// built.  Every workgroup building it costs less than the launch of its own, with one busy CU, that the build was before.
+// 2048 elements against 1024 keys: 9.0 + 6.8 us in two launches, 5.3 us in this one.
+template <int kWords>
 __global__ __launch_bounds__(kScalarBlock) void scalar_query_dot_kernel(const float* __restrict__ x, int d, int W, double dec_scale,
-                                                                        double threshold, const unsigned long long* __restrict__ B,
+                                                                        int narrow, double threshold, const unsigned long long* __restrict__ B,
                                                                         const float* __restrict__ Bw, int Sb, int R,
                                                                         unsigned long long* __restrict__ host) {
-    extern __shared__ unsigned long long As[];  // [slices][W]
-    constexpr int kRows = kScalarBlock / kLanes;
-    constexpr int kAhead = 8;                   // key slices requested up front
-    constexpr int kHeld = 8;                    // words of the query a wave keeps in registers between its two passes
-    __shared__ unsigned long long smax[kScalarWaves];
-    __shared__ int sneg[kScalarWaves];
+    extern __shared__ __attribute__((aligned(16))) unsigned long long As[];  // [64 slices][W], then x in whole chunks
+    constexpr int kRows = kScalarWaves, kParts = BSI_WAVE / kWords;
+    constexpr int kTogether = 3, kAhead = 2 * kTogether;  // key slices of a lane taken together, requested up front
+    float* const xs = reinterpret_cast<float*>(As + static_cast<size_t>(64) * W);
+    __shared__ uint2 smax[kScalarWaves];
     __shared__ double scores[kRows];
     const unsigned long long began = wall_clock64();
     const int tid = threadIdx.x, lane = tid & (BSI_WAVE - 1), wave = tid >> 6;
     const bool measures = blockIdx.x == gridDim.x - 1;
-    const int l = tid % kLanes, r0 = blockIdx.x * kRows + tid / kLanes;
+    const int l = lane % kWords, part = lane / kWords, r0 = blockIdx.x * kRows + wave;
+    // the vector into LDS, and its largest magnitude as float bits (the rounded magnitudes are in the same order; a NaN is
+    // rounded to the largest one, and to a negative value); the loads of a CU return in order: these before the keys'
+    unsigned m = 0u, mneg = 0u;
+    const int chunks = (d + BSI_CHUNK_ELEMS - 1) / BSI_CHUNK_ELEMS;
+    for (int e = tid; e < chunks * BSI_CHUNK_ELEMS; e += kScalarBlock) {
+        const float f = e < d ? x[e] : 0.0f;
+        xs[e] = f;
+        const unsigned bits = __float_as_uint(f) & 0x7fffffffu;
+        const unsigned nbits = f >= 0.0f ? 0u : bits;
+        m = bits > m ? bits : m;
+        mneg = nbits > mneg ? nbits : mneg;
+    }
     unsigned long long ahead[kAhead];
     {
         const int r = r0 < R ? r0 : R - 1, w = l < W ? l : W - 1;
 #pragma unroll
         for (int j = 0; j < kAhead; ++j)
-            ahead[j] = B[(static_cast<size_t>(r) * Sb + (j < Sb ? j : Sb - 1)) * W + w];
+            ahead[j] = B[(static_cast<size_t>(r) * Sb + (part + kParts * j < Sb ? part + kParts * j : Sb - 1)) * W + w];
     }
-
-    // the query: largest magnitude, then its planes
-    auto value = [&](int w) {
-        const int e = w * BSI_WAVE + lane;
-        const float f = x[e < d ? e : d - 1];
-        return e < d ? round_scaled(f, dec_scale) : 0LL;
-    };
-    long long held[kHeld];
-    unsigned long long m = 0ULL;
-    int neg = 0;
-    auto look = [&](long long v) {
-        const unsigned long long a = uabs_ll(v);
-        m = a > m ? a : m;
-        neg |= v < 0;
-    };
-#pragma unroll
-    for (int k = 0; k < kHeld; ++k) held[k] = value(wave + k * kScalarWaves);  // past the vector: zeros
-#pragma unroll
-    for (int k = 0; k < kHeld; ++k) look(held[k]);
-    for (int w = wave + kHeld * kScalarWaves; w < W; w += kScalarWaves) look(value(w));
-    m = wave_max_u64(m);
-    neg = __any(neg) ? 1 : 0;
-    if (lane == 0) {
-        smax[wave] = m;
-        sneg[wave] = neg;
-    }
+    m = wave_max_u32(m);
+    mneg = wave_max_u32(mneg);
+    if (lane == 0) smax[wave] = make_uint2(m, mneg);
     __syncthreads();
-    m = 0ULL;
-    neg = 0;
 #pragma unroll
     for (int w = 0; w < kScalarWaves; ++w) {
-        m = smax[w] > m ? smax[w] : m;
-        neg |= sneg[w];
+        m = smax[w].x > m ? smax[w].x : m;
+        mneg = smax[w].y > mneg ? smax[w].y : mneg;
     }
-    int S = m == 0ULL ? 2 : 64 - __clzll(static_cast<long long>(m)) + 2;  // the decimal builder's rule (bsi_vector_cuda.cpp:746-754)
+    const unsigned long long largest = uabs_ll(round_scaled(__uint_as_float(m), dec_scale));
+    const bool neg = uabs_ll(round_scaled(__uint_as_float(mneg), dec_scale)) != 0ULL;
+    int S = largest == 0ULL ? 2 : 64 - __clzll(static_cast<long long>(largest)) + 2;  // the decimal builder's rule (bsi_vector_cuda.cpp:746-754)
     if (S > 64) S = 64;
     S = __builtin_amdgcn_readfirstlane(S);
-    auto slice = [&](long long v, int w) {
-        unsigned long long mine = 0ULL;
-        for (int s = 0; s < S; ++s) {
-            const unsigned long long word = __ballot((static_cast<unsigned long long>(v) >> s) & 1ULL);
-            if (lane == s) mine = word;
-        }
-        if (lane < S) As[static_cast<size_t>(lane) * W + w] = mine;
-    };
+
+    // its planes.  Where every |x| (and 10^dec: narrow) is in the float32 quantiser's range the magnitudes are 32-bit integers:
+    // a wave takes a chunk of 256, and every byte of the integers goes through the builders' transposes (bsi_quant_device.h).
+    if (narrow && m < kQuantWideBits) {
+        const float scale = static_cast<float>(dec_scale);
+        const ChunkLane cl = chunk_lane(lane);
+        uint32_t* const As32 = reinterpret_cast<uint32_t*>(As);
+        for (int c = wave; c < chunks; c += kScalarWaves) {
+            const float4 f = *reinterpret_cast<const float4*>(xs + c * BSI_CHUNK_ELEMS + cl.quad);
+            const float fs[4] = {f.x, f.y, f.z, f.w};
+            uint32_t v[4];
 #pragma unroll
-    for (int k = 0; k < kHeld; ++k)
-        if (wave + k * kScalarWaves < W) slice(held[k], wave + k * kScalarWaves);
-    for (int w = wave + kHeld * kScalarWaves; w < W; w += kScalarWaves) slice(value(w), w);
+            for (int k = 0; k < 4; ++k) {
+                const int a = static_cast<int>(scaled_magnitude_f32<float>(fabsf(fs[k]), scale));
+                v[k] = static_cast<uint32_t>(fs[k] < 0.0f ? -a : a);
+            }
+            const int unit = c * 8 + (lane >> 3);
+            for (int s0 = 0; s0 < S; s0 += 8) {
+                const uint32_t plane = chunk_plane_dword(chunk_image_dword(pack_low_bytes(v[0], v[1], v[2], v[3]), cl), cl);
+                const int s = s0 + (lane & 7);
+                if (s < S && unit < 2 * W) As32[s * 2 * W + unit] = plane;
+#pragma unroll
+                for (int k = 0; k < 4; ++k) v[k] >>= 8;
+            }
+        }
+    } else {
+        for (int w = wave; w < W; w += kScalarWaves) {
+            const unsigned long long v = static_cast<unsigned long long>(round_scaled(xs[w * BSI_WAVE + lane], dec_scale));
+            unsigned long long mine = 0ULL;
+            for (int s = 0; s < S; ++s) {
+                const unsigned long long word = __ballot((v >> s) & 1ULL);
+                if (lane == s) mine = word;
+            }
+            if (lane < S) As[static_cast<size_t>(lane) * W + w] = mine;
+        }
+    }
     __syncthreads();
     const unsigned long long built = wall_clock64();
-    unsigned long long* const stamps = host + 4 + 3 * static_cast<size_t>(blockIdx.x);
+    const unsigned stamp = measures ? (gridDim.x < kScalarStamps ? gridDim.x : kScalarStamps) - 1 : blockIdx.x;
+    unsigned long long* const stamps = host + 4 + 3 * stamp;
 
     if (measures) {
         __shared__ unsigned long long swords[kScalarWaves];
@@ -127,75 +144,76 @@ __global__ __launch_bounds__(kScalarBlock) void scalar_query_dot_kernel(const fl
                 coded += scoded[w];
             }
             store_host(host, static_cast<unsigned long long>(S));
-            store_host(host + 1, static_cast<unsigned long long>(neg));
+            store_host(host + 1, neg ? 1ULL : 0ULL);
             store_host(host + 2, words);
             store_host(host + 3, static_cast<unsigned long long>(coded));
         }
     } else {
-        unsigned long long* const out = host + 4 + 3 * static_cast<size_t>(gridDim.x);
+        unsigned long long* const out = host + 4 + 3 * (gridDim.x < kScalarStamps ? gridDim.x : kScalarStamps);
         const int stride = (gridDim.x - 1) * kRows;
         for (int rb = blockIdx.x * kRows; rb < R; rb += stride) {
-            const int r = rb + tid / kLanes;
+            const int r = rb + wave;
             double acc = 0.0;
-            auto four = [&](const unsigned long long (&b)[4], int w, int j0) {
-                double part[4];
-                auto combine = [&](auto zero) {
-                    decltype(zero) t[4] = {zero, zero, zero, zero};
-                    for (int i = S - 1; i >= 0; --i) {
-                        const unsigned long long a = As[i * W + w];
-#pragma unroll
-                        for (int u = 0; u < 4; ++u) {
-                            const int c = __popcll(a & b[u]);
-                            t[u] = t[u] * 2 + ((neg && i == S - 1) ? -c : c);
-                        }
-                    }
-#pragma unroll
-                    for (int u = 0; u < 4; ++u) part[u] = static_cast<double>(t[u]);
-                };
-                if (S <= 24) combine(0);              // 64 * 2^24 < 2^31
-                else if (S <= 56) combine(0LL);       // 64 * 2^56 < 2^63
-                else combine(0.0);
-#pragma unroll
-                for (int u = 0; u < 4; ++u)
-                    if (j0 + u < Sb) acc += part[u] * static_cast<double>(Bw[static_cast<size_t>(r) * Sb + j0 + u]);
-            };
             if (r < R) {
                 const unsigned long long* row = B + static_cast<size_t>(r) * Sb * W;
-                for (int w = l; w < W; w += kLanes) {
+#pragma unroll 1
+                for (int w = l; w < W; w += kWords) {
                     const bool first = rb == static_cast<int>(blockIdx.x) * kRows && w == l;
-                    for (int j0 = 0; j0 < Sb; j0 += 4) {
-                        unsigned long long b[4];
+#pragma unroll 1
+                    for (int i0 = 0; i0 * kParts < Sb; i0 += kTogether) {
+                        unsigned long long b[kTogether];
 #pragma unroll
-                        for (int u = 0; u < 4; ++u) {
-                            if (first && j0 < kAhead) b[u] = j0 == 0 ? ahead[u] : ahead[4 + u];
-                            else b[u] = row[static_cast<size_t>(j0 + u < Sb ? j0 + u : Sb - 1) * W + w];
+                        for (int u = 0; u < kTogether; ++u) {
+                            const int j = part + kParts * (i0 + u);
+                            if (first && i0 < kAhead) b[u] = i0 == 0 ? ahead[u] : ahead[kTogether + u];
+                            else b[u] = row[static_cast<size_t>(j < Sb ? j : Sb - 1) * W + w];
                         }
-                        four(b, w, j0);
+                        double part_sum[kTogether];
+                        auto combine = [&](auto zero) {
+                            decltype(zero) t[kTogether];
+                            const unsigned long long top = As[(S - 1) * W + w];
+#pragma unroll
+                            for (int u = 0; u < kTogether; ++u) {
+                                const int c = __popcll(top & b[u]);
+                                t[u] = neg ? -c : c;
+                            }
+#pragma unroll 4
+                            for (int i = S - 2; i >= 0; --i) {
+                                const unsigned long long a = As[i * W + w];
+#pragma unroll
+                                for (int u = 0; u < kTogether; ++u) t[u] = t[u] * 2 + __popcll(a & b[u]);
+                            }
+#pragma unroll
+                            for (int u = 0; u < kTogether; ++u) part_sum[u] = static_cast<double>(t[u]);
+                        };
+                        if (S <= 24) combine(0);              // 64 * 2^24 < 2^31
+                        else if (S <= 56) combine(0LL);       // 64 * 2^56 < 2^63
+                        else combine(0.0);
+#pragma unroll
+                        for (int u = 0; u < kTogether; ++u) {
+                            const int j = part + kParts * (i0 + u);
+                            if (j < Sb) acc += part_sum[u] * static_cast<double>(Bw[static_cast<size_t>(r) * Sb + j]);
+                        }
                     }
                 }
             }
 #pragma unroll
-            for (int off = kLanes / 2; off > 0; off >>= 1) acc += __shfl_xor(acc, off, BSI_WAVE);
-            if (l == 0) scores[tid / kLanes] = acc;
+            for (int off = BSI_WAVE / 2; off > 0; off >>= 1) acc += __shfl_xor(acc, off, BSI_WAVE);
+            if (lane == 0) scores[wave] = acc;
             __syncthreads();
             if (tid < kRows && rb + tid < R) store_host(out + rb + tid, static_cast<unsigned long long>(__double_as_longlong(scores[tid])));
             __syncthreads();
         }
     }
-    if (tid == 0) {
+    if (tid == 0 && (measures || stamp < kScalarStamps - 1)) {
         store_host(stamps, began);
         store_host(stamps + 1, built);
         store_host(stamps + 2, wall_clock64());
     }
 }
 
-static int scalar_lanes(int64_t d) {  // the lanes of a row cover its words where they can
-    const int64_t W = (d + 63) / 64;
-    return W > 32 ? 64 : (W > 16 ? 32 : 16);
-}
-static int64_t scalar_groups(int64_t d, int64_t R) {
-    const int rows = kScalarBlock / scalar_lanes(d);
-    const int64_t groups = (R + rows - 1) / rows;
+static int64_t scalar_groups(int64_t R) {
+    const int64_t groups = (R + kScalarWaves - 1) / kScalarWaves;
     return 1 + (groups < kScalarMaxGroups ? groups : kScalarMaxGroups);
 }
 
@@ -205,7 +223,10 @@ using namespace bsi;
 
 extern "C" int64_t bsi_hip_scalar_query_max_elems(void) { return kScalarMaxElems; }
 
-extern "C" int64_t bsi_hip_scalar_query_host_words(int64_t d, int64_t R) { return 4 + 3 * scalar_groups(d, R) + R; }
+extern "C" int64_t bsi_hip_scalar_query_host_words(int64_t R) {
+    const int64_t groups = scalar_groups(R);
+    return 4 + 3 * (groups < kScalarStamps ? groups : kScalarStamps) + R;
+}
 
 extern "C" int bsi_hip_scalar_query_dot(const float* x, int64_t d, int decimal_places, double threshold, const uint64_t* B,
                                         const float* Bw, int Sb, int64_t R, double divisor, uint64_t* pinned, double* out,
@@ -223,22 +244,23 @@ extern "C" int bsi_hip_scalar_query_dot(const float* x, int64_t d, int decimal_p
         clock_khz.store(khz > 0 ? khz : 100000, std::memory_order_relaxed);
     }
     const int W = static_cast<int>((d + 63) / 64);
-    const int64_t groups = scalar_groups(d, R), words = bsi_hip_scalar_query_host_words(d, R);
+    const int64_t groups = scalar_groups(R), words = bsi_hip_scalar_query_host_words(R), stamped = (words - R - 4) / 3;
     volatile unsigned long long* const host = reinterpret_cast<volatile unsigned long long*>(pinned);
     for (int64_t i = 0; i < words; ++i) host[i] = kScalarPending;
     std::atomic_thread_fence(std::memory_order_seq_cst);
+    const double dec_scale = pow(10.0, static_cast<double>(decimal_places));
+    const int narrow = integer_decimal_scale(dec_scale) != 0 ? 1 : 0;
 #define BSI_SCALAR_DOT(L)                                                                                                  \
     {                                                                                                                      \
         static LdsOptIn once;                                                                                              \
-        lds_opt_in(once, reinterpret_cast<const void*>(&scalar_query_dot_kernel<L>), 64 * 256 * 8);                        \
-        launch(scalar_query_dot_kernel<L>, dim3(static_cast<unsigned>(groups)), dim3(kScalarBlock), static_cast<size_t>(64) * W * 8, \
-               st, x, static_cast<int>(d), W, pow(10.0, static_cast<double>(decimal_places)), threshold,                   \
+        lds_opt_in(once, reinterpret_cast<const void*>(&scalar_query_dot_kernel<L>), kScalarMaxElems * 12);                       \
+        launch(scalar_query_dot_kernel<L>, dim3(static_cast<unsigned>(groups)), dim3(kScalarBlock), static_cast<size_t>(W) * 512 + static_cast<size_t>((W + 3) / 4) * 1024, \
+               st, x, static_cast<int>(d), W, dec_scale, narrow, threshold,                   \
                reinterpret_cast<const unsigned long long*>(B), Bw, Sb, static_cast<int>(R),                                \
                reinterpret_cast<unsigned long long*>(pinned));                                                             \
     }
-    const int lanes = scalar_lanes(d);
-    if (lanes == 64) BSI_SCALAR_DOT(64)
-    else if (lanes == 32) BSI_SCALAR_DOT(32)
+    if (W > 32) BSI_SCALAR_DOT(64)
+    else if (W > 16) BSI_SCALAR_DOT(32)
     else BSI_SCALAR_DOT(16)
 #undef BSI_SCALAR_DOT
     BSI_LAUNCH_CHECK("scalar_query_dot_kernel");
@@ -257,7 +279,7 @@ extern "C" int bsi_hip_scalar_query_dot(const float* x, int64_t d, int decimal_p
     for (int64_t i = 0; i < words; ++i) BSI_HIP_CHECK(word(i));
     const volatile unsigned long long* const stamps = host + 4;
     unsigned long long began = stamps[0], built = stamps[1], ended = stamps[2];
-    for (int64_t g = 1; g < groups; ++g) {
+    for (int64_t g = 1; g < stamped; ++g) {
         if (stamps[3 * g] < began) began = stamps[3 * g];
         if (stamps[3 * g + 1] > built) built = stamps[3 * g + 1];
         if (stamps[3 * g + 2] > ended) ended = stamps[3 * g + 2];
@@ -266,7 +288,7 @@ extern "C" int bsi_hip_scalar_query_dot(const float* x, int64_t d, int decimal_p
     *build_ns = static_cast<int64_t>(static_cast<double>(built - began) * ns);
     *dot_ns = static_cast<int64_t>(static_cast<double>(ended - built) * ns);
     for (int i = 0; i < 4; ++i) info[i] = static_cast<int64_t>(host[i]);
-    const volatile double* const scores = reinterpret_cast<const volatile double*>(host + 4 + 3 * groups);
+    const volatile double* const scores = reinterpret_cast<const volatile double*>(host + 4 + 3 * stamped);
     for (int64_t r = 0; r < R; ++r) out[r] = scores[r] / divisor;
     return BSI_OK;
 }

@@ -582,17 +582,20 @@ PyObject* hybrid(PyObject*, PyObject* args) {
     if (!chunked) weights = at::detail::empty_cuda({Q, config.bits}, at::kFloat, device, std::nullopt);
     at::Tensor flags = at::detail::empty_cuda({S}, at::kInt, device, std::nullopt);
     at::Tensor lens = at::detail::empty_cuda({S}, at::kInt, device, std::nullopt);
-    at::Tensor off = at::detail::empty_cuda({S}, at::kLong, device, std::nullopt);
     at::Tensor pinned = at::detail::empty_cpu({S}, at::kInt, /*pin_memory=*/true);
     volatile int32_t* const host = static_cast<volatile int32_t*>(pinned.data_ptr());
     uint64_t* const w = static_cast<uint64_t*>(words.data_ptr());
     int64_t total = 0;
-    int rc = BSI_OK;
-    Py_BEGIN_ALLOW_THREADS
     for (int64_t s = 0; s < S; ++s) host[s] = -1;
-    rc = lib.build_measure(x.const_data_ptr(), code, Q, d, decimals, config.bits, chunked ? 1 : 0, threshold, w,
+    int rc = lib.build_measure(x.const_data_ptr(), code, Q, d, decimals, config.bits, chunked ? 1 : 0, threshold, w,
                            static_cast<float*>(scales.data_ptr()), chunked ? nullptr : static_cast<float*>(weights.data_ptr()),
                            static_cast<int32_t*>(flags.data_ptr()), static_cast<int32_t*>(lens.data_ptr()), const_cast<int32_t*>(host), st);
+    if (rc != BSI_OK) return fail_status(rc, "bsi_hip_build_measure");
+    // what can be made before the lengths are here
+    at::Tensor off = at::detail::empty_cuda({S}, at::kLong, device, std::nullopt);
+    Holder b(THPVariable_Wrap(off)), c(THPVariable_Wrap(lens)), f(THPVariable_Wrap(flags)), s(THPVariable_Wrap(std::move(scales))),
+        v(THPVariable_Wrap(std::move(weights)));
+    Py_BEGIN_ALLOW_THREADS
     // the stream is waited for only if the lengths are long in coming
     const auto until = std::chrono::steady_clock::now() + std::chrono::microseconds(500);
     bool waited = false;
@@ -607,14 +610,11 @@ PyObject* hybrid(PyObject*, PyObject* args) {
     Py_END_ALLOW_THREADS
     if (rc != BSI_OK) return fail_status(rc, "bsi_hip_build_measure");
     at::Tensor streams = at::detail::empty_cuda({total}, at::kLong, device, std::nullopt);
-    Py_BEGIN_ALLOW_THREADS
     rc = lib.ewah_emit_at(w, static_cast<int>(S), static_cast<int>(W), static_cast<const int32_t*>(flags.data_ptr()),
                           static_cast<const int32_t*>(lens.data_ptr()), static_cast<int64_t*>(off.data_ptr()),
                           static_cast<uint64_t*>(streams.data_ptr()), st);
-    Py_END_ALLOW_THREADS
     if (rc != BSI_OK) return fail_status(rc, "bsi_hip_ewah_emit_at");
-    Holder a(THPVariable_Wrap(std::move(streams))), b(THPVariable_Wrap(std::move(off))), c(THPVariable_Wrap(std::move(lens))),
-        f(THPVariable_Wrap(std::move(flags))), s(THPVariable_Wrap(std::move(scales))), v(THPVariable_Wrap(std::move(weights)));
+    Holder a(THPVariable_Wrap(std::move(streams)));
     return PyTuple_Pack(6, a.p, b.p, c.p, f.p, s.p, v.p);
     END_HANDLE_TH_ERRORS
 }
@@ -695,7 +695,7 @@ PyObject* scalar_query(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     if (capturing(st)) Py_RETURN_NONE;
     const int64_t R = words.size(0);
     at::Tensor out = at::detail::empty_cpu({R}, at::kDouble);
-    at::Tensor pinned = at::detail::empty_cpu({lib.scalar_query_host_words(d, R)}, at::kLong, /*pin_memory=*/true);
+    at::Tensor pinned = at::detail::empty_cpu({lib.scalar_query_host_words(R)}, at::kLong, /*pin_memory=*/true);
     int64_t info[4] = {0, 0, 0, 0}, build_ns = 0, dot_ns = 0;
     int rc = BSI_OK;
     Py_BEGIN_ALLOW_THREADS

@@ -76,11 +76,11 @@ int bsi_hip_quantize_trunc_to_int64(const void* x_device, int dtype, int64_t tot
  * when the call returns: x [d] float32 is built in decimal mode on the device (slice count from its largest magnitude), then
  * out[r] = the exact integer dot with key row r (canonical planes B [R, Sb, W64], slice weights Bw [R, Sb]) as float64,
  * divided by `divisor`.  info [4]: {slices, whether a value is negative, words the slices take in stored form at
- * `threshold`, run-length coded slices}.  pinned: bsi_hip_scalar_query_host_words(d, R) words of pinned host memory;
+ * `threshold`, run-length coded slices}.  pinned: bsi_hip_scalar_query_host_words(R) words of pinned host memory;
  * out, info: host memory.  build_ns / dot_ns: device-clock times of the two parts.  d at most
  * bsi_hip_scalar_query_max_elems(). */
 int64_t bsi_hip_scalar_query_max_elems(void);
-int64_t bsi_hip_scalar_query_host_words(int64_t d, int64_t R);
+int64_t bsi_hip_scalar_query_host_words(int64_t R);
 int bsi_hip_scalar_query_dot(const float* x_device, int64_t d, int decimal_places, double threshold, const uint64_t* B,
                              const float* Bw, int Sb, int64_t R, double divisor, uint64_t* pinned, double* out, int64_t* info,
                              int64_t* build_ns, int64_t* dot_ns, void* stream);
