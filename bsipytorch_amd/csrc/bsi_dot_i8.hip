@@ -118,6 +118,21 @@ __device__ unsigned long long g_timeline_cycles[kTimelineWorkgroups * 8];  // th
 #define BSI_STAMP(slot)
 #endif
 
+// A loader wave's share of a region that the next dot will read: one lane per 128-byte line, 64 lines per load.  The values
+// are summed only so that the loads stay; the store never happens.
+template <int kLoaders>
+__device__ __forceinline__ void i8_warm_lines(unsigned char* __restrict__ unused_lds, int lw, int lane, const unsigned char* __restrict__ warm,
+                                              long long warm_lines) {
+    const long long waves = static_cast<long long>(gridDim.x) * gridDim.y * gridDim.z * kLoaders;
+    const long long mine = ((static_cast<long long>(blockIdx.z) * gridDim.y + blockIdx.y) * gridDim.x + blockIdx.x) * kLoaders + lw;
+    const long long per = (warm_lines + waves - 1) / waves;
+    const long long first = mine * per;
+    const long long last = (first + per < warm_lines) ? first + per : warm_lines;
+    unsigned sum = 0;
+    for (long long l = first + lane; l < last; l += 64) sum += *reinterpret_cast<const volatile unsigned*>(warm + l * 128);
+    if (sum == 0x5ca1ab1eu && warm_lines < 0) unused_lds[lane] = 0;
+}
+
 // A loader wave of the int8-image kernels (lw = its number among the C::kLoaders loader waves; `consumers` MFMA
 // waves share the workgroup's barriers with it): 8 of the stage's groups of 8 rows (the TM key rows, then the TN
 // query rows: a load moves 1 KiB = 8 rows x 128 bytes), plus the chunk scales of 64 queries once per chunk.
@@ -257,19 +272,7 @@ __device__ __forceinline__ void i8_loader_wave(unsigned char* __restrict__ lds, 
         }
         lds_barrier();
     }
-    if (warm_lines > 0) {
-        // one lane per 128-byte line, 64 lines per load; this loader wave's share of the region.  The values
-        // are summed only so that the loads stay; the store below never happens.
-        const long long waves = static_cast<long long>(gridDim.x) * gridDim.y * gridDim.z * C::kLoaders;
-        const long long mine = ((static_cast<long long>(blockIdx.z) * gridDim.y + blockIdx.y) * gridDim.x + blockIdx.x) * C::kLoaders + lw;
-        const long long per = (warm_lines + waves - 1) / waves;
-        const long long first = mine * per;
-        const long long last = (first + per < warm_lines) ? first + per : warm_lines;
-        unsigned sum = 0;
-        for (long long l = first + lane; l < last; l += 64)
-            sum += *reinterpret_cast<const volatile unsigned*>(warm + l * 128);
-        if (sum == 0x5ca1ab1eu && warm_lines < 0) scale_lds[lane] = 0;
-    }
+    if (warm_lines > 0) i8_warm_lines<L>(scale_lds, lw, lane, warm, warm_lines);
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // nothing may still be writing LDS when the workgroup ends
 }
 
@@ -409,6 +412,61 @@ __device__ __forceinline__ void i8_store_half(const float (&v)[WM][WN][4], const
         }
 }
 
+// The end of a tile in the chain modes: every output takes its key's factor, the decimal scale and the bias, and is stored.
+// epi: the key factors and biases of the tile's TM rows, from the copy the loader waves staged in LDS (0 for rows past R and
+// for a call without bias): two 16-byte reads per 16-key tile.
+template <int TM, int WM, int WN, bool kHalf>
+__device__ __forceinline__ void i8_store_tile(const float (&accf)[WM][WN][4], const unsigned char* __restrict__ epi_lds, float down,
+                                              float scale_inv, bool has_bias, int out_dtype, float* __restrict__ out,
+                                              int64_t R_total, int64_t r0, int64_t q0, int wr, int wq, int64_t R, int64_t Q,
+                                              int ln, int lg, bool stream_out) {
+    const int64_t qw = q0 + wq * (WN * 16);
+    const float* epi = reinterpret_cast<const float*>(epi_lds);
+#pragma unroll
+    for (int a0 = 0; a0 < WM; a0 += 2) {  // two 16-key tiles at a time: what the stores pair up
+        const int64_t rw = r0 + wr * (WM * 16) + a0 * 16;
+        float v[2][WN][4], bi[2][4];
+#pragma unroll
+        for (int a = 0; a < 2; ++a) {
+            const int rl = wr * (WM * 16) + (a0 + a) * 16 + lg * 4;  // row of the tile
+            const float4 w4 = *reinterpret_cast<const float4*>(epi + rl);
+            const float4 b4 = *reinterpret_cast<const float4*>(epi + TM + rl);
+            const float bs[4] = {key_factor(w4.x), key_factor(w4.y), key_factor(w4.z), key_factor(w4.w)};
+            bi[a][0] = b4.x, bi[a][1] = b4.y, bi[a][2] = b4.z, bi[a][3] = b4.w;
+#pragma unroll
+            for (int b = 0; b < WN; ++b)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    // (acc * key scale) * scale_inv, then + bias: each step rounded on its own, as separate kernels would
+                    v[a][b][e] = ((accf[a0 + a][b][e] * down) * bs[e]) * scale_inv;
+                    if (has_bias && out_dtype == BSI_DTYPE_F32) v[a][b][e] = v[a][b][e] + bi[a][e];
+                }
+        }
+        if (kHalf && out_dtype != BSI_DTYPE_F32) {
+            i8_store_half<2, WN>(v, bi, has_bias, out_dtype, out, R_total, rw, qw, R, Q, ln, lg);
+            continue;
+        }
+        if (i8_store_lines<2, WN>(v, out, R_total, rw, qw, R, Q, ln, lg, stream_out)) continue;
+#pragma unroll
+        for (int a = 0; a < 2; ++a) {
+            const int64_t rb = rw + a * 16 + lg * 4;
+#pragma unroll
+            for (int b = 0; b < WN; ++b) {
+                const int64_t q = qw + b * 16 + ln;
+                if (q >= Q) continue;
+                float* dst = out + static_cast<size_t>(q) * R_total + rb;
+                if (rb + 3 < R && ((reinterpret_cast<uintptr_t>(dst) & 15) == 0)) {
+                    *reinterpret_cast<float4*>(dst) = make_float4(v[a][b][0], v[a][b][1], v[a][b][2], v[a][b][3]);
+                } else {
+#pragma unroll
+                    for (int e = 0; e < 4; ++e)
+                        if (rb + e < R) dst[e] = v[a][b][e];
+                }
+            }
+        }
+    }
+}
+
 // Which tile a workgroup takes.  Workgroups go to the eight XCDs in turn, and every XCD has an L2 of its own.  Plain order
 // (blockIdx = tile, key tile fastest) gives an XCD the same key tiles in every row of tiles where their number is a multiple
 // of 8; elsewhere every XCD came to fetch nearly all keys, once for each query tile.  There, XCD x takes a contiguous run of
@@ -421,11 +479,8 @@ struct I8Grid {
     unsigned by_band, by_height, by_last;  // floor(2^32 / n) + 1 of a band's tiles, its height, the last band's height; 0: n = 1
 };
 __device__ __forceinline__ unsigned divide_by(unsigned v, unsigned reciprocal) { return reciprocal != 0u ? __umulhi(v, reciprocal) : v; }
-__device__ __forceinline__ void i8_tile_of(const I8Grid& g, int& bx, int& by) {
-    bx = static_cast<int>(blockIdx.x);
-    by = static_cast<int>(blockIdx.y);
-    if (g.height == 0) return;
-    const unsigned id = blockIdx.x, total = static_cast<unsigned>(g.tiles_x) * static_cast<unsigned>(g.tiles_y);
+__device__ __forceinline__ void i8_tile_of(const I8Grid& g, unsigned id, int& bx, int& by) {
+    const unsigned total = static_cast<unsigned>(g.tiles_x) * static_cast<unsigned>(g.tiles_y);
     const unsigned xcd = id & 7u, per = total >> 3, rest = total & 7u;
     const unsigned at = (id >> 3) + xcd * per + (xcd < rest ? xcd : rest);
     const unsigned band = divide_by(at, g.by_band), in = at - band * static_cast<unsigned>(g.tiles_x * g.height);
@@ -489,7 +544,8 @@ __global__ __launch_bounds__((I8Cfg<TM, TN>::kBlock)) void dot_mfma_i8_kernel(
         by = (id / tiles_x) % tiles_y;
         seg = id / (tiles_x * tiles_y);
     } else {
-        i8_tile_of(plain_grid, bx, by);
+        bx = static_cast<int>(blockIdx.x), by = static_cast<int>(blockIdx.y);
+        if (plain_grid.height != 0) i8_tile_of(plain_grid, blockIdx.x, bx, by);
     }
     const int64_t r0 = static_cast<int64_t>(bx) * TM;
     const int64_t q0 = static_cast<int64_t>(by) * TN;
@@ -842,58 +898,260 @@ __global__ __launch_bounds__((I8Cfg<TM, TN>::kBlock)) void dot_mfma_i8_kernel(
                 if (kInts && int_off[a][b] >= 0 && e < int_rows[a])
                     chunk_ints[int_off[a][b] + static_cast<int64_t>(e) * chunks + (chunks - 1)] = v >> down_shift;
             }
-    // The key factors and biases of the wave's rows, from the copy the loader waves staged in LDS when the workgroup
-    // started (0 for rows past R and for a call without bias): two 16-byte reads per 16-key tile.
-    float bs[WM][4], bi[WM][4];
-    {
-        const float* epi = reinterpret_cast<const float*>(lds + 4 * C::kStage + C::kScaleBytes);
-#pragma unroll
-        for (int a = 0; a < WM; ++a) {
-            const int rl = wr * (WM * 16) + a * 16 + lg * 4;  // row of the tile
-            const float4 w4 = *reinterpret_cast<const float4*>(epi + rl);
-            const float4 b4 = *reinterpret_cast<const float4*>(epi + TM + rl);
-            bs[a][0] = key_factor(w4.x), bs[a][1] = key_factor(w4.y), bs[a][2] = key_factor(w4.z), bs[a][3] = key_factor(w4.w);
-            bi[a][0] = b4.x, bi[a][1] = b4.y, bi[a][2] = b4.z, bi[a][3] = b4.w;
-        }
-    }
-#pragma unroll
-    for (int a = 0; a < WM; ++a)
-#pragma unroll
-        for (int b = 0; b < WN; ++b)
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                // (acc * key scale) * scale_inv, then + bias: each step rounded on its own, as separate kernels would
-                float v = ((accf[a][b][e] * down) * bs[a][e]) * scale_inv;
-                if (bias != nullptr && out_dtype == BSI_DTYPE_F32) v = v + bi[a][e];
-                accf[a][b][e] = v;
-            }
-    if (kMode == kI8Chain && out_dtype != BSI_DTYPE_F32) {
-        i8_store_half<WM, WN>(accf, bi, bias != nullptr, out_dtype, out, R_total, r0 + wr * (WM * 16), q0 + wq * (WN * 16), R, Q, ln, lg);
-        return;
-    }
-    if (!i8_store_lines<WM, WN>(accf, out, R_total, r0 + wr * (WM * 16), q0 + wq * (WN * 16), R, Q, ln, lg, out_stream != 0)) {
-#pragma unroll
-        for (int a = 0; a < WM; ++a) {
-            const int64_t rb = r0 + wr * (WM * 16) + a * 16 + lg * 4;
-#pragma unroll
-            for (int b = 0; b < WN; ++b) {
-                const int64_t q = q0 + wq * (WN * 16) + b * 16 + ln;
-                if (q >= Q) continue;
-                float* dst = out + static_cast<size_t>(q) * R_total + rb;
-                if (rb + 3 < R && ((reinterpret_cast<uintptr_t>(dst) & 15) == 0)) {
-                    *reinterpret_cast<float4*>(dst) = make_float4(accf[a][b][0], accf[a][b][1], accf[a][b][2], accf[a][b][3]);
-                } else {
-#pragma unroll
-                    for (int e = 0; e < 4; ++e)
-                        if (rb + e < R) dst[e] = accf[a][b][e];
-                }
-            }
-        }
-    }
+    i8_store_tile<TM, WM, WN, kMode == kI8Chain>(accf, lds + 4 * C::kStage + C::kScaleBytes, down, scale_inv, bias != nullptr, out_dtype,
+                                                 out, R_total, r0, q0, wr, wq, R, Q, ln, lg, out_stream != 0);
 #ifdef BSI_TIMELINE
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the stamp below: the outputs have left the wave
     if (wave == 0) BSI_STAMP(kStampStored);
 #endif
+}
+
+// ------------------------------------------------------------------ int8 image, several tiles a workgroup
+//
+// Grids of more than one round: one workgroup per CU takes tiles `grid` apart and never drains its ring.  The loader waves go
+// on to the next tile's stages while the MFMA waves end one, so of what a workgroup of dot_mfma_i8_kernel spends outside the
+// chunk loop (4096 x 4096 x 16384, per tile: 15.0 us of loop, 1.7 to the first stage, 1.7 of stores, 0.9 until the next
+// workgroup starts) only the issue of the stores is left.  Same waves, ring, k-steps and chain, so the same bits.
+// us before and after: 4096 x 4096 x 16384 312, 294; 2048 x 2048 x 8192 47.1, 43.6; 2772 x 512 x 12800 46.7, 40.2;
+// 8192 x 1024 x 4096 58.1, 51.8; 1773 x 5376 x 8704 90.5, 88.3.  What is left at long rows is the chunk loop at the clock the
+// chip holds (1.7 GHz under this load): hiding the rest lowers it a little further.
+template <int TM, int TN>
+struct I8TilesCfg : I8Cfg<TM, TN> {
+    using C = I8Cfg<TM, TN>;
+    static constexpr int kLdsTiles = C::kLds + 3 * C::kEpilogueBytes;  // four sets of key factors and biases
+};
+
+// A loader wave: the stages of all the workgroup's tiles, one after the other; three stages ahead of the MFMA waves, across
+// the ends of tiles.
+template <typename C>
+__device__ __forceinline__ void i8_tiles_loader_wave(unsigned char* __restrict__ lds, int lw, int lane, const int8_t* __restrict__ A8,
+                                                     const float* __restrict__ qscale, int qscale_stride,
+                                                     const int8_t* __restrict__ K8, const float* __restrict__ Bw, int Sb, int chunks,
+                                                     int64_t R, int64_t Q, const float* __restrict__ bias, int key_tiled,
+                                                     const I8Grid& grid, unsigned tiles) {
+    constexpr int TM = C::kTM, TN = C::kTN;
+    constexpr int L = C::kLoaders, NI = C::kLoads, KG = TM / 8, QG = TN / 8;
+    constexpr int kEpi = (2 * (TM / 64) + L - 1) / L;
+    static_assert(KG % L == 0 && QG % L == 0 && NI == KG / L + QG / L, "loads per loader wave");
+    const uint32_t rowbytes = static_cast<uint32_t>(chunks) << 8, kblock = static_cast<uint32_t>(chunks) << 14;
+    const uint32_t lr = static_cast<uint32_t>(lane) >> 3, lc = static_cast<uint32_t>(lane) & 7;
+    uint32_t voff[NI];
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+        const bool is_key = i < KG / L;
+        const int gg = is_key ? lw + L * i : lw + L * (i - KG / L);
+        const uint32_t col = (lc ^ (static_cast<uint32_t>(gg & 1) * 4 + (lr >> 1))) * 16;
+        const bool tiled = is_key && key_tiled;
+        voff[i] = (tiled ? lr * 128 : lr * rowbytes) + col +
+                  (tiled ? static_cast<uint32_t>(gg >> 3) * kblock + static_cast<uint32_t>(gg & 7) * 1024
+                         : static_cast<uint32_t>(gg) * 8 * rowbytes);
+    }
+    const uint32_t kstep_bytes = key_tiled ? 8192u : 128u;
+    const uint32_t soff = static_cast<uint32_t>((lw % (TN >= 64 ? TN / 64 : 1)) * 64 + lane) * static_cast<uint32_t>(qscale_stride) * 4;
+    const int sstep = (qscale_stride == 1) ? 0 : 4;
+    const int halves = 2 * chunks, epi_at = halves > 2 ? 2 : 1;
+    unsigned id = blockIdx.x;       // the tile the next stage belongs to
+    int h = 0, ring = 0, tile = 0;  // its half-chunk there, its place in the ring (counted on), the tile's number here
+    bsi_rsrc rk, rq, rs, wrs, brs;
+    auto enter = [&] {
+        int bx, by;
+        if (grid.height != 0) {
+            i8_tile_of(grid, id, bx, by);
+        } else {
+            by = static_cast<int>(id / static_cast<unsigned>(grid.tiles_x));
+            bx = static_cast<int>(id) - by * grid.tiles_x;
+        }
+        const int64_t r0 = static_cast<int64_t>(bx) * TM, q0 = static_cast<int64_t>(by) * TN;
+        rk = key_tiled ? make_rsrc(K8 + static_cast<size_t>(r0 / 64) * kblock, static_cast<size_t>((R + 63) / 64 - r0 / 64) * kblock)
+                       : make_rsrc(K8 + static_cast<size_t>(r0) * rowbytes, static_cast<size_t>(R - r0) * rowbytes);
+        rq = make_rsrc(A8 + static_cast<size_t>(q0) * rowbytes, static_cast<size_t>(Q - q0) * rowbytes);
+        rs = make_rsrc(qscale + q0 * qscale_stride, static_cast<size_t>(Q - q0) * qscale_stride * 4);
+        wrs = make_rsrc(Bw + static_cast<size_t>(r0) * Sb, static_cast<size_t>(R - r0) * Sb * sizeof(float));
+        brs = make_rsrc(bias != nullptr ? bias + r0 : Bw, bias != nullptr ? static_cast<size_t>(R - r0) * sizeof(float) : 0);
+    };
+    enter();
+    auto issue = [&] {
+        if (h == halves) {
+            h = 0;
+            id += gridDim.x;
+            ++tile;
+            enter();
+        }
+        const uint32_t so_k = static_cast<uint32_t>(h) * kstep_bytes, so_q = static_cast<uint32_t>(h) * 128;
+#pragma unroll
+        for (int i = 0; i < NI; ++i) {
+            const int g = i < KG / L ? lw + L * i : KG + lw + L * (i - KG / L);
+            load16_to_lds(i < KG / L ? rk : rq, voff[i], i < KG / L ? so_k : so_q, lds + (ring & 3) * C::kStage + g * 1024);
+        }
+        if (h & 1)
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(
+                rs, BSI_LDS_PTR(lds + 4 * C::kStage + (((ring >> 1) & 3) * L + lw) * 256), 4, static_cast<int>(soff), (h >> 1) * sstep, 0, 0);
+        if (h == epi_at) {  // tiles of one chunk: the MFMA waves may still be reading the set of two tiles ago
+            unsigned char* const epi = lds + 4 * C::kStage + C::kScaleBytes + (tile & 3) * C::kEpilogueBytes;
+#pragma unroll
+            for (int k = 0; k < kEpi; ++k) {
+                const int j = (lw + L * k) % (2 * (TM / 64));
+                const bool is_bias = j >= TM / 64;
+                const int blk = is_bias ? j - TM / 64 : j;
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(is_bias ? brs : wrs, BSI_LDS_PTR(epi + (is_bias ? TM * 4 : 0) + blk * 256), 4,
+                                                         (blk * 64 + lane) * (is_bias ? 4 : Sb * 4), 0, 0, 0);
+            }
+        }
+        ++h;
+        ++ring;
+    };
+    const int mine = static_cast<int>((tiles - blockIdx.x + gridDim.x - 1) / gridDim.x), total = mine * halves;
+    issue();
+    issue();
+    if (total > 2) issue();
+    // The waits count the loads of the newer stages; the epilogue operands among them only make a wait stricter.
+    if (total > 2) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * NI + 1) : "memory");
+    else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    lds_barrier();
+    for (int g = 0; g < total; ++g) {
+        if (g + 3 < total) {
+            issue();
+            asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * NI + 1) : "memory");
+        } else if (g + 3 == total) {
+            asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NI + 1) : "memory");
+        } else {
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        }
+        lds_barrier();
+    }
+}
+
+template <int TM, int TN>
+__global__ __launch_bounds__((I8Cfg<TM, TN>::kBlock)) void dot_mfma_i8_tiles_kernel(
+    const int8_t* __restrict__ A8, const float* __restrict__ qscale, int qscale_stride, const int8_t* __restrict__ K8,
+    const float* __restrict__ Bw, int Sb, int chunks, int64_t R, int64_t Q, int down_shift, float scale_inv, int64_t R_total,
+    float* __restrict__ out, const float* __restrict__ bias, int key_tiled, const unsigned char* __restrict__ warm,
+    long long warm_lines, int out_stream, I8Grid grid, unsigned tiles, int out_dtype) {
+    using C = I8Cfg<TM, TN>;
+    constexpr int WM = C::kWM, WN = C::kWN, kMode = kI8Chain;
+    extern __shared__ __attribute__((aligned(16))) unsigned char lds[];  // I8TilesCfg::kLdsTiles
+    const int tid = threadIdx.x;
+    const int lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    if (wave >= C::kConsumers) {
+        const int lw = wave - C::kConsumers;
+        i8_tiles_loader_wave<C>(lds, lw, lane, A8, qscale, qscale_stride, K8, Bw, Sb, chunks, R, Q, bias, key_tiled, grid, tiles);
+        if (warm_lines > 0) i8_warm_lines<C::kLoaders>(lds + 4 * C::kStage, lw, lane, warm, warm_lines);
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // nothing may still be writing LDS when the workgroup ends
+        return;
+    }
+
+    // ---- MFMA waves (see dot_mfma_i8_kernel)
+    const int wr = wave & 1, wq = wave >> 1;
+    const int ln = lane & 15, lg = lane >> 4;
+    const int krow_off = (wr * (WM * 16) + ln) * 128;
+    const int qrow_off = C::kOperandK + (wq * (WN * 16) + ln) * 128;
+    int pcol[2];
+#pragma unroll
+    for (int kk = 0; kk < 2; ++kk) pcol[kk] = ((kk * 4 + lg) ^ (ln >> 1)) * 16;
+    float accf[WM][WN][4];
+    v4i acc0[WM][WN], acc1[WM][WN];
+#pragma unroll
+    for (int a = 0; a < WM; ++a)
+#pragma unroll
+        for (int b = 0; b < WN; ++b) {
+            acc0[a][b] = acc1[a][b] = (v4i){0, 0, 0, 0};
+#pragma unroll
+            for (int e = 0; e < 4; ++e) accf[a][b][e] = 0.0f;
+        }
+    const float down = __uint_as_float(static_cast<uint32_t>(127 - down_shift) << 23);
+    const int64_t int_off[WM][WN] = {};
+    const int int_rows[WM] = {};
+    float peak = 0.0f;
+    unsigned char* const scale_lds = lds + 4 * C::kStage;
+    const int qfirst = wq * (WN * 16);
+    const unsigned char* sread = scale_lds + (qfirst >> 6) * 256 + ((qfirst & 63) + ln) * 4;
+    float qsa[WN], qsb[WN];
+#pragma unroll
+    for (int b = 0; b < WN; ++b) qsa[b] = qsb[b] = 0.0f;
+    v4i ka[2][WM], qb[2][WN];
+    // the ring's two pairs of slots: the tile's even chunks sit in the pair at `even`, its odd ones in the other
+    int even = 0, odd = 2 * C::kStage, chunk0 = 0;
+#define BSI_TILES_CHUNK(here, next, acc, prev, qs)          \
+    BSI_I8_KSTEP_AT(0, here, acc, prev, qs);                \
+    lds_barrier();                                          \
+    BSI_I8_KSTEP_AT(1, (here) + C::kStage, acc, prev, qs);  \
+    BSI_I8_KSTEP_AT(2, (here) + C::kStage, acc, prev, qs);  \
+    lds_barrier();                                          \
+    BSI_I8_KSTEP_AT(3, next, acc, prev, qs);
+#define BSI_I8_KSTEP_AT(KS, at, acc, prev, qs)                                                                              \
+    i8_kstep<WM, WN, KS, kMode, false>(ka[(KS) & 1], qb[(KS) & 1], ka[((KS) + 1) & 1], qb[((KS) + 1) & 1],                  \
+                                       lds + (at) + krow_off + pcol[((KS) + 1) & 1],                                        \
+                                       lds + (at) + qrow_off + pcol[((KS) + 1) & 1], acc, prev, accf, qs, nullptr, int_off, \
+                                       int_rows, down_shift, chunks, peak);
+#define BSI_TILES_SCALES(dst, c)                                                               \
+    {                                                                                          \
+        _Pragma("unroll") for (int b = 0; b < WN; ++b) dst[b] =                                \
+            *reinterpret_cast<const float*>(sread + ((c) & 3) * (C::kLoaders * 256) + b * 64); \
+    }
+    lds_barrier();  // stage 0 is there
+#pragma unroll
+    for (int t = 0; t < WM; ++t) ka[0][t] = *reinterpret_cast<const v4i*>(lds + krow_off + t * 16 * 128 + pcol[0]);
+#pragma unroll
+    for (int t = 0; t < WN; ++t) qb[0][t] = *reinterpret_cast<const v4i*>(lds + qrow_off + t * 16 * 128 + pcol[0]);
+    __builtin_amdgcn_sched_barrier(0);
+    int tile = 0;
+#pragma nounroll
+    for (unsigned id = blockIdx.x; id < tiles; id += gridDim.x, ++tile) {
+        int c = 0;
+        for (; c + 1 < chunks; c += 2) {
+            BSI_TILES_CHUNK(even, odd, acc0, acc1, qsb);
+            BSI_TILES_SCALES(qsa, chunk0 + c);
+            BSI_TILES_CHUNK(odd, even, acc1, acc0, qsa);
+            BSI_TILES_SCALES(qsb, chunk0 + c + 1);
+        }
+        // the chain step of the last chunk; the last k-step has read the next tile's first operands
+        if (c < chunks) {
+            BSI_TILES_CHUNK(even, odd, acc0, acc1, qsb);
+            BSI_TILES_SCALES(qsa, chunk0 + c);
+            const int t = even;
+            even = odd;
+            odd = t;
+#pragma unroll
+            for (int a = 0; a < WM; ++a)
+#pragma unroll
+                for (int b = 0; b < WN; ++b)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) accf[a][b][e] = fmaf(static_cast<float>(acc0[a][b][e]), qsa[b], accf[a][b][e]);
+        } else {
+#pragma unroll
+            for (int a = 0; a < WM; ++a)
+#pragma unroll
+                for (int b = 0; b < WN; ++b)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) accf[a][b][e] = fmaf(static_cast<float>(acc1[a][b][e]), qsb[b], accf[a][b][e]);
+        }
+        chunk0 += chunks;
+        int bx, by;
+        if (grid.height != 0) {
+            i8_tile_of(grid, id, bx, by);
+        } else {
+            by = static_cast<int>(id / static_cast<unsigned>(grid.tiles_x));
+            bx = static_cast<int>(id) - by * grid.tiles_x;
+        }
+        // from values the compiler cannot see through, so that no address of the stores is held in registers over the chunk loop
+        int ln_late = ln, lg_late = lg;
+        asm volatile("" : "+v"(ln_late), "+v"(lg_late));
+        i8_store_tile<TM, WM, WN, true>(accf, lds + 4 * C::kStage + C::kScaleBytes + (tile & 3) * C::kEpilogueBytes, down, scale_inv,
+                                        bias != nullptr, out_dtype, out, R_total, static_cast<int64_t>(bx) * TM,
+                                        static_cast<int64_t>(by) * TN, wr, wq, R, Q, ln_late, lg_late, out_stream != 0);
+#pragma unroll
+        for (int b = 0; b < WN; ++b) qsb[b] = 0.0f;  // the first chunk's chain step adds nothing
+#pragma unroll
+        for (int a = 0; a < WM; ++a)
+#pragma unroll
+            for (int b = 0; b < WN; ++b)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) accf[a][b][e] = 0.0f;
+    }
+#undef BSI_TILES_CHUNK
+#undef BSI_I8_KSTEP_AT
+#undef BSI_TILES_SCALES
 }
 
 // ------------------------------------------------------------------ int8 image, one accumulator set per MFMA wave
@@ -1170,6 +1428,8 @@ static int stream_output() {
     return t_layer_output ? 0 : 1;
 }
 
+constexpr int kCus = 256;
+
 static I8Grid i8_grid(int64_t tiles_x, int64_t tiles_y, dim3* grid) {
     constexpr int64_t kBandTiles = 8;  // 4 and 16 take the same time within 2 %
     I8Grid g{static_cast<int>(tiles_x), static_cast<int>(tiles_y), 0, 0u, 0u, 0u};
@@ -1194,6 +1454,18 @@ static void launch_mfma_i8_tm(const int8_t* A8, const float* qscale, int stride,
     using C = I8Cfg<TM, TN>;
     dim3 grid;
     const I8Grid g = i8_grid((R + TM - 1) / TM, (Q + TN - 1) / TN, &grid);
+    const int64_t tiles = static_cast<int64_t>(g.tiles_x) * g.tiles_y;
+    // more than one round of the large tiles, which fill a CU's LDS
+    if constexpr (kMode == kI8Chain && TM == 128)
+        if (tiles > kCus && tiles * chunks < (int64_t{1} << 29)) {
+            static LdsOptIn once;
+            lds_opt_in(once, reinterpret_cast<const void*>(&dot_mfma_i8_tiles_kernel<TM, TN>), I8TilesCfg<TM, TN>::kLdsTiles);
+            launch((dot_mfma_i8_tiles_kernel<TM, TN>), dim3(kCus), dim3(C::kBlock), I8TilesCfg<TM, TN>::kLdsTiles, st, A8, qscale, stride,
+                   K8, Bw, Sb, chunks, R, Q, down_shift, scale_inv, R_total, out, bias, key_tiled,
+                   static_cast<const unsigned char*>(g_warm_ptr), static_cast<long long>(g_warm_bytes / 128), stream_output(), g,
+                   static_cast<unsigned>(tiles), t_out_dtype);
+            return;
+        }
     static LdsOptIn once0;
     lds_opt_in(once0, reinterpret_cast<const void*>(&dot_mfma_i8_kernel<TM, TN, kMode, false>), C::kLds);
     launch((dot_mfma_i8_kernel<TM, TN, kMode, false>), grid, dim3(C::kBlock), C::kLds, st, A8, qscale, stride, K8,
