@@ -73,6 +73,9 @@ PROTOTYPES = {
     "bsi_hip_linear_workspace_bytes": [_i64, _i64, _i],
     "bsi_hip_linear": [_vp, _i, _i64, _i64, _i, _i, _i, _vp, _sz, _vp, _i, _vp, _i, _i64, _f, _i64, _vp, _vp, _i, _vp,
                        _sz, _vp],
+    "bsi_hip_linear_coop_bytes": [],
+    "bsi_hip_linear_coop_serves": [_i64, _i64, _i64, _i, _i, _i, _i],
+    "bsi_hip_linear_coop_out": [_vp, _i, _i64, _i64, _i, _i, ctypes.c_uint64, _vp, _vp, _i, _vp, _i, _i64, _f, _i64, _vp, _vp, _i, _vp, _sz, _vp],
     "bsi_hip_linear_out": [_vp, _i, _i64, _i64, _i, _i, _i, _vp, _sz, _vp, _i, _vp, _i, _i64, _f, _i64, _vp, _vp, _i, _i, _vp,
                            _sz, _vp],
     "bsi_hip_dot_ewah_query": [_vp, _vp, _vp, _i, _i, _vp, _i, _vp, _vp, _i, _i64, _f, _vp, _vp, _vp],
@@ -110,6 +113,7 @@ _RESTYPES = {
     "bsi_hip_dot_split_scratch_bytes": _sz,
     "bsi_hip_dot_ewah_batch_workspace_bytes": _sz,
     "bsi_hip_linear_workspace_bytes": _sz,
+    "bsi_hip_linear_coop_bytes": _sz,
     "bsi_hip_dot_digits_workspace_bytes": _sz,
     "bsi_hip_int8_tiled_bytes": _sz,
     "bsi_hip_scalar_query_max_elems": _i64,

@@ -1,0 +1,199 @@
+// The query build of a small linear layer inside its dot's launch.
+//
+// A layer of a few rows is two launches, the query build and the dot, and the build is nothing but a launch: 2.2 us on the GPU
+// and 2.7 on the host for a fraction of a microsecond of work.  Building per workgroup repeats the work for every key tile;
+// building once for the device needs what one XCD wrote to become visible to the others.  So every XCD builds a copy of its
+// own: the workgroups on it take a share each, all of them read the copy through the L2 they share, and a share is announced
+// by a flag behind it.
+//
+// No workgroup depends on another one being resident.  A share's bytes do not depend on who builds it, so a workgroup that
+// has waited kCoopPatience for a share builds it itself.  Flags hold the launch's number, which no other launch has: nothing
+// is cleared between launches, and flags of earlier ones mean nothing.
+// Inside a launch the build is over 2.5 us after the first wave (16 rows of 4096: 1.5 until a wave has its chunk and has
+// quantised it, 0.3 to the flag, 0.5 to the last share): as long as the launch it replaces, but for the host.
+#pragma once
+#include "bsi_quant_device.h"
+
+namespace bsi {
+
+constexpr int kXcds = 8;
+constexpr int kCoopShares = 32;       // shares of a copy at most: one workgroup for each CU of an XCD
+constexpr int kCoopMaxItems = 1024;   // (row, chunk) items: 256 bytes of image and a scale each
+constexpr size_t kCoopFlagBytes = kXcds * kCoopShares * sizeof(unsigned long long);
+constexpr size_t kCoopCopyBytes = static_cast<size_t>(kCoopMaxItems) * (BSI_CHUNK_ELEMS + sizeof(float));
+constexpr size_t kCoopBytes = kCoopFlagBytes + kXcds * kCoopCopyBytes;
+constexpr int kCoopPatience = 2000;  // ticks of the 100 MHz clock: 20 us
+
+struct CoopBuild {
+    const void* x;
+    unsigned char* area;        // kCoopBytes: flags, then the copies (image, scales)
+    unsigned long long launch;  // this launch's number
+    long long d;
+    double dec_scale;
+    float scale;
+    int dtype, vec;             // BSI_DTYPE_*; rows can be loaded a quad at a time
+    int rows, chunks, slices;
+    int by_row;                 // one scale a row instead of one a chunk
+    int shares;                 // of a copy: chunk scales split the items, row scales the rows
+    int patience;               // ticks until a workgroup builds what it waits for
+};
+
+// Shares of a copy for a grid of `groups` workgroups, which go to the XCDs in turn.
+inline int coop_shares(unsigned groups, int pieces) {
+    int shares = static_cast<int>(groups / kXcds);
+    if (shares > kCoopShares) shares = kCoopShares;
+    if (shares > pieces) shares = pieces;
+    return shares < 1 ? 1 : shares;
+}
+
+// Row scales: the row's largest magnitude over the waves, then its quantised chunks.
+template <typename T, bool kVec>
+__device__ void coop_build_share(const CoopBuild& b, int share, int wave, int nwaves, int lane, uint32_t* __restrict__ image,
+                                 float* __restrict__ scales, unsigned* __restrict__ wave_max) {
+    const ChunkLane cl = chunk_lane(lane);
+    const QuantRange range = quant_range(b.slices);
+    const T* const x = static_cast<const T*>(b.x);
+    if (!b.by_row) {
+        const int items = b.rows * b.chunks;
+        const int first = items * share / b.shares, last = items * (share + 1) / b.shares;
+        auto load = [&](int item, float (&v)[4]) {
+            const int row = item / b.chunks;
+            load_chunk_quad<T, kVec>(x + row * b.d, b.d, item - row * b.chunks, cl, v);
+        };
+        auto emit = [&](int item, const float (&v)[4]) {
+            const unsigned mx = wave_max_u32(quad_max_bits(v));
+            int shift;
+            uint32_t bytes;
+            if (mx < kQuantWideBits) {
+                shift = quant_shift(mx, b.scale, b.slices);
+                bytes = quantise_quad<T>(v, b.scale, shift, range);
+            } else {
+                shift = compute_shift(wave_max_u64(quad_max_wide(v, b.dec_scale)), 0.0, 1, b.slices, 0.0f);
+                bytes = quantise_quad_wide(v, b.dec_scale, shift, b.slices);
+            }
+            image[item * 64 + lane] = chunk_image_dword(bytes, cl);
+            if (lane == 0) scales[item] = static_cast<float>(1ULL << shift);
+        };
+#pragma unroll 1
+        for (int item = first + wave; item < last; item += nwaves) {
+            float v[4];
+            load(item, v);
+            emit(item, v);
+        }
+        return;
+    }
+    const int first = b.rows * share / b.shares, last = b.rows * (share + 1) / b.shares;
+#pragma unroll 1
+    for (int row = first; row < last; ++row) {
+        const T* const xrow = x + row * b.d;
+        float held[4];
+        load_chunk_quad<T, kVec>(xrow, b.d, wave, cl, held);  // past the row: zeros
+        unsigned mx = quad_max_bits(held);
+        for (int c = wave + nwaves; c < b.chunks; c += nwaves) {
+            float v[4];
+            load_chunk_quad<T, kVec>(xrow, b.d, c, cl, v);
+            const unsigned m = quad_max_bits(v);
+            mx = m > mx ? m : mx;
+        }
+        mx = wave_max_u32(mx);
+        if (lane == 0) wave_max[wave] = mx;
+        lds_barrier();
+        for (int w = 0; w < nwaves; ++w) mx = wave_max[w] > mx ? wave_max[w] : mx;
+        lds_barrier();
+        const bool wide = mx >= kQuantWideBits;
+        int shift = quant_shift(mx, b.scale, b.slices);
+        if (wide) {  // rare: every wave looks at the whole row
+            unsigned long long m64 = 0ULL;
+            for (int c = 0; c < b.chunks; ++c) {
+                float v[4];
+                load_chunk_quad<T, kVec>(xrow, b.d, c, cl, v);
+                const unsigned long long m = quad_max_wide(v, b.dec_scale);
+                m64 = m > m64 ? m : m64;
+            }
+            shift = compute_shift(wave_max_u64(m64), 0.0, 1, b.slices, 0.0f);
+        }
+        if (wave == 0 && lane == 0) scales[row] = static_cast<float>(1ULL << shift);
+        for (int c = wave; c < b.chunks; c += nwaves) {
+            float v[4];
+            if (c == wave) {
+#pragma unroll
+                for (int k = 0; k < 4; ++k) v[k] = held[k];
+            } else {
+                load_chunk_quad<T, kVec>(xrow, b.d, c, cl, v);
+            }
+            const uint32_t bytes = wide ? quantise_quad_wide(v, b.dec_scale, shift, b.slices) : quantise_quad<T>(v, b.scale, shift, range);
+            image[(row * b.chunks + c) * 64 + lane] = chunk_image_dword(bytes, cl);
+        }
+    }
+}
+
+// Called by all waves of the workgroup (number `id` of the grid); 32 words of LDS at `shared`.  On return A8 and qscale point
+// to the whole build, in the copy of the XCD the workgroup runs on.  ahead(): loads for after the build.  Every wave but wave 0
+// issues them when the workgroup's share is built (a CU's loads return in order: not before), wave 0, which asks for the
+// flags, when all shares are.
+template <typename F>
+__device__ __forceinline__ void coop_build(const CoopBuild& b, unsigned id, unsigned* __restrict__ shared, const int8_t*& A8,
+                                           const float*& qscale, F&& ahead) {
+    const int lane = threadIdx.x & (BSI_WAVE - 1);
+    const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
+    const int nwaves = static_cast<int>(blockDim.x >> 6);
+    const unsigned xcd = __builtin_amdgcn_s_getreg((3 << 11) | 20) & (kXcds - 1);  // XCC_ID, bits 0 .. 3
+    unsigned long long* const flags = reinterpret_cast<unsigned long long*>(b.area) + xcd * kCoopShares;
+    unsigned char* const copy = b.area + kCoopFlagBytes + xcd * kCoopCopyBytes;
+    uint32_t* const image = reinterpret_cast<uint32_t*>(copy);
+    float* const scales = reinterpret_cast<float*>(copy + static_cast<size_t>(kCoopMaxItems) * BSI_CHUNK_ELEMS);
+    bool issued = false;
+    auto build = [&](int share) {
+        if (b.dtype == BSI_DTYPE_F32) {
+            if (b.vec) coop_build_share<float, true>(b, share, wave, nwaves, lane, image, scales, shared);
+            else coop_build_share<float, false>(b, share, wave, nwaves, lane, image, scales, shared);
+        } else if (b.dtype == BSI_DTYPE_F16) {
+            if (b.vec) coop_build_share<__half, true>(b, share, wave, nwaves, lane, image, scales, shared);
+            else coop_build_share<__half, false>(b, share, wave, nwaves, lane, image, scales, shared);
+        } else {
+            if (b.vec) coop_build_share<__hip_bfloat16, true>(b, share, wave, nwaves, lane, image, scales, shared);
+            else coop_build_share<__hip_bfloat16, false>(b, share, wave, nwaves, lane, image, scales, shared);
+        }
+        const int items = b.rows * b.chunks, had = items * (share + 1) / b.shares - items * share / b.shares;
+        if (b.by_row || wave < had) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the wave's stores have reached the L2
+        lds_barrier();
+        if (wave != 0 && !issued) {
+            ahead();
+            issued = true;
+        }
+        // A plain store, as the share's are: it stops in the L2 that the workgroups of this XCD share, where their agent-scope
+        // loads find it.  (An agent-scope store goes on to memory: the flags then come 1 to 2 us later.)
+        if (threadIdx.x == 0) __hip_atomic_store(flags + share, b.launch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    };
+    int share = id / kXcds < static_cast<unsigned>(b.shares) ? static_cast<int>(id / kXcds) : -1;
+    if (share < 0 && wave != 0) {
+        ahead();
+        issued = true;
+    }
+#pragma unroll 1
+    for (;;) {
+        if (share >= 0) build(share);
+        if (wave == 0) {
+            const unsigned long long since = wall_clock64();
+            unsigned long long missing;
+            for (;;) {
+                const bool here = lane >= b.shares ||
+                                  __hip_atomic_load(flags + (lane < kCoopShares ? lane : 0), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == b.launch;
+                missing = __ballot(!here);
+                if (missing == 0ULL || wall_clock64() - since > static_cast<unsigned>(b.patience)) break;
+            }
+            if (lane == 0) shared[0] = static_cast<unsigned>(missing);
+        }
+        lds_barrier();
+        const unsigned missing = static_cast<unsigned>(__builtin_amdgcn_readfirstlane(static_cast<int>(shared[0])));
+        lds_barrier();
+        if (missing == 0u) break;
+        share = __builtin_ctz(missing);
+    }
+    if (!issued) ahead();
+    asm volatile("" ::: "memory");
+    A8 = reinterpret_cast<const int8_t*>(copy);
+    qscale = scales;
+}
+
+}  // namespace bsi

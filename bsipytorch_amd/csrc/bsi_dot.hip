@@ -31,7 +31,12 @@
 // bsi_dot_i8.hip (int8 image of the keys), bsi_dot_few_rows.hip (a few query rows, planes streamed once),
 // bsi_dot_planes.hip (many rows on planes), bsi_dot_valu.hip (popcount cores, weighted slices, bias) and
 // bsi_dot_layouts.hip (operand layouts); bsi_dot_device.h holds the device helpers they share.
+#include "bsi_coop_build.h"
 #include "bsi_dot_internal.h"
+
+namespace bsi {
+static std::atomic<int> g_coop_patience{kCoopPatience};
+}  // namespace bsi
 
 using namespace bsi;
 
@@ -53,6 +58,10 @@ extern "C" int bsi_hip_set_option(int option, int value) {
         case BSI_OPT_I8_SPLIT:
             BSI_REQUIRE(value >= 0 && value <= 64, "split must be 0 (by cost), 1 (never) or a number of segments up to 64");
             g_i8_split = value;
+            return BSI_OK;
+        case BSI_OPT_COOP_PATIENCE:
+            BSI_REQUIRE(value >= 0, "patience must not be negative");
+            g_coop_patience = value;
             return BSI_OK;
         case BSI_OPT_BUILD_ITEMS:
             BSI_REQUIRE(value == 0 || value == 1 || value == 2 || value == 4 || value == 8, "items must be 0, 1, 2, 4 or 8");
@@ -348,6 +357,69 @@ extern "C" int bsi_hip_linear_out(const void* x, int dtype, int64_t Q, int64_t d
                                          Bw, Sb, R, Q, scale_inv, R_total, bias, static_cast<float*>(out), core, nullptr, 0, warm,
                                          warm_bytes, stream);
     t_out_dtype = BSI_DTYPE_F32;
+    return rc;
+}
+
+extern "C" size_t bsi_hip_linear_coop_bytes(void) { return kCoopBytes; }
+
+extern "C" int bsi_hip_linear_coop_serves(int64_t Q, int64_t d, int64_t R, int decimal_places, int fixed_bits, int b_layout, int Sb) {
+    const int64_t chunks = (d + 255) / 256;
+    if (Q < 1 || d < 1 || R < 1 || Q * chunks > kCoopMaxItems || decimal_places < 0 || decimal_places > 2 || fixed_bits < 2 || fixed_bits > 8)
+        return 0;
+    unsigned groups = 0;
+    int waves = 0;
+    if (b_layout == BSI_LAYOUT_TILED16) {
+        if (Q > kStreamMaxQ || Sb != 6) return 0;
+        stream_launch_shape(Q, R, static_cast<int>(chunks), &groups, &waves);
+    } else {
+        if ((b_layout != BSI_LAYOUT_INT8 && b_layout != BSI_LAYOUT_INT8_TILED) || Sb < 2 || Sb > 8) return 0;
+        i8_launch_shape(Q, R, &groups, &waves);
+    }
+    // Chunks that a wave of the build takes one after the other, each a load's latency: up to two chunk-scaled ones or one
+    // of a row (which has barriers besides) cost less than a launch.  us a pass, two launches and one: 16 x 512 x 1280 6.6, 4.8;
+    // 15 x 2560 x 5888 8.4, 7.3; 28 x 3072 x 4864 11.5, 10.6; 49 x 512 x 3328 6.9, 5.7; 121 x 512 x 14848 8.8, 8.1 -- beyond:
+    // 80 x 2304 x 4352 (4 rounds) 8.5, 8.9; 37 x 704 x 9728 (2 rows) 6.8, 7.6; 24 x 2304 x 256 7.4, 13.9.
+    const bool by_row = ((d + 63) / 64) % 4 != 0;
+    const int shares = coop_shares(groups, static_cast<int>(by_row ? Q : Q * chunks));
+    if (by_row) return Q <= shares && chunks <= waves ? 1 : 0;
+    return Q * chunks <= 2 * static_cast<int64_t>(shares) * waves ? 1 : 0;
+}
+
+extern "C" int bsi_hip_linear_coop_out(const void* x, int dtype, int64_t Q, int64_t d, int decimal_places, int fixed_bits, uint64_t launch_number,
+                                       void* area, const uint64_t* B, int b_layout, const float* Bw, int Sb, int64_t R, float scale_inv,
+                                       int64_t R_total, const float* bias, void* out, int out_dtype, const void* warm, size_t warm_bytes,
+                                       void* stream) {
+    BSI_REQUIRE(out_dtype == BSI_DTYPE_F32 || out_dtype == BSI_DTYPE_F16 || out_dtype == BSI_DTYPE_BF16, "unknown dtype code %d", out_dtype);
+    BSI_REQUIRE(dtype == BSI_DTYPE_F32 || dtype == BSI_DTYPE_F16 || dtype == BSI_DTYPE_BF16, "unknown dtype code %d", dtype);
+    if (!bsi_hip_linear_coop_serves(Q, d, R, decimal_places, fixed_bits, b_layout, Sb))
+        return fail(BSI_ERR_UNSUPPORTED, "no launch with the query build inside for this layer");
+    BSI_REQUIRE(x != nullptr && area != nullptr && launch_number != 0, "null pointer or launch number");
+    BSI_REQUIRE((reinterpret_cast<uintptr_t>(area) & 255) == 0, "the area must be 256-byte aligned");
+    const int W64 = static_cast<int>((d + 63) / 64), chunks = (W64 + 3) / 4;
+    const double dec_scale = pow(10.0, static_cast<double>(decimal_places));
+    const size_t esize = dtype == BSI_DTYPE_F32 ? 4 : 2;
+    CoopBuild c{};
+    c.x = x;
+    c.area = static_cast<unsigned char*>(area);
+    c.launch = launch_number;
+    c.d = d;
+    c.dec_scale = dec_scale;
+    c.scale = static_cast<float>(dec_scale);
+    c.dtype = dtype;
+    c.vec = d % 4 == 0 && reinterpret_cast<uintptr_t>(x) % (4 * esize) == 0 ? 1 : 0;
+    c.rows = static_cast<int>(Q);
+    c.chunks = chunks;
+    c.slices = fixed_bits;
+    c.patience = g_coop_patience.load(std::memory_order_relaxed);
+    c.by_row = W64 % 4 == 0 ? 0 : 1;  // the builder's rule
+    t_coop = &c;
+    t_out_dtype = out_dtype;
+    // the operands stand for the launch's own copies
+    const int rc = bsi_hip_dot_bias_warm(nullptr, static_cast<const int8_t*>(area), static_cast<const float*>(area), c.by_row ? 1 : chunks,
+                                         fixed_bits, W64, B, b_layout, Bw, Sb, R, Q, scale_inv, R_total, bias, static_cast<float*>(out),
+                                         BSI_CORE_MFMA, nullptr, 0, warm, warm_bytes, stream);
+    t_out_dtype = BSI_DTYPE_F32;
+    t_coop = nullptr;
     return rc;
 }
 

@@ -2,7 +2,7 @@
 // query image, with the query build inside, or with queries handed over as EWAH streams -- and the stream -> int8
 // image pass for larger batches of EWAH queries.
 #include "bsi_dot_internal.h"
-#include "bsi_quant_device.h"
+#include "bsi_coop_build.h"
 
 namespace bsi {
 
@@ -21,12 +21,14 @@ namespace bsi {
 
 constexpr int kStreamLdsInts = 16384;  // at most 64 KiB of chunk accumulators per pass
 
-template <int NT, int KT, bool kInts>
+// kBuild: the queries are quantised by this launch (bsi_coop_build.h); A8 and qscale are not looked at.
+template <int NT, int KT, bool kInts, bool kBuild>
 __global__ __launch_bounds__(1024) void dot_mfma_stream_kernel(
-    const int8_t* __restrict__ A8, const float* __restrict__ qscale, int qscale_stride,
+    const int8_t* A8, const float* qscale, int qscale_stride,
     const unsigned long long* __restrict__ B64,  // tiled key planes, Sb = 6
     const float* __restrict__ Bw, int chunks, int pass_chunks, int64_t R, int64_t Q, int down_shift, float scale_inv,
-    int64_t R_total, float* __restrict__ out, int* __restrict__ chunk_ints, const float* __restrict__ bias, int out_dtype) {
+    int64_t R_total, float* __restrict__ out, int* __restrict__ chunk_ints, const float* __restrict__ bias, int out_dtype,
+    CoopBuild coop) {
     extern __shared__ __attribute__((aligned(16))) int ints[];  // [pass_chunks][KT][NT][16 queries][16 keys]
     constexpr int kSlot = KT * NT * 256;
 
@@ -46,6 +48,18 @@ __global__ __launch_bounds__(1024) void dot_mfma_stream_kernel(
         ksrc[k] = B64 + static_cast<size_t>(t) * ktile + lane;
     }
     const size_t arow = static_cast<size_t>(chunks) * 256;
+    uint2 kc[KT][6];
+    auto load_keys = [&](int c) {
+#pragma unroll
+        for (int k = 0; k < KT; ++k)
+#pragma unroll
+            for (int j = 0; j < 6; ++j) {
+                const unsigned long long w = ksrc[k][(static_cast<size_t>(c) * 6 + j) * 64];
+                kc[k][j] = make_uint2(static_cast<uint32_t>(w), static_cast<uint32_t>(w >> 32));
+            }
+    };
+    if (kBuild)
+        coop_build(coop, blockIdx.x, reinterpret_cast<unsigned*>(ints), A8, qscale, [&] { load_keys(wave < pass_chunks ? wave : pass_chunks - 1); });
 
     // the chain lanes: tid <-> (key tile, query tile, query, key), keys fastest so output stores are contiguous
     float accf = 0.0f;
@@ -61,16 +75,7 @@ __global__ __launch_bounds__(1024) void dot_mfma_stream_kernel(
     for (int p0 = 0; p0 < chunks; p0 += pass_chunks) {
         const int pend = (p0 + pass_chunks < chunks) ? p0 + pass_chunks : chunks;
         int c = p0 + wave;
-        uint2 kc[KT][6];
-        if (c < pend) {
-#pragma unroll
-            for (int k = 0; k < KT; ++k)
-#pragma unroll
-                for (int j = 0; j < 6; ++j) {
-                    const unsigned long long w = ksrc[k][(static_cast<size_t>(c) * 6 + j) * 64];
-                    kc[k][j] = make_uint2(static_cast<uint32_t>(w), static_cast<uint32_t>(w >> 32));
-                }
-        }
+        if (c < pend && !(kBuild && p0 == 0)) load_keys(c);
         for (; c < pend; c += nwaves) {
             // query operands of this chunk (L2 resident), then the key planes of the wave's next chunk
             v4i qb[NT][4];
@@ -503,36 +508,50 @@ __global__ __launch_bounds__(kEwahToInt8Block) void ewah_streams_to_int8_kernel(
     }
 }
 
+static unsigned stream_groups(int64_t R, int key_tiles) { return static_cast<unsigned>(((R + 15) / 16 + key_tiles - 1) / key_tiles); }
+// one workgroup per CU at most: more waves each streaming their own chunks; else 8 and several workgroups
+static int stream_waves(unsigned groups, int chunks, int slot) {
+    int waves = groups <= 256 ? 16 : 8;
+    if (waves > chunks) waves = chunks;          // one chunk per wave and pass at least
+    if (waves < slot / 64) waves = slot / 64;    // the chain needs one lane per output
+    return waves > 16 ? 16 : waves;
+}
+// two key tiles per workgroup halve the query re-reads once there are enough tiles to fill the GPU
+static int stream_key_tiles(int64_t R) { return (R + 15) / 16 >= 1024 ? 2 : 1; }
+void stream_launch_shape(int64_t Q, int64_t R, int chunks, unsigned* groups, int* waves) {
+    const int kt = stream_key_tiles(R);
+    *groups = stream_groups(R, kt);
+    *waves = stream_waves(*groups, chunks, kt * (Q <= 16 ? 1 : 2) * 256);
+}
+
 template <int NT, int KT>
 static void launch_mfma_stream(const int8_t* A8, const float* qscale, int stride, const uint64_t* B, const float* Bw,
                                int chunks, int64_t R, int64_t Q, int down_shift, float scale_inv, int64_t R_total,
                                float* out, int32_t* chunk_ints, const float* bias, hipStream_t st) {
     constexpr int kSlot = KT * NT * 256;
-    const int64_t ntiles = (R + 15) / 16;
-    const dim3 grid(static_cast<unsigned>((ntiles + KT - 1) / KT), static_cast<unsigned>((Q + 16 * NT - 1) / (16 * NT)));
-    // one workgroup per CU at most: more waves each streaming their own chunks; else 8 and several workgroups
-    int waves = (grid.x * grid.y <= 256) ? 16 : 8;
-    if (waves > chunks) waves = chunks;             // one chunk per wave and pass at least
-    if (waves < kSlot / 64) waves = kSlot / 64;     // the chain needs one lane per output
-    if (waves > 16) waves = 16;
+    const dim3 grid(stream_groups(R, KT), static_cast<unsigned>((Q + 16 * NT - 1) / (16 * NT)));
+    const int waves = stream_waves(grid.x * grid.y, chunks, kSlot);
     int pass_chunks = kStreamLdsInts / kSlot;
     if (pass_chunks > chunks) pass_chunks = chunks;
     const size_t lds = static_cast<size_t>(pass_chunks) * kSlot * sizeof(int);
-    if (chunk_ints)
-        launch((dot_mfma_stream_kernel<NT, KT, true>), grid, dim3(waves * 64), lds, st, A8, qscale, stride,
-                           reinterpret_cast<const unsigned long long*>(B), Bw, chunks, pass_chunks, R, Q, down_shift,
-                           scale_inv, R_total, out, chunk_ints, bias, t_out_dtype);
-    else
-        launch((dot_mfma_stream_kernel<NT, KT, false>), grid, dim3(waves * 64), lds, st, A8, qscale, stride,
-                           reinterpret_cast<const unsigned long long*>(B), Bw, chunks, pass_chunks, R, Q, down_shift,
-                           scale_inv, R_total, out, chunk_ints, bias, t_out_dtype);
+#define BSI_STREAM_GO(INTS, BUILD, COOP)                                                                                      \
+    launch((dot_mfma_stream_kernel<NT, KT, INTS, BUILD>), grid, dim3(waves * 64), lds, st, A8, qscale, stride,                \
+           reinterpret_cast<const unsigned long long*>(B), Bw, chunks, pass_chunks, R, Q, down_shift, scale_inv, R_total, out, \
+           chunk_ints, bias, t_out_dtype, COOP)
+    if (chunk_ints) BSI_STREAM_GO(true, false, CoopBuild{});
+    else if (t_coop == nullptr) BSI_STREAM_GO(false, false, CoopBuild{});
+    else {
+        CoopBuild coop = *t_coop;
+        coop.shares = coop_shares(grid.x, coop.by_row ? coop.rows : coop.rows * coop.chunks);
+        BSI_STREAM_GO(false, true, coop);
+    }
+#undef BSI_STREAM_GO
 }
 
 void launch_mfma_stream_by_shape(const int8_t* A8, const float* qscale, int stride, const uint64_t* B, const float* Bw,
                                  int chunks, int64_t R, int64_t Q, int down_shift, float scale_inv, int64_t R_total,
                                  float* out, int32_t* chunk_ints, const float* bias, hipStream_t st) {
-    // two key tiles per workgroup halve the query re-reads once there are enough tiles to fill the GPU
-    const bool two = (R + 15) / 16 >= 1024;
+    const bool two = stream_key_tiles(R) == 2;
 #define BSI_STREAM_ARGS A8, qscale, stride, B, Bw, chunks, R, Q, down_shift, scale_inv, R_total, out, chunk_ints, bias, st
     if (Q <= 16) { if (two) launch_mfma_stream<1, 2>(BSI_STREAM_ARGS); else launch_mfma_stream<1, 1>(BSI_STREAM_ARGS); }
     else { if (two) launch_mfma_stream<2, 2>(BSI_STREAM_ARGS); else launch_mfma_stream<2, 1>(BSI_STREAM_ARGS); }

@@ -1,6 +1,6 @@
 // The matrix-core dot on the cached int8 image of the keys (the compute-bound calls), its probe of the L2 -> LDS
 // path, the timeline stamps, and the decimal-mode dot on int8 digit images that runs on the same kernel.
-#include "bsi_dot_device.h"
+#include "bsi_coop_build.h"
 #include "bsi_dot_internal.h"
 
 namespace bsi {
@@ -491,15 +491,16 @@ __device__ __forceinline__ void i8_tile_of(const I8Grid& g, unsigned id, int& bx
     by = static_cast<int>(first + in - x * (last ? left : static_cast<unsigned>(g.height)));
 }
 
-template <int TM, int TN, int kMode, bool kSplit>
+template <int TM, int TN, int kMode, bool kSplit, bool kBuild>
 __global__ __launch_bounds__((I8Cfg<TM, TN>::kBlock)) void dot_mfma_i8_kernel(
-    const int8_t* __restrict__ A8, const float* __restrict__ qscale, int qscale_stride,
+    const int8_t* A8, const float* qscale, int qscale_stride,
     const int8_t* __restrict__ K8,  // int8 key image [R, chunks * 256]
     const float* __restrict__ Bw, int Sb, int chunks, int64_t R, int64_t Q, int down_shift, float scale_inv,
     int64_t R_total, float* __restrict__ out, int* __restrict__ chunk_ints, const float* __restrict__ bias,
     int ndig, long long dig_stride, const long long* __restrict__ key_indices, int key_tiled,
     const unsigned char* __restrict__ warm, long long warm_lines, int out_stream, float* __restrict__ split_partials,
-    unsigned* __restrict__ split_counters, float split_limit, int split_shape, I8Grid plain_grid, int out_dtype) {
+    unsigned* __restrict__ split_counters, float split_limit, int split_shape, I8Grid plain_grid, int out_dtype, CoopBuild coop) {
+    // kBuild: the queries are quantised by this launch (bsi_coop_build.h); A8 and qscale are not looked at.
     // kSplit (chain mode only): a D-split launch.  gridDim.z workgroups share an output tile, each running the chain
     // over its own run of chunks from zero.  All operands of the chain are integers (times one power of two), so
     // as long as no value the chain takes exceeds 2^24 of its unit nothing is ever rounded, the value after every
@@ -527,6 +528,7 @@ __global__ __launch_bounds__((I8Cfg<TM, TN>::kBlock)) void dot_mfma_i8_kernel(
     constexpr int WM = C::kWM, WN = C::kWN;
     constexpr bool kInts = (kMode == kI8Ints), kSum = (kMode == kI8Sum);
     extern __shared__ __attribute__((aligned(16))) unsigned char lds[];  // C::kLds
+    if (kBuild) coop_build(coop, blockIdx.y * gridDim.x + blockIdx.x, reinterpret_cast<unsigned*>(lds), A8, qscale, [] {});
 
     const int tid = threadIdx.x;
     const int lane = tid & 63;
@@ -1420,6 +1422,7 @@ thread_local size_t g_warm_bytes = 0;
 // for the 16 MiB of Q512 R8192).  Measured both ways: streamed layer outputs cost an OPT-1.3B-shaped prefill 2 %
 // (4.89 -> 5.00 ms replayed), plain dot outputs cost the standalone dot 8 %.  BSI_OPT_OUTPUT_STORES overrides.
 thread_local int t_layer_output = 0;
+thread_local const CoopBuild* t_coop = nullptr;
 thread_local int t_out_dtype = BSI_DTYPE_F32;
 std::atomic<int> g_output_stores{0};  // 0 = by entry point, 1 = always plain, 2 = always nontemporal
 static int stream_output() {
@@ -1457,7 +1460,7 @@ static void launch_mfma_i8_tm(const int8_t* A8, const float* qscale, int stride,
     const int64_t tiles = static_cast<int64_t>(g.tiles_x) * g.tiles_y;
     // more than one round of the large tiles, which fill a CU's LDS
     if constexpr (kMode == kI8Chain && TM == 128)
-        if (tiles > kCus && tiles * chunks < (int64_t{1} << 29)) {
+        if (t_coop == nullptr && tiles > kCus && tiles * chunks < (int64_t{1} << 29)) {
             static LdsOptIn once;
             lds_opt_in(once, reinterpret_cast<const void*>(&dot_mfma_i8_tiles_kernel<TM, TN>), I8TilesCfg<TM, TN>::kLdsTiles);
             launch((dot_mfma_i8_tiles_kernel<TM, TN>), dim3(kCus), dim3(C::kBlock), I8TilesCfg<TM, TN>::kLdsTiles, st, A8, qscale, stride,
@@ -1466,13 +1469,25 @@ static void launch_mfma_i8_tm(const int8_t* A8, const float* qscale, int stride,
                    static_cast<unsigned>(tiles), t_out_dtype);
             return;
         }
+    if constexpr (kMode == kI8Chain)
+        if (t_coop != nullptr) {
+            CoopBuild coop = *t_coop;
+            coop.shares = coop_shares(grid.x * grid.y, coop.by_row ? coop.rows : coop.rows * coop.chunks);
+            static LdsOptIn once;
+            lds_opt_in(once, reinterpret_cast<const void*>(&dot_mfma_i8_kernel<TM, TN, kI8Chain, false, true>), C::kLds);
+            launch((dot_mfma_i8_kernel<TM, TN, kI8Chain, false, true>), grid, dim3(C::kBlock), C::kLds, st, A8, qscale, stride, K8, Bw, Sb,
+                   chunks, R, Q, down_shift, scale_inv, R_total, out, chunk_ints, bias, ndig, dig_stride, key_indices, key_tiled,
+                   static_cast<const unsigned char*>(g_warm_ptr), static_cast<long long>(g_warm_bytes / 128), stream_output(),
+                   static_cast<float*>(nullptr), static_cast<unsigned*>(nullptr), 0.0f, 0, g, t_out_dtype, coop);
+            return;
+        }
     static LdsOptIn once0;
-    lds_opt_in(once0, reinterpret_cast<const void*>(&dot_mfma_i8_kernel<TM, TN, kMode, false>), C::kLds);
-    launch((dot_mfma_i8_kernel<TM, TN, kMode, false>), grid, dim3(C::kBlock), C::kLds, st, A8, qscale, stride, K8,
+    lds_opt_in(once0, reinterpret_cast<const void*>(&dot_mfma_i8_kernel<TM, TN, kMode, false, false>), C::kLds);
+    launch((dot_mfma_i8_kernel<TM, TN, kMode, false, false>), grid, dim3(C::kBlock), C::kLds, st, A8, qscale, stride, K8,
                        Bw, Sb, chunks, R, Q, down_shift, scale_inv, R_total, out, chunk_ints, bias, ndig, dig_stride,
                        key_indices, key_tiled, static_cast<const unsigned char*>(g_warm_ptr),
                        static_cast<long long>(g_warm_bytes / 128), stream_output(), static_cast<float*>(nullptr),
-                       static_cast<unsigned*>(nullptr), 0.0f, 0, g, t_out_dtype);
+                       static_cast<unsigned*>(nullptr), 0.0f, 0, g, t_out_dtype, CoopBuild{});
 }
 
 // The D-split launch of the chain mode: `segments` workgroups per output tile, each over its own run of chunks (see
@@ -1491,13 +1506,13 @@ static void launch_mfma_i8_split(int segments, unsigned char* scratch, const int
     while ((1 << log2_segments) < segments) ++log2_segments;
     const float limit = __builtin_ldexpf(1.0f, 24 + down_shift - log2_segments);
     static LdsOptIn once0;
-    lds_opt_in(once0, reinterpret_cast<const void*>(&dot_mfma_i8_kernel<TM, TN, kI8Chain, true>), C::kLdsSplit);
-    launch((dot_mfma_i8_kernel<TM, TN, kI8Chain, true>), grid, dim3(C::kBlock), C::kLdsSplit, st, A8, qscale,
+    lds_opt_in(once0, reinterpret_cast<const void*>(&dot_mfma_i8_kernel<TM, TN, kI8Chain, true, false>), C::kLdsSplit);
+    launch((dot_mfma_i8_kernel<TM, TN, kI8Chain, true, false>), grid, dim3(C::kBlock), C::kLdsSplit, st, A8, qscale,
                        stride, K8, Bw, Sb, chunks, R, Q, down_shift, scale_inv, R_total, out, static_cast<int*>(nullptr), bias,
                        1, 0LL, static_cast<const long long*>(nullptr), key_tiled,
                        static_cast<const unsigned char*>(g_warm_ptr), static_cast<long long>(g_warm_bytes / 128),
                        stream_output(), reinterpret_cast<float*>(scratch + kSplitCounterBytes),
-                       reinterpret_cast<unsigned*>(scratch), limit, split_shape, I8Grid{}, t_out_dtype);
+                       reinterpret_cast<unsigned*>(scratch), limit, split_shape, I8Grid{}, t_out_dtype, CoopBuild{});
 }
 
 // Sum mode (ndig >= 1 digit images of the queries; int32 sums into chunk_ints when given, else the float epilogue)
@@ -1561,6 +1576,14 @@ int choose_i8_tile(int64_t R, int64_t Q, int64_t* cost_out) {
         if (cost[i] < cost[best]) best = i;
     if (cost_out) *cost_out = cost[best];
     return tiles[best];
+}
+
+void i8_launch_shape(int64_t Q, int64_t R, unsigned* groups, int* waves) {
+    const int tile = choose_i8_tile(R, Q);
+    const int64_t tm = tile == 64 || tile == 6432 ? 64 : 128, tn = tile == 6432 ? 32 : (tile == 64 || tile == 12864 ? 64 : 128);
+    *groups = static_cast<unsigned>(((R + tm - 1) / tm) * ((Q + tn - 1) / tn));
+    *waves = (tile == 64 ? I8Cfg<64, 64>::kBlock : tile == 6432 ? I8Cfg<64, 32>::kBlock : tile == 12864 ? I8Cfg<128, 64>::kBlock
+                                                                                     : I8Cfg<128, 128>::kBlock) / 64;
 }
 
 // D-split choice for a chain-mode call whose grid leaves most CUs idle: the 128 x 128 or 128 x 64 tile with `segments`
@@ -1633,7 +1656,7 @@ void launch_mfma_i8(const int8_t* A8, const float* qscale, int stride, const int
                            int chunks, int64_t R, int64_t Q, int down_shift, float scale_inv, int64_t R_total,
                            float* out, int32_t* chunk_ints, const float* bias, hipStream_t st, int key_tiled,
                            int ndig, long long dig_stride, const long long* key_indices) {
-    if (ndig == 0 && chunk_ints == nullptr) {
+    if (ndig == 0 && chunk_ints == nullptr && t_coop == nullptr) {
         int segments = 1;
         const int split_tile = choose_i8_split(R, Q, chunks, &segments);
         if (split_tile == 128) {
@@ -1648,7 +1671,7 @@ void launch_mfma_i8(const int8_t* A8, const float* qscale, int stride, const int
         }
     }
     const int tile = choose_i8_tile(R, Q);
-    if (tile == 1284 && ndig == 0) {
+    if (tile == 1284 && ndig == 0 && t_coop == nullptr) {
         launch_mfma_i8w<4>(A8, qscale, stride, K8, Bw, Sb, chunks, R, Q, down_shift, scale_inv, R_total, out, chunk_ints, bias,
                            st, key_tiled);
         return;

@@ -30,6 +30,9 @@ extern thread_local int t_layer_output;
 // Set by the entry points that write a half-precision layer output around their launch (BSI_DTYPE_*; F32 otherwise).  `out`
 // is then an array of that type; kernels that write float32 only are refused by dot_launch.
 extern thread_local int t_out_dtype;
+// Set by bsi_hip_linear_coop_out around its launch: the query build the kernel does itself (bsi_coop_build.h).
+struct CoopBuild;
+extern thread_local const CoopBuild* t_coop;
 int choose_i8_tile(int64_t R, int64_t Q, int64_t* cost_out = nullptr);
 // D-split of the chain-mode int8-image dot (bsi_hip_dot_attach_split_scratch): the calling thread's scratch region
 // (counters of kSplitCounterBytes, then the segments' partial sums) and the device it lies on; the option
@@ -41,6 +44,7 @@ extern thread_local unsigned char* t_split_scratch;
 extern thread_local size_t t_split_bytes;
 extern thread_local int t_split_device;
 extern std::atomic<int> g_i8_split;
+void i8_launch_shape(int64_t Q, int64_t R, unsigned* groups, int* waves);  // workgroups and their waves on the chosen tile
 int choose_i8_split(int64_t R, int64_t Q, int chunks, int* segments);
 void launch_mfma_i8(const int8_t* A8, const float* qscale, int stride, const int8_t* K8, const float* Bw, int Sb,
                     int chunks, int64_t R, int64_t Q, int down_shift, float scale_inv, int64_t R_total, float* out,
@@ -52,6 +56,8 @@ void launch_mfma_i8(const int8_t* A8, const float* qscale, int stride, const int
 void launch_mfma_stream_by_shape(const int8_t* A8, const float* qscale, int stride, const uint64_t* B, const float* Bw,
                                  int chunks, int64_t R, int64_t Q, int down_shift, float scale_inv, int64_t R_total,
                                  float* out, int32_t* chunk_ints, const float* bias, hipStream_t st);
+
+void stream_launch_shape(int64_t Q, int64_t R, int chunks, unsigned* groups, int* waves);  // its workgroups, their waves
 
 // ---- bsi_dot_valu.hip: the popcount kernels
 void launch_valu76(bool tiled, const uint64_t* A, const float* qscale, int stride, const uint64_t* B, const float* Bw,

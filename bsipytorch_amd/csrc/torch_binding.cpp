@@ -8,6 +8,7 @@
 #include <torch/csrc/autograd/python_variable.h>
 #include <torch/csrc/jit/frontend/tracer.h>
 #include <ATen/EmptyTensor.h>
+#include <ATen/ops/zeros.h>
 #include <ATen/hip/EmptyTensor.h>
 #include <c10/hip/HIPFunctions.h>
 #include <c10/hip/HIPGraphsC10Utils.h>
@@ -15,6 +16,7 @@
 
 #include <chrono>
 #include <cstring>
+#include <map>
 
 #include "../../include/bsi_hip.h"
 
@@ -33,6 +35,9 @@ struct Library {
     decltype(&bsi_hip_ewah_emit) ewah_emit;
     decltype(&bsi_hip_dot_ewah_batch) dot_ewah_batch;
     decltype(&bsi_hip_dot_ewah_batch_workspace_bytes) dot_ewah_batch_workspace_bytes;
+    decltype(&bsi_hip_linear_coop_out) linear_coop_out;
+    decltype(&bsi_hip_linear_coop_serves) linear_coop_serves;
+    decltype(&bsi_hip_linear_coop_bytes) linear_coop_bytes;
     decltype(&bsi_hip_scalar_query_dot) scalar_query_dot;
     decltype(&bsi_hip_build_measure) build_measure;
     decltype(&bsi_hip_ewah_emit_at) ewah_emit_at;
@@ -247,6 +252,40 @@ PyObject* build_key(PyObject*, PyObject* args) {
     END_HANDLE_TH_ERRORS
 }
 
+// The keys of the layer that runs next (set by quantize_model_bsi), touched by this dot's kernel; nullptr: none.
+const void* keys_to_warm(PyObject* layer, int64_t rows, const at::Device& device, size_t* bytes) {
+    PyObject* const next = rows > shared.stream_max ? get(layer, names._next_bsi_layer) : nullptr;
+    if (next == nullptr || next == Py_None) return nullptr;
+    Holder attrs(PyObject_GenericGetDict(next, nullptr));
+    PyObject* handle = attrs.p != nullptr ? get(attrs.p, names._bsi_keys_cuda) : nullptr;
+    Holder group_keys;
+    if (PyObject* g = attrs.p != nullptr ? get(attrs.p, names._fused) : nullptr; g != nullptr && PyTuple_Check(g)) {
+        group_keys.p = PyObject_GetAttr(PyTuple_GET_ITEM(g, 0), names.keys);
+        handle = group_keys.p;
+    }
+    PyErr_Clear();
+    Keys k;
+    int layout = 0;
+    return read_keys(handle, device, &k) ? key_operand(k, rows, &layout, bytes) : nullptr;
+}
+
+// The area of launches with the query build inside, one for each stream that has made one (at most kCoopAreas; other streams
+// take the two-launch path), until forget().  Under the interpreter lock.
+constexpr size_t kCoopAreas = 32;
+std::map<std::pair<int, hipStream_t>, at::Tensor> coop_areas;
+uint64_t coop_launches = 0;
+void* coop_area(const at::Device& device, hipStream_t st) {
+    const auto found = coop_areas.find({device.index(), st});
+    if (found != coop_areas.end()) return found->second.data_ptr();
+    if (coop_areas.size() >= kCoopAreas) return nullptr;
+    at::Tensor area = at::zeros({static_cast<int64_t>(lib.linear_coop_bytes())}, at::TensorOptions().dtype(at::kByte).device(device));
+    return coop_areas.emplace(std::make_pair(device.index(), st), std::move(area)).first->second.data_ptr();
+}
+PyObject* forget(PyObject*, PyObject*) {
+    coop_areas.clear();
+    Py_RETURN_NONE;
+}
+
 // linear(layer.__dict__, x) -> the layer's output, or None.
 PyObject* linear(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     if (nargs != 2 || !PyDict_Check(args[0])) {
@@ -290,6 +329,11 @@ PyObject* linear(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     PyObject* slot = nullptr;
     void* ws = nullptr;
     int64_t ws_bytes = 0;
+    int layout = 0;
+    size_t bytes = 0;
+    const void* const operand = key_operand(k, rows, &layout, &bytes);
+    void* const coop = !few && k.Sb <= 8 && lib.linear_coop_serves(rows, d, k.R, static_cast<int>(decimals), config.bits, layout, static_cast<int>(k.Sb))
+                           ? coop_area(device, st) : nullptr;
     if (few) {
         if (!known_few_rows(device.index(), rows, d)) Py_RETURN_NONE;
     } else {
@@ -298,14 +342,16 @@ PyObject* linear(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
         if (record == nullptr || !get_int(record, names.bytes, &ws_bytes) ||
             static_cast<size_t>(ws_bytes) < lib.linear_workspace_bytes(rows, d, config.bits))
             Py_RETURN_NONE;
-        Holder handle(PyLong_FromVoidPtr(st));
-        PyObject* const eager = get(record, names.eager);
-        PyObject* const mine = eager != nullptr ? PyDict_GetItem(eager, handle.p) : nullptr;
-        if (mine == nullptr || !PyTuple_Check(mine) || PyTuple_GET_SIZE(mine) != 2 || !THPVariable_Check(PyTuple_GET_ITEM(mine, 0)))
-            Py_RETURN_NONE;
-        ws = THPVariable_Unpack(PyTuple_GET_ITEM(mine, 0)).data_ptr();
-        slot = PyTuple_GET_ITEM(mine, 1);
-        if (!PyList_Check(slot) || PyList_GET_SIZE(slot) != 2 || !split_scratch(device.index(), rows, k.R, k.W)) Py_RETURN_NONE;
+        if (coop == nullptr) {
+            Holder handle(PyLong_FromVoidPtr(st));
+            PyObject* const eager = get(record, names.eager);
+            PyObject* const mine = eager != nullptr ? PyDict_GetItem(eager, handle.p) : nullptr;
+            if (mine == nullptr || !PyTuple_Check(mine) || PyTuple_GET_SIZE(mine) != 2 || !THPVariable_Check(PyTuple_GET_ITEM(mine, 0)))
+                Py_RETURN_NONE;
+            ws = THPVariable_Unpack(PyTuple_GET_ITEM(mine, 0)).data_ptr();
+            slot = PyTuple_GET_ITEM(mine, 1);
+            if (!PyList_Check(slot) || PyList_GET_SIZE(slot) != 2 || !split_scratch(device.index(), rows, k.R, k.W)) Py_RETURN_NONE;
+        }
     }
 
     Holder owned;  // the object that stands for x when it is not the caller's
@@ -321,7 +367,16 @@ PyObject* linear(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     const float inv = scale_inv(decimals, k.decimals);
     const void* const xp = x.const_data_ptr();
     int rc = BSI_OK;
-    if (few) {
+    if (coop != nullptr) {
+        size_t warm_bytes = 0;
+        const void* const warm = keys_to_warm(layer, rows, device, &warm_bytes);
+        // under the interpreter lock: launches on an area are in the order of their numbers
+        rc = lib.linear_coop_out(xp, in_code, rows, d, static_cast<int>(decimals), config.bits, ++coop_launches, coop,
+                                 static_cast<const uint64_t*>(operand), layout, k.weights->const_data_ptr<float>(), static_cast<int>(k.Sb),
+                                 k.R, inv, k.R, bias, out.data_ptr(), in_code, warm, warm_bytes, st);
+        if (rc != BSI_OK) return fail_status(rc, "bsi_hip_linear_coop_out");
+        count(layer, names.build_calls, 1);
+    } else if (few) {
         Py_BEGIN_ALLOW_THREADS
         rc = lib.linear_few_rows_out(xp, in_code, rows, d, static_cast<int>(decimals), config.bits,
                                      static_cast<const uint64_t*>(k.words->const_data_ptr()), k.weights->const_data_ptr<float>(),
@@ -345,23 +400,8 @@ PyObject* linear(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
         }
         Py_INCREF(x_object);
         PyList_SetItem(slot, 1, x_object);  // its address is not reused while the build stands for it
-        int layout = 0, warm_layout = 0;
-        size_t bytes = 0, warm_bytes = 0;
-        const void* const operand = key_operand(k, rows, &layout, &bytes);
-        const void* warm = nullptr;
-        PyObject* next = rows > shared.stream_max ? get(layer, names._next_bsi_layer) : nullptr;
-        if (next != nullptr && next != Py_None) {  // the keys of the layer that runs next, touched by this dot's kernel
-            Holder attrs(PyObject_GenericGetDict(next, nullptr));
-            PyObject* handle = attrs.p != nullptr ? get(attrs.p, names._bsi_keys_cuda) : nullptr;
-            Holder group_keys;
-            if (PyObject* g = attrs.p != nullptr ? get(attrs.p, names._fused) : nullptr; g != nullptr && PyTuple_Check(g)) {
-                group_keys.p = PyObject_GetAttr(PyTuple_GET_ITEM(g, 0), names.keys);
-                handle = group_keys.p;
-            }
-            PyErr_Clear();
-            Keys nk;
-            if (read_keys(handle, device, &nk)) warm = key_operand(nk, rows, &warm_layout, &warm_bytes);
-        }
+        size_t warm_bytes = 0;
+        const void* const warm = keys_to_warm(layer, rows, device, &warm_bytes);
         // under the interpreter lock: another thread on this stream must not find the slot before the build is enqueued,
         // nor enqueue a build of its own between the two launches
         rc = lib.linear_out(xp, in_code, rows, d, static_cast<int>(decimals), config.bits, rebuild, ws, static_cast<size_t>(ws_bytes),
@@ -756,6 +796,9 @@ PyObject* bind(PyObject*, PyObject* args) {
         !entry(entries, "bsi_hip_ewah_emit", &lib.ewah_emit) || !entry(entries, "bsi_hip_dot_ewah_batch", &lib.dot_ewah_batch) ||
         !entry(entries, "bsi_hip_dot_ewah_batch_workspace_bytes", &lib.dot_ewah_batch_workspace_bytes) ||
         !entry(entries, "bsi_hip_build_measure", &lib.build_measure) || !entry(entries, "bsi_hip_ewah_emit_at", &lib.ewah_emit_at) ||
+        !entry(entries, "bsi_hip_linear_coop_out", &lib.linear_coop_out) ||
+        !entry(entries, "bsi_hip_linear_coop_serves", &lib.linear_coop_serves) ||
+        !entry(entries, "bsi_hip_linear_coop_bytes", &lib.linear_coop_bytes) ||
         !entry(entries, "bsi_hip_scalar_query_dot", &lib.scalar_query_dot) ||
         !entry(entries, "bsi_hip_scalar_query_host_words", &lib.scalar_query_host_words) ||
         !take(state, "keys_type", &shared.keys_type) || !take(state, "batch_type", &shared.batch_type) ||
@@ -781,6 +824,7 @@ PyMethodDef methods[] = {
     {"dot_streams", reinterpret_cast<PyCFunction>(reinterpret_cast<void*>(dot_streams)), METH_FASTCALL, nullptr},
     {"linear", reinterpret_cast<PyCFunction>(reinterpret_cast<void*>(linear)), METH_FASTCALL, nullptr},
     {"scalar_query", reinterpret_cast<PyCFunction>(reinterpret_cast<void*>(scalar_query)), METH_FASTCALL, nullptr},
+    {"forget", forget, METH_NOARGS, nullptr},
     {"bind_layer", bind_layer, METH_VARARGS, nullptr},
     {"layer_call", reinterpret_cast<PyCFunction>(reinterpret_cast<void*>(layer_call)), METH_FASTCALL | METH_KEYWORDS, nullptr},
     {"dot", reinterpret_cast<PyCFunction>(reinterpret_cast<void*>(dot)), METH_FASTCALL, nullptr},

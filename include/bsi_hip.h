@@ -237,6 +237,8 @@ int bsi_hip_planes_to_int8_tiled(const uint64_t* words_device, int64_t rows, int
 #define BSI_OPT_I8_SPLIT 5 /* D-split of the int8-image dot (see bsi_hip_dot_attach_split_scratch): 1 = never, n >= 2 = n
                               segments (on the tile BSI_OPT_I8_TILE forces, 128 or 12864; 128 otherwise) whenever the
                               attached scratch holds them; 0 (default) = chosen per call by a cost model */
+#define BSI_OPT_COOP_PATIENCE 6 /* ticks of the 100 MHz clock that a workgroup of bsi_hip_linear_coop_out waits for a share of
+                                   the query build before it builds the share itself (default 2000; 0: at once) */
 int bsi_hip_set_option(int option, int value);
 
 /* Bytes of device workspace bsi_hip_dot needs for this shape and core (0 when none). */
@@ -378,6 +380,17 @@ int bsi_hip_linear_out(const void* x_device, int dtype, int64_t Q, int64_t d, in
                        void* workspace, size_t workspace_bytes, const uint64_t* B, int b_layout, const float* Bw, int Sb,
                        int64_t R, float scale_inv, int64_t R_total, const float* bias, void* out, int out_dtype, int core,
                        const void* warm, size_t warm_bytes, void* stream);
+
+/* A small layer in ONE launch: every XCD quantises the activations for the workgroups it runs (see
+ * bsi_hip_linear_coop_serves for the shapes; the same integers, scales and chain as bsi_hip_linear_out, so the same bits).
+ * area: bsi_hip_linear_coop_bytes() bytes of device memory, 256-aligned, zero when first used, for one stream's launches.
+ * launch_number: not 0 and another one for every launch on the area. */
+size_t bsi_hip_linear_coop_bytes(void);
+int bsi_hip_linear_coop_serves(int64_t Q, int64_t d, int64_t R, int decimal_places, int fixed_bits, int b_layout, int Sb);
+int bsi_hip_linear_coop_out(const void* x_device, int dtype, int64_t Q, int64_t d, int decimal_places, int fixed_bits,
+                            uint64_t launch_number, void* area, const uint64_t* B, int b_layout, const float* Bw, int Sb, int64_t R,
+                            float scale_inv, int64_t R_total, const float* bias, void* out, int out_dtype, const void* warm,
+                            size_t warm_bytes, void* stream);
 
 /* 1 when bsi_hip_linear_few_rows, for this shape, issues the loads of the whole query build before its first key
  * loads (the case in which the launch costs the GPU no more than the dot alone), 0 when some of the build waits
