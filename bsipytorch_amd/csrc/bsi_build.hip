@@ -12,6 +12,8 @@
 // (bsi_cuda_kernels_pack.cuh:129-174).
 #include "bsi_quant_device.h"
 
+#include <type_traits>
+
 namespace bsi {
 
 constexpr int kBlock = 256;
@@ -459,52 +461,99 @@ __global__ __launch_bounds__(kBlock) void build_fixed_row_fast_kernel(const T* _
     }
 }
 
+// Bytes of a quad as sign and magnitude (at most 127) -> shifted right with rounding (half away from zero), clamped and
+// moved to the byte's top as two's complement, four at a time: every step stays inside its byte.  The row's largest
+// magnitude gave the shift, so that a shifted magnitude is 2^(slices - 1) at most, and only a positive one is one too many.
+struct QuadShift {
+    uint32_t half, keep, xor_top, keep_top;
+    int shift, top, up;
+};
+__device__ __forceinline__ QuadShift quad_shift(int shift, int slices) {
+    QuadShift q;
+    q.shift = shift & 7;  // magnitudes of at most 127 never take more
+    q.half = ((1u << q.shift) >> 1) * 0x01010101u;
+    q.keep = (0xFFu >> q.shift) * 0x01010101u;
+    q.top = slices - 1;
+    q.up = 8 - slices;
+    q.xor_top = slices == 8 ? 0x80808080u : 0u;
+    q.keep_top = ((0xFFu << q.up) & 0xFFu) * 0x01010101u;
+    return q;
+}
+__device__ __forceinline__ uint32_t shift_quad_bytes(uint32_t sm, const QuadShift& q) {
+    const uint32_t neg1 = (sm >> 7) & 0x01010101u;
+    uint32_t m = (((sm & 0x7F7F7F7Fu) + q.half) >> q.shift) & q.keep;
+    m -= (m >> q.top) & (neg1 ^ 0x01010101u);
+    const uint32_t minus = m & ((neg1 << 8) - neg1);
+    const uint32_t biased = m + 0x80808080u - (minus << 1);  // 128 + the signed value
+    return ((biased << q.up) & q.keep_top) ^ q.xor_top;
+}
+
 // The whole of a fixed-bit key build for the common case: one workgroup = 16 rows (a tile of the tiled planes), a wave
-// each.  A wave reads its row once: the signed magnitudes of the first kHeld chunks stay in registers as 16-bit pairs
-// until the row's maximum is known (a row with |x| of 256 or more, and the rest of a longer row, is read again).  It
-// writes the int8 image, 256 contiguous bytes a chunk, and puts its planes' half-words into LDS, from where the
-// workgroup writes the tile's words of eight chunks at a time as one contiguous run (a row's own words lie 128 bytes
-// apart there).  Slice weights and shifts come out of the same launch.
-// 16384 x 4096 float32: 345 us in five launches (two passes over the rows in 64-bit integers, planes, tiled planes,
-// image, weights), 95 us: 370 MB at 3.9 TB/s.
+// each.  A wave reads its row once: the rounded magnitudes and signs of the first kHeld chunks stay in registers as bytes
+// until the row's maximum is known (a row with a magnitude over 127, |x| of 1.27 at two decimal places, and the rest of a
+// longer row are read again).  It writes the int8 image, 256 contiguous bytes a chunk, and puts its planes' half-words
+// into LDS, from where the workgroup writes the tile's words of eight chunks at a time as one contiguous run (a row's own
+// words lie 128 bytes apart there).  Slice weights and shifts come out of the same launch.
+//
+// Memory and VALU work are of the same order here (16384 x 4096 float32: 387 MB, 75 us at the rate of a large copy), and a
+// workgroup alternates between the two, so that two of them share a CU: 64 registers (with one a CU 8192 x 5120 bfloat16
+// takes 44 us instead of 31).  Float32 arithmetic rounds towards zero throughout the kernel: a * 10^dec + 0.5 then never rounds up to an integer that the exact
+// value does not reach, the conversion to a byte truncates, and every other float operation here is exact.
+// The stores are nontemporal: nobody reads the planes or the image before the launch is over, and lines that wait in the
+// L2s are written back at its end.  Before (16-bit pairs in registers for up to 16 chunks, plain stores) and now, us:
+// 16384 x 4096 float32 94.9 -> 79.2 (4.9 TB/s), 8192 x 8192 119.4 -> 85.7, 4096 x 4096 22.5 -> 18.6, 768 x 768 6.7 -> 4.5;
+// bfloat16 16384 x 4096 64.2 -> 54.3, 8192 x 5120 37.4 -> 26.7, 2048 x 2048 8.4 -> 7.3.
 constexpr int kKeyRows = 16, kKeyGroup = 8;
-template <typename T, bool kVec, int kHeld>
-__global__ __launch_bounds__(kKeyRows * BSI_WAVE) void build_keys_fast_kernel(
+template <typename T, bool kVec, int kHeld, int kLoads>
+__global__ __launch_bounds__(kKeyRows * BSI_WAVE, 8) void build_keys_fast_kernel(
     const T* __restrict__ x, int64_t R, int64_t d, int chunks, int slices, double dec_scale, float scale,
     unsigned long long* __restrict__ tiled, int8_t* __restrict__ image8, int* __restrict__ shifts, float* __restrict__ weights) {
     // [chunk][slice][word of the chunk][row], rows padded to 17 so that the half-words of a wave spread over the banks
     constexpr int kWordStride = 17, kSliceStride = 4 * kWordStride, kChunkStride = 8 * kSliceStride;
     __shared__ unsigned long long stage[kKeyGroup * kChunkStride];
+    __builtin_amdgcn_s_setreg(1 | (1 << 11), 3);  // MODE, the two rounding bits of float32: towards zero
     const int lane = threadIdx.x & (BSI_WAVE - 1);
     const int rr = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int64_t row = static_cast<int64_t>(blockIdx.x) * kKeyRows + rr;
     const bool have = row < R;
     const T* xrow = x + (have ? row : R - 1) * d;
     const ChunkLane cl = chunk_lane(lane);
-    uint32_t held[kHeld][2];
-    unsigned mx = 0u;
+    uint32_t held[kHeld];
+    float mxf = 0.0f;
+    auto take_max = [&](const float (&v)[4]) {  // a NaN stays
+        mxf = __builtin_elementwise_maximum(__builtin_elementwise_maximum(mxf, fabsf(v[0])), fabsf(v[1]));
+        mxf = __builtin_elementwise_maximum(__builtin_elementwise_maximum(mxf, fabsf(v[2])), fabsf(v[3]));
+    };
 #pragma unroll
-    for (int c = 0; c < kHeld; ++c) {
-        float v[4];
-        load_chunk_quad<T, kVec>(xrow, d, c, cl, v);  // past the row: zeros
-        const unsigned m = quad_max_bits(v);
-        mx = m > mx ? m : mx;
-        uint32_t b[4];
+    for (int c = 0; c < kHeld; c += kLoads) {
+        if (c >= chunks) break;
+        float v[kLoads][4];
 #pragma unroll
-        for (int k = 0; k < 4; ++k)
-            b[k] = __float_as_uint(copysignf(scaled_magnitude_f32<T>(fabsf(v[k]), scale), v[k]) + 12582912.0f);
-        held[c][0] = __builtin_amdgcn_perm(b[1], b[0], 0x05040100u);
-        held[c][1] = __builtin_amdgcn_perm(b[3], b[2], 0x05040100u);
+        for (int j = 0; j < kLoads; ++j) load_chunk_quad<T, kVec>(xrow, d, c + j, cl, v[j]);  // past the row: zeros
+#pragma unroll
+        for (int j = 0; j < kLoads; ++j) {
+            take_max(v[j]);
+            uint32_t m = 0u;
+            m = __builtin_amdgcn_cvt_pk_u8_f32(fmaf(fabsf(v[j][0]), scale, 0.5f), 0, m);
+            m = __builtin_amdgcn_cvt_pk_u8_f32(fmaf(fabsf(v[j][1]), scale, 0.5f), 1, m);
+            m = __builtin_amdgcn_cvt_pk_u8_f32(fmaf(fabsf(v[j][2]), scale, 0.5f), 2, m);
+            m = __builtin_amdgcn_cvt_pk_u8_f32(fmaf(fabsf(v[j][3]), scale, 0.5f), 3, m);
+            const uint32_t signs = __builtin_amdgcn_perm(
+                __builtin_amdgcn_perm(__float_as_uint(v[j][3]), __float_as_uint(v[j][2]), 0x0c0c0703u),
+                __builtin_amdgcn_perm(__float_as_uint(v[j][1]), __float_as_uint(v[j][0]), 0x0c0c0703u), 0x05040100u);
+            held[c + j] = bsel(m, signs, 0x7F7F7F7Fu);
+            asm volatile("" : "+v"(held[c + j]));  // packed here: sunk to its use it would keep four registers instead of one
+        }
+        __builtin_amdgcn_sched_barrier(0);
     }
     for (int c = kHeld; c < chunks; ++c) {
         float v[4];
         load_chunk_quad<T, kVec>(xrow, d, c, cl, v);
-        const unsigned m = quad_max_bits(v);
-        mx = m > mx ? m : mx;
+        take_max(v);
     }
-    mx = wave_max_u32(mx);
-    constexpr unsigned kHeldLimit = 0x43800000u;  // 256.0f: 127 times that fits a signed 16-bit magnitude
+    const unsigned mx = __builtin_amdgcn_readfirstlane(wave_max_u32(__float_as_uint(mxf) & 0x7FFFFFFFu));
     const bool wide = mx >= kQuantWideBits;
+    const bool in_bytes = !wide && scaled_magnitude_f32<float>(__uint_as_float(mx), scale) <= 127.0f;
     int shift = quant_shift(mx, scale, slices);
     if (wide) {
         unsigned long long m64 = 0ULL;
@@ -516,41 +565,31 @@ __global__ __launch_bounds__(kKeyRows * BSI_WAVE) void build_keys_fast_kernel(
         }
         shift = compute_shift(wave_max_u64(m64), 0.0, 1, slices, 0.0f);
     }
+    shift = __builtin_amdgcn_readfirstlane(shift);
     if (have && lane < slices) {
         const float w = static_cast<float>(1ULL << shift) * static_cast<float>(1 << lane);
         weights[row * slices + lane] = lane == slices - 1 ? -w : w;
         if (lane == 0) shifts[row] = shift;
     }
     const QuantRange range = quant_range(slices);
-    const float inv = __uint_as_float(static_cast<uint32_t>(127 - shift) << 23);
-    const int words_per_group = slices * 64;  // words of a chunk of the tile
-    for (int c0 = 0; c0 < chunks; c0 += kKeyGroup) {
+    const QuadShift in_byte = quad_shift(shift, slices);
+    auto group = [&](int c0, auto first_held) {
+        constexpr int kFirst = decltype(first_held)::value;  // the group's first chunk in `held`, or -1
         const int n = chunks - c0 < kKeyGroup ? chunks - c0 : kKeyGroup;
 #pragma unroll
         for (int u = 0; u < kKeyGroup; ++u) {
             const int c = c0 + u;
             if (u < n) {
                 uint32_t bytes;
-                if (c0 < kHeld && mx < kHeldLimit) {
-                    const uint32_t lo = c0 == 0 ? held[u][0] : held[(kKeyGroup + u) % kHeld][0];
-                    const uint32_t hi = c0 == 0 ? held[u][1] : held[(kKeyGroup + u) % kHeld][1];
-                    uint32_t b[4];
-#pragma unroll
-                    for (int k = 0; k < 4; ++k) {
-                        const uint32_t pair = k < 2 ? lo : hi;
-                        const float t = static_cast<float>(static_cast<int>(static_cast<int16_t>(pair >> (16 * (k & 1)))));
-                        const float q = truncf(fmaf(fabsf(t), inv, 0.5f));
-                        const float s = __builtin_amdgcn_fmed3f(copysignf(q, t), range.lo, range.hi);
-                        b[k] = __float_as_uint(fmaf(s, range.up, 12582912.0f));
-                    }
-                    bytes = pack_low_bytes(b[0], b[1], b[2], b[3]);
+                if (kFirst >= 0 && in_bytes) {
+                    bytes = shift_quad_bytes(held[(kFirst < 0 ? 0 : kFirst) + u], in_byte);
                 } else {
                     float v[4];
                     load_chunk_quad<T, kVec>(xrow, d, c, cl, v);
                     bytes = wide ? quantise_quad_wide(v, dec_scale, shift, slices) : quantise_quad<T>(v, scale, shift, range);
                 }
                 const uint32_t image = chunk_image_dword(bytes, cl);
-                if (have) reinterpret_cast<uint32_t*>(image8)[(static_cast<size_t>(row) * chunks + c) * (BSI_CHUNK_ELEMS / 4) + lane] = image;
+                if (have) __builtin_nontemporal_store(image, reinterpret_cast<uint32_t*>(image8) + (static_cast<size_t>(row) * chunks + c) * (BSI_CHUNK_ELEMS / 4) + lane);
                 const int sl = (lane & 7) - (8 - slices), unit = lane >> 3;
                 const uint32_t plane = chunk_plane_dword(image, cl);
                 if (sl >= 0)
@@ -559,13 +598,24 @@ __global__ __launch_bounds__(kKeyRows * BSI_WAVE) void build_keys_fast_kernel(
             }
         }
         __syncthreads();
-        unsigned long long* dst = tiled + (static_cast<size_t>(blockIdx.x) * chunks + c0) * words_per_group;
-        for (int o = threadIdx.x; o < n * words_per_group; o += kKeyRows * BSI_WAVE) {
-            const int u = o / words_per_group, w = o - u * words_per_group;  // w = slice * 64 + word * 16 + row
-            dst[o] = stage[u * kChunkStride + (w >> 6) * kSliceStride + ((w >> 4) & 3) * kWordStride + (w & 15)];
+        // a chunk's words by 512 threads (there are slices * 64 of them): thread w % 512 = slice * 64 + word * 16 + row
+        const int w = threadIdx.x & 511, words = slices * 64;
+        unsigned long long* dst = tiled + (static_cast<size_t>(blockIdx.x) * chunks + c0) * words + w;
+        const unsigned long long* src = stage + (w >> 6) * kSliceStride + ((w >> 4) & 3) * kWordStride + (w & 15);
+        if (w < words) {
+#pragma unroll
+            for (int u = 0; u < kKeyGroup; u += 2) {
+                const int v = u + (rr >> 3);
+                if (v < n) __builtin_nontemporal_store(src[v * kChunkStride], dst + static_cast<size_t>(v) * words);
+            }
         }
         __syncthreads();
-    }
+    };
+    group(0, std::integral_constant<int, 0>{});
+    if (kHeld > 8 && chunks > 8) group(8, std::integral_constant<int, (kHeld > 8) ? 8 : -1>{});
+    if (kHeld > 16 && chunks > 16) group(16, std::integral_constant<int, (kHeld > 16) ? 16 : -1>{});
+    if (kHeld > 24 && chunks > 24) group(24, std::integral_constant<int, (kHeld > 24) ? 24 : -1>{});
+    for (int c0 = kHeld; c0 < chunks; c0 += kKeyGroup) group(c0, std::integral_constant<int, -1>{});
 }
 
 static inline unsigned grid_for(int64_t waves) {
@@ -891,13 +941,19 @@ extern "C" int bsi_hip_build_fixed_keys(const void* x, int dtype, int64_t R, int
     BSI_REQUIRE(x && tiled && image && shifts && slice_weights, "null pointer");
     BSI_REQUIRE((R + kKeyRows - 1) / kKeyRows <= 0x7fffffffLL, "too many rows for one launch");
     const int chunks = static_cast<int>((d + 255) / 256);
-    // Chunks kept in registers: 16 for rows of 9 to 16 chunks, which then need no second read of any of them (4096 x 4096:
-    // 22.8 us against 29.5), 8 otherwise: two workgroups a CU instead of one (8192 x 2048: 19.5 us against 27.1).
-    BSI_DISPATCH_DTYPE(dtype, BSI_DISPATCH_BOOL(quads_aligned(x, dtype, d), kVec, BSI_DISPATCH_BOOL(chunks > 8 && chunks <= 16, kLong,
-        launch((build_keys_fast_kernel<T, kVec, kLong ? 16 : 8>), dim3(static_cast<unsigned>((R + kKeyRows - 1) / kKeyRows)),
-                           dim3(kKeyRows * BSI_WAVE), 0, as_stream(stream), static_cast<const T*>(x), R, d, chunks, fixed_bits,
-                           static_cast<double>(scale_int), static_cast<float>(scale_int),
-                           reinterpret_cast<unsigned long long*>(tiled), image, shifts, slice_weights))))
+    // Rows of up to 32 chunks stay in registers whole.  kHeld is the next of 8, 16 and 32, kLoads what the rest of the 64
+    // registers takes in flight (32 chunks, 8192 x 5120 bfloat16 with plain stores: 2, 4, 8 loads 44, 31, 34 us).
+    const int64_t tiles = (R + kKeyRows - 1) / kKeyRows;
+#define BSI_KEYS(kHeld, kLoads)                                                                                              \
+    BSI_DISPATCH_DTYPE(dtype, BSI_DISPATCH_BOOL(quads_aligned(x, dtype, d), kVec,                                             \
+        launch((build_keys_fast_kernel<T, kVec, kHeld, kLoads>), dim3(static_cast<unsigned>(tiles)),                 \
+               dim3(kKeyRows * BSI_WAVE), 0, as_stream(stream), static_cast<const T*>(x), R, d, chunks, fixed_bits,           \
+               static_cast<double>(scale_int), static_cast<float>(scale_int),                                                \
+               reinterpret_cast<unsigned long long*>(tiled), image, shifts, slice_weights)))
+    if (chunks <= 8) BSI_KEYS(8, 8)
+    else if (chunks <= 16) BSI_KEYS(16, 8)
+    else BSI_KEYS(32, 4)
+#undef BSI_KEYS
     BSI_LAUNCH_CHECK("build_keys_fast_kernel");
     return BSI_OK;
 }

@@ -69,3 +69,29 @@ def test_query_build_with_and_without_planes(hip, oracle, rows, d, dtype, kind):
     planes_dev = dev(want)
     hip.check(hip.lib.bsi_hip_planes_to_int8(planes_dev.data_ptr(), rows, 7, W, from_planes.data_ptr(), st()), "image")
     assert torch.equal(images[0], from_planes) and torch.equal(images[1], from_planes)
+
+
+@pytest.mark.parametrize("bits", [2, 6, 8])
+@pytest.mark.parametrize("largest", [1.2749, 1.275, 0.3149])
+@pytest.mark.parametrize("rows,d,dtype", [(17, 2049, torch.float32), (16, 2304, torch.float16), (3, 4352, torch.bfloat16),
+                                          (33, 8192, torch.float32), (5, 8450, torch.float16)])
+def test_key_build_from_bytes(hip, oracle, rows, d, dtype, largest, bits):
+    """Rows at the end of what is held as bytes, and past it; widths around the groups that are held."""
+    rng = np.random.default_rng(rows + d + bits)
+    x = torch.from_numpy(rng.uniform(-0.99 * largest, 0.99 * largest, (rows, d)).astype(np.float32))
+    x[:, d - 1], x[::2, d // 2] = 0.005, -largest
+    x = x.to(dtype)
+    ints, shifts, scales = oracle.quantize_fixed(x.to(torch.float32).numpy(), 2, bits, False)
+    planes, W, chunks = dev(oracle.pack(ints, bits)), (d + 63) // 64, (d + 255) // 256
+    want = [torch.zeros(((rows + 15) // 16, chunks, bits, 64), dtype=torch.int64, device="cuda"),
+            torch.zeros((rows, chunks * 256), dtype=torch.int8, device="cuda")]
+    hip.check(hip.lib.bsi_hip_tile_key_planes(planes.data_ptr(), rows, bits, W, want[0].data_ptr(), st()), "tile")
+    hip.check(hip.lib.bsi_hip_planes_to_int8(planes.data_ptr(), rows, bits, W, want[1].data_ptr(), st()), "image")
+    tiled, image = torch.full_like(want[0], 77), torch.full_like(want[1], 77)
+    sh, w = torch.full((rows,), -1, dtype=torch.int32, device="cuda"), torch.zeros((rows, bits), device="cuda")
+    xd, code = x.cuda(), {torch.float32: 0, torch.float16: 1, torch.bfloat16: 2}[dtype]
+    hip.check(hip.lib.bsi_hip_build_fixed_keys(xd.data_ptr(), code, rows, d, 2, bits, tiled.data_ptr(), image.data_ptr(),
+                                               sh.data_ptr(), w.data_ptr(), st()), "keys")
+    np.testing.assert_array_equal(sh.cpu().numpy(), shifts.reshape(-1))
+    np.testing.assert_array_equal(w[:, 0].cpu().numpy(), scales.reshape(-1))
+    assert torch.equal(tiled, want[0]) and torch.equal(image, want[1])
