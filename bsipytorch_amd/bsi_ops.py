@@ -104,6 +104,7 @@ def _flags() -> dict:
         dot_split=(_env_int("BSI_DOT_SPLIT", 1) or 0) != 0,
     )
     f = _flag_cache
+    f["one_launch_keys"] = 2 <= bits_k <= 8 and f["clip_k"] == 0.0 and f["tiled"] and f["key_image"] and not f["image_tiled"]
     if (2 <= bits_q <= 8 and f["chunk_scale"] and f["clip_k"] == 0.0 and f["core"] != _lib.CORE_VALU
             and not (f["profile"] or f["debug"] or f["dot_debug"])):
         _native.configure(bits_q, f["core"])  # the configurations its calls serve
@@ -745,8 +746,7 @@ def canonical_key_planes(keys: "PrebuiltBSIKeysCUDA") -> torch.Tensor:
 def _one_launch_key_build(f: dict, x: torch.Tensor, decimals: int) -> bool:
     """Whether bsi_hip_build_fixed_keys makes every representation this configuration keeps of a keyset: tiled planes and
     the row-major int8 image, from 2 to 8 bits, at most two decimal places and no clipping."""
-    return (x.numel() > 0 and 2 <= f["bits_k"] <= 8 and f["clip_k"] == 0.0 and 0 <= decimals <= 2 and f["tiled"] and f["key_image"]
-            and not f["image_tiled"])
+    return x.numel() > 0 and f["one_launch_keys"] and 0 <= decimals <= 2
 
 
 def build_bsi_keys_cuda(K: torch.Tensor, decimal_places: int, compress_threshold: float = 0.2):
@@ -754,6 +754,16 @@ def build_bsi_keys_cuda(K: torch.Tensor, decimal_places: int, compress_threshold
     Returns (handle, total_bytes_of_words, num_keys, d, W)."""
     _check(K.dim() == 2, "K must be 2D [num_keys, d]")
     f = _flags()
+    if f["one_launch_keys"] and not f["debug"]:
+        built = _native.build_keys(K, int(decimal_places), f["bits_k"])  # None: a call it does not serve
+        if built is not None:
+            words, ints8, shifts, weights, R, d = built
+            W, Sb = (d + 63) // 64, f["bits_k"]
+            h = PrebuiltBSIKeysCUDA.__new__(PrebuiltBSIKeysCUDA)  # every attribute of __init__ in one go: half of the call's host time
+            h.__dict__ = {"words": words, "layout": _lib.LAYOUT_TILED16, "ints8": ints8, "ints8_tiled": False,
+                          "slice_weights": weights, "shifts": shifts, "fixed": True, "digits8": None, "Sb": Sb, "W": W, "d": d,
+                          "num_keys": R, "decimals": int(decimal_places), "threshold": float(compress_threshold)}
+            return h, R * Sb * W * 8, R, d, W
     dev = _device()
     x = _as_build_input(K, dev)
     R, d = x.shape
@@ -1530,7 +1540,7 @@ def debug_quantize_int64_cpu(values: torch.Tensor, decimal_places: int) -> torch
 # The native host path reads these on every call, so what the functions above keep stays the one copy.
 _native.bind({name: ctypes.cast(getattr(lib, name), ctypes.c_void_p).value
               for name in ("bsi_hip_linear_few_rows_out", "bsi_hip_linear_out", "bsi_hip_linear_workspace_bytes", "bsi_hip_dot",
-                           "bsi_hip_build_fixed", "bsi_hip_ewah_measure", "bsi_hip_ewah_emit", "bsi_hip_dot_ewah_batch",
+                           "bsi_hip_build_fixed", "bsi_hip_build_fixed_keys", "bsi_hip_ewah_measure", "bsi_hip_ewah_emit", "bsi_hip_dot_ewah_batch",
                            "bsi_hip_dot_ewah_batch_workspace_bytes", "bsi_hip_scalar_query_dot",
                            "bsi_hip_build_measure", "bsi_hip_ewah_emit_at", "bsi_hip_linear_coop_out",
                            "bsi_hip_linear_coop_serves", "bsi_hip_linear_coop_bytes",

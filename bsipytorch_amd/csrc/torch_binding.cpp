@@ -31,6 +31,7 @@ struct Library {
     decltype(&bsi_hip_linear_workspace_bytes) linear_workspace_bytes;
     decltype(&bsi_hip_dot) dot;
     decltype(&bsi_hip_build_fixed) build_fixed;
+    decltype(&bsi_hip_build_fixed_keys) build_fixed_keys;
     decltype(&bsi_hip_ewah_measure) ewah_measure;
     decltype(&bsi_hip_ewah_emit) ewah_emit;
     decltype(&bsi_hip_dot_ewah_batch) dot_ewah_batch;
@@ -550,6 +551,40 @@ PyObject* build(PyObject*, PyObject* args) {
     END_HANDLE_TH_ERRORS
 }
 
+// build_keys(K, decimals, bits) -> (tiled planes, int8 image, shifts, slice weights, R, d), or None: the one-launch build of a
+// contiguous key matrix on the current device.
+PyObject* build_keys(PyObject*, PyObject* args) {
+    PyObject* o = nullptr;
+    int decimals = 0, bits = 0;
+    if (!PyArg_ParseTuple(args, "Oii", &o, &decimals, &bits)) return nullptr;
+    if (bits < 2 || bits > 8 || decimals < 0 || decimals > 2 || !THPVariable_CheckExact(o)) Py_RETURN_NONE;
+    HANDLE_TH_ERRORS
+    const at::Tensor& x = THPVariable_Unpack(o);
+    const int code = dtype_code(x.scalar_type());
+    if (!x.is_cuda() || code < 0 || x.dim() != 2 || x.numel() == 0 || !x.is_contiguous() ||
+        x.device().index() != c10::hip::current_device())
+        Py_RETURN_NONE;
+    const at::Device device = x.device();
+    hipStream_t const st = stream_of(device);
+    if (capturing(st)) Py_RETURN_NONE;
+    const int64_t R = x.size(0), d = x.size(1), chunks = (d + 255) / 256;
+    at::Tensor words = at::detail::empty_cuda({(R + 15) / 16, chunks, bits, 64}, at::kLong, device, std::nullopt);
+    at::Tensor image = at::detail::empty_cuda({R, chunks * 256}, at::kChar, device, std::nullopt);
+    at::Tensor shifts = at::detail::empty_cuda({R}, at::kInt, device, std::nullopt);
+    at::Tensor weights = at::detail::empty_cuda({R, bits}, at::kFloat, device, std::nullopt);
+    int rc = BSI_OK;
+    Py_BEGIN_ALLOW_THREADS
+    rc = lib.build_fixed_keys(x.const_data_ptr(), code, R, d, decimals, bits, static_cast<uint64_t*>(words.data_ptr()),
+                              static_cast<int8_t*>(image.data_ptr()), static_cast<int32_t*>(shifts.data_ptr()),
+                              static_cast<float*>(weights.data_ptr()), st);
+    Py_END_ALLOW_THREADS
+    if (rc != BSI_OK) return fail_status(rc, "bsi_hip_build_fixed_keys");
+    Holder w(THPVariable_Wrap(std::move(words))), i(THPVariable_Wrap(std::move(image))), s(THPVariable_Wrap(std::move(shifts))),
+        f(THPVariable_Wrap(std::move(weights)));
+    return Py_BuildValue("OOOOLL", w.p, i.p, s.p, f.p, static_cast<long long>(R), static_cast<long long>(d));
+    END_HANDLE_TH_ERRORS
+}
+
 // ewah_streams(words [S, W], threshold) -> (stream words, offsets, lengths, flags) of the slices' EWAH encoding, or None.
 PyObject* ewah_streams(PyObject*, PyObject* args) {
     PyObject* o = nullptr;
@@ -792,7 +827,8 @@ PyObject* bind(PyObject*, PyObject* args) {
     if (!PyArg_ParseTuple(args, "O!O!iiiL", &PyDict_Type, &entries, &PyDict_Type, &state, &few, &stream, &split, &lds)) return nullptr;
     if (!entry(entries, "bsi_hip_linear_few_rows_out", &lib.linear_few_rows_out) || !entry(entries, "bsi_hip_linear_out", &lib.linear_out) ||
         !entry(entries, "bsi_hip_linear_workspace_bytes", &lib.linear_workspace_bytes) || !entry(entries, "bsi_hip_dot", &lib.dot) ||
-        !entry(entries, "bsi_hip_build_fixed", &lib.build_fixed) || !entry(entries, "bsi_hip_ewah_measure", &lib.ewah_measure) ||
+        !entry(entries, "bsi_hip_build_fixed", &lib.build_fixed) ||
+        !entry(entries, "bsi_hip_build_fixed_keys", &lib.build_fixed_keys) || !entry(entries, "bsi_hip_ewah_measure", &lib.ewah_measure) ||
         !entry(entries, "bsi_hip_ewah_emit", &lib.ewah_emit) || !entry(entries, "bsi_hip_dot_ewah_batch", &lib.dot_ewah_batch) ||
         !entry(entries, "bsi_hip_dot_ewah_batch_workspace_bytes", &lib.dot_ewah_batch_workspace_bytes) ||
         !entry(entries, "bsi_hip_build_measure", &lib.build_measure) || !entry(entries, "bsi_hip_ewah_emit_at", &lib.ewah_emit_at) ||
@@ -819,6 +855,7 @@ PyMethodDef methods[] = {
     {"configure", configure, METH_VARARGS, nullptr},
     {"build_key", build_key, METH_VARARGS, nullptr},
     {"build", build, METH_VARARGS, nullptr},
+    {"build_keys", build_keys, METH_VARARGS, nullptr},
     {"hybrid", hybrid, METH_VARARGS, nullptr},
     {"ewah_streams", ewah_streams, METH_VARARGS, nullptr},
     {"dot_streams", reinterpret_cast<PyCFunction>(reinterpret_cast<void*>(dot_streams)), METH_FASTCALL, nullptr},

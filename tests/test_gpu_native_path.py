@@ -77,3 +77,20 @@ def test_threads_on_one_stream(ops):
     [t.start() for t in threads]
     [t.join() for t in threads]
     assert not wrong
+
+
+@pytest.mark.parametrize("rows,d,dtype", [(1, 64, torch.float32), (33, 300, torch.bfloat16), (64, 8192, torch.float16)])
+def test_key_build_matches_the_python_path(ops, rows, d, dtype):
+    from bsipytorch_amd import _native
+
+    torch.manual_seed(5)
+    K = (torch.randn(rows, d, device="cuda") * 0.1).to(dtype)
+    column_major = torch.empty(d, rows, dtype=dtype, device="cuda").t().copy_(K)
+    got, want = ops.build_bsi_keys_cuda(torch.nn.Parameter(K), 2, 0.5), ops.build_bsi_keys_cuda(K.double(), 2, 0.5)
+    assert _native.build_keys(K.double(), 2, 6) is None and _native.build_keys(K, 3, 6) is None
+    assert column_major.is_contiguous() or _native.build_keys(column_major, 2, 6) is None
+    assert got[1:] == want[1:]
+    a, b = vars(got[0]), vars(want[0])
+    assert set(a) == set(b) == set(vars(ops.PrebuiltBSIKeysCUDA()))
+    for name in a:
+        assert torch.equal(a[name], b[name]) if torch.is_tensor(a[name]) else a[name] == b[name], name
