@@ -313,7 +313,11 @@ PyObject* linear(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     PyObject* const buffers = get(layer, names._buffers);
     if (buffers == nullptr || !PyDict_Check(buffers)) Py_RETURN_NONE;
     const float* bias = nullptr;
-    if (PyObject* o = get(buffers, names.bias); o != nullptr && o != Py_None) {
+    // A layer without a bias has the buffer, None.  Without the buffer, or with an instance attribute in front of it, self.bias
+    // is something else: a parameter, a parametrization.
+    PyObject* const bias_object = get(buffers, names.bias);
+    if (bias_object == nullptr || get(layer, names.bias) != nullptr) Py_RETURN_NONE;
+    if (PyObject* o = bias_object; o != Py_None) {
         if (!THPVariable_Check(o)) Py_RETURN_NONE;
         const at::Tensor& b = THPVariable_Unpack(o);
         if (b.device() != device || b.scalar_type() != at::kFloat || b.dim() != 1 || b.numel() != k.R || !b.is_contiguous())

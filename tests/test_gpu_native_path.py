@@ -57,6 +57,36 @@ def test_calls_it_leaves_alone(ops):
                                                          layer._bsi_keys_cuda)
 
 
+@pytest.mark.parametrize("rows", [1, 16, 64])
+@pytest.mark.parametrize("how", ["parameter", "parametrization", "attribute"])
+def test_a_bias_that_is_no_buffer_is_added(ops, rows, how):
+    from bsipytorch_amd.linear import BSIQuantizedLinear
+    from torch.nn.utils import parametrize
+
+    torch.manual_seed(6)
+    layer = BSIQuantizedLinear(torch.nn.Linear(512, 96).cuda(), 2, 0.5)
+    x = torch.randn(rows, 512, device="cuda")
+    other = torch.randn(96, device="cuda")
+    with torch.no_grad():
+        for _ in range(2):  # the first call of a shape is the Python path's
+            before = layer(x)
+        if how == "parameter":
+            layer.bias = torch.nn.Parameter(other)
+        elif how == "parametrization":
+            class Other(torch.nn.Module):
+                def forward(self, bias):
+                    return other
+
+            parametrize.register_parametrization(layer, "bias", Other(), unsafe=True)
+        else:
+            layer.__dict__["bias"] = other
+        plain = BSIQuantizedLinear(torch.nn.Linear(512, 96, bias=False).cuda(), 2, 0.5)
+        plain._bsi_keys_cuda = layer._bsi_keys_cuda
+        for _ in range(2):
+            got = layer(x)
+            assert torch.equal(got, plain(x) + other) and not torch.equal(got, before)
+
+
 def test_threads_on_one_stream(ops):
     from bsipytorch_amd.linear import BSIQuantizedLinear
 
