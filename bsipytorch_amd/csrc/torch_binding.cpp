@@ -294,12 +294,11 @@ PyObject* linear(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
         return nullptr;
     }
     PyObject* const layer = args[0];
-    PyObject* x_object = args[1];
-    if (!config.on || !THPVariable_CheckExact(x_object) || !switches_at_default()) Py_RETURN_NONE;
+    if (!config.on || !THPVariable_CheckExact(args[1]) || !switches_at_default()) Py_RETURN_NONE;
     if (PyObject* o = get(layer, names._fused); o != nullptr && o != Py_None) Py_RETURN_NONE;
     if (get(layer, names.collect_stats) != Py_False) Py_RETURN_NONE;
     HANDLE_TH_ERRORS
-    at::Tensor x = THPVariable_Unpack(x_object);
+    at::Tensor x = THPVariable_Unpack(args[1]);
     const int in_code = dtype_code(x.scalar_type());
     if (!x.is_cuda() || x.layout() != at::kStrided || in_code < 0 || x.dim() < 1 || x.numel() == 0) Py_RETURN_NONE;
     const at::Device device = x.device();
@@ -359,13 +358,8 @@ PyObject* linear(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
         }
     }
 
-    Holder owned;  // the object that stands for x when it is not the caller's
     if (x.requires_grad()) x = x.detach();
     if (!x.is_contiguous()) x = x.contiguous();
-    if (&*x.unsafeGetTensorImpl() != THPVariable_Unpack(x_object).unsafeGetTensorImpl() && slot != nullptr) {
-        owned.p = THPVariable_Wrap(x);
-        x_object = owned.p;
-    }
     c10::SmallVector<int64_t, 5> sizes(x.sizes().begin(), x.sizes().end());
     sizes.back() = k.R;
     at::Tensor out = at::detail::empty_cuda(sizes, x.scalar_type(), device, std::nullopt);
@@ -389,30 +383,34 @@ PyObject* linear(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
         Py_END_ALLOW_THREADS
         if (rc != BSI_OK) return fail_status(rc, "bsi_hip_linear_few_rows_out");
     } else {
-        // a call on the tensor the workspace was last built from skips the build, as in bsi_ops.linear_cuda
-        int rebuild = 1;
-        if (x.is_inference()) {
-            Py_INCREF(Py_None);
-            PyList_SetItem(slot, 0, Py_None);
-        } else {
-            const BuildKey key = build_key_of(x, d, decimals, k.Sb);
-            PyObject* const last = PyList_GET_ITEM(slot, 0);
-            if (PyBytes_CheckExact(last) && PyBytes_GET_SIZE(last) == sizeof(key) &&
-                std::memcmp(PyBytes_AS_STRING(last), &key, sizeof(key)) == 0)
-                rebuild = 0;
-            else
-                PyList_SetItem(slot, 0, PyBytes_FromStringAndSize(reinterpret_cast<const char*>(&key), sizeof(key)));
-        }
-        Py_INCREF(x_object);
-        PyList_SetItem(slot, 1, x_object);  // its address is not reused while the build stands for it
         size_t warm_bytes = 0;
         const void* const warm = keys_to_warm(layer, rows, device, &warm_bytes);
-        // under the interpreter lock: another thread on this stream must not find the slot before the build is enqueued,
-        // nor enqueue a build of its own between the two launches
+        // a call on the tensor the workspace was last built from skips the build, as in bsi_ops.linear_cuda
+        int rebuild = 1;
+        Holder key, held;
+        if (!x.is_inference()) {
+            const BuildKey now = build_key_of(x, d, decimals, k.Sb);
+            PyObject* const last = PyList_GET_ITEM(slot, 0);
+            if (PyBytes_CheckExact(last) && PyBytes_GET_SIZE(last) == sizeof(now) && std::memcmp(PyBytes_AS_STRING(last), &now, sizeof(now)) == 0) {
+                rebuild = 0;
+            } else {
+                key.p = PyBytes_FromStringAndSize(reinterpret_cast<const char*>(&now), sizeof(now));
+                // An alias of its own holds the storage, whatever becomes of the caller's tensor (x.data = other keeps the object
+                // and its version and frees the storage): the address is not reused while the build stands for it.
+                held.p = THPVariable_Wrap(x.detach());
+                if (key.p == nullptr || held.p == nullptr) return nullptr;
+            }
+        }
+        if (rebuild != 0) PyList_SetItem(slot, 0, Py_NewRef(Py_None));  // until the build is enqueued
+        // under the interpreter lock: another thread must not enqueue a build of its own between the two launches
         rc = lib.linear_out(xp, in_code, rows, d, static_cast<int>(decimals), config.bits, rebuild, ws, static_cast<size_t>(ws_bytes),
                             static_cast<const uint64_t*>(operand), layout, k.weights->const_data_ptr<float>(), static_cast<int>(k.Sb),
                             k.R, inv, k.R, bias, out.data_ptr(), in_code, config.core, warm, warm_bytes, st);
         if (rc != BSI_OK) return fail_status(rc, "bsi_hip_linear_out");
+        if (rebuild != 0 && key.p != nullptr) {
+            PyList_SetItem(slot, 0, Py_NewRef(key.p));
+            PyList_SetItem(slot, 1, Py_NewRef(held.p));
+        }
         count(layer, names.build_calls, rebuild);
     }
     count(layer, names.dot_calls, 1);

@@ -87,6 +87,26 @@ def test_a_bias_that_is_no_buffer_is_added(ops, rows, how):
             assert torch.equal(got, plain(x) + other) and not torch.equal(got, before)
 
 
+@pytest.mark.parametrize("rows", [256, 512])
+def test_a_tensor_given_other_storage_is_built_anew(ops, rows):
+    from bsipytorch_amd.linear import BSIQuantizedLinear
+
+    torch.manual_seed(7)
+    d, out = 2048, 8192
+    assert not ops.lib.bsi_hip_linear_coop_serves(rows, d, out, 2, 7, 2, 6)  # build and dot in launches of their own
+    layer = BSIQuantizedLinear(torch.nn.Linear(d, out).cuda(), 2, 0.5)
+    x = torch.randn(rows, d, device="cuda")
+    other = torch.randn(rows, d, device="cuda")
+    with torch.no_grad():
+        want = layer(other).clone()
+        for _ in range(2):  # the first call of a shape is the Python path's
+            layer(x)
+        x.data = torch.empty(0, device="cuda")  # frees the storage; the version stays as it is
+        fresh = torch.empty(rows, d, device="cuda").copy_(other)  # where the freed one was, if nothing holds that
+        x.data = fresh
+        assert torch.equal(layer(x), want)
+
+
 def test_threads_on_one_stream(ops):
     from bsipytorch_amd.linear import BSIQuantizedLinear
 
