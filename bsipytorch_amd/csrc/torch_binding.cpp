@@ -139,10 +139,23 @@ int dtype_code(at::ScalarType t) {
     }
 }
 
+// What a launch reads of a tensor: address and storage, taken under the interpreter lock.  A tensor found in a Python
+// dictionary is only borrowed: once the lock is released (or Python code is called), another thread can put something else in
+// its place, or other data into it.
+struct Operand {
+    c10::Storage storage;
+    const void* data = nullptr;
+    size_t bytes = 0;
+    Operand() = default;
+    explicit Operand(const at::Tensor& t) : storage(t.storage()), data(t.const_data_ptr()), bytes(t.nbytes()) {}
+    template <typename T>
+    const T* as() const { return static_cast<const T*>(data); }
+};
+
 // A fixed-bit keyset's attributes as the dot needs them.
 struct Keys {
     int64_t Sb, W, d, R, decimals, layout;
-    const at::Tensor *words, *ints8, *weights;
+    Operand words, ints8, weights;  // ints8.data is null if there is no image
     bool tiled_image;
 };
 bool read_keys(PyObject* handle, const at::Device& device, Keys* k) {
@@ -156,20 +169,26 @@ bool read_keys(PyObject* handle, const at::Device& device, Keys* k) {
         !get_int(attrs.p, names.d, &k->d) || !get_int(attrs.p, names.num_keys, &k->R) ||
         !get_int(attrs.p, names.decimals, &k->decimals) || !get_int(attrs.p, names.layout, &k->layout))
         return false;
-    k->words = get_tensor(attrs.p, names.words);
-    k->ints8 = get_tensor(attrs.p, names.ints8);
-    k->weights = get_tensor(attrs.p, names.slice_weights);
+    const at::Tensor* const words = get_tensor(attrs.p, names.words);
+    const at::Tensor* const ints8 = get_tensor(attrs.p, names.ints8);
+    const at::Tensor* const weights = get_tensor(attrs.p, names.slice_weights);
     k->tiled_image = get(attrs.p, names.ints8_tiled) == Py_True;
-    return k->words != nullptr && k->weights != nullptr && k->words->device() == device && k->weights->device() == device &&
-           k->weights->is_contiguous() && k->R > 0 && k->Sb >= 2 && k->Sb <= 8;
+    if (words == nullptr || weights == nullptr || words->device() != device || weights->device() != device || !weights->is_contiguous() ||
+        k->R <= 0 || k->Sb < 2 || k->Sb > 8)
+        return false;
+    k->words = Operand(*words);
+    k->weights = Operand(*weights);
+    (void)weights->const_data_ptr<float>();  // raises for another type
+    if (ints8 != nullptr) k->ints8 = Operand(*ints8);
+    return true;
 }
 // What a dot of Q rows reads of the keyset (bsi_ops.key_operand).
 const void* key_operand(const Keys& k, int64_t Q, int* layout, size_t* bytes) {
-    const bool image = k.ints8 != nullptr && Q > shared.stream_max;
-    const at::Tensor& t = image ? *k.ints8 : *k.words;
+    const bool image = k.ints8.data != nullptr && Q > shared.stream_max;
+    const Operand& t = image ? k.ints8 : k.words;
     *layout = image ? (k.tiled_image ? BSI_LAYOUT_INT8_TILED : BSI_LAYOUT_INT8) : static_cast<int>(k.layout);
-    *bytes = t.nbytes();
-    return t.const_data_ptr();
+    *bytes = t.bytes;
+    return t.data;
 }
 
 PyObject* int_tuple(std::initializer_list<int64_t> values) {
@@ -293,7 +312,8 @@ PyObject* linear(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
         PyErr_SetString(PyExc_TypeError, "linear(layer.__dict__, x)");
         return nullptr;
     }
-    PyObject* const layer = args[0];
+    Holder layer_dict(Py_NewRef(args[0]));
+    PyObject* const layer = layer_dict.p;
     if (!config.on || !THPVariable_CheckExact(args[1]) || !switches_at_default()) Py_RETURN_NONE;
     if (PyObject* o = get(layer, names._fused); o != nullptr && o != Py_None) Py_RETURN_NONE;
     if (get(layer, names.collect_stats) != Py_False) Py_RETURN_NONE;
@@ -311,7 +331,7 @@ PyObject* linear(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     const int64_t d = k.d, rows = x.numel() / d, chunks = (k.W + 3) / 4;
     PyObject* const buffers = get(layer, names._buffers);
     if (buffers == nullptr || !PyDict_Check(buffers)) Py_RETURN_NONE;
-    const float* bias = nullptr;
+    Operand bias;
     // A layer without a bias has the buffer, None.  Without the buffer, or with an instance attribute in front of it, self.bias
     // is something else: a parameter, a parametrization.
     PyObject* const bias_object = get(buffers, names.bias);
@@ -321,15 +341,16 @@ PyObject* linear(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
         const at::Tensor& b = THPVariable_Unpack(o);
         if (b.device() != device || b.scalar_type() != at::kFloat || b.dim() != 1 || b.numel() != k.R || !b.is_contiguous())
             Py_RETURN_NONE;
-        bias = b.const_data_ptr<float>();
+        bias = Operand(b);
     }
     // half-precision output: the kernels that have it (bsi_ops.can_output_half)
     const bool six_tiled = k.Sb == 6 && k.layout == BSI_LAYOUT_TILED16;
-    if (in_code != BSI_DTYPE_F32 && !(rows > shared.stream_max ? k.ints8 != nullptr : six_tiled && chunks <= 32768)) Py_RETURN_NONE;
+    if (in_code != BSI_DTYPE_F32 && !(rows > shared.stream_max ? k.ints8.data != nullptr : six_tiled && chunks <= 32768)) Py_RETURN_NONE;
     hipStream_t const st = stream_of(device);
     if (capturing(st)) Py_RETURN_NONE;
 
     const bool few = rows <= shared.few_rows_max && six_tiled && k.W % 4 == 0 && chunks * rows * 260 <= shared.few_rows_lds;
+    Holder mine;  // the stream's (buffer, slot)
     PyObject* slot = nullptr;
     void* ws = nullptr;
     int64_t ws_bytes = 0;
@@ -349,11 +370,11 @@ PyObject* linear(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
         if (coop == nullptr) {
             Holder handle(PyLong_FromVoidPtr(st));
             PyObject* const eager = get(record, names.eager);
-            PyObject* const mine = eager != nullptr ? PyDict_GetItem(eager, handle.p) : nullptr;
-            if (mine == nullptr || !PyTuple_Check(mine) || PyTuple_GET_SIZE(mine) != 2 || !THPVariable_Check(PyTuple_GET_ITEM(mine, 0)))
+            mine.p = Py_XNewRef(eager != nullptr ? PyDict_GetItem(eager, handle.p) : nullptr);
+            if (mine.p == nullptr || !PyTuple_Check(mine.p) || PyTuple_GET_SIZE(mine.p) != 2 || !THPVariable_Check(PyTuple_GET_ITEM(mine.p, 0)))
                 Py_RETURN_NONE;
-            ws = THPVariable_Unpack(PyTuple_GET_ITEM(mine, 0)).data_ptr();
-            slot = PyTuple_GET_ITEM(mine, 1);
+            ws = THPVariable_Unpack(PyTuple_GET_ITEM(mine.p, 0)).data_ptr();
+            slot = PyTuple_GET_ITEM(mine.p, 1);
             if (!PyList_Check(slot) || PyList_GET_SIZE(slot) != 2 || !split_scratch(device.index(), rows, k.R, k.W)) Py_RETURN_NONE;
         }
     }
@@ -364,22 +385,23 @@ PyObject* linear(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     sizes.back() = k.R;
     at::Tensor out = at::detail::empty_cuda(sizes, x.scalar_type(), device, std::nullopt);
     const float inv = scale_inv(decimals, k.decimals);
-    const void* const xp = x.const_data_ptr();
+    const Operand xo(x);
+    const void* const xp = xo.data;
     int rc = BSI_OK;
     if (coop != nullptr) {
         size_t warm_bytes = 0;
         const void* const warm = keys_to_warm(layer, rows, device, &warm_bytes);
         // under the interpreter lock: launches on an area are in the order of their numbers
         rc = lib.linear_coop_out(xp, in_code, rows, d, static_cast<int>(decimals), config.bits, ++coop_launches, coop,
-                                 static_cast<const uint64_t*>(operand), layout, k.weights->const_data_ptr<float>(), static_cast<int>(k.Sb),
-                                 k.R, inv, k.R, bias, out.data_ptr(), in_code, warm, warm_bytes, st);
+                                 static_cast<const uint64_t*>(operand), layout, k.weights.as<float>(), static_cast<int>(k.Sb),
+                                 k.R, inv, k.R, bias.as<float>(), out.data_ptr(), in_code, warm, warm_bytes, st);
         if (rc != BSI_OK) return fail_status(rc, "bsi_hip_linear_coop_out");
         count(layer, names.build_calls, 1);
     } else if (few) {
         Py_BEGIN_ALLOW_THREADS
         rc = lib.linear_few_rows_out(xp, in_code, rows, d, static_cast<int>(decimals), config.bits,
-                                     static_cast<const uint64_t*>(k.words->const_data_ptr()), k.weights->const_data_ptr<float>(),
-                                     static_cast<int>(k.Sb), k.R, inv, k.R, bias, out.data_ptr(), in_code, st);
+                                     k.words.as<uint64_t>(), k.weights.as<float>(), static_cast<int>(k.Sb), k.R, inv, k.R,
+                                     bias.as<float>(), out.data_ptr(), in_code, st);
         Py_END_ALLOW_THREADS
         if (rc != BSI_OK) return fail_status(rc, "bsi_hip_linear_few_rows_out");
     } else {
@@ -404,8 +426,8 @@ PyObject* linear(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
         if (rebuild != 0) PyList_SetItem(slot, 0, Py_NewRef(Py_None));  // until the build is enqueued
         // under the interpreter lock: another thread must not enqueue a build of its own between the two launches
         rc = lib.linear_out(xp, in_code, rows, d, static_cast<int>(decimals), config.bits, rebuild, ws, static_cast<size_t>(ws_bytes),
-                            static_cast<const uint64_t*>(operand), layout, k.weights->const_data_ptr<float>(), static_cast<int>(k.Sb),
-                            k.R, inv, k.R, bias, out.data_ptr(), in_code, config.core, warm, warm_bytes, st);
+                            static_cast<const uint64_t*>(operand), layout, k.weights.as<float>(), static_cast<int>(k.Sb),
+                            k.R, inv, k.R, bias.as<float>(), out.data_ptr(), in_code, config.core, warm, warm_bytes, st);
         if (rc != BSI_OK) return fail_status(rc, "bsi_hip_linear_out");
         if (rebuild != 0 && key.p != nullptr) {
             PyList_SetItem(slot, 0, Py_NewRef(key.p));
@@ -502,15 +524,16 @@ PyObject* dot(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     if (chunked ? (scales->dim() != 2 || scales->size(0) != Q || W % 4 != 0 || scales->size(1) != chunks) : scales->numel() != Q)
         Py_RETURN_NONE;
     hipStream_t const st = stream_of(device);
+    const Operand planes(*words), image(*ints8), factors(*scales);
     if (capturing(st) || !split_scratch(device.index(), Q, k.R, W)) Py_RETURN_NONE;
     at::Tensor out = at::detail::empty_cuda({Q, k.R}, at::kFloat, device, std::nullopt);
     int layout = 0, rc = BSI_OK;
     size_t bytes = 0;
     const void* const operand = key_operand(k, Q, &layout, &bytes);
     Py_BEGIN_ALLOW_THREADS
-    rc = lib.dot(static_cast<const uint64_t*>(words->const_data_ptr()), static_cast<const int8_t*>(ints8->const_data_ptr()),
-                 scales->const_data_ptr<float>(), chunked ? static_cast<int>(chunks) : 1, static_cast<int>(Sa), static_cast<int>(W),
-                 static_cast<const uint64_t*>(operand), layout, k.weights->const_data_ptr<float>(), static_cast<int>(k.Sb), k.R, Q,
+    rc = lib.dot(planes.as<uint64_t>(), image.as<int8_t>(), factors.as<float>(), chunked ? static_cast<int>(chunks) : 1,
+                 static_cast<int>(Sa), static_cast<int>(W), static_cast<const uint64_t*>(operand), layout, k.weights.as<float>(),
+                 static_cast<int>(k.Sb), k.R, Q,
                  scale_inv(decimals, k.decimals), k.R, out.data_ptr<float>(), nullptr, config.core, nullptr, 0, st);
     Py_END_ALLOW_THREADS
     if (rc != BSI_OK) return fail_status(rc, "bsi_hip_dot");
@@ -541,9 +564,10 @@ PyObject* build(PyObject*, PyObject* args) {
     if (image) ints8 = at::detail::empty_cuda({Q, chunks * 256}, at::kChar, device, std::nullopt);
     scales = chunked ? at::detail::empty_cuda({Q, chunks}, at::kFloat, device, std::nullopt)
                      : at::detail::empty_cuda({Q}, at::kFloat, device, std::nullopt);
+    const Operand xo(x);
     int rc = BSI_OK;
     Py_BEGIN_ALLOW_THREADS
-    rc = lib.build_fixed(x.const_data_ptr(), code, Q, d, decimals, config.bits, chunked ? 1 : 0, 0.0f,
+    rc = lib.build_fixed(xo.data, code, Q, d, decimals, config.bits, chunked ? 1 : 0, 0.0f,
                          planes ? static_cast<uint64_t*>(words.data_ptr()) : nullptr, nullptr, static_cast<float*>(scales.data_ptr()),
                          image ? static_cast<int8_t*>(ints8.data_ptr()) : nullptr, st);
     Py_END_ALLOW_THREADS
@@ -574,9 +598,10 @@ PyObject* build_keys(PyObject*, PyObject* args) {
     at::Tensor image = at::detail::empty_cuda({R, chunks * 256}, at::kChar, device, std::nullopt);
     at::Tensor shifts = at::detail::empty_cuda({R}, at::kInt, device, std::nullopt);
     at::Tensor weights = at::detail::empty_cuda({R, bits}, at::kFloat, device, std::nullopt);
+    const Operand xo(x);
     int rc = BSI_OK;
     Py_BEGIN_ALLOW_THREADS
-    rc = lib.build_fixed_keys(x.const_data_ptr(), code, R, d, decimals, bits, static_cast<uint64_t*>(words.data_ptr()),
+    rc = lib.build_fixed_keys(xo.data, code, R, d, decimals, bits, static_cast<uint64_t*>(words.data_ptr()),
                               static_cast<int8_t*>(image.data_ptr()), static_cast<int32_t*>(shifts.data_ptr()),
                               static_cast<float*>(weights.data_ptr()), st);
     Py_END_ALLOW_THREADS
@@ -608,7 +633,8 @@ PyObject* ewah_streams(PyObject*, PyObject* args) {
     at::Tensor total_host = at::detail::empty_cpu({1}, at::kLong, /*pin_memory=*/true);
     volatile int64_t* const total = static_cast<volatile int64_t*>(total_host.data_ptr());
     *total = -1;
-    const uint64_t* const w = static_cast<const uint64_t*>(words.const_data_ptr());
+    const Operand wo(words);
+    const uint64_t* const w = wo.as<uint64_t>();
     int rc = BSI_OK;
     Py_BEGIN_ALLOW_THREADS
     rc = lib.ewah_measure(w, S, W, threshold, static_cast<int32_t*>(flags.data_ptr()), static_cast<int32_t*>(lens.data_ptr()),
@@ -726,6 +752,7 @@ PyObject* dot_streams(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
         scales->numel() != (chunked ? Q * chunks : Q))
         Py_RETURN_NONE;
     hipStream_t const st = stream_of(device);
+    const Operand so(*streams), oo(*off), lo(*len), factors(*scales);
     if (capturing(st) || !split_scratch(device.index(), Q, k.R, W)) Py_RETURN_NONE;
     at::Tensor out = at::detail::empty_cuda({Q, k.R}, at::kFloat, device, std::nullopt);
     const size_t need = lib.dot_ewah_batch_workspace_bytes(Q, static_cast<int>(W));
@@ -734,11 +761,9 @@ PyObject* dot_streams(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     size_t bytes = 0;
     const void* const operand = key_operand(k, Q, &layout, &bytes);
     Py_BEGIN_ALLOW_THREADS
-    rc = lib.dot_ewah_batch(static_cast<const uint64_t*>(streams->const_data_ptr()), static_cast<const int64_t*>(off->const_data_ptr()),
-                            static_cast<const int32_t*>(len->const_data_ptr()), static_cast<int>(Sa), static_cast<int>(W),
-                            static_cast<const float*>(scales->const_data_ptr()), chunked ? static_cast<int>(chunks) : 1,
-                            static_cast<const uint64_t*>(operand), layout, static_cast<const float*>(k.weights->const_data_ptr()),
-                            static_cast<int>(k.Sb), k.R, Q, scale_inv(decimals, k.decimals), k.R, nullptr,
+    rc = lib.dot_ewah_batch(so.as<uint64_t>(), oo.as<int64_t>(), lo.as<int32_t>(), static_cast<int>(Sa), static_cast<int>(W),
+                            factors.as<float>(), chunked ? static_cast<int>(chunks) : 1, static_cast<const uint64_t*>(operand), layout,
+                            k.weights.as<float>(), static_cast<int>(k.Sb), k.R, Q, scale_inv(decimals, k.decimals), k.R, nullptr,
                             static_cast<float*>(out.data_ptr()), nullptr, ws.data_ptr(), need, st);
     Py_END_ALLOW_THREADS
     if (rc != BSI_OK) return fail_status(rc, "bsi_hip_dot_ewah_batch");
@@ -774,12 +799,12 @@ PyObject* scalar_query(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     at::Tensor out = at::detail::empty_cpu({R}, at::kDouble);
     at::Tensor pinned = at::detail::empty_cpu({lib.scalar_query_host_words(R)}, at::kLong, /*pin_memory=*/true);
     int64_t info[4] = {0, 0, 0, 0}, build_ns = 0, dot_ns = 0;
+    const Operand xo(x), wo(words), fo(weights);
+    const int slices = static_cast<int>(words.size(1));
     int rc = BSI_OK;
     Py_BEGIN_ALLOW_THREADS
-    rc = lib.scalar_query_dot(x.const_data_ptr<float>(), d, static_cast<int>(decimals), threshold,
-                              static_cast<const uint64_t*>(words.const_data_ptr()), weights.const_data_ptr<float>(),
-                              static_cast<int>(words.size(1)), R, divisor, static_cast<uint64_t*>(pinned.data_ptr()),
-                              out.data_ptr<double>(), info, &build_ns, &dot_ns, st);
+    rc = lib.scalar_query_dot(xo.as<float>(), d, static_cast<int>(decimals), threshold, wo.as<uint64_t>(), fo.as<float>(), slices, R,
+                              divisor, static_cast<uint64_t*>(pinned.data_ptr()), out.data_ptr<double>(), info, &build_ns, &dot_ns, st);
     Py_END_ALLOW_THREADS
     if (rc != BSI_OK) return fail_status(rc, "bsi_hip_scalar_query_dot");
     Holder scores(THPVariable_Wrap(std::move(out)));

@@ -129,6 +129,40 @@ def test_threads_on_one_stream(ops):
     assert not wrong
 
 
+def test_operands_replaced_by_another_thread(ops):
+    from bsipytorch_amd.linear import BSIQuantizedLinear
+
+    torch.manual_seed(8)
+    layer = BSIQuantizedLinear(torch.nn.Linear(512, 256).cuda(), 2, 0.5)
+    kept = layer._bsi_keys_cuda
+    xs = [torch.randn(rows, 512, device="cuda") for rows in (1, 16, 512)]
+    batch, streams = ops.build_bsi_queries_cuda_batch_packed(xs[1], 2), ops.build_bsi_queries_cuda_batch_hybrid(xs[1], 2)
+
+    def results():
+        dots = [ops.batch_dot_product_multiquery_cuda_batch_caps(q, layer._bsi_keys_cuda)[0] for q in (batch, streams)]
+        return [layer(x) for x in xs] + dots
+
+    done = threading.Event()
+
+    def replace():
+        owners = [kept, batch, streams]
+        tensors = [{n: t for n, t in vars(o).items() if torch.is_tensor(t)} for o in owners]
+        while not done.is_set():
+            for owner, named in zip(owners, tensors):
+                vars(owner).update({n: t.clone() for n, t in named.items()})
+
+    with torch.no_grad():
+        want = results()
+        thread = threading.Thread(target=replace)
+        thread.start()
+        try:
+            for _ in range(300):
+                assert all(torch.equal(a, b) for a, b in zip(results(), want))
+        finally:
+            done.set()
+            thread.join()
+
+
 @pytest.mark.parametrize("rows,d,dtype", [(1, 64, torch.float32), (33, 300, torch.bfloat16), (64, 8192, torch.float16)])
 def test_key_build_matches_the_python_path(ops, rows, d, dtype):
     from bsipytorch_amd import _native
