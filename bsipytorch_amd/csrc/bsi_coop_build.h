@@ -9,6 +9,20 @@
 // No workgroup depends on another one being resident.  A share's bytes do not depend on who builds it, so a workgroup that
 // has waited kCoopPatience for a share builds it itself.  Flags hold the launch's number, which no other launch has: nothing
 // is cleared between launches, and flags of earlier ones mean nothing.
+//
+// What a reader relies on, since neither side of a flag is more than a relaxed access (an agent-scope release writes the L2
+// back: the flags come 1 to 2 us later; an agent-scope acquire also drops L2 lines: 16 x 4096 x 4096 7.4 -> 8.8 us, 15 x 2560
+// x 5888 7.3 -> 9.5):
+//  - A store is complete (vmcnt) when the XCD's L2 has it, and a copy is written and read by workgroups of its own XCD only:
+//    the index is XCC_ID, in the build and in the reads.
+//  - No L1 holds a line of a copy that another CU has written in this launch.  L1s and scalar caches are invalidated when a
+//    kernel starts, as every kernel that reads what an earlier one wrote needs; and within the launch nothing loads from a copy
+//    before all its flags are there, so that the first load of a line fetches it from the L2.  That is why coop_build hands
+//    out the copy's address only when it returns, and why ahead() must not load from `area`: a load there would compile and
+//    read right most of the time.
+//  - Flags are read past the L1 (agent scope) and share no line with a copy; a copy's lines belong to it alone.  Lines of the
+//    scales are written by several CUs, four bytes each: an L1 writes through and answers with no byte of a line that it
+//    has not fetched or written itself.
 // Inside a launch the build is over 2.5 us after the first wave (16 rows of 4096: 1.5 until a wave has its chunk and has
 // quantised it, 0.3 to the flag, 0.5 to the last share): as long as the launch it replaces, but for the host.
 #pragma once
@@ -22,6 +36,7 @@ constexpr int kCoopMaxItems = 1024;   // (row, chunk) items: 256 bytes of image 
 constexpr size_t kCoopFlagBytes = kXcds * kCoopShares * sizeof(unsigned long long);
 constexpr size_t kCoopCopyBytes = static_cast<size_t>(kCoopMaxItems) * (BSI_CHUNK_ELEMS + sizeof(float));
 constexpr size_t kCoopBytes = kCoopFlagBytes + kXcds * kCoopCopyBytes;
+static_assert(kCoopFlagBytes % 128 == 0 && kCoopCopyBytes % 128 == 0, "flags and copies share no cache line");
 constexpr int kCoopPatience = 2000;  // ticks of the 100 MHz clock: 20 us
 
 struct CoopBuild {
@@ -128,9 +143,9 @@ __device__ void coop_build_share(const CoopBuild& b, int share, int wave, int nw
 }
 
 // Called by all waves of the workgroup (number `id` of the grid); 32 words of LDS at `shared`.  On return A8 and qscale point
-// to the whole build, in the copy of the XCD the workgroup runs on.  ahead(): loads for after the build.  Every wave but wave 0
-// issues them when the workgroup's share is built (a CU's loads return in order: not before), wave 0, which asks for the
-// flags, when all shares are.
+// to the whole build, in the copy of the XCD the workgroup runs on.  ahead(): loads for after the build, of anything but the
+// area.  Every wave but wave 0 issues them when the workgroup's share is built (a CU's loads return in order: not before),
+// wave 0, which asks for the flags, when all shares are.
 template <typename F>
 __device__ __forceinline__ void coop_build(const CoopBuild& b, unsigned id, unsigned* __restrict__ shared, const int8_t*& A8,
                                            const float*& qscale, F&& ahead) {
