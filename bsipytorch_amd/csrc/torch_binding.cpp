@@ -289,17 +289,30 @@ const void* keys_to_warm(PyObject* layer, int64_t rows, const at::Device& device
     return read_keys(handle, device, &k) ? key_operand(k, rows, &layout, bytes) : nullptr;
 }
 
-// The area of launches with the query build inside, one for each stream that has made one (at most kCoopAreas; other streams
-// take the two-launch path), until forget().  Under the interpreter lock.
+// The areas of launches with the query build inside (2.1 MB each), one for each stream that has made one.  A stream without an
+// area takes the ones that no launch has used for kCoopIdle launches back and gets one if fewer than kCoopAreas are left;
+// otherwise its layers are two launches, so that streams in turn do not clear an area a call.  forget() gives all back.  An area
+// is allocated under its stream, so the allocator reuses it behind the launches on it.  Under the interpreter lock.
 constexpr size_t kCoopAreas = 32;
-std::map<std::pair<int, hipStream_t>, at::Tensor> coop_areas;
+constexpr uint64_t kCoopIdle = 4096;
+struct CoopArea {
+    at::Tensor memory;
+    uint64_t last;  // the last launch that used it
+};
+auto& coop_areas = *new std::map<std::pair<int, hipStream_t>, CoopArea>;  // never destroyed: the runtime may be gone by then
 uint64_t coop_launches = 0;
-void* coop_area(const at::Device& device, hipStream_t st) {
-    const auto found = coop_areas.find({device.index(), st});
-    if (found != coop_areas.end()) return found->second.data_ptr();
-    if (coop_areas.size() >= kCoopAreas) return nullptr;
-    at::Tensor area = at::zeros({static_cast<int64_t>(lib.linear_coop_bytes())}, at::TensorOptions().dtype(at::kByte).device(device));
-    return coop_areas.emplace(std::make_pair(device.index(), st), std::move(area)).first->second.data_ptr();
+at::Tensor coop_area(const at::Device& device, hipStream_t st) {
+    const std::pair<int, hipStream_t> key(device.index(), st);
+    auto found = coop_areas.find(key);
+    if (found == coop_areas.end()) {
+        for (auto it = coop_areas.begin(); it != coop_areas.end();)
+            it = coop_launches - it->second.last > kCoopIdle ? coop_areas.erase(it) : std::next(it);
+        if (coop_areas.size() >= kCoopAreas) return at::Tensor();
+        at::Tensor memory = at::zeros({static_cast<int64_t>(lib.linear_coop_bytes())}, at::TensorOptions().dtype(at::kByte).device(device));
+        found = coop_areas.emplace(key, CoopArea{std::move(memory), 0}).first;
+    }
+    found->second.last = coop_launches;
+    return found->second.memory;
 }
 PyObject* forget(PyObject*, PyObject*) {
     coop_areas.clear();
@@ -357,8 +370,8 @@ PyObject* linear(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     int layout = 0;
     size_t bytes = 0;
     const void* const operand = key_operand(k, rows, &layout, &bytes);
-    void* const coop = !few && k.Sb <= 8 && lib.linear_coop_serves(rows, d, k.R, static_cast<int>(decimals), config.bits, layout, static_cast<int>(k.Sb))
-                           ? coop_area(device, st) : nullptr;
+    const at::Tensor coop = !few && k.Sb <= 8 && lib.linear_coop_serves(rows, d, k.R, static_cast<int>(decimals), config.bits, layout, static_cast<int>(k.Sb))
+                           ? coop_area(device, st) : at::Tensor();
     if (few) {
         if (!known_few_rows(device.index(), rows, d)) Py_RETURN_NONE;
     } else {
@@ -367,7 +380,7 @@ PyObject* linear(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
         if (record == nullptr || !get_int(record, names.bytes, &ws_bytes) ||
             static_cast<size_t>(ws_bytes) < lib.linear_workspace_bytes(rows, d, config.bits))
             Py_RETURN_NONE;
-        if (coop == nullptr) {
+        if (!coop.defined()) {
             Holder handle(PyLong_FromVoidPtr(st));
             PyObject* const eager = get(record, names.eager);
             mine.p = Py_XNewRef(eager != nullptr ? PyDict_GetItem(eager, handle.p) : nullptr);
@@ -388,11 +401,11 @@ PyObject* linear(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     const Operand xo(x);
     const void* const xp = xo.data;
     int rc = BSI_OK;
-    if (coop != nullptr) {
+    if (coop.defined()) {
         size_t warm_bytes = 0;
         const void* const warm = keys_to_warm(layer, rows, device, &warm_bytes);
         // under the interpreter lock: launches on an area are in the order of their numbers
-        rc = lib.linear_coop_out(xp, in_code, rows, d, static_cast<int>(decimals), config.bits, ++coop_launches, coop,
+        rc = lib.linear_coop_out(xp, in_code, rows, d, static_cast<int>(decimals), config.bits, ++coop_launches, coop.data_ptr(),
                                  static_cast<const uint64_t*>(operand), layout, k.weights.as<float>(), static_cast<int>(k.Sb),
                                  k.R, inv, k.R, bias.as<float>(), out.data_ptr(), in_code, warm, warm_bytes, st);
         if (rc != BSI_OK) return fail_status(rc, "bsi_hip_linear_coop_out");

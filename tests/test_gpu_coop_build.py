@@ -59,3 +59,39 @@ def test_streams_side_by_side(ops):
                     got.append(layer(x.clone()))
             torch.cuda.synchronize()
             assert all(torch.equal(a, b) for a, b in zip(got, want))
+
+
+def test_areas_are_bounded_and_given_back(ops):
+    """33 streams for 32 areas: the one without runs its layers in two launches, until areas have been idle for 4096 launches."""
+    from bsipytorch_amd.linear import BSIQuantizedLinear
+
+    area = ops.lib.bsi_hip_linear_coop_bytes()
+    layer = BSIQuantizedLinear(torch.nn.Linear(1024, 2048).cuda(), 2, 0.5)
+    x = torch.randn(16, 1024, device="cuda")
+    streams = [torch.cuda.default_stream()] + [torch.cuda.Stream() for _ in range(32)]
+    assert len({s.cuda_stream for s in streams}) == 33
+
+    def on(stream):
+        with torch.cuda.stream(stream):
+            got = layer(x)
+        stream.synchronize()
+        return got
+
+    with torch.no_grad():
+        ops.linear_cuda_forget()
+        want = layer(x)
+        for _ in range(2):
+            assert all(torch.equal(on(s), want) for s in streams)
+        held = torch.cuda.memory_allocated()
+        assert held >= 32 * area
+        on(streams[-1])
+        assert torch.cuda.memory_allocated() < held + area
+        with torch.cuda.stream(streams[5]):
+            for _ in range(4200):
+                layer(x)
+        assert torch.cuda.memory_allocated() > held - area  # nothing is taken back before another stream asks
+        assert torch.equal(on(streams[-1]), want)
+        assert torch.cuda.memory_allocated() < held - 29 * area
+        assert all(torch.equal(on(s), want) for s in streams)
+    ops.linear_cuda_forget()
+    assert torch.cuda.memory_allocated() < held - 30 * area
