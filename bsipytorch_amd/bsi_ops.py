@@ -28,7 +28,8 @@ from typing import List, Optional
 
 import torch
 
-from . import _lib, _native
+from . import _lib
+from ._host import native as _native
 from ._lib import check, lib
 
 # --------------------------------------------------------------------------- flags
@@ -601,13 +602,31 @@ def build_bsi_query_cuda(q: torch.Tensor, decimal_places: int, compress_threshol
 def ewah_compress_slices(words2d: torch.Tensor, compress_threshold: float):
     """Density flags and stream lengths, their exclusive scan, and the emit pass for ``[S, W]`` words
     (bsi_vector_cuda.cpp:896-951); the host waits for the total length only.  Returns (comp_words, comp_off int64 [S], comp_len int32 [S], flags)."""
-    if words2d.shape[0] == 0:
-        none = torch.empty((0,), dtype=torch.int64, device=words2d.device)
+    S, W = words2d.shape
+    dev = words2d.device
+    if S == 0:
+        none = torch.empty((0,), dtype=torch.int64, device=dev)
         return none, none.clone(), none.to(torch.int32), none.to(torch.int32)
-    streams = _native.ewah_streams(words2d.contiguous(), float(compress_threshold))
-    _check(streams is not None, "ewah_compress_slices: the words must be int64 on the current device, outside a graph capture "
-                                "(the total length is read back)")
-    return streams
+    words2d = words2d.contiguous()
+    streams = _native.ewah_streams(words2d, float(compress_threshold))  # None: a call it does not serve
+    if streams is not None:
+        return streams
+    _check(words2d.is_cuda and words2d.element_size() == 8 and dev.index == torch.cuda.current_device() and not _capturing(),
+           "ewah_compress_slices: the words must be 64-bit, on the current device, outside a graph capture (the total length is "
+           "read back)")
+    st = _stream()
+    flags = torch.empty((S,), dtype=torch.int32, device=dev)
+    comp_len = torch.empty((S,), dtype=torch.int32, device=dev)
+    comp_off = torch.empty((S,), dtype=torch.int64, device=dev)
+    total = torch.empty((1,), dtype=torch.int64, pin_memory=True)
+    check(lib.bsi_hip_ewah_measure(words2d.data_ptr(), S, W, float(compress_threshold), flags.data_ptr(), comp_len.data_ptr(),
+                                   comp_off.data_ptr(), total.data_ptr(), st), "bsi_hip_ewah_measure")
+    torch.cuda.current_stream().synchronize()
+    comp_words = torch.empty((int(total),), dtype=torch.int64, device=dev)
+    if comp_words.numel() > 0:
+        check(lib.bsi_hip_ewah_emit(words2d.data_ptr(), S, W, flags.data_ptr(), comp_off.data_ptr(), comp_words.data_ptr(),
+                                    comp_len.data_ptr(), st), "bsi_hip_ewah_emit")
+    return comp_words, comp_off, comp_len, flags
 
 
 def build_bsi_query_cuda_hybrid(q: torch.Tensor, decimal_places: int, compress_threshold: float = 0.2):

@@ -19,7 +19,8 @@ from typing import Tuple
 import numpy as np
 import torch
 
-from . import _lib, _native
+from . import _lib
+from ._host import native as _native
 from ._lib import check, lib
 
 _SCALAR_MAX_ELEMS = lib.bsi_hip_scalar_query_max_elems()

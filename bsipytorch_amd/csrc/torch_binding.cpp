@@ -7,6 +7,7 @@
 // path behind them then serves it or raises its errors.  Launches recorded into a graph always take that path.
 #include <torch/csrc/autograd/python_variable.h>
 #include <torch/csrc/jit/frontend/tracer.h>
+#include <torch/version.h>
 #include <ATen/EmptyTensor.h>
 #include <ATen/ops/zeros.h>
 #include <ATen/hip/EmptyTensor.h>
@@ -911,7 +912,23 @@ PyModuleDef definition = {PyModuleDef_HEAD_INIT, "_native", "Host path of eager 
 
 }  // namespace
 
+// The functions reach into torch's own classes: another torch than the one they were compiled against is refused.
+static bool torch_fits() {
+    Holder torch(PyImport_ImportModule("torch"));
+    Holder version(torch.p != nullptr ? PyObject_GetAttrString(torch.p, "__version__") : nullptr);
+    const char* const have = version.p != nullptr && PyUnicode_Check(version.p) ? PyUnicode_AsUTF8(version.p) : nullptr;
+    if (have == nullptr) {
+        if (!PyErr_Occurred()) PyErr_SetString(PyExc_ImportError, "torch has no version");
+        return false;
+    }
+    const size_t n = std::strlen(TORCH_VERSION);
+    if (std::strncmp(have, TORCH_VERSION, n) == 0 && (have[n] == '\0' || have[n] == '+')) return true;
+    PyErr_Format(PyExc_ImportError, "built for torch %s, this is %s", TORCH_VERSION, have);
+    return false;
+}
+
 PyMODINIT_FUNC PyInit__native() {
+    if (!torch_fits()) return nullptr;
 #define X(n) names.n = PyUnicode_InternFromString(#n);
     NAMES(X)
 #undef X

@@ -15,7 +15,8 @@ from typing import Any, Dict, List, Union
 import torch
 import torch.nn as nn
 
-from . import _native, bsi_ops
+from . import bsi_ops
+from ._host import native as _native
 
 
 # Layers fed by the same activation tensor (q_proj / k_proj / v_proj) share one query build: the last built
