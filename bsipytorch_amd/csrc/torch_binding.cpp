@@ -463,6 +463,8 @@ bool plain_call(PyObject* self) {
     if (module.base == nullptr || reinterpret_cast<PyObject*>(type) != module.type || _PyType_Lookup(type, names.forward) != module.forward ||
         _PyType_Lookup(reinterpret_cast<PyTypeObject*>(module.base), names.__call__) != module.call || torch::jit::tracer::isTracing())
         return false;
+    // a profiler or debugger of Python frames sees a module by its __call__ and forward
+    if (const PyThreadState* const thread = PyThreadState_Get(); thread->c_profilefunc != nullptr || thread->c_tracefunc != nullptr) return false;
     for (PyObject* hooks : module.global_hooks)
         if (PyDict_GET_SIZE(hooks) != 0) return false;
     PyObject** const slot = _PyObject_GetDictPtr(self);

@@ -45,3 +45,25 @@ def test_whatever_hangs_on_a_call_is_honoured(ops, rows):
         assert torch.equal(layer(x), want) and len(calls) == 1
     with pytest.raises(TypeError):
         layer(x, x)
+
+
+def test_a_profiler_sees_the_modules(ops, tmp_path):
+    import sys
+
+    from bsipytorch_amd.linear import BSIQuantizedLinear
+
+    layer = BSIQuantizedLinear(torch.nn.Linear(512, 96).cuda(), 2, 0.5)
+    x = torch.randn(16, 512, device="cuda")
+    with torch.no_grad():
+        want = layer(x)
+        frames = []
+        sys.setprofile(lambda frame, event, arg: frames.append(frame.f_code) if event == "call" else None)
+        try:
+            got = layer(x)
+        finally:
+            sys.setprofile(None)
+        assert torch.equal(got, want) and BSIQuantizedLinear.forward.__code__ in frames
+        with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CPU], with_stack=True) as profile:
+            layer(x)
+    profile.export_chrome_trace(str(tmp_path / "trace.json"))
+    assert "nn.Module: BSIQuantizedLinear" in (tmp_path / "trace.json").read_text()
