@@ -9,6 +9,10 @@ import warnings
 
 import torch
 
+# torch.compile leaves a graph at a BSI layer, which runs as it does eagerly (one break a layer; its launches are no operators
+# that a graph could hold).  Dynamo's advice to report the builtin it breaks at is of no use to anybody.
+warnings.filterwarnings("ignore", message=r"Dynamo does not know how to trace the builtin `bsipytorch_amd\._native\.")
+
 
 class PythonPath:
     """``_native``'s functions for a process without it: every call is left to the Python path."""

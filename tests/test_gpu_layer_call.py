@@ -67,3 +67,33 @@ def test_a_profiler_sees_the_modules(ops, tmp_path):
             layer(x)
     profile.export_chrome_trace(str(tmp_path / "trace.json"))
     assert "nn.Module: BSIQuantizedLinear" in (tmp_path / "trace.json").read_text()
+
+def test_compiled_models_break_at_the_layer_without_a_warning(ops):
+    """torch.compile of a model with such a layer: the layer runs as it does eagerly, between the graphs."""
+    import os
+    import subprocess
+    import sys
+
+    code = """
+import torch
+from bsipytorch_amd.linear import BSIQuantizedLinear
+class Model(torch.nn.Module):
+    def __init__(self):
+        super().__init__()
+        self.a, self.b = (BSIQuantizedLinear(torch.nn.Linear(512, n).cuda(), 2, 0.5) for n in (512, 96))
+    def forward(self, x):
+        return self.b(torch.relu(self.a(x * 2))) * 3
+model = Model()
+for rows in (1, 16, 64):
+    x = torch.randn(rows, 512, device="cuda")
+    with torch.no_grad():
+        want = model(x)
+        torch._dynamo.reset()
+        compiled = torch.compile(model, backend="eager")
+        assert all(torch.equal(compiled(x), want) for _ in range(3))
+print("same")
+"""
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    run = subprocess.run([sys.executable, "-c", code], cwd=root, capture_output=True, text=True, timeout=100)
+    assert run.returncode == 0 and "same" in run.stdout, run.stderr
+    assert "Dynamo does not know how to trace" not in run.stderr, run.stderr
