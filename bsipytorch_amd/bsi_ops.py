@@ -1333,7 +1333,8 @@ def linear_cuda(x2d: torch.Tensor, keyset_cuda_cap, decimal_places: int, bias=No
         # of what a recorded launch may reuse (a second capture starting on the same static input builds anew)
         key = (key, capture_id())
     rebuild = 0 if (key is not None and slot[0] == key) else 1
-    slot[0], slot[1] = key, x2d  # holds the input, so that its address is not reused while the build stands for it
+    if rebuild:
+        slot[0] = None  # until the build is enqueued
     wsptr = buf.data_ptr()
     out = torch.empty((Q, R), dtype=out_dtype, device=x2d.device)
     core = f["core"]
@@ -1346,6 +1347,8 @@ def linear_cuda(x2d: torch.Tensor, keyset_cuda_cap, decimal_places: int, bias=No
                              kptr, klayout, keys.slice_weights.data_ptr(), keys.Sb, R,
                              _scale_inv(int(decimal_places), keys.decimals), R, _ptr(bias), out.data_ptr(), _dtype_code(out), core,
                                  wptr, wbytes, st), "bsi_hip_linear_out")
+    if rebuild:
+        slot[0], slot[1] = key, x2d  # holds the input, so that its address is not reused while the build stands for it
     _last_linear_rebuilt[0] = bool(rebuild)
     return out
 

@@ -295,3 +295,17 @@ def test_a_second_capture_on_the_same_static_input_builds_anew(ops, fuse):
         for a, b, want in zip(out1, out2, want0):
             assert torch.equal(a, want) and torch.equal(b, want)
     linear.forget_shared_builds()
+
+
+def test_a_launch_that_failed_leaves_no_build_behind(ops, monkeypatch):
+    """linear_cuda: the workspace is not taken for the build of a tensor whose launch was refused."""
+    torch.manual_seed(12)
+    keys = ops.build_bsi_keys_cuda(torch.randn(256, 512, device="cuda") * 0.1, 2, 0.5)[0]
+    x, other = torch.randn(64, 512, device="cuda"), torch.randn(64, 512, device="cuda")
+    want = ops.linear_cuda(x, keys, 2).clone()
+    ops.linear_cuda(other, keys, 2)
+    with monkeypatch.context() as m:
+        m.setattr(ops.lib, "bsi_hip_linear_out", lambda *args: 2)
+        with pytest.raises(RuntimeError):
+            ops.linear_cuda(x, keys, 2)
+    assert torch.equal(ops.linear_cuda(x, keys, 2), want)
