@@ -710,6 +710,14 @@ PyObject* hybrid(PyObject*, PyObject* args) {
                            static_cast<float*>(scales.data_ptr()), chunked ? nullptr : static_cast<float*>(weights.data_ptr()),
                            static_cast<int32_t*>(flags.data_ptr()), static_cast<int32_t*>(lens.data_ptr()), const_cast<int32_t*>(host), st);
     if (rc != BSI_OK) return fail_status(rc, "bsi_hip_build_measure");
+    // The kernel writes into `pinned` until the last length is there: an allocation that fails before that waits for it.
+    struct Writing {
+        hipStream_t stream;
+        bool done;
+        ~Writing() {
+            if (!done) (void)hipStreamSynchronize(stream);
+        }
+    } writing{st, false};
     // what can be made before the lengths are here
     at::Tensor off = at::detail::empty_cuda({S}, at::kLong, device, std::nullopt);
     Holder b(THPVariable_Wrap(off)), c(THPVariable_Wrap(lens)), f(THPVariable_Wrap(flags)), s(THPVariable_Wrap(std::move(scales))),
@@ -727,6 +735,7 @@ PyObject* hybrid(PyObject*, PyObject* args) {
         total += host[s];
     }
     Py_END_ALLOW_THREADS
+    writing.done = true;
     if (rc != BSI_OK) return fail_status(rc, "bsi_hip_build_measure");
     at::Tensor streams = at::detail::empty_cuda({total}, at::kLong, device, std::nullopt);
     rc = lib.ewah_emit_at(w, static_cast<int>(S), static_cast<int>(W), static_cast<const int32_t*>(flags.data_ptr()),
