@@ -320,6 +320,12 @@ PyObject* forget(PyObject*, PyObject*) {
     Py_RETURN_NONE;
 }
 
+// A Python object that owns a storage.
+PyObject* hold(const c10::Storage& storage) {
+    return PyCapsule_New(new c10::Storage(storage), nullptr,
+                         [](PyObject* o) { delete static_cast<c10::Storage*>(PyCapsule_GetPointer(o, nullptr)); });
+}
+
 // linear(layer.__dict__, x) -> the layer's output, or None.
 PyObject* linear(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     if (nargs != 2 || !PyDict_Check(args[0])) {
@@ -431,9 +437,9 @@ PyObject* linear(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
                 rebuild = 0;
             } else {
                 key.p = PyBytes_FromStringAndSize(reinterpret_cast<const char*>(&now), sizeof(now));
-                // An alias of its own holds the storage, whatever becomes of the caller's tensor (x.data = other keeps the object
-                // and its version and frees the storage): the address is not reused while the build stands for it.
-                held.p = THPVariable_Wrap(x.detach());
+                // The storage is held, not the caller's tensor (x.data = other keeps the object and its version and frees the
+                // storage): the address is not reused while the build stands for it.
+                held.p = hold(xo.storage);
                 if (key.p == nullptr || held.p == nullptr) return nullptr;
             }
         }
