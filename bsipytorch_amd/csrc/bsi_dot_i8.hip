@@ -916,7 +916,8 @@ __global__ __launch_bounds__((I8Cfg<TM, TN>::kBlock)) void dot_mfma_i8_kernel(
 // workgroup starts) only the issue of the stores is left.  Same waves, ring, k-steps and chain, so the same bits.
 // us before and after: 4096 x 4096 x 16384 312, 294; 2048 x 2048 x 8192 47.1, 43.6; 2772 x 512 x 12800 46.7, 40.2;
 // 8192 x 1024 x 4096 58.1, 51.8; 1773 x 5376 x 8704 90.5, 88.3.  What is left at long rows is the chunk loop at the clock the
-// chip holds (1.7 GHz under this load): hiding the rest lowers it a little further.
+// chip holds: the launch takes 557 k cycles, 262 k of them with the matrix pipes busy, at 1.9 GHz for the first twenty launches from
+// an idle GPU (292 us) and at 1.7 to 1.8 after that (310 to 330); hiding the rest lowers the clock a little further.
 template <int TM, int TN>
 struct I8TilesCfg : I8Cfg<TM, TN> {
     using C = I8Cfg<TM, TN>;

@@ -28,7 +28,8 @@ __device__ __forceinline__ void store_host(unsigned long long* p, unsigned long 
 // slice) instead of rows.
 // Bound by latency and by VALU issue in the slicing and the popcounts; the first key words are requested before the query is
 // built.  Every workgroup building it costs less than the launch of its own, with one busy CU, that the build was before.
-// 2048 elements against 1024 keys: 9.0 + 6.8 us in two launches, 5.3 us in this one.
+// 2048 elements against 1024 keys, by a kernel trace: 9.0 + 6.8 us in two launches, 6.6 us in this one (5.3 from the first
+// workgroup's clock to the last's, 3.1 of them until the query is built).
 template <int kWords>
 __global__ __launch_bounds__(kScalarBlock) void scalar_query_dot_kernel(const float* __restrict__ x, int d, int W, double dec_scale,
                                                                         int narrow, double threshold, const unsigned long long* __restrict__ B,
