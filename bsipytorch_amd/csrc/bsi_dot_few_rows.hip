@@ -3,6 +3,7 @@
 // image pass for larger batches of EWAH queries.
 #include "bsi_dot_internal.h"
 #include "bsi_coop_build.h"
+#include <type_traits>
 
 namespace bsi {
 
@@ -21,14 +22,17 @@ namespace bsi {
 
 constexpr int kStreamLdsInts = 16384;  // at most 64 KiB of chunk accumulators per pass
 
-// kBuild: the queries are quantised by this launch (bsi_coop_build.h); A8 and qscale are not looked at.
+// kBuild: the queries are quantised by this launch (bsi_coop_build.h); A8 and qscale are not looked at.  Only those instances
+// take the build's description: with it the workgroup's size, which lies behind the arguments, is in another cache line of
+// them, and its fetch holds up every wave's first key load.  us, with and without: 16 x 4096 x 16384 12.3, 11.8; 16 x 4096 x
+// 4096 5.25, 5.09; 1 x 4096 x 16384 10.5, 10.2; 1 x 16384 x 4096 11.1, 10.9 (1 x 4096 x 4096 4.06, 4.11).
 template <int NT, int KT, bool kInts, bool kBuild>
 __global__ __launch_bounds__(1024) void dot_mfma_stream_kernel(
     const int8_t* A8, const float* qscale, int qscale_stride,
     const unsigned long long* __restrict__ B64,  // tiled key planes, Sb = 6
     const float* __restrict__ Bw, int chunks, int pass_chunks, int64_t R, int64_t Q, int down_shift, float scale_inv,
     int64_t R_total, float* __restrict__ out, int* __restrict__ chunk_ints, const float* __restrict__ bias, int out_dtype,
-    CoopBuild coop) {
+    std::conditional_t<kBuild, CoopBuild, int> coop) {
     extern __shared__ __attribute__((aligned(16))) int ints[];  // [pass_chunks][KT][NT][16 queries][16 keys]
     constexpr int kSlot = KT * NT * 256;
 
@@ -58,7 +62,7 @@ __global__ __launch_bounds__(1024) void dot_mfma_stream_kernel(
                 kc[k][j] = make_uint2(static_cast<uint32_t>(w), static_cast<uint32_t>(w >> 32));
             }
     };
-    if (kBuild)
+    if constexpr (kBuild)
         coop_build(coop, blockIdx.x, reinterpret_cast<unsigned*>(ints), A8, qscale, [&] { load_keys(wave < pass_chunks ? wave : pass_chunks - 1); });
 
     // the chain lanes: tid <-> (key tile, query tile, query, key), keys fastest so output stores are contiguous
@@ -538,8 +542,8 @@ static void launch_mfma_stream(const int8_t* A8, const float* qscale, int stride
     launch((dot_mfma_stream_kernel<NT, KT, INTS, BUILD>), grid, dim3(waves * 64), lds, st, A8, qscale, stride,                \
            reinterpret_cast<const unsigned long long*>(B), Bw, chunks, pass_chunks, R, Q, down_shift, scale_inv, R_total, out, \
            chunk_ints, bias, t_out_dtype, COOP)
-    if (chunk_ints) BSI_STREAM_GO(true, false, CoopBuild{});
-    else if (t_coop == nullptr) BSI_STREAM_GO(false, false, CoopBuild{});
+    if (chunk_ints) BSI_STREAM_GO(true, false, 0);
+    else if (t_coop == nullptr) BSI_STREAM_GO(false, false, 0);
     else {
         CoopBuild coop = *t_coop;
         coop.shares = coop_shares(grid.x, coop.by_row ? coop.rows : coop.rows * coop.chunks);
