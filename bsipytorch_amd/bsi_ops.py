@@ -1354,7 +1354,8 @@ def linear_cuda(x2d: torch.Tensor, keyset_cuda_cap, decimal_places: int, bias=No
 
 
 def linear_cuda_forget() -> None:
-    """Drop what linear_cuda remembers of its last build (and the input tensor it holds)."""
+    """Drop what linear_cuda remembers of its last build (and the input it holds), and the streams' areas of launches with the
+    build inside."""
     for ws in _linear_ws.values():
         ws["capture"] = [None, None]
         for _, slot in ws["eager"].values():

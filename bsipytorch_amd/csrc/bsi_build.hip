@@ -1,11 +1,12 @@
 // BSI builder for gfx950: float -> rounded decimal ints -> block-floating shift -> fixed-bit
 // two's-complement values -> bit-planes in canonical [rows, slices, W64] words.
 //
-// wave64 mapping: one wavefront owns one 256-element chunk of one row.  A lane loads elements
-// lane, lane+64, lane+128, lane+192 of the chunk (four fully coalesced 256-byte wave loads), the
-// chunk maximum is a butterfly reduction across the wave, and one 64-bit `__ballot` per slice per
-// load IS the packed plane word (no lo/hi merge, no LDS, no block barrier).  The chunk-scale
-// build is therefore a single pass over the activations.
+// wave64 mapping of the general kernels: one wavefront owns one 256-element chunk of one row.  A lane
+// loads elements lane, lane+64, lane+128, lane+192 of the chunk (four fully coalesced 256-byte wave
+// loads), the chunk maximum is a butterfly reduction across the wave, and one 64-bit `__ballot` per
+// slice per load IS the packed plane word (no lo/hi merge, no LDS, no block barrier).  The chunk-scale
+// build is therefore a single pass over the activations.  The *_fast kernels (at most 8 slices, 0 to 2
+// decimal places, no clipping) hold four consecutive elements a lane instead (bsi_quant_device.h).
 //
 // Arithmetic follows the reference's quantiser kernels (bsi_ops/csrc/cuda/bsi_cuda_kernels_quant.cuh:
 // rounding :24-29, shift :82-108, rounded shift + clamp :205-226) and packer
