@@ -493,6 +493,7 @@ PyObject* layer_call(PyObject*, PyObject* const* args, Py_ssize_t nargs, PyObjec
         if (out != Py_None) return out;
         Py_DECREF(out);
     }
+    if (module.base == nullptr) return PyErr_Format(PyExc_RuntimeError, "layer_call before bind_layer");
     Holder base_call(PyObject_GetAttr(module.base, names.__call__));
     return base_call.p != nullptr ? PyObject_Vectorcall(base_call.p, args, nargs, kwnames) : nullptr;
 }
@@ -605,7 +606,7 @@ PyObject* build_keys(PyObject*, PyObject* args) {
     PyObject* o = nullptr;
     int decimals = 0, bits = 0;
     if (!PyArg_ParseTuple(args, "Oii", &o, &decimals, &bits)) return nullptr;
-    if (bits < 2 || bits > 8 || decimals < 0 || decimals > 2 || !THPVariable_CheckExact(o)) Py_RETURN_NONE;
+    if (lib.build_fixed_keys == nullptr || bits < 2 || bits > 8 || decimals < 0 || decimals > 2 || !THPVariable_CheckExact(o)) Py_RETURN_NONE;
     HANDLE_TH_ERRORS
     const at::Tensor& x = THPVariable_Unpack(o);
     const int code = dtype_code(x.scalar_type());
@@ -639,7 +640,7 @@ PyObject* ewah_streams(PyObject*, PyObject* args) {
     PyObject* o = nullptr;
     double threshold = 0.0;
     if (!PyArg_ParseTuple(args, "Od", &o, &threshold)) return nullptr;
-    if (!THPVariable_CheckExact(o)) Py_RETURN_NONE;
+    if (lib.ewah_measure == nullptr || !THPVariable_CheckExact(o)) Py_RETURN_NONE;
     HANDLE_TH_ERRORS
     const at::Tensor& words = THPVariable_Unpack(o);
     if (!words.is_cuda() || words.scalar_type() != at::kLong || words.dim() != 2 || words.size(0) < 1 || words.size(0) > INT32_MAX ||
@@ -809,7 +810,7 @@ PyObject* scalar_query(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
         PyErr_SetString(PyExc_TypeError, "scalar_query(x, words, weights, decimals, threshold, divisor)");
         return nullptr;
     }
-    if (!THPVariable_CheckExact(args[0]) || !THPVariable_Check(args[1]) || !THPVariable_Check(args[2])) Py_RETURN_NONE;
+    if (lib.scalar_query_dot == nullptr || !THPVariable_CheckExact(args[0]) || !THPVariable_Check(args[1]) || !THPVariable_Check(args[2])) Py_RETURN_NONE;
     const long decimals = PyLong_AsLong(args[3]);
     const double threshold = PyFloat_AsDouble(args[4]), divisor = PyFloat_AsDouble(args[5]);
     if (PyErr_Occurred()) return nullptr;

@@ -35,6 +35,22 @@ def test_import_without_the_module():
     assert r.returncode == 0 and "whole" in r.stdout, r.stderr
 
 
+def test_functions_of_an_unbound_module():
+    """Imported by itself the module knows no library and no layer class: every call is left alone, none ends the process."""
+    r = _run("import torch\n"
+             "from bsipytorch_amd import _native\n"
+             "x = torch.zeros(2, 64)\n"
+             "assert _native.linear({}, x) is None and _native.dot(x, x) is None and _native.dot_streams(x, x) is None\n"
+             "assert _native.build(x, 2, True, True) is None and _native.build_keys(x, 2, 6) is None and _native.hybrid(x, 2, 0.5) is None\n"
+             "assert _native.ewah_streams(x.long(), 0.5) is None and _native.scalar_query(x[0], x, x, 2, 0.5, 1.0) is None\n"
+             "try:\n"
+             "    _native.layer_call(torch.nn.ReLU(), x)\n"
+             "except RuntimeError as e:\n"
+             "    print(e)\n"
+             "_native.forget()")
+    assert r.returncode == 0 and "bind_layer" in r.stdout, (r.returncode, r.stderr)
+
+
 def test_another_torch_is_refused():
     r = _run("import torch\n"
              "torch.__version__ = '2.1.0'\n"
