@@ -153,43 +153,39 @@ struct Operand {
     const T* as() const { return static_cast<const T*>(data); }
 };
 
-// A fixed-bit keyset's attributes as the dot needs them.
+// A fixed-bit keyset's attributes as a dot of Q rows needs them.
 struct Keys {
-    int64_t Sb, W, d, R, decimals, layout;
-    Operand words, ints8, weights;  // ints8.data is null if there is no image
-    bool tiled_image;
+    int64_t Sb, W, d, R, decimals;
+    int layout, operand_layout;  // of the planes, of `operand`
+    bool image;                  // there is an int8 image
+    Operand operand, weights;    // operand: planes or image (bsi_ops.key_operand)
 };
-bool read_keys(PyObject* handle, const at::Device& device, Keys* k) {
+bool read_keys(PyObject* handle, const at::Device& device, int64_t Q, Keys* k) {
     if (handle == nullptr || reinterpret_cast<PyObject*>(Py_TYPE(handle)) != shared.keys_type) return false;
     Holder attrs(PyObject_GenericGetDict(handle, nullptr));
     if (attrs.p == nullptr) {
         PyErr_Clear();
         return false;
     }
+    int64_t layout = 0;
     if (get(attrs.p, names.fixed) != Py_True || !get_int(attrs.p, names.Sb, &k->Sb) || !get_int(attrs.p, names.W, &k->W) ||
         !get_int(attrs.p, names.d, &k->d) || !get_int(attrs.p, names.num_keys, &k->R) ||
-        !get_int(attrs.p, names.decimals, &k->decimals) || !get_int(attrs.p, names.layout, &k->layout))
+        !get_int(attrs.p, names.decimals, &k->decimals) || !get_int(attrs.p, names.layout, &layout))
         return false;
     const at::Tensor* const words = get_tensor(attrs.p, names.words);
     const at::Tensor* const ints8 = get_tensor(attrs.p, names.ints8);
     const at::Tensor* const weights = get_tensor(attrs.p, names.slice_weights);
-    k->tiled_image = get(attrs.p, names.ints8_tiled) == Py_True;
     if (words == nullptr || weights == nullptr || words->device() != device || weights->device() != device || !weights->is_contiguous() ||
         k->R <= 0 || k->Sb < 2 || k->Sb > 8)
         return false;
-    k->words = Operand(*words);
+    k->layout = k->operand_layout = static_cast<int>(layout);
+    k->image = ints8 != nullptr;
     k->weights = Operand(*weights);
     (void)weights->const_data_ptr<float>();  // raises for another type
-    if (ints8 != nullptr) k->ints8 = Operand(*ints8);
+    const bool use_image = k->image && Q > shared.stream_max;
+    k->operand = Operand(use_image ? *ints8 : *words);
+    if (use_image) k->operand_layout = get(attrs.p, names.ints8_tiled) == Py_True ? BSI_LAYOUT_INT8_TILED : BSI_LAYOUT_INT8;
     return true;
-}
-// What a dot of Q rows reads of the keyset (bsi_ops.key_operand).
-const void* key_operand(const Keys& k, int64_t Q, int* layout, size_t* bytes) {
-    const bool image = k.ints8.data != nullptr && Q > shared.stream_max;
-    const Operand& t = image ? k.ints8 : k.words;
-    *layout = image ? (k.tiled_image ? BSI_LAYOUT_INT8_TILED : BSI_LAYOUT_INT8) : static_cast<int>(k.layout);
-    *bytes = t.bytes;
-    return t.data;
 }
 
 PyObject* int_tuple(std::initializer_list<int64_t> values) {
@@ -286,8 +282,9 @@ const void* keys_to_warm(PyObject* layer, int64_t rows, const at::Device& device
     }
     PyErr_Clear();
     Keys k;
-    int layout = 0;
-    return read_keys(handle, device, &k) ? key_operand(k, rows, &layout, bytes) : nullptr;
+    if (!read_keys(handle, device, rows, &k)) return nullptr;
+    *bytes = k.operand.bytes;
+    return k.operand.data;
 }
 
 // The areas of launches with the query build inside (2.1 MB each), one for each stream that has made one.  A stream without an
@@ -343,12 +340,13 @@ PyObject* linear(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     if (!x.is_cuda() || x.layout() != at::kStrided || in_code < 0 || x.dim() < 1 || x.numel() == 0) Py_RETURN_NONE;
     const at::Device device = x.device();
     if (device.index() != c10::hip::current_device()) Py_RETURN_NONE;
+    const int64_t d = x.size(-1), rows = x.numel() / d;
     Keys k;
     int64_t decimals = 0;
-    if (!read_keys(get(layer, names._bsi_keys_cuda), device, &k) || !get_int(layer, names.decimalPlaces, &decimals) ||
-        decimals != k.decimals || decimals < 0 || x.size(-1) != k.d)
+    if (!read_keys(get(layer, names._bsi_keys_cuda), device, rows, &k) || !get_int(layer, names.decimalPlaces, &decimals) ||
+        decimals != k.decimals || decimals < 0 || d != k.d)
         Py_RETURN_NONE;
-    const int64_t d = k.d, rows = x.numel() / d, chunks = (k.W + 3) / 4;
+    const int64_t chunks = (k.W + 3) / 4;
     PyObject* const buffers = get(layer, names._buffers);
     if (buffers == nullptr || !PyDict_Check(buffers)) Py_RETURN_NONE;
     Operand bias;
@@ -365,7 +363,7 @@ PyObject* linear(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     }
     // half-precision output: the kernels that have it (bsi_ops.can_output_half)
     const bool six_tiled = k.Sb == 6 && k.layout == BSI_LAYOUT_TILED16;
-    if (in_code != BSI_DTYPE_F32 && !(rows > shared.stream_max ? k.ints8.data != nullptr : six_tiled && chunks <= 32768)) Py_RETURN_NONE;
+    if (in_code != BSI_DTYPE_F32 && !(rows > shared.stream_max ? k.image : six_tiled && chunks <= 32768)) Py_RETURN_NONE;
     hipStream_t const st = stream_of(device);
     if (capturing(st)) Py_RETURN_NONE;
 
@@ -374,10 +372,7 @@ PyObject* linear(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     PyObject* slot = nullptr;
     void* ws = nullptr;
     int64_t ws_bytes = 0;
-    int layout = 0;
-    size_t bytes = 0;
-    const void* const operand = key_operand(k, rows, &layout, &bytes);
-    const at::Tensor coop = !few && k.Sb <= 8 && lib.linear_coop_serves(rows, d, k.R, static_cast<int>(decimals), config.bits, layout, static_cast<int>(k.Sb))
+    const at::Tensor coop = !few && k.Sb <= 8 && lib.linear_coop_serves(rows, d, k.R, static_cast<int>(decimals), config.bits, k.operand_layout, static_cast<int>(k.Sb))
                            ? coop_area(device, st) : at::Tensor();
     if (few) {
         if (!known_few_rows(device.index(), rows, d)) Py_RETURN_NONE;
@@ -413,14 +408,14 @@ PyObject* linear(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
         const void* const warm = keys_to_warm(layer, rows, device, &warm_bytes);
         // under the interpreter lock: launches on an area are in the order of their numbers
         rc = lib.linear_coop_out(xp, in_code, rows, d, static_cast<int>(decimals), config.bits, ++coop_launches, coop.data_ptr(),
-                                 static_cast<const uint64_t*>(operand), layout, k.weights.as<float>(), static_cast<int>(k.Sb),
+                                 k.operand.as<uint64_t>(), k.operand_layout, k.weights.as<float>(), static_cast<int>(k.Sb),
                                  k.R, inv, k.R, bias.as<float>(), out.data_ptr(), in_code, warm, warm_bytes, st);
         if (rc != BSI_OK) return fail_status(rc, "bsi_hip_linear_coop_out");
         count(layer, names.build_calls, 1);
     } else if (few) {
         Py_BEGIN_ALLOW_THREADS
         rc = lib.linear_few_rows_out(xp, in_code, rows, d, static_cast<int>(decimals), config.bits,
-                                     k.words.as<uint64_t>(), k.weights.as<float>(), static_cast<int>(k.Sb), k.R, inv, k.R,
+                                     k.operand.as<uint64_t>(), k.weights.as<float>(), static_cast<int>(k.Sb), k.R, inv, k.R,
                                      bias.as<float>(), out.data_ptr(), in_code, st);
         Py_END_ALLOW_THREADS
         if (rc != BSI_OK) return fail_status(rc, "bsi_hip_linear_few_rows_out");
@@ -446,7 +441,7 @@ PyObject* linear(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
         if (rebuild != 0) PyList_SetItem(slot, 0, Py_NewRef(Py_None));  // until the build is enqueued
         // under the interpreter lock: another thread must not enqueue a build of its own between the two launches
         rc = lib.linear_out(xp, in_code, rows, d, static_cast<int>(decimals), config.bits, rebuild, ws, static_cast<size_t>(ws_bytes),
-                            static_cast<const uint64_t*>(operand), layout, k.weights.as<float>(), static_cast<int>(k.Sb),
+                            k.operand.as<uint64_t>(), k.operand_layout, k.weights.as<float>(), static_cast<int>(k.Sb),
                             k.R, inv, k.R, bias.as<float>(), out.data_ptr(), in_code, config.core, warm, warm_bytes, st);
         if (rc != BSI_OK) return fail_status(rc, "bsi_hip_linear_out");
         if (rebuild != 0 && key.p != nullptr) {
@@ -539,7 +534,7 @@ PyObject* dot(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     const bool chunked = chunk_scales != nullptr && chunk_scales->numel() > 0;
     const at::Tensor* const scales = chunked ? chunk_scales : row_scales;
     Keys k;
-    if (device.index() != c10::hip::current_device() || !read_keys(args[1], device, &k) || k.W != W || k.decimals != decimals ||
+    if (device.index() != c10::hip::current_device() || !read_keys(args[1], device, Q, &k) || k.W != W || k.decimals != decimals ||
         decimals < 0 || Q <= 0 || Sa < 2 || Sa > 8 || weights->size(0) != Q || weights->size(1) != Sa || scales == nullptr ||
         scales->device() != device || scales->scalar_type() != at::kFloat || !scales->is_contiguous() || ints8->device() != device ||
         !ints8->is_contiguous() || ints8->numel() != Q * chunks * 256 || !words->is_contiguous())
@@ -550,12 +545,10 @@ PyObject* dot(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     const Operand planes(*words), image(*ints8), factors(*scales);
     if (capturing(st) || !split_scratch(device.index(), Q, k.R, W)) Py_RETURN_NONE;
     at::Tensor out = at::detail::empty_cuda({Q, k.R}, at::kFloat, device, std::nullopt);
-    int layout = 0, rc = BSI_OK;
-    size_t bytes = 0;
-    const void* const operand = key_operand(k, Q, &layout, &bytes);
+    int rc = BSI_OK;
     Py_BEGIN_ALLOW_THREADS
     rc = lib.dot(planes.as<uint64_t>(), image.as<int8_t>(), factors.as<float>(), chunked ? static_cast<int>(chunks) : 1,
-                 static_cast<int>(Sa), static_cast<int>(W), static_cast<const uint64_t*>(operand), layout, k.weights.as<float>(),
+                 static_cast<int>(Sa), static_cast<int>(W), k.operand.as<uint64_t>(), k.operand_layout, k.weights.as<float>(),
                  static_cast<int>(k.Sb), k.R, Q,
                  scale_inv(decimals, k.decimals), k.R, out.data_ptr<float>(), nullptr, config.core, nullptr, 0, st);
     Py_END_ALLOW_THREADS
@@ -778,7 +771,7 @@ PyObject* dot_streams(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     const at::Device device = streams->device();
     const int64_t chunks = (W + 3) / 4;
     Keys k;
-    if (!streams->is_cuda() || device.index() != c10::hip::current_device() || !read_keys(args[1], device, &k) || k.W != W ||
+    if (!streams->is_cuda() || device.index() != c10::hip::current_device() || !read_keys(args[1], device, Q, &k) || k.W != W ||
         k.decimals != decimals || decimals < 0 || Q <= 0 || Sa < 2 || Sa > 8 || off->numel() != Q * Sa || len->numel() != Q * Sa ||
         scales->device() != device || !scales->is_contiguous() || (chunked && W % 4 != 0) ||
         scales->numel() != (chunked ? Q * chunks : Q))
@@ -789,12 +782,10 @@ PyObject* dot_streams(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     at::Tensor out = at::detail::empty_cuda({Q, k.R}, at::kFloat, device, std::nullopt);
     const size_t need = lib.dot_ewah_batch_workspace_bytes(Q, static_cast<int>(W));
     at::Tensor ws = at::detail::empty_cuda({static_cast<int64_t>(need)}, at::kByte, device, std::nullopt);
-    int layout = 0, rc = BSI_OK;
-    size_t bytes = 0;
-    const void* const operand = key_operand(k, Q, &layout, &bytes);
+    int rc = BSI_OK;
     Py_BEGIN_ALLOW_THREADS
     rc = lib.dot_ewah_batch(so.as<uint64_t>(), oo.as<int64_t>(), lo.as<int32_t>(), static_cast<int>(Sa), static_cast<int>(W),
-                            factors.as<float>(), chunked ? static_cast<int>(chunks) : 1, static_cast<const uint64_t*>(operand), layout,
+                            factors.as<float>(), chunked ? static_cast<int>(chunks) : 1, k.operand.as<uint64_t>(), k.operand_layout,
                             k.weights.as<float>(), static_cast<int>(k.Sb), k.R, Q, scale_inv(decimals, k.decimals), k.R, nullptr,
                             static_cast<float*>(out.data_ptr()), nullptr, ws.data_ptr(), need, st);
     Py_END_ALLOW_THREADS
