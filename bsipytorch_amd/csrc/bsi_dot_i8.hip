@@ -84,7 +84,10 @@ struct I8Cfg {
     static constexpr int kBlock = (kConsumers + kLoaders) * 64;
     static constexpr int kOperandK = TM * 128;         // bytes of the key tile of one half-chunk
     static constexpr int kStage = (TM + TN) * 128;     // keys then queries
-    static constexpr int kScaleBytes = 4 * kLoaders * 256;  // chunk scales: ring of 4 chunks x loader regions x 64 floats
+    // chunk scales: a ring of four groups of one or four chunks (i8_scale_shift), [query][chunk of the group] floats
+    static constexpr int kScaleRegions = TN >= 64 ? TN / 64 : 1;      // of 64 queries
+    static constexpr int kScaleGroup = kScaleRegions * 64 * 4 * 4;    // bytes
+    static constexpr int kScaleBytes = 4 * kScaleGroup;
     static constexpr int kEpilogueBytes = 2 * TM * 4;  // the tile's key factors, then its biases (chain modes)
     static constexpr int kLds = 4 * kStage + kScaleBytes + kEpilogueBytes;
     // D-split launches: one flag word per MFMA wave (a prefix of its chain came near the exactness limit), then the
@@ -94,6 +97,15 @@ struct I8Cfg {
     static_assert(kConsumers < 15, "flag words of the MFMA waves, then the decision word");
 };
 constexpr int kSplitLeave = 0, kSplitCombine = 1, kSplitRedo = 2;
+
+// How the chunk scales are fetched (kFour of the kernels): one float of each of 64 queries for every chunk, or four consecutive
+// floats of 16 queries, for the group of four chunks after the one a load is issued in.  The scales of a query are contiguous:
+// one float of 64 queries is up to 64 lines, half as many again as the operands of a chunk of the 64 x 64 tile have, four floats
+// of 16 are 16.  Rows of fewer than 16 chunks have several queries in a line and gain nothing for the code and the loads ahead
+// of the first group; nor do row scales.
+// us, one and four (64 x 64 tiles) 512 x 2048 x 8192 16.4, 15.5; 256 x 1024 x 8192 11.4, 10.5; (128 x 64) 512 x 4096 x 4096 12.5,
+// 11.7; (128 x 128) 512 x 8192 x 8192 34.5, 32.8 -- and at 8 chunks 512 x 8192 x 2048 11.2, 11.5, 512 x 2048 x 2048 5.8, 6.0.
+static bool i8_four_scales(int qscale_stride) { return qscale_stride >= 16; }
 
 // Timeline build (make TIMELINE=1, -DBSI_TIMELINE): one MFMA wave and one loader wave of every workgroup of
 // dot_mfma_i8_kernel stamp the 100 MHz wall clock at the points below, 8 slots per workgroup (the first
@@ -136,7 +148,7 @@ __device__ __forceinline__ void i8_warm_lines(unsigned char* __restrict__ unused
 // A loader wave of the int8-image kernels (lw = its number among the C::kLoaders loader waves; `consumers` MFMA
 // waves share the workgroup's barriers with it): 8 of the stage's groups of 8 rows (the TM key rows, then the TN
 // query rows: a load moves 1 KiB = 8 rows x 128 bytes), plus the chunk scales of 64 queries once per chunk.
-template <typename C, bool kSum>
+template <typename C, bool kSum, bool kFour>
 __device__ __forceinline__ void i8_loader_wave(unsigned char* __restrict__ lds, int lw, int lane,
                                                const int8_t* __restrict__ A8, const float* __restrict__ qscale,
                                                int qscale_stride, const int8_t* __restrict__ K8,
@@ -150,7 +162,7 @@ __device__ __forceinline__ void i8_loader_wave(unsigned char* __restrict__ lds, 
     // The key groups and the query groups both divide evenly among the loader waves: every loader moves KG / L key
     // groups, then QG / L query groups, so which operand a load belongs to is known at compile time.
     static_assert(KG % L == 0 && QG % L == 0 && NI == KG / L + QG / L, "loads per loader wave");
-    unsigned char* const scale_lds = lds + 4 * C::kStage;  // [chunk & 3][loader][64] floats
+    unsigned char* const scale_lds = lds + 4 * C::kStage;
     // The prologue below is kept short on purpose: it runs on one wave per SIMD while the whole workgroup waits for
     // the first stage.  No row is clamped: the offset of a lane's ROW (group and row inside it) travels in the
     // per-lane offset of the buffer load, which the hardware compares with the descriptor's size, so a row past its
@@ -186,11 +198,17 @@ __device__ __forceinline__ void i8_loader_wave(unsigned char* __restrict__ lds, 
                          : static_cast<uint32_t>(gg) * 8 * rowbytes32);
     }
     const uint32_t kstep_bytes = key_tiled ? 8192u : 128u;  // from one half-chunk of a key row to the next
-    // scales: loader wave lw fetches the 64 queries of group lw % (TN / 64) (waves fetching the same group
-    // write their own regions, so that every loader wave has the same number of loads in flight)
+    // Scales: a load takes those of 1 << sh chunks and 64 >> sh queries, lane = (query, chunk).  One chunk at a time, behind the second half of every chunk, its scales of the 64 queries of this wave's region; in groups of four, behind
+    // chunk c, the quarter c % 4 of those queries' for the group after the one c is in.  Waves of a region load the same.  The
+    // position inside the row travels in the per-lane offset: what a group has past the end of the last row is not read.
     const bsi_rsrc rs = make_rsrc(qscale + q0 * qscale_stride, static_cast<size_t>(Q - q0) * qscale_stride * 4);
-    const uint32_t soff = static_cast<uint32_t>((lw % (TN >= 64 ? TN / 64 : 1)) * 64 + lane) * static_cast<uint32_t>(qscale_stride) * 4;
-    const int sstep = (qscale_stride == 1) ? 0 : 4;
+    constexpr int sh = kFour ? 2 : 0;
+    const int sstep = (qscale_stride == 1) ? 0 : 4, region = lw % C::kScaleRegions;
+    const int soff = (region * 64 + (lane >> sh)) * qscale_stride * 4 + ((lane & ((1 << sh) - 1)) + first_chunk) * sstep;
+    auto load_scales = [&](int group, int quarter) {
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, BSI_LDS_PTR(scale_lds + (group & 3) * C::kScaleGroup + region * 1024 + quarter * 256), 4,
+                                                 soff + (quarter * 64 * qscale_stride + (group << sh) * sstep), 0, 0, 0);
+    };
     // issue() is called for h = 0, 1, 2, ... in order, h counted from the first half of chunk first_chunk (the
     // workgroup's share of the row in a D-split launch, else 0); in the sum mode (next_c, next_dg) follow the chunk
     // and the digit (counted from the top one) of the half-chunk to come
@@ -220,16 +238,15 @@ __device__ __forceinline__ void i8_loader_wave(unsigned char* __restrict__ lds, 
             load16_to_lds(is_key[i] ? rk : rq, voff[i], is_key[i] ? so_k : so_q,
                           lds + (h & 3) * C::kStage + g * 1024);
         }
-        if (!kSum && (h & 1)) {  // with the second half of chunk c = h / 2: its scales
-            const int c = hc >> 1;
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(
-                rs, BSI_LDS_PTR(scale_lds + ((c & 3) * C::kLoaders + lw) * 256), 4, static_cast<int>(soff),
-                (c + first_chunk) * sstep, 0, 0);
-        }
+        if (!kSum && (h & 1)) load_scales(kFour ? (hc >> 3) + 1 : hc >> 1, kFour ? (hc >> 1) & 3 : 0);
     };
     if (lw == 0) BSI_STAMP(kStampFirstIssue);
     issue(0);
     issue(1);
+    constexpr int kSharing = L / C::kScaleRegions;  // waves of a region: of a first group of four chunks each loads its part
+    constexpr int kFirst = !kSum && kFour ? 4 / kSharing : 0;
+#pragma unroll
+    for (int k = 0; k < kFirst; ++k) load_scales(0, lw / C::kScaleRegions + kSharing * k);
     issue(2);
     if (lw == 0) BSI_STAMP(kStampThreeIssued);
     // The epilogue's operands, staged once per workgroup behind the first three stages: the slice-0 weight (key
@@ -254,7 +271,7 @@ __device__ __forceinline__ void i8_loader_wave(unsigned char* __restrict__ lds, 
         }
     }
     // stage 0 landed (stage 1 + scales + stage 2 + the epilogue operands may be in flight)
-    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * NI + (kSum ? 0 : 1) + kEpi) : "memory");
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * NI + (kSum ? 0 : 1) + kFirst + kEpi) : "memory");
     lds_barrier();
     for (int h = 0; h < halves; ++h) {
         if (h + 3 < halves) {
@@ -413,6 +430,9 @@ __device__ __forceinline__ void i8_store_half(const float (&v)[WM][WN][4], const
 }
 
 // The end of a tile in the chain modes: every output takes its key's factor, the decimal scale and the bias, and is stored.
+// kHalf: the outputs are in the half-precision type out_dtype, else float32.  One kind of store a kernel: with both in one, a
+// launch of a few microseconds fetches instructions it does not run between those it does (us, both and one: 64 x 256 x 2048
+// 4.89, 4.77; 40 x 1024 x 1024 3.70, 3.55; 77 x 4800 x 1600 4.63, 4.48; 100 x 3000 x 1000 4.20, 4.03).
 // epi: the key factors and biases of the tile's TM rows, from the copy the loader waves staged in LDS (0 for rows past R and
 // for a call without bias): two 16-byte reads per 16-key tile.
 template <int TM, int WM, int WN, bool kHalf>
@@ -439,10 +459,10 @@ __device__ __forceinline__ void i8_store_tile(const float (&accf)[WM][WN][4], co
                 for (int e = 0; e < 4; ++e) {
                     // (acc * key scale) * scale_inv, then + bias: each step rounded on its own, as separate kernels would
                     v[a][b][e] = ((accf[a0 + a][b][e] * down) * bs[e]) * scale_inv;
-                    if (has_bias && out_dtype == BSI_DTYPE_F32) v[a][b][e] = v[a][b][e] + bi[a][e];
+                    if (!kHalf && has_bias) v[a][b][e] = v[a][b][e] + bi[a][e];
                 }
         }
-        if (kHalf && out_dtype != BSI_DTYPE_F32) {
+        if constexpr (kHalf) {
             i8_store_half<2, WN>(v, bi, has_bias, out_dtype, out, R_total, rw, qw, R, Q, ln, lg);
             continue;
         }
@@ -491,7 +511,7 @@ __device__ __forceinline__ void i8_tile_of(const I8Grid& g, unsigned id, int& bx
     by = static_cast<int>(first + in - x * (last ? left : static_cast<unsigned>(g.height)));
 }
 
-template <int TM, int TN, int kMode, bool kSplit, bool kBuild>
+template <int TM, int TN, int kMode, bool kSplit, bool kBuild, bool kFour, bool kHalf>
 __global__ __launch_bounds__((I8Cfg<TM, TN>::kBlock)) void dot_mfma_i8_kernel(
     const int8_t* A8, const float* qscale, int qscale_stride,
     const int8_t* __restrict__ K8,  // int8 key image [R, chunks * 256]
@@ -557,20 +577,20 @@ __global__ __launch_bounds__((I8Cfg<TM, TN>::kBlock)) void dot_mfma_i8_kernel(
     // the workgroup's run of chunks: all of them, or segment seg of nseg
     const int first_chunk = kSplit ? (chunks * seg) / nseg : 0;
     const int my_chunks = kSplit ? (chunks * (seg + 1)) / nseg - first_chunk : vchunks;
-    unsigned char* const scale_lds = lds + 4 * C::kStage;  // [chunk & 3][loader][64] floats
+    unsigned char* const scale_lds = lds + 4 * C::kStage;
     // kSplit: [MFMA wave] flags, [15] = decision
     volatile __attribute__((address_space(3))) int* const split_flags =
         reinterpret_cast<volatile __attribute__((address_space(3))) int*>(BSI_LDS_PTR(lds + C::kLds));
 
     if (wave >= C::kConsumers) {
         if (wave == C::kConsumers) BSI_STAMP(kStampLoaderEntry);
-        i8_loader_wave<C, kSum>(lds, wave - C::kConsumers, lane, A8, qscale, qscale_stride, K8, Bw, Sb, chunks, first_chunk,
+        i8_loader_wave<C, kSum, kFour>(lds, wave - C::kConsumers, lane, A8, qscale, qscale_stride, K8, Bw, Sb, chunks, first_chunk,
                                 my_chunks * 2, R, Q, r0, q0, rowbytes, bias, ndig, dig_stride, key_tiled, warm, warm_lines);
         if (kSplit) {
             lds_barrier();  // the MFMA waves have stored their partial sums
             lds_barrier();  // the decision is in LDS
             if (__builtin_amdgcn_readfirstlane(split_flags[15]) == kSplitRedo)
-                i8_loader_wave<C, kSum>(lds, wave - C::kConsumers, lane, A8, qscale, qscale_stride, K8, Bw, Sb, chunks, 0,
+                i8_loader_wave<C, kSum, kFour>(lds, wave - C::kConsumers, lane, A8, qscale, qscale_stride, K8, Bw, Sb, chunks, 0,
                                         chunks * 2, R, Q, r0, q0, rowbytes, bias, ndig, dig_stride, key_tiled, nullptr, 0);
         }
         if (wave == C::kConsumers) BSI_STAMP(kStampLoaderDone);
@@ -613,16 +633,17 @@ __global__ __launch_bounds__((I8Cfg<TM, TN>::kBlock)) void dot_mfma_i8_kernel(
             int_off[a][b] = (kInts && q < Q && r < R) ? (q * R + r) * chunks : -1;
         }
     }
-    // chunk scales of the lane's query columns, from the loaders' ring: region g holds queries 64 g .. + 63
+    // chunk scales of the lane's query columns, from the loaders' ring
+    constexpr int sh = kFour ? 2 : 0;
     const int qfirst = wq * (WN * 16);
-    const unsigned char* sread = scale_lds + (qfirst >> 6) * 256 + ((qfirst & 63) + ln) * 4;
+    const unsigned char* sread = scale_lds + (qfirst >> 6) * 1024 + (((qfirst & 63) + ln) << (2 + sh));
     float qsa[WN], qsb[WN];  // scales of even / odd chunks
 #pragma unroll
     for (int b = 0; b < WN; ++b) qsa[b] = qsb[b] = 0.0f;
 #define BSI_I8_SCALES(dst, c)                                                                                  \
     {                                                                                                          \
         _Pragma("unroll") for (int b = 0; b < WN; ++b) dst[b] =                                                \
-            *reinterpret_cast<const float*>(sread + ((c) & 3) * (C::kLoaders * 256) + b * 64);                 \
+            *reinterpret_cast<const float*>(sread + ((c) >> sh & 3) * C::kScaleGroup + ((c) & ((1 << sh) - 1)) * 4 + (b * 64 << sh)); \
     }
     // The k-steps run one behind their operand reads: k-step j's MFMAs cover the reads of k-step j + 1.  A
     // stage (half-chunk, two k-steps) is released to the loaders by the barrier that follows the k-step in
@@ -900,7 +921,7 @@ __global__ __launch_bounds__((I8Cfg<TM, TN>::kBlock)) void dot_mfma_i8_kernel(
                 if (kInts && int_off[a][b] >= 0 && e < int_rows[a])
                     chunk_ints[int_off[a][b] + static_cast<int64_t>(e) * chunks + (chunks - 1)] = v >> down_shift;
             }
-    i8_store_tile<TM, WM, WN, kMode == kI8Chain>(accf, lds + 4 * C::kStage + C::kScaleBytes, down, scale_inv, bias != nullptr, out_dtype,
+    i8_store_tile<TM, WM, WN, kMode == kI8Chain && kHalf>(accf, lds + 4 * C::kStage + C::kScaleBytes, down, scale_inv, bias != nullptr, out_dtype,
                                                  out, R_total, r0, q0, wr, wq, R, Q, ln, lg, out_stream != 0);
 #ifdef BSI_TIMELINE
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the stamp below: the outputs have left the wave
@@ -921,7 +942,8 @@ __global__ __launch_bounds__((I8Cfg<TM, TN>::kBlock)) void dot_mfma_i8_kernel(
 template <int TM, int TN>
 struct I8TilesCfg : I8Cfg<TM, TN> {
     using C = I8Cfg<TM, TN>;
-    static constexpr int kLdsTiles = C::kLds + 3 * C::kEpilogueBytes;  // four sets of key factors and biases
+    static constexpr int kScaleBytes = 4 * C::kLoaders * 256;  // chunk scales: ring of 4 chunks x loader regions x 64 floats
+    static constexpr int kLdsTiles = 4 * C::kStage + kScaleBytes + 4 * C::kEpilogueBytes;  // four sets of key factors and biases
 };
 
 // A loader wave: the stages of all the workgroup's tiles, one after the other; three stages ahead of the MFMA waves, across
@@ -990,7 +1012,7 @@ __device__ __forceinline__ void i8_tiles_loader_wave(unsigned char* __restrict__
             __builtin_amdgcn_raw_ptr_buffer_load_lds(
                 rs, BSI_LDS_PTR(lds + 4 * C::kStage + (((ring >> 1) & 3) * L + lw) * 256), 4, static_cast<int>(soff), (h >> 1) * sstep, 0, 0);
         if (h == epi_at) {  // tiles of one chunk: the MFMA waves may still be reading the set of two tiles ago
-            unsigned char* const epi = lds + 4 * C::kStage + C::kScaleBytes + (tile & 3) * C::kEpilogueBytes;
+            unsigned char* const epi = lds + 4 * C::kStage + I8TilesCfg<TM, TN>::kScaleBytes + (tile & 3) * C::kEpilogueBytes;
 #pragma unroll
             for (int k = 0; k < kEpi; ++k) {
                 const int j = (lw + L * k) % (2 * (TM / 64));
@@ -1024,7 +1046,7 @@ __device__ __forceinline__ void i8_tiles_loader_wave(unsigned char* __restrict__
     }
 }
 
-template <int TM, int TN>
+template <int TM, int TN, bool kHalf>
 __global__ __launch_bounds__((I8Cfg<TM, TN>::kBlock)) void dot_mfma_i8_tiles_kernel(
     const int8_t* __restrict__ A8, const float* __restrict__ qscale, int qscale_stride, const int8_t* __restrict__ K8,
     const float* __restrict__ Bw, int Sb, int chunks, int64_t R, int64_t Q, int down_shift, float scale_inv, int64_t R_total,
@@ -1075,10 +1097,15 @@ __global__ __launch_bounds__((I8Cfg<TM, TN>::kBlock)) void dot_mfma_i8_tiles_ker
     v4i ka[2][WM], qb[2][WN];
     // the ring's two pairs of slots: the tile's even chunks sit in the pair at `even`, its odd ones in the other
     int even = 0, odd = 2 * C::kStage, chunk0 = 0;
-#define BSI_TILES_CHUNK(here, next, acc, prev, qs)          \
+    // A chunk's own scales, which landed with its second half, are read in its middle: the next chunk's first chain step needs them,
+    // and read behind the chunk it waited for them (us: 4096 x 4096 x 16384 293 -> 284, 2048 x 2048 x 8192 42.0 -> 40.8; a workgroup
+    // of one tile gains nothing by it).
+#define BSI_TILES_CHUNK(here, next, acc, prev, qs, own, c)  \
     BSI_I8_KSTEP_AT(0, here, acc, prev, qs);                \
     lds_barrier();                                          \
     BSI_I8_KSTEP_AT(1, (here) + C::kStage, acc, prev, qs);  \
+    BSI_TILES_SCALES(own, c);                               \
+    __builtin_amdgcn_sched_barrier(0);                      \
     BSI_I8_KSTEP_AT(2, (here) + C::kStage, acc, prev, qs);  \
     lds_barrier();                                          \
     BSI_I8_KSTEP_AT(3, next, acc, prev, qs);
@@ -1103,15 +1130,12 @@ __global__ __launch_bounds__((I8Cfg<TM, TN>::kBlock)) void dot_mfma_i8_tiles_ker
     for (unsigned id = blockIdx.x; id < tiles; id += gridDim.x, ++tile) {
         int c = 0;
         for (; c + 1 < chunks; c += 2) {
-            BSI_TILES_CHUNK(even, odd, acc0, acc1, qsb);
-            BSI_TILES_SCALES(qsa, chunk0 + c);
-            BSI_TILES_CHUNK(odd, even, acc1, acc0, qsa);
-            BSI_TILES_SCALES(qsb, chunk0 + c + 1);
+            BSI_TILES_CHUNK(even, odd, acc0, acc1, qsb, qsa, chunk0 + c);
+            BSI_TILES_CHUNK(odd, even, acc1, acc0, qsa, qsb, chunk0 + c + 1);
         }
         // the chain step of the last chunk; the last k-step has read the next tile's first operands
         if (c < chunks) {
-            BSI_TILES_CHUNK(even, odd, acc0, acc1, qsb);
-            BSI_TILES_SCALES(qsa, chunk0 + c);
+            BSI_TILES_CHUNK(even, odd, acc0, acc1, qsb, qsa, chunk0 + c);
             const int t = even;
             even = odd;
             odd = t;
@@ -1140,7 +1164,7 @@ __global__ __launch_bounds__((I8Cfg<TM, TN>::kBlock)) void dot_mfma_i8_tiles_ker
         // from values the compiler cannot see through, so that no address of the stores is held in registers over the chunk loop
         int ln_late = ln, lg_late = lg;
         asm volatile("" : "+v"(ln_late), "+v"(lg_late));
-        i8_store_tile<TM, WM, WN, true>(accf, lds + 4 * C::kStage + C::kScaleBytes + (tile & 3) * C::kEpilogueBytes, down, scale_inv,
+        i8_store_tile<TM, WM, WN, kHalf>(accf, lds + 4 * C::kStage + I8TilesCfg<TM, TN>::kScaleBytes + (tile & 3) * C::kEpilogueBytes, down, scale_inv,
                                         bias != nullptr, out_dtype, out, R_total, static_cast<int64_t>(bx) * TM,
                                         static_cast<int64_t>(by) * TN, wr, wq, R, Q, ln_late, lg_late, out_stream != 0);
 #pragma unroll
@@ -1251,7 +1275,7 @@ __global__ __launch_bounds__((I8WCfg<WN>::kBlock)) void dot_mfma_i8w_kernel(
     unsigned char* const scale_lds = lds + 4 * C::kStage;
 
     if (wave >= W::kConsumers) {
-        i8_loader_wave<C, false>(lds, wave - W::kConsumers, lane, A8, qscale, qscale_stride, K8, Bw, Sb, chunks, 0, halves, R, Q,
+        i8_loader_wave<C, false, false>(lds, wave - W::kConsumers, lane, A8, qscale, qscale_stride, K8, Bw, Sb, chunks, 0, halves, R, Q,
                                  r0, q0, rowbytes, bias, 1, 0, key_tiled, warm, warm_lines);
         return;
     }
@@ -1291,15 +1315,16 @@ __global__ __launch_bounds__((I8WCfg<WN>::kBlock)) void dot_mfma_i8w_kernel(
             if (kInts && ql + b * 16 < Q) dump.qmask |= 1u << b;
     }
     // chunk scales of the lane's query columns, from the loaders' ring: 64 queries per region, region g = queries 64 g ..
+    constexpr int sh = 0;
     const int qfirst = wq * (16 * WN);
-    const unsigned char* sread = scale_lds + (qfirst >> 6) * 256 + ((qfirst & 63) + ln) * 4;
+    const unsigned char* sread = scale_lds + (qfirst >> 6) * 1024 + (((qfirst & 63) + ln) << (2 + sh));
     float qsa[WN], qsb[WN];  // scales of even / odd chunks (all zero before the first chunk: its "previous" chain adds 0)
 #pragma unroll
     for (int b = 0; b < WN; ++b) qsa[b] = qsb[b] = 0.0f;
 #define BSI_I8W_SCALES(dst, c)                                                                         \
     {                                                                                                  \
         _Pragma("unroll") for (int b = 0; b < WN; ++b) dst[b] =                                        \
-            *reinterpret_cast<const float*>(sread + ((c) & 3) * (C::kLoaders * 256) + b * 64);         \
+            *reinterpret_cast<const float*>(sread + ((c) >> sh & 3) * C::kScaleGroup + ((c) & ((1 << sh) - 1)) * 4 + (b * 64 << sh)); \
     }
     v4i ka[2][4], qb[2][WN];  // operand sets of even / odd k-steps
 #define BSI_I8W_KSTEP(KS, nslot, qc, qp, ic, ip)                                                                    \
@@ -1450,7 +1475,7 @@ static I8Grid i8_grid(int64_t tiles_x, int64_t tiles_y, dim3* grid) {
     return g;
 }
 
-template <int TM, int TN, int kMode>
+template <int TM, int TN, int kMode, bool kFour, bool kHalf>
 static void launch_mfma_i8_tm(const int8_t* A8, const float* qscale, int stride, const int8_t* K8, const float* Bw,
                               int Sb, int chunks, int64_t R, int64_t Q, int down_shift, float scale_inv,
                               int64_t R_total, float* out, int32_t* chunk_ints, const float* bias, hipStream_t st,
@@ -1463,8 +1488,8 @@ static void launch_mfma_i8_tm(const int8_t* A8, const float* qscale, int stride,
     if constexpr (kMode == kI8Chain && TM == 128)
         if (t_coop == nullptr && tiles > kCus && tiles * chunks < (int64_t{1} << 29)) {
             static LdsOptIn once;
-            lds_opt_in(once, reinterpret_cast<const void*>(&dot_mfma_i8_tiles_kernel<TM, TN>), I8TilesCfg<TM, TN>::kLdsTiles);
-            launch((dot_mfma_i8_tiles_kernel<TM, TN>), dim3(kCus), dim3(C::kBlock), I8TilesCfg<TM, TN>::kLdsTiles, st, A8, qscale, stride,
+            lds_opt_in(once, reinterpret_cast<const void*>(&dot_mfma_i8_tiles_kernel<TM, TN, kHalf>), I8TilesCfg<TM, TN>::kLdsTiles);
+            launch((dot_mfma_i8_tiles_kernel<TM, TN, kHalf>), dim3(kCus), dim3(C::kBlock), I8TilesCfg<TM, TN>::kLdsTiles, st, A8, qscale, stride,
                    K8, Bw, Sb, chunks, R, Q, down_shift, scale_inv, R_total, out, bias, key_tiled,
                    static_cast<const unsigned char*>(g_warm_ptr), static_cast<long long>(g_warm_bytes / 128), stream_output(), g,
                    static_cast<unsigned>(tiles), t_out_dtype);
@@ -1475,16 +1500,16 @@ static void launch_mfma_i8_tm(const int8_t* A8, const float* qscale, int stride,
             CoopBuild coop = *t_coop;
             coop.shares = coop_shares(grid.x * grid.y, coop.by_row ? coop.rows : coop.rows * coop.chunks);
             static LdsOptIn once;
-            lds_opt_in(once, reinterpret_cast<const void*>(&dot_mfma_i8_kernel<TM, TN, kI8Chain, false, true>), C::kLds);
-            launch((dot_mfma_i8_kernel<TM, TN, kI8Chain, false, true>), grid, dim3(C::kBlock), C::kLds, st, A8, qscale, stride, K8, Bw, Sb,
+            lds_opt_in(once, reinterpret_cast<const void*>(&dot_mfma_i8_kernel<TM, TN, kI8Chain, false, true, false, kHalf>), C::kLds);
+            launch((dot_mfma_i8_kernel<TM, TN, kI8Chain, false, true, false, kHalf>), grid, dim3(C::kBlock), C::kLds, st, A8, qscale, stride, K8, Bw, Sb,
                    chunks, R, Q, down_shift, scale_inv, R_total, out, chunk_ints, bias, ndig, dig_stride, key_indices, key_tiled,
                    static_cast<const unsigned char*>(g_warm_ptr), static_cast<long long>(g_warm_bytes / 128), stream_output(),
                    static_cast<float*>(nullptr), static_cast<unsigned*>(nullptr), 0.0f, 0, g, t_out_dtype, coop);
             return;
         }
     static LdsOptIn once0;
-    lds_opt_in(once0, reinterpret_cast<const void*>(&dot_mfma_i8_kernel<TM, TN, kMode, false, false>), C::kLds);
-    launch((dot_mfma_i8_kernel<TM, TN, kMode, false, false>), grid, dim3(C::kBlock), C::kLds, st, A8, qscale, stride, K8,
+    lds_opt_in(once0, reinterpret_cast<const void*>(&dot_mfma_i8_kernel<TM, TN, kMode, false, false, kFour, kHalf>), C::kLds);
+    launch((dot_mfma_i8_kernel<TM, TN, kMode, false, false, kFour, kHalf>), grid, dim3(C::kBlock), C::kLds, st, A8, qscale, stride, K8,
                        Bw, Sb, chunks, R, Q, down_shift, scale_inv, R_total, out, chunk_ints, bias, ndig, dig_stride,
                        key_indices, key_tiled, static_cast<const unsigned char*>(g_warm_ptr),
                        static_cast<long long>(g_warm_bytes / 128), stream_output(), static_cast<float*>(nullptr),
@@ -1493,7 +1518,7 @@ static void launch_mfma_i8_tm(const int8_t* A8, const float* qscale, int stride,
 
 // The D-split launch of the chain mode: `segments` workgroups per output tile, each over its own run of chunks (see
 // the head of dot_mfma_i8_kernel).  scratch: the calling thread's attached split scratch (counters, then partial sums).
-template <int TM, int TN>
+template <int TM, int TN, bool kHalf>
 static void launch_mfma_i8_split(int segments, unsigned char* scratch, const int8_t* A8, const float* qscale, int stride,
                                  const int8_t* K8, const float* Bw, int Sb, int chunks, int64_t R, int64_t Q, int down_shift,
                                  float scale_inv, int64_t R_total, float* out, const float* bias, hipStream_t st,
@@ -1507,8 +1532,8 @@ static void launch_mfma_i8_split(int segments, unsigned char* scratch, const int
     while ((1 << log2_segments) < segments) ++log2_segments;
     const float limit = __builtin_ldexpf(1.0f, 24 + down_shift - log2_segments);
     static LdsOptIn once0;
-    lds_opt_in(once0, reinterpret_cast<const void*>(&dot_mfma_i8_kernel<TM, TN, kI8Chain, true, false>), C::kLdsSplit);
-    launch((dot_mfma_i8_kernel<TM, TN, kI8Chain, true, false>), grid, dim3(C::kBlock), C::kLdsSplit, st, A8, qscale,
+    lds_opt_in(once0, reinterpret_cast<const void*>(&dot_mfma_i8_kernel<TM, TN, kI8Chain, true, false, false, kHalf>), C::kLdsSplit);
+    launch((dot_mfma_i8_kernel<TM, TN, kI8Chain, true, false, false, kHalf>), grid, dim3(C::kBlock), C::kLdsSplit, st, A8, qscale,
                        stride, K8, Bw, Sb, chunks, R, Q, down_shift, scale_inv, R_total, out, static_cast<int*>(nullptr), bias,
                        1, 0LL, static_cast<const long long*>(nullptr), key_tiled,
                        static_cast<const unsigned char*>(g_warm_ptr), static_cast<long long>(g_warm_bytes / 128),
@@ -1524,14 +1549,20 @@ static void launch_mfma_i8_t(int ndig, long long dig_stride, const long long* ke
                              int64_t R, int64_t Q, int down_shift, float scale_inv, int64_t R_total, float* out,
                              int32_t* chunk_ints, const float* bias, hipStream_t st) {
     if (ndig > 0)
-        launch_mfma_i8_tm<TM, TN, kI8Sum>(A8, qscale, stride, K8, Bw, Sb, chunks, R, Q, down_shift, scale_inv, R_total,
+        launch_mfma_i8_tm<TM, TN, kI8Sum, false, false>(A8, qscale, stride, K8, Bw, Sb, chunks, R, Q, down_shift, scale_inv, R_total,
                                           out, chunk_ints, bias, st, ndig, dig_stride, key_indices, key_tiled);
     else if (chunk_ints)
-        launch_mfma_i8_tm<TM, TN, kI8Ints>(A8, qscale, stride, K8, Bw, Sb, chunks, R, Q, down_shift, scale_inv, R_total,
+        launch_mfma_i8_tm<TM, TN, kI8Ints, false, false>(A8, qscale, stride, K8, Bw, Sb, chunks, R, Q, down_shift, scale_inv, R_total,
                                            out, chunk_ints, bias, st, 1, 0, nullptr, key_tiled);
-    else
-        launch_mfma_i8_tm<TM, TN, kI8Chain>(A8, qscale, stride, K8, Bw, Sb, chunks, R, Q, down_shift, scale_inv,
-                                            R_total, out, chunk_ints, bias, st, 1, 0, nullptr, key_tiled);
+    else {
+        const bool half = t_out_dtype != BSI_DTYPE_F32, four = i8_four_scales(stride);
+#define BSI_I8_CHAIN(four_, half_) \
+    launch_mfma_i8_tm<TM, TN, kI8Chain, four_, half_>(A8, qscale, stride, K8, Bw, Sb, chunks, R, Q, down_shift, scale_inv, R_total, out, \
+                                                      chunk_ints, bias, st, 1, 0, nullptr, key_tiled)
+        if (four) half ? BSI_I8_CHAIN(true, true) : BSI_I8_CHAIN(true, false);
+        else half ? BSI_I8_CHAIN(false, true) : BSI_I8_CHAIN(false, false);
+#undef BSI_I8_CHAIN
+    }
 }
 
 // The 128 x 128 tile on four MFMA waves of 64 x 64 with one accumulator set, and four loader waves (tile 1284; chain
@@ -1661,13 +1692,15 @@ void launch_mfma_i8(const int8_t* A8, const float* qscale, int stride, const int
         int segments = 1;
         const int split_tile = choose_i8_split(R, Q, chunks, &segments);
         if (split_tile == 128) {
-            launch_mfma_i8_split<128, 128>(segments, t_split_scratch, A8, qscale, stride, K8, Bw, Sb, chunks, R, Q, down_shift,
-                                           scale_inv, R_total, out, bias, st, key_tiled);
+            (t_out_dtype != BSI_DTYPE_F32 ? &launch_mfma_i8_split<128, 128, true> : &launch_mfma_i8_split<128, 128, false>)(
+                segments, t_split_scratch, A8, qscale, stride, K8, Bw, Sb, chunks, R, Q, down_shift, scale_inv, R_total, out, bias, st,
+                key_tiled);
             return;
         }
         if (split_tile == 12864) {
-            launch_mfma_i8_split<128, 64>(segments, t_split_scratch, A8, qscale, stride, K8, Bw, Sb, chunks, R, Q, down_shift,
-                                          scale_inv, R_total, out, bias, st, key_tiled);
+            (t_out_dtype != BSI_DTYPE_F32 ? &launch_mfma_i8_split<128, 64, true> : &launch_mfma_i8_split<128, 64, false>)(
+                segments, t_split_scratch, A8, qscale, stride, K8, Bw, Sb, chunks, R, Q, down_shift, scale_inv, R_total, out, bias, st,
+                key_tiled);
             return;
         }
     }
