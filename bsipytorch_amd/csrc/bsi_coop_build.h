@@ -62,8 +62,26 @@ inline int coop_shares(unsigned groups, int pieces) {
     return shares < 1 ? 1 : shares;
 }
 
+// Where dword `lane` of a (row, chunk) item lies in a copy, in dwords.  kFragments: in the order in which the few-rows kernel
+// takes its operands -- 16 rows at a time, then chunk, MFMA, quarter of its 64 elements, row -- so that each of its loads is one
+// run of up to 1 KiB; from rows one after the other a load takes 16 bytes out of every 64 of 16 rows, 32 lines.
+template <bool kFragments>
+__device__ __forceinline__ int coop_image_at(const CoopBuild& b, int row, int chunk, int lane) {
+    if (!kFragments) return (row * b.chunks + chunk) * 64 + lane;
+    const int first = row & ~15, rows = b.rows - first < 16 ? b.rows - first : 16;
+    return first * b.chunks * 64 + (((chunk * 4 + (lane >> 2 & 3)) * 4 + (lane >> 4)) * rows + (row & 15)) * 4 + (lane & 3);
+}
+
+// Where its scale lies: beside those of the chunk's other rows (kFragments), or of the row's other chunks.
+template <bool kFragments>
+__device__ __forceinline__ int coop_scale_at(const CoopBuild& b, int row, int chunk) {
+    if (!kFragments) return row * b.chunks + chunk;
+    const int first = row & ~15, rows = b.rows - first < 16 ? b.rows - first : 16;
+    return first * b.chunks + chunk * rows + (row & 15);
+}
+
 // Row scales: the row's largest magnitude over the waves, then its quantised chunks.
-template <typename T, bool kVec>
+template <typename T, bool kVec, bool kFragments>
 __device__ void coop_build_share(const CoopBuild& b, int share, int wave, int nwaves, int lane, uint32_t* __restrict__ image,
                                  float* __restrict__ scales, unsigned* __restrict__ wave_max) {
     const ChunkLane cl = chunk_lane(lane);
@@ -77,6 +95,7 @@ __device__ void coop_build_share(const CoopBuild& b, int share, int wave, int nw
             load_chunk_quad<T, kVec>(x + row * b.d, b.d, item - row * b.chunks, cl, v);
         };
         auto emit = [&](int item, const float (&v)[4]) {
+            const int row = item / b.chunks;
             const unsigned mx = wave_max_u32(quad_max_bits(v));
             int shift;
             uint32_t bytes;
@@ -87,8 +106,8 @@ __device__ void coop_build_share(const CoopBuild& b, int share, int wave, int nw
                 shift = compute_shift(wave_max_u64(quad_max_wide(v, b.dec_scale)), 0.0, 1, b.slices, 0.0f);
                 bytes = quantise_quad_wide(v, b.dec_scale, shift, b.slices);
             }
-            image[item * 64 + lane] = chunk_image_dword(bytes, cl);
-            if (lane == 0) scales[item] = static_cast<float>(1ULL << shift);
+            image[coop_image_at<kFragments>(b, row, item - row * b.chunks, lane)] = chunk_image_dword(bytes, cl);
+            if (lane == 0) scales[coop_scale_at<kFragments>(b, row, item - row * b.chunks)] = static_cast<float>(1ULL << shift);
         };
 #pragma unroll 1
         for (int item = first + wave; item < last; item += nwaves) {
@@ -138,7 +157,7 @@ __device__ void coop_build_share(const CoopBuild& b, int share, int wave, int nw
                 load_chunk_quad<T, kVec>(xrow, b.d, c, cl, v);
             }
             const uint32_t bytes = wide ? quantise_quad_wide(v, b.dec_scale, shift, b.slices) : quantise_quad<T>(v, b.scale, shift, range);
-            image[(row * b.chunks + c) * 64 + lane] = chunk_image_dword(bytes, cl);
+            image[coop_image_at<kFragments>(b, row, c, lane)] = chunk_image_dword(bytes, cl);
         }
     }
 }
@@ -147,7 +166,7 @@ __device__ void coop_build_share(const CoopBuild& b, int share, int wave, int nw
 // to the whole build, in the copy of the XCD the workgroup runs on.  ahead(): loads for after the build, of anything but the
 // area.  Every wave but wave 0 issues them when the workgroup's share is built (a CU's loads return in order: not before),
 // wave 0, which asks for the flags, when all shares are.
-template <typename F>
+template <bool kFragments, typename F>
 __device__ __forceinline__ void coop_build(const CoopBuild& b, unsigned id, unsigned* __restrict__ shared, const int8_t*& A8,
                                            const float*& qscale, F&& ahead) {
     const int lane = threadIdx.x & (BSI_WAVE - 1);
@@ -161,14 +180,14 @@ __device__ __forceinline__ void coop_build(const CoopBuild& b, unsigned id, unsi
     bool issued = false;
     auto build = [&](int share) {
         if (b.dtype == BSI_DTYPE_F32) {
-            if (b.vec) coop_build_share<float, true>(b, share, wave, nwaves, lane, image, scales, shared);
-            else coop_build_share<float, false>(b, share, wave, nwaves, lane, image, scales, shared);
+            if (b.vec) coop_build_share<float, true, kFragments>(b, share, wave, nwaves, lane, image, scales, shared);
+            else coop_build_share<float, false, kFragments>(b, share, wave, nwaves, lane, image, scales, shared);
         } else if (b.dtype == BSI_DTYPE_F16) {
-            if (b.vec) coop_build_share<__half, true>(b, share, wave, nwaves, lane, image, scales, shared);
-            else coop_build_share<__half, false>(b, share, wave, nwaves, lane, image, scales, shared);
+            if (b.vec) coop_build_share<__half, true, kFragments>(b, share, wave, nwaves, lane, image, scales, shared);
+            else coop_build_share<__half, false, kFragments>(b, share, wave, nwaves, lane, image, scales, shared);
         } else {
-            if (b.vec) coop_build_share<__hip_bfloat16, true>(b, share, wave, nwaves, lane, image, scales, shared);
-            else coop_build_share<__hip_bfloat16, false>(b, share, wave, nwaves, lane, image, scales, shared);
+            if (b.vec) coop_build_share<__hip_bfloat16, true, kFragments>(b, share, wave, nwaves, lane, image, scales, shared);
+            else coop_build_share<__hip_bfloat16, false, kFragments>(b, share, wave, nwaves, lane, image, scales, shared);
         }
         const int items = b.rows * b.chunks, had = items * (share + 1) / b.shares - items * share / b.shares;
         if (b.by_row || wave < had) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the wave's stores have reached the L2

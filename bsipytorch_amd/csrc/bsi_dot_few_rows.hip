@@ -22,7 +22,12 @@ namespace bsi {
 
 constexpr int kStreamLdsInts = 16384;  // at most 64 KiB of chunk accumulators per pass
 
-// kBuild: the queries are quantised by this launch (bsi_coop_build.h); A8 and qscale are not looked at.  Only those instances
+// kBuild: the queries are quantised by this launch (bsi_coop_build.h); A8 and qscale are not looked at.  The copy lies in the
+// order of the operand loads (coop_image_at: up to 1 KiB in one run a load, where rows one after the other are 32 lines a load and
+// the loads of 32 rows take longer than the key planes they are for), and a wave takes a chunk's scales with its operands and
+// leaves them in LDS, so that the chain asks memory for nothing.  us a layer, rows and the chain's own loads before, then now:
+// 16 x 4096 x 4096 bf16 8.7, 7.85; 32 x 4096 x 4096 11.05, 8.95; 32 x 8192 x 4096 f16 16.5, 12.4; 16 x 8192 x 4096 12.1, 10.5;
+// 24 x 2048 x 2048 f32 6.95, 6.25; 8 x 4096 x 4096 7.8, 7.6.  Only those instances
 // take the build's description: with it the workgroup's size, which lies behind the arguments, is in another cache line of
 // them, and its fetch holds up every wave's first key load.  us, with and without: 16 x 4096 x 16384 12.3, 11.8; 16 x 4096 x
 // 4096 5.25, 5.09; 1 x 4096 x 16384 10.5, 10.2; 1 x 16384 x 4096 11.1, 10.9 (1 x 4096 x 4096 4.06, 4.11).
@@ -33,8 +38,10 @@ __global__ __launch_bounds__(1024) void dot_mfma_stream_kernel(
     const float* __restrict__ Bw, int chunks, int pass_chunks, int64_t R, int64_t Q, int down_shift, float scale_inv,
     int64_t R_total, float* __restrict__ out, int* __restrict__ chunk_ints, const float* __restrict__ bias, int out_dtype,
     std::conditional_t<kBuild, CoopBuild, int> coop) {
-    extern __shared__ __attribute__((aligned(16))) int ints[];  // [pass_chunks][KT][NT][16 queries][16 keys]
+    // [pass_chunks][KT][NT][16 queries][16 keys]; kBuild: then the chunks' scales, [pass_chunks][NT][16 queries]
+    extern __shared__ __attribute__((aligned(16))) int ints[];
     constexpr int kSlot = KT * NT * 256;
+    float* const chunk_scales = reinterpret_cast<float*>(ints + static_cast<size_t>(pass_chunks) * kSlot);
 
     const int tid = threadIdx.x;
     const int lane = tid & 63;
@@ -63,7 +70,7 @@ __global__ __launch_bounds__(1024) void dot_mfma_stream_kernel(
             }
     };
     if constexpr (kBuild)
-        coop_build(coop, blockIdx.x, reinterpret_cast<unsigned*>(ints), A8, qscale, [&] { load_keys(wave < pass_chunks ? wave : pass_chunks - 1); });
+        coop_build<true>(coop, blockIdx.x, reinterpret_cast<unsigned*>(ints), A8, qscale, [&] { load_keys(wave < pass_chunks ? wave : pass_chunks - 1); });
 
     // the chain lanes: tid <-> (key tile, query tile, query, key), keys fastest so output stores are contiguous
     float accf = 0.0f;
@@ -83,13 +90,20 @@ __global__ __launch_bounds__(1024) void dot_mfma_stream_kernel(
         for (; c < pend; c += nwaves) {
             // query operands of this chunk (L2 resident), then the key planes of the wave's next chunk
             v4i qb[NT][4];
+            float qs[NT];
 #pragma unroll
             for (int t = 0; t < NT; ++t) {
                 const int64_t q = q0 + t * 16 + ln;
+                qs[t] = 0.0f;
                 if (q < Q) {
-                    const v4i* src = reinterpret_cast<const v4i*>(A8 + static_cast<size_t>(q) * arow + c * 256 + lg * 64);
+                    const int rows = Q - t * 16 < 16 ? static_cast<int>(Q) - t * 16 : 16;  // kBuild: coop_image_at's order
+                    const v4i* src = reinterpret_cast<const v4i*>(
+                        kBuild ? A8 + static_cast<size_t>(t) * 16 * arow + ((c * 16 + lg) * rows + ln) * 16
+                               : A8 + static_cast<size_t>(q) * arow + c * 256 + lg * 64);
+                    const int step = kBuild ? 4 * rows : 1;
+                    if constexpr (kBuild) qs[t] = qscale[coop.by_row ? t * 16 + ln : t * 16 * chunks + c * rows + ln];
 #pragma unroll
-                    for (int m = 0; m < 4; ++m) qb[t][m] = src[m];
+                    for (int m = 0; m < 4; ++m) qb[t][m] = src[m * step];
                 } else {
 #pragma unroll
                     for (int m = 0; m < 4; ++m) qb[t][m] = (v4i){0, 0, 0, 0};
@@ -125,6 +139,10 @@ __global__ __launch_bounds__(1024) void dot_mfma_stream_kernel(
                     *reinterpret_cast<v4i*>(&ints[(c - p0) * kSlot + (k * NT + t) * 256 + ln * 16 + lg * 4]) = acc;
                 }
             }
+            if (kBuild && lg == 0) {
+#pragma unroll
+                for (int t = 0; t < NT; ++t) chunk_scales[((c - p0) * NT + t) * 16 + ln] = qs[t];
+            }
             if (cnext < pend) {
 #pragma unroll
                 for (int k = 0; k < KT; ++k)
@@ -135,7 +153,7 @@ __global__ __launch_bounds__(1024) void dot_mfma_stream_kernel(
         __syncthreads();
         if (cvalid) {
             accf = chain_chunks(accf, p0, pend, down, [&](int cc) { return ints[(cc - p0) * kSlot + tid]; },
-                                [&](int cc) { return csrc[cc * sstep]; });
+                                [&](int cc) { return kBuild ? chunk_scales[((cc - p0) * NT + ct) * 16 + cn] : csrc[cc * sstep]; });
             if (kInts)
                 for (int cc = p0; cc < pend; ++cc)
                     chunk_ints[(cq * R + cr) * chunks + cc] = ints[(cc - p0) * kSlot + tid] >> down_shift;
@@ -537,7 +555,7 @@ static void launch_mfma_stream(const int8_t* A8, const float* qscale, int stride
     const int waves = stream_waves(grid.x * grid.y, chunks, kSlot);
     int pass_chunks = kStreamLdsInts / kSlot;
     if (pass_chunks > chunks) pass_chunks = chunks;
-    const size_t lds = static_cast<size_t>(pass_chunks) * kSlot * sizeof(int);
+    size_t lds = static_cast<size_t>(pass_chunks) * kSlot * sizeof(int);
 #define BSI_STREAM_GO(INTS, BUILD, COOP)                                                                                      \
     launch((dot_mfma_stream_kernel<NT, KT, INTS, BUILD>), grid, dim3(waves * 64), lds, st, A8, qscale, stride,                \
            reinterpret_cast<const unsigned long long*>(B), Bw, chunks, pass_chunks, R, Q, down_shift, scale_inv, R_total, out, \
@@ -547,6 +565,9 @@ static void launch_mfma_stream(const int8_t* A8, const float* qscale, int stride
     else {
         CoopBuild coop = *t_coop;
         coop.shares = coop_shares(grid.x, coop.by_row ? coop.rows : coop.rows * coop.chunks);
+        static LdsOptIn once;
+        lds_opt_in(once, reinterpret_cast<const void*>(&dot_mfma_stream_kernel<NT, KT, false, true>), kStreamLdsInts * 4 + 4096);
+        lds += static_cast<size_t>(pass_chunks) * NT * 16 * sizeof(float);
         BSI_STREAM_GO(false, true, coop);
     }
 #undef BSI_STREAM_GO

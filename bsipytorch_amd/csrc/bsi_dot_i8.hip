@@ -548,7 +548,7 @@ __global__ __launch_bounds__((I8Cfg<TM, TN>::kBlock)) void dot_mfma_i8_kernel(
     constexpr int WM = C::kWM, WN = C::kWN;
     constexpr bool kInts = (kMode == kI8Ints), kSum = (kMode == kI8Sum);
     extern __shared__ __attribute__((aligned(16))) unsigned char lds[];  // C::kLds
-    if (kBuild) coop_build(coop, blockIdx.y * gridDim.x + blockIdx.x, reinterpret_cast<unsigned*>(lds), A8, qscale, [] {});
+    if (kBuild) coop_build<false>(coop, blockIdx.y * gridDim.x + blockIdx.x, reinterpret_cast<unsigned*>(lds), A8, qscale, [] {});
 
     const int tid = threadIdx.x;
     const int lane = tid & 63;
