@@ -47,8 +47,8 @@ extern "C" int bsi_hip_set_option(int option, int value) {
             g_digits_route = value;
             return BSI_OK;
         case BSI_OPT_I8_TILE:
-            BSI_REQUIRE(value == 0 || value == 128 || value == 1284 || value == 12864 || value == 64 || value == 6432,
-                        "tile must be 0, 128, 1284, 12864, 64 or 6432");
+            BSI_REQUIRE(value == 0 || value == 128 || value == 1284 || value == 12864 || value == 64 || value == 6432 || value == 256,
+                        "tile must be 0, 128, 1284, 12864, 64, 6432 or 256");
             g_i8_tile = value;
             return BSI_OK;
         case BSI_OPT_OUTPUT_STORES:
@@ -297,7 +297,7 @@ extern "C" int bsi_hip_dot_static_scratch(const uint64_t* A, const float* A_chun
 
 // Workspace of bsi_hip_linear: the query operands of one build (planes, shifts, scales, int8 image), each 256-aligned.
 struct LinearWorkspace {
-    size_t words, shifts, scales, ints8, total;
+    size_t words, shifts, scales, ints8, large, total;  // large: what the integer sums of a large layer take
 };
 static LinearWorkspace linear_workspace(int64_t Q, int64_t d, int fixed_bits) {
     const size_t W = static_cast<size_t>((d + 63) / 64), chunks = static_cast<size_t>((d + 255) / 256);
@@ -307,7 +307,8 @@ static LinearWorkspace linear_workspace(int64_t Q, int64_t d, int fixed_bits) {
     w.shifts = up(static_cast<size_t>(Q) * fixed_bits * W * 8);
     w.scales = w.shifts + up(static_cast<size_t>(Q) * chunks * 4);
     w.ints8 = w.scales + up(static_cast<size_t>(Q) * chunks * 4);
-    w.total = w.ints8 + up(static_cast<size_t>(Q) * chunks * 256);
+    w.large = w.ints8 + up(static_cast<size_t>(Q) * chunks * 256);
+    w.total = w.large + i8_large_workspace_bytes(Q, static_cast<int>(chunks < (1 << 20) ? chunks : 1 << 20));
     return w;
 }
 
@@ -353,6 +354,20 @@ extern "C" int bsi_hip_linear_out(const void* x, int dtype, int64_t Q, int64_t d
         if (rc != BSI_OK) return rc;
     }
     t_out_dtype = out_dtype;
+    if (core == BSI_CORE_AUTO && b_layout == BSI_LAYOUT_INT8 && Sb >= 2 && Sb <= 8 && R_total >= R && R <= (1 << 25) && B != nullptr && Bw != nullptr &&
+        out != nullptr && (reinterpret_cast<uintptr_t>(B) & 15) == 0 && i8_large_serves(Q, R, chunks)) {
+        g_warm_ptr = warm;
+        g_warm_bytes = warm != nullptr ? warm_bytes : 0;
+        t_layer_output = 1;
+        launch_i8_large(ws + w.large, ints8, scales, chunk_scale ? chunks : 1, reinterpret_cast<const int8_t*>(B), Bw, fixed_bits, Sb, chunks, R, Q,
+                        scale_inv, R_total, static_cast<float*>(out), bias, as_stream(stream));
+        g_warm_ptr = nullptr;
+        g_warm_bytes = 0;
+        t_layer_output = 0;
+        t_out_dtype = BSI_DTYPE_F32;
+        BSI_LAUNCH_CHECK("dot_mfma_i8_large_kernel");
+        return BSI_OK;
+    }
     const int rc = bsi_hip_dot_bias_warm(planes ? words : nullptr, ints8, scales, chunk_scale ? chunks : 1, fixed_bits, W64, B, b_layout,
                                          Bw, Sb, R, Q, scale_inv, R_total, bias, static_cast<float*>(out), core, nullptr, 0, warm,
                                          warm_bytes, stream);

@@ -3,6 +3,8 @@
 #include "bsi_coop_build.h"
 #include "bsi_dot_internal.h"
 
+#include <type_traits>
+
 namespace bsi {
 
 // process-wide options set through bsi_hip_set_option (meanings beside their declarations in bsi_dot_internal.h)
@@ -97,6 +99,7 @@ struct I8Cfg {
     static_assert(kConsumers < 15, "flag words of the MFMA waves, then the decision word");
 };
 constexpr int kSplitLeave = 0, kSplitCombine = 1, kSplitRedo = 2;
+constexpr int kLargeTile = 256;  // dot_mfma_i8_large_kernel: keys and queries of a workgroup
 
 // How the chunk scales are fetched (kFour of the kernels): one float of each of 64 queries for every chunk, or four consecutive
 // floats of 16 queries, for the group of four chunks after the one a load is issued in.  The scales of a query are contiguous:
@@ -1046,18 +1049,24 @@ __device__ __forceinline__ void i8_tiles_loader_wave(unsigned char* __restrict__
     }
 }
 
-template <int TM, int TN, bool kHalf>
+template <int TM, int TN, bool kHalf, bool kLeft>
 __global__ __launch_bounds__((I8Cfg<TM, TN>::kBlock)) void dot_mfma_i8_tiles_kernel(
     const int8_t* __restrict__ A8, const float* __restrict__ qscale, int qscale_stride, const int8_t* __restrict__ K8,
     const float* __restrict__ Bw, int Sb, int chunks, int64_t R, int64_t Q, int down_shift, float scale_inv, int64_t R_total,
     float* __restrict__ out, const float* __restrict__ bias, int key_tiled, const unsigned char* __restrict__ warm,
-    long long warm_lines, int out_stream, I8Grid grid, unsigned tiles, int out_dtype) {
+    long long warm_lines, int out_stream, I8Grid grid, unsigned tiles, int out_dtype, std::conditional_t<kLeft, const unsigned*, int> left) {
+    // kLeft: only if dot_mfma_i8_large_kernel, before this launch, has left a tile of 256 queries to it (`left`, a word for each)
     using C = I8Cfg<TM, TN>;
     constexpr int WM = C::kWM, WN = C::kWN, kMode = kI8Chain;
     extern __shared__ __attribute__((aligned(16))) unsigned char lds[];  // I8TilesCfg::kLdsTiles
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    if constexpr (kLeft) {  // every wave looks for itself
+        unsigned any = 0u;
+        for (int64_t t = lane; t * kLargeTile < Q; t += 64) any |= left[t];
+        if (__ballot(any != 0u) == 0ull) return;
+    }
     if (wave >= C::kConsumers) {
         const int lw = wave - C::kConsumers;
         i8_tiles_loader_wave<C>(lds, lw, lane, A8, qscale, qscale_stride, K8, Bw, Sb, chunks, R, Q, bias, key_tiled, grid, tiles);
@@ -1179,6 +1188,351 @@ __global__ __launch_bounds__((I8Cfg<TM, TN>::kBlock)) void dot_mfma_i8_tiles_ker
 #undef BSI_TILES_CHUNK
 #undef BSI_I8_KSTEP_AT
 #undef BSI_TILES_SCALES
+}
+
+// ------------------------------------------------------------------ int8 image, 256 x 256 tiles of plain integer sums
+//
+// Large layers.  A chunk's scale is a power of two, and the integers of a row times its chunks' scales are multiples of the
+// smallest of them: written in that unit, most are int8 still -- the chunks of a row differ by a factor of two, the int8 image
+// has a bit to spare -- and the few that are not (outlier columns) keep their upper digit in a second image of which only the
+// blocks of 64 elements are read that have one.  The dot is then ONE int32 sum over the row, and if the row's magnitudes
+// times the largest key magnitude add up to no more than 2^24 units, every value the fp32 chain over the chunks takes is an
+// integer of at most 24 bits: it never rounds, and the sum is its result, bit for bit.  i8_units_kernel writes the images, the
+// masks of the blocks and the rows' units and checks that bound; a tile of queries with a row outside it, or with more
+// than a quarter of its blocks in the second image, is left to the chain, in a launch behind this one that otherwise ends at once.
+//
+// Without the chain there are no second accumulators and no scales, a wave holds 128 x 64 outputs and a workgroup 256 x 256:
+// half the bytes from the L2 and two thirds of the LDS reads a multiply-add, both of which the clock pays for.  Eight waves that load
+// for themselves (eight loads a half-chunk among 64 MFMAs; two waves a SIMD leave room for no others); LDS is a ring of five
+// slots of an operand's half-chunk, 256 rows x 128 bytes: K runs three stages ahead, Q two.
+// us a layer with its build, tiles of 128 x 128 and now: 4096 x 4096 x 16384 bf16 303, 260 (this kernel 222, 279 k cycles of its 504 k
+// with the matrix pipes busy); 2048 x 8192 x 8192 f32 161, 139; 2048 x 2048 x 16384 bf16 88.6, 84.4.  What is left: 400 cycles of
+// each half-chunk's 2450 at its barrier, the stores at the end of a round of tiles, the clock (2.1 GHz).  Tried beside it: touching
+// lines of later stages ahead of their loads (260 -> 275, the loads are not what is waited for), the loads in one run behind the
+// barrier (260 -> 267 -> 275 with their offsets worked out there too).
+constexpr int kLargeSlot = kLargeTile * 128, kLargeSlots = 5, kLargeLds = kLargeSlots * kLargeSlot;
+constexpr int kLargeMaskWords = 4, kLargeMaxChunks = 16 * kLargeMaskWords;  // 64-element blocks of a row, 64 a word
+constexpr uint32_t kNowhere = 0x80000000u;  // past the end of every operand
+
+// The images in units and what the dot needs to know of a row.  lo / hi: [Q][chunks * 256]; masks: [Q][words] of 64 blocks;
+// units: [Q], the factor of the row's sums, negative where the row has to go through the chain.
+constexpr int kUnitsBlock = 256, kUnitsHeld = kLargeMaxChunks * 16 / kUnitsBlock;
+__global__ __launch_bounds__(kUnitsBlock) void i8_units_kernel(const int8_t* __restrict__ A8, const float* __restrict__ qscale, int stride,
+                                                               int chunks, int Sa, int Sb, uint4* __restrict__ lo, uint4* __restrict__ hi,
+                                                               unsigned short* __restrict__ masks, float* __restrict__ units) {
+    constexpr int kUnitsWaves = kUnitsBlock / 64;
+    __shared__ unsigned shared[3][kUnitsWaves];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int64_t row = blockIdx.x;
+    const int pieces = chunks * 16, mask_pieces = (chunks * 4 + 63) / 64 * 4;  // of 16 bytes; of 16 mask bits
+    const uint4* const src = reinterpret_cast<const uint4*>(A8) + row * pieces;
+    const float* const scales = qscale + row * stride;
+    uint4 v[kUnitsHeld];
+    unsigned exponent[kUnitsHeld], least = 255u, odd = 0u;  // of the scales of pieces that are not all zero
+#pragma unroll
+    for (int j = 0; j < kUnitsHeld; ++j) {
+        const int p = tid + j * kUnitsBlock;
+        v[j] = make_uint4(0u, 0u, 0u, 0u);
+        exponent[j] = 255u;
+        if (p >= pieces) continue;
+        v[j] = src[p];
+        const unsigned bits = __float_as_uint(scales[stride == 1 ? 0 : p >> 4]);
+        if ((v[j].x | v[j].y | v[j].z | v[j].w) == 0u) continue;
+        if ((bits & 0x807FFFFFu) != 0u || bits < 0x20000000u || bits >= 0x60000000u) odd = 1u;  // no power of two, or a far one
+        exponent[j] = bits >> 23 & 255u;
+        least = exponent[j] < least ? exponent[j] : least;
+    }
+    least = ~wave_max_u32(~least);
+    if (lane == 0) shared[0][wave] = least;
+    __syncthreads();
+#pragma unroll
+    for (int w = 0; w < kUnitsWaves; ++w) least = shared[0][w] < least ? shared[0][w] : least;
+    unsigned total = 0u;  // of the row's magnitudes, in units: at most 2^14 elements of 2^15
+#pragma unroll
+    for (int j = 0; j < kUnitsHeld; ++j) {
+        const int p = tid + j * kUnitsBlock, at = wave + j * kUnitsWaves;
+        if (at >= mask_pieces) break;  // the whole wave
+        int up = exponent[j] == 255u ? 0 : static_cast<int>(exponent[j] - least) - (8 - Sa);  // the image holds a << (8 - Sa)
+        if (up > 8) {
+            odd = 1u;
+            up = 8;
+        }
+        const int left = up > 0 ? up : 0, right = up < 0 ? -up : 0;
+        uint32_t l[4], h[4];
+        const uint32_t in[4] = {v[j].x, v[j].y, v[j].z, v[j].w};
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            l[i] = h[i] = 0u;
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                const int a = ((static_cast<int>(in[i] << (24 - 8 * k)) >> 24) << left) >> right;
+                const int low = static_cast<int>(static_cast<uint32_t>(a) << 24) >> 24;
+                total += static_cast<unsigned>(a < 0 ? -a : a);
+                l[i] |= (static_cast<uint32_t>(a) & 255u) << (8 * k);
+                h[i] |= (static_cast<uint32_t>((a - low) >> 8) & 255u) << (8 * k);
+            }
+        }
+        // four neighbouring lanes hold a block of 64 elements
+        const unsigned long long any = __ballot((h[0] | h[1] | h[2] | h[3]) != 0u);
+        unsigned long long m = (any | any >> 1 | any >> 2 | any >> 3) & 0x1111111111111111ull;
+        m = (m | m >> 3) & 0x0303030303030303ull;
+        m = (m | m >> 6) & 0x000F000F000F000Full;
+        m = (m | m >> 12) & 0x000000FF000000FFull;
+        m = (m | m >> 24) & 0xFFFFull;
+        if (lane == 0) masks[row * mask_pieces + at] = static_cast<unsigned short>(m);
+        if (p < pieces) {
+            lo[row * pieces + p] = make_uint4(l[0], l[1], l[2], l[3]);
+            hi[row * pieces + p] = make_uint4(h[0], h[1], h[2], h[3]);
+        }
+    }
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) total += __shfl_xor(total, o, BSI_WAVE);
+    const bool any_odd = __ballot(odd != 0u) != 0ull;
+    if (lane == 0) {
+        shared[1][wave] = total;
+        shared[2][wave] = any_odd ? 1u : 0u;
+    }
+    __syncthreads();
+    if (tid == 0) {
+        unsigned long long sum = 0ull;
+        unsigned bad = 0u;
+        for (int w = 0; w < kUnitsWaves; ++w) {
+            sum += shared[1][w];
+            bad |= shared[2][w];
+        }
+        if (least == 255u) least = 127u;  // a row of zeros
+        // the key image holds b << (8 - Sb), |b| <= 2^(Sb - 1)
+        units[row] = bad != 0u || (sum << (Sb - 1)) > (1ull << 24) ? -1.0f : __uint_as_float((least - static_cast<unsigned>(8 - Sb)) << 23);
+    }
+}
+
+// The stages of a tile: its blocks in the upper image, two of any place a stage, then the half-chunks of the lower one.
+struct LargeStages {
+    unsigned long long mask[kLargeMaskWords];
+    int base, upper, half, halves;  // first block of mask[0]; stages left in the upper image; half-chunk to come; of the row
+    __device__ __forceinline__ uint32_t block() {  // byte offset inside a row of the next block of the upper image
+#pragma unroll
+        for (int i = 0; i < kLargeMaskWords; ++i)
+            if (mask[0] == 0ull) {
+#pragma unroll
+                for (int w = 0; w + 1 < kLargeMaskWords; ++w) mask[w] = mask[w + 1];
+                mask[kLargeMaskWords - 1] = 0ull;
+                base += 64;
+            }
+        if (mask[0] == 0ull) return kNowhere;
+        const int bit = __builtin_ctzll(mask[0]);
+        mask[0] &= mask[0] - 1ull;
+        return static_cast<uint32_t>(base + bit) * 64u;
+    }
+    // the next stage: where its two 64-byte columns lie, and whether in the upper image
+    __device__ __forceinline__ bool next(uint32_t& first, uint32_t& second) {
+        if (upper > 0) {
+            --upper;
+            first = block();
+            second = block();
+            return true;
+        }
+        first = half < halves ? static_cast<uint32_t>(half) * 128u : kNowhere;
+        second = first + 64u;
+        ++half;
+        return false;
+    }
+};
+
+template <bool kHalf>
+__global__ __launch_bounds__(512, 2) void dot_mfma_i8_large_kernel(
+    const int8_t* lo, const int8_t* hi, const unsigned long long* __restrict__ masks, const float* __restrict__ units, const int8_t* K8,
+    const float* __restrict__ Bw, int Sb, int chunks, int64_t R, int64_t Q, float scale_inv, int64_t R_total, float* __restrict__ out,
+    const float* __restrict__ bias, const unsigned char* __restrict__ warm, long long warm_lines, int out_stream, I8Grid grid, int out_dtype,
+    unsigned* __restrict__ left) {
+    extern __shared__ __attribute__((aligned(16))) unsigned char lds[];  // kLargeLds
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wr = wave & 1, wq = wave >> 1, ln = lane & 15, lg = lane >> 4;
+    int bx, by;
+    i8_tile_of(grid, blockIdx.x, bx, by);
+    const int64_t r0 = static_cast<int64_t>(bx) * kLargeTile, q0 = static_cast<int64_t>(by) * kLargeTile;
+    const uint32_t rowbytes = static_cast<uint32_t>(chunks) << 8;
+    const bsi_rsrc rk = make_rsrc(K8 + static_cast<size_t>(r0) * rowbytes, static_cast<size_t>(R - r0) * rowbytes);
+    const bsi_rsrc rlo = make_rsrc(lo + static_cast<size_t>(q0) * rowbytes, static_cast<size_t>(Q - q0) * rowbytes);
+    const bsi_rsrc rhi = make_rsrc(hi + static_cast<size_t>(q0) * rowbytes, static_cast<size_t>(Q - q0) * rowbytes);
+
+    // which blocks of the tile's rows are in the upper image, and whether the chain has to take them
+    LargeStages stages;
+    {
+        const int words = (chunks * 4 + 63) / 64;
+        unsigned long long* const ored = reinterpret_cast<unsigned long long*>(lds);
+        if (tid <= kLargeMaskWords) ored[tid] = 0ull;  // the last: a row for the chain
+        __syncthreads();
+        const int64_t q = q0 + tid;
+        const bool mine = tid < kLargeTile && q < Q;
+        if (wave < kLargeTile / 64) {
+#pragma unroll
+            for (int w = 0; w < kLargeMaskWords; ++w) {
+                unsigned long long m = mine && w < words ? masks[q * words + w] : 0ull;
+                if (__ballot(m != 0ull) == 0ull) continue;
+#pragma unroll
+                for (int o = 32; o > 0; o >>= 1) m |= __shfl_xor(m, o, BSI_WAVE);
+                if (lane == 0) atomicOr(ored + w, m);
+            }
+            if (__ballot(mine && units[q] < 0.0f) != 0ull && lane == 0) atomicOr(ored + kLargeMaskWords, 1ull);
+        }
+        __syncthreads();
+        const int bad = __builtin_amdgcn_readfirstlane(static_cast<int>(ored[kLargeMaskWords]));
+        int blocks = 0;
+#pragma unroll
+        for (int w = 0; w < kLargeMaskWords; ++w) {
+            const unsigned long long m = ored[w];
+            const unsigned a = __builtin_amdgcn_readfirstlane(static_cast<int>(static_cast<unsigned>(m)));
+            const unsigned b = __builtin_amdgcn_readfirstlane(static_cast<int>(static_cast<unsigned>(m >> 32)));
+            stages.mask[w] = static_cast<unsigned long long>(b) << 32 | a;
+            blocks += __builtin_popcountll(stages.mask[w]);
+        }
+        const bool leave = bad != 0 || blocks > chunks;  // a quarter of the 4 chunks blocks
+        if (bx == 0 && tid == 0) left[by] = leave ? 1u : 0u;
+        if (leave) return;
+        stages.base = stages.half = 0;
+        stages.upper = (blocks + 1) / 2;
+        stages.halves = 2 * chunks;
+        __syncthreads();  // the masks have been read: the ring may be written
+    }
+    const int uppers = stages.upper;
+
+    // loads: a wave moves rows 32 wave .. + 31 of an operand's stage, four loads of 8 rows x 128 bytes; lane = (row of the eight,
+    // 16-byte column), columns swizzled as in dot_mfma_i8_kernel
+    const uint32_t lr = static_cast<uint32_t>(lane) >> 3, lc = static_cast<uint32_t>(lane) & 7;
+    uint32_t col[2];
+#pragma unroll
+    for (int p = 0; p < 2; ++p) col[p] = lc ^ (static_cast<uint32_t>(p) * 4 + (lr >> 1));
+    const uint32_t row0 = (static_cast<uint32_t>(wave) * 32 + lr) * rowbytes, rows8 = 8 * rowbytes;
+    auto load = [&](bsi_rsrc r, int slot, const uint32_t (&off)[2], int i) {  // load i of four
+        load16_to_lds(r, off[i & 1] + static_cast<uint32_t>(i) * rows8, 0, lds + slot * kLargeSlot + wave * 4096 + i * 1024);
+    };
+    auto issue = [&](bsi_rsrc r, int slot, const uint32_t (&off)[2]) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) load(r, slot, off, i);
+    };
+    // the offsets of the next stage, the same for either operand; returns whether it is in the upper image
+    auto advance = [&](uint32_t (&off)[2]) {
+        uint32_t first, second;
+        const bool in_upper = stages.next(first, second);
+#pragma unroll
+        for (int p = 0; p < 2; ++p) off[p] = row0 + (col[p] & 3) * 16 + (col[p] >= 4 ? second : first);
+        return in_upper;
+    };
+    v4i acc[8][4];
+#pragma unroll
+    for (int a = 0; a < 8; ++a)
+#pragma unroll
+        for (int b = 0; b < 4; ++b) acc[a][b] = (v4i){0, 0, 0, 0};
+    const int koff = (wr * 128 + ln) * 128, qoff = (wq * 64 + ln) * 128;
+    int pcol[2];
+#pragma unroll
+    for (int kk = 0; kk < 2; ++kk) pcol[kk] = ((kk * 4 + lg) ^ (ln >> 1)) * 16;
+    v4i ka[2][8], qb[2][4];
+    // K0 Q0 K1 Q1 K2 into slots 0 .. 4; then, when stage s has been read, Q of stage s + 2 and K of stage s + 3
+    uint32_t off[2], late[2];  // offsets of the stage K comes from next, and Q
+    bool upper = advance(off), late_upper;
+    issue(rk, 0, off);
+    issue(upper ? rhi : rlo, 1, off);
+    upper = advance(off);
+    issue(rk, 2, off);
+    issue(upper ? rhi : rlo, 3, off);
+    upper = advance(off);
+    issue(rk, 4, off);
+    asm volatile("s_waitcnt vmcnt(12)" ::: "memory");
+    lds_barrier();
+    int sk = 0;  // slot of K of the stage; Q in the next one
+#pragma unroll
+    for (int b = 0; b < 4; ++b) qb[0][b] = *reinterpret_cast<const v4i*>(lds + kLargeSlot + qoff + b * 2048 + pcol[0]);
+#pragma unroll
+    for (int a = 0; a < 8; ++a) ka[0][a] = *reinterpret_cast<const v4i*>(lds + koff + a * 2048 + pcol[0]);
+    __builtin_amdgcn_sched_barrier(0);
+#define BSI_LARGE_KSTEP(cur, nxt, kbase, qbase, BESIDE)                                                                \
+    _Pragma("unroll") for (int a = 0; a < 8; ++a) {                                                                    \
+        _Pragma("unroll") for (int b = 0; b < 4; ++b) {                                                                \
+            acc[a][b] = __builtin_amdgcn_mfma_i32_16x16x64_i8(ka[cur][a], qb[cur][b], acc[a][b], 0, 0, 0);             \
+            const int t = a * 4 + b;                                                                                   \
+            if (t < 24 && (t & 1) == 0) {                                                                              \
+                const int r = t >> 1;                                                                                  \
+                if (r < 4) qb[nxt][r] = *reinterpret_cast<const v4i*>(lds + (qbase) + r * 2048);                       \
+                else ka[nxt][r - 4] = *reinterpret_cast<const v4i*>(lds + (kbase) + (r - 4) * 2048);                   \
+            }                                                                                                          \
+            BESIDE;                                                                                                    \
+            __builtin_amdgcn_sched_barrier(0);                                                                         \
+        }                                                                                                              \
+    }
+    // A stage.  Where the loads behind the barrier come from is worked out among the MFMAs of the first k-step (NEXT: `off` of K goes
+    // on to stage s + 3, that of Q is what it was), and they are issued among those of the second: in a run of their own they
+    // leave the matrix pipes idle, as all waves come to them at the same time.  The wait: stage s + 1 has landed (K of stage s + 2
+    // may be in flight); behind the barrier all of stage s has been read.
+#define BSI_LARGE_STAGE(NEXT, from)                                                                                                  \
+    {                                                                                                                              \
+        const int sq = sk + 1 >= kLargeSlots ? sk + 1 - kLargeSlots : sk + 1;                                                      \
+        const int nk = sk + 2 >= kLargeSlots ? sk + 2 - kLargeSlots : sk + 2, nq = sk + 3 >= kLargeSlots ? sk + 3 - kLargeSlots : sk + 3; \
+        BSI_LARGE_KSTEP(0, 1, sk * kLargeSlot + koff + pcol[1], sq * kLargeSlot + qoff + pcol[1], if (t == 24) {                   \
+            late[0] = off[0];                                                                                                      \
+            late[1] = off[1];                                                                                                      \
+            NEXT;                                                                                                                  \
+        });                                                                                                                        \
+        asm volatile("s_waitcnt vmcnt(4)" ::: "memory");                                                                           \
+        lds_barrier();                                                                                                             \
+        BSI_LARGE_KSTEP(1, 0, nk * kLargeSlot + koff + pcol[0], nq * kLargeSlot + qoff + pcol[0], {                                \
+            if (t >= 1 && t < 9 && (t & 1) == 1) load(from, sk, late, t >> 1);                                                     \
+            if (t >= 9 && t < 25 && (t & 3) == 1) load(rk, sq, off, (t - 9) >> 2);                                                 \
+        });                                                                                                                        \
+        sk = nk;                                                                                                                   \
+    }
+    if (uppers > 0) {
+#pragma nounroll
+        for (int s = 0; s < uppers; ++s) BSI_LARGE_STAGE(late_upper = upper; upper = advance(off), late_upper ? rhi : rlo);
+        // their sums move up by their eight bits
+#pragma unroll
+        for (int a = 0; a < 8; ++a)
+#pragma unroll
+            for (int b = 0; b < 4; ++b)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) acc[a][b][e] <<= 8;
+    }
+    // the lower image: `off` is that of half-chunk 2
+    uint32_t step = 128u;
+    int ahead = 3;  // the half-chunk that K goes on to; past the last one nothing is read
+#pragma nounroll
+    for (int s = 0; s < 2 * chunks; ++s) {
+        step = ahead == 2 * chunks ? kNowhere : (ahead > 2 * chunks ? 0u : 128u);
+        ++ahead;
+        BSI_LARGE_STAGE(off[0] += step; off[1] += step, rlo);
+    }
+#undef BSI_LARGE_STAGE
+#undef BSI_LARGE_KSTEP
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+    __syncthreads();  // the ring is free
+    float* const epi = reinterpret_cast<float*>(lds);
+    if (tid < kLargeTile) {
+        const int64_t r = r0 + tid;
+        epi[tid] = r < R ? Bw[r * Sb] : 0.0f;
+        epi[kLargeTile + tid] = (bias != nullptr && r < R) ? bias[r] : 0.0f;
+    }
+    float unit[4];
+#pragma unroll
+    for (int b = 0; b < 4; ++b) {
+        const int64_t q = q0 + wq * 64 + b * 16 + ln;
+        unit[b] = q < Q ? units[q] : 0.0f;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int a0 = 0; a0 < 8; a0 += 2) {  // two 16-key tiles at a time: piece wr * 4 + a0 / 2 of the 256 keys
+        float v[2][4][4];
+#pragma unroll
+        for (int a = 0; a < 2; ++a)
+#pragma unroll
+            for (int b = 0; b < 4; ++b)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) v[a][b][e] = static_cast<float>(acc[a0 + a][b][e]) * unit[b];  // exact
+        i8_store_tile<kLargeTile, 2, 4, kHalf>(v, lds, 1.0f, scale_inv, bias != nullptr, out_dtype, out, R_total, r0, q0, wr * 4 + a0 / 2, wq, R, Q,
+                                               ln, lg, out_stream != 0);
+    }
+    if (warm_lines > 0) i8_warm_lines<8>(lds, wave, lane, warm, warm_lines);
 }
 
 // ------------------------------------------------------------------ int8 image, one accumulator set per MFMA wave
@@ -1459,18 +1813,20 @@ static int stream_output() {
 
 constexpr int kCus = 256;
 
-static I8Grid i8_grid(int64_t tiles_x, int64_t tiles_y, dim3* grid) {
-    constexpr int64_t kBandTiles = 8;  // 4 and 16 take the same time within 2 %
-    I8Grid g{static_cast<int>(tiles_x), static_cast<int>(tiles_y), 0, 0u, 0u, 0u};
-    *grid = dim3(static_cast<unsigned>(tiles_x), static_cast<unsigned>(tiles_y));
-    const int64_t bands = (tiles_y + kBandTiles - 1) / kBandTiles, height = (tiles_y + bands - 1) / bands;
-    // the reciprocals give exact quotients while dividend times divisor stays below 2^32
-    if (tiles_x % 8 == 0 || tiles_x * tiles_y >= (int64_t{1} << 28) || tiles_x * tiles_y * tiles_x * height >= (int64_t{1} << 32)) return g;
+static I8Grid i8_bands(int64_t tiles_x, int64_t tiles_y, int64_t band) {  // in bands of about `band` query tiles
+    const int64_t bands = (tiles_y + band - 1) / band, height = (tiles_y + bands - 1) / bands;
     auto reciprocal = [](int64_t n) { return n == 1 ? 0u : static_cast<unsigned>((int64_t{1} << 32) / n + 1); };
-    g.height = static_cast<int>(height);
-    g.by_band = reciprocal(tiles_x * height);
-    g.by_height = reciprocal(height);
-    g.by_last = reciprocal(tiles_y - (tiles_y - 1) / height * height);
+    return I8Grid{static_cast<int>(tiles_x), static_cast<int>(tiles_y), static_cast<int>(height), reciprocal(tiles_x * height),
+                  reciprocal(height), reciprocal(tiles_y - (tiles_y - 1) / height * height)};
+}
+
+static I8Grid i8_grid(int64_t tiles_x, int64_t tiles_y, dim3* grid) {
+    const I8Grid g = i8_bands(tiles_x, tiles_y, 8);  // 4 and 16 take the same time within 2 %
+    // the reciprocals give exact quotients while dividend times divisor stays below 2^32
+    if (tiles_x % 8 == 0 || tiles_x * tiles_y >= (int64_t{1} << 28) || tiles_x * tiles_y * tiles_x * g.height >= (int64_t{1} << 32)) {
+        *grid = dim3(static_cast<unsigned>(tiles_x), static_cast<unsigned>(tiles_y));
+        return I8Grid{static_cast<int>(tiles_x), static_cast<int>(tiles_y), 0, 0u, 0u, 0u};
+    }
     *grid = dim3(static_cast<unsigned>(tiles_x * tiles_y));
     return g;
 }
@@ -1488,11 +1844,11 @@ static void launch_mfma_i8_tm(const int8_t* A8, const float* qscale, int stride,
     if constexpr (kMode == kI8Chain && TM == 128)
         if (t_coop == nullptr && tiles > kCus && tiles * chunks < (int64_t{1} << 29)) {
             static LdsOptIn once;
-            lds_opt_in(once, reinterpret_cast<const void*>(&dot_mfma_i8_tiles_kernel<TM, TN, kHalf>), I8TilesCfg<TM, TN>::kLdsTiles);
-            launch((dot_mfma_i8_tiles_kernel<TM, TN, kHalf>), dim3(kCus), dim3(C::kBlock), I8TilesCfg<TM, TN>::kLdsTiles, st, A8, qscale, stride,
+            lds_opt_in(once, reinterpret_cast<const void*>(&dot_mfma_i8_tiles_kernel<TM, TN, kHalf, false>), I8TilesCfg<TM, TN>::kLdsTiles);
+            launch((dot_mfma_i8_tiles_kernel<TM, TN, kHalf, false>), dim3(kCus), dim3(C::kBlock), I8TilesCfg<TM, TN>::kLdsTiles, st, A8, qscale, stride,
                    K8, Bw, Sb, chunks, R, Q, down_shift, scale_inv, R_total, out, bias, key_tiled,
                    static_cast<const unsigned char*>(g_warm_ptr), static_cast<long long>(g_warm_bytes / 128), stream_output(), g,
-                   static_cast<unsigned>(tiles), t_out_dtype);
+                   static_cast<unsigned>(tiles), t_out_dtype, 0);
             return;
         }
     if constexpr (kMode == kI8Chain)
@@ -1589,6 +1945,66 @@ static void launch_mfma_i8w(const int8_t* A8, const float* qscale, int stride, c
                            stream_output(), t_out_dtype);
 }
 
+// The large layers' launches: the images in units, the integer sums, and the chain for what they leave.  The rule, in us: a round of
+// 256 workgroups takes 1.07 a chunk and 0.5 with tiles of 128 x 128, 3.3 and 2.7 with tiles of 256 x 256; the images are written at
+// 0.75 a million elements; the launch that ends at once and the gaps are 7.  Measured, 128 x 128 and 256 x 256, at its edges:
+// 2048 x 2048 x 16384 88.6, 84.4 and 1024 x 4096 x 16384 80, 77 (taken); 2048 x 2048 x 8192 49, 56 and 3000 x 1600 x 12000 93, 108 (not).
+static size_t large_aligned(size_t v) { return (v + 255) / 256 * 256; }
+size_t i8_large_workspace_bytes(int64_t Q, int chunks) {
+    if (Q < kLargeMinQ || chunks > kLargeMaxChunks) return 0;
+    const size_t image = large_aligned(static_cast<size_t>(Q) * chunks * 256), words = static_cast<size_t>((chunks * 4 + 63) / 64);
+    return 2 * image + large_aligned(static_cast<size_t>(Q) * words * 8) + large_aligned(static_cast<size_t>(Q) * 4) +
+           large_aligned(static_cast<size_t>((Q + kLargeTile - 1) / kLargeTile) * 4);
+}
+
+bool i8_large_serves(int64_t Q, int64_t R, int chunks) {
+    const int forced = g_i8_tile.load(std::memory_order_relaxed);
+    if (Q < kLargeMinQ || chunks > kLargeMaxChunks || (forced != 0 && forced != kLargeTile)) return false;
+    const int64_t small = ((R + 127) / 128) * ((Q + 127) / 128), large = ((R + kLargeTile - 1) / kLargeTile) * ((Q + kLargeTile - 1) / kLargeTile);
+    // the tile kernels' own limits: ring positions and exact quotients in 32 bits
+    if (small * chunks >= (int64_t{1} << 29) || large * ((R + kLargeTile - 1) / kLargeTile) >= (int64_t{1} << 29)) return false;
+    if (forced == kLargeTile) return true;
+    if (small <= kCus) return false;
+    const double us_small = static_cast<double>((small + kCus - 1) / kCus) * (1.07 * chunks + 0.5);
+    const double us_large = static_cast<double>((large + kCus - 1) / kCus) * (3.3 * chunks + 2.7) + 7.0 + 7.5e-7 * static_cast<double>(Q) * chunks * 256;
+    return us_large < us_small;
+}
+
+template <bool kHalf>
+static void launch_i8_large_t(unsigned char* ws, const int8_t* A8, const float* qscale, int stride, const int8_t* K8, const float* Bw, int Sa,
+                              int Sb, int chunks, int64_t R, int64_t Q, float scale_inv, int64_t R_total, float* out, const float* bias,
+                              hipStream_t st) {
+    const size_t image = large_aligned(static_cast<size_t>(Q) * chunks * 256), words = static_cast<size_t>((chunks * 4 + 63) / 64);
+    unsigned char* const lo = ws;
+    unsigned char* const hi = lo + image;
+    unsigned char* const masks = hi + image;
+    float* const units = reinterpret_cast<float*>(masks + large_aligned(static_cast<size_t>(Q) * words * 8));
+    unsigned* const left = reinterpret_cast<unsigned*>(reinterpret_cast<unsigned char*>(units) + large_aligned(static_cast<size_t>(Q) * 4));
+    launch(i8_units_kernel, dim3(static_cast<unsigned>(Q)), dim3(kUnitsBlock), 0, st, A8, qscale, stride, chunks, Sa, Sb,
+           reinterpret_cast<uint4*>(lo), reinterpret_cast<uint4*>(hi), reinterpret_cast<unsigned short*>(masks), units);
+    const I8Grid g = i8_bands((R + kLargeTile - 1) / kLargeTile, (Q + kLargeTile - 1) / kLargeTile, 2);
+    static LdsOptIn once, once_left;
+    lds_opt_in(once, reinterpret_cast<const void*>(&dot_mfma_i8_large_kernel<kHalf>), kLargeLds);
+    const unsigned char* const warm = static_cast<const unsigned char*>(g_warm_ptr);
+    const long long warm_lines = static_cast<long long>(g_warm_bytes / 128);
+    launch((dot_mfma_i8_large_kernel<kHalf>), dim3(static_cast<unsigned>(g.tiles_x) * static_cast<unsigned>(g.tiles_y)), dim3(512), kLargeLds, st,
+           reinterpret_cast<const int8_t*>(lo), reinterpret_cast<const int8_t*>(hi), reinterpret_cast<const unsigned long long*>(masks), units, K8,
+           Bw, Sb, chunks, R, Q, scale_inv, R_total, out, bias, warm, warm_lines, stream_output(), g, t_out_dtype, left);
+    dim3 grid;
+    const I8Grid tiles = i8_grid((R + 127) / 128, (Q + 127) / 128, &grid);
+    using T = I8TilesCfg<128, 128>;
+    lds_opt_in(once_left, reinterpret_cast<const void*>(&dot_mfma_i8_tiles_kernel<128, 128, kHalf, true>), T::kLdsTiles);
+    const int64_t left_tiles = static_cast<int64_t>(tiles.tiles_x) * tiles.tiles_y;  // every workgroup of that kernel has a tile
+    launch((dot_mfma_i8_tiles_kernel<128, 128, kHalf, true>), dim3(static_cast<unsigned>(left_tiles < kCus ? left_tiles : kCus)), dim3(T::kBlock), T::kLdsTiles, st, A8, qscale, stride, K8, Bw, Sb, chunks,
+           R, Q, 16 - Sa - Sb, scale_inv, R_total, out, bias, 0, static_cast<const unsigned char*>(nullptr), 0LL, stream_output(), tiles,
+           static_cast<unsigned>(left_tiles), t_out_dtype, left);
+}
+void launch_i8_large(void* workspace, const int8_t* A8, const float* qscale, int stride, const int8_t* K8, const float* Bw, int Sa, int Sb,
+                     int chunks, int64_t R, int64_t Q, float scale_inv, int64_t R_total, float* out, const float* bias, hipStream_t st) {
+    (t_out_dtype != BSI_DTYPE_F32 ? &launch_i8_large_t<true> : &launch_i8_large_t<false>)(
+        static_cast<unsigned char*>(workspace), A8, qscale, stride, K8, Bw, Sa, Sb, chunks, R, Q, scale_inv, R_total, out, bias, st);
+}
+
 // Tile choice.  The 128 x 128 tile moves the fewest operand bytes per MAC and is the fastest whenever its grid
 // covers the 256 CUs (one workgroup per CU at a time) -- measured up to several rounds of 256.  A smaller grid
 // leaves CUs idle that smaller tiles would use: a workgroup's time per half-chunk is about 1 : 0.63 : 0.35 : 0.31
@@ -1597,7 +2013,7 @@ static void launch_mfma_i8w(const int8_t* A8, const float* qscale, int stride, c
 int choose_i8_tile(int64_t R, int64_t Q, int64_t* cost_out) {
     const int64_t n128 = ((R + 127) / 128) * ((Q + 127) / 128);
     if (cost_out) *cost_out = ((n128 + 255) / 256) * 100;
-    if (const int forced = g_i8_tile.load(std::memory_order_relaxed)) return forced;
+    if (const int forced = g_i8_tile.load(std::memory_order_relaxed); forced != 0 && forced != kLargeTile) return forced;
     if (n128 > 256) return 128;
     const int64_t cost[4] = {100, ((((R + 127) / 128) * ((Q + 63) / 64) + 255) / 256) * 63,
                              ((((R + 63) / 64) * ((Q + 63) / 64) + 255) / 256) * 35,

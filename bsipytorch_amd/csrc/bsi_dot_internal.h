@@ -51,6 +51,14 @@ void launch_mfma_i8(const int8_t* A8, const float* qscale, int stride, const int
                     int32_t* chunk_ints, const float* bias, hipStream_t st,
                     int key_tiled = 0, int ndig = 0, long long dig_stride = 0, const long long* key_indices = nullptr);
 
+// Large layers as plain integer sums (dot_mfma_i8_large_kernel): the workspace they take beside the query operands (0: none, the
+// rows are too few or too long), whether a call is one, and its launches.  The key image is row-major.
+constexpr int64_t kLargeMinQ = 512;
+size_t i8_large_workspace_bytes(int64_t Q, int chunks);
+bool i8_large_serves(int64_t Q, int64_t R, int chunks);
+void launch_i8_large(void* workspace, const int8_t* A8, const float* qscale, int stride, const int8_t* K8, const float* Bw, int Sa, int Sb,
+                     int chunks, int64_t R, int64_t Q, float scale_inv, int64_t R_total, float* out, const float* bias, hipStream_t st);
+
 // ---- bsi_dot_few_rows.hip: the plane-streaming kernel for up to kStreamMaxQ query rows on 6-plane tiled keys
 // (query tiles and key tiles per workgroup chosen from Q and R)
 void launch_mfma_stream_by_shape(const int8_t* A8, const float* qscale, int stride, const uint64_t* B, const float* Bw,

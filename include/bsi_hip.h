@@ -225,6 +225,8 @@ int bsi_hip_planes_to_int8_tiled(const uint64_t* words_device, int64_t rows, int
  * whose kernel selection is read from environment variables on every call (bsi_cuda_kernels_dot.cuh:2642). */
 #define BSI_OPT_I8_TILE 1 /* tile of the int8-image kernel: 128 (128 keys x 128 queries), 12864 (128 x 64), 64 (64 x 64),
                              6432 (64 x 32) or 1284 (128 x 128 on four MFMA waves of 64 x 64 with one accumulator set);
+                             256: bsi_hip_linear[_out] takes every layer of at least 512 rows of at most 16384 elements as
+                             integer sums on tiles of 256 x 256, other calls choose;
                              0 (default) = chosen per call from the grid each tile would give on the 256 CUs */
 #define BSI_OPT_DIGITS_ROUTE 2 /* bsi_hip_dot_digits: 1 = stacked digits and a combine pass, 2 = digits recombined in the
                                   accumulator where the int32 bound allows; 0 (default) = the cheaper by a cost estimate */
