@@ -504,8 +504,13 @@ __device__ __forceinline__ uint32_t shift_quad_bytes(uint32_t sm, const QuadShif
 // L2s are written back at its end.  Before (16-bit pairs in registers for up to 16 chunks, plain stores) and now, us:
 // 16384 x 4096 float32 94.9 -> 79.2 (4.9 TB/s), 8192 x 8192 119.4 -> 85.7, 4096 x 4096 22.5 -> 18.6, 768 x 768 6.7 -> 4.5;
 // bfloat16 16384 x 4096 64.2 -> 54.3, 8192 x 5120 37.4 -> 26.7, 2048 x 2048 8.4 -> 7.3.
+// kOnce: the loads are nontemporal too, for matrices that the memory-side cache does not hold, of up to 16 chunks a row (a longer
+// row takes longer that way, 4096 x 8192 bfloat16 31.4, 32.9) and whole lines (a line that two rows share is fetched twice, 12800 x
+// 1000 float32 15.8, 17.9).  us, plain and nontemporal: 16384 x 4096 float32 79.4, 75.7, bfloat16 54.3, 52.7; 11008 x 4096 float16
+// 38.9, 36.4; below the line 4096 x 4096 float32 (64 MiB) 21.1, 21.6.
+constexpr size_t kKeysOnceBytes = size_t{80} << 20;
 constexpr int kKeyRows = 16, kKeyGroup = 8;
-template <typename T, bool kVec, int kHeld, int kLoads>
+template <typename T, bool kVec, int kHeld, int kLoads, bool kOnce>
 __global__ __launch_bounds__(kKeyRows * BSI_WAVE, 8) void build_keys_fast_kernel(
     const T* __restrict__ x, int64_t R, int64_t d, int chunks, int slices, double dec_scale, float scale,
     unsigned long long* __restrict__ tiled, int8_t* __restrict__ image8, int* __restrict__ shifts, float* __restrict__ weights) {
@@ -530,7 +535,7 @@ __global__ __launch_bounds__(kKeyRows * BSI_WAVE, 8) void build_keys_fast_kernel
         if (c >= chunks) break;
         float v[kLoads][4];
 #pragma unroll
-        for (int j = 0; j < kLoads; ++j) load_chunk_quad<T, kVec>(xrow, d, c + j, cl, v[j]);  // past the row: zeros
+        for (int j = 0; j < kLoads; ++j) load_chunk_quad<T, kVec, kOnce>(xrow, d, c + j, cl, v[j]);  // past the row: zeros
 #pragma unroll
         for (int j = 0; j < kLoads; ++j) {
             take_max(v[j]);
@@ -945,15 +950,17 @@ extern "C" int bsi_hip_build_fixed_keys(const void* x, int dtype, int64_t R, int
     // Rows of up to 32 chunks stay in registers whole.  kHeld is the next of 8, 16 and 32, kLoads what the rest of the 64
     // registers takes in flight (32 chunks, 8192 x 5120 bfloat16 with plain stores: 2, 4, 8 loads 44, 31, 34 us).
     const int64_t tiles = (R + kKeyRows - 1) / kKeyRows;
-#define BSI_KEYS(kHeld, kLoads)                                                                                              \
+#define BSI_KEYS(kHeld, kLoads, kOnce)                                                                                              \
     BSI_DISPATCH_DTYPE(dtype, BSI_DISPATCH_BOOL(quads_aligned(x, dtype, d), kVec,                                             \
-        launch((build_keys_fast_kernel<T, kVec, kHeld, kLoads>), dim3(static_cast<unsigned>(tiles)),                 \
+        launch((build_keys_fast_kernel<T, kVec, kHeld, kLoads, kVec && kOnce>), dim3(static_cast<unsigned>(tiles)),                 \
                dim3(kKeyRows * BSI_WAVE), 0, as_stream(stream), static_cast<const T*>(x), R, d, chunks, fixed_bits,           \
                static_cast<double>(scale_int), static_cast<float>(scale_int),                                                \
                reinterpret_cast<unsigned long long*>(tiled), image, shifts, slice_weights)))
-    if (chunks <= 8) BSI_KEYS(8, 8)
-    else if (chunks <= 16) BSI_KEYS(16, 8)
-    else BSI_KEYS(32, 4)
+    const size_t row_bytes = static_cast<size_t>(d) * (dtype == BSI_DTYPE_F32 ? 4 : 2);
+    const bool once = row_bytes % 128 == 0 && reinterpret_cast<uintptr_t>(x) % 128 == 0 && row_bytes * static_cast<size_t>(R) >= kKeysOnceBytes;
+    if (chunks <= 8) { if (once) BSI_KEYS(8, 8, true) else BSI_KEYS(8, 8, false) }
+    else if (chunks <= 16) { if (once) BSI_KEYS(16, 8, true) else BSI_KEYS(16, 8, false) }
+    else BSI_KEYS(32, 4, false)
 #undef BSI_KEYS
     BSI_LAUNCH_CHECK("build_keys_fast_kernel");
     return BSI_OK;

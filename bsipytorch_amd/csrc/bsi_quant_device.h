@@ -9,6 +9,8 @@
 #pragma once
 #include "bsi_dot_device.h"
 
+#include <type_traits>
+
 namespace bsi {
 
 // Chunks whose largest |x| is below 2^16 (as float bits, so that infinities and NaNs are above) are quantised in float32
@@ -79,38 +81,33 @@ __device__ __forceinline__ float buffer_load_as_float<__hip_bfloat16>(bsi_rsrc r
 }
 
 // Four consecutive elements from element i on: one 16- or 8-byte load (i a multiple of 4, the buffer a multiple of 4
-// elements long and aligned to the load's size).
-template <typename T>
-__device__ __forceinline__ void buffer_load_quad(bsi_rsrc r, int i, float (&v)[4]);
-template <>
-__device__ __forceinline__ void buffer_load_quad<float>(bsi_rsrc r, int i, float (&v)[4]) {
-    typedef unsigned v4u __attribute__((ext_vector_type(4)));
-    const v4u u = __builtin_amdgcn_raw_buffer_load_b128(r, i * 4, 0, 0);
+// elements long and aligned to the load's size).  kOnce: a nontemporal load, of what is read once.
+template <typename T, bool kOnce>
+__device__ __forceinline__ void buffer_load_quad(bsi_rsrc r, int i, float (&v)[4]) {
+    constexpr int kCache = kOnce ? 2 : 0;
+    if constexpr (std::is_same_v<T, float>) {
+        typedef unsigned v4u __attribute__((ext_vector_type(4)));
+        const v4u u = __builtin_amdgcn_raw_buffer_load_b128(r, i * 4, 0, kCache);
 #pragma unroll
-    for (int k = 0; k < 4; ++k) v[k] = __uint_as_float(u[k]);
-}
-template <>
-__device__ __forceinline__ void buffer_load_quad<__half>(bsi_rsrc r, int i, float (&v)[4]) {
-    typedef unsigned v2u __attribute__((ext_vector_type(2)));
-    const v2u u = __builtin_amdgcn_raw_buffer_load_b64(r, i * 2, 0, 0);
+        for (int k = 0; k < 4; ++k) v[k] = __uint_as_float(u[k]);
+    } else {
+        typedef unsigned v2u __attribute__((ext_vector_type(2)));
+        const v2u u = __builtin_amdgcn_raw_buffer_load_b64(r, i * 2, 0, kCache);
 #pragma unroll
-    for (int k = 0; k < 4; ++k) v[k] = __half2float(__ushort_as_half(static_cast<unsigned short>(u[k >> 1] >> (16 * (k & 1)))));
-}
-template <>
-__device__ __forceinline__ void buffer_load_quad<__hip_bfloat16>(bsi_rsrc r, int i, float (&v)[4]) {
-    typedef unsigned v2u __attribute__((ext_vector_type(2)));
-    const v2u u = __builtin_amdgcn_raw_buffer_load_b64(r, i * 2, 0, 0);
-#pragma unroll
-    for (int k = 0; k < 4; ++k) v[k] = __uint_as_float((k & 1) ? (u[k >> 1] & 0xFFFF0000u) : (u[k >> 1] << 16));
+        for (int k = 0; k < 4; ++k) {
+            if constexpr (std::is_same_v<T, __half>) v[k] = __half2float(__ushort_as_half(static_cast<unsigned short>(u[k >> 1] >> (16 * (k & 1)))));
+            else v[k] = __uint_as_float((k & 1) ? (u[k >> 1] & 0xFFFF0000u) : (u[k >> 1] << 16));
+        }
+    }
 }
 
 // The lane's four elements of chunk c of a row; 0 past the row's end.  kVec: d and the row's address allow buffer_load_quad.
-template <typename T, bool kVec>
+template <typename T, bool kVec, bool kOnce = false>
 __device__ __forceinline__ void load_chunk_quad(const T* row, int64_t d, int c, const ChunkLane& cl, float (&v)[4]) {
     const bsi_rsrc r = make_rsrc(row, static_cast<size_t>(d) * sizeof(T));
     const int i = c * BSI_CHUNK_ELEMS + cl.quad;
     if (kVec) {
-        buffer_load_quad<T>(r, i, v);
+        buffer_load_quad<T, kOnce>(r, i, v);
     } else {
 #pragma unroll
         for (int k = 0; k < 4; ++k) v[k] = buffer_load_as_float<T>(r, i + k);
