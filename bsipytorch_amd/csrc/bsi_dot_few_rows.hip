@@ -21,6 +21,7 @@ namespace bsi {
 // whatever the number of waves.  Problems with more chunks than LDS slots run in several passes.
 
 constexpr int kStreamLdsInts = 16384;  // at most 64 KiB of chunk accumulators per pass
+constexpr int kStreamLds = kStreamLdsInts * 4 + 4096 + 16 * 2048;  // with their scales and 16 waves' query rows
 
 // kBuild: the queries are quantised by this launch (bsi_coop_build.h); A8 and qscale are not looked at.  The copy lies in the
 // order of the operand loads (coop_image_at: up to 1 KiB in one run a load, where rows one after the other are 32 lines a load and
@@ -31,6 +32,14 @@ constexpr int kStreamLdsInts = 16384;  // at most 64 KiB of chunk accumulators p
 // take the build's description: with it the workgroup's size, which lies behind the arguments, is in another cache line of
 // them, and its fetch holds up every wave's first key load.  us, with and without: 16 x 4096 x 16384 12.3, 11.8; 16 x 4096 x
 // 4096 5.25, 5.09; 1 x 4096 x 16384 10.5, 10.2; 1 x 16384 x 4096 11.1, 10.9 (1 x 4096 x 4096 4.06, 4.11).
+//
+// Without kBuild the image has its rows one after the other.  An operand's lanes want 64 bytes of each of 16 rows, and loads of
+// such pieces run at half the rate of whole lines (16 rows of a chunk: 24 KiB of key planes come with 4 KiB fetched as 8); so a
+// load takes 128 bytes of 8 rows, and the wave turns them round through 2 KiB of LDS, in which its sums lie afterwards.  The scales
+// go with them, as above.  us a dot, operands straight from memory, then so: 16 x 16384 x 4096 14.7, 12.2; 16 x 8192 x 8192 13.9,
+// 11.9; 24 x 8192 x 8192 18.7, 14.8; 32 x 4096 x 4096 7.6, 6.1; 16 x 8192 x 32768 44.8, 41.0; 8 x 16384 x 4096 12.6, 11.9;
+// 1 x 4096 x 32768 21.6, 21.5; 8 x 8192 x 16384 21.5, 21.5.  All 4 KiB of a chunk at once, in LDS of its own: 12.0 for the first,
+// but 22.5 for the last (a workgroup less on a CU).
 template <int NT, int KT, bool kInts, bool kBuild>
 __global__ __launch_bounds__(1024) void dot_mfma_stream_kernel(
     const int8_t* A8, const float* qscale, int qscale_stride,
@@ -38,7 +47,8 @@ __global__ __launch_bounds__(1024) void dot_mfma_stream_kernel(
     const float* __restrict__ Bw, int chunks, int pass_chunks, int64_t R, int64_t Q, int down_shift, float scale_inv,
     int64_t R_total, float* __restrict__ out, int* __restrict__ chunk_ints, const float* __restrict__ bias, int out_dtype,
     std::conditional_t<kBuild, CoopBuild, int> coop) {
-    // [pass_chunks][KT][NT][16 queries][16 keys]; kBuild: then the chunks' scales, [pass_chunks][NT][16 queries]
+    // [pass_chunks][KT][NT][16 queries][16 keys], then the chunks' scales, [pass_chunks][NT][16 queries]; without kBuild a chunk's
+    // query rows are turned round where its sums will lie, or, if those have no 2 KiB, in 2 KiB a wave behind all that
     extern __shared__ __attribute__((aligned(16))) int ints[];
     constexpr int kSlot = KT * NT * 256;
     float* const chunk_scales = reinterpret_cast<float*>(ints + static_cast<size_t>(pass_chunks) * kSlot);
@@ -59,6 +69,11 @@ __global__ __launch_bounds__(1024) void dot_mfma_stream_kernel(
         ksrc[k] = B64 + static_cast<size_t>(t) * ktile + lane;
     }
     const size_t arow = static_cast<size_t>(chunks) * 256;
+    // without kBuild: rows past the batch read 0; kMfmaMaxChunks keeps 32 rows of an image below 2^31 bytes
+    [[maybe_unused]] const int64_t rows_here = Q - q0 < NT * 16 ? Q - q0 : NT * 16;
+    [[maybe_unused]] const bsi_rsrc qrs = make_rsrc(A8 + static_cast<size_t>(q0) * arow, static_cast<size_t>(rows_here) * arow);
+    [[maybe_unused]] const bsi_rsrc srs = make_rsrc(qscale + q0 * qscale_stride, static_cast<size_t>(rows_here) * qscale_stride * 4);
+    [[maybe_unused]] v4i* const turn_here = reinterpret_cast<v4i*>(chunk_scales + static_cast<size_t>(pass_chunks) * NT * 16) + wave * 128;
     uint2 kc[KT][6];
     auto load_keys = [&](int c) {
 #pragma unroll
@@ -79,39 +94,44 @@ __global__ __launch_bounds__(1024) void dot_mfma_stream_kernel(
     const int64_t cq = q0 + ct * 16 + cn, cr = (tile0 + ck) * 16 + ckey;
     const bool cvalid = chain && cq < Q && cr < R;
     const float down = __uint_as_float(static_cast<uint32_t>(127 - down_shift) << 23);
-    const float* csrc = qscale + (cvalid ? cq : 0) * qscale_stride;
-    const int sstep = (qscale_stride == 1) ? 0 : 1;
     const EpilogueOperands eo = load_epilogue_operands(Bw, bias, R, cvalid, cr);
 
+    // passes but the last are whole rounds of the waves, so that a wave's next chunk is nwaves further on across them too and its
+    // planes are on their way while the chain runs
+    if (!kBuild) load_keys(wave < chunks ? wave : chunks - 1);
     for (int p0 = 0; p0 < chunks; p0 += pass_chunks) {
         const int pend = (p0 + pass_chunks < chunks) ? p0 + pass_chunks : chunks;
-        int c = p0 + wave;
-        if (c < pend && !(kBuild && p0 == 0)) load_keys(c);
-        for (; c < pend; c += nwaves) {
+        for (int c = p0 + wave; c < pend; c += nwaves) {
             // query operands of this chunk (L2 resident), then the key planes of the wave's next chunk
             v4i qb[NT][4];
             float qs[NT];
 #pragma unroll
             for (int t = 0; t < NT; ++t) {
-                const int64_t q = q0 + t * 16 + ln;
-                qs[t] = 0.0f;
-                if (q < Q) {
-                    const int rows = Q - t * 16 < 16 ? static_cast<int>(Q) - t * 16 : 16;  // kBuild: coop_image_at's order
-                    const v4i* src = reinterpret_cast<const v4i*>(
-                        kBuild ? A8 + static_cast<size_t>(t) * 16 * arow + ((c * 16 + lg) * rows + ln) * 16
-                               : A8 + static_cast<size_t>(q) * arow + c * 256 + lg * 64);
-                    const int step = kBuild ? 4 * rows : 1;
-                    if constexpr (kBuild) qs[t] = qscale[coop.by_row ? t * 16 + ln : t * 16 * chunks + c * rows + ln];
+                if constexpr (kBuild) {
+                    qs[t] = 0.0f;
+                    if (q0 + t * 16 + ln < Q) {
+                        const int rows = Q - t * 16 < 16 ? static_cast<int>(Q) - t * 16 : 16;  // coop_image_at's order
+                        const v4i* src = reinterpret_cast<const v4i*>(A8 + static_cast<size_t>(t) * 16 * arow + ((c * 16 + lg) * rows + ln) * 16);
+                        qs[t] = qscale[coop.by_row ? t * 16 + ln : t * 16 * chunks + c * rows + ln];
 #pragma unroll
-                    for (int m = 0; m < 4; ++m) qb[t][m] = src[m * step];
+                        for (int m = 0; m < 4; ++m) qb[t][m] = src[m * 4 * rows];
+                    } else {
+#pragma unroll
+                        for (int m = 0; m < 4; ++m) qb[t][m] = (v4i){0, 0, 0, 0};
+                    }
                 } else {
+                    const int uc = __builtin_amdgcn_readfirstlane(c);
+                    qs[t] = __int_as_float(__builtin_amdgcn_raw_buffer_load_b32(srs, (t * 16 + ln) * qscale_stride * 4,
+                                                                                qscale_stride == 1 ? 0 : uc * 4, 0));
 #pragma unroll
-                    for (int m = 0; m < 4; ++m) qb[t][m] = (v4i){0, 0, 0, 0};
+                    for (int m = 0; m < 4; ++m)  // 128 bytes of 8 rows
+                        qb[t][m] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(
+                            qrs, (t * 16 + (m & 1) * 8 + (lane >> 3)) * chunks * 256 + (m >> 1) * 128 + (lane & 7) * 16, uc * 256, 0));
                 }
             }
             uint2 kn[KT][6];
             const int cnext = c + nwaves;
-            if (cnext < pend) {
+            if (cnext < chunks) {
 #pragma unroll
                 for (int k = 0; k < KT; ++k)
 #pragma unroll
@@ -119,6 +139,26 @@ __global__ __launch_bounds__(1024) void dot_mfma_stream_kernel(
                         const unsigned long long w = ksrc[k][(static_cast<size_t>(cnext) * 6 + j) * 64];
                         kn[k][j] = make_uint2(static_cast<uint32_t>(w), static_cast<uint32_t>(w >> 32));
                     }
+            }
+            if constexpr (!kBuild) {
+                // half a chunk of 16 rows at a time; 16-byte column x of row r lies at x ^ (r & 7): conflict-free both ways.  A
+                // wave's LDS instructions are done in order.
+                v4i* const turn = kSlot >= 512 ? reinterpret_cast<v4i*>(ints + (c - p0) * kSlot) : turn_here;
+#pragma unroll
+                for (int t = 0; t < NT; ++t) {
+                    const v4i loaded[4] = {qb[t][0], qb[t][1], qb[t][2], qb[t][3]};
+#pragma unroll
+                    for (int h = 0; h < 2; ++h) {
+                        turn[lane ^ (lane >> 3)] = loaded[h * 2];
+                        turn[64 + (lane ^ (lane >> 3))] = loaded[h * 2 + 1];
+                        __builtin_amdgcn_wave_barrier();
+                        if ((lg >> 1) == h) {
+#pragma unroll
+                            for (int m = 0; m < 4; ++m) qb[t][m] = turn[ln * 8 + (((lg & 1) * 4 + m) ^ (ln & 7))];
+                        }
+                        __builtin_amdgcn_wave_barrier();
+                    }
+                }
             }
 #pragma unroll
             for (int k = 0; k < KT; ++k) {
@@ -139,11 +179,11 @@ __global__ __launch_bounds__(1024) void dot_mfma_stream_kernel(
                     *reinterpret_cast<v4i*>(&ints[(c - p0) * kSlot + (k * NT + t) * 256 + ln * 16 + lg * 4]) = acc;
                 }
             }
-            if (kBuild && lg == 0) {
+            if (lg == 0) {
 #pragma unroll
                 for (int t = 0; t < NT; ++t) chunk_scales[((c - p0) * NT + t) * 16 + ln] = qs[t];
             }
-            if (cnext < pend) {
+            if (cnext < chunks) {
 #pragma unroll
                 for (int k = 0; k < KT; ++k)
 #pragma unroll
@@ -153,7 +193,7 @@ __global__ __launch_bounds__(1024) void dot_mfma_stream_kernel(
         __syncthreads();
         if (cvalid) {
             accf = chain_chunks(accf, p0, pend, down, [&](int cc) { return ints[(cc - p0) * kSlot + tid]; },
-                                [&](int cc) { return kBuild ? chunk_scales[((cc - p0) * NT + ct) * 16 + cn] : csrc[cc * sstep]; });
+                                [&](int cc) { return chunk_scales[((cc - p0) * NT + ct) * 16 + cn]; });
             if (kInts)
                 for (int cc = p0; cc < pend; ++cc)
                     chunk_ints[(cq * R + cr) * chunks + cc] = ints[(cc - p0) * kSlot + tid] >> down_shift;
@@ -538,10 +578,13 @@ static int stream_waves(unsigned groups, int chunks, int slot) {
     if (waves < slot / 64) waves = slot / 64;    // the chain needs one lane per output
     return waves > 16 ? 16 : waves;
 }
-// two key tiles per workgroup halve the query re-reads once there are enough tiles to fill the GPU
-static int stream_key_tiles(int64_t R) { return (R + 15) / 16 >= 1024 ? 2 : 1; }
+// Two key tiles per workgroup halve the query re-reads once there are enough tiles to fill the GPU.  With two tiles of queries besides,
+// the sums take 4 KiB a chunk and the operands more than the registers a wave has.  us, one key tile and two: a dot of 16 x 8192 x
+// 32768 49.3, 43.5, 16 x 4096 x 65536 49.5, 45.2; 32 x 4096 x 65536 65.0, 69.1, 32 x 4096 x 16384 15.6, 16.4, 32 x 8192 x 16384
+// 33.7, 34.0, 32 x 12288 x 32768 94.4, 97.7, 17 x 16384 x 16384 57.3, 54.9; with the build inside 17 x 1024 x 16384 9.6, 14.8, 24 x 2048 x 16384 11.9, 16.9, 17 x 8192 x 16384 33.1, 38.4.
+static int stream_key_tiles(int64_t Q, int64_t R) { return Q <= 16 && (R + 15) / 16 >= 1024 ? 2 : 1; }
 void stream_launch_shape(int64_t Q, int64_t R, int chunks, unsigned* groups, int* waves) {
-    const int kt = stream_key_tiles(R);
+    const int kt = stream_key_tiles(Q, R);
     *groups = stream_groups(R, kt);
     *waves = stream_waves(*groups, chunks, kt * (Q <= 16 ? 1 : 2) * 256);
 }
@@ -553,21 +596,27 @@ static void launch_mfma_stream(const int8_t* A8, const float* qscale, int stride
     constexpr int kSlot = KT * NT * 256;
     const dim3 grid(stream_groups(R, KT), static_cast<unsigned>((Q + 16 * NT - 1) / (16 * NT)));
     const int waves = stream_waves(grid.x * grid.y, chunks, kSlot);
+    constexpr int kChunkBytes = (kSlot + NT * 16) * 4;
+    const size_t turn = kSlot < 512 && t_coop == nullptr ? static_cast<size_t>(waves) * 2048 : 0;
     int pass_chunks = kStreamLdsInts / kSlot;
+    // 8 waves: two workgroups a CU
+    if (turn != 0 && waves == 8 && pass_chunks * kChunkBytes + turn > 80 * 1024)
+        pass_chunks = (80 * 1024 - static_cast<int>(turn)) / kChunkBytes / 8 * 8;
     if (pass_chunks > chunks) pass_chunks = chunks;
-    size_t lds = static_cast<size_t>(pass_chunks) * kSlot * sizeof(int);
+    const size_t lds = static_cast<size_t>(pass_chunks) * kChunkBytes + turn;
 #define BSI_STREAM_GO(INTS, BUILD, COOP)                                                                                      \
-    launch((dot_mfma_stream_kernel<NT, KT, INTS, BUILD>), grid, dim3(waves * 64), lds, st, A8, qscale, stride,                \
-           reinterpret_cast<const unsigned long long*>(B), Bw, chunks, pass_chunks, R, Q, down_shift, scale_inv, R_total, out, \
-           chunk_ints, bias, t_out_dtype, COOP)
+    do {                                                                                                                      \
+        static LdsOptIn once;                                                                                                 \
+        lds_opt_in(once, reinterpret_cast<const void*>(&dot_mfma_stream_kernel<NT, KT, INTS, BUILD>), kStreamLds);             \
+        launch((dot_mfma_stream_kernel<NT, KT, INTS, BUILD>), grid, dim3(waves * 64), lds, st, A8, qscale, stride,            \
+               reinterpret_cast<const unsigned long long*>(B), Bw, chunks, pass_chunks, R, Q, down_shift, scale_inv, R_total, \
+               out, chunk_ints, bias, t_out_dtype, COOP);                                                                     \
+    } while (0)
     if (chunk_ints) BSI_STREAM_GO(true, false, 0);
     else if (t_coop == nullptr) BSI_STREAM_GO(false, false, 0);
     else {
         CoopBuild coop = *t_coop;
         coop.shares = coop_shares(grid.x, coop.by_row ? coop.rows : coop.rows * coop.chunks);
-        static LdsOptIn once;
-        lds_opt_in(once, reinterpret_cast<const void*>(&dot_mfma_stream_kernel<NT, KT, false, true>), kStreamLdsInts * 4 + 4096);
-        lds += static_cast<size_t>(pass_chunks) * NT * 16 * sizeof(float);
         BSI_STREAM_GO(false, true, coop);
     }
 #undef BSI_STREAM_GO
@@ -576,10 +625,10 @@ static void launch_mfma_stream(const int8_t* A8, const float* qscale, int stride
 void launch_mfma_stream_by_shape(const int8_t* A8, const float* qscale, int stride, const uint64_t* B, const float* Bw,
                                  int chunks, int64_t R, int64_t Q, int down_shift, float scale_inv, int64_t R_total,
                                  float* out, int32_t* chunk_ints, const float* bias, hipStream_t st) {
-    const bool two = stream_key_tiles(R) == 2;
 #define BSI_STREAM_ARGS A8, qscale, stride, B, Bw, chunks, R, Q, down_shift, scale_inv, R_total, out, chunk_ints, bias, st
-    if (Q <= 16) { if (two) launch_mfma_stream<1, 2>(BSI_STREAM_ARGS); else launch_mfma_stream<1, 1>(BSI_STREAM_ARGS); }
-    else { if (two) launch_mfma_stream<2, 2>(BSI_STREAM_ARGS); else launch_mfma_stream<2, 1>(BSI_STREAM_ARGS); }
+    if (Q > 16) launch_mfma_stream<2, 1>(BSI_STREAM_ARGS);
+    else if (stream_key_tiles(Q, R) == 2) launch_mfma_stream<1, 2>(BSI_STREAM_ARGS);
+    else launch_mfma_stream<1, 1>(BSI_STREAM_ARGS);
 #undef BSI_STREAM_ARGS
 }
 
@@ -593,7 +642,7 @@ struct FusedPlan {
 static FusedPlan fused_plan(int64_t Q, int chunks, int64_t R) {
     FusedPlan p;
     const int64_t ntiles = (R + 15) / 16;
-    p.key_tiles = ntiles >= 1024 ? 2 : 1;  // as bsi_hip_dot: two key tiles per workgroup once the GPU is full
+    p.key_tiles = ntiles >= 1024 ? 2 : 1;  // two key tiles per workgroup once the GPU is full
     p.grid = static_cast<unsigned>((ntiles + p.key_tiles - 1) / p.key_tiles);
     p.waves = (p.grid <= 256) ? 16 : 8;  // as the few-rows kernel: one workgroup per CU gets more waves
     if (p.waves > chunks) p.waves = chunks;
