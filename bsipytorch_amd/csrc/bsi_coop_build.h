@@ -33,6 +33,7 @@ namespace bsi {
 
 constexpr int kXcds = 8;
 constexpr int kCoopShares = 32;       // shares of a copy at most: one workgroup for each CU of an XCD
+constexpr int kCoopHeld = 8;          // chunks of a row that a wave builds by itself
 constexpr int kCoopMaxItems = 1024;   // (row, chunk) items: 256 bytes of image and a scale each
 constexpr size_t kCoopFlagBytes = kXcds * kCoopShares * sizeof(unsigned long long);
 constexpr size_t kCoopCopyBytes = static_cast<size_t>(kCoopMaxItems) * (BSI_CHUNK_ELEMS + sizeof(float));
@@ -50,6 +51,7 @@ struct CoopBuild {
     int dtype, vec;             // BSI_DTYPE_*; rows can be loaded a quad at a time
     int rows, chunks, slices;
     int by_row;                 // one scale a row instead of one a chunk
+    int row_per_wave;           // by_row: a wave builds a row (of kCoopHeld chunks at most) by itself: instances of their own
     int shares;                 // of a copy: chunk scales split the items, row scales the rows
     int patience;               // ticks until a workgroup builds what it waits for
 };
@@ -81,13 +83,13 @@ __device__ __forceinline__ int coop_scale_at(const CoopBuild& b, int row, int ch
 }
 
 // Row scales: the row's largest magnitude over the waves, then its quantised chunks.
-template <typename T, bool kVec, bool kFragments>
+template <typename T, bool kVec, bool kFragments, bool kRowPerWave>
 __device__ void coop_build_share(const CoopBuild& b, int share, int wave, int nwaves, int lane, uint32_t* __restrict__ image,
                                  float* __restrict__ scales, unsigned* __restrict__ wave_max) {
     const ChunkLane cl = chunk_lane(lane);
     const QuantRange range = quant_range(b.slices);
     const T* const x = static_cast<const T*>(b.x);
-    if (!b.by_row) {
+    if (!kRowPerWave && !b.by_row) {
         const int items = b.rows * b.chunks;
         const int first = items * share / b.shares, last = items * (share + 1) / b.shares;
         auto load = [&](int item, float (&v)[4]) {
@@ -118,6 +120,52 @@ __device__ void coop_build_share(const CoopBuild& b, int share, int wave, int nw
         return;
     }
     const int first = b.rows * share / b.shares, last = b.rows * (share + 1) / b.shares;
+    if constexpr (kRowPerWave) {
+#pragma unroll 1
+        for (int row = first + wave; row < last; row += nwaves) {
+            const T* const xrow = x + row * b.d;
+            unsigned mx = kQuantWideBits;
+            if constexpr (kVec) {
+                float held[kCoopHeld][4];
+#pragma unroll
+                for (int c = 0; c < kCoopHeld; ++c) load_chunk_quad<T, true>(xrow, b.d, c, cl, held[c]);  // past the row: zeros
+                mx = 0u;
+#pragma unroll
+                for (int c = 0; c < kCoopHeld; ++c) {
+                    const unsigned m = quad_max_bits(held[c]);
+                    mx = m > mx ? m : mx;
+                }
+                mx = wave_max_u32(mx);
+                if (mx < kQuantWideBits) {
+                    const int shift = quant_shift(mx, b.scale, b.slices);
+                    if (lane == 0) scales[row] = static_cast<float>(1ULL << shift);
+#pragma unroll
+                    for (int c = 0; c < kCoopHeld; ++c)
+                        if (c < b.chunks)
+                            image[coop_image_at<kFragments>(b, row, c, lane)] = chunk_image_dword(quantise_quad<T>(held[c], b.scale, shift, range), cl);
+                }
+            }
+            if (mx >= kQuantWideBits) {  // rare, as are rows that no quad can be loaded from: the general routine, a chunk at a time
+                unsigned long long m64 = 0ULL;
+#pragma unroll 1
+                for (int c = 0; c < b.chunks; ++c) {
+                    float v[4];
+                    load_chunk_quad<T, kVec>(xrow, b.d, c, cl, v);
+                    const unsigned long long m = quad_max_wide(v, b.dec_scale);
+                    m64 = m > m64 ? m : m64;
+                }
+                const int shift = compute_shift(wave_max_u64(m64), 0.0, 1, b.slices, 0.0f);
+                if (lane == 0) scales[row] = static_cast<float>(1ULL << shift);
+#pragma unroll 1
+                for (int c = 0; c < b.chunks; ++c) {
+                    float v[4];
+                    load_chunk_quad<T, kVec>(xrow, b.d, c, cl, v);
+                    image[coop_image_at<kFragments>(b, row, c, lane)] = chunk_image_dword(quantise_quad_wide(v, b.dec_scale, shift, b.slices), cl);
+                }
+            }
+        }
+        return;
+    }
 #pragma unroll 1
     for (int row = first; row < last; ++row) {
         const T* const xrow = x + row * b.d;
@@ -166,7 +214,7 @@ __device__ void coop_build_share(const CoopBuild& b, int share, int wave, int nw
 // to the whole build, in the copy of the XCD the workgroup runs on.  ahead(): loads for after the build, of anything but the
 // area.  Every wave but wave 0 issues them when the workgroup's share is built (a CU's loads return in order: not before),
 // wave 0, which asks for the flags, when all shares are.
-template <bool kFragments, typename F>
+template <bool kFragments, bool kRowPerWave, typename F>
 __device__ __forceinline__ void coop_build(const CoopBuild& b, unsigned id, unsigned* __restrict__ shared, const int8_t*& A8,
                                            const float*& qscale, F&& ahead) {
     const int lane = threadIdx.x & (BSI_WAVE - 1);
@@ -180,14 +228,14 @@ __device__ __forceinline__ void coop_build(const CoopBuild& b, unsigned id, unsi
     bool issued = false;
     auto build = [&](int share) {
         if (b.dtype == BSI_DTYPE_F32) {
-            if (b.vec) coop_build_share<float, true, kFragments>(b, share, wave, nwaves, lane, image, scales, shared);
-            else coop_build_share<float, false, kFragments>(b, share, wave, nwaves, lane, image, scales, shared);
+            if (b.vec) coop_build_share<float, true, kFragments, kRowPerWave>(b, share, wave, nwaves, lane, image, scales, shared);
+            else coop_build_share<float, false, kFragments, kRowPerWave>(b, share, wave, nwaves, lane, image, scales, shared);
         } else if (b.dtype == BSI_DTYPE_F16) {
-            if (b.vec) coop_build_share<__half, true, kFragments>(b, share, wave, nwaves, lane, image, scales, shared);
-            else coop_build_share<__half, false, kFragments>(b, share, wave, nwaves, lane, image, scales, shared);
+            if (b.vec) coop_build_share<__half, true, kFragments, kRowPerWave>(b, share, wave, nwaves, lane, image, scales, shared);
+            else coop_build_share<__half, false, kFragments, kRowPerWave>(b, share, wave, nwaves, lane, image, scales, shared);
         } else {
-            if (b.vec) coop_build_share<__hip_bfloat16, true, kFragments>(b, share, wave, nwaves, lane, image, scales, shared);
-            else coop_build_share<__hip_bfloat16, false, kFragments>(b, share, wave, nwaves, lane, image, scales, shared);
+            if (b.vec) coop_build_share<__hip_bfloat16, true, kFragments, kRowPerWave>(b, share, wave, nwaves, lane, image, scales, shared);
+            else coop_build_share<__hip_bfloat16, false, kFragments, kRowPerWave>(b, share, wave, nwaves, lane, image, scales, shared);
         }
         const int items = b.rows * b.chunks, had = items * (share + 1) / b.shares - items * share / b.shares;
         if (b.by_row || wave < had) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the wave's stores have reached the L2

@@ -377,7 +377,8 @@ extern "C" int bsi_hip_linear_out(const void* x, int dtype, int64_t Q, int64_t d
 
 extern "C" size_t bsi_hip_linear_coop_bytes(void) { return kCoopBytes; }
 
-extern "C" int bsi_hip_linear_coop_serves(int64_t Q, int64_t d, int64_t R, int decimal_places, int fixed_bits, int b_layout, int Sb) {
+// 0: not served; 1: a wave of the build takes a chunk at a time; 2: a whole row (kCoopHeld chunks at most)
+static int coop_plan(int64_t Q, int64_t d, int64_t R, int decimal_places, int fixed_bits, int b_layout, int Sb) {
     const int64_t chunks = (d + 255) / 256;
     if (Q < 1 || d < 1 || R < 1 || Q * chunks > kCoopMaxItems || decimal_places < 0 || decimal_places > 2 || fixed_bits < 2 || fixed_bits > 8)
         return 0;
@@ -393,11 +394,23 @@ extern "C" int bsi_hip_linear_coop_serves(int64_t Q, int64_t d, int64_t R, int d
     // Chunks that a wave of the build takes one after the other, each a load's latency: up to two chunk-scaled ones or one
     // of a row (which has barriers besides) cost less than a launch.  us a pass, two launches and one: 16 x 512 x 1280 6.6, 4.8;
     // 15 x 2560 x 5888 8.4, 7.3; 28 x 3072 x 4864 11.5, 10.6; 49 x 512 x 3328 6.9, 5.7; 121 x 512 x 14848 8.8, 8.1 -- beyond:
-    // 80 x 2304 x 4352 (4 rounds) 8.5, 8.9; 37 x 704 x 9728 (2 rows) 6.8, 7.6; 24 x 2304 x 256 7.4, 13.9.
+    // 80 x 2304 x 4352 (4 rounds) 8.5, 8.9; 24 x 2304 x 256 7.4, 13.9.
     const bool by_row = ((d + 63) / 64) % 4 != 0;
     const int shares = coop_shares(groups, static_cast<int>(by_row ? Q : Q * chunks));
-    if (by_row) return Q <= shares && chunks <= waves ? 1 : 0;
+    if (by_row) {
+        if (Q <= shares && chunks <= waves) return 1;
+        // A wave a row, for more rows: one load's latency too, but longer work and copies.  us, two launches (on a host that issues
+        // them in 8.4, and on one that takes 9.8) and one: 24 x 704 x 704 8.4, 9.5, 6.6; 24 x 1600 x 1600 8.1, 9.5, 6.6; 100 x 320 x
+        // 2000 8.5, 9.8, 6.8; 37 x 704 x 9728 8.5, 9.9, 7.0; 250 x 100 x 8192 8.7, 10.1, 7.6; 64 x 1600 x 4800 8.4, 9.8, 8.3; 77 x 1600 x
+        // 4800 8.7, 9.9, 8.8 -- beyond: 121 x 1600 x 6400 (847 items) 8.9, 9.8, 9.7; 128 x 832 x 12000 (376 workgroups, whose registers
+        // leave a CU one of them) 9.3, 9.9, 9.7.
+        return Q <= static_cast<int64_t>(shares) * waves && chunks <= kCoopHeld && d % 4 == 0 && Q * chunks <= 560 && groups <= 256 ? 2 : 0;
+    }
     return Q * chunks <= 2 * static_cast<int64_t>(shares) * waves ? 1 : 0;
+}
+
+extern "C" int bsi_hip_linear_coop_serves(int64_t Q, int64_t d, int64_t R, int decimal_places, int fixed_bits, int b_layout, int Sb) {
+    return coop_plan(Q, d, R, decimal_places, fixed_bits, b_layout, Sb) != 0 ? 1 : 0;
 }
 
 extern "C" int bsi_hip_linear_coop_out(const void* x, int dtype, int64_t Q, int64_t d, int decimal_places, int fixed_bits, uint64_t launch_number,
@@ -406,7 +419,8 @@ extern "C" int bsi_hip_linear_coop_out(const void* x, int dtype, int64_t Q, int6
                                        void* stream) {
     BSI_REQUIRE(out_dtype == BSI_DTYPE_F32 || out_dtype == BSI_DTYPE_F16 || out_dtype == BSI_DTYPE_BF16, "unknown dtype code %d", out_dtype);
     BSI_REQUIRE(dtype == BSI_DTYPE_F32 || dtype == BSI_DTYPE_F16 || dtype == BSI_DTYPE_BF16, "unknown dtype code %d", dtype);
-    if (!bsi_hip_linear_coop_serves(Q, d, R, decimal_places, fixed_bits, b_layout, Sb))
+    const int plan = coop_plan(Q, d, R, decimal_places, fixed_bits, b_layout, Sb);
+    if (plan == 0)
         return fail(BSI_ERR_UNSUPPORTED, "no launch with the query build inside for this layer");
     BSI_REQUIRE(x != nullptr && area != nullptr && launch_number != 0, "null pointer or launch number");
     BSI_REQUIRE((reinterpret_cast<uintptr_t>(area) & 255) == 0, "the area must be 256-byte aligned");
@@ -427,6 +441,7 @@ extern "C" int bsi_hip_linear_coop_out(const void* x, int dtype, int64_t Q, int6
     c.slices = fixed_bits;
     c.patience = g_coop_patience.load(std::memory_order_relaxed);
     c.by_row = W64 % 4 == 0 ? 0 : 1;  // the builder's rule
+    c.row_per_wave = plan == 2 ? 1 : 0;
     t_coop = &c;
     t_out_dtype = out_dtype;
     // the operands stand for the launch's own copies

@@ -40,13 +40,13 @@ constexpr int kStreamLds = kStreamLdsInts * 4 + 4096 + 16 * 2048;  // with their
 // 11.9; 24 x 8192 x 8192 18.7, 14.8; 32 x 4096 x 4096 7.6, 6.1; 16 x 8192 x 32768 44.8, 41.0; 8 x 16384 x 4096 12.6, 11.9;
 // 1 x 4096 x 32768 21.6, 21.5; 8 x 8192 x 16384 21.5, 21.5.  All 4 KiB of a chunk at once, in LDS of its own: 12.0 for the first,
 // but 22.5 for the last (a workgroup less on a CU).
-template <int NT, int KT, bool kInts, bool kBuild>
+template <int NT, int KT, bool kInts, int kBuild>
 __global__ __launch_bounds__(1024) void dot_mfma_stream_kernel(
     const int8_t* A8, const float* qscale, int qscale_stride,
     const unsigned long long* __restrict__ B64,  // tiled key planes, Sb = 6
     const float* __restrict__ Bw, int chunks, int pass_chunks, int64_t R, int64_t Q, int down_shift, float scale_inv,
     int64_t R_total, float* __restrict__ out, int* __restrict__ chunk_ints, const float* __restrict__ bias, int out_dtype,
-    std::conditional_t<kBuild, CoopBuild, int> coop) {
+    std::conditional_t<kBuild != 0, CoopBuild, int> coop) {
     // [pass_chunks][KT][NT][16 queries][16 keys], then the chunks' scales, [pass_chunks][NT][16 queries]; without kBuild a chunk's
     // query rows are turned round where its sums will lie, or, if those have no 2 KiB, in 2 KiB a wave behind all that
     extern __shared__ __attribute__((aligned(16))) int ints[];
@@ -85,7 +85,7 @@ __global__ __launch_bounds__(1024) void dot_mfma_stream_kernel(
             }
     };
     if constexpr (kBuild)
-        coop_build<true>(coop, blockIdx.x, reinterpret_cast<unsigned*>(ints), A8, qscale, [&] { load_keys(wave < pass_chunks ? wave : pass_chunks - 1); });
+        coop_build<true, kBuild == 2>(coop, blockIdx.x, reinterpret_cast<unsigned*>(ints), A8, qscale, [&] { load_keys(wave < pass_chunks ? wave : pass_chunks - 1); });
 
     // the chain lanes: tid <-> (key tile, query tile, query, key), keys fastest so output stores are contiguous
     float accf = 0.0f;
@@ -612,12 +612,13 @@ static void launch_mfma_stream(const int8_t* A8, const float* qscale, int stride
                reinterpret_cast<const unsigned long long*>(B), Bw, chunks, pass_chunks, R, Q, down_shift, scale_inv, R_total, \
                out, chunk_ints, bias, t_out_dtype, COOP);                                                                     \
     } while (0)
-    if (chunk_ints) BSI_STREAM_GO(true, false, 0);
-    else if (t_coop == nullptr) BSI_STREAM_GO(false, false, 0);
+    if (chunk_ints) BSI_STREAM_GO(true, 0, 0);
+    else if (t_coop == nullptr) BSI_STREAM_GO(false, 0, 0);
     else {
         CoopBuild coop = *t_coop;
         coop.shares = coop_shares(grid.x, coop.by_row ? coop.rows : coop.rows * coop.chunks);
-        BSI_STREAM_GO(false, true, coop);
+        if (coop.row_per_wave) BSI_STREAM_GO(false, 2, coop);
+        else BSI_STREAM_GO(false, 1, coop);
     }
 #undef BSI_STREAM_GO
 }

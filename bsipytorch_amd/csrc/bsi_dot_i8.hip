@@ -514,7 +514,7 @@ __device__ __forceinline__ void i8_tile_of(const I8Grid& g, unsigned id, int& bx
     by = static_cast<int>(first + in - x * (last ? left : static_cast<unsigned>(g.height)));
 }
 
-template <int TM, int TN, int kMode, bool kSplit, bool kBuild, bool kFour, bool kHalf>
+template <int TM, int TN, int kMode, bool kSplit, int kBuild, bool kFour, bool kHalf>
 __global__ __launch_bounds__((I8Cfg<TM, TN>::kBlock)) void dot_mfma_i8_kernel(
     const int8_t* A8, const float* qscale, int qscale_stride,
     const int8_t* __restrict__ K8,  // int8 key image [R, chunks * 256]
@@ -551,7 +551,7 @@ __global__ __launch_bounds__((I8Cfg<TM, TN>::kBlock)) void dot_mfma_i8_kernel(
     constexpr int WM = C::kWM, WN = C::kWN;
     constexpr bool kInts = (kMode == kI8Ints), kSum = (kMode == kI8Sum);
     extern __shared__ __attribute__((aligned(16))) unsigned char lds[];  // C::kLds
-    if (kBuild) coop_build<false>(coop, blockIdx.y * gridDim.x + blockIdx.x, reinterpret_cast<unsigned*>(lds), A8, qscale, [] {});
+    if constexpr (kBuild != 0) coop_build<false, kBuild == 2>(coop, blockIdx.y * gridDim.x + blockIdx.x, reinterpret_cast<unsigned*>(lds), A8, qscale, [] {});
 
     const int tid = threadIdx.x;
     const int lane = tid & 63;
@@ -1855,17 +1855,22 @@ static void launch_mfma_i8_tm(const int8_t* A8, const float* qscale, int stride,
         if (t_coop != nullptr) {
             CoopBuild coop = *t_coop;
             coop.shares = coop_shares(grid.x * grid.y, coop.by_row ? coop.rows : coop.rows * coop.chunks);
-            static LdsOptIn once;
-            lds_opt_in(once, reinterpret_cast<const void*>(&dot_mfma_i8_kernel<TM, TN, kI8Chain, false, true, false, kHalf>), C::kLds);
-            launch((dot_mfma_i8_kernel<TM, TN, kI8Chain, false, true, false, kHalf>), grid, dim3(C::kBlock), C::kLds, st, A8, qscale, stride, K8, Bw, Sb,
-                   chunks, R, Q, down_shift, scale_inv, R_total, out, chunk_ints, bias, ndig, dig_stride, key_indices, key_tiled,
-                   static_cast<const unsigned char*>(g_warm_ptr), static_cast<long long>(g_warm_bytes / 128), stream_output(),
-                   static_cast<float*>(nullptr), static_cast<unsigned*>(nullptr), 0.0f, 0, g, t_out_dtype, coop);
+            const auto go = [&](auto build) {
+                constexpr int kBuild = decltype(build)::value;
+                static LdsOptIn once;
+                lds_opt_in(once, reinterpret_cast<const void*>(&dot_mfma_i8_kernel<TM, TN, kI8Chain, false, kBuild, false, kHalf>), C::kLds);
+                launch((dot_mfma_i8_kernel<TM, TN, kI8Chain, false, kBuild, false, kHalf>), grid, dim3(C::kBlock), C::kLds, st, A8, qscale, stride, K8, Bw,
+                       Sb, chunks, R, Q, down_shift, scale_inv, R_total, out, chunk_ints, bias, ndig, dig_stride, key_indices, key_tiled,
+                       static_cast<const unsigned char*>(g_warm_ptr), static_cast<long long>(g_warm_bytes / 128), stream_output(),
+                       static_cast<float*>(nullptr), static_cast<unsigned*>(nullptr), 0.0f, 0, g, t_out_dtype, coop);
+            };
+            if (coop.row_per_wave) go(std::integral_constant<int, 2>{});
+            else go(std::integral_constant<int, 1>{});
             return;
         }
     static LdsOptIn once0;
-    lds_opt_in(once0, reinterpret_cast<const void*>(&dot_mfma_i8_kernel<TM, TN, kMode, false, false, kFour, kHalf>), C::kLds);
-    launch((dot_mfma_i8_kernel<TM, TN, kMode, false, false, kFour, kHalf>), grid, dim3(C::kBlock), C::kLds, st, A8, qscale, stride, K8,
+    lds_opt_in(once0, reinterpret_cast<const void*>(&dot_mfma_i8_kernel<TM, TN, kMode, false, 0, kFour, kHalf>), C::kLds);
+    launch((dot_mfma_i8_kernel<TM, TN, kMode, false, 0, kFour, kHalf>), grid, dim3(C::kBlock), C::kLds, st, A8, qscale, stride, K8,
                        Bw, Sb, chunks, R, Q, down_shift, scale_inv, R_total, out, chunk_ints, bias, ndig, dig_stride,
                        key_indices, key_tiled, static_cast<const unsigned char*>(g_warm_ptr),
                        static_cast<long long>(g_warm_bytes / 128), stream_output(), static_cast<float*>(nullptr),
@@ -1888,8 +1893,8 @@ static void launch_mfma_i8_split(int segments, unsigned char* scratch, const int
     while ((1 << log2_segments) < segments) ++log2_segments;
     const float limit = __builtin_ldexpf(1.0f, 24 + down_shift - log2_segments);
     static LdsOptIn once0;
-    lds_opt_in(once0, reinterpret_cast<const void*>(&dot_mfma_i8_kernel<TM, TN, kI8Chain, true, false, false, kHalf>), C::kLdsSplit);
-    launch((dot_mfma_i8_kernel<TM, TN, kI8Chain, true, false, false, kHalf>), grid, dim3(C::kBlock), C::kLdsSplit, st, A8, qscale,
+    lds_opt_in(once0, reinterpret_cast<const void*>(&dot_mfma_i8_kernel<TM, TN, kI8Chain, true, 0, false, kHalf>), C::kLdsSplit);
+    launch((dot_mfma_i8_kernel<TM, TN, kI8Chain, true, 0, false, kHalf>), grid, dim3(C::kBlock), C::kLdsSplit, st, A8, qscale,
                        stride, K8, Bw, Sb, chunks, R, Q, down_shift, scale_inv, R_total, out, static_cast<int*>(nullptr), bias,
                        1, 0LL, static_cast<const long long*>(nullptr), key_tiled,
                        static_cast<const unsigned char*>(g_warm_ptr), static_cast<long long>(g_warm_bytes / 128),
