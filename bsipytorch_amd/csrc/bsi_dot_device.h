@@ -138,6 +138,16 @@ __device__ __forceinline__ uint32_t half_output(float v, bool has_bias, float bi
     const uint32_t h = half_bits(v, dtype);
     return has_bias ? half_bits(half_value(h, dtype) + half_value(half_bits(bias, dtype), dtype), dtype) : h;
 }
+// Two outputs of a known type in one dword.  kBias: b0, b1 are biases rounded to the type already.
+template <int kType, bool kBias>
+__device__ __forceinline__ uint32_t half_pair(float v0, float v1, float b0, float b1) {
+    typedef float v2f __attribute__((ext_vector_type(2)));
+    using Half = std::conditional_t<kType == BSI_DTYPE_F16, _Float16, __bf16>;
+    typedef Half v2h __attribute__((ext_vector_type(2)));
+    uint32_t h = __builtin_bit_cast(uint32_t, __builtin_convertvector((v2f){v0, v1}, v2h));
+    if (kBias) h = __builtin_bit_cast(uint32_t, __builtin_convertvector((v2f){half_value(h & 0xFFFFu, kType) + b0, half_value(h >> 16, kType) + b1}, v2h));
+    return h;
+}
 // Element i of an output of any of the three types.
 __device__ __forceinline__ void store_output(float* out, size_t i, float v, bool has_bias, float bias, int dtype) {
     if (dtype == BSI_DTYPE_F32) out[i] = has_bias ? v + bias : v;
