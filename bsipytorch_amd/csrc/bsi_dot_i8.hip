@@ -1968,9 +1968,12 @@ static void launch_mfma_i8w(const int8_t* A8, const float* qscale, int stride, c
 }
 
 // The large layers' launches: the images in units, the integer sums, and the chain for what they leave.  The rule, in us: a round of
-// 256 workgroups takes 1.07 a chunk and 0.5 with tiles of 128 x 128, 3.3 and 2.7 with tiles of 256 x 256; the images are written at
-// 0.75 a million elements; the launch that ends at once and the gaps are 7.  Measured, 128 x 128 and 256 x 256, at its edges:
-// 2048 x 2048 x 16384 88.6, 84.4 and 1024 x 4096 x 16384 80, 77 (taken); 2048 x 2048 x 8192 49, 56 and 3000 x 1600 x 12000 93, 108 (not).
+// 256 workgroups takes 1 a chunk and 1 with tiles of 128 x 128; with tiles of 256 x 256 2.95 a chunk and 2, and 8 more for each round
+// but the last (all CUs store 32 MiB at the same time, with nothing else of theirs resident); the images are written at 0.75 a
+// million elements; the launch that ends at once and the gaps are 14.  Measured, 128 x 128 and 256 x 256, bf16: taken 1024 x 4096 x
+// 16384 73.6, 69.3; 4096 x 3072 x 16384 225, 207; 2048 x 8192 x 8192 150, 128.5; 1024 x 8192 x 16384 165, 123; not taken 4096 x 1024 x
+// 16384 92, 99; 4096 x 2048 x 16384 155, 160 (f32 176, 188); 4096 x 2048 x 8192 78, 85; 2048 x 4096 x 8192 74, 75 (f32 78, 81);
+// 4096 x 4096 x 4096 78, 80; 3000 x 4096 x 11008 160, 172; and, at its edge, 2048 x 2048 x 16384 81, 77 (f32 88, 88).
 static size_t large_aligned(size_t v) { return (v + 255) / 256 * 256; }
 size_t i8_large_workspace_bytes(int64_t Q, int chunks) {
     if (Q < kLargeMinQ || chunks > kLargeMaxChunks) return 0;
@@ -1987,8 +1990,8 @@ bool i8_large_serves(int64_t Q, int64_t R, int chunks) {
     if (small * chunks >= (int64_t{1} << 29) || large * ((R + kLargeTile - 1) / kLargeTile) >= (int64_t{1} << 29)) return false;
     if (forced == kLargeTile) return true;
     if (small <= kCus) return false;
-    const double us_small = static_cast<double>((small + kCus - 1) / kCus) * (1.07 * chunks + 0.5);
-    const double us_large = static_cast<double>((large + kCus - 1) / kCus) * (3.3 * chunks + 2.7) + 7.0 + 7.5e-7 * static_cast<double>(Q) * chunks * 256;
+    const double us_small = static_cast<double>((small + kCus - 1) / kCus) * (chunks + 1.0);
+    const double us_large = static_cast<double>((large + kCus - 1) / kCus) * (2.95 * chunks + 10.0) + 6.0 + 7.5e-7 * static_cast<double>(Q) * chunks * 256;
     return us_large < us_small;
 }
 
