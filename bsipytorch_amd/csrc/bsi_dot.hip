@@ -348,18 +348,26 @@ extern "C" int bsi_hip_linear_out(const void* x, int dtype, int64_t Q, int64_t d
     // BSI_CORE_AUTO falls back to for wide keys), and where the builder cannot leave them out.
     const bool planes = core == BSI_CORE_VALU || Sb < 2 || Sb > 8 || chunks > kMfmaMaxChunks ||
                         integer_decimal_scale(pow(10.0, static_cast<double>(decimal_places))) == 0;
-    if (rebuild) {
+    const bool large = core == BSI_CORE_AUTO && b_layout == BSI_LAYOUT_INT8 && Sb >= 2 && Sb <= 8 && R_total >= R && R <= (1 << 25) && B != nullptr &&
+                       Bw != nullptr && out != nullptr && (reinterpret_cast<uintptr_t>(B) & 15) == 0 && i8_large_serves(Q, R, chunks);
+    const bool units_there = rebuild && large && chunk_scale && !planes && Q <= 0x7fffffffLL / chunks;  // the units come out of the build
+    if (units_there) {
+        BSI_REQUIRE(dtype == BSI_DTYPE_F32 || dtype == BSI_DTYPE_F16 || dtype == BSI_DTYPE_BF16, "unknown dtype code %d", dtype);
+        BSI_REQUIRE(x != nullptr, "null pointer");
+        launch_build_units(ws + w.large, x, dtype, Q, d, fixed_bits, Sb, pow(10.0, static_cast<double>(decimal_places)), shifts, scales, ints8, chunks,
+                           as_stream(stream));
+        BSI_LAUNCH_CHECK("build_units_kernel");
+    } else if (rebuild) {
         const int rc = bsi_hip_build_fixed(x, dtype, Q, d, decimal_places, fixed_bits, chunk_scale, 0.0f, planes ? words : nullptr,
                                            shifts, scales, ints8, stream);
         if (rc != BSI_OK) return rc;
     }
     t_out_dtype = out_dtype;
-    if (core == BSI_CORE_AUTO && b_layout == BSI_LAYOUT_INT8 && Sb >= 2 && Sb <= 8 && R_total >= R && R <= (1 << 25) && B != nullptr && Bw != nullptr &&
-        out != nullptr && (reinterpret_cast<uintptr_t>(B) & 15) == 0 && i8_large_serves(Q, R, chunks)) {
+    if (large) {
         g_warm_ptr = warm;
         g_warm_bytes = warm != nullptr ? warm_bytes : 0;
         t_layer_output = 1;
-        launch_i8_large(ws + w.large, ints8, scales, chunk_scale ? chunks : 1, reinterpret_cast<const int8_t*>(B), Bw, fixed_bits, Sb, chunks, R, Q,
+        launch_i8_large(ws + w.large, units_there, ints8, scales, chunk_scale ? chunks : 1, reinterpret_cast<const int8_t*>(B), Bw, fixed_bits, Sb, chunks, R, Q,
                         scale_inv, R_total, static_cast<float*>(out), bias, as_stream(stream));
         g_warm_ptr = nullptr;
         g_warm_bytes = 0;

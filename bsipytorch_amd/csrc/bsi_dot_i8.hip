@@ -1233,6 +1233,55 @@ constexpr uint32_t kNowhere = 0x80000000u;  // past the end of every operand
 
 // The images in units and what the dot needs to know of a row.  lo / hi: [Q][chunks * 256]; masks: [Q][words] of 64 blocks;
 // units: [Q], the factor of the row's sums, negative where the row has to go through the chain.
+// Four elements in units: their bytes in either image.  exponent: of their scale, 255 where all are zero; least: of the row's unit.
+__device__ __forceinline__ void unit_bytes(uint32_t in, unsigned exponent, unsigned least, int Sa, uint32_t& low_bytes, uint32_t& high_bytes,
+                                           unsigned& total, unsigned& odd) {
+    int up = exponent == 255u ? 0 : static_cast<int>(exponent - least) - (8 - Sa);  // the image holds a << (8 - Sa)
+    if (up <= 0) {  // nearly all: every element is in the lower image, the four of them shifted together
+        const uint32_t sign = in >> 7 & 0x01010101u, keep = (0xFFu >> -up) * 0x01010101u;
+        low_bytes = (in >> -up & keep) | sign * (0xFFu & ~(0xFFu >> -up));
+        high_bytes = 0u;
+        total = __builtin_amdgcn_sad_u8(low_bytes ^ 0x80808080u, 0x80808080u, total);  // |a| is the distance of a + 128 and 128
+        return;
+    }
+    if (up > 8) {
+        odd = 1u;
+        up = 8;
+    }
+    low_bytes = high_bytes = 0u;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        const int a = (static_cast<int>(in << (24 - 8 * k)) >> 24) << up;
+        const int low = static_cast<int>(static_cast<uint32_t>(a) << 24) >> 24;
+        total += static_cast<unsigned>(a < 0 ? -a : a);
+        low_bytes |= (static_cast<uint32_t>(a) & 255u) << (8 * k);
+        high_bytes |= (static_cast<uint32_t>((a - low) >> 8) & 255u) << (8 * k);
+    }
+}
+// The factor of a row's sums, from what its waves have found; leaves with all of them past a barrier.
+template <int kWaves>
+__device__ __forceinline__ void unit_of_row(unsigned (&shared)[3][kWaves], int lane, int wave, unsigned total, unsigned odd, unsigned least, int Sb,
+                                            float* __restrict__ unit) {
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) total += __shfl_xor(total, o, BSI_WAVE);
+    const bool any_odd = __ballot(odd != 0u) != 0ull;
+    if (lane == 0) {
+        shared[1][wave] = total;
+        shared[2][wave] = any_odd ? 1u : 0u;
+    }
+    __syncthreads();
+    if (wave == 0 && lane == 0) {
+        unsigned long long sum = 0ull;
+        unsigned bad = 0u;
+        for (int w = 0; w < kWaves; ++w) {
+            sum += shared[1][w];
+            bad |= shared[2][w];
+        }
+        if (least == 255u) least = 127u;  // a row of zeros
+        // the key image holds b << (8 - Sb), |b| <= 2^(Sb - 1)
+        *unit = bad != 0u || (sum << (Sb - 1)) > (1ull << 24) ? -1.0f : __uint_as_float((least - static_cast<unsigned>(8 - Sb)) << 23);
+    }
+}
 constexpr int kUnitsBlock = 256, kUnitsHeld = kLargeMaxChunks * 16 / kUnitsBlock;
 __global__ __launch_bounds__(kUnitsBlock) void i8_units_kernel(const int8_t* __restrict__ A8, const float* __restrict__ qscale, int stride,
                                                                int chunks, int Sa, int Sb, uint4* __restrict__ lo, uint4* __restrict__ hi,
@@ -1269,26 +1318,10 @@ __global__ __launch_bounds__(kUnitsBlock) void i8_units_kernel(const int8_t* __r
     for (int j = 0; j < kUnitsHeld; ++j) {
         const int p = tid + j * kUnitsBlock, at = wave + j * kUnitsWaves;
         if (at >= mask_pieces) break;  // the whole wave
-        int up = exponent[j] == 255u ? 0 : static_cast<int>(exponent[j] - least) - (8 - Sa);  // the image holds a << (8 - Sa)
-        if (up > 8) {
-            odd = 1u;
-            up = 8;
-        }
-        const int left = up > 0 ? up : 0, right = up < 0 ? -up : 0;
         uint32_t l[4], h[4];
         const uint32_t in[4] = {v[j].x, v[j].y, v[j].z, v[j].w};
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            l[i] = h[i] = 0u;
-#pragma unroll
-            for (int k = 0; k < 4; ++k) {
-                const int a = ((static_cast<int>(in[i] << (24 - 8 * k)) >> 24) << left) >> right;
-                const int low = static_cast<int>(static_cast<uint32_t>(a) << 24) >> 24;
-                total += static_cast<unsigned>(a < 0 ? -a : a);
-                l[i] |= (static_cast<uint32_t>(a) & 255u) << (8 * k);
-                h[i] |= (static_cast<uint32_t>((a - low) >> 8) & 255u) << (8 * k);
-            }
-        }
+        for (int i = 0; i < 4; ++i) unit_bytes(in[i], exponent[j], least, Sa, l[i], h[i], total, odd);
         // four neighbouring lanes hold a block of 64 elements
         const unsigned long long any = __ballot((h[0] | h[1] | h[2] | h[3]) != 0u);
         unsigned long long m = (any | any >> 1 | any >> 2 | any >> 3) & 0x1111111111111111ull;
@@ -1302,24 +1335,83 @@ __global__ __launch_bounds__(kUnitsBlock) void i8_units_kernel(const int8_t* __r
             hi[row * pieces + p] = make_uint4(h[0], h[1], h[2], h[3]);
         }
     }
+    unit_of_row<kUnitsWaves>(shared, lane, wave, total, odd, least, Sb, units + row);
+}
+
+// The same with the build: a workgroup quantises a row, a chunk a wave at a time, and has the row's unit before it stores the
+// chunks.  For layers with chunk scales; writes what build_fixed_chunk_fast_kernel and then i8_units_kernel do, and does not read the
+// image, which only the chain looks at, again.  us, those two and this: 4096 x 4096 bf16 26.9, 22.3 (84 MB, 3.8 TB/s; 23.8 with the
+// shifts of unit_bytes an element at a time); a layer 4096 x 4096 x 16384 bf16 249, 245; 1024 x 4096 x 16384 70.3, 67.9; 2048 x 8192
+// x 8192 f32 134.4, 132; 4096 x 3072 x 16384 f16 211, 205.
+template <typename T, bool kVec, int kHeld>
+__global__ __launch_bounds__(kUnitsBlock) void build_units_kernel(const T* __restrict__ x, int64_t d, int chunks, int Sa, int Sb, double dec_scale,
+                                                                  float scale, int* __restrict__ shifts, float* __restrict__ scales,
+                                                                  uint32_t* __restrict__ image, uint32_t* __restrict__ lo, uint32_t* __restrict__ hi,
+                                                                  unsigned long long* __restrict__ masks, float* __restrict__ units) {
+    constexpr int kUnitsWaves = kUnitsBlock / 64;
+    __shared__ unsigned shared[3][kUnitsWaves];
+    __shared__ unsigned blocks[kLargeMaxChunks];  // of a chunk, which of its four blocks are in the upper image
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const size_t row = blockIdx.x;
+    const T* const src = x + row * static_cast<size_t>(d);
+    const ChunkLane cl = chunk_lane(lane);
+    const QuantRange range = quant_range(Sa);
+    if (tid < kLargeMaxChunks) blocks[tid] = 0u;
+    float v[kHeld][4];
 #pragma unroll
-    for (int o = 32; o > 0; o >>= 1) total += __shfl_xor(total, o, BSI_WAVE);
-    const bool any_odd = __ballot(odd != 0u) != 0ull;
-    if (lane == 0) {
-        shared[1][wave] = total;
-        shared[2][wave] = any_odd ? 1u : 0u;
-    }
-    __syncthreads();
-    if (tid == 0) {
-        unsigned long long sum = 0ull;
-        unsigned bad = 0u;
-        for (int w = 0; w < kUnitsWaves; ++w) {
-            sum += shared[1][w];
-            bad |= shared[2][w];
+    for (int j = 0; j < kHeld; ++j) load_chunk_quad<T, kVec>(src, d, wave + j * kUnitsWaves, cl, v[j]);  // past the row: zeros
+    uint32_t held[kHeld];
+    unsigned exponent[kHeld], least = 255u, odd = 0u, total = 0u;
+#pragma unroll
+    for (int j = 0; j < kHeld; ++j) {
+        const int c = wave + j * kUnitsWaves;
+        held[j] = 0u;
+        exponent[j] = 255u;
+        if (c >= chunks) continue;
+        const unsigned mx = wave_max_u32(quad_max_bits(v[j]));
+        int shift;
+        uint32_t bytes;
+        if (mx < kQuantWideBits) {
+            shift = quant_shift(mx, scale, Sa);
+            bytes = quantise_quad<T>(v[j], scale, shift, range);
+        } else {
+            shift = compute_shift(wave_max_u64(quad_max_wide(v[j], dec_scale)), 0.0, BSI_CHUNK_ELEMS, Sa, 0.0f);
+            bytes = quantise_quad_wide(v[j], dec_scale, shift, Sa);
         }
-        if (least == 255u) least = 127u;  // a row of zeros
-        // the key image holds b << (8 - Sb), |b| <= 2^(Sb - 1)
-        units[row] = bad != 0u || (sum << (Sb - 1)) > (1ull << 24) ? -1.0f : __uint_as_float((least - static_cast<unsigned>(8 - Sb)) << 23);
+        held[j] = chunk_image_dword(bytes, cl);
+        image[(row * chunks + c) * 64 + lane] = held[j];
+        if (lane == 0) {
+            shifts[row * chunks + c] = shift;
+            scales[row * chunks + c] = static_cast<float>(1ULL << shift);
+        }
+        if (__ballot(held[j] != 0u) != 0ull) exponent[j] = static_cast<unsigned>(127 + shift);
+        least = exponent[j] < least ? exponent[j] : least;
+    }
+    if (lane == 0) shared[0][wave] = least;
+    __syncthreads();
+#pragma unroll
+    for (int w = 0; w < kUnitsWaves; ++w) least = shared[0][w] < least ? shared[0][w] : least;
+#pragma unroll
+    for (int j = 0; j < kHeld; ++j) {
+        const int c = wave + j * kUnitsWaves;
+        if (c >= chunks) break;
+        uint32_t l, h;
+        unit_bytes(held[j], exponent[j], least, Sa, l, h, total, odd);
+        const unsigned long long any = __ballot(h != 0u);
+        if (lane == 0)
+            blocks[c] = ((any & 0xFFFFull) != 0ull ? 1u : 0u) | ((any & 0xFFFF0000ull) != 0ull ? 2u : 0u) |
+                        ((any & 0xFFFF00000000ull) != 0ull ? 4u : 0u) | (any >> 48 != 0ull ? 8u : 0u);
+        lo[(row * chunks + c) * 64 + lane] = l;
+        hi[(row * chunks + c) * 64 + lane] = h;
+    }
+    unit_of_row<kUnitsWaves>(shared, lane, wave, total, odd, least, Sb, units + row);
+    const int words = (chunks * 4 + 63) / 64;
+    if (tid < words) {
+        unsigned long long m = 0ull;
+#pragma unroll
+        for (int i = 0; i < 16; ++i) m |= static_cast<unsigned long long>(blocks[tid * 16 + i]) << (4 * i);
+        masks[row * words + tid] = m;
     }
 }
 
@@ -1995,26 +2087,62 @@ bool i8_large_serves(int64_t Q, int64_t R, int chunks) {
     return us_large < us_small;
 }
 
-template <bool kHalf>
-static void launch_i8_large_t(unsigned char* ws, const int8_t* A8, const float* qscale, int stride, const int8_t* K8, const float* Bw, int Sa,
-                              int Sb, int chunks, int64_t R, int64_t Q, float scale_inv, int64_t R_total, float* out, const float* bias,
-                              hipStream_t st) {
+struct LargeWorkspace {
+    unsigned char *lo, *hi, *masks;
+    float* units;
+    unsigned* left;
+};
+static LargeWorkspace large_workspace(void* workspace, int64_t Q, int chunks) {
     const size_t image = large_aligned(static_cast<size_t>(Q) * chunks * 256), words = static_cast<size_t>((chunks * 4 + 63) / 64);
-    unsigned char* const lo = ws;
-    unsigned char* const hi = lo + image;
-    unsigned char* const masks = hi + image;
-    float* const units = reinterpret_cast<float*>(masks + large_aligned(static_cast<size_t>(Q) * words * 8));
-    unsigned* const left = reinterpret_cast<unsigned*>(reinterpret_cast<unsigned char*>(units) + large_aligned(static_cast<size_t>(Q) * 4));
-    launch(i8_units_kernel, dim3(static_cast<unsigned>(Q)), dim3(kUnitsBlock), 0, st, A8, qscale, stride, chunks, Sa, Sb,
-           reinterpret_cast<uint4*>(lo), reinterpret_cast<uint4*>(hi), reinterpret_cast<unsigned short*>(masks), units);
+    LargeWorkspace w;
+    w.lo = static_cast<unsigned char*>(workspace);
+    w.hi = w.lo + image;
+    w.masks = w.hi + image;
+    w.units = reinterpret_cast<float*>(w.masks + large_aligned(static_cast<size_t>(Q) * words * 8));
+    w.left = reinterpret_cast<unsigned*>(reinterpret_cast<unsigned char*>(w.units) + large_aligned(static_cast<size_t>(Q) * 4));
+    return w;
+}
+
+template <typename T, bool kVec>
+static void launch_build_units_t(const LargeWorkspace& w, const void* x, int64_t Q, int64_t d, int Sa, int Sb, double dec_scale, int32_t* shifts, float* scales,
+                                 int8_t* ints8, int chunks, hipStream_t st) {
+#define BSI_BUILD_UNITS(HELD)                                                                                                                       \
+    launch((build_units_kernel<T, kVec, HELD>), dim3(static_cast<unsigned>(Q)), dim3(kUnitsBlock), 0, st, static_cast<const T*>(x), d, chunks, Sa, Sb, \
+           dec_scale, static_cast<float>(dec_scale), shifts, scales, reinterpret_cast<uint32_t*>(ints8), reinterpret_cast<uint32_t*>(w.lo),          \
+           reinterpret_cast<uint32_t*>(w.hi), reinterpret_cast<unsigned long long*>(w.masks), w.units)
+    if (chunks <= 16) BSI_BUILD_UNITS(4);
+    else if (chunks <= 32) BSI_BUILD_UNITS(8);
+    else BSI_BUILD_UNITS(16);
+#undef BSI_BUILD_UNITS
+}
+void launch_build_units(void* workspace, const void* x, int dtype, int64_t Q, int64_t d, int Sa, int Sb, double dec_scale, int32_t* shifts, float* scales,
+                        int8_t* ints8, int chunks, hipStream_t st) {
+    const LargeWorkspace w = large_workspace(workspace, Q, chunks);
+    const bool vec = d % 4 == 0 && reinterpret_cast<uintptr_t>(x) % (dtype == BSI_DTYPE_F32 ? 16 : 8) == 0;
+    const auto go = [&](auto zero) {
+        using T = decltype(zero);
+        (vec ? &launch_build_units_t<T, true> : &launch_build_units_t<T, false>)(w, x, Q, d, Sa, Sb, dec_scale, shifts, scales, ints8, chunks, st);
+    };
+    if (dtype == BSI_DTYPE_F32) go(float{});
+    else if (dtype == BSI_DTYPE_F16) go(__half{});
+    else go(__hip_bfloat16{});
+}
+
+template <bool kHalf>
+static void launch_i8_large_t(const LargeWorkspace& w, bool units_there, const int8_t* A8, const float* qscale, int stride, const int8_t* K8,
+                              const float* Bw, int Sa, int Sb, int chunks, int64_t R, int64_t Q, float scale_inv, int64_t R_total, float* out,
+                              const float* bias, hipStream_t st) {
+    if (!units_there)
+        launch(i8_units_kernel, dim3(static_cast<unsigned>(Q)), dim3(kUnitsBlock), 0, st, A8, qscale, stride, chunks, Sa, Sb,
+               reinterpret_cast<uint4*>(w.lo), reinterpret_cast<uint4*>(w.hi), reinterpret_cast<unsigned short*>(w.masks), w.units);
     const I8Grid g = i8_bands((R + kLargeTile - 1) / kLargeTile, (Q + kLargeTile - 1) / kLargeTile, 2);
     static LdsOptIn once, once_left;
     lds_opt_in(once, reinterpret_cast<const void*>(&dot_mfma_i8_large_kernel<kHalf>), kLargeLds);
     const unsigned char* const warm = static_cast<const unsigned char*>(g_warm_ptr);
     const long long warm_lines = static_cast<long long>(g_warm_bytes / 128);
     launch((dot_mfma_i8_large_kernel<kHalf>), dim3(static_cast<unsigned>(g.tiles_x) * static_cast<unsigned>(g.tiles_y)), dim3(512), kLargeLds, st,
-           reinterpret_cast<const int8_t*>(lo), reinterpret_cast<const int8_t*>(hi), reinterpret_cast<const unsigned long long*>(masks), units, K8,
-           Bw, Sb, chunks, R, Q, scale_inv, R_total, out, bias, warm, warm_lines, stream_output(), g, t_out_dtype, left);
+           reinterpret_cast<const int8_t*>(w.lo), reinterpret_cast<const int8_t*>(w.hi), reinterpret_cast<const unsigned long long*>(w.masks), w.units, K8,
+           Bw, Sb, chunks, R, Q, scale_inv, R_total, out, bias, warm, warm_lines, stream_output(), g, t_out_dtype, w.left);
     dim3 grid;
     const I8Grid tiles = i8_grid((R + 127) / 128, (Q + 127) / 128, &grid);
     using T = I8TilesCfg<128, 128>;
@@ -2022,12 +2150,12 @@ static void launch_i8_large_t(unsigned char* ws, const int8_t* A8, const float* 
     const int64_t left_tiles = static_cast<int64_t>(tiles.tiles_x) * tiles.tiles_y;  // every workgroup of that kernel has a tile
     launch((dot_mfma_i8_tiles_kernel<128, 128, kHalf, true>), dim3(static_cast<unsigned>(left_tiles < kCus ? left_tiles : kCus)), dim3(T::kBlock), T::kLdsTiles, st, A8, qscale, stride, K8, Bw, Sb, chunks,
            R, Q, 16 - Sa - Sb, scale_inv, R_total, out, bias, 0, static_cast<const unsigned char*>(nullptr), 0LL, stream_output(), tiles,
-           static_cast<unsigned>(left_tiles), t_out_dtype, left);
+           static_cast<unsigned>(left_tiles), t_out_dtype, w.left);
 }
-void launch_i8_large(void* workspace, const int8_t* A8, const float* qscale, int stride, const int8_t* K8, const float* Bw, int Sa, int Sb,
+void launch_i8_large(void* workspace, bool units_there, const int8_t* A8, const float* qscale, int stride, const int8_t* K8, const float* Bw, int Sa, int Sb,
                      int chunks, int64_t R, int64_t Q, float scale_inv, int64_t R_total, float* out, const float* bias, hipStream_t st) {
     (t_out_dtype != BSI_DTYPE_F32 ? &launch_i8_large_t<true> : &launch_i8_large_t<false>)(
-        static_cast<unsigned char*>(workspace), A8, qscale, stride, K8, Bw, Sa, Sb, chunks, R, Q, scale_inv, R_total, out, bias, st);
+        large_workspace(workspace, Q, chunks), units_there, A8, qscale, stride, K8, Bw, Sa, Sb, chunks, R, Q, scale_inv, R_total, out, bias, st);
 }
 
 // Tile choice.  The 128 x 128 tile moves the fewest operand bytes per MAC and is the fastest whenever its grid

@@ -56,7 +56,9 @@ void launch_mfma_i8(const int8_t* A8, const float* qscale, int stride, const int
 constexpr int64_t kLargeMinQ = 512;
 size_t i8_large_workspace_bytes(int64_t Q, int chunks);
 bool i8_large_serves(int64_t Q, int64_t R, int chunks);
-void launch_i8_large(void* workspace, const int8_t* A8, const float* qscale, int stride, const int8_t* K8, const float* Bw, int Sa, int Sb,
+void launch_build_units(void* workspace, const void* x, int dtype, int64_t Q, int64_t d, int Sa, int Sb, double dec_scale, int32_t* shifts, float* scales,
+                        int8_t* ints8, int chunks, hipStream_t st);  // the build of a layer with chunk scales that launch_i8_large serves
+void launch_i8_large(void* workspace, bool units_there, const int8_t* A8, const float* qscale, int stride, const int8_t* K8, const float* Bw, int Sa, int Sb,
                      int chunks, int64_t R, int64_t Q, float scale_inv, int64_t R_total, float* out, const float* bias, hipStream_t st);
 
 // ---- bsi_dot_few_rows.hip: the plane-streaming kernel for up to kStreamMaxQ query rows on 6-plane tiled keys
