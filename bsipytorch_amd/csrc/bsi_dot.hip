@@ -350,7 +350,7 @@ extern "C" int bsi_hip_linear_out(const void* x, int dtype, int64_t Q, int64_t d
                         integer_decimal_scale(pow(10.0, static_cast<double>(decimal_places))) == 0;
     const bool large = core == BSI_CORE_AUTO && b_layout == BSI_LAYOUT_INT8 && Sb >= 2 && Sb <= 8 && R_total >= R && R <= (1 << 25) && B != nullptr &&
                        Bw != nullptr && out != nullptr && (reinterpret_cast<uintptr_t>(B) & 15) == 0 && i8_large_serves(Q, R, chunks);
-    const bool units_there = rebuild && large && chunk_scale && !planes && Q <= 0x7fffffffLL / chunks;  // the units come out of the build
+    const bool units_there = rebuild && large && chunk_scale && !planes;  // the units come out of the build
     if (units_there) {
         BSI_REQUIRE(dtype == BSI_DTYPE_F32 || dtype == BSI_DTYPE_F16 || dtype == BSI_DTYPE_BF16, "unknown dtype code %d", dtype);
         BSI_REQUIRE(x != nullptr, "null pointer");

@@ -2066,9 +2066,11 @@ static void launch_mfma_i8w(const int8_t* A8, const float* qscale, int stride, c
 // 16384 73.6, 69.3; 4096 x 3072 x 16384 225, 207; 2048 x 8192 x 8192 150, 128.5; 1024 x 8192 x 16384 165, 123; not taken 4096 x 1024 x
 // 16384 92, 99; 4096 x 2048 x 16384 155, 160 (f32 176, 188); 4096 x 2048 x 8192 78, 85; 2048 x 4096 x 8192 74, 75 (f32 78, 81);
 // 4096 x 4096 x 4096 78, 80; 3000 x 4096 x 11008 160, 172; and, at its edge, 2048 x 2048 x 16384 81, 77 (f32 88, 88).
+// Beyond 1 GiB of image the layer keeps to the workspace it had without units, which would be two more.
+constexpr int64_t kLargeMaxItems = 1 << 22;  // (row, chunk) items
 static size_t large_aligned(size_t v) { return (v + 255) / 256 * 256; }
 size_t i8_large_workspace_bytes(int64_t Q, int chunks) {
-    if (Q < kLargeMinQ || chunks > kLargeMaxChunks) return 0;
+    if (Q < kLargeMinQ || chunks > kLargeMaxChunks || Q > kLargeMaxItems / chunks) return 0;
     const size_t image = large_aligned(static_cast<size_t>(Q) * chunks * 256), words = static_cast<size_t>((chunks * 4 + 63) / 64);
     return 2 * image + large_aligned(static_cast<size_t>(Q) * words * 8) + large_aligned(static_cast<size_t>(Q) * 4) +
            large_aligned(static_cast<size_t>((Q + kLargeTile - 1) / kLargeTile) * 4);
@@ -2076,7 +2078,7 @@ size_t i8_large_workspace_bytes(int64_t Q, int chunks) {
 
 bool i8_large_serves(int64_t Q, int64_t R, int chunks) {
     const int forced = g_i8_tile.load(std::memory_order_relaxed);
-    if (Q < kLargeMinQ || chunks > kLargeMaxChunks || (forced != 0 && forced != kLargeTile)) return false;
+    if (Q < kLargeMinQ || chunks > kLargeMaxChunks || Q > kLargeMaxItems / chunks || (forced != 0 && forced != kLargeTile)) return false;
     const int64_t small = ((R + 127) / 128) * ((Q + 127) / 128), large = ((R + kLargeTile - 1) / kLargeTile) * ((Q + kLargeTile - 1) / kLargeTile);
     // the tile kernels' own limits: ring positions and exact quotients in 32 bits
     if (small * chunks >= (int64_t{1} << 29) || large * ((R + kLargeTile - 1) / kLargeTile) >= (int64_t{1} << 29)) return false;
