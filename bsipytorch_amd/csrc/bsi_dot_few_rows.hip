@@ -607,7 +607,7 @@ static void launch_mfma_stream(const int8_t* A8, const float* qscale, int stride
 #define BSI_STREAM_GO(INTS, BUILD, COOP)                                                                                      \
     do {                                                                                                                      \
         static LdsOptIn once;                                                                                                 \
-        lds_opt_in(once, reinterpret_cast<const void*>(&dot_mfma_stream_kernel<NT, KT, INTS, BUILD>), kStreamLds);             \
+        if (lds > 64 * 1024) lds_opt_in(once, reinterpret_cast<const void*>(&dot_mfma_stream_kernel<NT, KT, INTS, BUILD>), kStreamLds); \
         launch((dot_mfma_stream_kernel<NT, KT, INTS, BUILD>), grid, dim3(waves * 64), lds, st, A8, qscale, stride,            \
                reinterpret_cast<const unsigned long long*>(B), Bw, chunks, pass_chunks, R, Q, down_shift, scale_inv, R_total, \
                out, chunk_ints, bias, t_out_dtype, COOP);                                                                     \
