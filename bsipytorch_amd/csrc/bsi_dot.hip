@@ -414,7 +414,16 @@ static int coop_plan(int64_t Q, int64_t d, int64_t R, int decimal_places, int fi
         // leave a CU one of them) 9.3, 9.9, 9.7.
         return Q <= static_cast<int64_t>(shares) * waves && chunks <= kCoopHeld && d % 4 == 0 && Q * chunks <= 560 && groups <= 256 ? 2 : 0;
     }
-    return Q * chunks <= 2 * static_cast<int64_t>(shares) * waves ? 1 : 0;
+    const int64_t items = Q * chunks, a_round = static_cast<int64_t>(shares) * waves;
+    if (items <= 2 * a_round) return 1;
+    // More rounds where few workgroups have few shares: the launch takes some 4.6 us, 0.45 a round and, for more than 32 rows, 0.4 a
+    // chunk (each a step of the dot).  us, two launches (on a host that issues them in 8.4, and on one that takes 9.9) and one: 33 x
+    // 1024 x 2048 (2.1 rounds) 8.6, 9.9, 6.6; 48 x 768 x 2048 8.4, 9.9, 6.2; 150 x 512 x 1536 (2.5) 8.5, 9.9, 6.2; 100 x 1024 x 3072 8.5,
+    // 10.0, 7.3; 120 x 512 x 1024 (3.8) 8.5, 9.9, 7.1; 128 x 1024 x 2048 (4) 8.3, 10.0, 7.9; 30 x 2048 x 1024 (3.8) 8.0, 9.2, 7.5 -- beyond:
+    // 36 x 2048 x 3072 (3) 8.3, 9.9, 8.8; 64 x 2048 x 4096 (4) 8.3, 9.7, 9.4; 48 x 1536 x 2048 (4.5) 8.3, 9.8, 8.8; 25 x 3072 x 1024
+    // (3.1) 7.9, 9.2, 8.2; 20 x 4096 x 1024 (2.5) 7.8, 9.1, 8.8; 250 x 1024 x 4096 (1000 items) 8.3, 8.5, 9.3.
+    if (items > 4 * a_round || items > 512) return 0;
+    return b_layout == BSI_LAYOUT_TILED16 ? (chunks <= 8 ? 1 : 0) : (9 * items + 8 * chunks * a_round <= 76 * a_round ? 1 : 0);
 }
 
 extern "C" int bsi_hip_linear_coop_serves(int64_t Q, int64_t d, int64_t R, int decimal_places, int fixed_bits, int b_layout, int Sb) {
