@@ -411,8 +411,11 @@ static int coop_plan(int64_t Q, int64_t d, int64_t R, int decimal_places, int fi
         // them in 8.4, and on one that takes 9.8) and one: 24 x 704 x 704 8.4, 9.5, 6.6; 24 x 1600 x 1600 8.1, 9.5, 6.6; 100 x 320 x
         // 2000 8.5, 9.8, 6.8; 37 x 704 x 9728 8.5, 9.9, 7.0; 250 x 100 x 8192 8.7, 10.1, 7.6; 64 x 1600 x 4800 8.4, 9.8, 8.3; 77 x 1600 x
         // 4800 8.7, 9.9, 8.8 -- beyond: 121 x 1600 x 6400 (847 items) 8.9, 9.8, 9.7; 128 x 832 x 12000 (376 workgroups, whose registers
-        // leave a CU one of them) 9.3, 9.9, 9.7.
-        return Q <= static_cast<int64_t>(shares) * waves && chunks <= kCoopHeld && d % 4 == 0 && Q * chunks <= 560 && groups <= 256 ? 2 : 0;
+        // leave a CU one of them) 9.3, 9.9, 9.7.  More rows than waves, where few workgroups have few shares: 60 x 704 x 1024 (1.9 rounds) 8.5,
+        // 9.6, 7.3; 250 x 320 x 1024 8.5, 9.9, 6.9; 90 x 900 x 1000 8.5, 9.9, 8.1; 200 x 448 x 700 (2.8) 8.5, 10.0, 8.2; 150 x 192 x 768 8.5,
+        // 9.8, 7.0 -- beyond: 60 x 896 x 768 (2.5) 8.5, 9.8, 8.3; 50 x 640 x 640 (3.1) 8.5, 9.9, 8.7; 128 x 832 x 640 8.5, 9.8, 9.3.
+        const int rounds = chunks <= 2 ? 3 : (chunks <= 4 ? 2 : 1);
+        return Q <= rounds * static_cast<int64_t>(shares) * waves && chunks <= kCoopHeld && d % 4 == 0 && Q * chunks <= 560 && groups <= 256 ? 2 : 0;
     }
     const int64_t items = Q * chunks, a_round = static_cast<int64_t>(shares) * waves;
     if (items <= 2 * a_round) return 1;

@@ -13,7 +13,8 @@ PATIENCE = 6  # BSI_OPT_COOP_PATIENCE
 
 
 @pytest.mark.parametrize("Q,d,R", [(24, 704, 704), (24, 1600, 1600), (32, 1924, 2000), (31, 260, 1024), (77, 1600, 4800), (70, 1980, 4000), (37, 704, 9728),
-                                   (250, 100, 8192), (100, 320, 2000), (33, 1860, 2048)])
+                                   (250, 100, 8192), (100, 320, 2000), (33, 1860, 2048),
+                                   (60, 704, 1024), (200, 448, 700), (90, 900, 1000), (150, 192, 768)])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("patience", [2000, 0])
 def test_same_bits_as_two_launches(ops, monkeypatch, Q, d, R, dtype, patience):
