@@ -23,7 +23,8 @@ namespace bsi {
 constexpr int kStreamLdsInts = 16384;  // at most 64 KiB of chunk accumulators per pass
 constexpr int kStreamLds = kStreamLdsInts * 4 + 4096 + 16 * 2048;  // with their scales and 16 waves' query rows
 
-// kBuild: the queries are quantised by this launch (bsi_coop_build.h); A8 and qscale are not looked at.  The copy lies in the
+// kBuild: the queries are quantised by this launch (bsi_coop_build.h; 1: a chunk a wave at a time, 2: a row); A8 and qscale are
+// not looked at.  The copy lies in the
 // order of the operand loads (coop_image_at: up to 1 KiB in one run a load, where rows one after the other are 32 lines a load and
 // the loads of 32 rows take longer than the key planes they are for), and a wave takes a chunk's scales with its operands and
 // leaves them in LDS, so that the chain asks memory for nothing.  us a layer, rows and the chain's own loads before, then now:

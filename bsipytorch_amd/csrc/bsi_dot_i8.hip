@@ -540,7 +540,8 @@ __global__ __launch_bounds__((I8Cfg<TM, TN>::kBlock)) void dot_mfma_i8_kernel(
     int ndig, long long dig_stride, const long long* __restrict__ key_indices, int key_tiled,
     const unsigned char* __restrict__ warm, long long warm_lines, int out_stream, float* __restrict__ split_partials,
     unsigned* __restrict__ split_counters, float split_limit, int split_shape, I8Grid plain_grid, int out_dtype, CoopBuild coop) {
-    // kBuild: the queries are quantised by this launch (bsi_coop_build.h); A8 and qscale are not looked at.
+    // kBuild: the queries are quantised by this launch (bsi_coop_build.h; 1: a chunk a wave at a time, 2: a row); A8 and qscale are
+    // not looked at.
     // kSplit (chain mode only): a D-split launch.  gridDim.z workgroups share an output tile, each running the chain
     // over its own run of chunks from zero.  All operands of the chain are integers (times one power of two), so
     // as long as no value the chain takes exceeds 2^24 of its unit nothing is ever rounded, the value after every
