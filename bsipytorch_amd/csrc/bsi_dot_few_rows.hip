@@ -24,10 +24,9 @@ constexpr int kStreamLdsInts = 16384;  // at most 64 KiB of chunk accumulators p
 constexpr int kStreamLds = kStreamLdsInts * 4 + 4096 + 16 * 2048;  // with their scales and 16 waves' query rows
 
 // kBuild: the queries are quantised by this launch (bsi_coop_build.h; 1: a chunk a wave at a time, 2: a row); A8 and qscale are
-// not looked at.  The copy lies in the
-// order of the operand loads (coop_image_at: up to 1 KiB in one run a load, where rows one after the other are 32 lines a load and
-// the loads of 32 rows take longer than the key planes they are for), and a wave takes a chunk's scales with its operands and
-// leaves them in LDS, so that the chain asks memory for nothing.  us a layer, rows and the chain's own loads before, then now:
+// not looked at.  The copy lies in the order of the operand loads (coop_image_at: up to 1 KiB in one run a load, where rows one
+// after the other are 32 lines a load and the loads of 32 rows take longer than the key planes they are for), and a wave takes a
+// chunk's scales with its operands and leaves them in LDS, so that the chain asks memory for nothing.  us a layer, rows and the chain's own loads before, then now:
 // 16 x 4096 x 4096 bf16 8.7, 7.85; 32 x 4096 x 4096 11.05, 8.95; 32 x 8192 x 4096 f16 16.5, 12.4; 16 x 8192 x 4096 12.1, 10.5;
 // 24 x 2048 x 2048 f32 6.95, 6.25; 8 x 4096 x 4096 7.8, 7.6.  Only those instances
 // take the build's description: with it the workgroup's size, which lies behind the arguments, is in another cache line of
@@ -35,8 +34,8 @@ constexpr int kStreamLds = kStreamLdsInts * 4 + 4096 + 16 * 2048;  // with their
 // 4096 5.25, 5.09; 1 x 4096 x 16384 10.5, 10.2; 1 x 16384 x 4096 11.1, 10.9 (1 x 4096 x 4096 4.06, 4.11).
 //
 // Without kBuild the image has its rows one after the other.  An operand's lanes want 64 bytes of each of 16 rows, and loads of
-// such pieces run at half the rate of whole lines (16 rows of a chunk: 24 KiB of key planes come with 4 KiB fetched as 8); so a
-// load takes 128 bytes of 8 rows, and the wave turns them round through 2 KiB of LDS, in which its sums lie afterwards.  The scales
+// such pieces run at half the rate of whole lines (a chunk is 3 KiB of a key tile's planes and 4 KiB of 16 query rows, which then
+// take as long as 8); so a load takes 128 bytes of 8 rows, and the wave turns them round through 2 KiB of LDS, in which its sums lie afterwards.  The scales
 // go with them, as above.  us a dot, operands straight from memory, then so: 16 x 16384 x 4096 14.7, 12.2; 16 x 8192 x 8192 13.9,
 // 11.9; 24 x 8192 x 8192 18.7, 14.8; 32 x 4096 x 4096 7.6, 6.1; 16 x 8192 x 32768 44.8, 41.0; 8 x 16384 x 4096 12.6, 11.9;
 // 1 x 4096 x 32768 21.6, 21.5; 8 x 8192 x 16384 21.5, 21.5.  All 4 KiB of a chunk at once, in LDS of its own: 12.0 for the first,
