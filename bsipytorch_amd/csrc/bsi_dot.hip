@@ -111,13 +111,9 @@ extern "C" int bsi_hip_dot_split_plan(int64_t R, int64_t Q, int W64, int* tile, 
 // 2 GiB: 128 rows of chunks * 256 bytes must stay below that.
 constexpr int kMfmaMaxChunks = 32768;
 
-// Validation, kernel selection and launch.  `bias` (optional) is added to every output; *bias_fused tells
-// the caller whether the selected kernel did that in its own epilogue.
-static int dot_launch(const uint64_t* A, const int8_t* A_ints8, const float* A_chunk_scales, int A_scale_stride,
-                      int Sa, int W64, const uint64_t* B, int b_layout, const float* Bw, int Sb, int64_t R, int64_t Q,
-                      float scale_inv, int64_t R_total, float* out, int32_t* chunk_ints, int core, void* workspace,
-                      size_t workspace_bytes, void* stream, const float* bias, bool* bias_fused) {
-    *bias_fused = false;
+// What every route of the fixed-bit dot asks of its operands; BSI_OK where there is nothing to do.
+static int check_dot(const uint64_t* A, const int8_t* A_ints8, const float* A_chunk_scales, int A_scale_stride, int Sa, int W64,
+                     const uint64_t* B, int b_layout, const float* Bw, int Sb, int64_t R, int64_t Q, int64_t R_total, const void* out) {
     BSI_REQUIRE(Q >= 0 && R >= 0, "negative Q or R");
     BSI_REQUIRE(W64 >= 1, "W64 must be >= 1");
     BSI_REQUIRE(Sa >= 1 && Sa <= 63 && Sb >= 1 && Sb <= 63, "Sa and Sb must be in [1, 63]");
@@ -138,6 +134,19 @@ static int dot_launch(const uint64_t* A, const int8_t* A_ints8, const float* A_c
                 "chunk scale stride mismatch: got %d expected %d (or 1 for row scales)", A_scale_stride, chunks);
     BSI_REQUIRE(B && Bw && out, "null pointer");
     BSI_REQUIRE(A || A_ints8, "neither query planes nor int8 queries given");
+    return BSI_OK;
+}
+
+// Validation, kernel selection and launch.  `bias` (optional) is added to every output; *bias_fused tells
+// the caller whether the selected kernel did that in its own epilogue.
+static int dot_launch(const uint64_t* A, const int8_t* A_ints8, const float* A_chunk_scales, int A_scale_stride,
+                      int Sa, int W64, const uint64_t* B, int b_layout, const float* Bw, int Sb, int64_t R, int64_t Q,
+                      float scale_inv, int64_t R_total, float* out, int32_t* chunk_ints, int core, void* workspace,
+                      size_t workspace_bytes, void* stream, const float* bias, bool* bias_fused) {
+    *bias_fused = false;
+    if (int rc = check_dot(A, A_ints8, A_chunk_scales, A_scale_stride, Sa, W64, B, b_layout, Bw, Sb, R, Q, R_total, out)) return rc;
+    if (Q == 0 || R == 0) return BSI_OK;
+    const int chunks = (W64 + 3) / 4;
     hipStream_t st = as_stream(stream);
 
     const bool mfma_ok = (Sa >= 2 && Sa <= 8 && Sb >= 2 && Sb <= 8);
@@ -348,8 +357,12 @@ extern "C" int bsi_hip_linear_out(const void* x, int dtype, int64_t Q, int64_t d
     // BSI_CORE_AUTO falls back to for wide keys), and where the builder cannot leave them out.
     const bool planes = core == BSI_CORE_VALU || Sb < 2 || Sb > 8 || chunks > kMfmaMaxChunks ||
                         integer_decimal_scale(pow(10.0, static_cast<double>(decimal_places))) == 0;
-    const bool large = core == BSI_CORE_AUTO && b_layout == BSI_LAYOUT_INT8 && Sb >= 2 && Sb <= 8 && R_total >= R && R <= (1 << 25) && B != nullptr &&
-                       Bw != nullptr && out != nullptr && (reinterpret_cast<uintptr_t>(B) & 15) == 0 && i8_large_serves(Q, R, chunks);
+    BSI_REQUIRE(warm != nullptr || warm_bytes == 0, "null warm-up region");
+    const bool large = core == BSI_CORE_AUTO && b_layout == BSI_LAYOUT_INT8 && Sb >= 2 && Sb <= 8 && i8_large_serves(Q, R, chunks);
+    if (large) {
+        if (int rc = check_dot(nullptr, ints8, scales, chunk_scale ? chunks : 1, fixed_bits, W64, B, b_layout, Bw, Sb, R, Q, R_total, out)) return rc;
+        BSI_REQUIRE((reinterpret_cast<uintptr_t>(B) & 15) == 0, "int8 key image must be 16-byte aligned");
+    }
     const bool units_there = rebuild && large && chunk_scale && !planes;  // the units come out of the build
     if (units_there) {
         BSI_REQUIRE(dtype == BSI_DTYPE_F32 || dtype == BSI_DTYPE_F16 || dtype == BSI_DTYPE_BF16, "unknown dtype code %d", dtype);
@@ -365,7 +378,7 @@ extern "C" int bsi_hip_linear_out(const void* x, int dtype, int64_t Q, int64_t d
     t_out_dtype = out_dtype;
     if (large) {
         g_warm_ptr = warm;
-        g_warm_bytes = warm != nullptr ? warm_bytes : 0;
+        g_warm_bytes = warm_bytes;
         t_layer_output = 1;
         launch_i8_large(ws + w.large, units_there, ints8, scales, chunk_scale ? chunks : 1, reinterpret_cast<const int8_t*>(B), Bw, fixed_bits, Sb, chunks, R, Q,
                         scale_inv, R_total, static_cast<float*>(out), bias, as_stream(stream));
