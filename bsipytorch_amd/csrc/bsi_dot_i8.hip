@@ -531,6 +531,14 @@ __device__ __forceinline__ void i8_tile_of(const I8Grid& g, unsigned id, int& bx
     by = static_cast<int>(first + in - x * (last ? left : static_cast<unsigned>(g.height)));
 }
 
+// The grid of so many of its query tiles.
+__device__ __forceinline__ void narrow_grid(I8Grid& g, int tiles_y) {
+    g.tiles_y = tiles_y;
+    if (g.height == 0) return;
+    const unsigned last = static_cast<unsigned>(tiles_y - (tiles_y - 1) / g.height * g.height);
+    g.by_last = last == 1u ? 0u : 0xFFFFFFFFu / last + 1u;
+}
+
 template <int TM, int TN, int kMode, bool kSplit, int kBuild, bool kFour, bool kHalf>
 __global__ __launch_bounds__((I8Cfg<TM, TN>::kBlock)) void dot_mfma_i8_kernel(
     const int8_t* A8, const float* qscale, int qscale_stride,
@@ -967,14 +975,30 @@ struct I8TilesCfg : I8Cfg<TM, TN> {
     static constexpr int kLdsTiles = 4 * C::kStage + kScaleBytes + 4 * C::kEpilogueBytes;  // four sets of key factors and biases
 };
 
+// The bands of kLargeTile queries that dot_mfma_i8_large_kernel leaves to the chain: their number, then the bands, in ascending order.
+// The tiles of that launch are those bands' own, two query tiles a band (one in a last band of half a tile), numbered through as if there were
+// no others: left_tile is the query tile of the matrix.
+template <bool kLeft>
+using LeftBands = std::conditional_t<kLeft, const unsigned*, int>;
+__device__ __forceinline__ int left_tile(const unsigned* __restrict__ left, int by) {
+    return 2 * static_cast<int>(left[1 + (by >> 1)]) + (by & 1);
+}
+__device__ __forceinline__ unsigned left_grid(const unsigned* __restrict__ left, I8Grid& g) {  // narrows g to them; the number of tiles
+    const int bands = static_cast<int>(left[0]);
+    if (bands == 0) return 0u;
+    const int half = (g.tiles_y & 1) != 0 && static_cast<int>(left[bands]) == g.tiles_y >> 1 ? 1 : 0;
+    narrow_grid(g, 2 * bands - half);
+    return static_cast<unsigned>(g.tiles_x) * static_cast<unsigned>(g.tiles_y);
+}
+
 // A loader wave: the stages of all the workgroup's tiles, one after the other; three stages ahead of the MFMA waves, across
 // the ends of tiles.
-template <typename C>
+template <typename C, bool kLeft>
 __device__ __forceinline__ void i8_tiles_loader_wave(unsigned char* __restrict__ lds, int lw, int lane, const int8_t* __restrict__ A8,
                                                      const float* __restrict__ qscale, int qscale_stride,
                                                      const int8_t* __restrict__ K8, const float* __restrict__ Bw, int Sb, int chunks,
                                                      int64_t R, int64_t Q, const float* __restrict__ bias, int key_tiled,
-                                                     const I8Grid& grid, unsigned tiles) {
+                                                     const I8Grid& grid, unsigned tiles, [[maybe_unused]] LeftBands<kLeft> left) {
     constexpr int TM = C::kTM, TN = C::kTN;
     constexpr int L = C::kLoaders, NI = C::kLoads, KG = TM / 8, QG = TN / 8;
     constexpr int kEpi = (2 * (TM / 64) + L - 1) / L;
@@ -1007,6 +1031,7 @@ __device__ __forceinline__ void i8_tiles_loader_wave(unsigned char* __restrict__
             by = static_cast<int>(id / static_cast<unsigned>(grid.tiles_x));
             bx = static_cast<int>(id) - by * grid.tiles_x;
         }
+        if constexpr (kLeft) by = left_tile(left, by);
         const int64_t r0 = static_cast<int64_t>(bx) * TM, q0 = static_cast<int64_t>(by) * TN;
         rk = key_tiled ? make_rsrc(K8 + static_cast<size_t>(r0 / 64) * kblock, static_cast<size_t>((R + 63) / 64 - r0 / 64) * kblock)
                        : make_rsrc(K8 + static_cast<size_t>(r0) * rowbytes, static_cast<size_t>(R - r0) * rowbytes);
@@ -1072,22 +1097,25 @@ __global__ __launch_bounds__((I8Cfg<TM, TN>::kBlock)) void dot_mfma_i8_tiles_ker
     const int8_t* __restrict__ A8, const float* __restrict__ qscale, int qscale_stride, const int8_t* __restrict__ K8,
     const float* __restrict__ Bw, int Sb, int chunks, int64_t R, int64_t Q, int down_shift, float scale_inv, int64_t R_total,
     float* __restrict__ out, const float* __restrict__ bias, int key_tiled, const unsigned char* __restrict__ warm,
-    long long warm_lines, int out_stream, I8Grid grid, unsigned tiles, int out_dtype, std::conditional_t<kLeft, const unsigned*, int> left) {
-    // kLeft: only if dot_mfma_i8_large_kernel, before this launch, has left a tile of 256 queries to it (`left`, a word for each)
+    long long warm_lines, int out_stream, I8Grid grid, unsigned tiles, int out_dtype, LeftBands<kLeft> left) {
+    // kLeft: the tiles of the bands that dot_mfma_i8_large_kernel, before this launch, has left to it; `grid` is that of all tiles.
+    // The keys of the next dot are touched here only if it has left them all (then none of its workgroups has).
     using C = I8Cfg<TM, TN>;
     constexpr int WM = C::kWM, WN = C::kWN, kMode = kI8Chain;
     extern __shared__ __attribute__((aligned(16))) unsigned char lds[];  // I8TilesCfg::kLdsTiles
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    if constexpr (kLeft) {  // every wave looks for itself
-        unsigned any = 0u;
-        for (int64_t t = lane; t * kLargeTile < Q; t += 64) any |= left[t];
-        if (__ballot(any != 0u) == 0ull) return;
+    if constexpr (kLeft) {  // the same in all waves of a workgroup
+        static_assert(2 * TN == kLargeTile, "two query tiles a band");
+        const unsigned all = tiles;
+        tiles = left_grid(left, grid);
+        if (blockIdx.x >= tiles) return;
+        if (tiles != all) warm_lines = 0;
     }
     if (wave >= C::kConsumers) {
         const int lw = wave - C::kConsumers;
-        i8_tiles_loader_wave<C>(lds, lw, lane, A8, qscale, qscale_stride, K8, Bw, Sb, chunks, R, Q, bias, key_tiled, grid, tiles);
+        i8_tiles_loader_wave<C, kLeft>(lds, lw, lane, A8, qscale, qscale_stride, K8, Bw, Sb, chunks, R, Q, bias, key_tiled, grid, tiles, left);
         if (warm_lines > 0) i8_warm_lines<C::kLoaders>(lds + 4 * C::kStage, lw, lane, warm, warm_lines);
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // nothing may still be writing LDS when the workgroup ends
         return;
@@ -1188,6 +1216,7 @@ __global__ __launch_bounds__((I8Cfg<TM, TN>::kBlock)) void dot_mfma_i8_tiles_ker
             by = static_cast<int>(id / static_cast<unsigned>(grid.tiles_x));
             bx = static_cast<int>(id) - by * grid.tiles_x;
         }
+        if constexpr (kLeft) by = left_tile(left, by);
         // from values the compiler cannot see through, so that no address of the stores is held in registers over the chunk loop
         int ln_late = ln, lg_late = lg;
         asm volatile("" : "+v"(ln_late), "+v"(lg_late));
@@ -1216,8 +1245,16 @@ __global__ __launch_bounds__((I8Cfg<TM, TN>::kBlock)) void dot_mfma_i8_tiles_ker
 // blocks of 64 elements are read that have one.  The dot is then ONE int32 sum over the row, and if the row's magnitudes
 // times the largest key magnitude add up to no more than 2^24 units, every value the fp32 chain over the chunks takes is an
 // integer of at most 24 bits: it never rounds, and the sum is its result, bit for bit.  i8_units_kernel writes the images, the
-// masks of the blocks and the rows' units and checks that bound; a tile of queries with a row outside it, or with more
-// than a quarter of its blocks in the second image, is left to the chain, in a launch behind this one that otherwise ends at once.
+// masks of the blocks and the rows' units and checks that bound; a band of 256 queries with a row outside it, or with more
+// than a quarter of its blocks in the second image, is left to the chain, in a launch behind this one that has those bands' tiles
+// only and ends at once where there are none.  large_bands_kernel says so of each band ahead of the launch, and each workgroup
+// works out the same two things from it: which bands are kept -- their tiles are numbered through, so that they fill the rounds of
+// workgroups of every XCD -- and whether the chain had better take all, as a launch of one round is no shorter for the bands it leaves.
+// us a layer, 0, 1, a quarter, half and all of the bands left, and tiles of 128 x 128: 4096 x 4096 x 16384 bf16 246, 264, 265, 282, 302,
+// 284; 2048 x 8192 x 8192 f32 141, 164, 163, 164, 163, 149; 4096 x 3072 x 16384 f16 199, 217, 217, 228, 245, 226; 1024 x 4096 x 16384 bf16
+// 76, 86, 86, 86, 86, 77.  (All tiles in the chain wherever one band was left: 1.8 times the time of none.  Tiles of the kept bands where
+// they lie in the matrix: 4096 x 4096 x 16384, a quarter 302, half 356.)  What a layer loses of which nothing is kept is the images, 8,
+// and three launches.
 //
 // Without the chain there are no second accumulators and no scales, a wave holds 128 x 64 outputs and a workgroup 256 x 256:
 // half the bytes from the L2 and two thirds of the LDS reads a multiply-add, both of which the clock pays for.  Eight waves that load
@@ -1449,64 +1486,118 @@ struct LargeStages {
     }
 };
 
+// The bands of kLargeTile queries, a workgroup each: which blocks are in the upper image for any of a band's rows, and how many stages
+// they are, or kToChain.
+constexpr unsigned kToChain = ~0u;
+__global__ __launch_bounds__(kLargeTile) void large_bands_kernel(const unsigned long long* __restrict__ masks, const float* __restrict__ units, int chunks,
+                                                                 int64_t Q, unsigned long long* __restrict__ bands, unsigned* __restrict__ uppers) {
+    constexpr int kWaves = kLargeTile / 64;
+    __shared__ unsigned long long ored[kWaves][kLargeMaskWords];
+    __shared__ unsigned bad[kWaves];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, words = (chunks * 4 + 63) / 64;
+    const int64_t q = static_cast<int64_t>(blockIdx.x) * kLargeTile + tid;
+    const bool mine = q < Q;
+    const bool odd = mine && units[q] < 0.0f;
+    unsigned long long m[kLargeMaskWords];
+#pragma unroll
+    for (int w = 0; w < kLargeMaskWords; ++w) m[w] = mine && w < words ? masks[q * words + w] : 0ull;
+#pragma unroll
+    for (int w = 0; w < kLargeMaskWords; ++w)
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) m[w] |= __shfl_xor(m[w], o, BSI_WAVE);
+    const bool any_odd = __ballot(odd) != 0ull;
+    if (lane == 0) {
+#pragma unroll
+        for (int w = 0; w < kLargeMaskWords; ++w) ored[wave][w] = m[w];
+        bad[wave] = any_odd ? 1u : 0u;
+    }
+    __syncthreads();
+    if (tid != 0) return;
+    unsigned chain = 0u;
+    int blocks = 0;
+    for (int w = 0; w < kLargeMaskWords; ++w) {
+        unsigned long long all = 0ull;
+        for (int i = 0; i < kWaves; ++i) all |= ored[i][w];
+        bands[static_cast<size_t>(blockIdx.x) * kLargeMaskWords + w] = all;
+        blocks += __builtin_popcountll(all);
+    }
+    for (int i = 0; i < kWaves; ++i) chain |= bad[i];
+    uppers[blockIdx.x] = chain != 0u || blocks > chunks ? kToChain : static_cast<unsigned>(blocks + 1) / 2;  // at most a quarter of the 4 chunks blocks
+}
+
+// What decides between the sums for some bands and the chain for all, in us (i8_large_serves): a round of workgroups of the sums and a
+// stage more in it, a round of the chain, the chain for all; tiles of either kernel beside one another.
+struct LargeCost {
+    float round, stage, chain, whole;
+    int across, small;
+};
+
 template <bool kHalf>
 __global__ __launch_bounds__(512, 2) void dot_mfma_i8_large_kernel(
-    const int8_t* lo, const int8_t* hi, const unsigned long long* __restrict__ masks, const float* __restrict__ units, const int8_t* K8,
-    const float* __restrict__ Bw, int Sb, int chunks, int64_t R, int64_t Q, float scale_inv, int64_t R_total, float* __restrict__ out,
-    const float* __restrict__ bias, const unsigned char* __restrict__ warm, long long warm_lines, int out_stream, I8Grid grid, int out_dtype,
-    unsigned* __restrict__ left) {
+    const int8_t* lo, const int8_t* hi, const unsigned long long* __restrict__ bands, const unsigned* __restrict__ uppers, LargeCost cost,
+    const float* __restrict__ units, const int8_t* K8, const float* __restrict__ Bw, int Sb, int chunks, int64_t R, int64_t Q, float scale_inv,
+    int64_t R_total, float* __restrict__ out, const float* __restrict__ bias, const unsigned char* __restrict__ warm, long long warm_lines,
+    int out_stream, I8Grid grid, int out_dtype, unsigned* __restrict__ left) {
+    // bands, uppers: of large_bands_kernel.  left: the list of the bands that the chain takes, for dot_mfma_i8_tiles_kernel behind this launch:
+    // those that large_bands_kernel has turned down, or all, where the sums for the others would not pay.
     extern __shared__ __attribute__((aligned(16))) unsigned char lds[];  // kLargeLds
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wr = wave & 1, wq = wave >> 1, ln = lane & 15, lg = lane >> 4;
+    const unsigned all_bands = static_cast<unsigned>(grid.tiles_y);
+    unsigned count = 0u, more = 0u;
+    for (unsigned t = 0; t < all_bands; t += 64) {
+        const unsigned u = t + lane < all_bands ? uppers[t + lane] : 0u;
+        count += __builtin_popcountll(__ballot(u == kToChain));
+        more += u == kToChain ? 0u : u;
+    }
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) more += __shfl_xor(more, o, BSI_WAVE);
+    const unsigned kept = all_bands - count, rounds = (kept * static_cast<unsigned>(cost.across) + 255u) / 256u;
+    const unsigned chained = (2u * count * static_cast<unsigned>(cost.small) + 255u) / 256u;
+    const float sums = static_cast<float>(rounds) * (cost.round + cost.stage * static_cast<float>(more) / static_cast<float>(kept > 0u ? kept : 1u)) - 8.0f;
+    const bool all = kept == 0u || sums + static_cast<float>(chained) * cost.chain > cost.whole;
+    if (blockIdx.x == 0 && wave == 0) {
+        unsigned at = 1u;
+        for (unsigned t = 0; t < all_bands; t += 64) {
+            const bool listed = t + lane < all_bands && (all || uppers[t + lane] == kToChain);
+            const unsigned long long m = __ballot(listed);
+            if (listed) left[at + __builtin_popcountll(m & ((1ull << lane) - 1ull))] = t + lane;
+            at += __builtin_popcountll(m);
+        }
+        if (lane == 0) left[0] = at - 1u;
+    }
+    // the tiles of the bands that are kept, numbered through as if there were no others: an XCD's run of them is as long as another's
+    if (all || blockIdx.x >= kept * static_cast<unsigned>(grid.tiles_x)) return;
+    if (count != 0u) narrow_grid(grid, static_cast<int>(kept));
     int bx, by;
     i8_tile_of(grid, blockIdx.x, bx, by);
+    if (count != 0u) {
+        int before = by;
+        for (unsigned t = 0; t < all_bands; t += 64) {
+            const bool keep = t + lane < all_bands && uppers[t + lane] != kToChain;
+            const unsigned long long m = __ballot(keep);
+            const int here = __builtin_popcountll(m);
+            if (before < here) {
+                by = static_cast<int>(t) + __builtin_ctzll(__ballot(keep && __builtin_popcountll(m & ((1ull << lane) - 1ull)) == before));
+                break;
+            }
+            before -= here;
+        }
+    }
     const int64_t r0 = static_cast<int64_t>(bx) * kLargeTile, q0 = static_cast<int64_t>(by) * kLargeTile;
     const uint32_t rowbytes = static_cast<uint32_t>(chunks) << 8;
     const bsi_rsrc rk = make_rsrc(K8 + static_cast<size_t>(r0) * rowbytes, static_cast<size_t>(R - r0) * rowbytes);
     const bsi_rsrc rlo = make_rsrc(lo + static_cast<size_t>(q0) * rowbytes, static_cast<size_t>(Q - q0) * rowbytes);
     const bsi_rsrc rhi = make_rsrc(hi + static_cast<size_t>(q0) * rowbytes, static_cast<size_t>(Q - q0) * rowbytes);
 
-    // which blocks of the tile's rows are in the upper image, and whether the chain has to take them
     LargeStages stages;
-    {
-        const int words = (chunks * 4 + 63) / 64;
-        unsigned long long* const ored = reinterpret_cast<unsigned long long*>(lds);
-        if (tid <= kLargeMaskWords) ored[tid] = 0ull;  // the last: a row for the chain
-        __syncthreads();
-        const int64_t q = q0 + tid;
-        const bool mine = tid < kLargeTile && q < Q;
-        if (wave < kLargeTile / 64) {
 #pragma unroll
-            for (int w = 0; w < kLargeMaskWords; ++w) {
-                unsigned long long m = mine && w < words ? masks[q * words + w] : 0ull;
-                if (__ballot(m != 0ull) == 0ull) continue;
-#pragma unroll
-                for (int o = 32; o > 0; o >>= 1) m |= __shfl_xor(m, o, BSI_WAVE);
-                if (lane == 0) atomicOr(ored + w, m);
-            }
-            if (__ballot(mine && units[q] < 0.0f) != 0ull && lane == 0) atomicOr(ored + kLargeMaskWords, 1ull);
-        }
-        __syncthreads();
-        const int bad = __builtin_amdgcn_readfirstlane(static_cast<int>(ored[kLargeMaskWords]));
-        int blocks = 0;
-#pragma unroll
-        for (int w = 0; w < kLargeMaskWords; ++w) {
-            const unsigned long long m = ored[w];
-            const unsigned a = __builtin_amdgcn_readfirstlane(static_cast<int>(static_cast<unsigned>(m)));
-            const unsigned b = __builtin_amdgcn_readfirstlane(static_cast<int>(static_cast<unsigned>(m >> 32)));
-            stages.mask[w] = static_cast<unsigned long long>(b) << 32 | a;
-            blocks += __builtin_popcountll(stages.mask[w]);
-        }
-        const bool leave = bad != 0 || blocks > chunks;  // a quarter of the 4 chunks blocks
-        if (bx == 0 && tid == 0) left[by] = leave ? 1u : 0u;
-        if (leave) return;
-        stages.base = stages.half = 0;
-        stages.upper = (blocks + 1) / 2;
-        stages.halves = 2 * chunks;
-        __syncthreads();  // the masks have been read: the ring may be written
-    }
-    const int uppers = stages.upper;
+    for (int w = 0; w < kLargeMaskWords; ++w) stages.mask[w] = bands[static_cast<size_t>(by) * kLargeMaskWords + w];
+    stages.base = stages.half = 0;
+    stages.upper = static_cast<int>(uppers[by]);
+    stages.halves = 2 * chunks;
+    const int upper_stages = stages.upper;
 
     // loads: a wave moves rows 32 wave .. + 31 of an operand's stage, four loads of 8 rows x 128 bytes; lane = (row of the eight,
     // 16-byte column), columns swizzled as in dot_mfma_i8_kernel
@@ -1593,9 +1684,9 @@ __global__ __launch_bounds__(512, 2) void dot_mfma_i8_large_kernel(
         });                                                                                                                        \
         sk = nk;                                                                                                                   \
     }
-    if (uppers > 0) {
+    if (upper_stages > 0) {
 #pragma nounroll
-        for (int s = 0; s < uppers; ++s) BSI_LARGE_STAGE(late_upper = upper; upper = advance(off), late_upper ? rhi : rlo);
+        for (int s = 0; s < upper_stages; ++s) BSI_LARGE_STAGE(late_upper = upper; upper = advance(off), late_upper ? rhi : rlo);
         // their sums move up by their eight bits
 #pragma unroll
         for (int a = 0; a < 8; ++a)
@@ -2060,7 +2151,7 @@ static void launch_mfma_i8w(const int8_t* A8, const float* qscale, int stride, c
                            stream_output(), t_out_dtype);
 }
 
-// The large layers' launches: the images in units, the integer sums, and the chain for what they leave.  The rule, in us: a round of
+// The large layers' launches: the images in units, the bands, the integer sums, and the chain for what they leave.  The rule, in us: a round of
 // 256 workgroups takes 1 a chunk and 1 with tiles of 128 x 128; with tiles of 256 x 256 2.95 a chunk and 2, and 8 more for each round
 // but the last (all CUs store 32 MiB at the same time, with nothing else of theirs resident); the images are written at 0.75 a
 // million elements; the launch that ends at once and the gaps are 14.  Measured, 128 x 128 and 256 x 256, bf16: taken 1024 x 4096 x
@@ -2073,8 +2164,9 @@ static size_t large_aligned(size_t v) { return (v + 255) / 256 * 256; }
 size_t i8_large_workspace_bytes(int64_t Q, int chunks) {
     if (Q < kLargeMinQ || chunks > kLargeMaxChunks || Q > kLargeMaxItems / chunks) return 0;
     const size_t image = large_aligned(static_cast<size_t>(Q) * chunks * 256), words = static_cast<size_t>((chunks * 4 + 63) / 64);
+    const size_t bands = static_cast<size_t>((Q + kLargeTile - 1) / kLargeTile);
     return 2 * image + large_aligned(static_cast<size_t>(Q) * words * 8) + large_aligned(static_cast<size_t>(Q) * 4) +
-           large_aligned(static_cast<size_t>((Q + kLargeTile - 1) / kLargeTile) * 4);
+           large_aligned(bands * kLargeMaskWords * 8) + large_aligned(bands * 4) + large_aligned((bands + 1) * 4);
 }
 
 bool i8_large_serves(int64_t Q, int64_t R, int chunks) {
@@ -2090,10 +2182,20 @@ bool i8_large_serves(int64_t Q, int64_t R, int chunks) {
     return us_large < us_small;
 }
 
+// The same figures for the sums of some bands beside the chain for the others; where the tile is asked for, the chain takes no more than it has to.
+static LargeCost large_cost(int64_t Q, int64_t R, int chunks) {
+    const int64_t small_x = (R + 127) / 128, small_y = (Q + 127) / 128;
+    const float chain = static_cast<float>(chunks + 1);
+    const bool forced = g_i8_tile.load(std::memory_order_relaxed) == kLargeTile;
+    return LargeCost{2.95f * chunks + 10.0f, 1.475f, chain, forced ? INFINITY : chain * static_cast<float>((small_x * small_y + kCus - 1) / kCus),
+                     static_cast<int>((R + kLargeTile - 1) / kLargeTile), static_cast<int>(small_x)};
+}
+
 struct LargeWorkspace {
     unsigned char *lo, *hi, *masks;
     float* units;
-    unsigned* left;
+    unsigned char* bands;
+    unsigned *uppers, *left;
 };
 static LargeWorkspace large_workspace(void* workspace, int64_t Q, int chunks) {
     const size_t image = large_aligned(static_cast<size_t>(Q) * chunks * 256), words = static_cast<size_t>((chunks * 4 + 63) / 64);
@@ -2102,7 +2204,10 @@ static LargeWorkspace large_workspace(void* workspace, int64_t Q, int chunks) {
     w.hi = w.lo + image;
     w.masks = w.hi + image;
     w.units = reinterpret_cast<float*>(w.masks + large_aligned(static_cast<size_t>(Q) * words * 8));
-    w.left = reinterpret_cast<unsigned*>(reinterpret_cast<unsigned char*>(w.units) + large_aligned(static_cast<size_t>(Q) * 4));
+    const size_t bands = static_cast<size_t>((Q + kLargeTile - 1) / kLargeTile);
+    w.bands = reinterpret_cast<unsigned char*>(w.units) + large_aligned(static_cast<size_t>(Q) * 4);
+    w.uppers = reinterpret_cast<unsigned*>(w.bands + large_aligned(bands * kLargeMaskWords * 8));
+    w.left = reinterpret_cast<unsigned*>(w.bands + large_aligned(bands * kLargeMaskWords * 8) + large_aligned(bands * 4));
     return w;
 }
 
@@ -2139,20 +2244,23 @@ static void launch_i8_large_t(const LargeWorkspace& w, bool units_there, const i
         launch(i8_units_kernel, dim3(static_cast<unsigned>(Q)), dim3(kUnitsBlock), 0, st, A8, qscale, stride, chunks, Sa, Sb,
                reinterpret_cast<uint4*>(w.lo), reinterpret_cast<uint4*>(w.hi), reinterpret_cast<unsigned short*>(w.masks), w.units);
     const I8Grid g = i8_bands((R + kLargeTile - 1) / kLargeTile, (Q + kLargeTile - 1) / kLargeTile, 2);
+    launch(large_bands_kernel, dim3(static_cast<unsigned>(g.tiles_y)), dim3(kLargeTile), 0, st, reinterpret_cast<const unsigned long long*>(w.masks), w.units,
+           chunks, Q, reinterpret_cast<unsigned long long*>(w.bands), w.uppers);
     static LdsOptIn once, once_left;
     lds_opt_in(once, reinterpret_cast<const void*>(&dot_mfma_i8_large_kernel<kHalf>), kLargeLds);
     const unsigned char* const warm = static_cast<const unsigned char*>(g_warm_ptr);
     const long long warm_lines = static_cast<long long>(g_warm_bytes / 128);
     launch((dot_mfma_i8_large_kernel<kHalf>), dim3(static_cast<unsigned>(g.tiles_x) * static_cast<unsigned>(g.tiles_y)), dim3(512), kLargeLds, st,
-           reinterpret_cast<const int8_t*>(w.lo), reinterpret_cast<const int8_t*>(w.hi), reinterpret_cast<const unsigned long long*>(w.masks), w.units, K8,
-           Bw, Sb, chunks, R, Q, scale_inv, R_total, out, bias, warm, warm_lines, stream_output(), g, t_out_dtype, w.left);
+           reinterpret_cast<const int8_t*>(w.lo), reinterpret_cast<const int8_t*>(w.hi), reinterpret_cast<const unsigned long long*>(w.bands),
+           static_cast<const unsigned*>(w.uppers), large_cost(Q, R, chunks), w.units, K8, Bw, Sb, chunks, R, Q, scale_inv, R_total, out, bias, warm,
+           warm_lines, stream_output(), g, t_out_dtype, w.left);
     dim3 grid;
     const I8Grid tiles = i8_grid((R + 127) / 128, (Q + 127) / 128, &grid);
     using T = I8TilesCfg<128, 128>;
     lds_opt_in(once_left, reinterpret_cast<const void*>(&dot_mfma_i8_tiles_kernel<128, 128, kHalf, true>), T::kLdsTiles);
-    const int64_t left_tiles = static_cast<int64_t>(tiles.tiles_x) * tiles.tiles_y;  // every workgroup of that kernel has a tile
+    const int64_t left_tiles = static_cast<int64_t>(tiles.tiles_x) * tiles.tiles_y;  // of all bands; a workgroup without a tile ends before its first load
     launch((dot_mfma_i8_tiles_kernel<128, 128, kHalf, true>), dim3(static_cast<unsigned>(left_tiles < kCus ? left_tiles : kCus)), dim3(T::kBlock), T::kLdsTiles, st, A8, qscale, stride, K8, Bw, Sb, chunks,
-           R, Q, 16 - Sa - Sb, scale_inv, R_total, out, bias, 0, static_cast<const unsigned char*>(nullptr), 0LL, stream_output(), tiles,
+           R, Q, 16 - Sa - Sb, scale_inv, R_total, out, bias, 0, warm, warm_lines, stream_output(), tiles,
            static_cast<unsigned>(left_tiles), t_out_dtype, w.left);
 }
 void launch_i8_large(void* workspace, bool units_there, const int8_t* A8, const float* qscale, int stride, const int8_t* K8, const float* Bw, int Sa, int Sb,
