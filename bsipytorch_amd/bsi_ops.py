@@ -1272,7 +1272,25 @@ def _linear_workspace(device, need: int, capturing: bool) -> dict:
 
 
 _reserved_linear_shapes: set = set()
-_linear_ws_need: dict = {}
+_linear_ws_need: dict = {}  # (Q, d, bits) -> bytes that any layer takes, bytes that every layer takes
+
+
+def _linear_workspace_need(device, Q: int, d: int, bits: int, klayout: int, Sb: int, R: int, core: int, capturing: bool) -> int:
+    """Bytes of linear_cuda's workspace for a call.  Only a large layer takes the images that its kernel reads; one that is recorded
+    where no call has asked for them does without (the kernels of the other layers), since a capture cannot allocate."""
+    span = _linear_ws_need.get((Q, d, bits))
+    if span is None:  # pure functions of the shape: asked once per shape, not once per forward
+        span = _linear_ws_need[(Q, d, bits)] = (int(lib.bsi_hip_linear_workspace_bytes(Q, d, bits)),
+                                                int(lib.bsi_hip_linear_workspace_bytes_for(Q, d, bits, 0, 0, 0, 0)))
+    most, least = span
+    if most == least:
+        return least
+    need = int(lib.bsi_hip_linear_workspace_bytes_for(Q, d, bits, klayout, Sb, R, core))
+    if capturing and need > least:
+        ws = _linear_ws.get(device.index)
+        if ws is not None and ws["bytes"] < need:
+            return least
+    return need
 
 
 def reserve_linear_workspace(x2d: torch.Tensor) -> None:
@@ -1283,7 +1301,7 @@ def reserve_linear_workspace(x2d: torch.Tensor) -> None:
     key = (x2d.device.index, int(x2d.shape[0]), int(x2d.shape[1]), bits)
     if key in _reserved_linear_shapes or not (2 <= bits <= 8) or _capturing():
         return
-    _linear_workspace(x2d.device, int(lib.bsi_hip_linear_workspace_bytes(key[1], key[2], bits)), False)
+    _linear_workspace(x2d.device, int(lib.bsi_hip_linear_workspace_bytes_for(key[1], key[2], bits, 0, 0, 0, 0)), False)
     _reserved_linear_shapes.add(key)
 
 
@@ -1314,11 +1332,10 @@ def linear_cuda(x2d: torch.Tensor, keyset_cuda_cap, decimal_places: int, bias=No
     Q, d, R = int(x2d.shape[0]), int(x2d.shape[1]), keys.num_keys
     _check_bias(bias, R, x2d.device)
     bits = f["bits_q"]
-    need = _linear_ws_need.get((Q, d, bits))
-    if need is None:  # a pure function of the shape: asked once per shape, not once per forward
-        need = _linear_ws_need[(Q, d, bits)] = int(lib.bsi_hip_linear_workspace_bytes(Q, d, bits))
+    core = f["core"]
+    kptr, klayout = key_operand(keys, Q, bits, core)
     capturing = _capturing()
-    ws = _linear_workspace(x2d.device, need, capturing)
+    ws = _linear_workspace(x2d.device, _linear_workspace_need(x2d.device, Q, d, bits, klayout, keys.Sb, R, core, capturing), capturing)
     st = _stream()
     if capturing:
         buf, slot = ws["capture_buf"], ws["capture"]
@@ -1337,8 +1354,6 @@ def linear_cuda(x2d: torch.Tensor, keyset_cuda_cap, decimal_places: int, bias=No
         slot[0] = None  # until the build is enqueued
     wsptr = buf.data_ptr()
     out = torch.empty((Q, R), dtype=out_dtype, device=x2d.device)
-    core = f["core"]
-    kptr, klayout = key_operand(keys, Q, bits, core)
     if Q >= _SPLIT_MIN_Q:
         _attach_split_scratch_for(x2d.device, Q, R, (d + 63) // 64)
     wptr, wbytes = _warm_region(_capsule(warm_keys, PrebuiltBSIKeysCUDA, "Invalid CUDA keys capsule") if warm_keys is not None
@@ -1562,7 +1577,7 @@ def debug_quantize_int64_cpu(values: torch.Tensor, decimal_places: int) -> torch
 
 # The native host path reads these on every call, so what the functions above keep stays the one copy.
 _native.bind({name: ctypes.cast(getattr(lib, name), ctypes.c_void_p).value
-              for name in ("bsi_hip_linear_few_rows_out", "bsi_hip_linear_out", "bsi_hip_linear_workspace_bytes", "bsi_hip_dot",
+              for name in ("bsi_hip_linear_few_rows_out", "bsi_hip_linear_out", "bsi_hip_linear_workspace_bytes_for", "bsi_hip_dot",
                            "bsi_hip_build_fixed", "bsi_hip_build_fixed_keys", "bsi_hip_ewah_measure", "bsi_hip_ewah_emit", "bsi_hip_dot_ewah_batch",
                            "bsi_hip_dot_ewah_batch_workspace_bytes", "bsi_hip_scalar_query_dot",
                            "bsi_hip_build_measure", "bsi_hip_ewah_emit_at", "bsi_hip_linear_coop_out",

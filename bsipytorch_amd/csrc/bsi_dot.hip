@@ -306,7 +306,7 @@ extern "C" int bsi_hip_dot_static_scratch(const uint64_t* A, const float* A_chun
 
 // Workspace of bsi_hip_linear: the query operands of one build (planes, shifts, scales, int8 image), each 256-aligned.
 struct LinearWorkspace {
-    size_t words, shifts, scales, ints8, large, total;  // large: what the integer sums of a large layer take
+    size_t words, shifts, scales, ints8, large, total;  // large: where what the integer sums of a large layer take begins
 };
 static LinearWorkspace linear_workspace(int64_t Q, int64_t d, int fixed_bits) {
     const size_t W = static_cast<size_t>((d + 63) / 64), chunks = static_cast<size_t>((d + 255) / 256);
@@ -324,6 +324,17 @@ static LinearWorkspace linear_workspace(int64_t Q, int64_t d, int fixed_bits) {
 extern "C" size_t bsi_hip_linear_workspace_bytes(int64_t Q, int64_t d, int fixed_bits) {
     if (Q <= 0 || d <= 0 || fixed_bits < 2 || fixed_bits > 8) return 0;
     return linear_workspace(Q, d, fixed_bits).total;
+}
+
+static bool linear_is_large(int64_t Q, int chunks, int b_layout, int Sb, int64_t R, int core) {
+    return core == BSI_CORE_AUTO && b_layout == BSI_LAYOUT_INT8 && Sb >= 2 && Sb <= 8 && R > 0 && i8_large_serves(Q, R, chunks);
+}
+
+extern "C" size_t bsi_hip_linear_workspace_bytes_for(int64_t Q, int64_t d, int fixed_bits, int b_layout, int Sb, int64_t R, int core) {
+    if (Q <= 0 || d <= 0 || fixed_bits < 2 || fixed_bits > 8) return 0;
+    const LinearWorkspace w = linear_workspace(Q, d, fixed_bits);
+    const int64_t chunks = (d + 255) / 256;
+    return chunks <= kMfmaMaxChunks && linear_is_large(Q, static_cast<int>(chunks), b_layout, Sb, R, core) ? w.total : w.large;
 }
 
 extern "C" int bsi_hip_linear(const void* x, int dtype, int64_t Q, int64_t d, int decimal_places, int fixed_bits, int rebuild,
@@ -344,7 +355,7 @@ extern "C" int bsi_hip_linear_out(const void* x, int dtype, int64_t Q, int64_t d
     if (Q == 0 || R == 0) return BSI_OK;
     const int W64 = static_cast<int>((d + 63) / 64), chunks = (W64 + 3) / 4;
     const LinearWorkspace w = linear_workspace(Q, d, fixed_bits);
-    BSI_REQUIRE(workspace != nullptr && workspace_bytes >= w.total, "workspace of %zu bytes needed, %zu given", w.total,
+    BSI_REQUIRE(workspace != nullptr && workspace_bytes >= w.large, "workspace of %zu bytes needed, %zu given", w.large,
                 workspace_bytes);
     BSI_REQUIRE((reinterpret_cast<uintptr_t>(workspace) & 255) == 0, "workspace must be 256-byte aligned");
     unsigned char* ws = static_cast<unsigned char*>(workspace);
@@ -358,7 +369,7 @@ extern "C" int bsi_hip_linear_out(const void* x, int dtype, int64_t Q, int64_t d
     const bool planes = core == BSI_CORE_VALU || Sb < 2 || Sb > 8 || chunks > kMfmaMaxChunks ||
                         integer_decimal_scale(pow(10.0, static_cast<double>(decimal_places))) == 0;
     BSI_REQUIRE(warm != nullptr || warm_bytes == 0, "null warm-up region");
-    const bool large = core == BSI_CORE_AUTO && b_layout == BSI_LAYOUT_INT8 && Sb >= 2 && Sb <= 8 && i8_large_serves(Q, R, chunks);
+    const bool large = workspace_bytes >= w.total && linear_is_large(Q, chunks, b_layout, Sb, R, core);
     if (large) {
         if (int rc = check_dot(nullptr, ints8, scales, chunk_scale ? chunks : 1, fixed_bits, W64, B, b_layout, Bw, Sb, R, Q, R_total, out)) return rc;
         BSI_REQUIRE((reinterpret_cast<uintptr_t>(B) & 15) == 0, "int8 key image must be 16-byte aligned");

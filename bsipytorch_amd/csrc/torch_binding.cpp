@@ -29,7 +29,7 @@ namespace {
 struct Library {
     decltype(&bsi_hip_linear_few_rows_out) linear_few_rows_out;
     decltype(&bsi_hip_linear_out) linear_out;
-    decltype(&bsi_hip_linear_workspace_bytes) linear_workspace_bytes;
+    decltype(&bsi_hip_linear_workspace_bytes_for) linear_workspace_bytes_for;
     decltype(&bsi_hip_dot) dot;
     decltype(&bsi_hip_build_fixed) build_fixed;
     decltype(&bsi_hip_build_fixed_keys) build_fixed_keys;
@@ -380,7 +380,8 @@ PyObject* linear(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
         Holder index(PyLong_FromLong(device.index()));
         PyObject* record = PyDict_GetItem(shared.linear_ws, index.p);
         if (record == nullptr || !get_int(record, names.bytes, &ws_bytes) ||
-            static_cast<size_t>(ws_bytes) < lib.linear_workspace_bytes(rows, d, config.bits))
+            static_cast<size_t>(ws_bytes) <
+                lib.linear_workspace_bytes_for(rows, d, config.bits, k.operand_layout, static_cast<int>(k.Sb), k.R, config.core))
             Py_RETURN_NONE;
         if (!coop.defined()) {
             Holder handle(PyLong_FromVoidPtr(st));
@@ -891,7 +892,7 @@ PyObject* bind(PyObject*, PyObject* args) {
     long long lds;
     if (!PyArg_ParseTuple(args, "O!O!iiiL", &PyDict_Type, &entries, &PyDict_Type, &state, &few, &stream, &split, &lds)) return nullptr;
     if (!entry(entries, "bsi_hip_linear_few_rows_out", &lib.linear_few_rows_out) || !entry(entries, "bsi_hip_linear_out", &lib.linear_out) ||
-        !entry(entries, "bsi_hip_linear_workspace_bytes", &lib.linear_workspace_bytes) || !entry(entries, "bsi_hip_dot", &lib.dot) ||
+        !entry(entries, "bsi_hip_linear_workspace_bytes_for", &lib.linear_workspace_bytes_for) || !entry(entries, "bsi_hip_dot", &lib.dot) ||
         !entry(entries, "bsi_hip_build_fixed", &lib.build_fixed) ||
         !entry(entries, "bsi_hip_build_fixed_keys", &lib.build_fixed_keys) || !entry(entries, "bsi_hip_ewah_measure", &lib.ewah_measure) ||
         !entry(entries, "bsi_hip_ewah_emit", &lib.ewah_emit) || !entry(entries, "bsi_hip_dot_ewah_batch", &lib.dot_ewah_batch) ||

@@ -368,9 +368,11 @@ int bsi_hip_linear_few_rows_out(const void* x_device, int dtype, int64_t Q, int6
  * batch_dot_product_multiquery_cuda_batch_caps), with one trip through the host binding instead of two and no
  * per-call operand allocations.  rebuild = 0 skips the build and reuses the workspace's contents (layers that
  * read the same activations; with the same core and keys of the same slice count: the query planes are built only where
- * the dot reads them).  workspace: bsi_hip_linear_workspace_bytes(Q, d, fixed_bits) bytes, 256-aligned,
- * owned by the caller; B / b_layout as for bsi_hip_dot (int8 image or planes); warm as for bsi_hip_dot_bias_warm. */
+ * the dot reads them).  workspace: bytes as below, 256-aligned, owned by the caller; B / b_layout as for bsi_hip_dot (int8 image or planes); warm as for bsi_hip_dot_bias_warm. */
+/* Bytes of workspace: what any layer of Q x d takes, and what one on these keys takes.  Large layers have two more images of
+ * the queries there; with a workspace that holds what R = 0 takes, but not those, they run on the kernels of the others. */
 size_t bsi_hip_linear_workspace_bytes(int64_t Q, int64_t d, int fixed_bits);
+size_t bsi_hip_linear_workspace_bytes_for(int64_t Q, int64_t d, int fixed_bits, int b_layout, int Sb, int64_t R, int core);
 int bsi_hip_linear(const void* x_device, int dtype, int64_t Q, int64_t d, int decimal_places, int fixed_bits, int rebuild,
                    void* workspace, size_t workspace_bytes, const uint64_t* B, int b_layout, const float* Bw, int Sb,
                    int64_t R, float scale_inv, int64_t R_total, const float* bias, float* out, int core, const void* warm,
