@@ -678,10 +678,9 @@ PyObject* ewah_streams(PyObject*, PyObject* args) {
 
 // hybrid(x, decimals, threshold) -> (stream words, offsets, lengths, flags, scales, slice weights or None), or None: the
 // fixed-bit build of a contiguous [Q, d] batch on the current device, every slice EWAH-encoded.  The host waits for the
-// lengths, which arrive while the build's kernel still runs: their sum is the size of the streams.  No stream is longer than its
-// slice and a marker, so the emit pass is launched before they are here, into memory for that many words, and the GPU does not
-// stand still until the host has added them up.  Streams that need less than three quarters of that are emitted again
-// into memory of their own size.  us a pass of 64 x 2048 with its dot on 2048 keys, emitted when the sum is known and now: 35.5, 32.3.
+// lengths, which arrive while the build's kernel still runs: their sum is the size of the streams.  (Emitting ahead of the lengths, into
+// memory for the most a batch can need, takes 1 to 1.5 us off a pass of 64 x 2048 or 256 x 4096, adds 3 where the batch compresses and
+// has to be emitted again, and the memory that is kept is up to a third more than the streams; not done.)
 PyObject* hybrid(PyObject*, PyObject* args) {
     PyObject* o = nullptr;
     int decimals = 0;
@@ -722,17 +721,8 @@ PyObject* hybrid(PyObject*, PyObject* args) {
             if (!done) (void)hipStreamSynchronize(stream);
         }
     } writing{st, false};
-    at::Tensor off = at::detail::empty_cuda({S}, at::kLong, device, std::nullopt);
-    const int64_t most = S * (W + 1);
-    at::Tensor streams = at::detail::empty_cuda({most}, at::kLong, device, std::nullopt);
-    auto emit = [&] {
-        return lib.ewah_emit_at(w, static_cast<int>(S), static_cast<int>(W), static_cast<const int32_t*>(flags.data_ptr()),
-                                static_cast<const int32_t*>(lens.data_ptr()), static_cast<int64_t*>(off.data_ptr()),
-                                static_cast<uint64_t*>(streams.data_ptr()), st);
-    };
-    rc = emit();
-    if (rc != BSI_OK) return fail_status(rc, "bsi_hip_ewah_emit_at");
     // what can be made before the lengths are here
+    at::Tensor off = at::detail::empty_cuda({S}, at::kLong, device, std::nullopt);
     Holder b(THPVariable_Wrap(off)), c(THPVariable_Wrap(lens)), f(THPVariable_Wrap(flags)), s(THPVariable_Wrap(std::move(scales))),
         v(THPVariable_Wrap(std::move(weights)));
     Py_BEGIN_ALLOW_THREADS
@@ -750,14 +740,11 @@ PyObject* hybrid(PyObject*, PyObject* args) {
     Py_END_ALLOW_THREADS
     writing.done = true;
     if (rc != BSI_OK) return fail_status(rc, "bsi_hip_build_measure");
-    if (total < most - most / 4) {
-        streams = at::detail::empty_cuda({total}, at::kLong, device, std::nullopt);
-        rc = emit();
-        if (rc != BSI_OK) return fail_status(rc, "bsi_hip_ewah_emit_at");
-    } else {
-        streams.unsafeGetTensorImpl()->set_sizes_contiguous({total});
-        streams.storage().set_nbytes(static_cast<size_t>(total) * 8);
-    }
+    at::Tensor streams = at::detail::empty_cuda({total}, at::kLong, device, std::nullopt);
+    rc = lib.ewah_emit_at(w, static_cast<int>(S), static_cast<int>(W), static_cast<const int32_t*>(flags.data_ptr()),
+                          static_cast<const int32_t*>(lens.data_ptr()), static_cast<int64_t*>(off.data_ptr()),
+                          static_cast<uint64_t*>(streams.data_ptr()), st);
+    if (rc != BSI_OK) return fail_status(rc, "bsi_hip_ewah_emit_at");
     Holder a(THPVariable_Wrap(std::move(streams)));
     return PyTuple_Pack(6, a.p, b.p, c.p, f.p, s.p, v.p);
     END_HANDLE_TH_ERRORS

@@ -1,5 +1,5 @@
-"""The streams of a hybrid batch are emitted before their lengths are on the host: the tensors hold what the streams need and no
-more, whether they stay where they were emitted (three quarters of the most a batch can need, or more) or are emitted again."""
+"""The streams of a hybrid batch: the tensors hold what the streams need and no more, call after call, whatever share of the batch
+compresses."""
 import io
 
 import pytest
