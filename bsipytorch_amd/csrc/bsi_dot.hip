@@ -438,8 +438,15 @@ static int coop_plan(int64_t Q, int64_t d, int64_t R, int decimal_places, int fi
         // leave a CU one of them) 9.3, 9.9, 9.7.  More rows than waves, where few workgroups have few shares: 60 x 704 x 1024 (1.9 rounds) 8.5,
         // 9.6, 7.3; 250 x 320 x 1024 8.5, 9.9, 6.9; 90 x 900 x 1000 8.5, 9.9, 8.1; 200 x 448 x 700 (2.8) 8.5, 10.0, 8.2; 150 x 192 x 768 8.5,
         // 9.8, 7.0 -- beyond: 60 x 896 x 768 (2.5) 8.5, 9.8, 8.3; 50 x 640 x 640 (3.1) 8.5, 9.9, 8.7; 128 x 832 x 640 8.5, 9.8, 9.3.
+        // The edge at 560 items, us in two launches on three hosts and in one: 539 items (77 x 1600 x 4800) 7.6, 8.8, 9.2, 8.2; 560 (70 x 1984 x
+        // 4000) -, 9.2, 10.0, 8.6; beyond: 588 (84 x 1600 x 4800) 7.6, 8.7, 9.0, 8.2; 600 (150 x 960 x 4000) 7.1, 8.7, 9.0, 8.1; 630 (90 x 1600 x
+        // 4800) 7.7, 8.7, 8.7, 8.4; 660 (220 x 704 x 6000) 9.2, -, 9.7, 10.0; 720 (120 x 1472 x 4096) 7.3, 8.6, 8.9, 8.2; 720 (90 x 1984 x 5000)
+        // 8.2, -, 8.8, 9.1; 728 (104 x 1600 x 4800) 8.1, 8.9, 9.1, 9.6; 784 (112 x 1600 x 4800) 8.1, -, 9.2, 9.6; 900 (300 x 576 x 2048) 7.1, -,
+        // 8.9, 8.5.  One launch is bound by the GPU, two by the host: up to some 600 items it gains on most hosts and loses at most half a
+        // microsecond on the fastest; from 730 on it loses on all.  Rows beyond 512: 500 x 192 x 2000 -, 9.0, 9.4, 7.9, but 550 x
+        // 192 x 2000 -, 9.2, 9.3, 10.0 and 560 x 100 x 2000 -, 9.3, 9.5, 9.7.
         const int rounds = chunks <= 2 ? 3 : (chunks <= 4 ? 2 : 1);
-        return Q <= rounds * static_cast<int64_t>(shares) * waves && chunks <= kCoopHeld && d % 4 == 0 && Q * chunks <= 560 && groups <= 256 ? 2 : 0;
+        return Q <= 512 && Q <= rounds * static_cast<int64_t>(shares) * waves && chunks <= kCoopHeld && d % 4 == 0 && Q * chunks <= 560 && groups <= 256 ? 2 : 0;
     }
     const int64_t items = Q * chunks, a_round = static_cast<int64_t>(shares) * waves;
     if (items <= 2 * a_round) return 1;
