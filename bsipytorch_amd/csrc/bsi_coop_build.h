@@ -20,9 +20,12 @@
 //    before all its flags are there, so that the first load of a line fetches it from the L2.  That is why coop_build hands
 //    out the copy's address only when it returns, and why ahead() must not load from `area`: a load there would compile and
 //    read right most of the time.
-//  - Flags are read past the L1 (agent scope) and share no line with a copy; a copy's lines belong to it alone.  Lines of the
-//    scales are written by several CUs, four bytes each: an L1 writes through and answers with no byte of a line that it
-//    has not fetched or written itself.
+//  - Flags are read past the L1 (agent scope) and share no line with a copy; a copy's lines belong to it alone.
+//  - Lines of a copy that several CUs write lose no byte of it: an L1 writes through the bytes that were stored and no others, the
+//    L2 puts them together, and an L1 answers with no byte of a line that it has not fetched or written itself.  Such are the lines of
+//    the scales, four bytes a wave, and, in the order of the few-rows kernel's operands (kFragments), those of the image: a line of
+//    128 bytes holds 16 of each of eight rows, written by up to eight waves of as many CUs.  In rows one after the other an item's 256
+//    bytes are two lines, and one wave's.
 // Inside a launch of 16 rows of 4096 the workgroups have the whole build 3.2 us after the first wave has begun (wall clock stamps:
 // 1.3 until a wave has its chunk and has quantised it, 0.9 to the flag, the stamps' own stores among that, 0.6 to the last
 // share); 2.3 us at 16 rows of 512.  That is as long as the launch it replaces, but for the host.
