@@ -17,6 +17,8 @@
 //           dot_mfma_ws_kernel       many rows on tiled planes (producer waves recombine the planes)
 //           dot_mfma_kernel          canonical planes or slice counts other than 6
 //
+// Shapes in the comments are rows x width x keys.
+//
 // Operands whose slice count follows the data (decimal mode) carry float slice weights instead of scales:
 //   dot_weighted_kernel      popcounts per slice pair, summed exactly in float64 (any Sa, Sb <= 64)
 //   dot_mfma_i8_kernel in its int32-sum mode on int8 digit images (planes_to_digits_kernel), the digits put back

@@ -1,6 +1,6 @@
 // The dot for a few query rows (decode steps): kernels that stream the packed key planes once -- on a built int8
 // query image, with the query build inside, or with queries handed over as EWAH streams -- and the stream -> int8
-// image pass for larger batches of EWAH queries.
+// image pass for larger batches of EWAH queries.  Shapes in the comments are rows x width x keys.
 #include "bsi_dot_internal.h"
 #include "bsi_coop_build.h"
 #include <type_traits>

@@ -1,5 +1,6 @@
 // The matrix-core dot on the cached int8 image of the keys (the compute-bound calls), its probe of the L2 -> LDS
 // path, the timeline stamps, and the decimal-mode dot on int8 digit images that runs on the same kernel.
+// Shapes in the comments are rows x width x keys.
 #include "bsi_coop_build.h"
 #include "bsi_dot_internal.h"
 
@@ -79,7 +80,7 @@ struct I8Cfg {
     static constexpr int kConsumers = 2 * kWavesN;
     static constexpr int kGroups = (TM + TN) / 8;      // groups of 8 operand rows (1 KiB per half-chunk) in a stage
     // loader waves: one per SIMD (the more waves issue a stage's loads, the faster it comes) -- but two for the
-    // 64 x 64 tile, measured: on one machine 512 x 2048 x 8192 takes 17.4 us with two and 18.7 with four (with four
+    // 64 x 64 tile, measured: on one machine 512 x 8192 x 2048 takes 17.4 us with two and 18.7 with four (with four
     // or with eight MFMA waves alike), while the 64 x 32 and 128 x 64 tiles gain 5 to 10 % from four
     static constexpr int kLoaders = (TM == 64 && TN == 64) ? 2 : 4;
     static constexpr int kLoads = (kGroups + kLoaders - 1) / kLoaders;  // loads per loader wave and stage
@@ -106,8 +107,8 @@ constexpr int kLargeTile = 256;  // dot_mfma_i8_large_kernel: keys and queries o
 // one float of 64 queries is up to 64 lines, half as many again as the operands of a chunk of the 64 x 64 tile have, four floats
 // of 16 are 16.  Rows of fewer than 16 chunks have several queries in a line and gain nothing for the code and the loads ahead
 // of the first group; nor do row scales.
-// us, one and four (64 x 64 tiles) 512 x 2048 x 8192 16.4, 15.5; 256 x 1024 x 8192 11.4, 10.5; (128 x 64) 512 x 4096 x 4096 12.5,
-// 11.7; (128 x 128) 512 x 8192 x 8192 34.5, 32.8 -- and at 8 chunks 512 x 8192 x 2048 11.2, 11.5, 512 x 2048 x 2048 5.8, 6.0.
+// us, one and four (64 x 64 tiles) 512 x 8192 x 2048 16.4, 15.5; 256 x 8192 x 1024 11.4, 10.5; (128 x 64) 512 x 4096 x 4096 12.5,
+// 11.7; (128 x 128) 512 x 8192 x 8192 34.5, 32.8 -- and at 8 chunks 512 x 2048 x 8192 11.2, 11.5, 512 x 2048 x 2048 5.8, 6.0.
 static bool i8_four_scales(int qscale_stride) { return qscale_stride >= 16; }
 
 // Timeline build (make TIMELINE=1, -DBSI_TIMELINE): one MFMA wave and one loader wave of every workgroup of
@@ -394,7 +395,8 @@ __device__ __forceinline__ bool i8_store_lines(const float (&v)[WM][WN][4], floa
 // keys, so a store instruction writes 64 contiguous bytes per query.
 // The type and whether there is a bias are looked at once a call, not once an output: 25 instructions a store where there were 175,
 // a branch, two conversions and a choice for each of its eight outputs.  us a layer, before and now: 512 x 2048 x 8192 bf16 17.6, 16.1;
-// 1024 x 4096 x 4096 bf16 28.1, 26.8; 333 x 2048 x 2048 f16 9.5, 9.2; 4096 x 4096 x 16384 bf16 270, 266, with tiles of 128 x 128 321, 310.
+// 1024 x 4096 x 4096 bf16 28.1, 26.8; 4096 x 4096 x 16384 bf16 270, 266, with tiles of 128 x 128 321, 310.  Of 333 x 2048 x 2048 f16 the
+// kernel, 7.1, 6.6; the layer is bound by the host, and no faster.
 template <int WM, int WN>
 __device__ __forceinline__ void i8_store_half(const float (&v)[WM][WN][4], const float (&bi)[WM][4], bool has_bias, int dtype,
                                               float* __restrict__ out, int64_t R_total, int64_t rw, int64_t qw, int64_t R,
@@ -451,8 +453,8 @@ __device__ __forceinline__ void i8_store_half(const float (&v)[WM][WN][4], const
 
 // The end of a tile in the chain modes: every output takes its key's factor, the decimal scale and the bias, and is stored.
 // kHalf: the outputs are in the half-precision type out_dtype, else float32.  One kind of store a kernel: with both in one, a
-// launch of a few microseconds fetches instructions it does not run between those it does (us, both and one: 64 x 256 x 2048
-// 4.89, 4.77; 40 x 1024 x 1024 3.70, 3.55; 77 x 4800 x 1600 4.63, 4.48; 100 x 3000 x 1000 4.20, 4.03).
+// launch of a few microseconds fetches instructions it does not run between those it does (us, both and one: 64 x 2048 x 256
+// 4.89, 4.77; 40 x 1024 x 1024 3.70, 3.55; 77 x 1600 x 4800 4.63, 4.48; 100 x 1000 x 3000 4.20, 4.03).
 // epi: the key factors and biases of the tile's TM rows, from the copy the loader waves staged in LDS (0 for rows past R and
 // for a call without bias): two 16-byte reads per 16-key tile.
 template <int TM, int WM, int WN, bool kHalf>
@@ -1254,15 +1256,16 @@ __global__ __launch_bounds__((I8Cfg<TM, TN>::kBlock)) void dot_mfma_i8_tiles_ker
 // 284; 2048 x 8192 x 8192 f32 141, 164, 163, 164, 163, 149; 4096 x 3072 x 16384 f16 199, 217, 217, 228, 245, 226; 1024 x 4096 x 16384 bf16
 // 76, 86, 86, 86, 86, 77.  (All tiles in the chain wherever one band was left: 1.8 times the time of none.  Tiles of the kept bands where
 // they lie in the matrix: 4096 x 4096 x 16384, a quarter 302, half 356.)  What a layer loses of which nothing is kept is the images, 8,
-// and three launches.
+// and two launches.
 //
 // Without the chain there are no second accumulators and no scales, a wave holds 128 x 64 outputs and a workgroup 256 x 256:
 // half the bytes from the L2 and two thirds of the LDS reads a multiply-add, both of which the clock pays for.  Eight waves that load
 // for themselves (eight loads a half-chunk among 64 MFMAs; two waves a SIMD leave room for no others); LDS is a ring of five
 // slots of an operand's half-chunk, 256 rows x 128 bytes: K runs three stages ahead, Q two.
-// us a layer with its build, tiles of 128 x 128 and now: 4096 x 4096 x 16384 bf16 303, 260 (this kernel 222, 279 k cycles of its 504 k
-// with the matrix pipes busy); 2048 x 8192 x 8192 f32 161, 139; 2048 x 2048 x 16384 bf16 88.6, 84.4.  What is left: 400 cycles of
-// each half-chunk's 2450 at its barrier, the stores at the end of a round of tiles, the clock (2.1 GHz).  Tried beside it: touching
+// us a layer with its build, tiles of 128 x 128 and now: 4096 x 4096 x 16384 bf16 283, 246 (this kernel 222); 2048 x 8192 x 8192 f32 152,
+// 141; 4096 x 3072 x 16384 f16 227, 199; 1024 x 4096 x 16384 bf16 78, 76.  Of the launch's 483 k cycles the matrix pipes are busy in 280 k.
+// A tile of 4096 (stamps): 4 to 5 us until its first stage is there and 4.2 for its stores, at 2.1 to 2.4 GHz with the pipes idle, 41 to 47
+// of loop at 1.75 to 1.87, 2260 to 2410 cycles a stage and 2048 of them MFMA.  Tried beside it: touching
 // lines of later stages ahead of their loads (260 -> 275, the loads are not what is waited for), the loads in one run behind the
 // barrier (260 -> 267 -> 275 with their offsets worked out there too).
 constexpr int kLargeSlot = kLargeTile * 128, kLargeSlots = 5, kLargeLds = kLargeSlots * kLargeSlot;
