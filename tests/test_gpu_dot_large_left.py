@@ -53,6 +53,39 @@ def test_same_bits_by_the_rule(hip, ops, Q, d, R, left):
     assert torch.equal(call(hip, layer, x, 0), call(hip, layer, x.clone(), 128))
 
 
+def test_replays_find_other_bands_left(hip, ops):
+    """One recorded layer, replayed on inputs of which none, some and all bands are left."""
+    layer, Q, d = layer_of(1024, 700), 1153, 1024
+    static = inputs(Q, d, (), 1)
+    hip.check(hip.lib.bsi_hip_set_option(hip.OPT_I8_TILE, 256), "tile")
+    try:
+        with torch.no_grad():
+            layer(static)
+            torch.cuda.synchronize()
+            graph = torch.cuda.CUDAGraph()
+            with torch.cuda.graph(graph):
+                out = layer(static)
+    finally:
+        hip.check(hip.lib.bsi_hip_set_option(hip.OPT_I8_TILE, 0), "tile")
+    for left in ((), (1,), (0, 1, 2, 3, 4), (4,), (), (0, 2)):
+        x = inputs(Q, d, left, 2 + len(left))
+        static.copy_(x)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, call(hip, layer, x, 128))
+
+
+@pytest.mark.parametrize("left", [(), (2,), (0, 1, 2, 3, 4)])
+def test_with_the_next_layers_keys_touched(hip, ops, left):
+    """By the sums' workgroups, or by the chain's where all bands are left."""
+    from bsipytorch_amd.linear import quantize_model_bsi
+
+    model = quantize_model_bsi(torch.nn.Sequential(torch.nn.Linear(768, 1024), torch.nn.Linear(1024, 300)).cuda().eval(), 2,
+                               compress_threshold=0.5, verbose=False)
+    x = inputs(1100, 768, left, 11)
+    assert torch.equal(call(hip, model, x, 256), call(hip, model, x.clone(), 128))
+
+
 @pytest.mark.parametrize("Q, d, R", [(4096, 4096, 16384), (2048, 8192, 8192)])
 def test_a_band_that_is_left_costs_its_own_time(hip, ops, Q, d, R):
     """One band: its chain, or the whole layer's instead of the sums where that is less.  Both kernels in full are 1.8 times the time;
