@@ -50,6 +50,7 @@ PROTOTYPES = {
     "bsi_hip_ewah_size": [_vp, _i, _i, _vp, _vp, _vp],
     "bsi_hip_ewah_measure": [_vp, _i, _i, _d, _vp, _vp, _vp, _vp, _vp],
     "bsi_hip_build_measure": [_vp, _i, _i64, _i64, _i, _i, _i, _d, _vp, _vp, _vp, _vp, _vp, _vp, _vp],
+    "bsi_hip_build_measure_rows": [_vp, _i, _i64, _i64, _i, _i, _i, _d, _vp, _vp, _vp, _vp, _vp, _vp, _vp],
     "bsi_hip_ewah_emit_at": [_vp, _i, _i, _vp, _vp, _vp, _vp, _vp],
     "bsi_hip_ewah_emit": [_vp, _i, _i, _vp, _vp, _vp, _vp, _vp],
     "bsi_hip_ewah_decompress": [_vp, _i, _i, _vp, _vp],

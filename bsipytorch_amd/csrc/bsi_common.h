@@ -241,7 +241,10 @@ __device__ __forceinline__ void ewah_expand_wave(const unsigned long long* __res
         o += n_run;
         int n_lit = static_cast<int>(lit < static_cast<unsigned>(W - o) ? lit : static_cast<unsigned>(W - o));
         if (n_lit > in_len - idx) n_lit = in_len - idx;
-        for (int k = lane; k < n_lit; k += BSI_WAVE) dst[o + k] = in[idx + k];
+        // literals that the window holds are written from it: reading them again is a round trip to memory behind the window's own
+        const int rel = idx - win_at, held = n_lit < BSI_WAVE - rel ? n_lit : BSI_WAVE - rel;
+        if (lane >= rel && lane < rel + held) dst[o + lane - rel] = win;
+        for (int k = held + lane; k < n_lit; k += BSI_WAVE) dst[o + k] = in[idx + k];
         o += n_lit;
         idx += n_lit;
         if (static_cast<unsigned>(n_lit) < lit) break;     // clipped: the reference loop stops here too

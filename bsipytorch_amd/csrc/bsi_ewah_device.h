@@ -26,10 +26,11 @@ __device__ __forceinline__ int compress_flag(unsigned long long count, int W, do
 // One wave encodes one slice of W words (out == nullptr: size pass only).  Returns the stream length in every lane.
 // The stream is the reference's greedy one (bsi_cuda_kernels_ewah.cuh:118-232): [marker: run of equal clean words,
 // only when the slice is flagged][literals up to the next clean word] ..., an unflagged slice being one marker with
-// W literals.
+// W literals.  `first` is the lane's word of the first block (0 past the slice): a kernel that has other loads to wait for asks
+// for it beside them.
 __device__ __forceinline__ unsigned long long ewah_encode_wave(const unsigned long long* __restrict__ base, int W,
                                                                int compress, unsigned long long* __restrict__ out,
-                                                               int lane) {
+                                                               int lane, unsigned long long first) {
     const unsigned long long lt = (1ULL << lane) - 1ULL;  // lanes below this one
     unsigned long long n_starts = 0, n_lits = 0;          // markers / literal words before the current block
     // the segment that is open when a block begins: where it started, literals before it, its marker's place
@@ -40,7 +41,7 @@ __device__ __forceinline__ unsigned long long ewah_encode_wave(const unsigned lo
     for (int b = 0; b < W; b += BSI_WAVE) {
         const int i = b + lane;
         const bool valid = i < W;
-        const unsigned long long v = valid ? base[i] : 0ULL;
+        const unsigned long long v = b == 0 ? first : (valid ? base[i] : 0ULL);
         const bool clean = compress && valid && (v == 0ULL || v == ~0ULL);
         unsigned long long pv = __shfl_up(v, 1, BSI_WAVE);
         bool pc = __shfl_up(static_cast<int>(clean), 1, BSI_WAVE) != 0;
@@ -94,6 +95,10 @@ __device__ __forceinline__ unsigned long long ewah_encode_wave(const unsigned lo
         out[open_pos] = (run_len ? open_bit : 0ULL) | ((run_len & 0xFFFFFFFFULL) << 1) | (seg_lits << 33);
     }
     return n_starts + n_lits;
+}
+__device__ __forceinline__ unsigned long long ewah_encode_wave(const unsigned long long* __restrict__ base, int W, int compress,
+                                                               unsigned long long* __restrict__ out, int lane) {
+    return ewah_encode_wave(base, W, compress, out, lane, lane < W ? base[lane] : 0ULL);
 }
 
 }  // namespace bsi

@@ -41,7 +41,7 @@ struct Library {
     decltype(&bsi_hip_linear_coop_serves) linear_coop_serves;
     decltype(&bsi_hip_linear_coop_bytes) linear_coop_bytes;
     decltype(&bsi_hip_scalar_query_dot) scalar_query_dot;
-    decltype(&bsi_hip_build_measure) build_measure;
+    decltype(&bsi_hip_build_measure_rows) build_measure_rows;
     decltype(&bsi_hip_ewah_emit_at) ewah_emit_at;
     decltype(&bsi_hip_scalar_query_host_words) scalar_query_host_words;
 } lib;
@@ -678,7 +678,7 @@ PyObject* ewah_streams(PyObject*, PyObject* args) {
 
 // hybrid(x, decimals, threshold) -> (stream words, offsets, lengths, flags, scales, slice weights or None), or None: the
 // fixed-bit build of a contiguous [Q, d] batch on the current device, every slice EWAH-encoded.  The host waits for the
-// lengths, which arrive while the build's kernel still runs: their sum is the size of the streams.  (Emitting ahead of the lengths, into
+// lengths, which arrive a row at a time while the build's kernel still runs: their sum is the size of the streams.  (Emitting ahead of the lengths, into
 // memory for the most a batch can need, takes 1 to 1.5 us off a pass of 64 x 2048 or 256 x 4096, adds 3 where the batch compresses and
 // has to be emitted again, and the memory that is kept is up to a third more than the streams; not done.)
 PyObject* hybrid(PyObject*, PyObject* args) {
@@ -695,7 +695,7 @@ PyObject* hybrid(PyObject*, PyObject* args) {
     const at::Device device = x.device();
     hipStream_t const st = stream_of(device);
     const int64_t Q = x.size(0), d = x.size(1), W = (d + 63) / 64, chunks = (d + 255) / 256, S = Q * config.bits;
-    if (W > 1024 || S > 8192 || capturing(st)) Py_RETURN_NONE;  // bsi_hip_build_measure's limits
+    if (W > 1024 || S > 8192 || capturing(st)) Py_RETURN_NONE;  // bsi_hip_build_measure_rows's limits
     const bool chunked = W % 4 == 0;
     at::Tensor words = at::detail::empty_cuda({S, W}, at::kLong, device, std::nullopt);
     at::Tensor scales = chunked ? at::detail::empty_cuda({Q, chunks}, at::kFloat, device, std::nullopt)
@@ -704,15 +704,15 @@ PyObject* hybrid(PyObject*, PyObject* args) {
     if (!chunked) weights = at::detail::empty_cuda({Q, config.bits}, at::kFloat, device, std::nullopt);
     at::Tensor flags = at::detail::empty_cuda({S}, at::kInt, device, std::nullopt);
     at::Tensor lens = at::detail::empty_cuda({S}, at::kInt, device, std::nullopt);
-    at::Tensor pinned = at::detail::empty_cpu({S}, at::kInt, /*pin_memory=*/true);
+    at::Tensor pinned = at::detail::empty_cpu({Q}, at::kInt, /*pin_memory=*/true);
     volatile int32_t* const host = static_cast<volatile int32_t*>(pinned.data_ptr());
     uint64_t* const w = static_cast<uint64_t*>(words.data_ptr());
     int64_t total = 0;
-    for (int64_t s = 0; s < S; ++s) host[s] = -1;
-    int rc = lib.build_measure(x.const_data_ptr(), code, Q, d, decimals, config.bits, chunked ? 1 : 0, threshold, w,
+    for (int64_t q = 0; q < Q; ++q) host[q] = -1;
+    int rc = lib.build_measure_rows(x.const_data_ptr(), code, Q, d, decimals, config.bits, chunked ? 1 : 0, threshold, w,
                            static_cast<float*>(scales.data_ptr()), chunked ? nullptr : static_cast<float*>(weights.data_ptr()),
                            static_cast<int32_t*>(flags.data_ptr()), static_cast<int32_t*>(lens.data_ptr()), const_cast<int32_t*>(host), st);
-    if (rc != BSI_OK) return fail_status(rc, "bsi_hip_build_measure");
+    if (rc != BSI_OK) return fail_status(rc, "bsi_hip_build_measure_rows");
     // The kernel writes into `pinned` until the last length is there: an allocation that fails before that waits for it.
     struct Writing {
         hipStream_t stream;
@@ -729,17 +729,17 @@ PyObject* hybrid(PyObject*, PyObject* args) {
     // the stream is waited for only if the lengths are long in coming
     const auto until = std::chrono::steady_clock::now() + std::chrono::microseconds(500);
     bool waited = false;
-    for (int64_t s = 0; s < S && rc == BSI_OK; ++s) {
-        while (host[s] < 0 && !waited)
+    for (int64_t q = 0; q < Q && rc == BSI_OK; ++q) {
+        while (host[q] < 0 && !waited)
             if (std::chrono::steady_clock::now() > until) {
                 waited = true;
                 if (hipStreamSynchronize(st) != hipSuccess) rc = BSI_ERR_HIP;
             }
-        total += host[s];
+        total += host[q];
     }
     Py_END_ALLOW_THREADS
     writing.done = true;
-    if (rc != BSI_OK) return fail_status(rc, "bsi_hip_build_measure");
+    if (rc != BSI_OK) return fail_status(rc, "bsi_hip_build_measure_rows");
     at::Tensor streams = at::detail::empty_cuda({total}, at::kLong, device, std::nullopt);
     rc = lib.ewah_emit_at(w, static_cast<int>(S), static_cast<int>(W), static_cast<const int32_t*>(flags.data_ptr()),
                           static_cast<const int32_t*>(lens.data_ptr()), static_cast<int64_t*>(off.data_ptr()),
@@ -884,7 +884,7 @@ PyObject* bind(PyObject*, PyObject* args) {
         !entry(entries, "bsi_hip_build_fixed_keys", &lib.build_fixed_keys) || !entry(entries, "bsi_hip_ewah_measure", &lib.ewah_measure) ||
         !entry(entries, "bsi_hip_ewah_emit", &lib.ewah_emit) || !entry(entries, "bsi_hip_dot_ewah_batch", &lib.dot_ewah_batch) ||
         !entry(entries, "bsi_hip_dot_ewah_batch_workspace_bytes", &lib.dot_ewah_batch_workspace_bytes) ||
-        !entry(entries, "bsi_hip_build_measure", &lib.build_measure) || !entry(entries, "bsi_hip_ewah_emit_at", &lib.ewah_emit_at) ||
+        !entry(entries, "bsi_hip_build_measure_rows", &lib.build_measure_rows) || !entry(entries, "bsi_hip_ewah_emit_at", &lib.ewah_emit_at) ||
         !entry(entries, "bsi_hip_linear_coop_out", &lib.linear_coop_out) ||
         !entry(entries, "bsi_hip_linear_coop_serves", &lib.linear_coop_serves) ||
         !entry(entries, "bsi_hip_linear_coop_bytes", &lib.linear_coop_bytes) ||

@@ -183,10 +183,14 @@ int bsi_hip_ewah_emit(const uint64_t* words_device, int S, int W, const int32_t*
  * every slice in the same launch: words [Q, fixed_bits, W64], scales [Q, ceil(d / 256)] or [Q], weights [Q, fixed_bits]
  * (slice weights, row scales only), flags / lens [Q * fixed_bits]; lens_host: the lengths again, in pinned host memory, each
  * stored once.  BSI_ERR_UNSUPPORTED beyond 1024 words a slice or 8192 slices.  bsi_hip_ewah_emit_at: offsets and streams
- * from the flags and lengths (lens 16-byte aligned). */
+ * from the flags and lengths (lens 16-byte aligned).  bsi_hip_build_measure_rows: to the host goes the sum of a row's lengths
+ * (row_lens_host [Q], pinned, each stored once), a fixed_bits-th of the words on the way to the host. */
 int bsi_hip_build_measure(const void* x_device, int dtype, int64_t Q, int64_t d, int decimal_places, int fixed_bits, int chunk_scale,
                           double threshold, uint64_t* words, float* scales, float* weights, int32_t* flags, int32_t* lens,
                           int32_t* lens_host, void* stream);
+int bsi_hip_build_measure_rows(const void* x_device, int dtype, int64_t Q, int64_t d, int decimal_places, int fixed_bits, int chunk_scale,
+                               double threshold, uint64_t* words, float* scales, float* weights, int32_t* flags, int32_t* lens,
+                               int32_t* row_lens_host, void* stream);
 int bsi_hip_ewah_emit_at(const uint64_t* words_device, int S, int W, const int32_t* flags_device, const int32_t* lens_device,
                          int64_t* off_device, uint64_t* out_device, void* stream);
 /* One stream -> W literal words.  Replaces launch_ewah_decompress (ewah.cuh:35-42). */
