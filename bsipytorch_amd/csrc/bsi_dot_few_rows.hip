@@ -823,10 +823,18 @@ extern "C" int bsi_hip_dot_ewah_batch(const uint64_t* comp_words, const int64_t*
     BSI_REQUIRE(A_scale_stride == chunks || A_scale_stride == 1,
                 "chunk scale stride mismatch: got %d expected %d (or 1 for row scales)", A_scale_stride, chunks);
     hipStream_t st = as_stream(stream);
-    // A few rows against the packed planes: the call is bound by streaming the keys once, and each workgroup can
-    // afford to expand the queries itself -- the decode is part of the dot kernel's load stage.
+    // A few rows against the packed planes: each workgroup can afford to expand the queries itself -- the decode is part of the
+    // dot kernel's load stage.  Every workgroup repeats it, though, and more than 16 rows stream the keys twice, so with more than
+    // eight rows, or eight's worth of 4096 elements, a launch for the decode pays for itself.  us a pass of build and dot, decode
+    // inside and in a launch ahead (rows x width x keys): 4 x 4096 x 4096 27.2, 29.0; 8 x 2048 x 2048 27.8, 29.1; 8 x 4096 x 4096
+    // 28.9, 28.9 -- beyond: 4 x 8192 x 1024 31.2, 29.6; 8 x 8192 x 1024 32.8, 30.2; 12 x 768 x 768 33.7, 29.5; 12 x 2048 x 2048
+    // 30.8, 29.1; 16 x 2048 x 8192 33.4, 28.9; 32 x 1600 x 4800 42.2, 30.9; 32 x 4096 x 4096 39.5, 31.1.  Calls without a workspace
+    // have no choice.
     const int64_t group = Q < kEwahQueriesPerGroup ? Q : kEwahQueriesPerGroup;
-    if (Q <= kStreamMaxQ && b_layout == BSI_LAYOUT_TILED16 && Sb == 6 &&
+    const size_t need = bsi_hip_dot_ewah_batch_workspace_bytes(Q, W64);
+    const bool decode_ahead = (Q > 8 || Q * chunks >= 128) && workspace != nullptr && workspace_bytes >= need &&
+                              (reinterpret_cast<uintptr_t>(workspace) & 15) == 0;
+    if (!decode_ahead && Q <= kStreamMaxQ && b_layout == BSI_LAYOUT_TILED16 && Sb == 6 &&
         ewah_plane_region(static_cast<int>(group), Sa, chunks * 4) + 128 <= 120 * 1024)
         return launch_stream_ewah(comp_words, comp_off, comp_len, Sa, W64, A_chunk_scales, A_scale_stride, B, Bw, R, Q,
                                   scale_inv, R_total, bias, out, chunk_ints, st);
@@ -834,7 +842,6 @@ extern "C" int bsi_hip_dot_ewah_batch(const uint64_t* comp_words, const int64_t*
     // streams there would repeat the decode and the plane -> int8 recombination once per key tile (32 times at
     // Q512 x R2048).  The call's load stage therefore runs once, as a launch of its own: streams -> int8 query
     // image in the workspace (the verbatim planes are never materialised), then the dot on that image.
-    const size_t need = bsi_hip_dot_ewah_batch_workspace_bytes(Q, W64);
     BSI_REQUIRE(workspace != nullptr && workspace_bytes >= need, "%zu bytes of workspace needed for the int8 query image (got %zu)",
                 need, workspace_bytes);
     BSI_REQUIRE((reinterpret_cast<uintptr_t>(workspace) & 15) == 0, "workspace must be 16-byte aligned");

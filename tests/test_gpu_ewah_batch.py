@@ -1,5 +1,5 @@
 """Query batches kept as EWAH streams (the batched hybrid form) through bsi_hip_dot_ewah_batch: the decode runs in
-the dot's load stage -- inside the few-rows kernel up to 32 rows on tiled planes, as the call's first launch above --
+the dot's load stage -- inside the few-rows kernel for a few rows on tiled planes, as the call's first launch above --
 and the result must be what the same dot gives on the verbatim planes: integer accumulators and fp32 outputs
 bit-identical to the oracle.  Streams come from the oracle's encoder (so the test does not depend on the GPU
 encoder) and, through the ``bsi_ops`` mirror, from the GPU encoder, which must write the same words."""

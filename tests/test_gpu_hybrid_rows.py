@@ -49,3 +49,29 @@ def test_literals_around_the_window(ops, W):
     assert _lib.lib.bsi_hip_ewah_decompress_batch(comp.data_ptr(), off.data_ptr(), lens.data_ptr(), 6, W, out.data_ptr(),
                                                   torch.cuda.current_stream().cuda_stream) == 0
     np.testing.assert_array_equal(out.cpu().numpy().view(np.uint64), words)
+
+
+@pytest.mark.parametrize("Q,d,R", [(8, 2048, 300), (9, 2048, 300), (16, 1600, 77), (17, 257, 40), (32, 2048, 130), (3, 8192, 50), (4, 8192, 50)])
+def test_decode_inside_the_dot_and_ahead_of_it(ops, Q, d, R):
+    from bsipytorch_amd import _lib
+
+    gen = torch.Generator(device="cuda").manual_seed(Q + d)
+    x = torch.randn(Q, d, generator=gen, device="cuda").relu()
+    keys = ops.build_bsi_keys_cuda(torch.randn(R, d, generator=gen, device="cuda") * 0.02, 2, 0.5)[0]
+    h = ops.build_bsi_queries_cuda_batch_hybrid(x, 2, 0.5)
+    planes, layout = keys.words, keys.layout
+    assert layout == _lib.LAYOUT_TILED16
+    scales = h.chunk_scales if h.chunk_scales is not None else h.row_scales
+    stride = scales.shape[1] if h.chunk_scales is not None else 1
+    need, got = int(_lib.lib.bsi_hip_dot_ewah_batch_workspace_bytes(Q, h.W)), []
+    for size in (0, need):
+        ws = torch.empty(max(size, 16), dtype=torch.uint8, device="cuda")
+        out = torch.full((Q, R), float("nan"), device="cuda")
+        rc = _lib.lib.bsi_hip_dot_ewah_batch(h.comp_words.data_ptr(), h.comp_off.data_ptr(), h.comp_len.data_ptr(), h.Sa, h.W, scales.data_ptr(),
+                                             stride, planes.data_ptr(), layout, keys.slice_weights.data_ptr(), 6, R, Q, float(np.float32(1e-4)),
+                                             R, None, out.data_ptr(), None, ws.data_ptr() if size else None, size,
+                                             torch.cuda.current_stream().cuda_stream)
+        assert rc == 0
+        got.append(out.cpu())
+    assert torch.equal(got[0], got[1])
+    assert torch.equal(got[0], ops.batch_dot_product_multiquery_cuda_batch_caps(h, keys)[0].cpu())
