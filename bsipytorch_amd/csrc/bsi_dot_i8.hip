@@ -351,16 +351,21 @@ __device__ __forceinline__ void i8_kstep(const v4i (&ka)[WM], const v4i (&qb)[WN
 // query ln of each) stored in whole 128-byte lines.  Stored as it lies, a store instruction writes 64 bytes per query
 // (4 lanes x 16 bytes): half a line.  Here neighbouring query lanes first swap one of two vertically adjacent tiles
 // (a, a + 1), so that the even lane holds keys 0 .. 15 of both queries and the odd lane keys 16 .. 31; a store then
-// writes, for one query of the pair, 8 lanes x 16 bytes = the 32 consecutive keys of a line.  Only for a tile that
-// lies wholly inside the output and whose lines are aligned; returns false (nothing stored) otherwise.  stream_out: nontemporal stores.
+// writes, for one query of the pair, 8 lanes x 16 bytes = the 32 consecutive keys of a line.  Queries past the last are left out;
+// false (nothing stored) where the wave's keys do not all lie inside.  An output whose rows do not begin at lines takes the
+// same stores (16 bytes at any multiple of 4, which global memory takes; plain ones, since two of them share a line).
+// stream_out: nontemporal stores.
+// An output of 4801 keys was stored a float a lane before.  us, before and now: 2000 x 1600 x 4801 as a dot 41.6, 27.0, as a layer 48.1,
+// 33.1 (4800 keys: 31.7), 512 x 1601 x 4801 17.9, 14.2; 1000 x 1024 x 2046 12.7, 10.7; f16 (i8_store_half) 2000 x 1600 x 4801 46.8, 41.0,
+// 1000 x 1024 x 2050 14.3, 11.0.  What is left over is stored an output at a time, without the 16-byte form it had for aligned
+// places: with that in the kernel the others are 1.5 % slower (2048 x 768 x 3072 17.6, 17.9).
 template <int WM, int WN>
 __device__ __forceinline__ bool i8_store_lines(const float (&v)[WM][WN][4], float* __restrict__ out, int64_t R_total,
                                                int64_t rw, int64_t qw, int64_t R, int64_t Q, int ln, int lg,
                                                bool stream_out) {
     static_assert(WM % 2 == 0, "tiles are paired along the keys");
-    const bool whole = rw + WM * 16 <= R && qw + WN * 16 <= Q && (R_total & 31) == 0 && (rw & 31) == 0 &&
-                       (reinterpret_cast<uintptr_t>(out) & 127) == 0;
-    if (!whole) return false;
+    if (rw + WM * 16 > R) return false;
+    if ((R_total & 31) != 0 || (reinterpret_cast<uintptr_t>(out) & 127) != 0) stream_out = false;
     const bool odd = (ln & 1) != 0;
 #pragma unroll
     for (int a = 0; a < WM; a += 2)
@@ -379,11 +384,12 @@ __device__ __forceinline__ bool i8_store_lines(const float (&v)[WM][WN][4], floa
             float* dst = out + static_cast<size_t>(qe) * R_total + rw + a * 16 + (odd ? 16 : 0) + lg * 4;
             if (stream_out) {  // the output leaves the caches as it is written
                 typedef float v4f __attribute__((ext_vector_type(4)));
-                __builtin_nontemporal_store((v4f){x[0], x[1], x[2], x[3]}, reinterpret_cast<v4f*>(dst));
-                __builtin_nontemporal_store((v4f){y[0], y[1], y[2], y[3]}, reinterpret_cast<v4f*>(dst + R_total));
+                if (qe < Q) __builtin_nontemporal_store((v4f){x[0], x[1], x[2], x[3]}, reinterpret_cast<v4f*>(dst));
+                if (qe + 1 < Q) __builtin_nontemporal_store((v4f){y[0], y[1], y[2], y[3]}, reinterpret_cast<v4f*>(dst + R_total));
             } else {
-                *reinterpret_cast<float4*>(dst) = make_float4(x[0], x[1], x[2], x[3]);
-                *reinterpret_cast<float4*>(dst + R_total) = make_float4(y[0], y[1], y[2], y[3]);
+                typedef float v4f __attribute__((ext_vector_type(4), aligned(4)));
+                if (qe < Q) *reinterpret_cast<v4f*>(dst) = (v4f){x[0], x[1], x[2], x[3]};
+                if (qe + 1 < Q) *reinterpret_cast<v4f*>(dst + R_total) = (v4f){y[0], y[1], y[2], y[3]};
             }
         }
     return true;
@@ -402,8 +408,7 @@ __device__ __forceinline__ void i8_store_half(const float (&v)[WM][WN][4], const
                                               float* __restrict__ out, int64_t R_total, int64_t rw, int64_t qw, int64_t R,
                                               int64_t Q, int ln, int lg) {
     unsigned short* const out16 = reinterpret_cast<unsigned short*>(out);
-    const bool whole = rw + WM * 16 <= R && qw + WN * 16 <= Q && (R_total & 7) == 0 && (reinterpret_cast<uintptr_t>(out) & 15) == 0;
-    if (whole) {
+    if (rw + WM * 16 <= R) {
         const auto store = [&](auto type, auto biased) {
             constexpr int kType = decltype(type)::value;
             constexpr bool kBias = decltype(biased)::value;
@@ -425,8 +430,10 @@ __device__ __forceinline__ void i8_store_half(const float (&v)[WM][WN][4], const
                     const auto lo = __builtin_amdgcn_permlane16_swap(p[0][0], p[1][0], false, false);
                     const auto hi = __builtin_amdgcn_permlane16_swap(p[0][1], p[1][1], false, false);
                     const int64_t q = qw + b * 16 + ln;
-                    *reinterpret_cast<uint4*>(out16 + static_cast<size_t>(q) * R_total + rw + (a + (lg & 1)) * 16 + (lg >> 1) * 8) =
-                        make_uint4(lo[0], hi[0], lo[1], hi[1]);
+                    typedef uint32_t v4u __attribute__((ext_vector_type(4), aligned(2)));
+                    if (q < Q)
+                        *reinterpret_cast<v4u*>(out16 + static_cast<size_t>(q) * R_total + rw + (a + (lg & 1)) * 16 + (lg >> 1) * 8) =
+                            (v4u){lo[0], hi[0], lo[1], hi[1]};
                 }
         };
         const auto of_type = [&](auto type) {
@@ -497,13 +504,9 @@ __device__ __forceinline__ void i8_store_tile(const float (&accf)[WM][WN][4], co
                 const int64_t q = qw + b * 16 + ln;
                 if (q >= Q) continue;
                 float* dst = out + static_cast<size_t>(q) * R_total + rb;
-                if (rb + 3 < R && ((reinterpret_cast<uintptr_t>(dst) & 15) == 0)) {
-                    *reinterpret_cast<float4*>(dst) = make_float4(v[a][b][0], v[a][b][1], v[a][b][2], v[a][b][3]);
-                } else {
 #pragma unroll
-                    for (int e = 0; e < 4; ++e)
-                        if (rb + e < R) dst[e] = v[a][b][e];
-                }
+                for (int e = 0; e < 4; ++e)
+                    if (rb + e < R) dst[e] = v[a][b][e];
             }
         }
     }
