@@ -2008,14 +2008,23 @@ thread_local size_t g_warm_bytes = 0;
 // nontemporal stores: the dirty lines then do not wait in the L2s for the write-back at the kernel's end (1.2 us less
 // for the 16 MiB of Q512 R8192).  Measured both ways: streamed layer outputs cost an OPT-1.3B-shaped prefill 2 %
 // (4.89 -> 5.00 ms replayed), plain dot outputs cost the standalone dot 8 %.  BSI_OPT_OUTPUT_STORES overrides.
+// A layer's outputs are streamed as well from 80 MiB of float32 on, in rows of 2048 elements and more: that is more than the L2s hold
+// (32 MiB) whoever reads them next, and on their way through the caches they push out keys that other tiles still need.  us a layer, and
+// with torch.relu of its output behind it, plain and streamed: 2048 x 4096 x 11008 148, 113 and 176, 175; 2300 x 4096 x 11008 136, 126 and
+// 167, 167; 4096 x 4096 x 16384 279, 268 and 359, 351 -- fewer outputs, and what the layer gains the next kernel loses: 1600 x 4096 x 11008
+// (70 MB) 117, 92 and 136, 140; 4096 x 4096 x 4096 (67 MB) 95.6, 87.5 and 111, 113; shorter rows, whose tiles wait for their stores: 4096 x
+// 256 x 5376 24.6, 26.0; 4096 x 512 x 8192 40.0, 40.2; 3000 x 512 x 16384 51.8, 52.0.
+// Half-precision outputs have plain stores only: no difference up to 134 MB.
 thread_local int t_layer_output = 0;
 thread_local const CoopBuild* t_coop = nullptr;
 thread_local int t_out_dtype = BSI_DTYPE_F32;
 std::atomic<int> g_output_stores{0};  // 0 = by entry point, 1 = always plain, 2 = always nontemporal
-static int stream_output() {
+constexpr int64_t kStreamedOutputs = 20 << 20;  // float32 outputs of a layer
+constexpr int kStreamedChunks = 8;
+static int stream_output(int64_t R_total, int64_t Q, int chunks) {
     const int forced = g_output_stores.load(std::memory_order_relaxed);
     if (forced != 0) return forced == 2 ? 1 : 0;
-    return t_layer_output ? 0 : 1;
+    return t_layer_output && (R_total * Q < kStreamedOutputs || chunks < kStreamedChunks) ? 0 : 1;
 }
 
 constexpr int kCus = 256;
@@ -2054,7 +2063,7 @@ static void launch_mfma_i8_tm(const int8_t* A8, const float* qscale, int stride,
             lds_opt_in(once, reinterpret_cast<const void*>(&dot_mfma_i8_tiles_kernel<TM, TN, kHalf, false>), I8TilesCfg<TM, TN>::kLdsTiles);
             launch((dot_mfma_i8_tiles_kernel<TM, TN, kHalf, false>), dim3(kCus), dim3(C::kBlock), I8TilesCfg<TM, TN>::kLdsTiles, st, A8, qscale, stride,
                    K8, Bw, Sb, chunks, R, Q, down_shift, scale_inv, R_total, out, bias, key_tiled,
-                   static_cast<const unsigned char*>(g_warm_ptr), static_cast<long long>(g_warm_bytes / 128), stream_output(), g,
+                   static_cast<const unsigned char*>(g_warm_ptr), static_cast<long long>(g_warm_bytes / 128), stream_output(R_total, Q, chunks), g,
                    static_cast<unsigned>(tiles), t_out_dtype, 0);
             return;
         }
@@ -2068,7 +2077,7 @@ static void launch_mfma_i8_tm(const int8_t* A8, const float* qscale, int stride,
                 lds_opt_in(once, reinterpret_cast<const void*>(&dot_mfma_i8_kernel<TM, TN, kI8Chain, false, kBuild, false, kHalf>), C::kLds);
                 launch((dot_mfma_i8_kernel<TM, TN, kI8Chain, false, kBuild, false, kHalf>), grid, dim3(C::kBlock), C::kLds, st, A8, qscale, stride, K8, Bw,
                        Sb, chunks, R, Q, down_shift, scale_inv, R_total, out, chunk_ints, bias, ndig, dig_stride, key_indices, key_tiled,
-                       static_cast<const unsigned char*>(g_warm_ptr), static_cast<long long>(g_warm_bytes / 128), stream_output(),
+                       static_cast<const unsigned char*>(g_warm_ptr), static_cast<long long>(g_warm_bytes / 128), stream_output(R_total, Q, chunks),
                        static_cast<float*>(nullptr), static_cast<unsigned*>(nullptr), 0.0f, 0, g, t_out_dtype, coop);
             };
             if (coop.row_per_wave) go(std::integral_constant<int, 2>{});
@@ -2080,7 +2089,7 @@ static void launch_mfma_i8_tm(const int8_t* A8, const float* qscale, int stride,
     launch((dot_mfma_i8_kernel<TM, TN, kMode, false, 0, kFour, kHalf>), grid, dim3(C::kBlock), C::kLds, st, A8, qscale, stride, K8,
                        Bw, Sb, chunks, R, Q, down_shift, scale_inv, R_total, out, chunk_ints, bias, ndig, dig_stride,
                        key_indices, key_tiled, static_cast<const unsigned char*>(g_warm_ptr),
-                       static_cast<long long>(g_warm_bytes / 128), stream_output(), static_cast<float*>(nullptr),
+                       static_cast<long long>(g_warm_bytes / 128), stream_output(R_total, Q, chunks), static_cast<float*>(nullptr),
                        static_cast<unsigned*>(nullptr), 0.0f, 0, g, t_out_dtype, CoopBuild{});
 }
 
@@ -2105,7 +2114,7 @@ static void launch_mfma_i8_split(int segments, unsigned char* scratch, const int
                        stride, K8, Bw, Sb, chunks, R, Q, down_shift, scale_inv, R_total, out, static_cast<int*>(nullptr), bias,
                        1, 0LL, static_cast<const long long*>(nullptr), key_tiled,
                        static_cast<const unsigned char*>(g_warm_ptr), static_cast<long long>(g_warm_bytes / 128),
-                       stream_output(), reinterpret_cast<float*>(scratch + kSplitCounterBytes),
+                       stream_output(R_total, Q, chunks), reinterpret_cast<float*>(scratch + kSplitCounterBytes),
                        reinterpret_cast<unsigned*>(scratch), limit, split_shape, I8Grid{}, t_out_dtype, CoopBuild{});
 }
 
@@ -2150,11 +2159,11 @@ static void launch_mfma_i8w(const int8_t* A8, const float* qscale, int stride, c
     if (chunk_ints)
         launch((dot_mfma_i8w_kernel<WN, true>), grid, dim3(W::kBlock), C::kLds, st, A8, qscale, stride, K8, Bw, Sb,
                            chunks, R, Q, down_shift, scale_inv, R_total, out, chunk_ints, bias, key_tiled, warm, warm_lines,
-                           stream_output(), t_out_dtype);
+                           stream_output(R_total, Q, chunks), t_out_dtype);
     else
         launch((dot_mfma_i8w_kernel<WN, false>), grid, dim3(W::kBlock), C::kLds, st, A8, qscale, stride, K8, Bw, Sb,
                            chunks, R, Q, down_shift, scale_inv, R_total, out, chunk_ints, bias, key_tiled, warm, warm_lines,
-                           stream_output(), t_out_dtype);
+                           stream_output(R_total, Q, chunks), t_out_dtype);
 }
 
 // The large layers' launches: the images in units, the bands, the integer sums, and the chain for what they leave.  The rule, in us: a round of
@@ -2259,14 +2268,14 @@ static void launch_i8_large_t(const LargeWorkspace& w, bool units_there, const i
     launch((dot_mfma_i8_large_kernel<kHalf>), dim3(static_cast<unsigned>(g.tiles_x) * static_cast<unsigned>(g.tiles_y)), dim3(512), kLargeLds, st,
            reinterpret_cast<const int8_t*>(w.lo), reinterpret_cast<const int8_t*>(w.hi), reinterpret_cast<const unsigned long long*>(w.bands),
            static_cast<const unsigned*>(w.uppers), large_cost(Q, R, chunks), w.units, K8, Bw, Sb, chunks, R, Q, scale_inv, R_total, out, bias, warm,
-           warm_lines, stream_output(), g, t_out_dtype, w.left);
+           warm_lines, stream_output(R_total, Q, chunks), g, t_out_dtype, w.left);
     dim3 grid;
     const I8Grid tiles = i8_grid((R + 127) / 128, (Q + 127) / 128, &grid);
     using T = I8TilesCfg<128, 128>;
     lds_opt_in(once_left, reinterpret_cast<const void*>(&dot_mfma_i8_tiles_kernel<128, 128, kHalf, true>), T::kLdsTiles);
     const int64_t left_tiles = static_cast<int64_t>(tiles.tiles_x) * tiles.tiles_y;  // of all bands; a workgroup without a tile ends before its first load
     launch((dot_mfma_i8_tiles_kernel<128, 128, kHalf, true>), dim3(static_cast<unsigned>(left_tiles < kCus ? left_tiles : kCus)), dim3(T::kBlock), T::kLdsTiles, st, A8, qscale, stride, K8, Bw, Sb, chunks,
-           R, Q, 16 - Sa - Sb, scale_inv, R_total, out, bias, 0, warm, warm_lines, stream_output(), tiles,
+           R, Q, 16 - Sa - Sb, scale_inv, R_total, out, bias, 0, warm, warm_lines, stream_output(R_total, Q, chunks), tiles,
            static_cast<unsigned>(left_tiles), t_out_dtype, w.left);
 }
 void launch_i8_large(void* workspace, bool units_there, const int8_t* A8, const float* qscale, int stride, const int8_t* K8, const float* Bw, int Sa, int Sb,

@@ -239,7 +239,8 @@ int bsi_hip_planes_to_int8_tiled(const uint64_t* words_device, int64_t rows, int
 #define BSI_OPT_OUTPUT_STORES 4 /* how the int8-image kernels store whole output tiles: 1 = plain stores (the output stays
                                    in the caches for the next kernel), 2 = nontemporal stores (it leaves them as it is
                                    written); 0 (default) = plain from the linear-layer entry points (bsi_hip_dot_bias,
-                                   bsi_hip_dot_bias_warm, bsi_hip_linear), nontemporal from the other dot entry points */
+                                   bsi_hip_dot_bias_warm, bsi_hip_linear) below 80 MiB of outputs or 2048 elements a row,
+                                   nontemporal from there on and from the other dot entry points */
 #define BSI_OPT_I8_SPLIT 5 /* D-split of the int8-image dot (see bsi_hip_dot_attach_split_scratch): 1 = never, n >= 2 = n
                               segments (on the tile BSI_OPT_I8_TILE forces, 128 or 12864; 128 otherwise) whenever the
                               attached scratch holds them; 0 (default) = chosen per call by a cost model */

@@ -42,3 +42,24 @@ def test_rows_that_begin_anywhere(ops, dtype, tile, Q, R, stride, offset):
     assert torch.equal(rows[:, :R].contiguous().view(BITS[dtype]), want.contiguous().view(BITS[dtype]))
     assert not torch.isnan(want).any()
     assert torch.isnan(buf[:offset]).all() and torch.isnan(rows[:, R:]).all() and torch.isnan(buf[offset + Q * stride:]).all()
+
+
+@pytest.mark.parametrize("Q,d,R", [(1281, 2048, 16384), (2561, 2000, 8192), (5130, 2048, 4100)])
+def test_large_float32_outputs_streamed(ops, Q, d, R):
+    """80 MiB of outputs and 2048 elements a row: the stores' kind changes, not what they write."""
+    from bsipytorch_amd import _lib
+    from bsipytorch_amd.linear import BSIQuantizedLinear
+
+    gen = torch.Generator(device="cuda").manual_seed(R)
+    x = torch.randn(Q, d, generator=gen, device="cuda")
+    dense = torch.nn.Linear(d, R, device="cuda")
+    layer = BSIQuantizedLinear(dense, 2, 0.5)
+    got = []
+    try:
+        for kind in (0, 1, 2):
+            assert _lib.lib.bsi_hip_set_option(4, kind) == 0
+            with torch.no_grad():
+                got.append(layer(x.clone()))
+    finally:
+        _lib.lib.bsi_hip_set_option(4, 0)
+    assert torch.equal(got[0], got[1]) and torch.equal(got[0], got[2])
