@@ -59,6 +59,18 @@ struct CoopBuild {
     int patience;               // ticks until a workgroup builds what it waits for
 };
 
+// Workgroups of a launch whose dot has `groups`: a few tiles leave most CUs idle, and their few workgroups would build round after
+// round, so there are as many as a build of one round has shares of waves (row scales: of rows), one for each CU at most.  The
+// kernels tell those without a tile by themselves.  33 x 768 x 768 is 12 tiles and 99 items: 9.7 us in two launches, 6.4 in one.
+// Not for fewer than kCoopMinKeys keys: those are fed what wider layers beside them are fed, and take over its build, which a build
+// inside the launch is not (18 x 512 x 64 behind a layer of the same tensor: one launch either way).
+constexpr int kCoopMinKeys = 256;
+inline unsigned coop_groups(unsigned groups, int64_t keys, const CoopBuild& b, int waves) {
+    if (keys < kCoopMinKeys) return groups;
+    const int pieces = b.by_row ? b.rows : b.rows * b.chunks, a_share = b.by_row && !b.row_per_wave ? 1 : waves;
+    const int shares = (pieces + a_share - 1) / a_share < kCoopShares ? (pieces + a_share - 1) / a_share : kCoopShares;
+    return groups < static_cast<unsigned>(shares * kXcds) ? static_cast<unsigned>(shares * kXcds) : groups;
+}
 // Shares of a copy for a grid of `groups` workgroups, which go to the XCDs in turn.
 inline int coop_shares(unsigned groups, int pieces) {
     int shares = static_cast<int>(groups / kXcds);
@@ -218,7 +230,7 @@ __device__ void coop_build_share(const CoopBuild& b, int share, int wave, int nw
 
 // Called by all waves of the workgroup (number `id` of the grid); 32 words of LDS at `shared`.  On return A8 and qscale point
 // to the whole build, in the copy of the XCD the workgroup runs on.  ahead(): loads for after the build, of anything but the
-// area.  Every wave but wave 0 issues them when the workgroup's share is built (a CU's loads return in order: not before),
+// area, inside for any id.  Every wave but wave 0 issues them when the workgroup's share is built (a CU's loads return in order: not before),
 // wave 0, which asks for the flags, when all shares are.
 template <bool kFragments, bool kRowPerWave, typename F>
 __device__ __forceinline__ void coop_build(const CoopBuild& b, unsigned id, unsigned* __restrict__ shared, const int8_t*& A8,

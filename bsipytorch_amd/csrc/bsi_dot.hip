@@ -427,39 +427,51 @@ static int coop_plan(int64_t Q, int64_t d, int64_t R, int decimal_places, int fi
     }
     // Chunks that a wave of the build takes one after the other, each a load's latency: up to two chunk-scaled ones or one
     // of a row (which has barriers besides) cost less than a launch.  us a pass, two launches and one: 16 x 512 x 1280 6.6, 4.8;
-    // 15 x 2560 x 5888 8.4, 7.3; 28 x 3072 x 4864 11.5, 10.6; 49 x 512 x 3328 6.9, 5.7; 121 x 512 x 14848 8.8, 8.1 -- beyond:
-    // 80 x 2304 x 4352 (4 rounds) 8.5, 8.9; 24 x 2304 x 256 7.4, 13.9.
+    // 15 x 2560 x 5888 8.4, 7.3; 28 x 3072 x 4864 11.5, 10.6; 49 x 512 x 3328 6.9, 5.7; 121 x 512 x 14848 8.8, 8.1.
     const bool by_row = ((d + 63) / 64) % 4 != 0;
-    const int shares = coop_shares(groups, static_cast<int>(by_row ? Q : Q * chunks));
+    CoopBuild b{};
+    b.rows = static_cast<int>(Q);
+    b.chunks = static_cast<int>(chunks);
+    b.by_row = by_row ? 1 : 0;
+    const int pieces = static_cast<int>(by_row ? Q : Q * chunks);
     if (by_row) {
-        if (Q <= shares && chunks <= waves) return 1;
+        if (Q <= coop_shares(coop_groups(groups, R, b, waves), pieces) && chunks <= waves) return 1;
+        b.row_per_wave = 1;
+        const int shares = coop_shares(coop_groups(groups, R, b, waves), pieces);
         // A wave a row, for more rows: one load's latency too, but longer work and copies.  us, two launches (on a host that issues
         // them in 8.4, and on one that takes 9.8) and one: 24 x 704 x 704 8.4, 9.5, 6.6; 24 x 1600 x 1600 8.1, 9.5, 6.6; 100 x 320 x
         // 2000 8.5, 9.8, 6.8; 37 x 704 x 9728 8.5, 9.9, 7.0; 250 x 100 x 8192 8.7, 10.1, 7.6; 64 x 1600 x 4800 8.4, 9.8, 8.3; 77 x 1600 x
         // 4800 8.7, 9.9, 8.8 -- beyond: 121 x 1600 x 6400 (847 items) 8.9, 9.8, 9.7; 128 x 832 x 12000 (376 workgroups, whose registers
-        // leave a CU one of them) 9.3, 9.9, 9.7.  More rows than waves, where few workgroups have few shares: 60 x 704 x 1024 (1.9 rounds) 8.5,
-        // 9.6, 7.3; 250 x 320 x 1024 8.5, 9.9, 6.9; 90 x 900 x 1000 8.5, 9.9, 8.1; 200 x 448 x 700 (2.8) 8.5, 10.0, 8.2; 150 x 192 x 768 8.5,
-        // 9.8, 7.0 -- beyond: 60 x 896 x 768 (2.5) 8.5, 9.8, 8.3; 50 x 640 x 640 (3.1) 8.5, 9.9, 8.7; 128 x 832 x 640 8.5, 9.8, 9.3.
-        // The edge at 560 items, us in two launches on three hosts and in one: 539 items (77 x 1600 x 4800) 7.6, 8.8, 9.2, 8.2; 560 (70 x 1984 x
-        // 4000) -, 9.2, 10.0, 8.6; beyond: 588 (84 x 1600 x 4800) 7.6, 8.7, 9.0, 8.2; 600 (150 x 960 x 4000) 7.1, 8.7, 9.0, 8.1; 630 (90 x 1600 x
-        // 4800) 7.7, 8.7, 8.7, 8.4; 660 (220 x 704 x 6000) 9.2, -, 9.7, 10.0; 720 (120 x 1472 x 4096) 7.3, 8.6, 8.9, 8.2; 720 (90 x 1984 x 5000)
-        // 8.2, -, 8.8, 9.1; 728 (104 x 1600 x 4800) 8.1, 8.9, 9.1, 9.6; 784 (112 x 1600 x 4800) 8.1, -, 9.2, 9.6; 900 (300 x 576 x 2048) 7.1, -,
-        // 8.9, 8.5.  One launch is bound by the GPU, two by the host: up to some 600 items it gains on most hosts and loses at most half a
-        // microsecond on the fastest; from 730 on it loses on all.  Rows beyond 512: 500 x 192 x 2000 -, 9.0, 9.4, 7.9, but 550 x
-        // 192 x 2000 -, 9.2, 9.3, 10.0 and 560 x 100 x 2000 -, 9.3, 9.5, 9.7.
+        // leave a CU one of them) 9.3, 9.9, 9.7.  Few tiles, with workgroups for the build beside them (-, the second host, one): 40 x 320 x 320
+        // 9.7, 6.5; 200 x 704 x 704 9.4, 6.5; 500 x 320 x 320 9.6, 7.1; 128 x 1600 x 512 (896 items) 9.5, 8.0; 300 x 704 x 704 (900) 9.5, 7.0.
+        // The edge at 560 items for more than 1024 keys, us in two launches on three hosts and in one: 539 items (77 x 1600 x 4800) 7.6, 8.8, 9.2,
+        // 8.2; 560 (70 x 1984 x 4000) -, 9.2, 10.0, 8.6; beyond: 588 (84 x 1600 x 4800) 7.6, 8.7, 9.0, 8.2; 600 (150 x 960 x 4000) 7.1, 8.7, 9.0,
+        // 8.1; 630 (90 x 1600 x 4800) 7.7, 8.7, 8.7, 8.4; 660 (220 x 704 x 6000) 9.2, -, 9.7, 10.0; 720 (120 x 1472 x 4096) 7.3, 8.6, 8.9, 8.2; 720
+        // (90 x 1984 x 5000) 8.2, -, 8.8, 9.1; 728 (104 x 1600 x 4800) 8.1, 8.9, 9.1, 9.6; 784 (112 x 1600 x 4800) 8.1, -, 9.2, 9.6; 900 (300 x
+        // 576 x 2048) 7.1, -, 8.9, 8.5.  One launch is bound by the GPU, two by the host: up to some 600 items it gains on most hosts and loses
+        // at most half a microsecond on the fastest; from 730 on it loses on all.  Rows beyond 512: 500 x 192 x 2000 -, 9.0, 9.4, 7.9,
+        // but 550 x 192 x 2000 -, 9.2, 9.3, 10.0 and 560 x 100 x 2000 -, 9.3, 9.5, 9.7.
         const int rounds = chunks <= 2 ? 3 : (chunks <= 4 ? 2 : 1);
-        return Q <= 512 && Q <= rounds * static_cast<int64_t>(shares) * waves && chunks <= kCoopHeld && d % 4 == 0 && Q * chunks <= 560 && groups <= 256 ? 2 : 0;
+        return Q <= 512 && Q <= rounds * static_cast<int64_t>(shares) * waves && chunks <= kCoopHeld && d % 4 == 0 &&
+                       Q * chunks <= (R <= 1024 ? 1000 : 560) && groups <= 256
+                   ? 2 : 0;
     }
-    const int64_t items = Q * chunks, a_round = static_cast<int64_t>(shares) * waves;
-    if (items <= 2 * a_round) return 1;
-    // More rounds where few workgroups have few shares: the launch takes some 4.6 us, 0.45 a round and, for more than 32 rows, 0.4 a
-    // chunk (each a step of the dot).  us, two launches (on a host that issues them in 8.4, and on one that takes 9.9) and one: 33 x
-    // 1024 x 2048 (2.1 rounds) 8.6, 9.9, 6.6; 48 x 768 x 2048 8.4, 9.9, 6.2; 150 x 512 x 1536 (2.5) 8.5, 9.9, 6.2; 100 x 1024 x 3072 8.5,
-    // 10.0, 7.3; 120 x 512 x 1024 (3.8) 8.5, 9.9, 7.1; 128 x 1024 x 2048 (4) 8.3, 10.0, 7.9; 30 x 2048 x 1024 (3.8) 8.0, 9.2, 7.5 -- beyond:
-    // 36 x 2048 x 3072 (3) 8.3, 9.9, 8.8; 64 x 2048 x 4096 (4) 8.3, 9.7, 9.4; 48 x 1536 x 2048 (4.5) 8.3, 9.8, 8.8; 25 x 3072 x 1024
-    // (3.1) 7.9, 9.2, 8.2; 20 x 4096 x 1024 (2.5) 7.8, 9.1, 8.8; 250 x 1024 x 4096 (1000 items) 8.3, 8.5, 9.3.
-    if (items > 4 * a_round || items > 512) return 0;
-    return b_layout == BSI_LAYOUT_TILED16 ? (chunks <= 8 ? 1 : 0) : (9 * items + 8 * chunks * a_round <= 76 * a_round ? 1 : 0);
+    const int64_t items = Q * chunks, a_round = static_cast<int64_t>(coop_shares(coop_groups(groups, R, b, waves), pieces)) * waves;
+    if (b_layout == BSI_LAYOUT_TILED16) {
+        // us, two launches and one, with workgroups for the build where the tiles are few: 24 x 2304 x 256 9.3, 6.7; 32 x 2048 x 1024 9.1, 6.1;
+        // 24 x 4096 x 512 9.0, 7.7; 32 x 4096 x 512 9.2, 7.8.
+        return items <= 2 * a_round || (items <= 4 * a_round && items <= 512 && chunks <= 8) ? 1 : 0;
+    }
+    if (items <= 2 * static_cast<int64_t>(coop_shares(groups, pieces)) * waves) return 1;
+    // More rounds: the launch takes some 3.75 us, 0.755 a round, 0.32 a chunk (each a step of the dot) and 1.9 for a million outputs, half a
+    // microsecond more or less (35 sizes of 33 to 512 rows); two launches 8.3 on a host that issues them fast and 9.6 on others.  us, two launches
+    // there and one: 33 x 256 x 256 9.6, 6.1; 33 x 768 x 768 9.7, 6.4; 100 x 768 x 768 9.6, 6.5; 256 x 768 x 768 9.7, 7.2; 333 x 512 x 512 9.7, 6.9;
+    // 512 x 512 x 512 9.6, 7.8; 64 x 1536 x 1536 9.3, 6.8; 128 x 1536 x 1536 9.4, 8.0; 48 x 2048 x 2048 9.4, 8.1; 256 x 1024 x 1024 9.6, 8.2; 256 x
+    // 768 x 3072 9.4, 8.0 -- beyond: 100 x 2048 x 2048 9.4, 9.5; 128 x 2048 x 2048 9.4, 10.0; 48 x 4096 x 1024 9.9, 11.5; 256 x 1024 x 4096 9.5, 9.7; 512 x
+    // 512 x 4096 9.7, 9.7; 333 x 768 x 3072 9.6, 9.3.
+    const double us = 0.755 * static_cast<double>(items) / static_cast<double>(a_round) + 0.32 * static_cast<double>(chunks) +
+                      1.9e-6 * static_cast<double>(Q) * static_cast<double>(R);
+    return groups <= 256 && us <= 4.4 ? 1 : 0;
 }
 
 extern "C" int bsi_hip_linear_coop_serves(int64_t Q, int64_t d, int64_t R, int decimal_places, int fixed_bits, int b_layout, int Sb) {

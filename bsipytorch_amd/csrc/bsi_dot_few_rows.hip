@@ -84,6 +84,8 @@ __global__ __launch_bounds__(1024) void dot_mfma_stream_kernel(
                 kc[k][j] = make_uint2(static_cast<uint32_t>(w), static_cast<uint32_t>(w >> 32));
             }
     };
+    // Workgroups beyond the tiles, there for the build (coop_groups), go on with the last tile and store nothing: a branch past the rest
+    // costs the others 0.2 us (16 x 4096 x 4096 7.8 -> 8.0).
     if constexpr (kBuild)
         coop_build<true, kBuild == 2>(coop, blockIdx.x, reinterpret_cast<unsigned*>(ints), A8, qscale, [&] { load_keys(wave < pass_chunks ? wave : pass_chunks - 1); });
 
@@ -594,7 +596,7 @@ static void launch_mfma_stream(const int8_t* A8, const float* qscale, int stride
                                int chunks, int64_t R, int64_t Q, int down_shift, float scale_inv, int64_t R_total,
                                float* out, int32_t* chunk_ints, const float* bias, hipStream_t st) {
     constexpr int kSlot = KT * NT * 256;
-    const dim3 grid(stream_groups(R, KT), static_cast<unsigned>((Q + 16 * NT - 1) / (16 * NT)));
+    dim3 grid(stream_groups(R, KT), static_cast<unsigned>((Q + 16 * NT - 1) / (16 * NT)));
     const int waves = stream_waves(grid.x * grid.y, chunks, kSlot);
     constexpr int kChunkBytes = (kSlot + NT * 16) * 4;
     const size_t turn = kSlot < 512 && t_coop == nullptr ? static_cast<size_t>(waves) * 2048 : 0;
@@ -616,6 +618,7 @@ static void launch_mfma_stream(const int8_t* A8, const float* qscale, int stride
     else if (t_coop == nullptr) BSI_STREAM_GO(false, 0, 0);
     else {
         CoopBuild coop = *t_coop;
+        grid.x = coop_groups(grid.x, R, coop, waves);
         coop.shares = coop_shares(grid.x, coop.by_row ? coop.rows : coop.rows * coop.chunks);
         if (coop.row_per_wave) BSI_STREAM_GO(false, 2, coop);
         else BSI_STREAM_GO(false, 1, coop);

@@ -582,7 +582,20 @@ __global__ __launch_bounds__((I8Cfg<TM, TN>::kBlock)) void dot_mfma_i8_kernel(
     constexpr int WM = C::kWM, WN = C::kWN;
     constexpr bool kInts = (kMode == kI8Ints), kSum = (kMode == kI8Sum);
     extern __shared__ __attribute__((aligned(16))) unsigned char lds[];  // C::kLds
-    if constexpr (kBuild != 0) coop_build<false, kBuild == 2>(coop, blockIdx.y * gridDim.x + blockIdx.x, reinterpret_cast<unsigned*>(lds), A8, qscale, [] {});
+    // Which tile, and the first loads' arguments, worked out ahead of the build and held over it: behind it each would be a fetch that all waves
+    // wait for.  us, fetched with a branch for workgroups without a tile, and held: 128 x 1024 x 4096 7.5, 7.2; 64 x 960 x 4000 6.8, 6.5.
+    [[maybe_unused]] int built_x = static_cast<int>(blockIdx.x), built_y = static_cast<int>(blockIdx.y);
+    if constexpr (kBuild != 0) {
+        if (plain_grid.height != 0) {
+            const int tiles = plain_grid.tiles_x * plain_grid.tiles_y;
+            if (built_x < tiles) i8_tile_of(plain_grid, blockIdx.x, built_x, built_y);
+            else built_y = plain_grid.tiles_y;
+        }
+        if (built_y >= plain_grid.tiles_y) built_y = -1;
+        asm volatile("" : "+s"(built_x), "+s"(built_y), "+s"(K8), "+s"(chunks), "+s"(Q), "+s"(R));
+        coop_build<false, kBuild == 2>(coop, blockIdx.y * gridDim.x + blockIdx.x, reinterpret_cast<unsigned*>(lds), A8, qscale, [] {});
+        if (built_y < 0) return;  // there for the build (coop_groups)
+    }
 
     const int tid = threadIdx.x;
     const int lane = tid & 63;
@@ -601,7 +614,8 @@ __global__ __launch_bounds__((I8Cfg<TM, TN>::kBlock)) void dot_mfma_i8_kernel(
         seg = id / (tiles_x * tiles_y);
     } else {
         bx = static_cast<int>(blockIdx.x), by = static_cast<int>(blockIdx.y);
-        if (plain_grid.height != 0) i8_tile_of(plain_grid, blockIdx.x, bx, by);
+        if constexpr (kBuild != 0) bx = built_x, by = built_y;
+        else if (plain_grid.height != 0) i8_tile_of(plain_grid, blockIdx.x, bx, by);
     }
     const int64_t r0 = static_cast<int64_t>(bx) * TM;
     const int64_t q0 = static_cast<int64_t>(by) * TN;
@@ -2070,7 +2084,10 @@ static void launch_mfma_i8_tm(const int8_t* A8, const float* qscale, int stride,
     if constexpr (kMode == kI8Chain)
         if (t_coop != nullptr) {
             CoopBuild coop = *t_coop;
-            coop.shares = coop_shares(grid.x * grid.y, coop.by_row ? coop.rows : coop.rows * coop.chunks);
+            const unsigned all = coop_groups(grid.x * grid.y, R, coop, C::kBlock / 64);
+            if (g.height != 0) grid.x = all;
+            else grid.y = (all + grid.x - 1) / grid.x;
+            coop.shares = coop_shares(all, coop.by_row ? coop.rows : coop.rows * coop.chunks);
             const auto go = [&](auto build) {
                 constexpr int kBuild = decltype(build)::value;
                 static LdsOptIn once;
