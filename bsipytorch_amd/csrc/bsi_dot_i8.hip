@@ -351,20 +351,21 @@ __device__ __forceinline__ void i8_kstep(const v4i (&ka)[WM], const v4i (&qb)[WN
 // query ln of each) stored in whole 128-byte lines.  Stored as it lies, a store instruction writes 64 bytes per query
 // (4 lanes x 16 bytes): half a line.  Here neighbouring query lanes first swap one of two vertically adjacent tiles
 // (a, a + 1), so that the even lane holds keys 0 .. 15 of both queries and the odd lane keys 16 .. 31; a store then
-// writes, for one query of the pair, 8 lanes x 16 bytes = the 32 consecutive keys of a line.  Queries past the last are left out;
-// false (nothing stored) where the wave's keys do not all lie inside.  An output whose rows do not begin at lines takes the
+// writes, for one query of the pair, 8 lanes x 16 bytes = the 32 consecutive keys of a line.  Queries and keys past the last
+// are left out.  An output whose rows do not begin at lines takes the
 // same stores (16 bytes at any multiple of 4, which global memory takes; plain ones, since two of them share a line).
 // stream_out: nontemporal stores.
 // An output of 4801 keys was stored a float a lane before.  us, before and now: 2000 x 1600 x 4801 as a dot 41.6, 27.0, as a layer 48.1,
 // 33.1 (4800 keys: 31.7), 512 x 1601 x 4801 17.9, 14.2; 1000 x 1024 x 2046 12.7, 10.7; f16 (i8_store_half) 2000 x 1600 x 4801 46.8, 41.0,
-// 1000 x 1024 x 2050 14.3, 11.0.  What is left over is stored an output at a time, without the 16-byte form it had for aligned
-// places: with that in the kernel the others are 1.5 % slower (2048 x 768 x 3072 17.6, 17.9).
+// 1000 x 1024 x 2050 14.3, 11.0.  The wave that has the last keys stores an output at a time, from the same registers: a second
+// way to them in a kernel, or a second copy of the stores without their masks, costs the others 1 to 4 % (us: 2048 x 768 x 3072 17.9 for 17.6,
+// 512 x 256 x 4096 bf16 in one launch 7.3 for 7.0).
 template <int WM, int WN>
-__device__ __forceinline__ bool i8_store_lines(const float (&v)[WM][WN][4], float* __restrict__ out, int64_t R_total,
+__device__ __forceinline__ void i8_store_lines(const float (&v)[WM][WN][4], float* __restrict__ out, int64_t R_total,
                                                int64_t rw, int64_t qw, int64_t R, int64_t Q, int ln, int lg,
                                                bool stream_out) {
     static_assert(WM % 2 == 0, "tiles are paired along the keys");
-    if (rw + WM * 16 > R) return false;
+    const bool inside = rw + WM * 16 <= R;
     if ((R_total & 31) != 0 || (reinterpret_cast<uintptr_t>(out) & 127) != 0) stream_out = false;
     const bool odd = (ln & 1) != 0;
 #pragma unroll
@@ -382,17 +383,25 @@ __device__ __forceinline__ bool i8_store_lines(const float (&v)[WM][WN][4], floa
             }
             const int64_t qe = qw + b * 16 + (ln & ~1);
             float* dst = out + static_cast<size_t>(qe) * R_total + rw + a * 16 + (odd ? 16 : 0) + lg * 4;
-            if (stream_out) {  // the output leaves the caches as it is written
-                typedef float v4f __attribute__((ext_vector_type(4)));
-                if (qe < Q) __builtin_nontemporal_store((v4f){x[0], x[1], x[2], x[3]}, reinterpret_cast<v4f*>(dst));
-                if (qe + 1 < Q) __builtin_nontemporal_store((v4f){y[0], y[1], y[2], y[3]}, reinterpret_cast<v4f*>(dst + R_total));
+            typedef float v4f __attribute__((ext_vector_type(4), aligned(4)));
+            if (inside) {
+                if (stream_out) {  // the output leaves the caches as it is written
+                    typedef float v4f_aligned __attribute__((ext_vector_type(4)));
+                    if (qe < Q) __builtin_nontemporal_store((v4f_aligned){x[0], x[1], x[2], x[3]}, reinterpret_cast<v4f_aligned*>(dst));
+                    if (qe + 1 < Q) __builtin_nontemporal_store((v4f_aligned){y[0], y[1], y[2], y[3]}, reinterpret_cast<v4f_aligned*>(dst + R_total));
+                } else {
+                    if (qe < Q) *reinterpret_cast<v4f*>(dst) = (v4f){x[0], x[1], x[2], x[3]};
+                    if (qe + 1 < Q) *reinterpret_cast<v4f*>(dst + R_total) = (v4f){y[0], y[1], y[2], y[3]};
+                }
             } else {
-                typedef float v4f __attribute__((ext_vector_type(4), aligned(4)));
-                if (qe < Q) *reinterpret_cast<v4f*>(dst) = (v4f){x[0], x[1], x[2], x[3]};
-                if (qe + 1 < Q) *reinterpret_cast<v4f*>(dst + R_total) = (v4f){y[0], y[1], y[2], y[3]};
+                const int64_t keys = R - (rw + a * 16 + (odd ? 16 : 0) + lg * 4);  // from the lane's first on
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    if (qe < Q && e < keys) dst[e] = x[e];
+                    if (qe + 1 < Q && e < keys) dst[R_total + e] = y[e];
+                }
             }
         }
-    return true;
 }
 
 // The same output tile in a half-precision type (v before the bias; `bi` the biases of the lane's rows).  The lane's four
@@ -408,54 +417,46 @@ __device__ __forceinline__ void i8_store_half(const float (&v)[WM][WN][4], const
                                               float* __restrict__ out, int64_t R_total, int64_t rw, int64_t qw, int64_t R,
                                               int64_t Q, int ln, int lg) {
     unsigned short* const out16 = reinterpret_cast<unsigned short*>(out);
-    if (rw + WM * 16 <= R) {
-        const auto store = [&](auto type, auto biased) {
-            constexpr int kType = decltype(type)::value;
-            constexpr bool kBias = decltype(biased)::value;
-            float rounded[WM][4];
+    const bool inside = rw + WM * 16 <= R;
+    const auto store = [&](auto type, auto biased) {
+        constexpr int kType = decltype(type)::value;
+        constexpr bool kBias = decltype(biased)::value;
+        float rounded[WM][4];
 #pragma unroll
-            for (int a = 0; a < WM; ++a)
+        for (int a = 0; a < WM; ++a)
 #pragma unroll
-                for (int e = 0; e < 4; ++e) rounded[a][e] = kBias ? half_value(half_bits(bi[a][e], kType), kType) : 0.0f;
+            for (int e = 0; e < 4; ++e) rounded[a][e] = kBias ? half_value(half_bits(bi[a][e], kType), kType) : 0.0f;
 #pragma unroll
-            for (int a = 0; a < WM; a += 2)
+        for (int a = 0; a < WM; a += 2)
 #pragma unroll
-                for (int b = 0; b < WN; ++b) {
-                    uint32_t p[2][2];
+            for (int b = 0; b < WN; ++b) {
+                uint32_t p[2][2];
 #pragma unroll
-                    for (int t = 0; t < 2; ++t)
+                for (int t = 0; t < 2; ++t)
 #pragma unroll
-                        for (int h = 0; h < 2; ++h)
-                            p[t][h] = half_pair<kType, kBias>(v[a + t][b][2 * h], v[a + t][b][2 * h + 1], rounded[a + t][2 * h], rounded[a + t][2 * h + 1]);
-                    const auto lo = __builtin_amdgcn_permlane16_swap(p[0][0], p[1][0], false, false);
-                    const auto hi = __builtin_amdgcn_permlane16_swap(p[0][1], p[1][1], false, false);
-                    const int64_t q = qw + b * 16 + ln;
-                    typedef uint32_t v4u __attribute__((ext_vector_type(4), aligned(2)));
-                    if (q < Q)
-                        *reinterpret_cast<v4u*>(out16 + static_cast<size_t>(q) * R_total + rw + (a + (lg & 1)) * 16 + (lg >> 1) * 8) =
-                            (v4u){lo[0], hi[0], lo[1], hi[1]};
+                    for (int h = 0; h < 2; ++h)
+                        p[t][h] = half_pair<kType, kBias>(v[a + t][b][2 * h], v[a + t][b][2 * h + 1], rounded[a + t][2 * h], rounded[a + t][2 * h + 1]);
+                const auto lo = __builtin_amdgcn_permlane16_swap(p[0][0], p[1][0], false, false);
+                const auto hi = __builtin_amdgcn_permlane16_swap(p[0][1], p[1][1], false, false);
+                const int64_t q = qw + b * 16 + ln, first = rw + (a + (lg & 1)) * 16 + (lg >> 1) * 8;
+                typedef uint32_t v4u __attribute__((ext_vector_type(4), aligned(2)));
+                const v4u eight = {lo[0], hi[0], lo[1], hi[1]};
+                unsigned short* const dst = out16 + static_cast<size_t>(q) * R_total + first;
+                if (inside) {
+                    if (q < Q) *reinterpret_cast<v4u*>(dst) = eight;
+                } else {
+#pragma unroll
+                    for (int e = 0; e < 8; ++e)
+                        if (q < Q && first + e < R) dst[e] = static_cast<unsigned short>(eight[e >> 1] >> (16 * (e & 1)));
                 }
-        };
-        const auto of_type = [&](auto type) {
-            if (has_bias) store(type, std::true_type{});
-            else store(type, std::false_type{});
-        };
-        if (dtype == BSI_DTYPE_F16) of_type(std::integral_constant<int, BSI_DTYPE_F16>{});
-        else of_type(std::integral_constant<int, BSI_DTYPE_BF16>{});
-        return;
-    }
-#pragma unroll
-    for (int a = 0; a < WM; ++a)
-#pragma unroll
-        for (int b = 0; b < WN; ++b) {
-            const int64_t rb = rw + a * 16 + lg * 4, q = qw + b * 16 + ln;
-            if (q >= Q) continue;
-#pragma unroll
-            for (int e = 0; e < 4; ++e)
-                if (rb + e < R)
-                    out16[static_cast<size_t>(q) * R_total + rb + e] =
-                        static_cast<unsigned short>(half_output(v[a][b][e], has_bias, bi[a][e], dtype));
-        }
+            }
+    };
+    const auto of_type = [&](auto type) {
+        if (has_bias) store(type, std::true_type{});
+        else store(type, std::false_type{});
+    };
+    if (dtype == BSI_DTYPE_F16) of_type(std::integral_constant<int, BSI_DTYPE_F16>{});
+    else of_type(std::integral_constant<int, BSI_DTYPE_BF16>{});
 }
 
 // The end of a tile in the chain modes: every output takes its key's factor, the decimal scale and the bias, and is stored.
@@ -495,20 +496,7 @@ __device__ __forceinline__ void i8_store_tile(const float (&accf)[WM][WN][4], co
             i8_store_half<2, WN>(v, bi, has_bias, out_dtype, out, R_total, rw, qw, R, Q, ln, lg);
             continue;
         }
-        if (i8_store_lines<2, WN>(v, out, R_total, rw, qw, R, Q, ln, lg, stream_out)) continue;
-#pragma unroll
-        for (int a = 0; a < 2; ++a) {
-            const int64_t rb = rw + a * 16 + lg * 4;
-#pragma unroll
-            for (int b = 0; b < WN; ++b) {
-                const int64_t q = qw + b * 16 + ln;
-                if (q >= Q) continue;
-                float* dst = out + static_cast<size_t>(q) * R_total + rb;
-#pragma unroll
-                for (int e = 0; e < 4; ++e)
-                    if (rb + e < R) dst[e] = v[a][b][e];
-            }
-        }
+        i8_store_lines<2, WN>(v, out, R_total, rw, qw, R, Q, ln, lg, stream_out);
     }
 }
 
@@ -913,24 +901,7 @@ __global__ __launch_bounds__((I8Cfg<TM, TN>::kBlock)) void dot_mfma_i8_kernel(
                         if (bias != nullptr) v = v + biv[a][e];
                         accf[a][b][e] = v;
                     }
-            if (i8_store_lines<WM, WN>(accf, out, R_total, r0 + wr * (WM * 16), q0 + wq * (WN * 16), R, Q, ln, lg, out_stream != 0)) return;
-#pragma unroll
-            for (int a = 0; a < WM; ++a) {
-                const int64_t rb = r0 + wr * (WM * 16) + a * 16 + lg * 4;
-#pragma unroll
-                for (int b = 0; b < WN; ++b) {
-                    const int64_t q = q0 + wq * (WN * 16) + b * 16 + ln;
-                    if (q >= Q) continue;
-                    float* dst = out + static_cast<size_t>(q) * R_total + rb;
-                    if (rb + 3 < R && ((reinterpret_cast<uintptr_t>(dst) & 15) == 0)) {
-                        *reinterpret_cast<float4*>(dst) = make_float4(accf[a][b][0], accf[a][b][1], accf[a][b][2], accf[a][b][3]);
-                    } else {
-#pragma unroll
-                        for (int e = 0; e < 4; ++e)
-                            if (rb + e < R) dst[e] = accf[a][b][e];
-                    }
-                }
-            }
+            i8_store_lines<WM, WN>(accf, out, R_total, r0 + wr * (WM * 16), q0 + wq * (WN * 16), R, Q, ln, lg, out_stream != 0);
             return;
         }
 #pragma unroll
@@ -1971,24 +1942,7 @@ __global__ __launch_bounds__((I8WCfg<WN>::kBlock)) void dot_mfma_i8w_kernel(
         i8_store_half<4, WN>(accf, bi, bias != nullptr, out_dtype, out, R_total, r0 + wr * 64, q0 + wq * (16 * WN), R, Q, ln, lg);
         return;
     }
-    if (i8_store_lines<4, WN>(accf, out, R_total, r0 + wr * 64, q0 + wq * (16 * WN), R, Q, ln, lg, out_stream != 0)) return;
-#pragma unroll
-    for (int a = 0; a < 4; ++a) {
-        const int64_t rb = r0 + wr * 64 + a * 16 + lg * 4;
-#pragma unroll
-        for (int b = 0; b < WN; ++b) {
-            const int64_t q = q0 + wq * (16 * WN) + b * 16 + ln;
-            if (q >= Q) continue;
-            float* dst = out + static_cast<size_t>(q) * R_total + rb;
-            if (rb + 3 < R && ((reinterpret_cast<uintptr_t>(dst) & 15) == 0)) {
-                *reinterpret_cast<float4*>(dst) = make_float4(accf[a][b][0], accf[a][b][1], accf[a][b][2], accf[a][b][3]);
-            } else {
-#pragma unroll
-                for (int e = 0; e < 4; ++e)
-                    if (rb + e < R) dst[e] = accf[a][b][e];
-            }
-        }
-    }
+    i8_store_lines<4, WN>(accf, out, R_total, r0 + wr * 64, q0 + wq * (16 * WN), R, Q, ln, lg, out_stream != 0);
 }
 
 // out[q, idx[r]] = float(sum_{i,j} I[i Q + q, j R + r] * 2^(7 (i + j) - preshift) * Aw[q, 0] * Bw[r, 0]) * scale_inv
