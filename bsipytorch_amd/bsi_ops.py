@@ -1577,7 +1577,7 @@ def debug_quantize_int64_cpu(values: torch.Tensor, decimal_places: int) -> torch
 
 # The native host path reads these on every call, so what the functions above keep stays the one copy.
 _native.bind({name: ctypes.cast(getattr(lib, name), ctypes.c_void_p).value
-              for name in ("bsi_hip_linear_few_rows_out", "bsi_hip_linear_out", "bsi_hip_linear_workspace_bytes_for", "bsi_hip_dot",
+              for name in ("bsi_hip_linear_few_rows_out", "bsi_hip_linear_few_rows_shares", "bsi_hip_linear_out", "bsi_hip_linear_workspace_bytes_for", "bsi_hip_dot",
                            "bsi_hip_build_fixed", "bsi_hip_build_fixed_keys", "bsi_hip_ewah_measure", "bsi_hip_ewah_emit", "bsi_hip_dot_ewah_batch",
                            "bsi_hip_dot_ewah_batch_workspace_bytes", "bsi_hip_scalar_query_dot",
                            "bsi_hip_build_measure_rows", "bsi_hip_ewah_emit_at", "bsi_hip_linear_coop_out",

@@ -710,6 +710,17 @@ extern "C" int bsi_hip_linear_few_rows_upfront(int64_t Q, int64_t d, int64_t R) 
     return p.per_wave <= p.upfront ? 1 : 0;
 }
 
+// A build that every workgroup repeats costs a round of loads for each item a wave has beyond those up front; the one that an XCD's
+// workgroups share costs a wait.  us, each (rows x width x keys): 4 x 8192 x 8192 20.0, 11.9; 4 x 5120 x 5120 13.5, 8.7; 4 x 4096 x 11008 14.5,
+// 11.7; 3 x 4096 x 5120 9.6, 8.1; 3 x 4096 x 11008 12.2, 11.7; 2 x 8192 x 8192 14.6, 11.9; 2 x 5120 x 5120 9.5, 8.7; with two key tiles a
+// workgroup 2 x 4096 x 16384 12.9, 11.8; 3 x 2304 x 16384 9.9, 8.9 -- where the loads hide it, or one more: 4 x 4096 x 4096 6.8, 7.4; 2 x
+// 4096 x 11008 10.2, 11.5; 1 x 8192 x 8192 11.2, 11.8; 2 x 2304 x 16384 8.5, 8.8.
+extern "C" int bsi_hip_linear_few_rows_shares(int64_t Q, int64_t d, int64_t R) {
+    if (Q < 1 || Q > kFusedMaxQ || d < 1 || R < 1) return 0;
+    const FusedPlan p = fused_plan(Q, static_cast<int>((d + 255) / 256), R);
+    return p.per_wave > p.upfront + (p.key_tiles == 2 ? 1 : 0) ? 1 : 0;
+}
+
 static int linear_few_rows(const void* x, int dtype, int64_t Q, int64_t d, int decimal_places, int fixed_bits,
                            const uint64_t* B_tiled, const float* Bw, int Sb, int64_t R, float scale_inv, int64_t R_total,
                            const float* bias, float* out, void* stream) {

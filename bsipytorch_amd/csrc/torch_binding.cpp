@@ -28,6 +28,7 @@ namespace {
 // Entry points of the library the Python side has loaded (bind()).
 struct Library {
     decltype(&bsi_hip_linear_few_rows_out) linear_few_rows_out;
+    decltype(&bsi_hip_linear_few_rows_shares) linear_few_rows_shares;
     decltype(&bsi_hip_linear_out) linear_out;
     decltype(&bsi_hip_linear_workspace_bytes_for) linear_workspace_bytes_for;
     decltype(&bsi_hip_dot) dot;
@@ -372,7 +373,8 @@ PyObject* linear(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     PyObject* slot = nullptr;
     void* ws = nullptr;
     int64_t ws_bytes = 0;
-    const at::Tensor coop = !few && k.Sb <= 8 && lib.linear_coop_serves(rows, d, k.R, static_cast<int>(decimals), config.bits, k.operand_layout, static_cast<int>(k.Sb))
+    const bool own_build = few && lib.linear_few_rows_shares(rows, d, k.R) == 0;
+    const at::Tensor coop = !own_build && k.Sb <= 8 && lib.linear_coop_serves(rows, d, k.R, static_cast<int>(decimals), config.bits, k.operand_layout, static_cast<int>(k.Sb))
                            ? coop_area(device, st) : at::Tensor();
     if (few) {
         if (!known_few_rows(device.index(), rows, d)) Py_RETURN_NONE;
@@ -412,7 +414,7 @@ PyObject* linear(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
                                  k.operand.as<uint64_t>(), k.operand_layout, k.weights.as<float>(), static_cast<int>(k.Sb),
                                  k.R, inv, k.R, bias.as<float>(), out.data_ptr(), in_code, warm, warm_bytes, st);
         if (rc != BSI_OK) return fail_status(rc, "bsi_hip_linear_coop_out");
-        count(layer, names.build_calls, 1);
+        if (!few) count(layer, names.build_calls, 1);
     } else if (few) {
         Py_BEGIN_ALLOW_THREADS
         rc = lib.linear_few_rows_out(xp, in_code, rows, d, static_cast<int>(decimals), config.bits,
@@ -878,7 +880,8 @@ PyObject* bind(PyObject*, PyObject* args) {
     int few, stream, split;
     long long lds;
     if (!PyArg_ParseTuple(args, "O!O!iiiL", &PyDict_Type, &entries, &PyDict_Type, &state, &few, &stream, &split, &lds)) return nullptr;
-    if (!entry(entries, "bsi_hip_linear_few_rows_out", &lib.linear_few_rows_out) || !entry(entries, "bsi_hip_linear_out", &lib.linear_out) ||
+    if (!entry(entries, "bsi_hip_linear_few_rows_out", &lib.linear_few_rows_out) ||
+        !entry(entries, "bsi_hip_linear_few_rows_shares", &lib.linear_few_rows_shares) || !entry(entries, "bsi_hip_linear_out", &lib.linear_out) ||
         !entry(entries, "bsi_hip_linear_workspace_bytes_for", &lib.linear_workspace_bytes_for) || !entry(entries, "bsi_hip_dot", &lib.dot) ||
         !entry(entries, "bsi_hip_build_fixed", &lib.build_fixed) ||
         !entry(entries, "bsi_hip_build_fixed_keys", &lib.build_fixed_keys) || !entry(entries, "bsi_hip_ewah_measure", &lib.ewah_measure) ||

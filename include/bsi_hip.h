@@ -406,6 +406,8 @@ int bsi_hip_linear_coop_out(const void* x_device, int dtype, int64_t Q, int64_t 
  * behind the key traffic (then the one launch still saves host time, but build + dot is the faster pair on the
  * GPU).  A host-side query: no GPU work.  No counterpart in the reference. */
 int bsi_hip_linear_few_rows_upfront(int64_t Q, int64_t d, int64_t R);
+/* 1 where the build takes the kernel so many rounds that bsi_hip_linear_coop_out, whose workgroups share it, costs less. */
+int bsi_hip_linear_few_rows_shares(int64_t Q, int64_t d, int64_t R);
 
 /* The same dot for ONE query whose slices are EWAH streams (the hybrid query form of
  * build_bsi_query_cuda_hybrid, bsi_cuda.cpp:386-431): stream s at comp_words + comp_off[s], comp_len[s]
