@@ -4,6 +4,7 @@
 #include "bsi_quant_device.h"
 
 #include <chrono>
+#include <cstring>
 
 namespace bsi {
 
@@ -17,7 +18,7 @@ __device__ __forceinline__ void store_host(unsigned long long* p, unsigned long 
     __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
-// out[r] = sum_{i,j,w} popcount(A[i, w] & B[r, j, w]) * Aw[i] * Bw[r, j], exact in float64 while below 2^53, where A are the
+// out[r] = sum_{i,j,w} popcount(A[i, w] & B[r, j, w]) * Aw[i] * Bw[r, j] / divisor, the sum exact in float64 while below 2^53, where A are the
 // planes of the decimal build of x (round half away from zero of x * 10^dec, the slice count from the largest magnitude).
 // host: {slices, whether a value is negative, words of the stored form, run-length coded slices}, three clock values of
 // kScalarStamps workgroups (begin, query built, end), then the R scores: pinned memory, each word stored once, so that the
@@ -33,7 +34,7 @@ __device__ __forceinline__ void store_host(unsigned long long* p, unsigned long 
 template <int kWords>
 __global__ __launch_bounds__(kScalarBlock) void scalar_query_dot_kernel(const float* __restrict__ x, int d, int W, double dec_scale,
                                                                         int narrow, double threshold, const unsigned long long* __restrict__ B,
-                                                                        const float* __restrict__ Bw, int Sb, int R,
+                                                                        const float* __restrict__ Bw, int Sb, int R, double divisor,
                                                                         unsigned long long* __restrict__ host) {
     extern __shared__ __attribute__((aligned(16))) unsigned long long As[];  // [64 slices][W], then x in whole chunks
     constexpr int kRows = kScalarWaves, kParts = BSI_WAVE / kWords;
@@ -202,7 +203,7 @@ __global__ __launch_bounds__(kScalarBlock) void scalar_query_dot_kernel(const fl
             for (int off = BSI_WAVE / 2; off > 0; off >>= 1) acc += __shfl_xor(acc, off, BSI_WAVE);
             if (lane == 0) scores[wave] = acc;
             __syncthreads();
-            if (tid < kRows && rb + tid < R) store_host(out + rb + tid, static_cast<unsigned long long>(__double_as_longlong(scores[tid])));
+            if (tid < kRows && rb + tid < R) store_host(out + rb + tid, static_cast<unsigned long long>(__double_as_longlong(scores[tid] / divisor)));
             __syncthreads();
         }
     }
@@ -257,7 +258,7 @@ extern "C" int bsi_hip_scalar_query_dot(const float* x, int64_t d, int decimal_p
         lds_opt_in(once, reinterpret_cast<const void*>(&scalar_query_dot_kernel<L>), kScalarMaxElems * 12);                       \
         launch(scalar_query_dot_kernel<L>, dim3(static_cast<unsigned>(groups)), dim3(kScalarBlock), static_cast<size_t>(W) * 512 + static_cast<size_t>((W + 3) / 4) * 1024, \
                st, x, static_cast<int>(d), W, dec_scale, narrow, threshold,                   \
-               reinterpret_cast<const unsigned long long*>(B), Bw, Sb, static_cast<int>(R),                                \
+               reinterpret_cast<const unsigned long long*>(B), Bw, Sb, static_cast<int>(R), divisor,                       \
                reinterpret_cast<unsigned long long*>(pinned));                                                             \
     }
     if (W > 32) BSI_SCALAR_DOT(64)
@@ -268,16 +269,25 @@ extern "C" int bsi_hip_scalar_query_dot(const float* x, int64_t d, int decimal_p
     // The words come while the kernel still runs; the stream is waited for only if they are long in coming.
     const auto until = std::chrono::steady_clock::now() + std::chrono::microseconds(500);
     bool waited = false;
-    auto word = [&](int64_t i) {
-        while (host[i] == kScalarPending && !waited) {
+    auto word = [&](int64_t i, unsigned long long& v) {
+        while ((v = host[i]) == kScalarPending && !waited) {
             if (std::chrono::steady_clock::now() > until) {
                 waited = true;
-                return hipStreamSynchronize(st);
+                const hipError_t status = hipStreamSynchronize(st);
+                v = host[i];
+                return status;
             }
         }
         return hipSuccess;
     };
-    for (int64_t i = 0; i < words; ++i) BSI_HIP_CHECK(word(i));
+    // The scores go to the caller as they come, divided on the GPU: a pass of divisions behind the last of them, over lines that have been
+    // read before, was 1.5 us of a call of 1024 scores of 2048 elements (19.8, 18.3) and 4 of one of 4096 x 4096 (27.3, 23.1).
+    unsigned long long v = 0ULL;
+    for (int64_t r = 0; r < R; ++r) {
+        BSI_HIP_CHECK(word(4 + 3 * stamped + r, v));
+        std::memcpy(out + r, &v, sizeof v);
+    }
+    for (int64_t i = 0; i < 4 + 3 * stamped; ++i) BSI_HIP_CHECK(word(i, v));  // the clocks at the end come behind the scores
     const volatile unsigned long long* const stamps = host + 4;
     unsigned long long began = stamps[0], built = stamps[1], ended = stamps[2];
     for (int64_t g = 1; g < stamped; ++g) {
@@ -289,7 +299,5 @@ extern "C" int bsi_hip_scalar_query_dot(const float* x, int64_t d, int decimal_p
     *build_ns = static_cast<int64_t>(static_cast<double>(built - began) * ns);
     *dot_ns = static_cast<int64_t>(static_cast<double>(ended - built) * ns);
     for (int i = 0; i < 4; ++i) info[i] = static_cast<int64_t>(host[i]);
-    const volatile double* const scores = reinterpret_cast<const volatile double*>(host + 4 + 3 * stamped);
-    for (int64_t r = 0; r < R; ++r) out[r] = scores[r] / divisor;
     return BSI_OK;
 }
