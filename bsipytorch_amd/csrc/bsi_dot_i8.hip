@@ -357,51 +357,63 @@ __device__ __forceinline__ void i8_kstep(const v4i (&ka)[WM], const v4i (&qb)[WN
 // stream_out: nontemporal stores.
 // An output of 4801 keys was stored a float a lane before.  us, before and now: 2000 x 1600 x 4801 as a dot 41.6, 27.0, as a layer 48.1,
 // 33.1 (4800 keys: 31.7), 512 x 1601 x 4801 17.9, 14.2; 1000 x 1024 x 2046 12.7, 10.7; f16 (i8_store_half) 2000 x 1600 x 4801 46.8, 41.0,
-// 1000 x 1024 x 2050 14.3, 11.0.  The wave that has the last keys stores an output at a time, from the same registers: a second
-// way to them in a kernel, or a second copy of the stores without their masks, costs the others 1 to 4 % (us: 2048 x 768 x 3072 17.9 for 17.6,
-// 512 x 256 x 4096 bf16 in one launch 7.3 for 7.0).
+// 1000 x 1024 x 2050 14.3, 11.0.  Tiles that lie inside keep stores without masks (us, with masks in all: 4000 x 512 x 4096 25.1 for 24.2, a
+// dot of 1600 x 768 x 4096 12.1 for 11.6); the last keys are stored an output at a time, from the same registers.
 template <int WM, int WN>
 __device__ __forceinline__ void i8_store_lines(const float (&v)[WM][WN][4], float* __restrict__ out, int64_t R_total,
                                                int64_t rw, int64_t qw, int64_t R, int64_t Q, int ln, int lg,
                                                bool stream_out) {
     static_assert(WM % 2 == 0, "tiles are paired along the keys");
-    const bool inside = rw + WM * 16 <= R;
     if ((R_total & 31) != 0 || (reinterpret_cast<uintptr_t>(out) & 127) != 0) stream_out = false;
     const bool odd = (ln & 1) != 0;
+    float* const mine = out + (qw + (ln & ~1)) * R_total + rw + (odd ? 16 : 0) + lg * 4;
+    typedef float v4f __attribute__((ext_vector_type(4), aligned(4)));
+    const auto each = [&](auto put) {
 #pragma unroll
-    for (int a = 0; a < WM; a += 2)
+        for (int a = 0; a < WM; a += 2)
 #pragma unroll
-        for (int b = 0; b < WN; ++b) {
-            float x[4], y[4];
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const float give = odd ? v[a][b][e] : v[a + 1][b][e];
-                // quad_perm [1, 0, 3, 2]: the value of the neighbouring query lane
-                const float got = __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(give), 0xB1, 0xF, 0xF, false));
-                x[e] = odd ? got : v[a][b][e];       // the pair's even query: keys 16 (odd lane) + 4 lg ..
-                y[e] = odd ? v[a + 1][b][e] : got;   // the pair's odd query
-            }
-            const int64_t qe = qw + b * 16 + (ln & ~1);
-            float* dst = out + static_cast<size_t>(qe) * R_total + rw + a * 16 + (odd ? 16 : 0) + lg * 4;
-            typedef float v4f __attribute__((ext_vector_type(4), aligned(4)));
-            if (inside) {
-                if (stream_out) {  // the output leaves the caches as it is written
-                    typedef float v4f_aligned __attribute__((ext_vector_type(4)));
-                    if (qe < Q) __builtin_nontemporal_store((v4f_aligned){x[0], x[1], x[2], x[3]}, reinterpret_cast<v4f_aligned*>(dst));
-                    if (qe + 1 < Q) __builtin_nontemporal_store((v4f_aligned){y[0], y[1], y[2], y[3]}, reinterpret_cast<v4f_aligned*>(dst + R_total));
-                } else {
-                    if (qe < Q) *reinterpret_cast<v4f*>(dst) = (v4f){x[0], x[1], x[2], x[3]};
-                    if (qe + 1 < Q) *reinterpret_cast<v4f*>(dst + R_total) = (v4f){y[0], y[1], y[2], y[3]};
-                }
-            } else {
-                const int64_t keys = R - (rw + a * 16 + (odd ? 16 : 0) + lg * 4);  // from the lane's first on
+            for (int b = 0; b < WN; ++b) {
+                v4f x, y;
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
-                    if (qe < Q && e < keys) dst[e] = x[e];
-                    if (qe + 1 < Q && e < keys) dst[R_total + e] = y[e];
+                    const float give = odd ? v[a][b][e] : v[a + 1][b][e];
+                    // quad_perm [1, 0, 3, 2]: the value of the neighbouring query lane
+                    const float got = __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(give), 0xB1, 0xF, 0xF, false));
+                    x[e] = odd ? got : v[a][b][e];       // the pair's even query: keys 16 (odd lane) + 4 lg ..
+                    y[e] = odd ? v[a + 1][b][e] : got;   // the pair's odd query
                 }
+                put(mine + static_cast<int64_t>(b * 16) * R_total + a * 16, x, y, a, b);
             }
+    };
+    if (rw + WM * 16 <= R && qw + WN * 16 <= Q) {
+        if (stream_out) {  // the output leaves the caches as it is written
+            typedef float v4f_aligned __attribute__((ext_vector_type(4)));
+            each([&](float* dst, v4f x, v4f y, int, int) {
+                __builtin_nontemporal_store(static_cast<v4f_aligned>(x), reinterpret_cast<v4f_aligned*>(dst));
+                __builtin_nontemporal_store(static_cast<v4f_aligned>(y), reinterpret_cast<v4f_aligned*>(dst + R_total));
+            });
+        } else {
+            each([&](float* dst, v4f x, v4f y, int, int) {
+                *reinterpret_cast<v4f*>(dst) = x;
+                *reinterpret_cast<v4f*>(dst + R_total) = y;
+            });
         }
+        return;
+    }
+    if (qw >= Q) return;
+    each([&](float* dst, v4f x, v4f y, int a, int b) {
+        const int64_t queries = Q - (qw + b * 16 + (ln & ~1)), keys = R - (rw + a * 16 + (odd ? 16 : 0) + lg * 4);  // from the lane's first on
+        if (rw + WM * 16 <= R) {
+            if (queries > 0) *reinterpret_cast<v4f*>(dst) = x;
+            if (queries > 1) *reinterpret_cast<v4f*>(dst + R_total) = y;
+            return;
+        }
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            if (queries > 0 && e < keys) dst[e] = x[e];
+            if (queries > 1 && e < keys) dst[R_total + e] = y[e];
+        }
+    });
 }
 
 // The same output tile in a half-precision type (v before the bias; `bi` the biases of the lane's rows).  The lane's four
@@ -1207,11 +1219,9 @@ __global__ __launch_bounds__((I8Cfg<TM, TN>::kBlock)) void dot_mfma_i8_tiles_ker
             bx = static_cast<int>(id) - by * grid.tiles_x;
         }
         if constexpr (kLeft) by = left_tile(left, by);
-        // The lane's number is made anew where the compiler cannot see it, so that neither it nor an address of the stores is held over the chunk
-        // loop: there is no register for one, and fetched from scratch it is a round trip a tile (2048 x 768 x 3072 f32 17.75 us, 17.4).
-        int lane_late;
-        asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(lane_late));
-        const int ln_late = lane_late & 15, lg_late = lane_late >> 4;
+        // from values the compiler cannot see through, so that no address of the stores is held in registers over the chunk loop
+        int ln_late = ln, lg_late = lg;
+        asm volatile("" : "+v"(ln_late), "+v"(lg_late));
         i8_store_tile<TM, WM, WN, kHalf>(accf, lds + 4 * C::kStage + I8TilesCfg<TM, TN>::kScaleBytes + (tile & 3) * C::kEpilogueBytes, down, scale_inv,
                                         bias != nullptr, out_dtype, out, R_total, static_cast<int64_t>(bx) * TM,
                                         static_cast<int64_t>(by) * TN, wr, wq, R, Q, ln_late, lg_late, out_stream != 0);
