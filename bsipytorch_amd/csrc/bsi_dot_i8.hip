@@ -2272,10 +2272,16 @@ void launch_i8_large(void* workspace, bool units_there, const int8_t* A8, const 
 // leaves CUs idle that smaller tiles would use: a workgroup's time per half-chunk is about 1 : 0.63 : 0.35 : 0.31
 // for 128 x 128 : 128 x 64 : 64 x 64 : 64 x 32, so take the least (rounds of 256 workgroups x time), the larger
 // tile on a tie.  g_i8_tile forces a tile (tuning and tests).
-int choose_i8_tile(int64_t R, int64_t Q, int64_t* cost_out) {
+int choose_i8_tile(int64_t R, int64_t Q, int64_t* cost_out, int chunks) {
     const int64_t n128 = ((R + 127) / 128) * ((Q + 127) / 128);
     if (cost_out) *cost_out = ((n128 + 255) / 256) * 100;
     if (const int forced = g_i8_tile.load(std::memory_order_relaxed); forced != 0 && forced != kLargeTile) return forced;
+    // Half a round over: three rounds of 128 x 64 for two, where rows are short enough for a tile's start and stores to count (chunks: of the
+    // rows where the caller's kernel has both forms).  us a layer, 128 x 128 and 128 x 64, 512 and 1024 wide: 768 x 8192 keys bf16 14.3, 13.5
+    // and 17.7, 17.1; 1280 x 4096 f32 15.4, 14.5 and 18.9, 18.3; 3000 x 1920 bf16 15.2, 14.1 and 20.5, 18.8; 530 x 8192 f32 14.7, 13.5 and
+    // 17.3, 17.0 -- 2048 wide 768 x 8192 f32 25.2, 25.7, 1536 x 4096 bf16 26.2, 26.7; 256 wide 1280 x 4096 bf16 12.5, 11.5, but 768 x 8192 14.3, 16.1.  A
+    // dot, which streams its outputs out, from three chunks on: 640 x 1024 x 8192 14.4, 12.4; 768 x 512 x 8192 9.7, 10.2 (its caller leaves `chunks` out).
+    if (n128 > 256 && n128 <= 384 && chunks >= 2 && chunks <= 4 && ((R + 127) / 128) * ((Q + 63) / 64) <= 768) return 12864;
     if (n128 > 256) return 128;
     const int64_t cost[4] = {100, ((((R + 127) / 128) * ((Q + 63) / 64) + 255) / 256) * 63,
                              ((((R + 63) / 64) * ((Q + 63) / 64) + 255) / 256) * 35,
@@ -2382,7 +2388,7 @@ void launch_mfma_i8(const int8_t* A8, const float* qscale, int stride, const int
             return;
         }
     }
-    const int tile = choose_i8_tile(R, Q);
+    const int tile = choose_i8_tile(R, Q, nullptr, ndig == 0 && chunk_ints == nullptr && t_coop == nullptr && (t_layer_output || chunks > 2) ? chunks : 0);
     if (tile == 1284 && ndig == 0 && t_coop == nullptr) {
         launch_mfma_i8w<4>(A8, qscale, stride, K8, Bw, Sb, chunks, R, Q, down_shift, scale_inv, R_total, out, chunk_ints, bias,
                            st, key_tiled);

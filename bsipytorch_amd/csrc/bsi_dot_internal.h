@@ -33,7 +33,7 @@ extern thread_local int t_out_dtype;
 // Set by bsi_hip_linear_coop_out around its launch: the query build the kernel does itself (bsi_coop_build.h).
 struct CoopBuild;
 extern thread_local const CoopBuild* t_coop;
-int choose_i8_tile(int64_t R, int64_t Q, int64_t* cost_out = nullptr);
+int choose_i8_tile(int64_t R, int64_t Q, int64_t* cost_out = nullptr, int chunks = 0);
 // D-split of the chain-mode int8-image dot (bsi_hip_dot_attach_split_scratch): the calling thread's scratch region
 // (counters of kSplitCounterBytes, then the segments' partial sums) and the device it lies on; the option
 // BSI_OPT_I8_SPLIT; the choice itself (tile 128 / 12864 and *segments, or 0).
