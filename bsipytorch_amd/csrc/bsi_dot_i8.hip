@@ -614,8 +614,28 @@ __global__ __launch_bounds__((I8Cfg<TM, TN>::kBlock)) void dot_mfma_i8_kernel(
         seg = id / (tiles_x * tiles_y);
     } else {
         bx = static_cast<int>(blockIdx.x), by = static_cast<int>(blockIdx.y);
-        if constexpr (kBuild != 0) bx = built_x, by = built_y;
-        else if (plain_grid.height != 0) i8_tile_of(plain_grid, blockIdx.x, bx, by);
+        if constexpr (kBuild != 0) {
+            bx = built_x, by = built_y;
+        } else if (kMode == kI8Chain && TM * TN < 128 * 128 && split_shape != 0) {
+            // a part of one of the 128 x 128 tiles that are left (launch_mfma_i8_rest); a part past the last key or query does the first one's work
+            constexpr int kAcross = 128 / TM;
+            const unsigned rest = static_cast<unsigned>(split_shape) & 255u;
+            unsigned id = blockIdx.x, part = 0u;
+            while (id >= rest) id -= rest, ++part;
+            id += static_cast<unsigned>(split_shape) >> 8;
+            if (plain_grid.height != 0) {
+                i8_tile_of(plain_grid, id, bx, by);
+            } else {
+                by = static_cast<int>(id / static_cast<unsigned>(plain_grid.tiles_x));
+                bx = static_cast<int>(id) - by * plain_grid.tiles_x;
+            }
+            bx = bx * kAcross + static_cast<int>(part % kAcross);
+            by = by * (128 / TN) + static_cast<int>(part / kAcross);
+            if (static_cast<int64_t>(bx) * TM >= R) --bx;
+            if (static_cast<int64_t>(by) * TN >= Q) --by;
+        } else if (plain_grid.height != 0) {
+            i8_tile_of(plain_grid, blockIdx.x, bx, by);
+        }
     }
     const int64_t r0 = static_cast<int64_t>(bx) * TM;
     const int64_t q0 = static_cast<int64_t>(by) * TN;
@@ -2027,6 +2047,31 @@ static I8Grid i8_grid(int64_t tiles_x, int64_t tiles_y, dim3* grid) {
     return g;
 }
 
+// The last round of a grid of 128 x 128 tiles, where it would leave half of the CUs idle: its tiles as quarters or halves, a CU each, in a
+// launch of their own, which costs some 4 us and takes a round of 0.35 or 0.63.  Tiles of that launch, or 0.  us a layer in one launch and in
+// two: up to 64 tiles, 4096 wide 281 x 12483 keys bf16 38.6, 34.5; 600 x 8192 bf16 35.8, 34.3; 1100 x 4096 f32 38.6, 37.3; 8192 wide 1100 x 4096 f32
+// 69.8, 62.3; 600 x 8192 bf16 64.0, 58.5 -- 2048 wide 600 x 8192 f32 23.9, 24.8; up to 128 tiles, 8192 wide 768 x 8192 f32 82, 77; 3594 x 1536 bf16 84,
+// 79 -- 4096 wide 768 x 8192 f32 39.9, 41.7; 777 x 11008 bf16 53.9, 53.6.
+static int64_t i8_rest(int64_t tiles, int chunks) {
+    const int64_t rest = tiles % kCus;
+    if (tiles >= (1 << 22) || rest > kCus / 2) return 0;
+    return chunks >= (rest <= kCus / 4 ? 12 : 24) ? rest : 0;
+}
+template <int TM, int TN, bool kFour, bool kHalf>
+static void launch_mfma_i8_rest(int64_t first, int64_t rest, const I8Grid& g, const int8_t* A8, const float* qscale, int stride, const int8_t* K8,
+                                const float* Bw, int Sb, int chunks, int64_t R, int64_t Q, int down_shift, float scale_inv, int64_t R_total,
+                                float* out, const float* bias, hipStream_t st, int key_tiled) {
+    using C = I8Cfg<TM, TN>;
+    constexpr int kParts = 128 / TM * (128 / TN);
+    static LdsOptIn once;
+    lds_opt_in(once, reinterpret_cast<const void*>(&dot_mfma_i8_kernel<TM, TN, kI8Chain, false, 0, kFour, kHalf>), C::kLds);
+    launch((dot_mfma_i8_kernel<TM, TN, kI8Chain, false, 0, kFour, kHalf>), dim3(static_cast<unsigned>(rest * kParts)), dim3(C::kBlock), C::kLds, st, A8,
+           qscale, stride, K8, Bw, Sb, chunks, R, Q, down_shift, scale_inv, R_total, out, static_cast<int32_t*>(nullptr), bias, 0, 0LL,
+           static_cast<const long long*>(nullptr), key_tiled, static_cast<const unsigned char*>(g_warm_ptr), static_cast<long long>(g_warm_bytes / 128),
+           stream_output(R_total, Q, chunks), static_cast<float*>(nullptr), static_cast<unsigned*>(nullptr), 0.0f,
+           static_cast<int>(rest | first << 8), g, t_out_dtype, CoopBuild{});
+}
+
 template <int TM, int TN, int kMode, bool kFour, bool kHalf>
 static void launch_mfma_i8_tm(const int8_t* A8, const float* qscale, int stride, const int8_t* K8, const float* Bw,
                               int Sb, int chunks, int64_t R, int64_t Q, int down_shift, float scale_inv,
@@ -2041,10 +2086,16 @@ static void launch_mfma_i8_tm(const int8_t* A8, const float* qscale, int stride,
         if (t_coop == nullptr && tiles > kCus && tiles * chunks < (int64_t{1} << 29)) {
             static LdsOptIn once;
             lds_opt_in(once, reinterpret_cast<const void*>(&dot_mfma_i8_tiles_kernel<TM, TN, kHalf, false>), I8TilesCfg<TM, TN>::kLdsTiles);
+            const int64_t rest = TN == 128 ? i8_rest(tiles, chunks) : 0;
             launch((dot_mfma_i8_tiles_kernel<TM, TN, kHalf, false>), dim3(kCus), dim3(C::kBlock), I8TilesCfg<TM, TN>::kLdsTiles, st, A8, qscale, stride,
-                   K8, Bw, Sb, chunks, R, Q, down_shift, scale_inv, R_total, out, bias, key_tiled,
-                   static_cast<const unsigned char*>(g_warm_ptr), static_cast<long long>(g_warm_bytes / 128), stream_output(R_total, Q, chunks), g,
-                   static_cast<unsigned>(tiles), t_out_dtype, 0);
+                   K8, Bw, Sb, chunks, R, Q, down_shift, scale_inv, R_total, out, bias, key_tiled, static_cast<const unsigned char*>(g_warm_ptr),
+                   rest != 0 ? 0LL : static_cast<long long>(g_warm_bytes / 128), stream_output(R_total, Q, chunks), g, static_cast<unsigned>(tiles - rest),
+                   t_out_dtype, 0);
+            if constexpr (TN == 128) {
+                if (rest != 0)
+                    (rest <= kCus / 4 ? &launch_mfma_i8_rest<64, 64, kFour, kHalf> : &launch_mfma_i8_rest<128, 64, kFour, kHalf>)(
+                        tiles - rest, rest, g, A8, qscale, stride, K8, Bw, Sb, chunks, R, Q, down_shift, scale_inv, R_total, out, bias, st, key_tiled);
+            }
             return;
         }
     if constexpr (kMode == kI8Chain)
