@@ -544,6 +544,7 @@ __device__ __forceinline__ void narrow_grid(I8Grid& g, int tiles_y) {
     g.by_last = last == 1u ? 0u : 0xFFFFFFFFu / last + 1u;
 }
 
+constexpr int kParts = 3;
 template <int TM, int TN, int kMode, bool kSplit, int kBuild, bool kFour, bool kHalf>
 __global__ __launch_bounds__((I8Cfg<TM, TN>::kBlock)) void dot_mfma_i8_kernel(
     const int8_t* A8, const float* qscale, int qscale_stride,
@@ -554,7 +555,8 @@ __global__ __launch_bounds__((I8Cfg<TM, TN>::kBlock)) void dot_mfma_i8_kernel(
     const unsigned char* __restrict__ warm, long long warm_lines, int out_stream, float* __restrict__ split_partials,
     unsigned* __restrict__ split_counters, float split_limit, int split_shape, I8Grid plain_grid, int out_dtype, CoopBuild coop) {
     // kBuild: the queries are quantised by this launch (bsi_coop_build.h; 1: a chunk a wave at a time, 2: a row); A8 and qscale are
-    // not looked at.
+    // not looked at.  kParts (in its place, since it excludes it): the workgroups take parts of the 128 x 128 tiles that split_shape names
+    // (launch_mfma_i8_rest); instances of their own, since the others start 0.1 to 0.2 us later with it.
     // kSplit (chain mode only): a D-split launch.  gridDim.z workgroups share an output tile, each running the chain
     // over its own run of chunks from zero.  All operands of the chain are integers (times one power of two), so
     // as long as no value the chain takes exceeds 2^24 of its unit nothing is ever rounded, the value after every
@@ -585,7 +587,7 @@ __global__ __launch_bounds__((I8Cfg<TM, TN>::kBlock)) void dot_mfma_i8_kernel(
     // Which tile, and the first loads' arguments, worked out ahead of the build and held over it: behind it each would be a fetch that all waves
     // wait for.  us, fetched with a branch for workgroups without a tile, and held: 128 x 1024 x 4096 7.5, 7.2; 64 x 960 x 4000 6.8, 6.5.
     [[maybe_unused]] int built_x = static_cast<int>(blockIdx.x), built_y = static_cast<int>(blockIdx.y);
-    if constexpr (kBuild != 0) {
+    if constexpr (kBuild == 1 || kBuild == 2) {
         if (plain_grid.height != 0) {
             const int tiles = plain_grid.tiles_x * plain_grid.tiles_y;
             if (built_x < tiles) i8_tile_of(plain_grid, blockIdx.x, built_x, built_y);
@@ -614,10 +616,9 @@ __global__ __launch_bounds__((I8Cfg<TM, TN>::kBlock)) void dot_mfma_i8_kernel(
         seg = id / (tiles_x * tiles_y);
     } else {
         bx = static_cast<int>(blockIdx.x), by = static_cast<int>(blockIdx.y);
-        if constexpr (kBuild != 0) {
+        if constexpr (kBuild == 1 || kBuild == 2) {
             bx = built_x, by = built_y;
-        } else if (kMode == kI8Chain && TM * TN < 128 * 128 && split_shape != 0) {
-            // a part of one of the 128 x 128 tiles that are left (launch_mfma_i8_rest); a part past the last key or query does the first one's work
+        } else if constexpr (kBuild == kParts) {  // a part past the last key or query does the first one's work
             constexpr int kAcross = 128 / TM;
             const unsigned rest = static_cast<unsigned>(split_shape) & 255u;
             unsigned id = blockIdx.x, part = 0u;
@@ -2062,10 +2063,9 @@ static void launch_mfma_i8_rest(int64_t first, int64_t rest, const I8Grid& g, co
                                 const float* Bw, int Sb, int chunks, int64_t R, int64_t Q, int down_shift, float scale_inv, int64_t R_total,
                                 float* out, const float* bias, hipStream_t st, int key_tiled) {
     using C = I8Cfg<TM, TN>;
-    constexpr int kParts = 128 / TM * (128 / TN);
     static LdsOptIn once;
-    lds_opt_in(once, reinterpret_cast<const void*>(&dot_mfma_i8_kernel<TM, TN, kI8Chain, false, 0, kFour, kHalf>), C::kLds);
-    launch((dot_mfma_i8_kernel<TM, TN, kI8Chain, false, 0, kFour, kHalf>), dim3(static_cast<unsigned>(rest * kParts)), dim3(C::kBlock), C::kLds, st, A8,
+    lds_opt_in(once, reinterpret_cast<const void*>(&dot_mfma_i8_kernel<TM, TN, kI8Chain, false, kParts, kFour, kHalf>), C::kLds);
+    launch((dot_mfma_i8_kernel<TM, TN, kI8Chain, false, kParts, kFour, kHalf>), dim3(static_cast<unsigned>(rest * (128 / TM) * (128 / TN))), dim3(C::kBlock), C::kLds, st, A8,
            qscale, stride, K8, Bw, Sb, chunks, R, Q, down_shift, scale_inv, R_total, out, static_cast<int32_t*>(nullptr), bias, 0, 0LL,
            static_cast<const long long*>(nullptr), key_tiled, static_cast<const unsigned char*>(g_warm_ptr), static_cast<long long>(g_warm_bytes / 128),
            stream_output(R_total, Q, chunks), static_cast<float*>(nullptr), static_cast<unsigned*>(nullptr), 0.0f,
