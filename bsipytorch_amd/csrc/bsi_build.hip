@@ -504,11 +504,13 @@ __device__ __forceinline__ uint32_t shift_quad_bytes(uint32_t sm, const QuadShif
 // L2s are written back at its end.  Before (16-bit pairs in registers for up to 16 chunks, plain stores) and now, us:
 // 16384 x 4096 float32 94.9 -> 79.2 (4.9 TB/s), 8192 x 8192 119.4 -> 85.7, 4096 x 4096 22.5 -> 18.6, 768 x 768 6.7 -> 4.5;
 // bfloat16 16384 x 4096 64.2 -> 54.3, 8192 x 5120 37.4 -> 26.7, 2048 x 2048 8.4 -> 7.3.
-// kOnce: the loads are nontemporal too, for matrices that the memory-side cache does not hold, of up to 16 chunks a row (a longer
-// row takes longer that way, 4096 x 8192 bfloat16 31.4, 32.9) and whole lines (a line that two rows share is fetched twice, 12800 x
-// 1000 float32 15.8, 17.9).  us, plain and nontemporal: 16384 x 4096 float32 79.4, 75.7, bfloat16 54.3, 52.7; 11008 x 4096 float16
-// 38.9, 36.4; below the line 4096 x 4096 float32 (64 MiB) 21.1, 21.6.
-constexpr size_t kKeysOnceBytes = size_t{80} << 20;
+// kOnce: the loads are nontemporal too, for matrices that the memory-side cache does not hold, of whole lines (a line that two
+// rows share is fetched twice, 12800 x 1000 float32 15.8, 17.9).  us, plain and nontemporal: 16384 x 4096 float32 79.4, 75.7,
+// bfloat16 54.3, 52.7; 11008 x 4096 float16 38.9, 36.4; below the line 4096 x 4096 float32 (64 MiB) 21.1, 21.6.
+// Rows of 17 to 32 chunks, with four loads of a wave in flight instead of eight, pay more for a miss, and their line lies
+// higher: 8192 x 8192 float32 86.7, 78.3, bfloat16 59.9, 54.5; 13000 x 5120 float32 82.8, 78.9; of 108 MB 3295 x 8192 float32
+// 36.3, 35.3, 12408 x 4352 bfloat16 48.4, 47.8; of 100 MB 3051 x 8192 float32 34.9, 35.6; of 84 MB 8203 x 5120 bfloat16 32.0, 39.3.
+constexpr size_t kKeysOnceBytes = size_t{80} << 20, kKeysOnceLongBytes = size_t{100} << 20;
 constexpr int kKeyRows = 16, kKeyGroup = 8;
 template <typename T, bool kVec, int kHeld, int kLoads, bool kOnce>
 __global__ __launch_bounds__(kKeyRows * BSI_WAVE, 8) void build_keys_fast_kernel(
@@ -957,10 +959,11 @@ extern "C" int bsi_hip_build_fixed_keys(const void* x, int dtype, int64_t R, int
                static_cast<double>(scale_int), static_cast<float>(scale_int),                                                \
                reinterpret_cast<unsigned long long*>(tiled), image, shifts, slice_weights)))
     const size_t row_bytes = static_cast<size_t>(d) * (dtype == BSI_DTYPE_F32 ? 4 : 2);
-    const bool once = row_bytes % 128 == 0 && reinterpret_cast<uintptr_t>(x) % 128 == 0 && row_bytes * static_cast<size_t>(R) >= kKeysOnceBytes;
+    const bool once = row_bytes % 128 == 0 && reinterpret_cast<uintptr_t>(x) % 128 == 0 &&
+                      row_bytes * static_cast<size_t>(R) >= (chunks <= 16 ? kKeysOnceBytes : kKeysOnceLongBytes);
     if (chunks <= 8) { if (once) BSI_KEYS(8, 8, true) else BSI_KEYS(8, 8, false) }
     else if (chunks <= 16) { if (once) BSI_KEYS(16, 8, true) else BSI_KEYS(16, 8, false) }
-    else BSI_KEYS(32, 4, false)
+    else { if (once) BSI_KEYS(32, 4, true) else BSI_KEYS(32, 4, false) }
 #undef BSI_KEYS
     BSI_LAUNCH_CHECK("build_keys_fast_kernel");
     return BSI_OK;
