@@ -105,7 +105,7 @@ extern "C" int bsi_hip_dot_attach_split_scratch(void* scratch_device, size_t byt
 extern "C" int bsi_hip_dot_split_plan(int64_t R, int64_t Q, int W64, int* tile, int* segments) {
     BSI_REQUIRE(tile && segments && R >= 1 && Q >= 1 && W64 >= 1, "bad arguments");
     const int split_tile = choose_i8_split(R, Q, (W64 + 3) / 4, segments);
-    *tile = split_tile != 0 ? split_tile : choose_i8_tile(R, Q, nullptr, (W64 + 3) / 4);
+    *tile = split_tile != 0 ? split_tile : choose_i8_tile(R, Q, nullptr, W64 > 8 ? (W64 + 3) / 4 : 0);
     return BSI_OK;
 }
 

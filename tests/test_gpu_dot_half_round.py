@@ -9,7 +9,7 @@ from test_gpu_parity import ops  # noqa: F401  (fixture)
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("Q,d,R,tile", [(768, 512, 8192, 12864), (769, 512, 8192, 128), (1281, 1024, 2946, 12864), (530, 260, 8191, 12864), (768, 1025, 8192, 128),
+@pytest.mark.parametrize("Q,d,R,tile", [(768, 520, 8192, 12864), (769, 512, 8192, 128), (1281, 1024, 2946, 12864), (530, 600, 8191, 12864), (768, 512, 8192, 128), (768, 1025, 8192, 128),
                                         (768, 256, 8192, 128), (1024, 512, 4096, 128)])
 def test_same_bits(ops, Q, d, R, tile):
     from bsipytorch_amd import _lib
