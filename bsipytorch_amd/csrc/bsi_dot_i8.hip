@@ -135,12 +135,16 @@ __device__ unsigned long long g_timeline_cycles[kTimelineWorkgroups * 8];  // th
 #endif
 
 // A loader wave's share of a region that the next dot will read: one lane per 128-byte line, 64 lines per load.  The values
-// are summed only so that the loads stay; the store never happens.
+// are summed only so that the loads stay; the store never happens.  The lines are shared among the workgroups that come here: all of the
+// grid, or, tiles != 0, those that have a tile (number `tile` of `tiles`; the others of a launch with the build inside, coop_groups, leave
+// before).  us a layer of 400 MB of linked layers, unlinked, with the lines shared among the whole grid of such launches, and so: 64 x
+// 768 x 768 6.5, 6.7, 6.4; 128 x 768 x 768 6.9, 7.1, 6.8; 256 x 768 x 768 8.1, 8.4, 8.1; 128 x 1024 x 1024 8.1, 8.3, 7.9.
 template <int kLoaders>
 __device__ __forceinline__ void i8_warm_lines(unsigned char* __restrict__ unused_lds, int lw, int lane, const unsigned char* __restrict__ warm,
-                                              long long warm_lines) {
-    const long long waves = static_cast<long long>(gridDim.x) * gridDim.y * gridDim.z * kLoaders;
-    const long long mine = ((static_cast<long long>(blockIdx.z) * gridDim.y + blockIdx.y) * gridDim.x + blockIdx.x) * kLoaders + lw;
+                                              long long warm_lines, int tile = 0, int tiles = 0) {
+    const long long groups = tiles != 0 ? tiles : static_cast<long long>(gridDim.x) * gridDim.y * gridDim.z;
+    const long long group = tiles != 0 ? tile : (static_cast<long long>(blockIdx.z) * gridDim.y + blockIdx.y) * gridDim.x + blockIdx.x;
+    const long long waves = groups * kLoaders, mine = group * kLoaders + lw;
     const long long per = (warm_lines + waves - 1) / waves;
     const long long first = mine * per;
     const long long last = (first + per < warm_lines) ? first + per : warm_lines;
@@ -160,7 +164,7 @@ __device__ __forceinline__ void i8_loader_wave(unsigned char* __restrict__ lds, 
                                                int halves, int64_t R, int64_t Q, int64_t r0, int64_t q0, size_t rowbytes,
                                                const float* __restrict__ bias, int ndig, long long dig_stride,
                                                int key_tiled, const unsigned char* __restrict__ warm,
-                                               long long warm_lines) {
+                                               long long warm_lines, int tile = 0, int tiles = 0) {
     constexpr int TM = C::kTM, TN = C::kTN;
     constexpr int L = C::kLoaders, NI = C::kLoads, KG = TM / 8, QG = TN / 8;
     // The key groups and the query groups both divide evenly among the loader waves: every loader moves KG / L key
@@ -293,7 +297,7 @@ __device__ __forceinline__ void i8_loader_wave(unsigned char* __restrict__ lds, 
         }
         lds_barrier();
     }
-    if (warm_lines > 0) i8_warm_lines<L>(scale_lds, lw, lane, warm, warm_lines);
+    if (warm_lines > 0) i8_warm_lines<L>(scale_lds, lw, lane, warm, warm_lines, tile, tiles);
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // nothing may still be writing LDS when the workgroup ends
 }
 
@@ -653,8 +657,10 @@ __global__ __launch_bounds__((I8Cfg<TM, TN>::kBlock)) void dot_mfma_i8_kernel(
 
     if (wave >= C::kConsumers) {
         if (wave == C::kConsumers) BSI_STAMP(kStampLoaderEntry);
+        constexpr bool kHelpers = kBuild == 1 || kBuild == 2;  // workgroups beyond the tiles do not come here
         i8_loader_wave<C, kSum, kFour>(lds, wave - C::kConsumers, lane, A8, qscale, qscale_stride, K8, Bw, Sb, chunks, first_chunk,
-                                my_chunks * 2, R, Q, r0, q0, rowbytes, bias, ndig, dig_stride, key_tiled, warm, warm_lines);
+                                my_chunks * 2, R, Q, r0, q0, rowbytes, bias, ndig, dig_stride, key_tiled, warm, warm_lines,
+                                kHelpers ? by * plain_grid.tiles_x + bx : 0, kHelpers ? plain_grid.tiles_x * plain_grid.tiles_y : 0);
         if (kSplit) {
             lds_barrier();  // the MFMA waves have stored their partial sums
             lds_barrier();  // the decision is in LDS
