@@ -7,7 +7,11 @@
 // by a flag behind it.
 //
 // No workgroup depends on another one being resident.  A share's bytes do not depend on who builds it, so a workgroup that
-// has waited kCoopPatience for a share builds it itself.  Flags hold the launch's number, which no other launch has: nothing
+// has waited kCoopPatience for a share builds it itself, waits half as long for the next, and so on down to an eighth: beside kernels
+// that hold the CUs, most shares of a copy may belong to workgroups that have not begun.  Every CU of an XCD begins at another missing
+// share, and between two a workgroup looks at all flags.  us a layer beside a layer of 4096 x 4096 x 16384 on another stream (256 workgroups
+// with all LDS of a CU each), median of 36, with a whole patience for every share and the lowest one first, and so: 16 x 4096 x 4096
+// 154, 80 (whole patience, from different shares: 107); 33 x 768 x 768, 128 x 1024 x 1024, 333 x 512 x 512 40 to 50 either way.  Flags hold the launch's number, which no other launch has: nothing
 // is cleared between launches, and flags of earlier ones mean nothing.
 //
 // What a reader relies on, since neither side of a flag is more than a relaxed access (an agent-scope release writes the L2
@@ -55,7 +59,7 @@ struct CoopBuild {
     int rows, chunks, slices;
     int by_row;                 // one scale a row instead of one a chunk
     int row_per_wave;           // by_row: a wave builds a row (of kCoopHeld chunks at most) by itself: instances of their own
-    int shares;                 // of a copy: chunk scales split the items, row scales the rows
+    int shares;                 // of a copy: chunk scales split the items, row scales the rows (ahead of the launch: asked for, or 0)
     int patience;               // ticks until a workgroup builds what it waits for
 };
 
@@ -71,9 +75,10 @@ inline unsigned coop_groups(unsigned groups, int64_t keys, const CoopBuild& b, i
     const int shares = (pieces + a_share - 1) / a_share < kCoopShares ? (pieces + a_share - 1) / a_share : kCoopShares;
     return groups < static_cast<unsigned>(shares * kXcds) ? static_cast<unsigned>(shares * kXcds) : groups;
 }
-// Shares of a copy for a grid of `groups` workgroups, which go to the XCDs in turn.
-inline int coop_shares(unsigned groups, int pieces) {
-    int shares = static_cast<int>(groups / kXcds);
+// Shares of a copy for a grid of `groups` workgroups, which go to the XCDs in turn; or as many as are asked for (a test's shares
+// that no workgroup owns).
+inline int coop_shares(unsigned groups, int pieces, int asked = 0) {
+    int shares = asked > 0 ? asked : static_cast<int>(groups / kXcds);
     if (shares > kCoopShares) shares = kCoopShares;
     if (shares > pieces) shares = pieces;
     return shares < 1 ? 1 : shares;
@@ -271,6 +276,7 @@ __device__ __forceinline__ void coop_build(const CoopBuild& b, unsigned id, unsi
         ahead();
         issued = true;
     }
+    unsigned patience = static_cast<unsigned>(b.patience);
 #pragma unroll 1
     for (;;) {
         if (share >= 0) build(share);
@@ -281,7 +287,7 @@ __device__ __forceinline__ void coop_build(const CoopBuild& b, unsigned id, unsi
                 const bool here = lane >= b.shares ||
                                   __hip_atomic_load(flags + (lane < kCoopShares ? lane : 0), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == b.launch;
                 missing = __ballot(!here);
-                if (missing == 0ULL || wall_clock64() - since > static_cast<unsigned>(b.patience)) break;
+                if (missing == 0ULL || wall_clock64() - since > patience) break;
             }
             if (lane == 0) shared[0] = static_cast<unsigned>(missing);
         }
@@ -289,7 +295,10 @@ __device__ __forceinline__ void coop_build(const CoopBuild& b, unsigned id, unsi
         const unsigned missing = static_cast<unsigned>(__builtin_amdgcn_readfirstlane(static_cast<int>(shared[0])));
         lds_barrier();
         if (missing == 0u) break;
-        share = __builtin_ctz(missing);
+        // HW_ID, CU and shader engine: every CU of an XCD begins elsewhere
+        const unsigned cu = __builtin_amdgcn_s_getreg((7 << 11) | (8 << 6) | 4), from = ((cu & 7u) * 4u + (cu >> 5 & 3u)) % kCoopShares;
+        share = static_cast<int>((__builtin_ctz(__builtin_rotateright32(missing, from)) + from) % kCoopShares);
+        if (patience > kCoopPatience / 8) patience >>= 1;
     }
     if (!issued) ahead();
     asm volatile("" ::: "memory");

@@ -37,7 +37,7 @@
 #include "bsi_dot_internal.h"
 
 namespace bsi {
-static std::atomic<int> g_coop_patience{kCoopPatience};
+static std::atomic<int> g_coop_patience{kCoopPatience}, g_coop_shares{0};
 }  // namespace bsi
 
 using namespace bsi;
@@ -64,6 +64,10 @@ extern "C" int bsi_hip_set_option(int option, int value) {
         case BSI_OPT_COOP_PATIENCE:
             BSI_REQUIRE(value >= 0, "patience must not be negative");
             g_coop_patience = value;
+            return BSI_OK;
+        case BSI_OPT_COOP_SHARES:
+            BSI_REQUIRE(value >= 0 && value <= kCoopShares, "shares must be 0 (by the launch) to %d", kCoopShares);
+            g_coop_shares = value;
             return BSI_OK;
         case BSI_OPT_BUILD_ITEMS:
             BSI_REQUIRE(value == 0 || value == 1 || value == 2 || value == 4 || value == 8, "items must be 0, 1, 2, 4 or 8");
@@ -505,6 +509,7 @@ extern "C" int bsi_hip_linear_coop_out(const void* x, int dtype, int64_t Q, int6
     c.chunks = chunks;
     c.slices = fixed_bits;
     c.patience = g_coop_patience.load(std::memory_order_relaxed);
+    c.shares = g_coop_shares.load(std::memory_order_relaxed);
     c.by_row = W64 % 4 == 0 ? 0 : 1;  // the builder's rule
     c.row_per_wave = plan == 2 ? 1 : 0;
     t_coop = &c;

@@ -86,8 +86,10 @@ __global__ __launch_bounds__(1024) void dot_mfma_stream_kernel(
     };
     // Workgroups beyond the tiles, there for the build (coop_groups), go on with the last tile and store nothing: a branch past the rest
     // costs the others 0.2 us (16 x 4096 x 4096 7.8 -> 8.0).
-    if constexpr (kBuild)
+    if constexpr (kBuild) {
+        asm volatile("" : "+s"(R), "+s"(Q));  // held over the build: a fetch behind it is one that all waves wait for (12 x 4096 x 11008 12.4, 11.5 us)
         coop_build<true, kBuild == 2>(coop, blockIdx.x, reinterpret_cast<unsigned*>(ints), A8, qscale, [&] { load_keys(wave < pass_chunks ? wave : pass_chunks - 1); });
+    }
 
     // the chain lanes: tid <-> (key tile, query tile, query, key), keys fastest so output stores are contiguous
     float accf = 0.0f;
@@ -619,7 +621,7 @@ static void launch_mfma_stream(const int8_t* A8, const float* qscale, int stride
     else {
         CoopBuild coop = *t_coop;
         grid.x = coop_groups(grid.x, R, coop, waves);
-        coop.shares = coop_shares(grid.x, coop.by_row ? coop.rows : coop.rows * coop.chunks);
+        coop.shares = coop_shares(grid.x, coop.by_row ? coop.rows : coop.rows * coop.chunks, coop.shares);
         if (coop.row_per_wave) BSI_STREAM_GO(false, 2, coop);
         else BSI_STREAM_GO(false, 1, coop);
     }

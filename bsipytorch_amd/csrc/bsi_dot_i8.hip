@@ -2110,7 +2110,7 @@ static void launch_mfma_i8_tm(const int8_t* A8, const float* qscale, int stride,
             const unsigned all = coop_groups(grid.x * grid.y, R, coop, C::kBlock / 64);
             if (g.height != 0) grid.x = all;
             else grid.y = (all + grid.x - 1) / grid.x;
-            coop.shares = coop_shares(all, coop.by_row ? coop.rows : coop.rows * coop.chunks);
+            coop.shares = coop_shares(all, coop.by_row ? coop.rows : coop.rows * coop.chunks, coop.shares);
             const auto go = [&](auto build) {
                 constexpr int kBuild = decltype(build)::value;
                 static LdsOptIn once;
