@@ -468,11 +468,15 @@ static int coop_plan(int64_t Q, int64_t d, int64_t R, int decimal_places, int fi
     }
     if (items <= 2 * static_cast<int64_t>(coop_shares(groups, pieces)) * waves) return 1;
     // More rounds: the launch takes some 3.75 us, 0.755 a round, 0.32 a chunk (each a step of the dot) and 1.9 for a million outputs, half a
-    // microsecond more or less (35 sizes of 33 to 512 rows); two launches 8.3 on a host that issues them fast and 9.6 on others.  us, two launches
-    // there and one: 33 x 256 x 256 9.6, 6.1; 33 x 768 x 768 9.7, 6.4; 100 x 768 x 768 9.6, 6.5; 256 x 768 x 768 9.7, 7.2; 333 x 512 x 512 9.7, 6.9;
-    // 512 x 512 x 512 9.6, 7.8; 64 x 1536 x 1536 9.3, 6.8; 128 x 1536 x 1536 9.4, 8.0; 48 x 2048 x 2048 9.4, 8.1; 256 x 1024 x 1024 9.6, 8.2; 256 x
-    // 768 x 3072 9.4, 8.0 -- beyond: 100 x 2048 x 2048 9.4, 9.5; 128 x 2048 x 2048 9.4, 10.0; 48 x 4096 x 1024 9.9, 11.5; 256 x 1024 x 4096 9.5, 9.7; 512 x
-    // 512 x 4096 9.7, 9.7; 333 x 768 x 3072 9.6, 9.3.
+    // microsecond more or less (64 sizes of 33 to 512 rows); two launches 8.3 to 8.8 on most hosts.  us, two launches there and one: 33 x 768 x
+    // 768 8.6, 5.7; 256 x 768 x 768 8.4, 7.5; 333 x 768 x 768 8.5, 8.4; 128 x 1024 x 1024 8.5, 6.9; 200 x 1024 x 1024 8.5, 7.8; 100 x 1536 x 1536
+    // 8.5, 7.7; 33 x 2048 x 2048 8.7, 7.0; 64 x 2048 x 2048 8.7, 8.2; 256 x 768 x 3072 8.5, 7.9 -- beyond: 128 x 1536 x 1536 8.6, 8.1; 256 x 1024 x
+    // 1024 8.5, 8.7; 200 x 1024 x 4096 8.6, 8.4; 512 x 512 x 2048 8.5, 8.9; 100 x 2048 x 2048 8.6, 8.9; 333 x 768 x 3072 8.4, 9.2.  A host in its
+    // fastest state issues two launches in 6.8: 256 x 512 x 512 6.8, 6.4; 333 x 512 x 512 6.8, 7.1; 512 x 512 x 512 6.8, 8.2.
+    // Layers that are fed one tensor (q, k and v) share a build in two launches and not in one: three of them and nothing else, us, 33 x 768 x
+    // 768 20.8, 17.2; 200 x 768 x 768 20.2, 20.1; 256 x 768 x 768 20.3, 21.6; 512 x 512 x 512 15.9, 22.7.  In a decoder, whose other kernels leave the GPU
+    // waiting for the host, one launch still gains there: passes through three or four layers of 333 x 512 472, 432; 512 x 512 470, 442; 333 x 768
+    // 356, 332; 200 x 1024 351, 327.  So the line lies where a single layer gains on most hosts.
     const double us = 0.755 * static_cast<double>(items) / static_cast<double>(a_round) + 0.32 * static_cast<double>(chunks) +
                       1.9e-6 * static_cast<double>(Q) * static_cast<double>(R);
     return groups <= 256 && us <= 4.4 ? 1 : 0;

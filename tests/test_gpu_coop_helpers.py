@@ -44,7 +44,7 @@ def test_same_bits_as_two_launches(ops, monkeypatch, Q, d, R, dtype, patience):
         ops.linear_cuda_forget()
 
 
-@pytest.mark.parametrize("Q, d, R, served", [(48, 2048, 2048, 1), (128, 2048, 2048, 0), (33, 4096, 1024, 0), (256, 768, 3072, 1), (512, 512, 512, 1),
+@pytest.mark.parametrize("Q, d, R, served", [(48, 2048, 2048, 1), (128, 2048, 2048, 0), (33, 4096, 1024, 0), (256, 768, 3072, 1), (512, 512, 512, 1), (128, 1536, 1536, 0), (256, 1024, 1024, 0), (64, 2048, 2048, 1), (200, 1024, 1024, 1), (100, 1536, 1536, 1),
                                              (512, 512, 4096, 0), (128, 1600, 512, 1), (128, 1600, 1600, 0), (300, 704, 256, 1), (300, 704, 255, 0)])
 def test_where_the_rule_lies(ops, Q, d, R, served):
     assert ops.lib.bsi_hip_linear_coop_serves(Q, d, R, 2, 7, 2, 6) == served
