@@ -73,6 +73,7 @@ PROTOTYPES = {
     "bsi_hip_linear_few_rows_upfront": [_i64, _i64, _i64],
     "bsi_hip_linear_few_rows_shares": [_i64, _i64, _i64],
     "bsi_hip_linear_workspace_bytes": [_i64, _i64, _i],
+    "bsi_hip_linear_plan": [_i64, _i64, _i64, _i64, _i, ctypes.POINTER(ctypes.c_int), ctypes.POINTER(ctypes.c_int)],
     "bsi_hip_linear_workspace_bytes_for": [_i64, _i64, _i, _i, _i, _i64, _i],
     "bsi_hip_linear": [_vp, _i, _i64, _i64, _i, _i, _i, _vp, _sz, _vp, _i, _vp, _i, _i64, _f, _i64, _vp, _vp, _i, _vp,
                        _sz, _vp],

@@ -109,7 +109,7 @@ extern "C" int bsi_hip_dot_attach_split_scratch(void* scratch_device, size_t byt
 extern "C" int bsi_hip_dot_split_plan(int64_t R, int64_t Q, int W64, int* tile, int* segments) {
     BSI_REQUIRE(tile && segments && R >= 1 && Q >= 1 && W64 >= 1, "bad arguments");
     const int split_tile = choose_i8_split(R, Q, (W64 + 3) / 4, segments);
-    *tile = split_tile != 0 ? split_tile : choose_i8_tile(R, Q, nullptr, W64 > 8 ? (W64 + 3) / 4 : 0);
+    *tile = split_tile != 0 ? split_tile : choose_i8_chain_tile(R, Q, (W64 + 3) / 4, false);
     return BSI_OK;
 }
 
@@ -341,6 +341,19 @@ extern "C" size_t bsi_hip_linear_workspace_bytes_for(int64_t Q, int64_t d, int f
     const LinearWorkspace w = linear_workspace(Q, d, fixed_bits);
     const int64_t chunks = (d + 255) / 256;
     return chunks <= kMfmaMaxChunks && linear_is_large(Q, static_cast<int>(chunks), b_layout, Sb, R, core) ? w.total : w.large;
+}
+
+extern "C" int bsi_hip_linear_plan(int64_t Q, int64_t d, int64_t R, int64_t R_total, int out_dtype, int* tile, int* streamed) {
+    BSI_REQUIRE(tile && streamed && Q >= 1 && d >= 1 && R >= 1 && R_total >= R && d <= 256LL * kMfmaMaxChunks, "bad arguments");
+    const int chunks = static_cast<int>((d + 255) / 256);
+    int segments = 1;
+    const int split_tile = choose_i8_split(R, Q, chunks, &segments);
+    const bool large = i8_large_serves(Q, R, chunks);
+    *tile = large ? kLargeTile : split_tile != 0 ? split_tile : choose_i8_chain_tile(R, Q, chunks, true);
+    t_layer_output = 1;
+    *streamed = out_dtype == BSI_DTYPE_F32 && R_total % 32 == 0 ? stream_output(R_total, Q, chunks) : 0;
+    t_layer_output = 0;
+    return BSI_OK;
 }
 
 extern "C" int bsi_hip_linear(const void* x, int dtype, int64_t Q, int64_t d, int decimal_places, int fixed_bits, int rebuild,

@@ -100,7 +100,6 @@ struct I8Cfg {
     static_assert(kConsumers < 15, "flag words of the MFMA waves, then the decision word");
 };
 constexpr int kSplitLeave = 0, kSplitCombine = 1, kSplitRedo = 2;
-constexpr int kLargeTile = 256;  // dot_mfma_i8_large_kernel: keys and queries of a workgroup
 
 // How the chunk scales are fetched (kFour of the kernels): one float of each of 64 queries for every chunk, or four consecutive
 // floats of 16 queries, for the group of four chunks after the one a load is issued in.  The scales of a query are contiguous:
@@ -2028,7 +2027,7 @@ thread_local int t_out_dtype = BSI_DTYPE_F32;
 std::atomic<int> g_output_stores{0};  // 0 = by entry point, 1 = always plain, 2 = always nontemporal
 constexpr int64_t kStreamedOutputs = 20 << 20;  // float32 outputs of a layer
 constexpr int kStreamedChunks = 8;
-static int stream_output(int64_t R_total, int64_t Q, int chunks) {
+int stream_output(int64_t R_total, int64_t Q, int chunks) {
     const int forced = g_output_stores.load(std::memory_order_relaxed);
     if (forced != 0) return forced == 2 ? 1 : 0;
     return t_layer_output && (R_total * Q < kStreamedOutputs || chunks < kStreamedChunks) ? 0 : 1;
@@ -2211,8 +2210,14 @@ static void launch_mfma_i8w(const int8_t* A8, const float* qscale, int stride, c
 // but the last (all CUs store 32 MiB at the same time, with nothing else of theirs resident); the images are written at 0.75 a
 // million elements; the launch that ends at once and the gaps are 14.  Measured, 128 x 128 and 256 x 256, bf16: taken 1024 x 4096 x
 // 16384 73.6, 69.3; 4096 x 3072 x 16384 225, 207; 2048 x 8192 x 8192 150, 128.5; 1024 x 8192 x 16384 165, 123; not taken 4096 x 1024 x
-// 16384 92, 99; 4096 x 2048 x 16384 155, 160 (f32 176, 188); 4096 x 2048 x 8192 78, 85; 2048 x 4096 x 8192 74, 75 (f32 78, 81);
-// 4096 x 4096 x 4096 78, 80; 3000 x 4096 x 11008 160, 172; and, at its edge, 2048 x 2048 x 16384 81, 77 (f32 88, 88).
+// 16384 92, 99; 4096 x 2048 x 16384 155, 160; 4096 x 2048 x 8192 78, 85; 2048 x 4096 x 8192 74, 75 (f32 78, 81);
+// 4096 x 4096 x 4096 78, 80; 3000 x 4096 x 11008 160, 172; and, at its edge, 2048 x 2048 x 16384 81, 77.  Float32 outputs that are streamed
+// (stream_output), taken: 4096 x 4096 x 16384 313, 267; 4096 x 3072 x 16384 246, 224; 4096 x 4096 x 8192 156, 148; not taken: 4096 x 2048 x 16384
+// 165, 168; 2048 x 2048 x 16384 88, 93; 2048 x 4096 x 11008 114, 128; 3000 x 4096 x 11008 166, 183; 4096 x 4096 x 6144 122, 142, and, where it would
+// gain, 1536 x 8192 x 16384 238, 214; 2500 x 6144 x 8448 180, 173.
+// A last round that runs as parts (i8_rest) is charged whole: charged as the parts take by themselves, layers would go to 128 x 128 that
+// lose there.  128 x 128 with parts, and 256 x 256: bf16 2555 x 6144 x 5120 98.8, 96.1; 3276 x 8192 x 4096 142, 125; 3510 x 8192 x 3584 139, 127;
+// 1287 x 5120 x 9472 85.2, 78.8; 3113 x 4096 x 9216 133, 128; f32 2555 x 6144 x 5120 114, 105; 3510 x 8192 x 3584 165, 140.
 // Beyond 1 GiB of image the layer keeps to the workspace it had without units, which would be two more.
 constexpr int64_t kLargeMaxItems = 1 << 22;  // (row, chunk) items
 static size_t large_aligned(size_t v) { return (v + 255) / 256 * 256; }
@@ -2329,16 +2334,10 @@ void launch_i8_large(void* workspace, bool units_there, const int8_t* A8, const 
 // leaves CUs idle that smaller tiles would use: a workgroup's time per half-chunk is about 1 : 0.63 : 0.35 : 0.31
 // for 128 x 128 : 128 x 64 : 64 x 64 : 64 x 32, so take the least (rounds of 256 workgroups x time), the larger
 // tile on a tie.  g_i8_tile forces a tile (tuning and tests).
-int choose_i8_tile(int64_t R, int64_t Q, int64_t* cost_out, int chunks) {
+int choose_i8_tile(int64_t R, int64_t Q, int64_t* cost_out) {
     const int64_t n128 = ((R + 127) / 128) * ((Q + 127) / 128);
     if (cost_out) *cost_out = ((n128 + 255) / 256) * 100;
     if (const int forced = g_i8_tile.load(std::memory_order_relaxed); forced != 0 && forced != kLargeTile) return forced;
-    // Half a round over: three rounds of 128 x 64 for two, where rows are short enough for a tile's start and stores to count (chunks: of the
-    // rows where the caller's kernel has both forms).  us a layer, 128 x 128 and 128 x 64, 512 and 1024 wide: 768 x 8192 keys bf16 14.3, 13.5
-    // and 17.7, 17.1; 1280 x 4096 f32 15.4, 14.5 and 18.9, 18.3; 3000 x 1920 bf16 15.2, 14.1 and 20.5, 18.8; 530 x 8192 f32 14.7, 13.5 and
-    // 17.3, 17.0 -- 2048 wide 768 x 8192 f32 25.2, 25.7, 1536 x 4096 bf16 26.2, 26.7; 256 wide 1280 x 4096 bf16 12.5, 11.5, but 768 x 8192 14.3, 16.1.  A
-    // dot, which streams its outputs out, from three chunks on: 640 x 1024 x 8192 14.4, 12.4; 768 x 512 x 8192 9.7, 10.2 (its caller leaves `chunks` out).
-    if (n128 > 256 && n128 <= 384 && chunks >= 2 && chunks <= 4 && ((R + 127) / 128) * ((Q + 63) / 64) <= 768) return 12864;
     if (n128 > 256) return 128;
     const int64_t cost[4] = {100, ((((R + 127) / 128) * ((Q + 63) / 64) + 255) / 256) * 63,
                              ((((R + 63) / 64) * ((Q + 63) / 64) + 255) / 256) * 35,
@@ -2349,6 +2348,18 @@ int choose_i8_tile(int64_t R, int64_t Q, int64_t* cost_out, int chunks) {
         if (cost[i] < cost[best]) best = i;
     if (cost_out) *cost_out = cost[best];
     return tiles[best];
+}
+
+// Half a round over: three rounds of 128 x 64 for two, where rows are short enough for a tile's start and stores to count.  us a layer, 128
+// x 128 and 128 x 64, 512 and 1024 wide: 768 x 8192 keys bf16 14.3, 13.5 and 17.7, 17.1; 1280 x 4096 f32 15.4, 14.5 and 18.9, 18.3; 3000 x
+// 1920 bf16 15.2, 14.1 and 20.5, 18.8; 530 x 8192 f32 14.7, 13.5 and 17.3, 17.0 -- 2048 wide 768 x 8192 f32 25.2, 25.7, 1536 x 4096 bf16 26.2,
+// 26.7; 256 wide 1280 x 4096 bf16 12.5, 11.5, but 768 x 8192 14.3, 16.1.  A dot, which streams its outputs out, from three chunks on: 640 x
+// 1024 x 8192 14.4, 12.4; 768 x 512 x 8192 9.7, 10.2.
+int choose_i8_chain_tile(int64_t R, int64_t Q, int chunks, bool layer) {
+    const int tile = choose_i8_tile(R, Q);
+    const int64_t n128 = ((R + 127) / 128) * ((Q + 127) / 128);
+    if (tile != 128 || g_i8_tile.load(std::memory_order_relaxed) == 128 || n128 <= 256 || n128 > 384) return tile;
+    return chunks >= (layer ? 2 : 3) && chunks <= 4 && ((R + 127) / 128) * ((Q + 63) / 64) <= 768 ? 12864 : tile;
 }
 
 void i8_launch_shape(int64_t Q, int64_t R, unsigned* groups, int* waves) {
@@ -2429,7 +2440,8 @@ void launch_mfma_i8(const int8_t* A8, const float* qscale, int stride, const int
                            int chunks, int64_t R, int64_t Q, int down_shift, float scale_inv, int64_t R_total,
                            float* out, int32_t* chunk_ints, const float* bias, hipStream_t st, int key_tiled,
                            int ndig, long long dig_stride, const long long* key_indices) {
-    if (ndig == 0 && chunk_ints == nullptr && t_coop == nullptr) {
+    const bool chain = ndig == 0 && chunk_ints == nullptr && t_coop == nullptr;
+    if (chain) {
         int segments = 1;
         const int split_tile = choose_i8_split(R, Q, chunks, &segments);
         if (split_tile == 128) {
@@ -2445,7 +2457,7 @@ void launch_mfma_i8(const int8_t* A8, const float* qscale, int stride, const int
             return;
         }
     }
-    const int tile = choose_i8_tile(R, Q, nullptr, ndig == 0 && chunk_ints == nullptr && t_coop == nullptr && (t_layer_output || chunks > 2) ? chunks : 0);
+    const int tile = chain ? choose_i8_chain_tile(R, Q, chunks, t_layer_output != 0) : choose_i8_tile(R, Q);
     if (tile == 1284 && ndig == 0 && t_coop == nullptr) {
         launch_mfma_i8w<4>(A8, qscale, stride, K8, Bw, Sb, chunks, R, Q, down_shift, scale_inv, R_total, out, chunk_ints, bias,
                            st, key_tiled);

@@ -33,7 +33,12 @@ extern thread_local int t_out_dtype;
 // Set by bsi_hip_linear_coop_out around its launch: the query build the kernel does itself (bsi_coop_build.h).
 struct CoopBuild;
 extern thread_local const CoopBuild* t_coop;
-int choose_i8_tile(int64_t R, int64_t Q, int64_t* cost_out = nullptr, int chunks = 0);
+constexpr int kLargeTile = 256;  // dot_mfma_i8_large_kernel: keys and queries of a workgroup
+int choose_i8_tile(int64_t R, int64_t Q, int64_t* cost_out = nullptr);
+// The tile of a dot that keeps neither chunk integers nor a build of its own (layer: one of a linear layer, whose outputs are not streamed out).
+int choose_i8_chain_tile(int64_t R, int64_t Q, int chunks, bool layer);
+// Whether such a call's float32 outputs of whole lines are stored past the caches.
+int stream_output(int64_t R_total, int64_t Q, int chunks);
 // D-split of the chain-mode int8-image dot (bsi_hip_dot_attach_split_scratch): the calling thread's scratch region
 // (counters of kSplitCounterBytes, then the segments' partial sums) and the device it lies on; the option
 // BSI_OPT_I8_SPLIT; the choice itself (tile 128 / 12864 and *segments, or 0).

@@ -239,7 +239,7 @@ int bsi_hip_planes_to_int8_tiled(const uint64_t* words_device, int64_t rows, int
 #define BSI_OPT_OUTPUT_STORES 4 /* how the int8-image kernels store whole output tiles: 1 = plain stores (the output stays
                                    in the caches for the next kernel), 2 = nontemporal stores (it leaves them as it is
                                    written); 0 (default) = plain from the linear-layer entry points (bsi_hip_dot_bias,
-                                   bsi_hip_dot_bias_warm, bsi_hip_linear) below 80 MiB of outputs or 2048 elements a row,
+                                   bsi_hip_dot_bias_warm, bsi_hip_linear) below 80 MiB of float32 outputs or 2048 elements a row,
                                    nontemporal from there on and from the other dot entry points */
 #define BSI_OPT_I8_SPLIT 5 /* D-split of the int8-image dot (see bsi_hip_dot_attach_split_scratch): 1 = never, n >= 2 = n
                               segments (on the tile BSI_OPT_I8_TILE forces, 128 or 12864; 128 otherwise) whenever the
@@ -402,6 +402,10 @@ int bsi_hip_linear_coop_out(const void* x_device, int dtype, int64_t Q, int64_t 
                             uint64_t launch_number, void* area, const uint64_t* B, int b_layout, const float* Bw, int Sb, int64_t R,
                             float scale_inv, int64_t R_total, const float* bias, void* out, int out_dtype, const void* warm,
                             size_t warm_bytes, void* stream);
+
+/* What bsi_hip_linear_out does on int8-image keys of 6 planes: the tile (as BSI_OPT_I8_TILE names them; 256: integer sums) and whether
+ * outputs that begin at a line are stored past the caches.  Host-side queries like the next two. */
+int bsi_hip_linear_plan(int64_t Q, int64_t d, int64_t R, int64_t R_total, int out_dtype, int* tile, int* streamed);
 
 /* 1 when bsi_hip_linear_few_rows, for this shape, issues the loads of the whole query build before its first key
  * loads (the case in which the launch costs the GPU no more than the dot alone), 0 when some of the build waits

@@ -1,5 +1,7 @@
 """Outputs whose rows begin anywhere, tiles past whose last query or key the output ends: every int8-image kernel writes what it writes
 into aligned rows, and nothing beside them."""
+import ctypes
+
 import pytest
 import torch
 
@@ -44,12 +46,17 @@ def test_rows_that_begin_anywhere(ops, dtype, tile, Q, R, stride, offset):
     assert torch.isnan(buf[:offset]).all() and torch.isnan(rows[:, R:]).all() and torch.isnan(buf[offset + Q * stride:]).all()
 
 
-@pytest.mark.parametrize("Q,d,R", [(1281, 2048, 16384), (2561, 2000, 8192), (5130, 2048, 4100)])
-def test_large_float32_outputs_streamed(ops, Q, d, R):
-    """80 MiB of outputs and 2048 elements a row: the stores' kind changes, not what they write."""
+@pytest.mark.parametrize("Q,d,R,streamed", [(1281, 2048, 16384, 1), (2561, 2000, 8192, 1), (5130, 2048, 4100, 0), (5130, 2048, 4128, 1), (1279, 2048, 16384, 0),
+                                            (5130, 1792, 4128, 0)])
+def test_large_float32_outputs_streamed(ops, Q, d, R, streamed):
+    """80 MiB of outputs and more than 1792 elements a row, rows of whole lines: the stores' kind changes, not what they write."""
     from bsipytorch_amd import _lib
     from bsipytorch_amd.linear import BSIQuantizedLinear
 
+    tile, plan = ctypes.c_int(), ctypes.c_int()
+    for dtype, want in ((_lib.DTYPE_F32, streamed), (_lib.DTYPE_BF16, 0)):
+        assert _lib.lib.bsi_hip_linear_plan(Q, d, R, R, dtype, ctypes.byref(tile), ctypes.byref(plan)) == 0
+        assert plan.value == want
     gen = torch.Generator(device="cuda").manual_seed(R)
     x = torch.randn(Q, d, generator=gen, device="cuda")
     dense = torch.nn.Linear(d, R, device="cuda")
