@@ -7,11 +7,13 @@
 // by a flag behind it.
 //
 // No workgroup depends on another one being resident.  A share's bytes do not depend on who builds it, so a workgroup that
-// has waited kCoopPatience for a share builds it itself, waits half as long for the next, and so on down to an eighth: beside kernels
-// that hold the CUs, most shares of a copy may belong to workgroups that have not begun.  Every CU of an XCD begins at another missing
-// share, and between two a workgroup looks at all flags.  us a layer beside a layer of 4096 x 4096 x 16384 on another stream (256 workgroups
-// with all LDS of a CU each), median of 36, with a whole patience for every share and the lowest one first, and so: 16 x 4096 x 4096
-// 154, 80 (whole patience, from different shares: 107); 33 x 768 x 768, 128 x 1024 x 1024, 333 x 512 x 512 40 to 50 either way.  Flags hold the launch's number, which no other launch has: nothing
+// has waited kCoopPatience for a share builds it itself: beside kernels that hold the CUs, most shares of a copy may belong to workgroups
+// that have not begun.  Every CU of an XCD begins at another missing share, and between two a workgroup looks at all flags.  us a layer of
+// 16 x 4096 x 4096 beside one of 4096 x 4096 x 16384 on another stream (256 workgroups with all LDS of a CU each), median of 36: 150 with
+// a patience of 20 us and the lowest share first for all, 106 from different shares, 83 with 10 us, 64 to 71 with 5, 62 with 3; layers of a
+// few tiles 35 to 50 in all forms.  On an idle GPU a build takes 2 to 5 us from the first workgroup's begin, and a share is waited for from
+// the end of the own one.  (Half the patience for every further share: 78, but the few-rows kernel then keeps other arguments in
+// registers: 12 x 4096 x 11008 12.1, 11.5; 16 x 5376 x 7168 10.2, 10.4; 12 x 2048 x 8192 6.3, 6.5.)  Flags hold the launch's number, which no other launch has: nothing
 // is cleared between launches, and flags of earlier ones mean nothing.
 //
 // What a reader relies on, since neither side of a flag is more than a relaxed access (an agent-scope release writes the L2
@@ -46,7 +48,7 @@ constexpr size_t kCoopFlagBytes = kXcds * kCoopShares * sizeof(unsigned long lon
 constexpr size_t kCoopCopyBytes = static_cast<size_t>(kCoopMaxItems) * (BSI_CHUNK_ELEMS + sizeof(float));
 constexpr size_t kCoopBytes = kCoopFlagBytes + kXcds * kCoopCopyBytes;
 static_assert(kCoopFlagBytes % 128 == 0 && kCoopCopyBytes % 128 == 0, "flags and copies share no cache line");
-constexpr int kCoopPatience = 2000;  // ticks of the 100 MHz clock: 20 us
+constexpr int kCoopPatience = 500;  // ticks of the 100 MHz clock: 5 us
 
 struct CoopBuild {
     const void* x;
@@ -276,7 +278,6 @@ __device__ __forceinline__ void coop_build(const CoopBuild& b, unsigned id, unsi
         ahead();
         issued = true;
     }
-    unsigned patience = static_cast<unsigned>(b.patience);
 #pragma unroll 1
     for (;;) {
         if (share >= 0) build(share);
@@ -287,7 +288,7 @@ __device__ __forceinline__ void coop_build(const CoopBuild& b, unsigned id, unsi
                 const bool here = lane >= b.shares ||
                                   __hip_atomic_load(flags + (lane < kCoopShares ? lane : 0), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == b.launch;
                 missing = __ballot(!here);
-                if (missing == 0ULL || wall_clock64() - since > patience) break;
+                if (missing == 0ULL || wall_clock64() - since > static_cast<unsigned>(b.patience)) break;
             }
             if (lane == 0) shared[0] = static_cast<unsigned>(missing);
         }
@@ -295,10 +296,9 @@ __device__ __forceinline__ void coop_build(const CoopBuild& b, unsigned id, unsi
         const unsigned missing = static_cast<unsigned>(__builtin_amdgcn_readfirstlane(static_cast<int>(shared[0])));
         lds_barrier();
         if (missing == 0u) break;
-        // HW_ID, CU and shader engine: every CU of an XCD begins elsewhere
-        const unsigned cu = __builtin_amdgcn_s_getreg((7 << 11) | (8 << 6) | 4), from = ((cu & 7u) * 4u + (cu >> 5 & 3u)) % kCoopShares;
+        // HW_ID, CU and shader engine: every CU of an XCD begins elsewhere, and neighbours (the first to be given work) far apart
+        const unsigned cu = __builtin_amdgcn_s_getreg((7 << 11) | (8 << 6) | 4), from = ((cu & 7u) * 4u + (cu >> 5 & 3u)) * 13u % kCoopShares;
         share = static_cast<int>((__builtin_ctz(__builtin_rotateright32(missing, from)) + from) % kCoopShares);
-        if (patience > kCoopPatience / 8) patience >>= 1;
     }
     if (!issued) ahead();
     asm volatile("" ::: "memory");

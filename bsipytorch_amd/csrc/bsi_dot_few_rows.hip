@@ -86,10 +86,8 @@ __global__ __launch_bounds__(1024) void dot_mfma_stream_kernel(
     };
     // Workgroups beyond the tiles, there for the build (coop_groups), go on with the last tile and store nothing: a branch past the rest
     // costs the others 0.2 us (16 x 4096 x 4096 7.8 -> 8.0).
-    if constexpr (kBuild) {
-        asm volatile("" : "+s"(R), "+s"(Q));  // held over the build: a fetch behind it is one that all waves wait for (12 x 4096 x 11008 12.4, 11.5 us)
+    if constexpr (kBuild)
         coop_build<true, kBuild == 2>(coop, blockIdx.x, reinterpret_cast<unsigned*>(ints), A8, qscale, [&] { load_keys(wave < pass_chunks ? wave : pass_chunks - 1); });
-    }
 
     // the chain lanes: tid <-> (key tile, query tile, query, key), keys fastest so output stores are contiguous
     float accf = 0.0f;

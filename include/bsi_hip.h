@@ -244,8 +244,8 @@ int bsi_hip_planes_to_int8_tiled(const uint64_t* words_device, int64_t rows, int
 #define BSI_OPT_I8_SPLIT 5 /* D-split of the int8-image dot (see bsi_hip_dot_attach_split_scratch): 1 = never, n >= 2 = n
                               segments (on the tile BSI_OPT_I8_TILE forces, 128 or 12864; 128 otherwise) whenever the
                               attached scratch holds them; 0 (default) = chosen per call by a cost model */
-#define BSI_OPT_COOP_PATIENCE 6 /* ticks of the 100 MHz clock that a workgroup of bsi_hip_linear_coop_out waits for the query
-                                   build before it builds what is missing itself (default 2000; 0: at once) */
+#define BSI_OPT_COOP_PATIENCE 6 /* ticks of the 100 MHz clock that a workgroup of bsi_hip_linear_coop_out waits for a share of
+                                   the query build before it builds the share itself (default 500; 0: at once) */
 #define BSI_OPT_COOP_SHARES 7 /* shares of the build of bsi_hip_linear_coop_out on each XCD, at most 32; 0 (default) = as many as
                                  it has workgroups.  More of them leaves shares to nobody, so that the wait runs out (tests) */
 int bsi_hip_set_option(int option, int value);
