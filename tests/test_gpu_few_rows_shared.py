@@ -8,7 +8,7 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("Q,d,R,shares", [(2, 2304, 16384, 0), (2, 4096, 16384, 1), (2, 5120, 5120, 1), (3, 4096, 5120, 1), (4, 4096, 4096, 0), (4, 8192, 2048, 1),
-                                          (1, 8192, 8192, 0), (4, 1024, 77, 0)])
+                                          (1, 8192, 8192, 0), (4, 1024, 77, 0), (3, 8186, 1024, 1), (2, 5110, 5120, 1)])  # the last two: rows that no quad can be loaded from
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 def test_same_bits(ops, monkeypatch, Q, d, R, shares, dtype):
     from bsipytorch_amd import _native
